@@ -119,6 +119,16 @@ def build_scan_pieces(q_lens, target: int = SCAN_PIECES_TARGET):
     return np.asarray(pieces, dtype=np.int32).reshape(-1, 3), np.asarray(first, dtype=np.int32)
 
 
+def _retention_blocks(proj, q_col, k_col, v_col, dim, vdim, cos_sin, rot_dims, layout) -> bool:
+    """Rows that the block form on the matrix cores takes: bf16, 128 key channels, 128 or 256 value channels (its waves hold 32
+    columns each), 16-byte loads, a rotation whose partners lie in groups of four.  Only steps cut into pieces reach it:
+    8192 rows of 32 heads with 128 x 256 states take 0.70 ms there and 2.29 ms token by token;
+    steps of short sequences have no pieces and walk their few tokens one by one."""
+    return (proj.dtype == torch.bfloat16 and dim == 128 and vdim in (128, 256) and rot_dims % 8 == 0 and layout in (0, 1)
+            and proj.stride(0) % 8 == 0 and proj.data_ptr() % 16 == 0 and (q_col | k_col | v_col) % 8 == 0
+            and (rot_dims == 0 or (cos_sin.data_ptr() % 16 == 0 and cos_sin.is_contiguous())))
+
+
 def recurrent_scan(proj, q_col: int, k_col: int, v_col: int, heads: int, dim: int, vdim: int, state, state_off: int,
                    seq_cu, seq_state, positions, *, decay=None, cos_sin=None, rot_dims: int = 0, layout: int = 0,
                    k_scale: float = 1.0, gate_bias=None, gate_lower=None, pieces=None, min_decay: float = 0.0,
@@ -158,6 +168,18 @@ def recurrent_scan(proj, q_col: int, k_col: int, v_col: int, heads: int, dim: in
     assert (gate_bias is not None and gate_lower is not None) if gated else (rot_dims == 0 or cos_sin.shape[1] == rot_dims)
     assert rot_dims <= dim and rot_dims % 2 == 0 and not (act and (gated or rot_dims))
     out = torch.empty((proj.shape[0], heads, vdim), dtype=torch.float32, device=proj.device)
+    if pieces is not None and not gated and _retention_blocks(proj, q_col, k_col, v_col, dim, vdim, cos_sin, rot_dims, layout):
+        pc, sp = pieces
+        _i32(pc, sp)
+        assert pc.shape[1] == 3 and sp.numel() == seq_cu.numel() and pc.is_contiguous()
+        ws_state = torch.empty((pc.shape[0], heads, dim, vdim), dtype=torch.float32, device=proj.device)
+        o._check(o._kernels().vpsa_retention_scan(
+            o._p(proj), c_long(proj.stride(0)), c_int(q_col), c_int(k_col), c_int(v_col), c_int(heads), c_int(vdim),
+            _at(state, state_off), c_long(state.stride(0)), o._p(seq_cu), o._p(seq_state), c_int(seq_state.numel()),
+            o._p(positions), o._p(decay), o._p(cos_sin), c_int(rot_dims), c_int(layout), c_float(k_scale),
+            c_int(1 if act else 0), o._p(out), o._p(pc), o._p(sp), c_int(pc.shape[0]), o._p(ws_state), o._stream()),
+            "retention_scan")
+        return out
     # what enters the recurrence besides v, prepared in fp32 by a pass of its own: q' | k' (| gates)
     prep = torch.empty((proj.shape[0], heads, 3 if gated else 2, dim), dtype=torch.float32, device=proj.device)
     pc = sp = ws_state = ws_decay = None
