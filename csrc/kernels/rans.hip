@@ -11,21 +11,29 @@
 // share statistics), ctx_len symbols each.  A context is cut into spc streams; stream j owns
 // symbols j, j + spc, j + 2 spc, ... so that at every step the 64 lanes of a wave touch 64
 // consecutive bytes (coalesced loads in the encoder, coalesced stores in the decoder).
-// One thread codes one stream.  Per context: a 256-entry frequency table normalised to 2^12,
+// One thread codes one stream; a workgroup is one wave (64 streams), so that a page's 16384 streams reach every CU: what bounds
+// both directions is a stream's chain of dependent steps, not arithmetic or bytes.  The chain is kept short:
+//   encoder  symbols and their table entries are read a batch of eight ahead, the division by a symbol's frequency is a
+//            multiplication, coded bytes leave four at a time;
+//   decoder  one table entry per step (symbol, frequency and offset within it), the wave's coded bytes staged in LDS and
+//            consumed from a register window, at most two bytes a step without a loop.
+// Page of a 32-layer cache with 8 KV heads (4.2 M symbols): coding loop 107 -> 25 us, with tables and gathering 150 -> 47; decoding
+// 118 -> 33 us (before: 64 workgroups, symbols and coded bytes read and written one at a time from memory, divisions).
+// Per context: a 256-entry frequency table normalised to 2^12,
 // built from a histogram of that very page (it travels with the blob: 512 B per context).
 // Coder: 32-bit state, byte-wise renormalisation, lower bound 2^23.  The encoder runs over its
 // symbols backwards and writes its bytes backwards into a private scratch slot, so the decoder
-// reads forwards; vpsa_rans_pack then gathers the slots into one dense byte string at the
-// offsets given by the prefix sum of the sizes.
+// reads forwards; the slots are then gathered into one dense byte string at the prefix sum of the sizes.
 #include "common.h"
 
 #define RANS_BITS 12
 #define RANS_M (1u << RANS_BITS)
 #define RANS_LOW (1u << 23)
+#define RANS_HIST_BLOCKS 64
 
-// grid (blocks_per_ctx, n_ctx), block 256.  hist must be zeroed by the caller.
-__global__ __launch_bounds__(256) void rans_hist_kernel(const uint8_t* __restrict__ sym,
-                                                        uint32_t* __restrict__ hist, long ctx_len) {
+// grid (blocks_per_ctx, n_ctx), block 256: a block's own histogram -> part[ctx][block][256].
+__global__ __launch_bounds__(256) void rans_hist_kernel(const uint8_t* __restrict__ sym, uint32_t* __restrict__ part,
+                                                        long ctx_len) {
   __shared__ uint32_t h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
@@ -39,21 +47,36 @@ __global__ __launch_bounds__(256) void rans_hist_kernel(const uint8_t* __restric
     atomicAdd(&h[w >> 24], 1u);
   }
   __syncthreads();
-  if (h[threadIdx.x]) atomicAdd(&hist[blockIdx.y * 256 + threadIdx.x], h[threadIdx.x]);
+  part[((long)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x] = h[threadIdx.x];
+}
+
+// What the encoder needs of a symbol of frequency f and start c.  With s = ceil(log2 f) and m = ceil(2^(31 + s) / f) the
+// quotient x / f of x < 2^31 is floor(x m / 2^(31 + s)): the product is off by less than x f / (f 2^(31 + s)) < 1 / f.  The new
+// state (x / f) 4096 + x % f + c is x + (x / f) (4096 - f) + c.  f = 1 would need m = 2^31 and a shift to the left; m = 2^32 - 1
+// gives x - 1 instead (x >= 1), and c + 4095 makes up for it.
+// Words: m | f 2^19 | f 2^27 (or what no state reaches) | s - 1 (5 bits), 4096 - f (13), start (14).
+__device__ __forceinline__ u32x4 rans_enc_entry(uint32_t f, uint32_t c) {
+  if (f == 0) return (u32x4){0, 0, 0, 0};
+  const uint32_t one = f << 19, two = f < 16 ? f << 27 : 0xffffffffu;
+  if (f == 1) return (u32x4){0xffffffffu, one, two, 4095u << 5 | (c + 4095u) << 18};
+  const uint32_t s = 32 - __clz(f - 1);
+  const uint64_t m = ((1ull << (31 + s)) + f - 1) / f;
+  return (u32x4){(uint32_t)m, one, two, (s - 1) | (RANS_M - f) << 5 | c << 18};
 }
 
 // grid n_ctx, block 256.  freq[s] = max(1, round(count * 4096 / total)) for symbols that occur,
 // then the entry with the largest frequency (lowest index on ties) absorbs the rounding error
-// so that the table sums to exactly 4096.  err[0] is set if that entry would drop below 1.
-__global__ __launch_bounds__(256) void rans_normalize_kernel(const uint32_t* __restrict__ hist,
-                                                             uint16_t* __restrict__ freq,
-                                                             uint16_t* __restrict__ cum, long ctx_len,
-                                                             int* __restrict__ err) {
+// so that the table sums to exactly 4096.  err[ctx]: that entry would drop below 1.
+__global__ __launch_bounds__(256) void rans_normalize_kernel(const uint32_t* __restrict__ part, int parts,
+                                                             uint16_t* __restrict__ freq, u32x4* __restrict__ table,
+                                                             long ctx_len, int* __restrict__ err) {
   __shared__ int sf[256];
   __shared__ int si[256];
   __shared__ int scan[256];
   const int t = threadIdx.x;
-  const uint32_t c = hist[blockIdx.x * 256 + t];
+  uint32_t c = 0;
+#pragma unroll 8
+  for (int i = 0; i < parts; ++i) c += part[((long)blockIdx.x * parts + i) * 256 + t];
   int f = 0;
   if (c) {
     f = (int)(((unsigned long long)c * RANS_M + (unsigned long long)(ctx_len / 2)) /
@@ -81,10 +104,8 @@ __global__ __launch_bounds__(256) void rans_normalize_kernel(const uint32_t* __r
   __syncthreads();
   if (t == imax) {
     f += diff;
-    if (f < 1) {
-      err[0] = 1;
-      f = 1;
-    }
+    err[blockIdx.x] = f < 1;
+    if (f < 1) f = 1;
   }
   // exclusive scan of the final frequencies
   scan[t] = f;
@@ -96,87 +117,273 @@ __global__ __launch_bounds__(256) void rans_normalize_kernel(const uint32_t* __r
     __syncthreads();
   }
   freq[blockIdx.x * 256 + t] = (uint16_t)f;
-  cum[blockIdx.x * 256 + t] = (uint16_t)(scan[t] - f);
+  table[blockIdx.x * 256 + t] = rans_enc_entry((uint32_t)f, (uint32_t)(scan[t] - f));
 }
 
-// grid (spc / 256, n_ctx), block 256.  cap = scratch bytes per stream (2 * symbols per stream).
-__global__ __launch_bounds__(256) void rans_encode_kernel(
-    const uint8_t* __restrict__ sym, const uint16_t* __restrict__ freq, const uint16_t* __restrict__ cum,
-    uint8_t* __restrict__ scratch, uint32_t* __restrict__ states, uint16_t* __restrict__ sizes,
-    long ctx_len, int spc, int cap) {
-  __shared__ uint16_t sf[256], sc[256];
-  const int ctx = blockIdx.y;
-  sf[threadIdx.x] = freq[ctx * 256 + threadIdx.x];
-  sc[threadIdx.x] = cum[ctx * 256 + threadIdx.x];
-  __syncthreads();
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  const long gs = (long)ctx * spc + j;
-  const uint8_t* p = sym + (long)ctx * ctx_len + j;
-  uint8_t* buf = scratch + gs * cap;
-  const int len = (int)(ctx_len / spc);
-  int pos = cap;
+// grid (spc / 64, n_ctx), block 64.  slot = scratch bytes per stream (2 * symbols per stream, up to a multiple of 4).
+// Symbols come through LDS and coded bytes leave through it, RANS_TILE symbols at a time: a load from memory in the loop would
+// wait for the stores before it.  Every step writes the two bytes it could emit below the position and moves it by those that
+// it does emit, without a branch; byte p of the 64 streams lies side by side, so that moving is all the address takes.
+// The table entries of a batch are read while the batch before is coded.  (A word at a time gathered in registers and stored to
+// the slot in the loop took 37 us a page, this 25.)
+#define RANS_TILE 256
+__global__ __launch_bounds__(64) void rans_encode_kernel(const uint8_t* __restrict__ sym, const u32x4* __restrict__ table,
+                                                         uint8_t* __restrict__ scratch, uint32_t* __restrict__ states,
+                                                         uint16_t* __restrict__ sizes, uint32_t* __restrict__ group_bytes,
+                                                         long ctx_len, int spc, int slot) {
+  constexpr int B = 8, WORDS = RANS_TILE / 2 + 1;  // two bytes a symbol, and a word begun in the tile before
+  __shared__ u32x4 tab[256];
+  __shared__ __attribute__((aligned(16))) uint8_t rows[RANS_TILE * 64];
+  __shared__ uint8_t bytes[WORDS * 4 * 64];
+  const int ctx = blockIdx.y, t = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tab[t + 64 * i] = table[ctx * 256 + t + 64 * i];
+  const long gs = (long)ctx * spc + blockIdx.x * 64 + t;
+  const uint8_t* p = sym + (long)ctx * ctx_len + blockIdx.x * 64;
+  const bool wide = ((uintptr_t)sym & 15) == 0;  // every row of 64 streams starts a multiple of 64 further on
+  uint32_t* out = reinterpret_cast<uint32_t*>(scratch + gs * slot + slot);  // the end of what is still to be written
   uint32_t x = RANS_LOW;
-  for (int k = len - 1; k >= 0; --k) {
-    const uint32_t s = p[(long)k * spc];
-    const uint32_t f = sf[s];
-    const uint32_t x_max = ((RANS_LOW >> RANS_BITS) << 8) * f;
-    while (x >= x_max && pos > 0) {
-      buf[--pos] = (uint8_t)(x & 0xff);
-      x >>= 8;
+  int pos = WORDS * 4, done = 0;  // in the tile's bytes, counted down; bytes of earlier tiles
+  for (int k1 = (int)(ctx_len / spc); k1 > 0; k1 -= RANS_TILE) {
+    const int k0 = max(k1 - RANS_TILE, 0), n = k1 - k0;
+    __syncthreads();
+    if (wide) {
+#pragma unroll
+      for (int i = 0; i < RANS_TILE / 16; ++i) {
+        const int r = i * 16 + (t >> 2);
+        if (r < n) *reinterpret_cast<u32x4*>(rows + r * 64 + (t & 3) * 16) =
+            *reinterpret_cast<const u32x4*>(p + (long)(k0 + r) * spc + (t & 3) * 16);
+      }
+    } else {
+#pragma unroll 16
+      for (int r = t >> 4; r < n; r += 4)
+        *reinterpret_cast<uint32_t*>(rows + r * 64 + (t & 15) * 4) =
+            *reinterpret_cast<const uint32_t*>(p + (long)(k0 + r) * spc + (t & 15) * 4);
     }
-    x = ((x / f) << RANS_BITS) + (x % f) + sc[s];
+    __syncthreads();
+    u32x4 nx[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) nx[i] = tab[rows[max(n - 1 - i, 0) * 64 + t]];
+    int at = (pos - 2) * 64 + t;
+    for (int k = n - 1; k >= 0; k -= B) {
+      u32x4 e[B];
+#pragma unroll
+      for (int i = 0; i < B; ++i) e[i] = nx[i];
+#pragma unroll
+      for (int i = 0; i < B; ++i) nx[i] = tab[rows[max(k - B - i, 0) * 64 + t]];
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        if (k - i < 0) break;
+        const uint32_t w = e[i][3];
+        bytes[at + 64] = (uint8_t)x;
+        bytes[at] = (uint8_t)(x >> 8);
+        const int n8 = (x >= e[i][1] ? 8 : 0) + (x >= e[i][2] ? 8 : 0);  // x < 2^31 and f 2^19 >= 2^19: never more than two
+        x >>= n8;
+        at -= n8 * 8;
+        // x < f 2^19 now: the quotient has 19 bits
+        x += __umul24(__umulhi(x, e[i][0]) >> (w & 31), (w >> 5) & 0x1fff) + (w >> 18);
+      }
+    }
+    pos = ((at - t) >> 6) + 2;
+    // whole words to the slot, the word begun goes on in the next tile
+    const bool last = k0 == 0;
+    const int w_lo = last ? pos >> 2 : (pos + 3) >> 2, n_w = WORDS - w_lo;
+#pragma unroll 8
+    for (int w = WORDS - 1; w >= w_lo; --w) {
+      const uint8_t* b = bytes + w * 256 + t;
+      out[w - WORDS] = b[0] | b[64] << 8 | b[128] << 16 | (uint32_t)b[192] << 24;
+    }
+    if (last) {
+      done += WORDS * 4 - pos;
+    } else {
+      done += n_w * 4;
+      out -= n_w;
+      const int part = w_lo * 4 - pos;  // bytes of a begun word
+      if (part)
+        for (int i = 0; i < 4; ++i) bytes[((WORDS - 1) * 4 + i) * 64 + t] = bytes[((w_lo - 1) * 4 + i) * 64 + t];
+      pos = WORDS * 4 - part;
+    }
   }
   states[gs] = x;
-  sizes[gs] = (uint16_t)(cap - pos);
+  sizes[gs] = (uint16_t)done;
+  int sum = done;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if (t == 0) group_bytes[ctx * gridDim.x + blockIdx.x] = (uint32_t)sum;
 }
 
-// One thread per stream: move its bytes from the scratch slot to the dense output.
+// Exclusive prefix of one value per lane.
+__device__ __forceinline__ int wave_before(int v) {
+  const int lane = threadIdx.x & 63;
+  int incl = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += u;
+  }
+  return incl - v;
+}
+
+// Block 256, one workgroup per 64 streams: their bytes from the scratch slots to the dense output.  The group's place is the sum
+// of the groups before it (a few hundred values: cheaper than a scan of its own).  The last workgroup leaves
+// meta = coded bytes | contexts whose table could not be normalised.
 __global__ __launch_bounds__(256) void rans_pack_kernel(const uint8_t* __restrict__ scratch,
                                                         const uint16_t* __restrict__ sizes,
-                                                        const long* __restrict__ offsets,
-                                                        uint8_t* __restrict__ out, long n_streams,
-                                                        int cap) {
-  const long gs = (long)blockIdx.x * 256 + threadIdx.x;
-  if (gs >= n_streams) return;
-  const int n = sizes[gs];
-  const uint8_t* src = scratch + gs * cap + (cap - n);
-  uint8_t* dst = out + offsets[gs];
-  for (int i = 0; i < n; ++i) dst[i] = src[i];
-}
-
-// grid (spc / 256, n_ctx), block 256.  coded_len bounds every read (a damaged blob decodes to
-// garbage, never out of bounds).
-__global__ __launch_bounds__(256) void rans_decode_kernel(
-    const uint8_t* __restrict__ coded, long coded_len, const long* __restrict__ offsets,
-    const uint32_t* __restrict__ states, const uint16_t* __restrict__ freq,
-    const uint16_t* __restrict__ cum, uint8_t* __restrict__ sym, long ctx_len, int spc) {
-  __shared__ uint16_t sf[256], sc[256];
-  __shared__ uint8_t slot2sym[RANS_M];
-  const int ctx = blockIdx.y;
-  {
-    const uint32_t f = freq[ctx * 256 + threadIdx.x], c = cum[ctx * 256 + threadIdx.x];
-    sf[threadIdx.x] = (uint16_t)f;
-    sc[threadIdx.x] = (uint16_t)c;
-    for (uint32_t i = c; i < c + f && i < RANS_M; ++i) slot2sym[i] = (uint8_t)threadIdx.x;
+                                                        const uint32_t* __restrict__ group_bytes,
+                                                        uint8_t* __restrict__ out, int slot, const int* __restrict__ err,
+                                                        int n_ctx, long* __restrict__ meta) {
+  __shared__ long part[4];
+  __shared__ int at[64], len[64];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, group = blockIdx.x;
+  long sum = 0;
+  for (int i = t; i < group; i += 256) sum += group_bytes[i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if (lane == 0) part[wave] = sum;
+  if (wave == 0) {
+    const int n = sizes[(long)group * 64 + lane];
+    at[lane] = wave_before(n);
+    len[lane] = n;
   }
   __syncthreads();
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  const long gs = (long)ctx * spc + j;
-  uint8_t* out = sym + (long)ctx * ctx_len + j;
-  const int len = (int)(ctx_len / spc);
-  long rp = offsets[gs];
-  uint32_t x = states[gs];
-  for (int k = 0; k < len; ++k) {
-    const uint32_t slot = x & (RANS_M - 1);
-    const uint32_t s = slot2sym[slot];
-    out[(long)k * spc] = (uint8_t)s;
-    x = (uint32_t)sf[s] * (x >> RANS_BITS) + slot - sc[s];
-    while (x < RANS_LOW) {
-      const uint32_t b = (rp >= 0 && rp < coded_len) ? coded[rp] : 0u;
-      ++rp;
-      x = (x << 8) | b;
+  const long base = part[0] + part[1] + part[2] + part[3];
+#pragma unroll 8
+  for (int i = 0; i < 16; ++i) {
+    const int s = wave * 16 + i, n = len[s];
+    const uint8_t* src = scratch + ((long)group * 64 + s) * slot + (slot - n);
+    uint8_t* dst = out + base + at[s];
+    uint8_t v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = lane + 64 * q < n ? src[lane + 64 * q] : 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (lane + 64 * q < n) dst[lane + 64 * q] = v[q];
+    for (int q = lane + 256; q < n; q += 64) dst[q] = src[q];
+  }
+  if (group == (int)gridDim.x - 1) {
+    int bad = 0;
+    for (int i = t; i < n_ctx; i += 256) bad += err[i];
+    bad = __syncthreads_count(bad != 0);
+    if (t == 0) {
+      meta[0] = base + group_bytes[group];
+      meta[1] = bad;
     }
   }
+}
+
+// grid n_ctx, block 1024: a context's 4096 decoder entries, symbol | (freq - 1) << 8 | (slot - cum) << 20, and the bytes of its
+// streams.  (A damaged table gives entries of some symbol; every field is masked to its width.)
+__global__ __launch_bounds__(1024) void rans_decode_tables_kernel(const uint16_t* __restrict__ freq, uint32_t* __restrict__ table,
+                                                                  const uint16_t* __restrict__ sizes, int spc,
+                                                                  long* __restrict__ ctx_bytes) {
+  __shared__ uint32_t cum[256], fr[256];
+  __shared__ long part[16];
+  const int t = threadIdx.x;
+  uint32_t f = 0;
+  if (t < 256) {
+    f = freq[blockIdx.x * 256 + t];
+    fr[t] = f;
+  }
+  long sum = 0;
+  for (int i = t; i < spc; i += 1024) sum += sizes[(long)blockIdx.x * spc + i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if ((t & 63) == 0) part[t >> 6] = sum;
+  const int before = wave_before((int)f);  // (of the wave's 64 symbols)
+  if (t < 256) cum[t] = before;
+  __syncthreads();
+  if (t == 0) {
+    long s = 0;
+    for (int w = 0; w < 16; ++w) s += part[w];
+    ctx_bytes[blockIdx.x] = s;
+  }
+  if (t < 256) {
+    uint32_t c = cum[t];
+    for (int w = 0; w < (t >> 6); ++w) c += cum[w * 64 + 63] + fr[w * 64 + 63];
+    f = c;
+  }
+  __syncthreads();
+  if (t < 256) cum[t] = f;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t slot = t + 1024 * i;
+    int s = 0;  // the last symbol that starts at or before the slot (those before it with the same start do not occur)
+#pragma unroll
+    for (int step = 128; step > 0; step >>= 1)
+      if (cum[s + step] <= slot) s += step;
+    table[blockIdx.x * (long)RANS_M + slot] = (uint32_t)s | ((fr[s] - 1) & 0xfff) << 8 | ((slot - cum[s]) & 0xfff) << 20;
+  }
+}
+
+// A stream's symbols; `word` reads words i and i + 1 of the wave's coded bytes, from LDS or (streams too long for it) from memory.
+// Two copies of the loop: one that may load from memory waits for its own stores at every step.  The words around the next
+// byte are read in the same wait as the state's table entry.
+template <typename F>
+__device__ __forceinline__ void rans_decode_stream(F word, uint32_t rp, uint32_t x, const uint32_t* tab,
+                                                   uint8_t* __restrict__ out, int len, int spc) {
+  for (int k = 0; k < len; ++k) {
+    const uint32_t e = tab[x & (RANS_M - 1)];
+    const uint64_t w = word(rp >> 2);
+    const uint32_t lo = (uint32_t)w, hi = (uint32_t)(w >> 32);
+    *out = (uint8_t)e;
+    out += spc;
+    const uint32_t q = x >> RANS_BITS;  // 20 bits (19 of a state the encoder leaves)
+    x = __umul24((e >> 8) & 0xfff, q) + (q + (e >> 20));
+    const uint32_t b = __builtin_amdgcn_alignbyte(hi, lo, rp & 3);  // the next byte lowest
+    const uint32_t x1 = (x << 8) | (b & 0xff), x2 = (x1 << 8) | ((b >> 8) & 0xff);
+    const bool one = x < RANS_LOW, two = x < (RANS_LOW >> 8);
+    x = two ? x2 : one ? x1 : x;
+    rp += one + two;
+  }
+}
+
+// grid (spc / 64, n_ctx), block 64.  The wave's coded bytes lie side by side, behind those of the contexts and of the context's
+// streams before it; they are staged when they fit (a stream's share of LDS_WORDS is 320 bytes, a symbol rarely takes one).
+// coded_len bounds every read (a damaged blob decodes to garbage, never out of bounds), and a step takes at most two bytes
+// whatever the state is.
+__global__ __launch_bounds__(64) void rans_decode_kernel(const uint8_t* __restrict__ coded, long coded_len,
+                                                         const long* __restrict__ ctx_bytes, const uint16_t* __restrict__ sizes,
+                                                         const uint32_t* __restrict__ states, const uint32_t* __restrict__ table,
+                                                         uint8_t* __restrict__ sym, long ctx_len, int spc) {
+  constexpr int LDS_WORDS = 64 * 80;
+  __shared__ __attribute__((aligned(16))) uint32_t tab[RANS_M];
+  __shared__ uint32_t bytes[LDS_WORDS];
+  const int ctx = blockIdx.y, t = threadIdx.x;
+  const u32x4* tp = reinterpret_cast<const u32x4*>(table + (long)ctx * RANS_M);
+#pragma unroll
+  for (int i = 0; i < RANS_M / 256; ++i) reinterpret_cast<u32x4*>(tab)[t + 64 * i] = tp[t + 64 * i];
+  const uint16_t* sz = sizes + (long)ctx * spc;
+  long first = 0;  // byte of the wave's first stream
+  for (int i = t; i < ctx; i += 64) first += ctx_bytes[i];
+  for (int i = t; i < (int)blockIdx.x * 64; i += 64) first += sz[i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
+  const int n = sz[blockIdx.x * 64 + t], before = wave_before(n), all = __shfl(before + n, 63, 64);
+  const uint32_t x = states[(long)ctx * spc + blockIdx.x * 64 + t];
+  // words of the coded bytes, counted from the aligned word that holds byte 0
+  const int lead = (int)((uintptr_t)coded & 3);
+  const uint32_t* cw = reinterpret_cast<const uint32_t*>(coded - lead);
+  const long n_words = (coded_len + lead + 3) >> 2;
+  const long w0 = (first + lead) >> 2, w1 = min((first + all + lead + 3) >> 2, n_words);
+  const bool staged = w1 - w0 < LDS_WORDS;
+  const int held = staged ? max((int)(w1 - w0), 0) : 0;
+#pragma unroll 8
+  for (int i = t; i < held; i += 64) bytes[i] = cw[w0 + i];
+  __syncthreads();
+  uint8_t* out = sym + (long)ctx * ctx_len + blockIdx.x * 64 + t;
+  const int len = (int)(ctx_len / spc);
+  const uint32_t rp = (uint32_t)((first + lead) & 3) + (uint32_t)before;
+  if (staged)
+    rans_decode_stream([&](uint32_t i) {
+      const uint32_t at = min(i, (uint32_t)LDS_WORDS - 2);
+      return (uint64_t)bytes[at + 1] << 32 | bytes[at];
+    }, rp, x, tab, out, len, spc);
+  else
+    rans_decode_stream([&](uint32_t i) {
+      const uint32_t lo = w0 + i < n_words ? cw[w0 + i] : 0u, hi = w0 + i + 1 < n_words ? cw[w0 + i + 1] : 0u;
+      return (uint64_t)hi << 32 | lo;
+    }, rp, x, tab, out, len, spc);
 }
 
 static bool rans_shape_ok(long n, int n_ctx, int spc) {
@@ -187,64 +394,53 @@ static bool rans_shape_ok(long n, int n_ctx, int spc) {
   return len >= 1 && 2 * len <= 65535;
 }
 
-// Pass 1: histogram -> table -> per-stream coding into scratch.  hist [n_ctx * 256] u32 must be
-// zero; scratch holds n_ctx * spc slots of 2 * (ctx_len / spc) bytes.
-VPSA_EXPORT int vpsa_rans_encode(const void* sym, long n, int n_ctx, int spc, void* hist, void* freq,
-                                 void* cum, void* scratch, void* states, void* sizes, int* err,
-                                 hipStream_t stream) {
+static int rans_slot(long n, int n_ctx, int spc) { return (int)((2 * (n / n_ctx / spc) + 3) & ~3L); }
+
+// Bytes of the encoder's workspace (0: the shape is not taken): histograms | table | errors | bytes per 64 streams | slots.
+VPSA_EXPORT long vpsa_rans_workspace(long n, int n_ctx, int spc) {
+  if (!rans_shape_ok(n, n_ctx, spc)) return 0;
+  return (long)n_ctx * (RANS_HIST_BLOCKS * 1024 + 4096 + 16) + (long)n_ctx * spc * (4 + rans_slot(n, n_ctx, spc));
+}
+
+// Histogram -> table -> per-stream coding -> dense bytes.  freq u16 [n_ctx * 256], states u32 and sizes u16 [n_ctx * spc], coded
+// with room for 2 n bytes, meta i64 [2] = coded bytes, contexts that could not be normalised; ws 16-byte aligned.
+VPSA_EXPORT int vpsa_rans_encode(const void* sym, long n, int n_ctx, int spc, void* ws, void* freq, void* states, void* sizes,
+                                 void* coded, long* meta, hipStream_t stream) {
   if (!rans_shape_ok(n, n_ctx, spc)) return -1;
-  const long ctx_len = n / n_ctx;
-  const int cap = (int)(2 * (ctx_len / spc));
-  int hb = (int)((ctx_len / 4 + 255) / 256);
-  if (hb > 64) hb = 64;
-  hipLaunchKernelGGL(rans_hist_kernel, dim3(hb, n_ctx), dim3(256), 0, stream, (const uint8_t*)sym,
-                     (uint32_t*)hist, ctx_len);
-  hipLaunchKernelGGL(rans_normalize_kernel, dim3(n_ctx), dim3(256), 0, stream, (const uint32_t*)hist,
-                     (uint16_t*)freq, (uint16_t*)cum, ctx_len, err);
-  hipLaunchKernelGGL(rans_encode_kernel, dim3(spc / 256, n_ctx), dim3(256), 0, stream,
-                     (const uint8_t*)sym, (const uint16_t*)freq, (const uint16_t*)cum,
-                     (uint8_t*)scratch, (uint32_t*)states, (uint16_t*)sizes, ctx_len, spc, cap);
+  const long ctx_len = n / n_ctx, groups = (long)n_ctx * spc / 64;
+  const int slot = rans_slot(n, n_ctx, spc);
+  const long per_block = (ctx_len / 4 + 255) / 256;
+  const int hb = (int)(per_block > RANS_HIST_BLOCKS ? RANS_HIST_BLOCKS : per_block);
+  uint32_t* part = (uint32_t*)ws;
+  u32x4* table = (u32x4*)((char*)ws + (long)n_ctx * RANS_HIST_BLOCKS * 1024);
+  int* err = (int*)(table + (long)n_ctx * 256);
+  uint32_t* group_bytes = (uint32_t*)((char*)err + (long)n_ctx * 16);
+  uint8_t* scratch = (uint8_t*)(group_bytes + (long)n_ctx * spc);
+  hipLaunchKernelGGL(rans_hist_kernel, dim3(hb, n_ctx), dim3(256), 0, stream, (const uint8_t*)sym, part, ctx_len);
+  hipLaunchKernelGGL(rans_normalize_kernel, dim3(n_ctx), dim3(256), 0, stream, part, hb, (uint16_t*)freq, table, ctx_len, err);
+  hipLaunchKernelGGL(rans_encode_kernel, dim3(spc / 64, n_ctx), dim3(64), 0, stream, (const uint8_t*)sym, table, scratch,
+                     (uint32_t*)states, (uint16_t*)sizes, group_bytes, ctx_len, spc, slot);
+  hipLaunchKernelGGL(rans_pack_kernel, dim3((unsigned)groups), dim3(256), 0, stream, scratch, (const uint16_t*)sizes, group_bytes,
+                     (uint8_t*)coded, slot, err, n_ctx, meta);
   return 0;
 }
 
-// Pass 2: offsets = exclusive prefix sum of sizes (computed by the caller).
-VPSA_EXPORT int vpsa_rans_pack(const void* scratch, const void* sizes, const long* offsets, void* out,
-                               long n, int n_ctx, int spc, hipStream_t stream) {
-  if (!rans_shape_ok(n, n_ctx, spc)) return -1;
-  const long n_streams = (long)n_ctx * spc;
-  const int cap = (int)(2 * (n / n_ctx / spc));
-  hipLaunchKernelGGL(rans_pack_kernel, dim3((unsigned)((n_streams + 255) / 256)), dim3(256), 0, stream,
-                     (const uint8_t*)scratch, (const uint16_t*)sizes, offsets, (uint8_t*)out,
-                     n_streams, cap);
-  return 0;
+// Bytes of the decoder's workspace: tables | bytes per context.
+VPSA_EXPORT long vpsa_rans_decode_workspace(long n, int n_ctx, int spc) {
+  if (!rans_shape_ok(n, n_ctx, spc)) return 0;
+  return (long)n_ctx * (RANS_M * 4 + 8);
 }
 
-// cum is recomputed here from freq (only freq travels in the blob); cum_ws [n_ctx * 256] u16.
-__global__ __launch_bounds__(256) void rans_cum_kernel(const uint16_t* __restrict__ freq,
-                                                       uint16_t* __restrict__ cum) {
-  __shared__ int scan[256];
-  const int t = threadIdx.x;
-  const int f = freq[blockIdx.x * 256 + t];
-  scan[t] = f;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const int v = t >= off ? scan[t - off] : 0;
-    __syncthreads();
-    scan[t] += v;
-    __syncthreads();
-  }
-  cum[blockIdx.x * 256 + t] = (uint16_t)(scan[t] - f);
-}
-
-VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const long* offsets,
-                                 const void* states, const void* freq, void* cum_ws, void* sym, long n,
-                                 int n_ctx, int spc, hipStream_t stream) {
+// Only freq, states and sizes travel beside the coded bytes; ws 16-byte aligned.
+VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* states, const void* freq, const void* sizes,
+                                 void* ws, void* sym, long n, int n_ctx, int spc, hipStream_t stream) {
   if (!rans_shape_ok(n, n_ctx, spc)) return -1;
   const long ctx_len = n / n_ctx;
-  hipLaunchKernelGGL(rans_cum_kernel, dim3(n_ctx), dim3(256), 0, stream, (const uint16_t*)freq,
-                     (uint16_t*)cum_ws);
-  hipLaunchKernelGGL(rans_decode_kernel, dim3(spc / 256, n_ctx), dim3(256), 0, stream,
-                     (const uint8_t*)coded, coded_len, offsets, (const uint32_t*)states,
-                     (const uint16_t*)freq, (const uint16_t*)cum_ws, (uint8_t*)sym, ctx_len, spc);
+  uint32_t* table = (uint32_t*)ws;
+  long* ctx_bytes = (long*)(table + (long)n_ctx * RANS_M);
+  hipLaunchKernelGGL(rans_decode_tables_kernel, dim3(n_ctx), dim3(1024), 0, stream, (const uint16_t*)freq, table,
+                     (const uint16_t*)sizes, spc, ctx_bytes);
+  hipLaunchKernelGGL(rans_decode_kernel, dim3(spc / 64, n_ctx), dim3(64), 0, stream, (const uint8_t*)coded, coded_len, ctx_bytes,
+                     (const uint16_t*)sizes, (const uint32_t*)states, table, (uint8_t*)sym, ctx_len, spc);
   return 0;
 }

@@ -705,6 +705,26 @@ def test_rans_gpu_matches_numpy_definition_bit_for_bit(n_ctx, spc, per_stream):
     assert junk.shape == sym.shape
 
 
+@pytest.mark.parametrize("spc,per_stream,skip", [(256, 1, 0), (256, 3, 4), (512, 257, 8), (256, 516, 1)])
+def test_rans_remainders_of_tiles_and_batches(spc, per_stream, skip):
+    """Streams of a symbol, of less than a batch, of one more than a tile of 256 and of two tiles and a word; symbols that do not
+    start on the wide loads' boundaries."""
+    import numpy as np
+
+    g = torch.Generator().manual_seed(per_stream)
+    n_ctx, n = 2, 2 * spc * per_stream
+    sym = torch.randint(-60, 60, (n,), generator=g).to(torch.int8)
+    dev = torch.zeros(n + skip, dtype=torch.int8, device=DEV)[skip:]
+    dev.copy_(sym)
+    f_ref, st_ref, sz_ref, co_ref = ref.rans_encode(sym.numpy(), n_ctx, spc)
+    freq, states, sizes, coded = ops.rans_encode(dev, n_ctx, spc)
+    assert np.array_equal(states.cpu().numpy().view(np.uint32), st_ref) and np.array_equal(coded.cpu().numpy(), co_ref)
+    assert np.array_equal(sizes.cpu().numpy().view(np.uint16), sz_ref)
+    odd = torch.zeros(coded.numel() + 3, dtype=torch.uint8, device=DEV)[3:]  # coded bytes at an odd address
+    odd.copy_(coded)
+    assert torch.equal(ops.rans_decode(freq, states, sizes, odd, n, n_ctx, spc).cpu(), sym)
+
+
 def test_cachegen_page_on_gpu_uses_the_rans_stage_and_matches_the_host_coder(monkeypatch):
     from vllm_production_stack_amd.kv.serde import SERDE_CACHEGEN_RANS, PageSerde, _HDR
 

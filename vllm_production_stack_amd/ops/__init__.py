@@ -33,7 +33,7 @@ def _kernels():
             "vpsa_moe_topk_softmax", "vpsa_moe_align", "vpsa_moe_permute", "vpsa_moe_combine",
             "vpsa_moe_gemv", "vpsa_moe_mfma", "vpsa_lora_shrink", "vpsa_lora_expand",
             "vpsa_skinny_gemm", "vpsa_hbm_read_probe", "vpsa_set_gemm_variant", "vpsa_stream_gemm",
-            "vpsa_stream_gemm_splits", "vpsa_set_stream_targets", "vpsa_rans_encode", "vpsa_rans_pack",
+            "vpsa_stream_gemm_splits", "vpsa_set_stream_targets", "vpsa_rans_encode",
             "vpsa_rans_decode", "vpsa_sample", "vpsa_grouped_gemm", "vpsa_packed_gemm",
             "vpsa_packed_gemm_splits", "vpsa_set_packed_target", "vpsa_dense_decode_attention", "vpsa_dense_attention",
             "vpsa_tile_gemm", "vpsa_tile_gemm_debug", "vpsa_paged_prefill_split",
@@ -48,7 +48,8 @@ def _kernels():
             "vpsa_embed_rmsnorm", "vpsa_depth_mix_rmsnorm", "vpsa_poly_norm", "vpsa_soft_cap", "vpsa_mingru",
         ):
             getattr(lib, name).restype = c_int
-        lib.vpsa_prefill_split_record_bytes.restype = c_long
+        for name in ("vpsa_prefill_split_record_bytes", "vpsa_rans_workspace", "vpsa_rans_decode_workspace"):
+            getattr(lib, name).restype = c_long
         if os.environ.get("VPSA_PREFILL_VARIANT"):  # pin one prefill kernel for A/B runs
             lib.vpsa_set_prefill_variant(c_int(int(os.environ["VPSA_PREFILL_VARIANT"])))
         _lib = lib
@@ -951,13 +952,16 @@ def kv_scatter_pages(staging, page_ids, pool):
     _check(rc, "kv_scatter_pages")
 
 
-def cachegen_encode(staging, levels, unit_elems, n_layers):
-    """bf16 staging -> (int8 symbols, fp32 group scales).  ``levels``: int32 tensor [n_layers]."""
+def cachegen_encode(staging, levels, unit_elems, n_layers, scales=None):
+    """bf16 staging -> (int8 symbols, fp32 group scales, in ``scales`` where given).  ``levels``: int32 tensor [n_layers]."""
     if not staging.is_cuda:
-        return reference.cachegen_encode(staging, levels.tolist(), unit_elems, n_layers)
+        sym, sc = reference.cachegen_encode(staging, levels.tolist(), unit_elems, n_layers)
+        return sym, sc if scales is None else scales.copy_(sc)
     n = staging.numel()
     sym = torch.empty((n,), dtype=torch.int8, device=staging.device)
-    scales = torch.empty((n // 64,), dtype=torch.float32, device=staging.device)
+    if scales is None:
+        scales = torch.empty((n // 64,), dtype=torch.float32, device=staging.device)
+    assert scales.dtype == torch.float32 and scales.is_contiguous() and scales.numel() == n // 64
     assert levels.dtype == torch.int32 and levels.is_cuda
     rc = _kernels().vpsa_cachegen_encode(_p(staging), _p(sym), _p(scales), _p(levels), c_long(n),
                                          c_long(unit_elems), c_int(n_layers), _stream())
@@ -997,31 +1001,36 @@ def rans_encode(sym, n_ctx, spc=RANS_SPC):
         return (torch.from_numpy(f.view(np.int16).reshape(-1).copy()), torch.from_numpy(st.view(np.int32).copy()),
                 torch.from_numpy(sz.view(np.int16).copy()), torch.from_numpy(co.copy()))
     sym = sym.contiguous().view(torch.uint8).view(-1)
+    if sym.data_ptr() % 4:  # (a slice at an odd offset: the histogram reads words)
+        sym = sym.clone()
     n, dev = sym.numel(), sym.device
     n_streams = n_ctx * spc
     if n % n_ctx or (n // n_ctx) % spc:
         raise ValueError("rans_encode: symbols do not divide into contexts / streams")
-    cap = 2 * (n // n_ctx // spc)
-    hist = torch.zeros(n_ctx * 256, dtype=torch.int32, device=dev)
     freq = torch.empty(n_ctx * 256, dtype=torch.int16, device=dev)
-    cum = torch.empty(n_ctx * 256, dtype=torch.int16, device=dev)
-    scratch = torch.empty(n_streams * cap, dtype=torch.uint8, device=dev)
     states = torch.empty(n_streams, dtype=torch.int32, device=dev)
     sizes = torch.empty(n_streams, dtype=torch.int16, device=dev)
-    err = torch.zeros(1, dtype=torch.int32, device=dev)
-    lib = _kernels()
-    _check(lib.vpsa_rans_encode(_p(sym), c_long(n), c_int(n_ctx), c_int(spc), _p(hist), _p(freq), _p(cum),
-                                _p(scratch), _p(states), _p(sizes), _p(err), _stream()), "rans_encode")
-    sz64 = sizes.to(torch.int64)
-    ends = torch.cumsum(sz64, 0)
-    offsets = ends - sz64
-    total, bad = torch.stack([ends[-1], err[0].to(torch.int64)]).tolist()  # one synchronisation
+    coded = torch.empty(2 * n, dtype=torch.uint8, device=dev)
+    total, bad = rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc).tolist()  # one synchronisation
     if bad:
         raise RuntimeError("rans_encode: frequency table could not be normalised")
-    coded = torch.empty(int(total), dtype=torch.uint8, device=dev)
-    _check(lib.vpsa_rans_pack(_p(scratch), _p(sizes), _p(offsets), _p(coded), c_long(n), c_int(n_ctx),
-                              c_int(spc), _stream()), "rans_pack")
-    return freq, states, sizes, coded
+    return freq, states, sizes, coded[:total].clone()
+
+
+def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC):
+    """``rans_encode`` on the device into the caller's tensors (``coded`` with room for two bytes a symbol), without a
+    synchronisation -> int64 [2] on the device: coded bytes, and contexts whose table could not be normalised (nothing of
+    the result is valid unless 0)."""
+    n, dev, lib = sym.numel(), sym.device, _kernels()
+    n_streams = n_ctx * spc
+    assert sym.is_cuda and sym.is_contiguous() and sym.element_size() == 1 and sym.data_ptr() % 4 == 0
+    assert all(t.is_contiguous() and t.numel() * t.element_size() >= b for t, b in (
+        (freq, 512 * n_ctx), (states, 4 * n_streams), (sizes, 2 * n_streams), (coded, 2 * n)))
+    ws = torch.empty(max(1, int(lib.vpsa_rans_workspace(c_long(n), c_int(n_ctx), c_int(spc)))), dtype=torch.uint8, device=dev)
+    meta = torch.empty(2, dtype=torch.int64, device=dev)
+    _check(lib.vpsa_rans_encode(_p(sym), c_long(n), c_int(n_ctx), c_int(spc), _p(ws), _p(freq), _p(states), _p(sizes), _p(coded),
+                                _p(meta), _stream()), "rans_encode")
+    return meta
 
 
 def rans_decode(freq, states, sizes, coded, n, n_ctx, spc=RANS_SPC):
@@ -1033,13 +1042,12 @@ def rans_decode(freq, states, sizes, coded, n, n_ctx, spc=RANS_SPC):
                                     sizes.numpy().view(np.uint16), coded.numpy(), n, n_ctx, spc)
         return torch.from_numpy(out.view(np.int8).copy())
     dev = coded.device
-    sz64 = sizes.to(torch.int64)
-    offsets = torch.cumsum(sz64, 0) - sz64
-    cum = torch.empty(n_ctx * 256, dtype=torch.int16, device=dev)
+    lib = _kernels()
+    assert coded.is_contiguous() and freq.numel() >= n_ctx * 256 and min(states.numel(), sizes.numel()) >= n_ctx * spc
+    ws = torch.empty(max(1, int(lib.vpsa_rans_decode_workspace(c_long(n), c_int(n_ctx), c_int(spc)))), dtype=torch.uint8, device=dev)
     sym = torch.empty(n, dtype=torch.int8, device=dev)
-    _check(_kernels().vpsa_rans_decode(_p(coded), c_long(coded.numel()), _p(offsets), _p(states), _p(freq),
-                                       _p(cum), _p(sym), c_long(n), c_int(n_ctx), c_int(spc), _stream()),
-           "rans_decode")
+    _check(lib.vpsa_rans_decode(_p(coded), c_long(coded.numel()), _p(states), _p(freq), _p(sizes), _p(ws), _p(sym), c_long(n),
+                                c_int(n_ctx), c_int(spc), _stream()), "rans_decode")
     return sym
 
 
