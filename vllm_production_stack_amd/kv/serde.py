@@ -22,6 +22,7 @@ from __future__ import annotations
 import ctypes
 import os
 import struct
+import threading
 
 import numpy as np
 import torch
@@ -87,6 +88,12 @@ class PageSerde:
         self.unit_elems = n_kv * ops.PAGE * head_dim
         self.levels = levels or default_levels(n_layers)
         self._levels_dev: dict = {}
+        # Pinned buffers that pages pass through on their way between host and device, each with the event of the copy that
+        # last read it: a pageable copy of a page's 3.5 MB takes 0.65 ms to the host and 0.13 ms to the device, a pinned one
+        # 0.07.  One for encoding; two for decoding, so that a page is copied in while the one before is on its way.
+        self._out_lock, self._in_lock = threading.Lock(), threading.Lock()
+        self._out_buf: torch.Tensor | None = None
+        self._in_bufs: list = [[None, None], [None, None]]
 
     def _header(self, payload_len: int) -> bytes:
         return _HDR.pack(MAGIC, 1, self.kind, self.n_layers, self.n_kv, self.head_dim, ops.PAGE,
@@ -100,6 +107,10 @@ class PageSerde:
             raw = flat.contiguous().cpu().view(torch.uint8).numpy().tobytes()
             return _HDR.pack(MAGIC, 1, SERDE_NAIVE, self.n_layers, self.n_kv, self.head_dim, ops.PAGE,
                              len(raw)) + raw
+        if self._rans_ok(flat.device):
+            with self._out_lock:
+                payload = self._rans_page(flat)
+                return b"".join((self._rans_header(payload.size), memoryview(payload)))
         sym_np, sc_np = self.quantize(flat)
         return self.pack(sym_np, sc_np)
 
@@ -112,14 +123,39 @@ class PageSerde:
         rANS entropy stage, one device-to-host copy of the finished payload -> (payload, None).
         Otherwise the int8 symbols and fp32 scales come back for the host range coder
         -> (symbols, scales)."""
-        lv = self._levels_dev.get(flat.device)
-        if lv is None:
-            lv = torch.tensor(self.levels, dtype=torch.int32, device=flat.device)
-            self._levels_dev[flat.device] = lv
-        sym, scales = ops.cachegen_encode(flat.contiguous(), lv, self.unit_elems, self.n_layers)
         if self._rans_ok(flat.device):
-            return self.rans_payload(sym, scales), None
+            with self._out_lock:
+                return self._rans_page(flat).copy(), None
+        sym, scales = ops.cachegen_encode(flat.contiguous(), self._levels(flat.device), self.unit_elems, self.n_layers)
         return sym.cpu().numpy(), scales.float().cpu().numpy()
+
+    def _levels(self, device) -> torch.Tensor:
+        lv = self._levels_dev.get(device)
+        if lv is None:
+            lv = self._levels_dev[device] = torch.tensor(self.levels, dtype=torch.int32, device=device)
+        return lv
+
+    def _rans_page(self, flat: torch.Tensor) -> np.ndarray:
+        """The kind-2 payload of a page, in the pinned buffer (valid until the lock is given up).  Every stage writes its part
+        of the payload where it belongs; one copy brings the finished payload over."""
+        n, dev, n_streams = flat.numel(), flat.device, self.n_layers * ops.RANS_SPC
+        a = _RANS_HDR.size
+        o = np.cumsum([0, 4 * (n // 64), 512 * self.n_layers, 4 * n_streams, 2 * n_streams]).tolist()
+        body = torch.empty(o[4] + 2 * n, dtype=torch.uint8, device=dev)
+        sym, _ = ops.cachegen_encode(flat.contiguous(), self._levels(dev), self.unit_elems, self.n_layers,
+                                     scales=body[:o[1]].view(torch.float32))
+        total, bad = ops.rans_encode_into(sym.view(-1), self.n_layers, body[o[1]:o[2]], body[o[2]:o[3]], body[o[3]:o[4]],
+                                          body[o[4]:]).tolist()
+        if bad:
+            raise RuntimeError("rans_encode: frequency table could not be normalised")
+        size = a + o[4] + total
+        if self._out_buf is None or self._out_buf.numel() < size:
+            self._out_buf = torch.empty(size + size // 8, dtype=torch.uint8, pin_memory=True)
+        self._out_buf[a:size].copy_(body[:o[4] + total], non_blocking=True)
+        torch.cuda.current_stream(dev).synchronize()
+        payload = self._out_buf.numpy()[:size]
+        payload[:a] = np.frombuffer(_RANS_HDR.pack(ops.RANS_SPC, n_streams, total), dtype=np.uint8)
+        return payload
 
     def rans_payload(self, sym: torch.Tensor, scales: torch.Tensor) -> np.ndarray:
         """Entropy-code quantised symbols where they are and return the kind-2 payload bytes."""
@@ -129,12 +165,14 @@ class PageSerde:
         head = _RANS_HDR.pack(ops.RANS_SPC, states.numel(), coded.numel())
         return np.concatenate([np.frombuffer(head, dtype=np.uint8), body.cpu().numpy()])
 
+    def _rans_header(self, payload_len: int) -> bytes:
+        return _HDR.pack(MAGIC, 1, SERDE_CACHEGEN_RANS, self.n_layers, self.n_kv, self.head_dim, ops.PAGE, payload_len)
+
     def pack(self, sym_np: np.ndarray, sc_np: np.ndarray | None) -> bytes:
         """Host half: frame a finished rANS payload, or range-code the symbols (releases the
         GIL: safe to run on worker threads)."""
         if sc_np is None:
-            return _HDR.pack(MAGIC, 1, SERDE_CACHEGEN_RANS, self.n_layers, self.n_kv, self.head_dim,
-                             ops.PAGE, sym_np.size) + sym_np.tobytes()
+            return b"".join((self._rans_header(sym_np.size), memoryview(np.ascontiguousarray(sym_np)).cast("B")))
         coded = rc_encode(sym_np, 2 * self.unit_elems, self.n_layers)
         payload = sc_np.tobytes() + struct.pack("<Q", len(coded)) + coded
         return self._header(len(payload)) + payload
@@ -190,7 +228,7 @@ class PageSerde:
         cuts = np.cumsum([a, 4 * n_groups, 2 * 256 * self.n_layers, 4 * n_streams, 2 * n_streams, coded_len])
         if n_streams != self.n_layers * spc or cuts[-1] > payload.size:
             raise ValueError("damaged cachegen payload")
-        body = torch.from_numpy(payload[a:cuts[-1]].copy()).to(device)
+        body = self._to_device(payload[a:cuts[-1]], device)
         o = cuts - a
         scales = body[o[0]:o[1]].view(torch.float32)
         freq = body[o[1]:o[2]].view(torch.int16)
@@ -199,6 +237,24 @@ class PageSerde:
         coded = body[o[4]:o[5]]
         sym = ops.rans_decode(freq, states, sizes, coded, self.page_elems, self.n_layers, spc)
         return ops.cachegen_decode(sym, scales, self.unit_elems)
+
+    def _to_device(self, data: np.ndarray, device) -> torch.Tensor:
+        """Host bytes on ``device``, through the next pinned buffer on a GPU (without waiting for the copy)."""
+        if torch.device(device).type != "cuda":
+            return torch.from_numpy(data.copy()).to(device)
+        with self._in_lock:
+            buf, read = slot = self._in_bufs[0]
+            self._in_bufs.reverse()
+            if read is not None:
+                read.synchronize()  # the copy that last read it has left
+            if buf is None or buf.numel() < data.size:
+                buf = slot[0] = torch.empty(data.size + data.size // 8, dtype=torch.uint8, pin_memory=True)
+            np.copyto(buf.numpy()[:data.size], data)
+            body = torch.empty(data.size, dtype=torch.uint8, device=device)
+            body.copy_(buf[:data.size], non_blocking=True)
+            slot[1] = torch.cuda.Event()
+            slot[1].record(torch.cuda.current_stream(body.device))
+        return body
 
     def restore(self, got: tuple, device) -> torch.Tensor:
         """Finish what ``unpack`` started (its "codec" and "rans" results)."""
