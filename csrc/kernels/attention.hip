@@ -2069,25 +2069,59 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
   }
 }
 
-// merge split partials: grid = (num_seqs, n_q), block = 128 (one channel per thread)
+// Merge split partials: grid (num_seqs, n_q), block 128 = four groups of 32 threads, a thread with four channels of every fourth
+// split.  A launch of a few hundred short workgroups is bound by dependent loads: eight partials of a thread are in flight at
+// once, before the maxima that weigh them are there (32 splits of one sequence: 11.6 -> 4.6 us; one channel per thread and one
+// split after the other before).
 __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restrict__ ws_o,
                                                             const float* __restrict__ ws_ml,
                                                             uint16_t* __restrict__ out,
                                                             long out_stride, int n_q,
                                                             int num_splits) {
-  const int seq = blockIdx.x, head = blockIdx.y, d = threadIdx.x;
+  __shared__ f32x4 half[32];
+  const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, g = tid >> 5, c4 = (tid & 31) * 4;
   const long base = ((long)seq * n_q + head) * num_splits;
-  float M = NEG_BIG;
-  for (int s = 0; s < num_splits; ++s) M = fmaxf(M, ws_ml[(base + s) * 2]);
-  float L = 0.f, acc = 0.f;
-  for (int s = 0; s < num_splits; ++s) {
-    const float f = __builtin_amdgcn_exp2f(ws_ml[(base + s) * 2] - M);
-    L += ws_ml[(base + s) * 2 + 1] * f;
-    acc += ws_o[(base + s) * HEAD_DIM + d] * f;
+  const float* po = ws_o + base * HEAD_DIM + c4;
+  const float* pm = ws_ml + base * 2;
+  f32x4 v[8];
+  float m[8];
+  auto fetch = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int s = min(s0 + 4 * i, num_splits - 1);
+      v[i] = *reinterpret_cast<const f32x4*>(po + (long)s * HEAD_DIM);
+      m[i] = pm[2 * s];
+    }
+  };
+  fetch(g);
+  float M = NEG_BIG, L = 0.f;
+  for (int s = lane; s < num_splits; s += 64) M = fmaxf(M, pm[2 * s]);
+  M = wave_reduce_max(M);
+  for (int s = lane; s < num_splits; s += 64) L += pm[2 * s + 1] * __builtin_amdgcn_exp2f(pm[2 * s] - M);
+  L = wave_reduce_sum(L);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = g; s0 < num_splits; s0 += 32) {
+    if (s0 != g) fetch(s0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (s0 + 4 * i < num_splits) acc += v[i] * __builtin_amdgcn_exp2f(m[i] - M);
   }
-  const float r = L > 0.f ? acc / L : 0.f;
-  bf16_t b = (bf16_t)r;
-  out[(long)seq * out_stride + head * HEAD_DIM + d] = __builtin_bit_cast(uint16_t, b);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] += __shfl_xor(acc[i], 32, 64);
+  if (tid >= 64 && tid < 96) half[tid - 64] = acc;
+  __syncthreads();
+  if (tid >= 32) return;
+  acc += half[tid];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = L > 0.f ? acc[i] / L : 0.f;
+  const u32x2 w = {pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+  uint16_t* o = out + (long)seq * out_stride + head * HEAD_DIM + c4;
+  if (((uintptr_t)o & 7) == 0) {
+    *reinterpret_cast<u32x2*>(o) = w;
+  } else {  // rows of a tensor that starts or steps off the eight-byte boundaries
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (uint16_t)(w[i >> 1] >> (16 * (i & 1)));
+  }
 }
 
 // 0 = one register set per wave, 1 = software-pipelined (two register sets), 2 = page-paired,

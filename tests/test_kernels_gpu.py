@@ -417,6 +417,23 @@ def test_paged_decode_matches_reference(n_q, n_kv, splits, variant):
     assert err < REL_TOL, err
 
 
+@pytest.mark.parametrize("splits,lead", [(2, 0), (31, 2), (32, 0), (33, 1), (70, 0)])
+def test_paged_decode_merges_any_number_of_splits(splits, lead):
+    """Partials of more splits than the merge holds at once, splits without keys, output rows off the wide stores' boundaries."""
+    torch.manual_seed(15)
+    n_q, n_kv, hd, ctx = 8, 2, 128, [1, 700, 4500]
+    pages = (max(ctx) + ops.PAGE - 1) // ops.PAGE
+    pool = _v_offset_pool(len(ctx) * pages, 1, n_kv, seed=16)
+    bt = _block_tables(len(ctx), pages, pool.shape[0], 17)
+    q = torch.randn(len(ctx), n_q * hd, device=DEV).to(BF)
+    ctx_t = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    out = torch.zeros(len(ctx), n_q * hd + lead, device=DEV, dtype=BF)[:, lead:]
+    out_ref = torch.zeros_like(q)
+    ops.paged_decode(q, out, pool, 0, bt, ctx_t, n_q, n_kv, hd, hd ** -0.5, num_splits=splits)
+    ref.paged_decode(q, out_ref, pool, 0, bt, ctx_t, n_q, n_kv, hd, hd ** -0.5)
+    assert _rel_row_err(out.contiguous(), out_ref, n_q) < REL_TOL
+
+
 @pytest.mark.parametrize("variant", [0, 2, 4, -1])
 def test_paged_decode_bench_shape(variant):
     """The decode step of the headline bench: 40 sequences of ~22k keys each, their 345 pages
