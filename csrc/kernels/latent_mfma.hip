@@ -30,6 +30,7 @@
 // (max = sink, sum = 1).  With key-range splits every split writes unnormalised partial outputs and
 // (max, sum) to a workspace and a merge kernel adds the sink and normalises.
 #include "common.h"
+#include <utility>
 
 namespace {
 
@@ -40,6 +41,8 @@ struct LatTile {
 };
 
 __device__ __forceinline__ u32x4 ld16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr float LOG2E = 1.4426950408889634f, LN2 = 0.6931471805599453f;
 
@@ -262,6 +265,289 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
   }
 }
 
+// The same walk for wide entries (RANK + ROT a multiple of 64, value accumulators of a wave in registers): pages go straight
+// into LDS, two of them, and the second product reads its transposed operand from the K image through the transposing LDS read.
+// What it replaces was bound by staging: a page passed through 128 registers into a K and a V^T image (137 KB of LDS writes with
+// 4 x 4 transposes) between two barriers, and a decode tile of 32 heads left two of the four waves idle meanwhile.
+//   * Image: 64 rows of ENTRY values without padding; a row's 16-byte chunk j lies at j ^ f(row), f = (row / 2 % 4) * 2 +
+//     row / 8 % 2 (applied to the source address: a wave's load fills 1 KiB of LDS in lane order).  The 16 rows of a K fragment
+//     then cover all banks, and so do the 8 rows x 32 bytes that half a wave reads transposed.
+//   * ds_read_b64_tr_b16 gives lane (c, g) the keys 4 g .. 4 g + 3 of channel c: the order in which the S accumulators hold them.
+//   * Two pages are on their way except while one is multiplied: the page after next is asked for as soon as its buffer is free,
+//     before the next one is waited for (a counted wait).  Waiting for each page before asking for another left 4.5 TB/s.
+//   * Decode rows of at most 32 heads (KSPLIT 4): eight waves, four of which share 16 slots and take 16 keys of every page each;
+//     their softmax states and outputs are merged through LDS at the end.  With 64 slots a tile keeps four waves busy by itself.
+//   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
+// Decode rows with their merge, in a graph: 32 sequences of 3.5k entries on average, 32 heads, 8 splits (137 MB) 70.5 -> 52.5 us, 8
+// of 26k entries 113 -> 76; a single sequence of 2k entries, a page per split, has nothing to overlap: 23.9 -> 26.7.  Prefill
+// tiles, 1500 rows of 16 heads behind 4500 entries: 854 -> 737.
+
+// o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
+// their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
+// channels a tile, keys 16 apart, eight tiles a block; 16 keys: one read a tile, sixteen tiles a block.
+template <int ROW, int J>
+__device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8& pf, const uint32_t (&at)[4]) {
+  u32x2 r[16];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %16 offset:%20\n\tds_read_b64_tr_b16 %1, %16 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %2, %17 offset:%20\n\tds_read_b64_tr_b16 %3, %17 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %4, %18 offset:%20\n\tds_read_b64_tr_b16 %5, %18 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %6, %19 offset:%20\n\tds_read_b64_tr_b16 %7, %19 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %8, %16 offset:%22\n\tds_read_b64_tr_b16 %9, %16 offset:%23\n\t"
+      "ds_read_b64_tr_b16 %10, %17 offset:%22\n\tds_read_b64_tr_b16 %11, %17 offset:%23\n\t"
+      "ds_read_b64_tr_b16 %12, %18 offset:%22\n\tds_read_b64_tr_b16 %13, %18 offset:%23\n\t"
+      "ds_read_b64_tr_b16 %14, %19 offset:%22\n\tds_read_b64_tr_b16 %15, %19 offset:%23\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7]), "=&v"(r[8]),
+        "=&v"(r[9]), "=&v"(r[10]), "=&v"(r[11]), "=&v"(r[12]), "=&v"(r[13]), "=&v"(r[14]), "=&v"(r[15])
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(J * 256), "n"(J * 256 + 16 * ROW), "n"(J * 256 + 128),
+        "n"(J * 256 + 128 + 16 * ROW)
+      : "memory");
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const u32x4 a = {r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]};
+    o[8 * J + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), pf, o[8 * J + i], 0, 0, 0);
+  }
+}
+
+template <int J>
+__device__ __forceinline__ void transposed_products16(f32x4* o, const s16x4& pf, const uint32_t (&at)[4]) {
+  u32x2 r[8];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8 offset:%12\n\tds_read_b64_tr_b16 %1, %9 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %2, %10 offset:%12\n\tds_read_b64_tr_b16 %3, %11 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:%13\n\tds_read_b64_tr_b16 %5, %9 offset:%13\n\t"
+      "ds_read_b64_tr_b16 %6, %10 offset:%13\n\tds_read_b64_tr_b16 %7, %11 offset:%13\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(J * 256), "n"(J * 256 + 128)
+      : "memory");
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    o[8 * J + i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, r[i]), pf, o[8 * J + i], 0, 0, 0);
+}
+
+template <int ROW, int... J>
+__device__ __forceinline__ void all_products(f32x4* o, const bf16x8& pf, const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
+  (transposed_products<ROW, J>(o, pf, at), ...);
+}
+template <int... J>
+__device__ __forceinline__ void all_products16(f32x4* o, const s16x4& pf, const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
+  (transposed_products16<J>(o, pf, at), ...);
+}
+
+template <int RANK, int ROT, int KSPLIT>
+__global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void latent_wide_kernel(
+    const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
+    long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
+    int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
+    const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
+    int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+  constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, DT = RANK / 16, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW;
+  static_assert(KSPLIT == 1 || KSPLIT == 4, "all keys or a quarter of them");
+  constexpr int WAVES = KSPLIT == 4 ? 8 : 4;
+  constexpr int NI = PAGE_BYTES / (1024 * WAVES);  // KiB of a page that a wave loads
+  constexpr int NT = 4 / KSPLIT;                   // 16-key tiles of a page that a wave takes
+  static_assert(ENTRY % 64 == 0 && DT % 8 == 0, "chunks are exchanged within groups of eight");
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15, g = lane >> 4;
+  const int sg = KSPLIT == 4 ? wave >> 2 : wave, kh = KSPLIT == 4 ? wave & 3 : 0;  // slots, keys
+  LatTile t;
+  if (tiles) {
+    const int* e = tiles + 6 * blockIdx.x;
+    t = {e[0], e[1], e[2], e[3], e[4], e[5]};
+  } else {
+    const int runs = (heads + 63) >> 6;
+    const int row = blockIdx.x / runs, h0 = (blockIdx.x % runs) << 6;
+    t = {row, row, 1, positions[row], h0, min(64, heads - h0)};
+  }
+  if (t.seq < 0) return;
+  const int slot = sg * 16 + c16;
+  const bool valid = slot < t.n_tok * t.hcount;
+  const bool wave_active = sg * 16 < t.n_tok * t.hcount;  // wave-uniform
+  const float scale2 = scale * LOG2E;
+  const int tok = valid ? slot / t.hcount : 0;
+  const int head = t.head0 + (valid ? slot % t.hcount : 0);
+  const long row = t.row0 + tok;
+  const int my_pos = valid ? t.pos0 + tok : -1;
+  const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
+  const int p_first = max(0, t.pos0 - window + 1) / PAGE;
+  const int per = (n_pages - p_first + splits - 1) / splits;
+  const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
+  const int my_first = my_pos - window;
+  const int* bt = block_tables + (long)t.seq * bt_stride;
+
+  int src_off[NI];  // bytes into a page of what this lane loads into byte (WAVES i + wave) * 1024 + lane * 16 of the image
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int o = (WAVES * i + wave) * 1024 + lane * 16, r = o / ROW, ch = (o % ROW) >> 4;
+    src_off[i] = r * ROW + ((ch ^ (((r >> 1) & 3) << 1 | ((r >> 3) & 1))) << 4);
+  }
+  auto load_page = [&](int p, int buf) {
+    const char* src = reinterpret_cast<const char*>(cache + (long)bt[p] * page_stride);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + src_off[i]),
+                                       (__attribute__((address_space(3))) void*)(lds + buf * PAGE_BYTES + (WAVES * i + wave) * 1024),
+                                       16, 0, KSPLIT == 4 ? 2 : 0);  // 2: non-temporal
+  };
+  if (p_begin < p_end) load_page(p_begin, 0);  // (the older loads: the loop counts the page behind them)
+
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {  // (a slot past the tile reads the tile's first query: no branches between the loads)
+    const int d = 32 * ks + 8 * g;
+    const u32x4 v = 32 * ks < RANK ? ld16(q_lat + row * ql_row + head * ql_head + d) : ld16(q_rot + row * qr_row + head * qr_head + (d - RANK));
+    qf[ks] = __builtin_bit_cast(bf16x8, valid ? v : (u32x4){0u, 0u, 0u, 0u});
+  }
+  const bool seeded = splits == 1 && sink != nullptr && valid && kh == 0;
+  float m = seeded ? sink[head] * LOG2E : -INFINITY;
+  float l = seeded ? 1.f : 0.f;
+  f32x4 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  // K fragment of (key tile nt, step ks): row 16 nt + c16, chunk 4 ks + g; V^T fragment of (d tile dt, 16 keys from 16 n):
+  // the lane points at row 16 n + 4 g + lane / 4 % 4, channels 16 dt + 4 (lane % 4)
+  const int fk = ((c16 >> 1) & 3) << 1 | (c16 >> 3);
+  int koff[2], voff[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) koff[i] = (16 * NT * kh + c16) * ROW + (((i * 4 + g) ^ fk) << 4);
+  const int vr = 4 * g + ((lane >> 2) & 3), fv = ((vr >> 1) & 3) << 1 | (vr >> 3);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    voff[i] = (16 * NT * kh + vr) * ROW + (((2 * i + ((lane & 3) >> 1)) ^ fv) << 4) + (lane & 1) * 8;
+
+  auto multiply = [&](int p, int buf) {
+    const char* img = lds + buf * PAGE_BYTES;
+    f32x4 s[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) s[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128 + nt * 16 * ROW);
+        s[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], s[nt], 0, 0, 0);
+      }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) s[nt] *= scale2;
+    if (p * PAGE + PAGE - 1 > t.pos0 || p * PAGE <= t.pos0 + t.n_tok - 1 - window) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = p * PAGE + 16 * (NT * kh + nt) + 4 * g + e;
+          if (key > my_pos || key <= my_first) s[nt][e] = -INFINITY;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[nt][e]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m, mx);
+    const bool dead = mn == -INFINITY;
+    const float mref = dead ? 0.f : mn;
+    const float corr = dead ? 1.f : __builtin_amdgcn_exp2f(m - mref);
+    float ps = 0.f;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float pv = __builtin_amdgcn_exp2f(s[nt][e] - mref);
+        s[nt][e] = pv;
+        ps += pv;
+      }
+    ps += __shfl_xor(ps, 16, 64);
+    ps += __shfl_xor(ps, 32, 64);
+    l = l * corr + ps;
+    m = mn;
+    if (!__all(corr == 1.f)) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
+    }
+    const uint32_t page = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + buf * PAGE_BYTES;
+    if constexpr (KSPLIT == 4) {
+      const uint32_t at[4] = {page + voff[0], page + voff[1], page + voff[2], page + voff[3]};
+      const u32x2 w = {pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3])};
+      all_products16(o, __builtin_bit_cast(s16x4, w), at, std::make_integer_sequence<int, DT / 8>());
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const uint32_t half = page + kk * 32 * ROW;
+        const uint32_t at[4] = {half + voff[0], half + voff[1], half + voff[2], half + voff[3]};
+        const u32x4 w = {pack_bf16x2(s[2 * kk][0], s[2 * kk][1]), pack_bf16x2(s[2 * kk][2], s[2 * kk][3]),
+                         pack_bf16x2(s[2 * kk + 1][0], s[2 * kk + 1][1]), pack_bf16x2(s[2 * kk + 1][2], s[2 * kk + 1][3])};
+        all_products<ROW>(o, __builtin_bit_cast(bf16x8, w), at, std::make_integer_sequence<int, DT / 8>());
+      }
+    }
+  };
+
+  if (p_begin + 1 < p_end) load_page(p_begin + 1, 1);
+  for (int p = p_begin; p < p_end; ++p) {
+    const int buf = (p - p_begin) & 1;
+    // this page has landed (mine: all but the NI loads of the page behind it; everyone's: the barrier)
+    if (p + 1 < p_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (wave_active) multiply(p, buf);
+    if (p + 2 < p_end) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // my reads of this buffer are done; everyone's: the barrier
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      load_page(p + 2, buf);
+    }
+  }
+
+  if constexpr (KSPLIT == 4) {  // the four key quarters: 2 joins 0 and 3 joins 1, then 1 joins 0
+#pragma unroll
+    for (int step = 2; step > 0; step >>= 1) {
+      __syncthreads();  // no page is read any more (and none is on its way); the other pair has read what it joined
+      f32x4* rec = reinterpret_cast<f32x4*>(lds) + ((sg * 2 + (kh & (step - 1))) * (DT + 1)) * 64 + lane;
+      if (kh >= step && kh < 2 * step) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) rec[dt * 64] = o[dt];
+        rec[DT * 64] = (f32x4){m, l, 0.f, 0.f};
+      }
+      __syncthreads();
+      if (kh < step) {
+        const f32x4 ml = rec[DT * 64];
+        const float mn = fmaxf(m, ml[0]), mref = mn == -INFINITY ? 0.f : mn;
+        const float f0 = __builtin_amdgcn_exp2f(m - mref), f1 = __builtin_amdgcn_exp2f(ml[0] - mref);
+        l = l * f0 + ml[1] * f1;
+        m = mn;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = o[dt] * f0 + rec[dt * 64] * f1;
+      }
+    }
+    if (kh) return;
+  }
+  if (!valid) return;
+  if (splits == 1) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    uint16_t* dst = out + row * o_row + head * o_head + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      u32x2 w = {pack_bf16x2(o[dt][0] * inv, o[dt][1] * inv), pack_bf16x2(o[dt][2] * inv, o[dt][3] * inv)};
+      *reinterpret_cast<u32x2*>(dst + 16 * dt) = w;
+    }
+  } else {
+    const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + slot;
+    float* dst = ws_o + rec * RANK + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(dst + 16 * dt) = o[dt];
+    if (g == 0) {
+      ws_ml[2 * rec] = m * LN2;
+      ws_ml[2 * rec + 1] = l;
+    }
+  }
+}
+
 // One workgroup per (tile, slot): out = sum_s o_s exp(m_s - M) / (sum_s l_s exp(m_s - M) + exp(sink - M)).  The splits'
 // factors are made once, by a wave with a split per lane; a thread then owns runs of 4 channels, all loads of a run in
 // flight together.
@@ -320,21 +606,28 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
            const void* cache, long page_stride, const int* block_tables, int bt_stride, const int* tiles,
            const int* positions, int n_tiles, int heads, const float* sink, void* out, long o_row, long o_head,
            float scale, int window, int splits, float* ws_o, float* ws_ml, hipStream_t st) {
-  constexpr int LDS = 64 * ((ROT_ONLY ? ROT : RANK + ROT) * 2 + 16) + RANK * (64 * 2 + 16);
-  static bool attr_set = false;
-  if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)latent_mfma_kernel<RANK, ROT, ROT_ONLY>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            LDS) != hipSuccess)
-      return -2;
-    attr_set = true;
+  // entries of 512 + 64 values: pages straight into LDS (narrower ones keep three waves per SIMD in the kernel above)
+  constexpr bool WIDE = !ROT_ONLY && RANK == 512 && ROT == 64;
+  auto* kernel = latent_mfma_kernel<RANK, ROT, ROT_ONLY>;
+  int lds = 64 * ((ROT_ONLY ? ROT : RANK + ROT) * 2 + 16) + RANK * (64 * 2 + 16);
+  static bool attr_set[2] = {false, false};
+  int which = 0;
+  if constexpr (WIDE) {
+    which = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
+    kernel = which ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 1>;
+    lds = 2 * 64 * (RANK + ROT) * 2;
   }
-  latent_mfma_kernel<RANK, ROT, ROT_ONLY><<<dim3(n_tiles, splits), dim3(256), LDS, st>>>(
+  if (!attr_set[which]) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
+    attr_set[which] = true;
+  }
+  kernel<<<dim3(n_tiles, splits), dim3(which ? 512 : 256), lds, st>>>(
       (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
       page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
       window, splits, ws_o, ws_ml);
   if (splits > 1)
-    latent_merge_kernel<<<dim3(n_tiles, 64), dim3(128), 0, st>>>(ws_o, ws_ml, tiles, heads, sink, (uint16_t*)out,
-                                                                 o_row, o_head, splits, RANK);
+    latent_merge_kernel<<<dim3(n_tiles, tiles ? 64 : min(heads, 64)), dim3(128), 0, st>>>(
+        ws_o, ws_ml, tiles, heads, sink, (uint16_t*)out, o_row, o_head, splits, RANK);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -1,0 +1,63 @@
+"""Latent attention over entries of 512 + 64 values against float64: head counts around the waves' shares, page and split remainders,
+windows, sinks, prefill tiles."""
+
+import pytest
+import torch
+
+from vllm_production_stack_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV, BF = torch.device("cuda"), torch.bfloat16
+RANK, ROT, PAGE = 512, 64, 64
+
+
+def setup(ctx, rows_of, heads, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    n = [-(-c // PAGE) for c in ctx]
+    pool = (torch.randn(sum(n) + 1, 8 + PAGE * (RANK + ROT), generator=g, device=DEV) * 0.5).to(BF)
+    order = torch.randperm(sum(n), generator=g, device=DEV).int().tolist()
+    table, at = [], 0
+    for k in n:
+        table.append(order[at:at + k] + [0] * (max(n) - k))
+        at += k
+    t = sum(rows_of)
+    q = (torch.randn(t, heads, RANK + ROT, generator=g, device=DEV) * 0.7).to(BF)
+    return pool, torch.tensor(table, dtype=torch.int32, device=DEV), q, torch.randn(heads, generator=g, device=DEV)
+
+
+def expected(pool, table, q, sink, ctx, rows_of, scale, window):
+    out, at = [], 0
+    for s, (c, n) in enumerate(zip(ctx, rows_of)):
+        ent = pool[table[s, : -(-c // PAGE)].long(), 8:].reshape(-1, RANK + ROT)[:c].double()
+        sc = (q[at:at + n].double().reshape(-1, RANK + ROT) @ ent.t()).view(n, -1, c) * scale
+        pos = torch.arange(c - n, c, device=DEV)[:, None, None]
+        key = torch.arange(c, device=DEV)[None, None]
+        sc.masked_fill_((key > pos) | (key <= pos - window), float("-inf"))
+        p = torch.softmax(torch.cat([sc, sink.double().view(1, -1, 1).expand(n, -1, 1)], 2), 2)[..., :c]
+        out.append((p.reshape(-1, c) @ ent[:, :RANK]).view(n, -1, RANK))
+        at += n
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("heads", [1, 16, 17, 32, 33, 64, 70])
+@pytest.mark.parametrize("splits,window", [(1, 1 << 30), (3, 1 << 30), (8, 100)])
+def test_decode_rows(heads, splits, window):
+    ctx = [1, 64, 65, 127, 300, 1000]
+    pool, table, q, sink = setup(ctx, [1] * len(ctx), heads, heads)
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    out = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, None, pos, sink, 0.05, splits=splits, window=window)
+    want = expected(pool, table, q, sink, ctx, [1] * len(ctx), 0.05, window)
+    # weights and results in 16 bits: half a unit in the last place each, 2^-9 of the norm
+    assert float((out.double() - want).norm() / want.norm()) < 6e-3
+
+
+@pytest.mark.parametrize("heads", [3, 16, 64])
+def test_prefill_tiles(heads):
+    ctx, rows_of = [70, 500, 130], [70, 33, 1]
+    pool, table, q, sink = setup(ctx, rows_of, heads, 90 + heads)
+    seq = torch.tensor([s for s, n in enumerate(rows_of) for _ in range(n)], dtype=torch.int32, device=DEV)
+    pos = torch.cat([torch.arange(c - n, c, dtype=torch.int32) for c, n in zip(ctx, rows_of)]).to(DEV)
+    tiles = torch.from_numpy(ops.build_latent_tiles(rows_of, ctx, heads)).to(DEV)
+    out = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, seq, pos, sink, 0.05, tiles=tiles)
+    want = expected(pool, table, q, sink, ctx, rows_of, 0.05, 1 << 30)
+    assert float((out.double() - want).norm() / want.norm()) < 6e-3
