@@ -608,7 +608,7 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
            float scale, int window, int splits, float* ws_o, float* ws_ml, hipStream_t st) {
   // entries of 512 + 64 values: pages straight into LDS (narrower ones keep three waves per SIMD in the kernel above)
   constexpr bool WIDE = !ROT_ONLY && RANK == 512 && ROT == 64;
-  auto* kernel = latent_mfma_kernel<RANK, ROT, ROT_ONLY>;
+  decltype(&latent_mfma_kernel<32, 64, true>) kernel;  // (both kernels take the same arguments)
   int lds = 64 * ((ROT_ONLY ? ROT : RANK + ROT) * 2 + 16) + RANK * (64 * 2 + 16);
   static bool attr_set[2] = {false, false};
   int which = 0;
@@ -616,6 +616,8 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
     which = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
     kernel = which ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 1>;
     lds = 2 * 64 * (RANK + ROT) * 2;
+  } else {
+    kernel = latent_mfma_kernel<RANK, ROT, ROT_ONLY>;
   }
   if (!attr_set[which]) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;

@@ -1,0 +1,237 @@
+// Projections of up to a few hundred token rows for gfx950: y[M, N] = x[M, K] . W[N, K]^T, the sizes of decode batches and of a new
+// turn's prompt.  Too few rows for 256 x 256 tiles (a tile would be mostly padding and too few CUs would stream the weights):
+// the job is to pull W through HBM once at full rate, with the token rows beside it.
+//   * A workgroup owns 128 weight rows (PAIR: 64 gate and the 64 matching up rows) and up to 128 token rows; the reduction is
+//     split over workgroups until about every CU has one (splits of whole 64-element chunks, not necessarily equal).
+//   * Both operands go from memory straight into LDS (rows of 128 bytes, 16-byte chunk j of row r at j ^ (r ^ r / 8) % 8, so that
+//     the 16 rows of a fragment cover all banks), four stages of which three are on their way: 64 to 96 KiB a CU in flight.
+//   * One barrier a chunk, counted waits.  A wave multiplies 32 weight rows with all token tiles on v_mfma_f32_16x16x32_bf16;
+//     its accumulators hold four consecutive outputs of a token, as in the streaming kernel of gemm.hip, whose reduction
+//     (partial sums in 32 bits, fixed order) closes a split product.
+//   * Workgroups start at different chunks of their range (see `first`).
+// 28672 x 4096 with the gated unit: 8 rows 45.2 -> 39.4 us (5.96 TB/s of weights), 64 rows 57.2 -> 42.1; 128256 x 4096, 8 rows: 191 -> 161
+// (6.5 TB/s); 4096 x 14336, 88 rows: 50.1 -> 31.6.  The whole range stands at the dispatch in ops/__init__.py.
+#include "common.h"
+
+namespace {
+
+constexpr int BN = 128, BK = 64, STAGES = 4, ROWB = BK * 2;
+
+__device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
+
+template <int MT, bool PAIR>
+__global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __restrict__ x, long x_stride,
+                                                          const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
+                                                          uint16_t* __restrict__ y, long y_stride, float* __restrict__ ws, int M,
+                                                          int N, int K, int S) {
+  constexpr int XI = (MT + 1) / 2;            // KiB of token rows that a wave loads of a stage (the last ones twice where MT is odd)
+  constexpr int NL = 4 + XI;                  // loads of a stage
+  // weights are read once: non-temporal loads, except where the partial sums of many rows want the memory-side cache as well
+  constexpr int POLICY = PAIR || MT <= 3 ? 2 : 0;
+  constexpr int STAGE = (BN + 16 * MT) * ROWB;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15, g = lane >> 4;
+  const int n_out = PAIR ? N >> 1 : N;
+  const int n0 = blockIdx.x * (PAIR ? BN / 2 : BN), m0 = blockIdx.z * 128;
+  const int chunks = K / BK, per = chunks / S, extra = chunks % S, sp = blockIdx.y;
+  const int c0 = sp * per + min(sp, extra), n = per + (sp < extra ? 1 : 0);
+  const int mrows = min(M - m0, 16 * MT);
+
+  // bytes from the operands' first chunk to what this lane loads: 8 rows of 8 chunks a KiB
+  uint32_t woff[4], xoff[XI];
+  int wlds[4], xlds[XI];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int kib = 4 * i + wave, r = 8 * kib + (lane >> 3);
+    const int row = PAIR ? n0 + (r & 63) + (r >> 6) * n_out : n0 + r;
+    woff[i] = (uint32_t)row * (uint32_t)(K * 2) + (((lane & 7) ^ swz(r)) << 4);
+    wlds[i] = kib * 1024;
+  }
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int kib = min(4 * i + wave, 2 * MT - 1), r = 8 * kib + (lane >> 3);
+    xoff[i] = (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)) + (((lane & 7) ^ swz(r)) << 4);  // rows past the last repeat it
+    xlds[i] = BN * ROWB + kib * 1024;
+  }
+  const char* wp = reinterpret_cast<const char*>(w) + (long)c0 * ROWB;
+  const char* xp = reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB;
+  // Workgroups walk their chunks from different ones on: rows whose length is a power of two put a chunk of all 128 rows on the
+  // same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
+  const int first = n > 0 ? (int)(blockIdx.x * 3 % n) : 0;
+  auto load = [&](int i_c) {
+    char* st = lds + (i_c & (STAGES - 1)) * STAGE;
+    const int c = i_c + first < n ? i_c + first : i_c + first - n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wp + (long)c * ROWB + woff[i]),
+                                       (__attribute__((address_space(3))) void*)(st + wlds[i]), 16, 0, POLICY);
+#pragma unroll
+    for (int i = 0; i < XI; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp + (long)c * ROWB + xoff[i]),
+                                       (__attribute__((address_space(3))) void*)(st + xlds[i]), 16, 0, 0);
+  };
+  // fragments: row c16 of a 16-row tile, chunk 4 ks + g
+  const int fr = c16 * ROWB, f0 = ((g ^ swz(c16)) << 4), f1 = (((4 + g) ^ swz(c16)) << 4);
+  const int arow[2] = {PAIR ? 16 * wave : 32 * wave, PAIR ? 64 + 16 * wave : 32 * wave + 16};
+  f32x4 acc[2][MT];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[a][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  for (int c = 0; c < STAGES - 1 && c < n; ++c) load(c);
+  for (int c = 0; c < n; ++c) {
+    // chunk c has landed (mine: all but the loads of the two chunks behind it) and my reads of chunk c - 1 are done;
+    // everyone's: the barrier
+    if (c + 2 < n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * NL) : "memory");
+    else if (c + 1 < n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NL) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (c + STAGES - 1 < n) load(c + STAGES - 1);
+    const char* st = lds + (c & (STAGES - 1)) * STAGE;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 a[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        // swz(16 m + c16) = swz(c16) ^ (2 m) % 8: the tile's number moves its chunks by an even step
+        const int sw = ((2 * (arow[i] >> 4)) & 7) << 4;
+        a[i] = *reinterpret_cast<const bf16x8*>(st + arow[i] * ROWB + fr + ((ks ? f1 : f0) ^ sw));
+      }
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(st + (BN + 16 * t) * ROWB + fr + ((ks ? f1 : f0) ^ (((2 * t) & 7) << 4)));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][t], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int j = 16 * t + c16;
+    if (j >= mrows) continue;
+    if (S > 1) {
+      float* p = ws + ((long)sp * M + m0 + j) * N;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<f32x4*>(p + n0 + (PAIR ? 16 * wave + i * n_out : arow[i]) + 4 * g) = acc[i][t];
+    } else if (PAIR) {
+      f32x4 s = acc[0][t];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] = s[r] / (1.f + __expf(-s[r])) * acc[1][t][r];
+      const u32x2 o = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+      *reinterpret_cast<u32x2*>(y + (long)(m0 + j) * y_stride + n0 + 16 * wave + 4 * g) = o;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int col = n0 + arow[i] + 4 * g;
+        f32x4 s = acc[i][t];
+        if (bias != nullptr) {
+          const u32x2 bb = *reinterpret_cast<const u32x2*>(bias + col);
+          s[0] += bf16lo(bb[0]);
+          s[1] += bf16hi(bb[0]);
+          s[2] += bf16lo(bb[1]);
+          s[3] += bf16hi(bb[1]);
+        }
+        const u32x2 o = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+        *reinterpret_cast<u32x2*>(y + (long)(m0 + j) * y_stride + col) = o;
+      }
+    }
+  }
+}
+
+// out[m, n .. n + 3] = epilogue(sum_s ws[s, m, n .. n + 3]); one thread per 4 output columns, eight partials in flight.
+template <bool PAIR>
+__global__ __launch_bounds__(256) void mid_reduce_kernel(const float* __restrict__ ws, const uint16_t* __restrict__ bias,
+                                                         uint16_t* __restrict__ y, long y_stride, int M, int N, int S) {
+  const int n_out = PAIR ? N >> 1 : N;
+  const int col = (blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
+  if (col >= n_out) return;
+  const float* p = ws + (long)m * N + col;
+  const long step = (long)M * N;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f}, s2 = s;
+  for (int i0 = 0; i0 < S; i0 += 8) {
+    f32x4 v[8], v2[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const long at = (long)min(i0 + i, S - 1) * step;
+      v[i] = *reinterpret_cast<const f32x4*>(p + at);
+      if (PAIR) v2[i] = *reinterpret_cast<const f32x4*>(p + at + n_out);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i0 + i < S) {
+        s += v[i];
+        if (PAIR) s2 += v2[i];
+      }
+  }
+  if (PAIR) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s[r] = s[r] / (1.f + __expf(-s[r])) * s2[r];
+  } else if (bias != nullptr) {
+    const u32x2 bb = *reinterpret_cast<const u32x2*>(bias + col);
+    s[0] += bf16lo(bb[0]);
+    s[1] += bf16hi(bb[0]);
+    s[2] += bf16lo(bb[1]);
+    s[3] += bf16hi(bb[1]);
+  }
+  const u32x2 o = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+  *reinterpret_cast<u32x2*>(y + (long)m * y_stride + col) = o;
+}
+
+template <int MT, bool PAIR>
+int launch_mid(const void* x, long xs, const void* w, const void* bias, void* y, long ys, float* ws, int M, int N, int K, int S,
+               hipStream_t stream) {
+  constexpr int LDS = STAGES * (BN + 16 * MT) * ROWB;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)mid_gemm_kernel<MT, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+      return -2;
+    attr_set = true;
+  }
+  const int n_out = PAIR ? N / 2 : N;
+  mid_gemm_kernel<MT, PAIR><<<dim3(n_out / (PAIR ? BN / 2 : BN), S, (M + 127) / 128), 256, LDS, stream>>>(
+      (const uint16_t*)x, xs, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ys, ws, M, N, K, S);
+  if (S > 1)
+    mid_reduce_kernel<PAIR><<<dim3((n_out / 4 + 255) / 256, M), 256, 0, stream>>>(ws, (const uint16_t*)bias, (uint16_t*)y, ys, M, N, S);
+  return 0;
+}
+
+}  // namespace
+
+// Workgroups along the reduction for a shape, 0 where the kernel does not tile it: as many as fill the chip's 256 CUs once, none
+// shorter than eight chunks (the three on their way at the start are a third of it).
+VPSA_EXPORT int vpsa_mid_gemm_splits(int M, int N, int K, int pair) {
+  const int n_out = pair ? N / 2 : N, bn = pair ? BN / 2 : BN;
+  if (M <= 0 || n_out <= 0 || (pair && (N & 1)) || n_out % bn != 0 || K % BK != 0 || (long)N * K * 2 >= (1L << 32)) return 0;
+  const int blocks = n_out / bn * ((M + 127) / 128);
+  int s = 256 / blocks;
+  const int most = K / BK / 8;
+  if (s > most) s = most;
+  return s < 1 ? 1 : s;
+}
+
+// x [M, K] (row stride xs elements, 16-byte aligned rows), w [N, K] contiguous, bias [N] or null, y [M, N] (or [M, N / 2] when
+// pair != 0; row stride ys).  ws: fp32 workspace of S * M * N elements (unused when S == 1).
+VPSA_EXPORT int vpsa_mid_gemm(const void* x, long xs, const void* w, const void* bias, void* y, long ys, void* ws, int M, int N,
+                              int K, int pair, int S, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if ((xs & 7) || (ys & 3) || (((uintptr_t)x | (uintptr_t)w) & 15) || ((uintptr_t)y & 7) || xs * 256 >= (1L << 31)) return -1;
+  if (S <= 0 || S != vpsa_mid_gemm_splits(M, N, K, pair) || (pair && bias) || (S > 1 && !ws) || M > 65535) return -1;
+#define MID(MT)                                                                                                       \
+  return pair ? launch_mid<MT, true>(x, xs, w, bias, y, ys, (float*)ws, M, N, K, S, stream)                           \
+              : launch_mid<MT, false>(x, xs, w, bias, y, ys, (float*)ws, M, N, K, S, stream)
+  switch (M >= 128 ? 8 : (M + 15) / 16) {
+    case 1: MID(1);
+    case 2: MID(2);
+    case 3: MID(3);
+    case 4: MID(4);
+    case 5: MID(5);
+    case 6: MID(6);
+    case 7: MID(7);
+    default: MID(8);
+  }
+#undef MID
+}

@@ -1,0 +1,49 @@
+"""Projections of up to a few hundred rows: row counts around tiles and row blocks, fewer chunks than stages, uneven splits, bias, the gated
+unit, strided rows, and what the dispatch leaves to other kernels."""
+
+import pytest
+import torch
+
+from vllm_production_stack_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV, BF = torch.device("cuda"), torch.bfloat16
+
+
+@pytest.fixture
+def any_shape(monkeypatch):
+    monkeypatch.setattr(ops, "MID_MIN_FILL", 0.0)
+    monkeypatch.setattr(ops, "MID_ROWS", ops.MID_ROWS_LONG)
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 48, 63, 80, 97, 112, 127, 128, 129, 200, 256])
+@pytest.mark.parametrize("n,k,kind", [(128, 64, ""), (256, 192, "bias"), (128, 1088, ""), (256, 2624, "bias"), (384, 1088, "pair"), (256, 128, "pair")])
+def test_matches_float64(any_shape, m, n, k, kind):
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, generator=g, device=DEV).to(BF)[:, :k]   # rows of a wider tensor
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF)
+    b = torch.randn(n, generator=g, device=DEV).to(BF) if kind == "bias" else None
+    got = ops._mid_gemm(x, w, b, kind == "pair")
+    assert got is not None
+    want = x.double() @ w.double().t()
+    if kind == "pair":
+        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
+    elif b is not None:
+        want = want + b.double()
+    # sums in 32 bits, one rounding to 16: half a unit in the last place, 2^-9, of every value
+    assert float(((got.double() - want).abs() - want.abs() * 2 ** -8 - 1e-5).max()) < 0
+    assert torch.equal(got, ops._mid_gemm(x, w, b, kind == "pair"))    # fixed order of the partial sums
+
+
+def test_dispatch():
+    w = torch.zeros(4096, 4096, device=DEV, dtype=BF)
+    x = torch.zeros(300, 4096, device=DEV, dtype=BF)
+    assert ops._mid_gemm(x[:40], w, None, False) is not None
+    assert ops._mid_gemm(x[:120], w, None, False) is None              # partial sums of three quarters of the weights' bytes
+    assert ops._mid_gemm(x, w, None, False) is None
+    assert ops._mid_gemm(x[:40], w[:3584], None, False) is not None    # 224 workgroups
+    assert ops._mid_gemm(x[:40], w[:2048], None, False) is None        # 128
+    assert ops._mid_gemm(x[:40, 1:], w[:, 1:].contiguous(), None, False) is None   # a reduction that is no multiple of a chunk
+    assert ops._mid_gemm(x[:40].float(), w, None, False) is None
+    with torch.enable_grad():
+        assert ops._mid_gemm(x[:40].clone().requires_grad_(), w, None, False) is None

@@ -41,7 +41,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -667,6 +667,59 @@ def _stream_gemm(x2, w, bias, pair):
     return out if rc == 0 else None
 
 
+# ``mid_gemm`` (128 weight rows a workgroup, both operands straight into LDS) against what ran before, microseconds in a graph over
+# weights that no cache holds (library with its activation pass, or the kernels above up to 16 rows / mid_gemm):
+#   28672 x 4096 pair    1 row 43.6/39.4    24 rows 50.4/40.2    64 rows 57.2/42.1    104 rows 60.6/55.5    128 rows 61.9/53.3
+#   4096 x 14336         1     25.1/21.4    24      29.0/23.1    64      39.2/28.1    128      75.2/38.8    200      56.9/53.3
+#   6144 x 4096          1     12.9/12.0    24      14.4/13.6    64      17.5/16.6    104      23.2/21.6    200      26.2/32.3
+#   4096 x 4096          1      9.8/10.0    24      13.1/11.4    64      14.9/13.9    104      16.1/17.6
+#   128256 x 4096        1      190/162     24       198/167     64       214/191     104       236/243
+#   57344 x 8192 pair    1      172/146     64       194/161     104      203/219
+#   8192 x 28672         1       90/76      64       147/105     200      311/204
+#   3584 x 18944         1       46/25      24       108/26      200      121/66
+#   37888 x 3584 pair    1     48.4/53.6    64      64.9/65.7  (296 workgroups: a second round nearly empty)
+#   2048 x 2048          1      5.7/7.2     64       8.7/9.9   (64 workgroups)
+MID_MIN_FILL = 0.75      # of the rounds of one workgroup per CU
+MID_ROWS = 96            # every shape that fills the chip
+MID_ROWS_ONE_ROUND = 128  # one round, and partial sums (32 bits, written and read) below three quarters of the weights' bytes
+MID_ROWS_LONG = 256      # reductions beyond 8192, where the library's pick is poor at every batch
+
+
+def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
+    """Workgroups along the reduction when ``mid_gemm`` should take the shape, else 0."""
+    if not 0 < m <= MID_ROWS_LONG:
+        return 0
+    splits = int(_kernels().vpsa_mid_gemm_splits(c_int(m), c_int(n), c_int(k), c_int(1 if pair else 0)))
+    if splits <= 0:
+        return 0
+    wgs = (n // 128) * splits * (-(-m // 128))  # (a pair's workgroup holds 64 gate and 64 up rows)
+    if wgs < MID_MIN_FILL * TILE_CUS * (-(-wgs // TILE_CUS)):
+        return 0
+    if m <= MID_ROWS or (not pair and k > STREAM_MAX_K):
+        return splits
+    if m <= MID_ROWS_ONE_ROUND and wgs <= TILE_CUS and (splits == 1 if pair else 16 * m * splits <= 3 * k):
+        return splits
+    return 0
+
+
+def _mid_gemm(x2, w, bias, pair):
+    """Projection of up to a few hundred rows (``csrc/kernels/mid_gemm.hip``), or None where another kernel is the better choice."""
+    if not (_skinny_enabled and x2.is_cuda and x2.dim() == 2 and x2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1]))
+            and not (torch.is_grad_enabled() and (x2.requires_grad or w.requires_grad))):
+        return None
+    m, n, k = x2.shape[0], w.shape[0], w.shape[1]
+    splits = _mid_splits(m, n, k, pair)
+    if splits <= 0:
+        return None
+    out = torch.empty((m, n // 2 if pair else n), dtype=x2.dtype, device=x2.device)
+    ws = torch.empty((splits * m * n,), dtype=torch.float32, device=x2.device) if splits > 1 else None
+    rc = _kernels().vpsa_mid_gemm(_p(x2), c_long(x2.stride(0)), _p(w), _p(bias), _p(out), c_long(out.stride(0)), _p(ws), c_int(m),
+                                  c_int(n), c_int(k), c_int(1 if pair else 0), c_int(splits), _stream())
+    return out if rc == 0 else None
+
+
 def pack_weight(w: torch.Tensor) -> torch.Tensor:
     """[N, K] -> the same matrix in matrix-core tile order, [N / 16][K / 32][16][32] flattened
     (N a multiple of 16, K of 32): what ``packed_linear`` streams.  A second copy of the weight."""
@@ -706,7 +759,7 @@ def _skinny_ok(x, w, bias):
             and x.stride(1) == 1 and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous())))
 
 
-# Dispatch thresholds measured on MI355X (profiles/gemm_micro_graph.jsonl, HIP-graph replay,
+# Dispatch thresholds of shapes that mid_gemm below does not take, measured on MI355X (profiles/gemm_micro_graph.jsonl, HIP-graph replay,
 # Llama-3-8B shapes, microseconds: library / register-direct / streaming kernel):
 #   o-proj  4096x4096   1-16 rows: 14.9-15.0 /  9.6-11.4 / 11.1-14.4   -> register-direct
 #   qkv     6144x4096   1-16 rows: 14.2      / 14.0-19.2 / 12.8-14.0   -> streaming
@@ -775,7 +828,8 @@ def tile_rows(x, w, pair: bool = False) -> int:
 
 def linear(x, w, bias=None, packed=None):
     """y = x @ w.T (+ bias).  Prefill-sized batches run the hand-written 256 x 256 MFMA kernel
-    (``csrc/kernels/tile_gemm.hip``) when its tiles fill the chip; decode batches of up to 16 rows
+    (``csrc/kernels/tile_gemm.hip``) when its tiles fill the chip; batches of up to a hundred rows or so ``mid_gemm.hip``
+    where its workgroups do (``_mid_splits``), of up to 16 rows otherwise
     the weight-streaming MFMA kernels of ``csrc/kernels/gemm.hip`` (which one depends on the
     weight's shape); everything else goes to the library GEMM (hipBLASLt).  ``packed``:
     ``pack_weight(w)`` when the caller keeps one (decode-only steps): up to 64 rows then stream
@@ -784,6 +838,9 @@ def linear(x, w, bias=None, packed=None):
         y = packed_linear(x, packed, w.shape[0], w.shape[1], bias, False)
         if y is not None:
             return y
+    y = _mid_gemm(x, w, bias, False)
+    if y is not None:
+        return y
     if x.dim() == 2 and x.shape[0] <= SMALL_BATCH_ROWS and _skinny_ok(x, w, bias):
         y = None
         if w.numel() <= DIRECT_MAX_WEIGHT_ELEMS:
@@ -837,13 +894,16 @@ def qkv_linear(x, w, bias, q_cols: int):
 
 
 def gate_up_silu(x, w_gate_up, packed=None):
-    """silu(x @ Wg.T) * (x @ Wu.T) for ``w_gate_up = [Wg; Wu]``: fused in one kernel for decode
-    batches (weight-streaming kernels) and for prefill batches (SwiGLU epilogue of the 256 x 256
+    """silu(x @ Wg.T) * (x @ Wu.T) for ``w_gate_up = [Wg; Wu]``: fused in one kernel for
+    batches of up to a hundred rows or so (``mid_gemm`` and the weight-streaming kernels) and for prefill batches (SwiGLU epilogue of the 256 x 256
     MFMA kernel); library GEMM + activation kernel for what neither takes.  ``packed`` as in ``linear``."""
     if packed is not None and x.dim() == 2 and x.shape[0] <= PACKED_MAX_ROWS and _skinny_ok(x, w_gate_up, None):
         y = packed_linear(x, packed, w_gate_up.shape[0], w_gate_up.shape[1], None, True)
         if y is not None:
             return y
+    y = _mid_gemm(x, w_gate_up, None, True)
+    if y is not None:
+        return y
     if x.dim() == 2 and x.shape[0] <= PAIR_STREAM_MAX_ROWS and _skinny_ok(x, w_gate_up, None):
         y = _stream_gemm(x, w_gate_up, None, True)
         if y is None and x.shape[0] <= 8:
