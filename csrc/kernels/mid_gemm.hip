@@ -19,67 +19,51 @@ constexpr int BN = 128, BK = 64, STAGES = 4, ROWB = BK * 2;
 
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-template <int MT, bool PAIR>
-__global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __restrict__ x, long x_stride,
-                                                          const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
-                                                          uint16_t* __restrict__ y, long y_stride, float* __restrict__ ws, int M,
-                                                          int N, int K, int S) {
-  constexpr int XI = (MT + 1) / 2;            // KiB of token rows that a wave loads of a stage (the last ones twice where MT is odd)
-  constexpr int NL = 4 + XI;                  // loads of a stage
-  // weights are read once: non-temporal loads, except where the partial sums of many rows want the memory-side cache as well
-  constexpr int POLICY = PAIR || MT <= 3 ? 2 : 0;
-  constexpr int STAGE = (BN + 16 * MT) * ROWB;
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// acc[i][t] += W tile i of the wave x token tile t over chunks [0, n) of both operands: NA * 64 weight rows and MT * 16 token rows a
+// chunk, all of it in LDS stages.  wrow(r) / xrow(r): bytes from wp / xp to row r's first chunk; arow: the wave's weight tiles (rows
+// within the workgroup's).  POLICY of the weight loads: 2 = non-temporal.  Nothing is on its way or read any more on return.
+template <int MT, int NA, int POLICY, typename WRow, typename XRow>
+__device__ __forceinline__ void stream_product(const char* __restrict__ wp, const char* __restrict__ xp, WRow wrow, XRow xrow, int n,
+                                               int first, char* lds, const int (&arow)[NA], f32x4 (&acc)[NA][MT]) {
+  constexpr int WI = 2 * NA;        // KiB of weight rows that a wave loads of a stage
+  constexpr int XI = (MT + 1) / 2;  // and of token rows (the last ones twice where MT is odd)
+  constexpr int NL = WI + XI;       // loads of a stage
+  constexpr int BN = 64 * NA, STAGE = (BN + 16 * MT) * ROWB;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g = lane >> 4;
-  const int n_out = PAIR ? N >> 1 : N;
-  const int n0 = blockIdx.x * (PAIR ? BN / 2 : BN), m0 = blockIdx.z * 128;
-  const int chunks = K / BK, per = chunks / S, extra = chunks % S, sp = blockIdx.y;
-  const int c0 = sp * per + min(sp, extra), n = per + (sp < extra ? 1 : 0);
-  const int mrows = min(M - m0, 16 * MT);
-
-  // bytes from the operands' first chunk to what this lane loads: 8 rows of 8 chunks a KiB
-  uint32_t woff[4], xoff[XI];
-  int wlds[4], xlds[XI];
+  // what this lane loads: 8 rows of 8 chunks a KiB
+  uint32_t woff[WI], xoff[XI];
+  int xlds[XI];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int kib = 4 * i + wave, r = 8 * kib + (lane >> 3);
-    const int row = PAIR ? n0 + (r & 63) + (r >> 6) * n_out : n0 + r;
-    woff[i] = (uint32_t)row * (uint32_t)(K * 2) + (((lane & 7) ^ swz(r)) << 4);
-    wlds[i] = kib * 1024;
+  for (int i = 0; i < WI; ++i) {
+    const int r = 8 * (4 * i + wave) + (lane >> 3);
+    woff[i] = wrow(r) + (((lane & 7) ^ swz(r)) << 4);
   }
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
     const int kib = min(4 * i + wave, 2 * MT - 1), r = 8 * kib + (lane >> 3);
-    xoff[i] = (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)) + (((lane & 7) ^ swz(r)) << 4);  // rows past the last repeat it
+    xoff[i] = xrow(r) + (((lane & 7) ^ swz(r)) << 4);
     xlds[i] = BN * ROWB + kib * 1024;
   }
-  const char* wp = reinterpret_cast<const char*>(w) + (long)c0 * ROWB;
-  const char* xp = reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB;
-  // Workgroups walk their chunks from different ones on: rows whose length is a power of two put a chunk of all 128 rows on the
-  // same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
-  const int first = n > 0 ? (int)(blockIdx.x * 3 % n) : 0;
   auto load = [&](int i_c) {
     char* st = lds + (i_c & (STAGES - 1)) * STAGE;
     const int c = i_c + first < n ? i_c + first : i_c + first - n;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < WI; ++i)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wp + (long)c * ROWB + woff[i]),
-                                       (__attribute__((address_space(3))) void*)(st + wlds[i]), 16, 0, POLICY);
+                                       (__attribute__((address_space(3))) void*)(st + (4 * i + wave) * 1024), 16, 0, POLICY);
 #pragma unroll
     for (int i = 0; i < XI; ++i)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp + (long)c * ROWB + xoff[i]),
                                        (__attribute__((address_space(3))) void*)(st + xlds[i]), 16, 0, 0);
   };
-  // fragments: row c16 of a 16-row tile, chunk 4 ks + g
-  const int fr = c16 * ROWB, f0 = ((g ^ swz(c16)) << 4), f1 = (((4 + g) ^ swz(c16)) << 4);
-  const int arow[2] = {PAIR ? 16 * wave : 32 * wave, PAIR ? 64 + 16 * wave : 32 * wave + 16};
-  f32x4 acc[2][MT];
+  // fragments: row c16 of a 16-row tile, chunk 4 ks + g; swz(16 m + c16) = swz(c16) ^ (2 m) % 8: a tile's number moves its chunks
+  // by an even step
+  const int fr = c16 * ROWB, f[2] = {(g ^ swz(c16)) << 4, ((4 + g) ^ swz(c16)) << 4};
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int i = 0; i < NA; ++i)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[a][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
+    for (int t = 0; t < MT; ++t) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
   for (int c = 0; c < STAGES - 1 && c < n; ++c) load(c);
   for (int c = 0; c < n; ++c) {
     // chunk c has landed (mine: all but the loads of the two chunks behind it) and my reads of chunk c - 1 are done;
@@ -93,21 +77,45 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
     const char* st = lds + (c & (STAGES - 1)) * STAGE;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 a[2];
+      bf16x8 a[NA];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        // swz(16 m + c16) = swz(c16) ^ (2 m) % 8: the tile's number moves its chunks by an even step
-        const int sw = ((2 * (arow[i] >> 4)) & 7) << 4;
-        a[i] = *reinterpret_cast<const bf16x8*>(st + arow[i] * ROWB + fr + ((ks ? f1 : f0) ^ sw));
-      }
+      for (int i = 0; i < NA; ++i)
+        a[i] = *reinterpret_cast<const bf16x8*>(st + arow[i] * ROWB + fr + (f[ks] ^ ((2 * (arow[i] >> 4) & 7) << 4)));
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(st + (BN + 16 * t) * ROWB + fr + ((ks ? f1 : f0) ^ (((2 * t) & 7) << 4)));
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(st + (BN + 16 * t) * ROWB + fr + (f[ks] ^ ((2 * t & 7) << 4)));
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][t], 0, 0, 0);
+        for (int i = 0; i < NA; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][t], 0, 0, 0);
       }
     }
   }
+  __syncthreads();
+}
+
+template <int MT, bool PAIR>
+__global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __restrict__ x, long x_stride,
+                                                          const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
+                                                          uint16_t* __restrict__ y, long y_stride, float* __restrict__ ws, int M,
+                                                          int N, int K, int S) {
+  // weights are read once: non-temporal loads, except where the partial sums of many rows want the memory-side cache as well
+  constexpr int POLICY = PAIR || MT <= 3 ? 2 : 0;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, g = lane >> 4;
+  const int n_out = PAIR ? N >> 1 : N;
+  const int n0 = blockIdx.x * (PAIR ? BN / 2 : BN), m0 = blockIdx.z * 128;
+  const int chunks = K / BK, per = chunks / S, extra = chunks % S, sp = blockIdx.y;
+  const int c0 = sp * per + min(sp, extra), n = per + (sp < extra ? 1 : 0);
+  const int mrows = min(M - m0, 16 * MT);
+  const int arow[2] = {PAIR ? 16 * wave : 32 * wave, PAIR ? 64 + 16 * wave : 32 * wave + 16};
+  f32x4 acc[2][MT];
+  // Workgroups walk their chunks from different ones on: rows whose length is a power of two put a chunk of all 128 rows on the
+  // same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
+  stream_product<MT, 2, POLICY>(
+      reinterpret_cast<const char*>(w) + (long)c0 * ROWB, reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB,
+      [&](int r) { return (uint32_t)(PAIR ? n0 + (r & 63) + (r >> 6) * n_out : n0 + r) * (uint32_t)(K * 2); },
+      [&](int r) { return (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)); },  // rows past the last repeat it
+      n, n > 0 ? (int)(blockIdx.x * 3 % n) : 0, lds, arow, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int j = 16 * t + c16;
@@ -138,6 +146,65 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
         const u32x2 o = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
         *reinterpret_cast<u32x2*>(y + (long)(m0 + j) * y_stride + col) = o;
       }
+    }
+  }
+}
+
+// The experts of a decode-sized batch: every routed expert's weights are streamed once against its rows (more than 16 MT rows: once
+// for each 16 MT).  UNIT: grid (inter / 64, experts), act[row] = unit(gate, up) of x[sorted_tok[row]], rows sorted by expert; act_limit >
+// 0: min(g, limit) * sigmoid(alpha g) * (clamp(u) + bias), else silu(g) * u; row_scale: factors of gate and up.  Else grid
+// (hidden / 64, experts), y[row] = W2 act[row] (64 weight rows a workgroup: with 128 a layer's 4096 rows leave one workgroup per CU
+// and no slack for experts without rows).
+// Against 16-row tiles that went from memory into registers, 64 bytes a row and load, 8 experts of 28672 x 4096 and 4096 x
+// 14336: 540 -> 435 us a mixture of 16 tokens, 283 -> 248 of 4; a decode step of two layers, 8 tokens 1105 -> 921, 48 tokens 1420 -> 1116.
+template <int MT, bool UNIT>
+__global__ __launch_bounds__(256, 1) void mid_experts_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                             const int* __restrict__ offsets, const int* __restrict__ sorted_tok,
+                                                             uint16_t* __restrict__ y, int N, int K, float act_limit,
+                                                             float act_alpha, float act_bias, const float* __restrict__ row_scale) {
+  constexpr int NA = UNIT ? 2 : 1;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int e = blockIdx.y, r0 = offsets[e], n_e = offsets[e + 1] - r0;
+  if (n_e <= 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, g = lane >> 4;
+  const int n_out = UNIT ? N >> 1 : N, n0 = blockIdx.x * 64, n = K / BK;
+  int arow[NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) arow[i] = 64 * i + 16 * wave;
+  for (int m0 = 0; m0 < n_e; m0 += 16 * MT) {
+    const int last = min(n_e - m0, 16 * MT) - 1;
+    f32x4 acc[NA][MT];
+    stream_product<MT, NA, 2>(
+        reinterpret_cast<const char*>(w + (long)e * N * K), reinterpret_cast<const char*>(x),
+        [&](int r) { return (uint32_t)(n0 + (r & 63) + (r >> 6) * n_out) * (uint32_t)(K * 2); },
+        [&](int r) {
+          const int row = r0 + m0 + min(r, last);
+          return (uint32_t)(UNIT ? sorted_tok[row] : row) * (uint32_t)(K * 2);
+        },
+        n, (int)((blockIdx.x * 3 + e) % n), lds, arow, acc);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int j = 16 * t + c16;
+      if (j > last) continue;
+      const long row = r0 + m0 + j;
+      f32x4 s = acc[0][t];
+      if (UNIT) {
+        const float rs = row_scale ? row_scale[row] : 1.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float gt = s[r] * rs, up = acc[NA - 1][t][r] * rs;
+          if (act_limit > 0.f) {
+            gt = fminf(gt, act_limit);
+            up = fminf(fmaxf(up, -act_limit), act_limit) + act_bias;
+            s[r] = gt / (1.f + __expf(-act_alpha * gt)) * up;
+          } else {
+            s[r] = gt / (1.f + __expf(-gt)) * up;
+          }
+        }
+      }
+      const u32x2 o = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+      *reinterpret_cast<u32x2*>(y + row * n_out + n0 + 16 * wave + 4 * g) = o;
     }
   }
 }
@@ -199,7 +266,55 @@ int launch_mid(const void* x, long xs, const void* w, const void* bias, void* y,
   return 0;
 }
 
+template <int MT>
+int launch_experts(const void* x, const void* w13, const void* w2, const int* offsets, const int* sorted_tok, void* act, void* y,
+                   int n_experts, int hidden, int inter, float act_limit, float act_alpha, float act_bias, const float* row_scale,
+                   hipStream_t stream) {
+  constexpr int UNIT_LDS = STAGES * (128 + 16 * MT) * ROWB, DOWN_LDS = STAGES * (64 + 16 * MT) * ROWB;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)mid_experts_kernel<MT, true>, hipFuncAttributeMaxDynamicSharedMemorySize, UNIT_LDS) != hipSuccess ||
+        hipFuncSetAttribute((const void*)mid_experts_kernel<MT, false>, hipFuncAttributeMaxDynamicSharedMemorySize, DOWN_LDS) != hipSuccess)
+      return -2;
+    attr_set = true;
+  }
+  mid_experts_kernel<MT, true><<<dim3(inter / 64, n_experts), 256, UNIT_LDS, stream>>>(
+      (const uint16_t*)x, (const uint16_t*)w13, offsets, sorted_tok, (uint16_t*)act, 2 * inter, hidden, act_limit, act_alpha, act_bias,
+      row_scale);
+  mid_experts_kernel<MT, false><<<dim3(hidden / 64, n_experts), 256, DOWN_LDS, stream>>>(
+      (const uint16_t*)act, (const uint16_t*)w2, offsets, nullptr, (uint16_t*)y, hidden, inter, 0.f, 1.f, 0.f, nullptr);
+  return 0;
+}
+
 }  // namespace
+
+// x [tokens, hidden]; w13 [E, 2*inter, hidden]; w2 [E, hidden, inter]; offsets [E+1] and sorted_tok [tokens*topk] from
+// vpsa_moe_align; act [tokens*topk, inter] and y [tokens*topk, hidden] are workspaces in expert-sorted row order.  No host
+// synchronisation and a launch shape that does not depend on the routing: HIP-graph capturable.  act_limit > 0: the clamped gated
+// unit (limit, alpha, bias) instead of SwiGLU.  row_scale (sorted order, or null): gate and up of a row are multiplied by it before
+// the activation (a factor on the row's input).
+VPSA_EXPORT int vpsa_moe_mfma_act(const void* x, const void* w13, const void* w2, const int* offsets, const int* sorted_tok,
+                                  void* act, void* y, int tokens, int topk, int n_experts, int hidden, int inter, float act_limit,
+                                  float act_alpha, float act_bias, const float* row_scale, hipStream_t stream) {
+  if (tokens * topk <= 0) return 0;
+  if (n_experts < 1 || n_experts > 65535 || hidden % 128 != 0 || inter % 512 != 0) return -1;
+  if ((long)inter * hidden * 4 >= (1L << 32) || (long)tokens * topk * (hidden > inter ? hidden : inter) * 2 >= (1L << 32)) return -1;
+  // an expert sees each token at most once: tokens bounds its row count
+#define EXPERTS(MT)                                                                                                         \
+  return launch_experts<MT>(x, w13, w2, offsets, sorted_tok, act, y, n_experts, hidden, inter, act_limit, act_alpha, act_bias, \
+                            row_scale, stream)
+  if (tokens <= 16) EXPERTS(1);
+  if (tokens <= 32) EXPERTS(2);
+  if (tokens <= 48) EXPERTS(3);
+  EXPERTS(4);
+#undef EXPERTS
+}
+
+VPSA_EXPORT int vpsa_moe_mfma(const void* x, const void* w13, const void* w2, const int* offsets, const int* sorted_tok, void* act,
+                              void* y, int tokens, int topk, int n_experts, int hidden, int inter, hipStream_t stream) {
+  return vpsa_moe_mfma_act(x, w13, w2, offsets, sorted_tok, act, y, tokens, topk, n_experts, hidden, inter, 0.f, 1.f, 0.f, nullptr,
+                           stream);
+}
 
 // Workgroups along the reduction for a shape, 0 where the kernel does not tile it: as many as fill the chip's 256 CUs once, none
 // shorter than eight chunks (the three on their way at the start are a third of it).

@@ -1188,15 +1188,26 @@ def moe_combine(y, weights, pos, tokens):
     return out
 
 
-# Decode batches up to this many tokens take the expert-grouped matrix-core kernels.  Measured
-# on one Mixtral-8x7B layer (MI355X): 0.48-0.54 ms for 4-32 tokens (5.2 TB/s of expert weights)
-# against 0.57-0.59 ms for all-experts batched GEMM; from ~64 tokens on the token tiles are
-# re-read through L2 by every wave and the batched GEMM is faster.
+# Batches whose experts see few rows each take the kernels that stream every routed expert's weights once (``csrc/kernels/mid_gemm.hip``)
+# instead of the 256-row tiles: up to this many tokens, and up to this many rows an expert on average (a pass takes 64).  One mixture,
+# microseconds in a graph, tiles / streaming: 8 experts of 28672 x 4096, two a token: 16 tokens 660/435, 48 660/425, 128 674/491, 192
+# 682/619, 224 683/696, 256 rows of a prompt 730/910; 16 experts of 2048 x 2048, four a token: 48 66.5/40.6, 192 69.9/46.7, 224 72.0/67.5.
 MOE_MFMA_MAX_TOKENS = int(os.environ.get("VPSA_MOE_MFMA_MAX_TOKENS", "48"))
+MOE_STREAM_ROWS = 48
+
+
+def moe_streams_experts(tokens: int, topk: int, experts: int) -> bool:
+    return MOE_MFMA_MAX_TOKENS > 0 and (tokens <= MOE_MFMA_MAX_TOKENS or tokens * topk <= MOE_STREAM_ROWS * experts)
 
 
 def moe_mfma_supported(hidden: int, inter: int) -> bool:
     return hidden % 128 == 0 and inter % 512 == 0
+
+
+def _rows16(x):
+    """``x`` contiguous with its first row on a 16-byte boundary (what loads straight into LDS take)."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
 def moe_experts_grouped(x, w13, w2, ids, weights, foreign=False, combine=True):
@@ -1219,7 +1230,7 @@ def moe_experts_grouped(x, w13, w2, ids, weights, foreign=False, combine=True):
     offsets, pos, sorted_tok = moe_align(ids, n_experts + (1 if foreign else 0))
     act = torch.empty((t * k, inter), dtype=x.dtype, device=x.device)
     y = torch.empty((t * k, hidden), dtype=x.dtype, device=x.device)
-    rc = _kernels().vpsa_moe_mfma(_p(x.contiguous()), _p(w13), _p(w2), _p(offsets), _p(sorted_tok),
+    rc = _kernels().vpsa_moe_mfma(_p(_rows16(x)), _p(w13), _p(w2), _p(offsets), _p(sorted_tok),
                                   _p(act), _p(y), c_int(t), c_int(k), c_int(n_experts),
                                   c_int(hidden), c_int(inter), _stream())
     _check(rc, "moe_mfma")

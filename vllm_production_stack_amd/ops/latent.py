@@ -559,7 +559,7 @@ def moe_units(x, w13, w2, ids, act: str = "silu", bucket: bool = False):
     o = _ops()
     t, k = ids.shape
     if act == "silu" and moe_units_grouped(x, w13, w2):
-        if t <= o.MOE_MFMA_MAX_TOKENS and o.moe_mfma_supported(x.shape[1], w2.shape[2]):
+        if o.moe_streams_experts(t, k, w13.shape[0]) and o.moe_mfma_supported(x.shape[1], w2.shape[2]):
             return o.moe_experts_grouped(x, w13, w2, ids, None, foreign=bucket, combine=False)
         return o.moe_experts_prefill(x, w13, w2, ids, None, foreign=bucket, combine=False)
     offsets, pos, sorted_tok = o.moe_align(ids, w13.shape[0] + (1 if bucket else 0))
@@ -612,12 +612,12 @@ def moe_glu_grouped(x, w13, w2, ids, limit: float, alpha: float = 1.702, up_bias
     offsets, pos, sorted_tok, *sw = o.moe_align(ids, w13.shape[0], scale)
     sw = sw[0] if sw else None
     hidden, inter = x.shape[1], w2.shape[2]
-    if t <= o.MOE_MFMA_MAX_TOKENS and o.moe_mfma_supported(hidden, inter) and limit > 0:
+    if o.moe_streams_experts(t, k, w13.shape[0]) and o.moe_mfma_supported(hidden, inter) and limit > 0:
         # decode-sized batches: each routed unit's weights streamed once against its few tokens
         # (the kernels of the top-k softmax mixtures, with this unit's activation)
         act = torch.empty((t * k, inter), dtype=x.dtype, device=x.device)
         y = torch.empty((t * k, hidden), dtype=x.dtype, device=x.device)
-        o._check(o._kernels().vpsa_moe_mfma_act(o._p(x), o._p(w13), o._p(w2), o._p(offsets), o._p(sorted_tok), o._p(act),
+        o._check(o._kernels().vpsa_moe_mfma_act(o._p(o._rows16(x)), o._p(w13), o._p(w2), o._p(offsets), o._p(sorted_tok), o._p(act),
                                                 o._p(y), c_int(t), c_int(k), c_int(w13.shape[0]), c_int(hidden),
                                                 c_int(inter), c_float(limit), c_float(alpha), c_float(up_bias),
                                                 o._p(sw), o._stream()), "moe_mfma_act")
