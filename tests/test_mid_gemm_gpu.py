@@ -69,3 +69,20 @@ def test_experts(tokens, routing):
         want += wt[:, j:j + 1].double() * torch.stack([w2[c].double() @ act[t] for t, c in enumerate(ids[:, j].tolist())])
     # activations, unit outputs and result rounded to 16 bits: 2^-9 of the norm each
     assert float((got.double() - want).norm() / want.norm()) < 6e-3
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 256, 1024), (3, 1280, 1088), (16, 4096, 1024), (17, 5120, 1088), (40, 8192, 2624), (130, 128, 1088)])
+def test_sum_with_residual_and_norm(any_shape, m, n, k):
+    """One reduction against the separate passes: the same roundings, so the residual stream is equal and the norm differs by its
+    sum of squares' order (one unit in the last place of 16 bits)."""
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=DEV).to(BF)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF)
+    res, ln = torch.randn(m, n, generator=g, device=DEV).to(BF), torch.randn(n, generator=g, device=DEV).to(BF)
+    want_res = res.clone()
+    want = ops.rms_norm(ops._mid_gemm(x, w, None, False), ln, 1e-5, want_res)
+    got = ops.linear_add_norm(x, w, res, ln, 1e-5)
+    assert got is not None and torch.equal(res, want_res)
+    assert float(((got.float() - want.float()).abs() - want.float().abs() * 2 ** -7).max()) <= 0
+    kept = res.clone()
+    assert ops.linear_add_norm(x[:, 1:], w[:, 1:].contiguous(), res, ln, 1e-5) is None and torch.equal(res, kept)

@@ -273,6 +273,17 @@ class TransformerModel:
             return self._lora(name, layer, x, h, meta)
         return tp_all_reduce(self._lora(name, layer, x, ops.linear(x, w, None, packed), meta))
 
+    def _out_norm(self, name: str, layer: int, x: torch.Tensor, w: torch.Tensor, packed, residual: torch.Tensor,
+                  norm: torch.Tensor, meta: BatchMeta) -> torch.Tensor:
+        """An output projection, its all-reduce, the residual stream's update and the norm that reads it next."""
+        eps = self.cfg.norm_eps
+        if self.tp_size == 1 and packed is None and (self.lora is None or meta.lora_slots is None):
+            y = ops.linear_add_norm(x, w, residual, norm, eps)
+            if y is not None:
+                return y
+        h = self._out_proj(name, layer, x, w, packed, residual, meta)
+        return ops.rms_norm(residual, norm, eps) if h is None else ops.rms_norm(h, norm, eps, residual)
+
     def _lora(self, name: str, layer: int, x: torch.Tensor, y: torch.Tensor, meta: BatchMeta):
         if self.lora is not None and meta.lora_slots is not None:
             self.lora.apply(name, layer, x, y, meta.lora_slots)
@@ -291,9 +302,13 @@ class TransformerModel:
             h = pp_recv(shape, self.dtype, self.device, pp.prev)
             residual = pp_recv(shape, self.dtype, self.device, pp.prev)
         decode_only = meta.num_prefill_seqs == 0
+        adapters = self.lora is not None and meta.lora_slots is not None
+        x = None  # the norm the next layer starts with, where the projection before it made it
         for li, lw in enumerate(self.layers):
             gl = self.first_layer + li  # global layer index (adapters are keyed by it)
-            if residual is None:
+            if x is not None:
+                pass
+            elif residual is None:
                 residual = h
                 x = ops.rms_norm(h, lw.ln1, cfg.norm_eps)
             elif h is None:  # the previous projection's epilogue already updated the residual stream
@@ -302,19 +317,20 @@ class TransformerModel:
                 x = ops.rms_norm(h, lw.ln1, cfg.norm_eps, residual)
             qkv = self._lora("qkv", gl, x, ops.qkv_linear(x, lw.wqkv, lw.bqkv, self.n_q * self.head_dim), meta)
             attn = self._attention(qkv, pool, li, meta)
-            h = self._out_proj("o", gl, attn, lw.wo, None, residual, meta)
-            x = ops.rms_norm(residual, lw.ln2, cfg.norm_eps) if h is None else ops.rms_norm(h, lw.ln2, cfg.norm_eps, residual)
+            x = self._out_norm("o", gl, attn, lw.wo, None, residual, lw.ln2, meta)
             if cfg.num_experts > 0:
-                h = self._moe(x, lw, decode_only)
+                h, x = tp_all_reduce(self._moe(x, lw, decode_only)), None
+                continue
+            if adapters:
+                gu = self._lora("gate_up", gl, x, F.linear(x, lw.w_gate_up), meta)
+                act = ops.silu_and_mul(gu)
             else:
-                if self.lora is not None and meta.lora_slots is not None:
-                    gu = self._lora("gate_up", gl, x, F.linear(x, lw.w_gate_up), meta)
-                    act = ops.silu_and_mul(gu)
-                else:
-                    act = ops.gate_up_silu(x, lw.w_gate_up, lw.w_gate_up_p if decode_only else None)
-                h = self._out_proj("down", gl, act, lw.w_down, lw.w_down_p if decode_only else None, residual, meta)
-            if cfg.num_experts > 0:
-                h = tp_all_reduce(h)
+                act = ops.gate_up_silu(x, lw.w_gate_up, lw.w_gate_up_p if decode_only else None)
+            packed = lw.w_down_p if decode_only else None
+            if li + 1 < len(self.layers):
+                x = self._out_norm("down", gl, act, lw.w_down, packed, residual, self.layers[li + 1].ln1, meta)
+            else:
+                h, x = self._out_proj("down", gl, act, lw.w_down, packed, residual, meta), None
         if not pp.is_last:
             if h is None:  # the last projection added itself into the residual stream
                 h = torch.zeros_like(residual)

@@ -41,7 +41,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -702,22 +702,42 @@ def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
     return 0
 
 
-def _mid_gemm(x2, w, bias, pair):
-    """Projection of up to a few hundred rows (``csrc/kernels/mid_gemm.hip``), or None where another kernel is the better choice."""
+def _mid_takes(x2, w, bias, pair) -> int:
+    """``_mid_splits`` for operands that ``mid_gemm`` reads, else 0."""
     if not (_skinny_enabled and x2.is_cuda and x2.dim() == 2 and x2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
             and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1]))
             and not (torch.is_grad_enabled() and (x2.requires_grad or w.requires_grad))):
+        return 0
+    return _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair)
+
+
+def _mid_gemm(x2, w, bias, pair):
+    """Projection of up to a few hundred rows (``csrc/kernels/mid_gemm.hip``), or None where another kernel is the better choice."""
+    splits = _mid_takes(x2, w, bias, pair)
+    if not splits:
         return None
     m, n, k = x2.shape[0], w.shape[0], w.shape[1]
-    splits = _mid_splits(m, n, k, pair)
-    if splits <= 0:
-        return None
     out = torch.empty((m, n // 2 if pair else n), dtype=x2.dtype, device=x2.device)
     ws = torch.empty((splits * m * n,), dtype=torch.float32, device=x2.device) if splits > 1 else None
     rc = _kernels().vpsa_mid_gemm(_p(x2), c_long(x2.stride(0)), _p(w), _p(bias), _p(out), c_long(out.stride(0)), _p(ws), c_int(m),
                                   c_int(n), c_int(k), c_int(1 if pair else 0), c_int(splits), _stream())
     return out if rc == 0 else None
+
+
+def linear_add_norm(x, w, residual, weight, eps):
+    """``residual += x @ w.T`` and the norm of the new rows, ``rmsnorm(residual) * weight``, when ``mid_gemm`` splits the product: its
+    reduction then makes both.  None (and nothing done) otherwise."""
+    splits = _mid_takes(x, w, None, False)
+    m, n = x.shape[0], w.shape[0]
+    if (splits < 2 or n > 8192 or residual.shape != (m, n) or residual.dtype != torch.bfloat16 or not residual.is_contiguous()
+            or weight.dtype != torch.bfloat16 or weight.shape != (n,) or not weight.is_contiguous()):
+        return None
+    y = torch.empty_like(residual)
+    ws = torch.empty((splits * m * n,), dtype=torch.float32, device=x.device)
+    rc = _kernels().vpsa_mid_gemm_norm(_p(x), c_long(x.stride(0)), _p(w), _p(residual), _p(weight), _p(y), _p(ws), c_int(m), c_int(n),
+                                       c_int(w.shape[1]), c_int(splits), c_float(eps), _stream())
+    return y if rc == 0 else None
 
 
 def pack_weight(w: torch.Tensor) -> torch.Tensor:
