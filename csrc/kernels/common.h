@@ -34,6 +34,10 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// Rotary embedding of channels (x, y) = (i, i + 64); the products' order is written out so that every kernel rounds it alike.
+__device__ __forceinline__ float rope_lo(float x, float y, float c, float s) { return fmaf(x, c, -(y * s)); }
+__device__ __forceinline__ float rope_hi(float x, float y, float c, float s) { return fmaf(x, s, y * c); }
+
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

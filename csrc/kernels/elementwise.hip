@@ -137,8 +137,8 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(
     if (h < n_q + n_kv) {
       if (rotary) {
         const float x0 = bf16lo(lo), x1 = bf16hi(lo), y0 = bf16lo(hi), y1 = bf16hi(hi);
-        lo = pack_bf16x2(x0 * c.x - y0 * s.x, x1 * c.y - y1 * s.y);
-        hi = pack_bf16x2(y0 * c.x + x0 * s.x, y1 * c.y + x1 * s.y);
+        lo = pack_bf16x2(rope_lo(x0, y0, c.x, s.x), rope_lo(x1, y1, c.y, s.y));
+        hi = pack_bf16x2(rope_hi(x0, y0, c.x, s.x), rope_hi(x1, y1, c.y, s.y));
         p[j] = lo;
         p[32 + j] = hi;
       }

@@ -86,3 +86,24 @@ def test_sum_with_residual_and_norm(any_shape, m, n, k):
     assert float(((got.float() - want.float()).abs() - want.float().abs() * 2 ** -7).max()) <= 0
     kept = res.clone()
     assert ops.linear_add_norm(x[:, 1:], w[:, 1:].contiguous(), res, ln, 1e-5) is None and torch.equal(res, kept)
+
+
+@pytest.mark.parametrize("m,n_q,n_kv,bias", [(1, 32, 8, False), (3, 5, 1, True), (17, 8, 8, True), (40, 32, 8, False)])
+def test_sum_with_rotation_and_cache_write(any_shape, m, n_q, n_kv, bias):
+    """Query rows and the pages that a decode step's projection leaves against the separate passes, one row without a slot."""
+    g = torch.Generator(device=DEV).manual_seed(m)
+    k, n = 1088, (n_q + 2 * n_kv) * 128
+    x = torch.randn(m, k, generator=g, device=DEV).to(BF)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF)
+    b = torch.randn(n, generator=g, device=DEV).to(BF) if bias else None
+    pages = m + 2
+    pool = torch.randn(pages, 2, 2, n_kv * 64 * 128, generator=g, device=DEV).to(BF)
+    positions = torch.randint(0, 500, (m,), generator=g, device=DEV, dtype=torch.int32)
+    slots = torch.randperm(pages * 64, generator=g, device=DEV)[:m]
+    slots[m // 2] = slots[m // 2] if m == 1 else -1
+    ang = torch.rand(500, 64, generator=g, device=DEV) * 6.28
+    cos_sin = torch.cat([ang.cos(), ang.sin()], dim=1).contiguous()
+    want_pool, qkv = pool.clone(), ops._mid_gemm(x, w, b, False)
+    ops.rope_and_cache(qkv, positions, slots, cos_sin, want_pool, 1, n_q, n_kv, 128)
+    q = ops.decode_qkv(x, w, b, pool, 1, positions, slots, cos_sin, n_q, n_kv)
+    assert torch.equal(q, qkv[:, :n_q * 128]) and torch.equal(pool, want_pool)

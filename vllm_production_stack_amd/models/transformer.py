@@ -315,8 +315,13 @@ class TransformerModel:
                 x = ops.rms_norm(residual, lw.ln1, cfg.norm_eps)
             else:
                 x = ops.rms_norm(h, lw.ln1, cfg.norm_eps, residual)
-            qkv = self._lora("qkv", gl, x, ops.qkv_linear(x, lw.wqkv, lw.bqkv, self.n_q * self.head_dim), meta)
-            attn = self._attention(qkv, pool, li, meta)
+            attn = None
+            if decode_only and not adapters:
+                attn = ops.decode_attention_block(x, lw.wqkv, lw.bqkv, pool, li, meta, self.n_q, self.n_kv, self.head_dim,
+                                                  self.scale, self.cos_sin)
+            if attn is None:
+                qkv = self._lora("qkv", gl, x, ops.qkv_linear(x, lw.wqkv, lw.bqkv, self.n_q * self.head_dim), meta)
+                attn = self._attention(qkv, pool, li, meta)
             x = self._out_norm("o", gl, attn, lw.wo, None, residual, lw.ln2, meta)
             if cfg.num_experts > 0:
                 h, x = tp_all_reduce(self._moe(x, lw, decode_only)), None

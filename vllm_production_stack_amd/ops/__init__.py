@@ -41,7 +41,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -738,6 +738,41 @@ def linear_add_norm(x, w, residual, weight, eps):
     rc = _kernels().vpsa_mid_gemm_norm(_p(x), c_long(x.stride(0)), _p(w), _p(residual), _p(weight), _p(y), _p(ws), c_int(m), c_int(n),
                                        c_int(w.shape[1]), c_int(splits), c_float(eps), _stream())
     return y if rc == 0 else None
+
+
+def decode_qkv(x, w, bias, pool, layer, positions, slots, cos_sin, n_q, n_kv):
+    """q / k / v projection, rotary embedding and cache write of one token per sequence, when ``mid_gemm`` splits the projection: its
+    reduction then rotates and writes the cache.  The query rows [T, n_q * 128], or None (and nothing done) otherwise."""
+    splits = _mid_takes(x, w, bias, False)
+    m = x.shape[0]
+    if splits < 2 or pool.dtype != torch.bfloat16 or w.shape[0] != (n_q + 2 * n_kv) * HEAD_DIM_HIP:
+        return None
+    assert positions.dtype == torch.int32 and slots.dtype == torch.int64 and positions.shape[0] >= m and slots.shape[0] >= m
+    assert cos_sin.dtype == torch.float32 and cos_sin.shape[1] == HEAD_DIM_HIP
+    q = torch.empty((m, n_q * HEAD_DIM_HIP), dtype=x.dtype, device=x.device)
+    ws = torch.empty((splits * m * w.shape[0],), dtype=torch.float32, device=x.device)
+    base = pool.data_ptr() + layer * pool.stride(1) * 2
+    rc = _kernels().vpsa_mid_gemm_qkv(_p(x), c_long(x.stride(0)), _p(w), _p(bias), _p(q), _p(ws), c_int(m), c_int(w.shape[1]),
+                                      c_int(splits), _p(positions), _p(slots), _p(cos_sin), c_void_p(base), c_long(pool.stride(0)),
+                                      c_long(pool.stride(2)), c_int(n_q), c_int(n_kv), _stream())
+    return q if rc == 0 else None
+
+
+def decode_attention_block(x, w, bias, pool, layer, meta, n_q, n_kv, head_dim, scale, cos_sin):
+    """Projection, rotary embedding, cache write and attention of a decode-only step where ``decode_qkv`` takes the first three.
+    [T, n_q * head_dim], or None (and nothing done) otherwise."""
+    if isinstance(pool, LayerGroupedPool):
+        pool, layer = pool.for_layer(layer)
+    if (meta.num_prefill_seqs > 0 or meta.num_decode != x.shape[0] or meta.slots is None or head_dim != HEAD_DIM_HIP
+            or _generic_attention(x, head_dim)):
+        return None
+    q = decode_qkv(x, w, bias, pool, layer, meta.positions, meta.slots, cos_sin, n_q, n_kv)
+    if q is None:
+        return None
+    out = torch.empty_like(q)
+    paged_decode(q, out, pool, layer, meta.dec_block_tables, meta.dec_ctx_lens, n_q, n_kv, head_dim, scale,
+                 getattr(meta, "dec_num_splits", 1) or 1, getattr(meta, "dec_ws_o", None), getattr(meta, "dec_ws_ml", None))
+    return out
 
 
 def pack_weight(w: torch.Tensor) -> torch.Tensor:
