@@ -103,6 +103,92 @@ VPSA_EXPORT int vpsa_rmsnorm(const void* x, void* residual, const void* w, void*
 }
 
 // ---------------------------------------------------------------------------------
+// y = layer norm(x [+ residual]) * w + b; residual is updated in place with the sum.  Bytes bound
+// it: a wave holds a row in registers (CHUNKS runs of 8 channels a lane), so x and the residual are
+// read once and mean and variance (of the deviations, in 32 bits) cost no second pass.  Four rows a
+// workgroup.  12000 rows of 768: 12.2 us with the residual, where the sum (9.2) and the library's
+// norm (21.2) were two launches; 8 rows 2.8 and 5.0; 12 speech layers of 8 windows 5.11 -> 4.69 ms.
+// ---------------------------------------------------------------------------------
+template <int CHUNKS>
+__global__ __launch_bounds__(256) void layernorm_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ residual,
+                                                        const uint16_t* __restrict__ w, const uint16_t* __restrict__ b,
+                                                        uint16_t* __restrict__ y, int rows, int hidden, long x_stride,
+                                                        float eps) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const uint16_t* xr = x + (long)row * x_stride;
+  uint16_t* rr = residual ? residual + (long)row * hidden : nullptr;
+  float v[CHUNKS][8];
+  u32x4 ww[CHUNKS], bb[CHUNKS];
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = (c * 64 + lane) * 8;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[c][k] = 0.f;
+    if (i >= hidden) continue;
+    const u32x4 a = *reinterpret_cast<const u32x4*>(xr + i);
+    ww[c] = *reinterpret_cast<const u32x4*>(w + i);
+    bb[c] = *reinterpret_cast<const u32x4*>(b + i);
+    u32x4 o = a;
+    if (rr) {
+      const u32x4 old = *reinterpret_cast<const u32x4*>(rr + i);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = pack_bf16x2(bf16lo(a[k]) + bf16lo(old[k]), bf16hi(a[k]) + bf16hi(old[k]));
+      *reinterpret_cast<u32x4*>(rr + i) = o;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[c][2 * k] = bf16lo(o[k]);
+      v[c][2 * k + 1] = bf16hi(o[k]);
+      sum += v[c][2 * k] + v[c][2 * k + 1];
+    }
+  }
+  const float mean = wave_reduce_sum(sum) / (float)hidden;
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c)
+    if ((c * 64 + lane) * 8 < hidden)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        v[c][k] -= mean;
+        ss += v[c][k] * v[c][k];
+      }
+  const float inv = rsqrtf(wave_reduce_sum(ss) / (float)hidden + eps);
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = (c * 64 + lane) * 8;
+    if (i >= hidden) continue;
+    u32x4 o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      o[k] = pack_bf16x2(fmaf(v[c][2 * k] * inv, bf16lo(ww[c][k]), bf16lo(bb[c][k])),
+                         fmaf(v[c][2 * k + 1] * inv, bf16hi(ww[c][k]), bf16hi(bb[c][k])));
+    *reinterpret_cast<u32x4*>(y + (long)row * hidden + i) = o;
+  }
+}
+
+// x [rows, hidden] (row stride x_stride elements), residual / y contiguous or residual null; 16-byte aligned rows, hidden a
+// multiple of 8 up to 2048.
+VPSA_EXPORT int vpsa_layernorm(const void* x, void* residual, const void* w, const void* b, void* y, int rows, int hidden,
+                               long x_stride, float eps, hipStream_t stream) {
+  if (rows <= 0) return 0;
+  if (hidden <= 0 || hidden % 8 != 0 || hidden > 2048 || (x_stride & 7)) return -1;
+  if (((uintptr_t)x | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)b | (uintptr_t)y) & 15) return -1;
+#define LAUNCH(C)                                                                                                     \
+  hipLaunchKernelGGL(layernorm_kernel<C>, dim3((rows + 3) / 4), dim3(256), 0, stream, (const uint16_t*)x,             \
+                     (uint16_t*)residual, (const uint16_t*)w, (const uint16_t*)b, (uint16_t*)y, rows, hidden, x_stride, eps)
+  switch ((hidden + 511) / 512) {
+    case 1: LAUNCH(1); break;
+    case 2: LAUNCH(2); break;
+    case 3: LAUNCH(3); break;
+    default: LAUNCH(4); break;
+  }
+#undef LAUNCH
+  return 0;
+}
+
+// ---------------------------------------------------------------------------------
 // Rotary embedding (NeoX pairing: channel i rotates with i + 64) applied in place to the
 // Q and K heads of a fused QKV activation, fused with the paged KV-cache write.
 //   qkv        [tokens, (n_q + 2 n_kv) * 128] bf16, row stride qkv_stride

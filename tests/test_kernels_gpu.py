@@ -1163,3 +1163,20 @@ def test_lora_shrink_expand_mixed_adapters(t, in_dim, outs, r_pad):
     torch.testing.assert_close(y.float(), y_ref.float(), atol=3e-2, rtol=2e-2)
     assert torch.equal(y[~has], y0[~has])  # rows without an adapter are untouched
     assert torch.equal(y[:, off:], y0[:, off:])
+
+
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 384), (5, 512), (4, 520), (13, 768), (6, 1280), (9, 2048)])
+@pytest.mark.parametrize("add", [False, True])
+def test_layer_norm_matches_float64(rows, hidden, add):
+    """Rows and channels around a wave's runs, an offset that a one-pass variance would lose, strided rows, the sum in place."""
+    g = torch.Generator(device=DEV).manual_seed(rows + hidden)
+    x = (torch.randn(rows, hidden + 8, generator=g, device=DEV) + 30).to(BF)[:, :hidden]
+    w, b = torch.randn(hidden, generator=g, device=DEV).to(BF), torch.randn(hidden, generator=g, device=DEV).to(BF)
+    res = torch.randn(rows, hidden, generator=g, device=DEV).to(BF) if add else None
+    s = x if res is None else x + res
+    want = torch.nn.functional.layer_norm(s.double(), (hidden,), w.double(), b.double(), 1e-5)
+    with torch.no_grad():
+        got = ops.layer_norm(x, w, b, 1e-5, res)
+    assert res is None or torch.equal(res, s)
+    # one rounding to 16 bits (2^-9 of the value); 32-bit sums of values near 30 are off by 30 * 2^-22 of a deviation near 1
+    assert float(((got.double() - want).abs() - want.abs() * 2 ** -8 - 2e-4).max()) < 0

@@ -331,8 +331,9 @@ class WhisperModel:
         return sum(t.numel() * t.element_size() for t in self.w.values())
 
     # ------------------------------------------------------------------ blocks
-    def _ln(self, x, prefix):
-        return F.layer_norm(x, (x.shape[-1],), self.w[prefix + ".weight"], self.w[prefix + ".bias"], 1e-5)
+    def _ln(self, x, prefix, residual=None):
+        """Layer norm of ``x``, or of ``residual`` after ``x`` has been added to it in place."""
+        return ops.layer_norm(x, self.w[prefix + ".weight"], self.w[prefix + ".bias"], 1e-5, residual)
 
     def _lin(self, x, prefix):
         return F.linear(x, self.w[prefix + ".weight"], self.w.get(prefix + ".bias"))
@@ -368,14 +369,14 @@ class WhisperModel:
         x = F.gelu(self._conv3(mel.to(self.dtype).transpose(1, 2), "encoder.conv1", 1))
         x = F.gelu(self._conv3(x, "encoder.conv2", 2))
         x = x + w["encoder.embed_positions.weight"][: x.shape[1]]
+        h = None
         for i in range(c.encoder_layers):
             p = f"encoder.layers.{i}"
-            h = self._ln(x, p + ".self_attn_layer_norm")
+            h = self._ln(x, p + ".self_attn_layer_norm") if h is None else self._ln(h, p + ".self_attn_layer_norm", x)
             a = _attend(self._lin(h, p + ".self_attn.q_proj"), self._lin(h, p + ".self_attn.k_proj"),
                         self._lin(h, p + ".self_attn.v_proj"), c.encoder_heads)
-            x = x + self._lin(a, p + ".self_attn.out_proj")
-            x = x + self._mlp(self._ln(x, p + ".final_layer_norm"), p)
-        return self._ln(x, "encoder.layer_norm")
+            h = self._mlp(self._ln(self._lin(a, p + ".self_attn.out_proj"), p + ".final_layer_norm", x), p)
+        return self._ln(x, "encoder.layer_norm") if h is None else self._ln(h, "encoder.layer_norm", x)
 
     @torch.inference_mode()
     def cross_kv(self, enc: torch.Tensor) -> list[tuple[torch.Tensor, torch.Tensor]]:
@@ -410,11 +411,9 @@ class WhisperModel:
                 v_all = torch.cat([cache[i][1], v_new], dim=1)
             cache[i] = (k_all, v_all)
             a = _attend(self._lin(h, p + ".self_attn.q_proj"), k_all, v_all, c.decoder_heads, mask)
-            x = x + self._lin(a, p + ".self_attn.out_proj")
-            h = self._ln(x, p + ".encoder_attn_layer_norm")
+            h = self._ln(self._lin(a, p + ".self_attn.out_proj"), p + ".encoder_attn_layer_norm", x)
             a = _attend(self._lin(h, p + ".encoder_attn.q_proj"), cross[i][0], cross[i][1], c.decoder_heads)
-            x = x + self._lin(a, p + ".encoder_attn.out_proj")
-            x = x + self._mlp(self._ln(x, p + ".final_layer_norm"), p)
+            x = x + self._mlp(self._ln(self._lin(a, p + ".encoder_attn.out_proj"), p + ".final_layer_norm", x), p)
         x = self._ln(x[:, -1], "decoder.layer_norm")
         return F.linear(x, w["decoder.embed_tokens.weight"]).float()
 
@@ -496,11 +495,10 @@ class WhisperModel:
             kc, vc = st["kc"][i][:b], st["vc"][i][:b]
             kc.index_copy_(1, pos, qkv[:, None, d:2 * d])
             vc.index_copy_(1, pos, qkv[:, None, 2 * d:])
-            x = x + lin(self._attend1(qkv[:, :d], kc, vc, pos, mask), p + ".self_attn.out_proj")
-            h = self._ln(x, p + ".encoder_attn_layer_norm")
+            h = self._ln(lin(self._attend1(qkv[:, :d], kc, vc, pos, mask), p + ".self_attn.out_proj"),
+                         p + ".encoder_attn_layer_norm", x)
             a = self._attend1(lin(h, p + ".encoder_attn.q_proj"), st["ck"][i][:b], st["cv"][i][:b], None, None)
-            x = x + lin(a, p + ".encoder_attn.out_proj")
-            h = self._ln(x, p + ".final_layer_norm")
+            h = self._ln(lin(a, p + ".encoder_attn.out_proj"), p + ".final_layer_norm", x)
             x = x + lin(F.gelu(lin(h, p + ".fc1")), p + ".fc2")
         logits = ops.linear(self._ln(x, "decoder.layer_norm"), w["decoder.embed_tokens.weight"]).float()
         logits.masked_fill_(st["suppress"], float("-inf"))

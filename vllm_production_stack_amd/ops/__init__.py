@@ -41,7 +41,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -137,6 +137,25 @@ def rms_norm(x, weight, eps, residual=None, out=None):
                                  c_float(eps), _stream())
     _check(rc, "rms_norm")
     return out.view(x.shape)
+
+
+def layer_norm(x, weight, bias, eps, residual=None):
+    """y = layer norm(x [+ residual]) * weight + bias.  ``residual`` (contiguous) is updated in place with the sum."""
+    hidden = x.shape[-1]
+    ts = (x, weight, bias) if residual is None else (x, weight, bias, residual)
+    rows_at = x.stride(-2) if x.dim() == 2 else hidden
+    if (x.is_cuda and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts) and hidden % 8 == 0
+            and hidden <= 2048 and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and rows_at % 8 == 0))
+            and weight.is_contiguous() and bias.is_contiguous() and not torch.is_grad_enabled()
+            and (residual is None or (residual.is_contiguous() and residual.shape == x.shape))):
+        y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+        rc = _kernels().vpsa_layernorm(_p(x), _p(residual), _p(weight), _p(bias), _p(y), c_int(x.numel() // hidden), c_int(hidden),
+                                       c_long(rows_at), c_float(eps), _stream())
+        _check(rc, "layer_norm")
+        return y
+    if residual is not None:
+        x = residual.add_(x)
+    return torch.nn.functional.layer_norm(x, (hidden,), weight, bias, eps)
 
 
 # --------------------------------------------------------------------------- rope + cache write
