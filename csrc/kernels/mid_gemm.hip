@@ -463,14 +463,16 @@ static int mid_product(const void* x, long xs, const void* w, const void* bias, 
 #define MID(MT)                                                                                             \
   return pair ? launch_mid<MT, true>(x, xs, w, bias, y, ys, (float*)ws, M, N, K, S, stream)                 \
               : launch_mid<MT, false>(x, xs, w, bias, y, ys, (float*)ws, M, N, K, S, stream)
-  switch (M >= 128 ? 8 : (M + 15) / 16) {
+  // Above 96 rows the whole block of eight tiles: what bounds it there is the schedule and not the rows (7 tiles are no faster than
+  // 8 on the gated unit and slower elsewhere: steps of 97 and 110 rows behind cached tokens 3.45 and 3.12 ms with 7, 3.33 and 3.01
+  // with 8; below, 90 rows take 2.68 with 6 and 2.85 with 8, 72 rows 2.57 with 5 and 2.75).
+  switch (M > 96 ? 8 : (M + 15) / 16) {
     case 1: MID(1);
     case 2: MID(2);
     case 3: MID(3);
     case 4: MID(4);
     case 5: MID(5);
     case 6: MID(6);
-    case 7: MID(7);
     default: MID(8);
   }
 #undef MID
