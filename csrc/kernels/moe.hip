@@ -5,8 +5,8 @@
 //   3. moe_permute:      gather activation rows into expert-sorted order
 //   4. moe_combine:      out[t] = sum_k w[t,k] * y[pos[t,k]]  (gather form: no atomics, so
 //                        the result is bitwise reproducible)
-// The expert GEMMs themselves run on the matrix cores through the library GEMM on each
-// expert's contiguous row range.
+// The experts' products on those row ranges: mid_experts_kernel (mid_gemm.hip) up to 48 rows an expert on average, the
+// grouped form of tile_gemm.hip above, per-pair kernels for a single token.
 #include "common.h"
 
 #define MAX_EXPERTS 64        // top-k softmax keeps a token's scores in registers
