@@ -336,6 +336,22 @@ __device__ __forceinline__ void all_products16(f32x4* o, const s16x4& pf, const 
   (transposed_products16<J>(o, pf, at), ...);
 }
 
+// How many of `splits` key ranges a decode row of `pages` pages is cut into.  A workgroup fills a CU (two pages in LDS) and what it
+// does once - queries, the join, a partial result of 64 KB - takes about as long as four pages, so more workgroups than a
+// round of 256 only pay if their ranges are long: 100 sequences of 1000 entries in 8 ranges of two pages were four rounds.  In a
+// graph with the merge, all ranges -> those used: 100 x 1000 entries 86 -> 45 us, 40 x 3000 (7 -> 6) 64 -> 44, 33 x 12000
+// (8 -> 7) 144 -> 98, 128 x 100 37 -> 25; one sequence of 2000 keeps its 32 and its 26.
+constexpr int WIDE_ONCE = 4;
+__device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
+  int best = 1 << 30, used = splits;
+  for (int r = 1; rows * splits > 256; ++r) {
+    const int e = min(splits, max(1, r * 256 / rows)), cost = (rows * e + 255) / 256 * ((pages + e - 1) / e + WIDE_ONCE);
+    if (cost < best) best = cost, used = e;
+    if (e == splits) break;
+  }
+  return used;
+}
+
 template <int RANK, int ROT, int KSPLIT>
 __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void latent_wide_kernel(
     const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
@@ -373,8 +389,17 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
   const int my_pos = valid ? t.pos0 + tok : -1;
   const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
   const int p_first = max(0, t.pos0 - window + 1) / PAGE;
-  const int per = (n_pages - p_first + splits - 1) / splits;
+  const int used = tiles ? splits : wide_splits(n_pages - p_first, gridDim.x, splits);
+  const int per = (n_pages - p_first + used - 1) / used;
   const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
+  if (splits > 1 && p_begin >= p_end) {  // nothing to see: the merge passes over the record
+    if (tid < t.n_tok * t.hcount) {
+      const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + tid;
+      ws_ml[2 * rec] = -INFINITY;
+      ws_ml[2 * rec + 1] = 0.f;
+    }
+    return;
+  }
   const int my_first = my_pos - window;
   const int* bt = block_tables + (long)t.seq * bt_stride;
 
@@ -588,8 +613,9 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(const float* __restri
       f32x4 v[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        v[i] = s0 + i < splits ? *reinterpret_cast<const f32x4*>(ws_o + (rec0 + 64L * (s0 + i)) * rank + d)
-                               : (f32x4){0.f, 0.f, 0.f, 0.f};
+        v[i] = s0 + i < splits && fac[s0 + i] != 0.f
+                   ? *reinterpret_cast<const f32x4*>(ws_o + (rec0 + 64L * (s0 + i)) * rank + d)
+                   : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float f = s0 + i < splits ? fac[s0 + i] : 0.f;

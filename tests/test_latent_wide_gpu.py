@@ -51,6 +51,17 @@ def test_decode_rows(heads, splits, window):
     assert float((out.double() - want).norm() / want.norm()) < 6e-3
 
 
+@pytest.mark.parametrize("heads,rows,splits,window", [(16, 43, 6, 1 << 30), (32, 100, 8, 1 << 30), (64, 33, 8, 1 << 30), (16, 90, 3, 200), (70, 300, 2, 64)])
+def test_decode_batches_beyond_a_round(heads, rows, splits, window):
+    """More workgroups than CUs: fewer ranges are used than the caller's workspace holds, and some rows see one page or one key."""
+    ctx = [1 + (37 * i * i) % 900 for i in range(rows)]
+    pool, table, q, sink = setup(ctx, [1] * rows, heads, rows)
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    out = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, None, pos, sink, 0.05, splits=splits, window=window)
+    want = expected(pool, table, q, sink, ctx, [1] * rows, 0.05, window)
+    assert float((out.double() - want).norm() / want.norm()) < 6e-3   # as above
+
+
 @pytest.mark.parametrize("heads", [3, 16, 64])
 def test_prefill_tiles(heads):
     ctx, rows_of = [70, 500, 130], [70, 33, 1]
