@@ -341,6 +341,8 @@ __device__ __forceinline__ void all_products16(f32x4* o, const s16x4& pf, const 
 // round of 256 only pay if their ranges are long: 100 sequences of 1000 entries in 8 ranges of two pages were four rounds.  In a
 // graph with the merge, all ranges -> those used: 100 x 1000 entries 86 -> 45 us, 40 x 3000 (7 -> 6) 64 -> 44, 33 x 12000
 // (8 -> 7) 144 -> 98, 128 x 100 37 -> 25; one sequence of 2000 keeps its 32 and its 26.
+// `rows` are those of the step's batch bucket, not of the launch: a row's ranges, and with them the order of its sums, are the same
+// in a captured step that is padded to the bucket and in an eager one that is not.
 constexpr int WIDE_ONCE = 4;
 __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   int best = 1 << 30, used = splits;
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
     int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
     const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
-    int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+    int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
   constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, DT = RANK / 16, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW;
   static_assert(KSPLIT == 1 || KSPLIT == 4, "all keys or a quarter of them");
   constexpr int WAVES = KSPLIT == 4 ? 8 : 4;
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
   const int my_pos = valid ? t.pos0 + tok : -1;
   const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
   const int p_first = max(0, t.pos0 - window + 1) / PAGE;
-  const int used = tiles ? splits : wide_splits(n_pages - p_first, gridDim.x, splits);
+  const int used = tiles ? splits : wide_splits(n_pages - p_first, bucket, splits);
   const int per = (n_pages - p_first + used - 1) / used;
   const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
   if (splits > 1 && p_begin >= p_end) {  // nothing to see: the merge passes over the record
@@ -631,28 +633,31 @@ template <int RANK, int ROT, bool ROT_ONLY>
 int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long qr_row, long qr_head,
            const void* cache, long page_stride, const int* block_tables, int bt_stride, const int* tiles,
            const int* positions, int n_tiles, int heads, const float* sink, void* out, long o_row, long o_head,
-           float scale, int window, int splits, float* ws_o, float* ws_ml, hipStream_t st) {
+           float scale, int window, int splits, float* ws_o, float* ws_ml, int bucket, hipStream_t st) {
   // entries of 512 + 64 values: pages straight into LDS (narrower ones keep three waves per SIMD in the kernel above)
-  constexpr bool WIDE = !ROT_ONLY && RANK == 512 && ROT == 64;
-  decltype(&latent_mfma_kernel<32, 64, true>) kernel;  // (both kernels take the same arguments)
-  int lds = 64 * ((ROT_ONLY ? ROT : RANK + ROT) * 2 + 16) + RANK * (64 * 2 + 16);
   static bool attr_set[2] = {false, false};
-  int which = 0;
-  if constexpr (WIDE) {
-    which = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
-    kernel = which ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 1>;
-    lds = 2 * 64 * (RANK + ROT) * 2;
+  auto ready = [](const void* kernel, int lds, bool* done) {
+    if (!*done) *done = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+    return *done;
+  };
+  if constexpr (!ROT_ONLY && RANK == 512 && ROT == 64) {
+    constexpr int LDS = 2 * 64 * (RANK + ROT) * 2;
+    const int quarters = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
+    const auto kernel = quarters ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 1>;
+    if (!ready((const void*)kernel, LDS, &attr_set[quarters])) return -2;
+    kernel<<<dim3(n_tiles, splits), dim3(quarters ? 512 : 256), LDS, st>>>(
+        (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
+        page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
+        window, splits, ws_o, ws_ml, bucket);
   } else {
-    kernel = latent_mfma_kernel<RANK, ROT, ROT_ONLY>;
+    constexpr int LDS = 64 * ((ROT_ONLY ? ROT : RANK + ROT) * 2 + 16) + RANK * (64 * 2 + 16);
+    const auto kernel = latent_mfma_kernel<RANK, ROT, ROT_ONLY>;
+    if (!ready((const void*)kernel, LDS, &attr_set[0])) return -2;
+    kernel<<<dim3(n_tiles, splits), dim3(256), LDS, st>>>(
+        (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
+        page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
+        window, splits, ws_o, ws_ml);
   }
-  if (!attr_set[which]) {
-    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
-    attr_set[which] = true;
-  }
-  kernel<<<dim3(n_tiles, splits), dim3(which ? 512 : 256), lds, st>>>(
-      (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
-      page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
-      window, splits, ws_o, ws_ml);
   if (splits > 1)
     latent_merge_kernel<<<dim3(n_tiles, tiles ? 64 : min(heads, 64)), dim3(128), 0, st>>>(
         ws_o, ws_ml, tiles, heads, sink, (uint16_t*)out, o_row, o_head, splits, RANK);
@@ -688,14 +693,16 @@ VPSA_EXPORT int vpsa_latent_mfma_expanded(int rank, int rot) {
 // (n_tiles = rows * ceil(heads / 64), positions [rows]).  Row and head strides in elements; every query
 // and output vector 16-byte / 8-byte aligned.  q_lat null: see ROT_ONLY above.  window >= 1 (a query sees itself and the window - 1 entries before
 // it; any window of at least the context length is plain causal attention).  splits > 1 needs ws_o [n_tiles * splits * 64 * rank] and
-// ws_ml [n_tiles * splits * 64 * 2] floats.
+// ws_ml [n_tiles * splits * 64 * 2] floats.  bucket: the n_tiles that the choice of a decode row's key ranges goes by, where that is
+// more than this launch's.
 VPSA_EXPORT int vpsa_latent_attention_mfma(const void* q_lat, long ql_row, long ql_head, const void* q_rot,
                                            long qr_row, long qr_head, const void* cache, long page_stride,
                                            const int* block_tables, int bt_stride, const int* tiles,
                                            const int* positions, int n_tiles, int heads, const float* sink, void* out,
                                            long o_row, long o_head, int rank, int rot, float scale, int window,
-                                           int splits, float* ws_o, float* ws_ml, hipStream_t st) {
+                                           int splits, float* ws_o, float* ws_ml, int bucket, hipStream_t st) {
   if (n_tiles <= 0) return 0;
+  if (bucket < n_tiles) bucket = n_tiles;
   if (window < 1 || splits > MERGE_MAX) return -1;
   if (splits < 1 || splits > 65535 || (splits > 1 && (!ws_o || !ws_ml)) || (!tiles && !positions)) return -1;
   if (((ql_row | ql_head | qr_row | qr_head) & 7) || ((o_row | o_head) & 3) || (page_stride & 7)) return -1;
@@ -703,7 +710,7 @@ VPSA_EXPORT int vpsa_latent_attention_mfma(const void* q_lat, long ql_row, long 
   if (!q_lat && rank == R && rot == C)                                                                              \
     return launch<R, C, true>(q_lat, ql_row, ql_head, q_rot, qr_row, qr_head, cache, page_stride, block_tables,      \
                               bt_stride, tiles, positions, n_tiles, heads, sink, out, o_row, o_head, scale, window,   \
-                              splits, ws_o, ws_ml, st);
+                              splits, ws_o, ws_ml, bucket, st);
   LAT_EXPANDED(LAT_ONLY)
 #undef LAT_ONLY
   if (!q_lat) return -1;
@@ -711,7 +718,7 @@ VPSA_EXPORT int vpsa_latent_attention_mfma(const void* q_lat, long ql_row, long 
   if (rank == R && rot == C)                                                                                        \
     return launch<R, C, false>(q_lat, ql_row, ql_head, q_rot, qr_row, qr_head, cache, page_stride, block_tables, bt_stride, \
                         tiles, positions, n_tiles, heads, sink, out, o_row, o_head, scale, window, splits, ws_o,      \
-                        ws_ml, st);
+                        ws_ml, bucket, st);
   LAT_SHAPES(LAT_CASE)
 #undef LAT_CASE
   return -1;

@@ -115,6 +115,20 @@ def test_batched_requests_are_independent():
         assert alone == t
 
 
+def test_eager_decode_steps_name_the_bucket_of_their_captured_twin():
+    """Kernels that cut a row's keys by the rows of a step need the padded count: six sequences decode as a graph of eight."""
+    eng = make_engine()
+    seen, forward = [], eng.runner.model.forward
+
+    def spy(ids, pool, meta):
+        seen.append((meta.num_decode, meta.dec_bucket))
+        return forward(ids, pool, meta)
+
+    eng.runner.model.forward = spy
+    eng.generate([[17 + i] * 5 for i in range(6)], SamplingParams(max_tokens=4, temperature=0, ignore_eos=True))
+    assert (6, 8) in seen and all(b == eng.runner._bucket(n) for n, b in seen if n)
+
+
 def test_preemption_recomputes_correctly():
     g = torch.Generator().manual_seed(4)
     prompts = [torch.randint(16, 500, (100,), generator=g).tolist() for _ in range(4)]

@@ -62,6 +62,22 @@ def test_decode_batches_beyond_a_round(heads, rows, splits, window):
     assert float((out.double() - want).norm() / want.norm()) < 6e-3   # as above
 
 
+@pytest.mark.parametrize("heads,rows,bucket", [(16, 36, 40), (32, 33, 40), (32, 65, 80), (16, 100, 128), (70, 20, 24)])
+def test_padded_and_unpadded_batches_sum_alike(heads, rows, bucket):
+    """The rows of an eager step and of the captured step that holds more rows: equal bits."""
+    ctx = [700 + (531 * i) % 3000 for i in range(rows)]
+    pool, table, q, sink = setup(ctx, [1] * rows, heads, rows)
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    splits = ops.decode_num_splits(bucket, 1, 32768)
+    assert bucket * splits > 256   # more workgroups than CUs: the kernel chooses among the ranges
+    pad = torch.nn.functional.pad
+    more = bucket - rows
+    graph = ops.latent_attention(pad(q, (0, 0, 0, 0, 0, more))[..., :RANK], pad(q, (0, 0, 0, 0, 0, more))[..., RANK:], pool, 8,
+                                 pad(table, (0, 0, 0, more)), None, pad(pos, (0, more)), sink, 0.05, splits=splits)
+    eager = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, None, pos, sink, 0.05, splits=splits, bucket=bucket)
+    assert torch.equal(eager, graph[:rows])
+
+
 @pytest.mark.parametrize("heads", [3, 16, 64])
 def test_prefill_tiles(heads):
     ctx, rows_of = [70, 500, 130], [70, 33, 1]

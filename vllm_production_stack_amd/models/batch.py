@@ -21,6 +21,7 @@ class BatchMeta:
     dec_block_tables: torch.Tensor | None = None  # int32 [num_decode, max_pages]
     dec_ctx_lens: torch.Tensor | None = None  # int32 [num_decode]  (includes the new token)
     dec_num_splits: int = 1
+    dec_bucket: int = 0  # rows of the captured step that would run the decode part (0: as many as there are)
     dec_ws_o: torch.Tensor | None = None
     dec_ws_ml: torch.Tensor | None = None
     # prefill part

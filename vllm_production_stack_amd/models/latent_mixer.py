@@ -133,6 +133,7 @@ class LatentAttention:
         offset = lw.cache_offset if cache_offset is None else cache_offset
         window = m.window or NO_WINDOW
         splits = getattr(meta, "dec_num_splits", 1) or 1
+        bucket = getattr(meta, "dec_bucket", 0)
         if m.window:  # no key range shorter than two pages
             splits = max(1, min(splits, ((m.window + PAGE - 1) // PAGE + 1) // 2))
         plan = (getattr(meta, "pre_expand", None) or {}).get((m.heads, m.window)) if self._expands(m) else None
@@ -143,7 +144,8 @@ class LatentAttention:
             if nd > 0:
                 q_lat = torch.bmm(q[:nd, :, :m.dim].transpose(0, 1), lw.w_uk).transpose(0, 1)
                 o_lat = ops.latent_attention(q_lat, q[:nd, :, m.dim:], pool, offset, meta.dec_block_tables, None,
-                                             meta.positions[:nd], lw.sink, m.scale, splits=splits, window=window)
+                                             meta.positions[:nd], lw.sink, m.scale, splits=splits, window=window,
+                                             bucket=bucket)
                 torch.bmm(o_lat.transpose(0, 1), lw.w_uv, out=o[:nd].transpose(0, 1))
             return o
         # [heads, T, dim] x [heads, dim, kv_rank]: the unrotated query in latent space
@@ -152,7 +154,8 @@ class LatentAttention:
         o_lat = torch.empty((t, m.heads, m.kv_rank), dtype=q.dtype, device=q.device)
         if nd > 0:
             ops.latent_attention(q_lat[:nd], q_rot[:nd], pool, offset, meta.dec_block_tables, None,
-                                 meta.positions[:nd], lw.sink, m.scale, out=o_lat[:nd], splits=splits, window=window)
+                                 meta.positions[:nd], lw.sink, m.scale, out=o_lat[:nd], splits=splits, window=window,
+                                 bucket=bucket)
         if meta.num_prefill_seqs > 0:
             ops.latent_attention(q_lat[nd:], q_rot[nd:], pool, offset, meta.pre_block_tables,
                                  meta.pre_row_seq, meta.positions[nd:], lw.sink, m.scale, out=o_lat[nd:],

@@ -281,7 +281,7 @@ def _mfma_ok(q_lat, q_rot, pool, out) -> bool:
 
 
 def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, positions, sink, scale: float, out=None,
-                     tiles=None, splits: int = 1, window: int = NO_WINDOW):
+                     tiles=None, splits: int = 1, window: int = NO_WINDOW, bucket: int = 0):
     """Causal attention of query rows over their sequences' cache entries, in latent space.
 
     q_lat [T, heads, rank] and q_rot [T, heads, rot] (views with contiguous last dim); row ``i``
@@ -294,7 +294,10 @@ def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, pos
 
     bf16 entries of a shape the matrix-core kernel tiles take it: decode batches as they are (with
     ``splits`` key ranges per row, merged by a second launch), prefill rows when ``tiles`` (the device
-    copy of ``build_latent_tiles``) describes them.  Everything else takes the plain kernel."""
+    copy of ``build_latent_tiles``) describes them.  Everything else takes the plain kernel.
+
+    ``bucket``: rows of the captured step that would run this decode batch padded.  How a row's keys are cut follows that
+    count, so that both steps sum in the same order."""
     t, heads = q_rot.shape[:2]
     rank = q_lat.shape[2] if q_lat is not None else out.shape[2]
     assert 1 <= window <= NO_WINDOW
@@ -320,6 +323,7 @@ def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, pos
             n_tiles, splits = tiles.shape[0], 1
         else:
             n_tiles = t * ((heads + LATENT_TILE_SLOTS - 1) // LATENT_TILE_SLOTS)
+            bucket *= n_tiles // t
         ws_o = ws_ml = None
         if splits > 1:
             ws_o = torch.empty((n_tiles * splits * LATENT_TILE_SLOTS * rank,), dtype=torch.float32, device=out.device)
@@ -329,7 +333,7 @@ def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, pos
             c_long(q_rot.stride(1)), _layer_base(pool, offset, rank + rot), c_long(pool.stride(0)), o._p(block_tables),
             c_int(block_tables.stride(0)), o._p(tiles), o._p(positions), c_int(n_tiles), c_int(heads), o._p(sink),
             o._p(out), c_long(out.stride(0)), c_long(out.stride(1)), c_int(rank), c_int(rot), c_float(scale),
-            c_int(window), c_int(splits), o._p(ws_o), o._p(ws_ml), o._stream()), "latent_attention_mfma")
+            c_int(window), c_int(splits), o._p(ws_o), o._p(ws_ml), c_int(bucket), o._stream()), "latent_attention_mfma")
         return out
     if q_lat is None:
         raise ValueError("value | key entries: operands the tile kernel does not take")
