@@ -42,8 +42,6 @@ struct LatTile {
 
 __device__ __forceinline__ u32x4 ld16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
 constexpr float LOG2E = 1.4426950408889634f, LN2 = 0.6931471805599453f;
 
 // (entries of up to 256 values leave registers for three waves per SIMD; at 320 they would spill and lose)
@@ -275,16 +273,18 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //   * ds_read_b64_tr_b16 gives lane (c, g) the keys 4 g .. 4 g + 3 of channel c: the order in which the S accumulators hold them.
 //   * Two pages are on their way except while one is multiplied: the page after next is asked for as soon as its buffer is free,
 //     before the next one is waited for (a counted wait).  Waiting for each page before asking for another left 4.5 TB/s.
-//   * Decode rows of at most 32 heads (KSPLIT 4): eight waves, four of which share 16 slots and take 16 keys of every page each;
-//     their softmax states and outputs are merged through LDS at the end.  With 64 slots a tile keeps four waves busy by itself.
+//   * Decode rows of at most 32 heads (QUARTERS): eight waves, four of which share 16 slots.  Each scores 16 keys of a page, the
+//     four exchange scores through 8 KB of LDS, keep the same softmax state and sum a quarter of the channels over all 64 keys.
+//     (With keys and states of its own a wave held all channels, and joining the four moved 130 KB through LDS at the end: 4 to 5 us
+//     that ranges of one or two pages could not hide.)  With 64 slots a tile keeps four waves busy by itself.
 //   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
-// Decode rows with their merge, in a graph: 32 sequences of 3.5k entries on average, 32 heads, 8 splits (137 MB) 70.5 -> 52.5 us, 8
-// of 26k entries 113 -> 76; a single sequence of 2k entries, a page per split, has nothing to overlap: 23.9 -> 26.7.  Prefill
-// tiles, 1500 rows of 16 heads behind 4500 entries: 854 -> 737.
+// Decode rows with their merge, in a graph, pages from memory; staged through registers / this: 32 heads, 32 sequences of 4k entries in 8
+// ranges 65 / 40 us, 8 of 8k in 32 42 / 31, one of 26k in 32 86 / 48, one of 2k, a page a range, 17.4 / 17.7; 16 heads, one of 2k 16.0 / 15.1.
+// Prefill tiles, 1500 rows of 16 heads behind 4500 entries: 855 / 728.
 
 // o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
 // their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
-// channels a tile, keys 16 apart, eight tiles a block; 16 keys: one read a tile, sixteen tiles a block.
+// channels a tile, keys 16 apart, eight tiles a block.
 template <int ROW, int J>
 __device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8& pf, const uint32_t (&at)[4]) {
   u32x2 r[16];
@@ -310,37 +310,15 @@ __device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8& pf, 
   }
 }
 
-template <int J>
-__device__ __forceinline__ void transposed_products16(f32x4* o, const s16x4& pf, const uint32_t (&at)[4]) {
-  u32x2 r[8];
-  asm volatile(
-      "ds_read_b64_tr_b16 %0, %8 offset:%12\n\tds_read_b64_tr_b16 %1, %9 offset:%12\n\t"
-      "ds_read_b64_tr_b16 %2, %10 offset:%12\n\tds_read_b64_tr_b16 %3, %11 offset:%12\n\t"
-      "ds_read_b64_tr_b16 %4, %8 offset:%13\n\tds_read_b64_tr_b16 %5, %9 offset:%13\n\t"
-      "ds_read_b64_tr_b16 %6, %10 offset:%13\n\tds_read_b64_tr_b16 %7, %11 offset:%13\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
-      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(J * 256), "n"(J * 256 + 128)
-      : "memory");
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    o[8 * J + i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, r[i]), pf, o[8 * J + i], 0, 0, 0);
-}
-
 template <int ROW, int... J>
 __device__ __forceinline__ void all_products(f32x4* o, const bf16x8& pf, const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
   (transposed_products<ROW, J>(o, pf, at), ...);
 }
-template <int... J>
-__device__ __forceinline__ void all_products16(f32x4* o, const s16x4& pf, const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
-  (transposed_products16<J>(o, pf, at), ...);
-}
-
 // How many of `splits` key ranges a decode row of `pages` pages is cut into.  A workgroup fills a CU (two pages in LDS) and what it
-// does once - queries, the join, a partial result of 64 KB - takes about as long as four pages, so more workgroups than a
-// round of 256 only pay if their ranges are long: 100 sequences of 1000 entries in 8 ranges of two pages were four rounds.  In a
-// graph with the merge, all ranges -> those used: 100 x 1000 entries 86 -> 45 us, 40 x 3000 (7 -> 6) 64 -> 44, 33 x 12000
-// (8 -> 7) 144 -> 98, 128 x 100 37 -> 25; one sequence of 2000 keeps its 32 and its 26.
+// does once - queries, the first page's way, a partial result of 64 KB - takes about as long as four pages (two or three give the
+// same times), so more workgroups than a round of 256 only pay if their ranges are long: 100 sequences of 1000 entries in 8 ranges
+// of two pages were four rounds.  In a graph with the merge, all ranges / those used: 100 x 1000 entries 72 / 42 us, 40 x 3000 (7 / 6) 55 / 40,
+// 33 x 12000 (8 / 7) 139 / 94; 128 x 100, where a row has two pages, 22.5 / 24.
 // `rows` are those of the step's batch bucket, not of the launch: a row's ranges, and with them the order of its sums, are the same
 // in a captured step that is padded to the bucket and in an eager one that is not.
 constexpr int WIDE_ONCE = 4;
@@ -354,23 +332,23 @@ __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   return used;
 }
 
-template <int RANK, int ROT, int KSPLIT>
-__global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void latent_wide_kernel(
+template <int RANK, int ROT, bool QUARTERS>
+__global__ __launch_bounds__(QUARTERS ? 512 : 256, QUARTERS ? 2 : 1) void latent_wide_kernel(
     const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
     long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
     int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
     const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
     int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
   constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, DT = RANK / 16, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW;
-  static_assert(KSPLIT == 1 || KSPLIT == 4, "all keys or a quarter of them");
-  constexpr int WAVES = KSPLIT == 4 ? 8 : 4;
+  constexpr int WAVES = QUARTERS ? 8 : 4;
   constexpr int NI = PAGE_BYTES / (1024 * WAVES);  // KiB of a page that a wave loads
-  constexpr int NT = 4 / KSPLIT;                   // 16-key tiles of a page that a wave takes
-  static_assert(ENTRY % 64 == 0 && DT % 8 == 0, "chunks are exchanged within groups of eight");
+  constexpr int NT = QUARTERS ? 1 : 4;             // 16-key tiles of a page that a wave scores
+  constexpr int DW = QUARTERS ? DT / 4 : DT;       // 16-channel tiles that it sums
+  static_assert(ENTRY % 64 == 0 && DW % 8 == 0, "chunks are exchanged within groups of eight");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c16 = lane & 15, g = lane >> 4;
-  const int sg = KSPLIT == 4 ? wave >> 2 : wave, kh = KSPLIT == 4 ? wave & 3 : 0;  // slots, keys
+  const int sg = QUARTERS ? wave >> 2 : wave, part = QUARTERS ? wave & 3 : 0;  // slots; keys and channels
   LatTile t;
   if (tiles) {
     const int* e = tiles + 6 * blockIdx.x;
@@ -388,6 +366,20 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
   const int tok = valid ? slot / t.hcount : 0;
   const int head = t.head0 + (valid ? slot % t.hcount : 0);
   const long row = t.row0 + tok;
+  // (a slot past the tile reads the tile's first query, and nothing of it is stored: no branch, no select.)  In a single round every
+  // range may be used, and the queries are on their way while the row's position and page are looked up (one sequence of 2k entries
+  // 18.6 -> 17.7 us); with more, most of the workgroups have nothing to do (100 x 400 entries 37 -> 31 if they don't load them).
+  bf16x8 qf[KS];
+  auto load_q = [&]() {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int d = 32 * ks + 8 * g;
+      qf[ks] = __builtin_bit_cast(
+          bf16x8, 32 * ks < RANK ? ld16(q_lat + row * ql_row + head * ql_head + d) : ld16(q_rot + row * qr_row + head * qr_head + (d - RANK)));
+    }
+  };
+  const bool all_used = bucket * splits <= 256;
+  if (all_used) load_q();
   const int my_pos = valid ? t.pos0 + tok : -1;
   const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
   const int p_first = max(0, t.pos0 - window + 1) / PAGE;
@@ -402,6 +394,7 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     }
     return;
   }
+  if (!all_used) load_q();
   const int my_first = my_pos - window;
   const int* bt = block_tables + (long)t.seq * bt_stride;
 
@@ -417,61 +410,66 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     for (int i = 0; i < NI; ++i)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + src_off[i]),
                                        (__attribute__((address_space(3))) void*)(lds + buf * PAGE_BYTES + (WAVES * i + wave) * 1024),
-                                       16, 0, KSPLIT == 4 ? 2 : 0);  // 2: non-temporal
+                                       16, 0, QUARTERS ? 2 : 0);  // 2: non-temporal
   };
-  if (p_begin < p_end) load_page(p_begin, 0);  // (the older loads: the loop counts the page behind them)
-
-  bf16x8 qf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {  // (a slot past the tile reads the tile's first query: no branches between the loads)
-    const int d = 32 * ks + 8 * g;
-    const u32x4 v = 32 * ks < RANK ? ld16(q_lat + row * ql_row + head * ql_head + d) : ld16(q_rot + row * qr_row + head * qr_head + (d - RANK));
-    qf[ks] = __builtin_bit_cast(bf16x8, valid ? v : (u32x4){0u, 0u, 0u, 0u});
-  }
-  const bool seeded = splits == 1 && sink != nullptr && valid && kh == 0;
+  const bool seeded = splits == 1 && sink != nullptr && valid;
   float m = seeded ? sink[head] * LOG2E : -INFINITY;
   float l = seeded ? 1.f : 0.f;
-  f32x4 o[DT];
+  f32x4 o[DW];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < DW; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   // K fragment of (key tile nt, step ks): row 16 nt + c16, chunk 4 ks + g; V^T fragment of (d tile dt, 16 keys from 16 n):
   // the lane points at row 16 n + 4 g + lane / 4 % 4, channels 16 dt + 4 (lane % 4)
   const int fk = ((c16 >> 1) & 3) << 1 | (c16 >> 3);
   int koff[2], voff[4];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) koff[i] = (16 * NT * kh + c16) * ROW + (((i * 4 + g) ^ fk) << 4);
+  for (int i = 0; i < 2; ++i) koff[i] = (16 * NT * part + c16) * ROW + (((i * 4 + g) ^ fk) << 4);
   const int vr = 4 * g + ((lane >> 2) & 3), fv = ((vr >> 1) & 3) << 1 | (vr >> 3);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    voff[i] = (16 * NT * kh + vr) * ROW + (((2 * i + ((lane & 3) >> 1)) ^ fv) << 4) + (lane & 1) * 8;
+    voff[i] = vr * ROW + (((2 * i + ((lane & 3) >> 1)) ^ fv) << 4) + (lane & 1) * 8 + part * DW * 32;
 
+  f32x4* scores = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;  // of four key quarters
   auto multiply = [&](int p, int buf) {
     const char* img = lds + buf * PAGE_BYTES;
-    f32x4 s[NT];
+    f32x4 s[4];
+    if (wave_active) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) s[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int nt = 0; nt < NT; ++nt) s[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+      for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128 + nt * 16 * ROW);
-        s[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], s[nt], 0, 0, 0);
-      }
+        for (int nt = 0; nt < NT; ++nt) {
+          const bf16x8 a = *reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128 + nt * 16 * ROW);
+          s[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], s[nt], 0, 0, 0);
+        }
+      if constexpr (QUARTERS) scores[part * 64] = s[0];
+    }
+    if constexpr (QUARTERS) {  // (not __syncthreads, which would wait for the page behind this one)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    if (!wave_active) return;
+    if constexpr (QUARTERS) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) s[nt] *= scale2;
+      for (int nt = 0; nt < 4; ++nt) s[nt] = scores[nt * 64];
+    }
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) s[nt] *= scale2;
     if (p * PAGE + PAGE - 1 > t.pos0 || p * PAGE <= t.pos0 + t.n_tok - 1 - window) {
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+      for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int key = p * PAGE + 16 * (NT * kh + nt) + 4 * g + e;
+          const int key = p * PAGE + 16 * nt + 4 * g + e;
           if (key > my_pos || key <= my_first) s[nt][e] = -INFINITY;
         }
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[nt][e]);
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -482,7 +480,7 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     const float corr = dead ? 1.f : __builtin_amdgcn_exp2f(m - mref);
     float ps = 0.f;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float pv = __builtin_amdgcn_exp2f(s[nt][e] - mref);
@@ -495,25 +493,20 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     m = mn;
     if (!__all(corr == 1.f)) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
+      for (int dt = 0; dt < DW; ++dt) o[dt] *= corr;
     }
     const uint32_t page = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + buf * PAGE_BYTES;
-    if constexpr (KSPLIT == 4) {
-      const uint32_t at[4] = {page + voff[0], page + voff[1], page + voff[2], page + voff[3]};
-      const u32x2 w = {pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3])};
-      all_products16(o, __builtin_bit_cast(s16x4, w), at, std::make_integer_sequence<int, DT / 8>());
-    } else {
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const uint32_t half = page + kk * 32 * ROW;
-        const uint32_t at[4] = {half + voff[0], half + voff[1], half + voff[2], half + voff[3]};
-        const u32x4 w = {pack_bf16x2(s[2 * kk][0], s[2 * kk][1]), pack_bf16x2(s[2 * kk][2], s[2 * kk][3]),
-                         pack_bf16x2(s[2 * kk + 1][0], s[2 * kk + 1][1]), pack_bf16x2(s[2 * kk + 1][2], s[2 * kk + 1][3])};
-        all_products<ROW>(o, __builtin_bit_cast(bf16x8, w), at, std::make_integer_sequence<int, DT / 8>());
-      }
+    for (int kk = 0; kk < 2; ++kk) {
+      const uint32_t half = page + kk * 32 * ROW;
+      const uint32_t at[4] = {half + voff[0], half + voff[1], half + voff[2], half + voff[3]};
+      const u32x4 w = {pack_bf16x2(s[2 * kk][0], s[2 * kk][1]), pack_bf16x2(s[2 * kk][2], s[2 * kk][3]),
+                       pack_bf16x2(s[2 * kk + 1][0], s[2 * kk + 1][1]), pack_bf16x2(s[2 * kk + 1][2], s[2 * kk + 1][3])};
+      all_products<ROW>(o, __builtin_bit_cast(bf16x8, w), at, std::make_integer_sequence<int, DW / 8>());
     }
   };
 
+  if (p_begin < p_end) load_page(p_begin, 0);
   if (p_begin + 1 < p_end) load_page(p_begin + 1, 1);
   for (int p = p_begin; p < p_end; ++p) {
     const int buf = (p - p_begin) & 1;
@@ -522,7 +515,7 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (wave_active) multiply(p, buf);
+    multiply(p, buf);
     if (p + 2 < p_end) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // my reads of this buffer are done; everyone's: the barrier
       __builtin_amdgcn_s_barrier();
@@ -531,44 +524,21 @@ __global__ __launch_bounds__(KSPLIT == 4 ? 512 : 256, KSPLIT == 4 ? 2 : 1) void 
     }
   }
 
-  if constexpr (KSPLIT == 4) {  // the four key quarters: 2 joins 0 and 3 joins 1, then 1 joins 0
-#pragma unroll
-    for (int step = 2; step > 0; step >>= 1) {
-      __syncthreads();  // no page is read any more (and none is on its way); the other pair has read what it joined
-      f32x4* rec = reinterpret_cast<f32x4*>(lds) + ((sg * 2 + (kh & (step - 1))) * (DT + 1)) * 64 + lane;
-      if (kh >= step && kh < 2 * step) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) rec[dt * 64] = o[dt];
-        rec[DT * 64] = (f32x4){m, l, 0.f, 0.f};
-      }
-      __syncthreads();
-      if (kh < step) {
-        const f32x4 ml = rec[DT * 64];
-        const float mn = fmaxf(m, ml[0]), mref = mn == -INFINITY ? 0.f : mn;
-        const float f0 = __builtin_amdgcn_exp2f(m - mref), f1 = __builtin_amdgcn_exp2f(ml[0] - mref);
-        l = l * f0 + ml[1] * f1;
-        m = mn;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[dt] = o[dt] * f0 + rec[dt * 64] * f1;
-      }
-    }
-    if (kh) return;
-  }
   if (!valid) return;
   if (splits == 1) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    uint16_t* dst = out + row * o_row + head * o_head + 4 * g;
+    uint16_t* dst = out + row * o_row + head * o_head + part * DW * 16 + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
+    for (int dt = 0; dt < DW; ++dt) {
       u32x2 w = {pack_bf16x2(o[dt][0] * inv, o[dt][1] * inv), pack_bf16x2(o[dt][2] * inv, o[dt][3] * inv)};
       *reinterpret_cast<u32x2*>(dst + 16 * dt) = w;
     }
   } else {
     const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + slot;
-    float* dst = ws_o + rec * RANK + 4 * g;
+    float* dst = ws_o + rec * RANK + part * DW * 16 + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(dst + 16 * dt) = o[dt];
-    if (g == 0) {
+    for (int dt = 0; dt < DW; ++dt) *reinterpret_cast<f32x4*>(dst + 16 * dt) = o[dt];
+    if (g == 0 && part == 0) {
       ws_ml[2 * rec] = m * LN2;
       ws_ml[2 * rec + 1] = l;
     }
@@ -641,11 +611,11 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
     return *done;
   };
   if constexpr (!ROT_ONLY && RANK == 512 && ROT == 64) {
-    constexpr int LDS = 2 * 64 * (RANK + ROT) * 2;
     const int quarters = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
-    const auto kernel = quarters ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 1>;
-    if (!ready((const void*)kernel, LDS, &attr_set[quarters])) return -2;
-    kernel<<<dim3(n_tiles, splits), dim3(quarters ? 512 : 256), LDS, st>>>(
+    const int lds = 2 * 64 * (RANK + ROT) * 2 + (quarters ? 8 * 1024 : 0);
+    const auto kernel = quarters ? latent_wide_kernel<RANK, ROT, true> : latent_wide_kernel<RANK, ROT, false>;
+    if (!ready((const void*)kernel, lds, &attr_set[quarters])) return -2;
+    kernel<<<dim3(n_tiles, splits), dim3(quarters ? 512 : 256), lds, st>>>(
         (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
         page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
         window, splits, ws_o, ws_ml, bucket);
