@@ -1180,3 +1180,18 @@ def test_layer_norm_matches_float64(rows, hidden, add):
     assert res is None or torch.equal(res, s)
     # one rounding to 16 bits (2^-9 of the value); 32-bit sums of values near 30 are off by 30 * 2^-22 of a deviation near 1
     assert float(((got.double() - want).abs() - want.abs() * 2 ** -8 - 2e-4).max()) < 0
+
+
+@torch.no_grad()
+def test_layer_norm_takes_and_refuses_what_the_library_does():
+    x, w, b = (torch.randn(n, device=DEV).to(BF) for n in (8 * 256, 256, 256))
+    rows = x.view(8, 256)
+    want = torch.nn.functional.layer_norm(rows[:1], (256,), w, b, 1e-5)
+    odd = torch.as_strided(rows, (1, 256), (3, 1))          # one row: its stride says nothing
+    assert torch.allclose(ops.layer_norm(odd, w, b, 1e-5).float(), want.float(), rtol=2 ** -7, atol=1e-2)
+    no_bias = torch.nn.functional.layer_norm(rows, (256,), w, None, 1e-5)
+    assert torch.equal(ops.layer_norm(rows, w, None, 1e-5), no_bias)
+    assert ops.layer_norm(rows[:0], w, b, 1e-5).shape == (0, 256)
+    for bad_w, bad_b in ((w[:248], b), (w, b[:128]), (w.view(2, 128), b), (w.cpu(), b), (w, b.cpu())):
+        with pytest.raises(RuntimeError):
+            ops.layer_norm(rows, bad_w, bad_b, 1e-5)

@@ -143,10 +143,11 @@ def layer_norm(x, weight, bias, eps, residual=None):
     """y = layer norm(x [+ residual]) * weight + bias.  ``residual`` (contiguous) is updated in place with the sum."""
     hidden = x.shape[-1]
     ts = (x, weight, bias) if residual is None else (x, weight, bias, residual)
-    rows_at = x.stride(-2) if x.dim() == 2 else hidden
-    if (x.is_cuda and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts) and hidden % 8 == 0
-            and hidden <= 2048 and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and rows_at % 8 == 0))
-            and weight.is_contiguous() and bias.is_contiguous() and not torch.is_grad_enabled()
+    rows_at = x.stride(0) if x.dim() == 2 and x.shape[0] > 1 else hidden
+    if (x.is_cuda and 0 < hidden <= 2048 and hidden % 8 == 0 and not torch.is_grad_enabled()
+            and all(t is not None and t.device == x.device and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts)
+            and all(t.shape == (hidden,) and t.is_contiguous() for t in (weight, bias)) and rows_at % 8 == 0
+            and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1))
             and (residual is None or (residual.is_contiguous() and residual.shape == x.shape))):
         y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         rc = _kernels().vpsa_layernorm(_p(x), _p(residual), _p(weight), _p(bias), _p(y), c_int(x.numel() // hidden), c_int(hidden),
