@@ -355,3 +355,19 @@ def test_a_pool_cut_into_layer_groups_generates_the_same_tokens():
     pd = make_engine("tiny-llama-gqa", kv_layer_groups=3, kv_transfer=KVTransferConfig(kv_role="kv_consumer"))
     assert isinstance(pd.runner.pool, torch.Tensor)
     pd.shutdown()
+
+
+@pytest.mark.parametrize("value,want", [(None, [True, True, True, False]), ("16", [True, False, False, False]),
+                                        ("300", [True, True, True, True]), ("0", [False] * 4)])
+def test_token_bound_of_the_streaming_expert_kernels(value, want):
+    """VPSA_MOE_MFMA_MAX_TOKENS is the bound when it is set; without it few rows an expert are reason enough."""
+    import os
+    import subprocess
+    import sys
+
+    env = {k: v for k, v in os.environ.items() if k != "VPSA_MOE_MFMA_MAX_TOKENS"}
+    if value is not None:
+        env["VPSA_MOE_MFMA_MAX_TOKENS"] = value
+    code = "from vllm_production_stack_amd import ops; print([ops.moe_streams_experts(t, 2, 8) for t in (16, 48, 192, 300)])"
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, check=True).stdout
+    assert out.splitlines()[-1] == str(want)

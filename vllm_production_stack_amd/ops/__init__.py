@@ -1264,15 +1264,18 @@ def moe_combine(y, weights, pos, tokens):
 
 
 # Batches whose experts see few rows each take the kernels that stream every routed expert's weights once (``csrc/kernels/mid_gemm.hip``)
-# instead of the 256-row tiles: up to this many tokens, and up to this many rows an expert on average (a pass takes 64).  One mixture,
-# microseconds in a graph, tiles / streaming: 8 experts of 28672 x 4096, two a token: 16 tokens 660/435, 48 660/425, 128 674/491, 192
-# 682/619, 224 683/696, 256 rows of a prompt 730/910; 16 experts of 2048 x 2048, four a token: 48 66.5/40.6, 192 69.9/46.7, 224 72.0/67.5.
+# instead of the 256-row tiles: either few tokens, or few rows an expert on average (a pass takes 64).  One mixture, microseconds in a
+# graph, tiles / streaming: 8 experts of 28672 x 4096, two a token: 16 tokens 660/435, 48 660/425, 128 674/491, 192 682/619, 224 683/696, 256
+# rows of a prompt 730/910; 16 of 2048 x 2048, four a token: 48 66.5/40.6, 192 69.9/46.7, 224 72.0/67.5; 32, four a token: 384 131/112; 64,
+# eight a token: 384 251/170; 128: 768 540/323; 256 of 4096 x 2048: 768 2348/1082.  Where one expert sees every token as well (a pass of
+# its own for each 64): 8 experts 192 tokens 705/714, 16 90/96, 32 384 185/180, 64 384 317/206, 128 768 618/401.
+# VPSA_MOE_MFMA_MAX_TOKENS sets the bound on the tokens and leaves the rows out of it (0: never).
 MOE_MFMA_MAX_TOKENS = int(os.environ.get("VPSA_MOE_MFMA_MAX_TOKENS", "48"))
-MOE_STREAM_ROWS = 48
+MOE_STREAM_ROWS = 0 if "VPSA_MOE_MFMA_MAX_TOKENS" in os.environ else 48
 
 
 def moe_streams_experts(tokens: int, topk: int, experts: int) -> bool:
-    return MOE_MFMA_MAX_TOKENS > 0 and (tokens <= MOE_MFMA_MAX_TOKENS or tokens * topk <= MOE_STREAM_ROWS * experts)
+    return tokens <= MOE_MFMA_MAX_TOKENS or (MOE_MFMA_MAX_TOKENS > 0 and tokens * topk <= MOE_STREAM_ROWS * experts)
 
 
 def moe_mfma_supported(hidden: int, inter: int) -> bool:
