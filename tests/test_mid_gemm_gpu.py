@@ -49,6 +49,22 @@ def test_dispatch():
         assert ops._mid_gemm(x[:40].clone().requires_grad_(), w, None, False) is None
 
 
+@pytest.mark.parametrize("m", [1, 24, 90])
+def test_operands_on_another_device_are_refused(m):
+    """A weight, bias or norm that still lies on the host raises, as in the library, and no kernel reads it."""
+    x = torch.zeros(m, 4096, device=DEV, dtype=BF)
+    w, b = torch.zeros(4096, 4096, device=DEV, dtype=BF), torch.zeros(4096, device=DEV, dtype=BF)
+    for bad_w, bad_b in ((w.cpu(), None), (w.cpu(), b), (w, b.cpu())):
+        with pytest.raises(RuntimeError):
+            ops.linear(x, bad_w, bad_b)
+    with pytest.raises(RuntimeError):
+        ops.gate_up_silu(x, w.cpu())
+    res = torch.zeros(m, 4096, device=DEV, dtype=BF)
+    assert ops.linear_add_norm(x, w.cpu(), res, b, 1e-5) is None
+    assert ops.linear_add_norm(x, w, res.cpu(), b, 1e-5) is None
+    assert ops.linear_add_norm(x, w, res, b.cpu(), 1e-5) is None
+
+
 @pytest.mark.parametrize("tokens", [1, 2, 16, 17, 33, 49, 65, 130])
 @pytest.mark.parametrize("routing", ["spread", "one expert"])
 def test_experts(tokens, routing):

@@ -724,9 +724,10 @@ def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
 
 def _mid_takes(x2, w, bias, pair) -> int:
     """``_mid_splits`` for operands that ``mid_gemm`` reads, else 0."""
-    if not (_skinny_enabled and x2.is_cuda and x2.dim() == 2 and x2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
-            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1]))
+    if not (_skinny_enabled and x2.is_cuda and w.device == x2.device and x2.dim() == 2 and x2.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
+            and (bias is None or (bias.device == x2.device and bias.dtype == torch.bfloat16 and bias.is_contiguous()
+                                  and bias.shape == w.shape[:1]))
             and not (torch.is_grad_enabled() and (x2.requires_grad or w.requires_grad))):
         return 0
     return _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair)
@@ -751,7 +752,8 @@ def linear_add_norm(x, w, residual, weight, eps):
     splits = _mid_takes(x, w, None, False)
     m, n = x.shape[0], w.shape[0]
     if (splits < 2 or n > 8192 or residual.shape != (m, n) or residual.dtype != torch.bfloat16 or not residual.is_contiguous()
-            or weight.dtype != torch.bfloat16 or weight.shape != (n,) or not weight.is_contiguous()):
+            or residual.device != x.device or weight.device != x.device or weight.dtype != torch.bfloat16 or weight.shape != (n,)
+            or not weight.is_contiguous()):
         return None
     y = torch.empty_like(residual)
     ws = torch.empty((splits * m * n,), dtype=torch.float32, device=x.device)
@@ -829,9 +831,9 @@ def packed_linear(x2, wp, n: int, k: int, bias=None, pair: bool = False):
 
 
 def _skinny_ok(x, w, bias):
-    return (_skinny_enabled and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and w.is_contiguous() and x.dim() == 2 and 0 < x.shape[0] <= SKINNY_MAX_ROWS
-            and x.stride(1) == 1 and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous())))
+    return (_skinny_enabled and x.is_cuda and w.device == x.device and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and w.is_contiguous() and x.dim() == 2 and 0 < x.shape[0] <= SKINNY_MAX_ROWS and x.stride(1) == 1
+            and (bias is None or (bias.device == x.device and bias.dtype == torch.bfloat16 and bias.is_contiguous())))
 
 
 # Dispatch thresholds of shapes that mid_gemm below does not take, measured on MI355X (profiles/gemm_micro_graph.jsonl, HIP-graph replay,
