@@ -65,6 +65,33 @@ def test_operands_on_another_device_are_refused(m):
     assert ops.linear_add_norm(x, w, res, b.cpu(), 1e-5) is None
 
 
+@pytest.mark.parametrize("m", [24, 90])
+def test_calls_that_something_follows_stay_with_the_library(m):
+    """Gradients of the bias alone, forward-mode tangents, vmap and traces, at rows where the kernel takes plain calls."""
+    from torch.autograd import forward_ad
+
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x, w = (torch.randn(n, 4096, generator=g, device=DEV).to(BF) for n in (m, 4096))
+    b = torch.randn(4096, generator=g, device=DEV).to(BF)
+    assert ops._mid_takes(x, w, b, False)
+    lib = torch.nn.functional.linear
+    with torch.enable_grad():
+        leaf = b.clone().requires_grad_()
+        ops.linear(x, w, leaf).sum().backward()
+        assert torch.equal(leaf.grad, torch.full_like(b, m))
+    with torch.no_grad(), forward_ad.dual_level():
+        t = torch.randn(m, 4096, generator=g, device=DEV).to(BF)
+        got = forward_ad.unpack_dual(ops.linear(forward_ad.make_dual(x, t), w, b)).tangent
+        assert got is not None and torch.equal(got, lib(t, w))
+    with torch.no_grad():
+        xs = torch.stack([x, x.flip(0), -x])
+        assert torch.func.vmap(lambda q: ops.linear(q, w))(xs).shape == (3, m, 4096)
+        traced = torch.jit.trace(lambda q: ops.linear(q, w, b), (x,), check_trace=False)
+        assert torch.equal(traced(xs[1]), lib(xs[1], w, b))
+        ln = torch.func.vmap(lambda q: ops.layer_norm(q, b[:1024], b[1024:2048], 1e-5))(xs[..., :1024])
+        assert torch.equal(ln, torch.nn.functional.layer_norm(xs[..., :1024], (1024,), b[:1024], b[1024:2048], 1e-5))
+
+
 @pytest.mark.parametrize("tokens", [1, 2, 16, 17, 33, 49, 65, 130])
 @pytest.mark.parametrize("routing", ["spread", "one expert"])
 def test_experts(tokens, routing):

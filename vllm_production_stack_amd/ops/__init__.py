@@ -13,6 +13,7 @@ import ctypes
 from ctypes import c_float, c_int, c_long, c_void_p
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _native
 from . import reference
@@ -144,7 +145,7 @@ def layer_norm(x, weight, bias, eps, residual=None):
     hidden = x.shape[-1]
     ts = (x, weight, bias) if residual is None else (x, weight, bias, residual)
     rows_at = x.stride(0) if x.dim() == 2 and x.shape[0] > 1 else hidden
-    if (x.is_cuda and 0 < hidden <= 2048 and hidden % 8 == 0 and not torch.is_grad_enabled()
+    if (x.is_cuda and 0 < hidden <= 2048 and hidden % 8 == 0 and not _followed(*ts)
             and all(t is not None and t.device == x.device and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in ts)
             and all(t.shape == (hidden,) and t.is_contiguous() for t in (weight, bias)) and rows_at % 8 == 0
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1))
@@ -722,15 +723,23 @@ def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
     return 0
 
 
+def _followed(*ts) -> bool:
+    """True where something follows a call from outside and would lose sight of it in a kernel launch: gradients of its operands,
+    forward-mode tangents, a function transform (vmap), a trace or a dispatch mode."""
+    return ((torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)) or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() > 0)
+
+
 def _mid_takes(x2, w, bias, pair) -> int:
     """``_mid_splits`` for operands that ``mid_gemm`` reads, else 0."""
     if not (_skinny_enabled and x2.is_cuda and w.device == x2.device and x2.dim() == 2 and x2.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
             and (bias is None or (bias.device == x2.device and bias.dtype == torch.bfloat16 and bias.is_contiguous()
-                                  and bias.shape == w.shape[:1]))
-            and not (torch.is_grad_enabled() and (x2.requires_grad or w.requires_grad))):
+                                  and bias.shape == w.shape[:1]))):
         return 0
-    return _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair)
+    splits = _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair)
+    return 0 if splits and _followed(x2, w, bias) else splits
 
 
 def _mid_gemm(x2, w, bias, pair):
