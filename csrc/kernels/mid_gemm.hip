@@ -4,7 +4,7 @@
 //   * A workgroup owns 128 weight rows (PAIR: 64 gate and the 64 matching up rows) and up to 128 token rows; the reduction is
 //     split over workgroups until about every CU has one (splits of whole 64-element chunks, not necessarily equal).
 //   * Both operands go from memory straight into LDS (rows of 128 bytes, 16-byte chunk j of row r at j ^ (r ^ r / 8) % 8, so that
-//     the 16 rows of a fragment cover all banks), four stages of which three are on their way: 64 to 96 KiB a CU in flight.
+//     the 16 rows of a fragment cover all banks), four stages of which three are on their way: 54 to 96 KiB a CU in flight.
 //   * One barrier a chunk, counted waits.  A wave multiplies 32 weight rows with all token tiles on v_mfma_f32_16x16x32_bf16;
 //     its accumulators hold four consecutive outputs of a token, as in the streaming kernel of gemm.hip, whose reduction
 //     (partial sums in 32 bits, fixed order) closes a split product.
@@ -20,11 +20,13 @@ constexpr int BN = 128, BK = 64, STAGES = 4, ROWB = BK * 2;
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
 // acc[i][t] += W tile i of the wave x token tile t over chunks [0, n) of both operands: NA * 64 weight rows and MT * 16 token rows a
-// chunk, all of it in LDS stages.  wrow(r) / xrow(r): bytes from wp / xp to row r's first chunk; arow: the wave's weight tiles (rows
-// within the workgroup's).  POLICY of the weight loads: 2 = non-temporal.  Nothing is on its way or read any more on return.
-template <int MT, int NA, int POLICY, typename WRow, typename XRow>
-__device__ __forceinline__ void stream_product(const char* __restrict__ wp, const char* __restrict__ xp, WRow wrow, XRow xrow, int n,
-                                               int first, char* lds, const int (&arow)[NA], f32x4 (&acc)[NA][MT]) {
+// chunk, all of it in LDS stages.  The weight rows lie w_row bytes apart from wp on, those from the 64th on w_half further; xrow(r): bytes
+// from xp to row r's first chunk; arow: the wave's weight tiles (rows within the workgroup's).  POLICY of the weight loads: 2 =
+// non-temporal.  Nothing is on its way or read any more on return.
+template <int MT, int NA, int POLICY, typename XRow>
+__device__ __forceinline__ void stream_product(const char* __restrict__ wp, uint32_t w_row, long w_half, const char* __restrict__ xp,
+                                               XRow xrow, int n, int first, char* lds, const int (&arow)[NA],
+                                               f32x4 (&acc)[NA][MT]) {
   constexpr int WI = 2 * NA;        // KiB of weight rows that a wave loads of a stage
   constexpr int XI = (MT + 1) / 2;  // and of token rows (the last ones twice where MT is odd)
   constexpr int NL = WI + XI;       // loads of a stage
@@ -37,7 +39,7 @@ __device__ __forceinline__ void stream_product(const char* __restrict__ wp, cons
 #pragma unroll
   for (int i = 0; i < WI; ++i) {
     const int r = 8 * (4 * i + wave) + (lane >> 3);
-    woff[i] = wrow(r) + (((lane & 7) ^ swz(r)) << 4);
+    woff[i] = (r & 63) * w_row + (((lane & 7) ^ swz(r)) << 4);
   }
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
@@ -50,7 +52,7 @@ __device__ __forceinline__ void stream_product(const char* __restrict__ wp, cons
     const int c = i_c + first < n ? i_c + first : i_c + first - n;
 #pragma unroll
     for (int i = 0; i < WI; ++i)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wp + (long)c * ROWB + woff[i]),
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wp + (i >> 1) * w_half + (long)c * ROWB + woff[i]),
                                        (__attribute__((address_space(3))) void*)(st + (4 * i + wave) * 1024), 16, 0, POLICY);
 #pragma unroll
     for (int i = 0; i < XI; ++i)
@@ -112,8 +114,8 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
   // Workgroups walk their chunks from different ones on: rows whose length is a power of two put a chunk of all 128 rows on the
   // same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
   stream_product<MT, 2, POLICY>(
-      reinterpret_cast<const char*>(w) + (long)c0 * ROWB, reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB,
-      [&](int r) { return (uint32_t)(PAIR ? n0 + (r & 63) + (r >> 6) * n_out : n0 + r) * (uint32_t)(K * 2); },
+      reinterpret_cast<const char*>(w + (long)n0 * K) + (long)c0 * ROWB, (uint32_t)(K * 2), (PAIR ? n_out : 64) * (long)(K * 2),
+      reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB,
       [&](int r) { return (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)); },  // rows past the last repeat it
       n, n > 0 ? (int)(blockIdx.x * 3 % n) : 0, lds, arow, acc);
 #pragma unroll
@@ -176,12 +178,9 @@ __global__ __launch_bounds__(256, 1) void mid_experts_kernel(const uint16_t* __r
     const int last = min(n_e - m0, 16 * MT) - 1;
     f32x4 acc[NA][MT];
     stream_product<MT, NA, 2>(
-        reinterpret_cast<const char*>(w + (long)e * N * K), reinterpret_cast<const char*>(x),
-        [&](int r) { return (uint32_t)(n0 + (r & 63) + (r >> 6) * n_out) * (uint32_t)(K * 2); },
-        [&](int r) {
-          const int row = r0 + m0 + min(r, last);
-          return (uint32_t)(UNIT ? sorted_tok[row] : row) * (uint32_t)(K * 2);
-        },
+        reinterpret_cast<const char*>(w + ((long)e * N + n0) * K), (uint32_t)(K * 2), n_out * (long)(K * 2),
+        reinterpret_cast<const char*>(UNIT ? x : x + (long)(r0 + m0) * K),
+        [&](int r) { return (uint32_t)(UNIT ? sorted_tok[r0 + m0 + min(r, last)] : min(r, last)) * (uint32_t)(K * 2); },
         n, (int)((blockIdx.x * 3 + e) % n), lds, arow, acc);
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
@@ -425,7 +424,8 @@ VPSA_EXPORT int vpsa_moe_mfma_act(const void* x, const void* w13, const void* w2
                                   float act_alpha, float act_bias, const float* row_scale, hipStream_t stream) {
   if (tokens * topk <= 0) return 0;
   if (n_experts < 1 || n_experts > 65535 || hidden % 128 != 0 || inter % 512 != 0) return -1;
-  if ((long)inter * hidden * 4 >= (1L << 32) || (long)tokens * topk * (hidden > inter ? hidden : inter) * 2 >= (1L << 32)) return -1;
+  if (((uintptr_t)x | (uintptr_t)w13 | (uintptr_t)w2 | (uintptr_t)act) & 15) return -1;
+  if ((long)tokens * hidden * 2 >= (1L << 32) || (hidden > inter ? hidden : inter) >= (1 << 24)) return -1;  // offsets of 32 bits
   // an expert sees each token at most once: tokens bounds its row count
 #define EXPERTS(MT)                                                                                                         \
   return launch_experts<MT>(x, w13, w2, offsets, sorted_tok, act, y, n_experts, hidden, inter, act_limit, act_alpha, act_bias, \

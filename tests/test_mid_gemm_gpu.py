@@ -114,6 +114,51 @@ def test_experts(tokens, routing):
     assert float((got.double() - want).norm() / want.norm()) < 6e-3
 
 
+def test_experts_of_a_large_batch():
+    """Rows of the activations beyond the first 4 GiB: an early and a late expert's tokens against float64."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    e, h, i, t = 4, 128, 16384, 65600
+    x = torch.randn(t, h, generator=g, device=DEV).to(BF)
+    w13 = (torch.randn(e, 2 * i, h, generator=g, device=DEV) * h ** -0.5).to(BF)
+    w2 = (torch.randn(e, h, i, generator=g, device=DEV) * i ** -0.5).to(BF)
+    ids = torch.stack([torch.arange(t, device=DEV) % e, (torch.arange(t, device=DEV) + 1) % e], 1).int()
+    wt = torch.rand(t, 2, generator=g, device=DEV)
+    got = ops.moe_experts_grouped(x, w13, w2, ids, wt)
+    for row in (0, 1, 2, 3, 30000, t - 4, t - 3, t - 2, t - 1):
+        want = torch.zeros(h, dtype=torch.float64, device=DEV)
+        for c, p in zip(ids[row].tolist(), wt[row].double()):
+            gu = w13[c].double() @ x[row].double()
+            want += p * (w2[c].double() @ (torch.nn.functional.silu(gu[:i]) * gu[i:]))
+        assert float((got[row].double() - want).norm() / want.norm()) < 6e-3   # as above
+
+
+def test_an_expert_beyond_four_gigabytes():
+    g = torch.Generator(device=DEV).manual_seed(5)
+    h, i = 16384, 65536 + 512
+    x = torch.randn(3, h, generator=g, device=DEV).to(BF)
+    w13 = torch.empty(1, 2 * i, h, device=DEV, dtype=BF).normal_(0, h ** -0.5, generator=g)
+    w2 = torch.empty(1, h, i, device=DEV, dtype=BF).normal_(0, i ** -0.5, generator=g)
+    got = ops.moe_experts_grouped(x, w13, w2, torch.zeros(3, 1, dtype=torch.int32, device=DEV), torch.ones(3, 1, device=DEV))
+    gu = torch.cat([x.float() @ c.float().t() for c in w13[0].split(16384)], 1)
+    act = torch.nn.functional.silu(gu[:, :i]) * gu[:, i:]
+    want = torch.cat([act @ c.float().t() for c in w2[0].split(4096)], 1)
+    assert float((got.float() - want).norm() / want.norm()) < 6e-3   # as above
+
+
+def test_experts_off_the_16_byte_boundary():
+    """Weights and rows that start two bytes into a buffer give what aligned copies give."""
+    g = torch.Generator(device=DEV).manual_seed(4)
+
+    def odd(*shape):
+        n = torch.Size(shape).numel()
+        return (torch.randn(n + 1, generator=g, device=DEV) * 0.1).to(BF)[1:].view(shape)
+
+    x, w13, w2 = odd(20, 256), odd(4, 1024, 256), odd(4, 256, 512)
+    ids = torch.randint(0, 4, (20, 1), generator=g, device=DEV, dtype=torch.int32)
+    wt = torch.ones(20, 1, device=DEV)
+    assert torch.equal(ops.moe_experts_grouped(x, w13, w2, ids, wt), ops.moe_experts_grouped(x.clone(), w13.clone(), w2.clone(), ids, wt))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 256, 1024), (3, 1280, 1088), (16, 4096, 1024), (17, 5120, 1088), (40, 8192, 2624), (130, 128, 1088)])
 def test_sum_with_residual_and_norm(any_shape, m, n, k):
     """One reduction against the separate passes: the same roundings, so the residual stream is equal and the norm differs by its

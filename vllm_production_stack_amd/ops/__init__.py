@@ -1294,7 +1294,7 @@ def moe_mfma_supported(hidden: int, inter: int) -> bool:
 
 
 def _rows16(x):
-    """``x`` contiguous with its first row on a 16-byte boundary (what loads straight into LDS take)."""
+    """``x`` contiguous and on a 16-byte boundary (what loads straight into LDS take)."""
     x = x.contiguous()
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
@@ -1316,10 +1316,17 @@ def moe_experts_grouped(x, w13, w2, ids, weights, foreign=False, combine=True):
     assert w13.shape[1] == 2 * inter and w13.shape[2] == hidden and w2.shape[1] == hidden
     assert w13.is_contiguous() and w2.is_contiguous() and ids.dtype == torch.int32
     assert moe_mfma_supported(hidden, inter), (hidden, inter)
+    if t > 1 and t * hidden >= 1 << 31:  # the kernels reach a batch's rows with offsets of 32 bits
+        cut = [moe_experts_grouped(x[i], w13, w2, ids[i], None if weights is None else weights[i], foreign, combine)
+               for i in (slice(0, t // 2), slice(t // 2, t))]
+        if combine:
+            return torch.cat(cut)
+        return torch.cat([cut[0][0], cut[1][0]]), torch.cat([cut[0][1], cut[1][1] + t // 2 * k])
+    x, w13, w2 = _rows16(x), _rows16(w13), _rows16(w2)
     offsets, pos, sorted_tok = moe_align(ids, n_experts + (1 if foreign else 0))
     act = torch.empty((t * k, inter), dtype=x.dtype, device=x.device)
     y = torch.empty((t * k, hidden), dtype=x.dtype, device=x.device)
-    rc = _kernels().vpsa_moe_mfma(_p(_rows16(x)), _p(w13), _p(w2), _p(offsets), _p(sorted_tok),
+    rc = _kernels().vpsa_moe_mfma(_p(x), _p(w13), _p(w2), _p(offsets), _p(sorted_tok),
                                   _p(act), _p(y), c_int(t), c_int(k), c_int(n_experts),
                                   c_int(hidden), c_int(inter), _stream())
     _check(rc, "moe_mfma")

@@ -621,7 +621,8 @@ def moe_glu_grouped(x, w13, w2, ids, limit: float, alpha: float = 1.702, up_bias
         # (the kernels of the top-k softmax mixtures, with this unit's activation)
         act = torch.empty((t * k, inter), dtype=x.dtype, device=x.device)
         y = torch.empty((t * k, hidden), dtype=x.dtype, device=x.device)
-        o._check(o._kernels().vpsa_moe_mfma_act(o._p(o._rows16(x)), o._p(w13), o._p(w2), o._p(offsets), o._p(sorted_tok), o._p(act),
+        x, w13, w2 = o._rows16(x), o._rows16(w13), o._rows16(w2)
+        o._check(o._kernels().vpsa_moe_mfma_act(o._p(x), o._p(w13), o._p(w2), o._p(offsets), o._p(sorted_tok), o._p(act),
                                                 o._p(y), c_int(t), c_int(k), c_int(w13.shape[0]), c_int(hidden),
                                                 c_int(inter), c_float(limit), c_float(alpha), c_float(up_bias),
                                                 o._p(sw), o._stream()), "moe_mfma_act")
