@@ -764,6 +764,81 @@ def test_cachegen_page_on_gpu_uses_the_rans_stage_and_matches_the_host_coder(mon
     assert (on_cpu - back.float()).abs().max().item() <= 0.02 * back.float().abs().max().item()
 
 
+def _codec_pages(n, geometry=(4, 2, 64)):
+    """Pages that code to sizes between a few and nearly all of their symbols, small and large in turn."""
+    layers, kv, hd = geometry
+    g = torch.Generator(device=DEV).manual_seed(n)
+    pages = []
+    for i in range(n):
+        page = torch.randn(layers * 2 * kv * 64 * hd, generator=g, device=DEV)
+        if i % 2 == 0:
+            page[torch.rand(page.shape, generator=g, device=DEV) < 0.98] = 0
+        pages.append(page.to(BF))
+    return pages
+
+
+def test_page_serialiser_reuses_its_pinned_buffers():
+    """Buffers that grow and are written again, results that outlive them, and decodes that follow each other while the stream is
+    still busy: every page as a serialiser of its own makes it."""
+    from vllm_production_stack_amd.kv.serde import PageSerde
+
+    def fresh():
+        return PageSerde(4, 2, 64, BF, "cachegen", levels=[31, 31, 15, 15])
+
+    pages, serde = _codec_pages(6), fresh()
+    want = [fresh().encode(p) for p in pages]
+    assert len(want[1]) > 2 * len(want[0])                       # (an eighth more than the last page is what a buffer holds)
+    halves = [serde.quantize(p) for p in pages]                  # payloads that later pages must not overwrite
+    assert [serde.encode(p) for p in pages] == want
+    assert [serde.pack(*h) for h in halves] == want
+    back = [fresh().decode(b, DEV).clone() for b in want]
+    torch.cuda.synchronize()
+    a = torch.randn(4096, 4096, device=DEV)
+    for _ in range(20):                                          # the copies below queue up behind these
+        a = a @ a * 1e-3
+    got = [serde.decode(b, DEV) for b in want]
+    assert all(torch.equal(x, y) for x, y in zip(got, back))
+
+
+def test_page_serialiser_does_not_make_threads_wait_for_each_other(monkeypatch):
+    """A thread in the middle of a page, on its own stream, while another encodes and decodes pages of its own."""
+    import threading
+
+    from vllm_production_stack_amd.kv.serde import PageSerde
+
+    pages, serde = _codec_pages(4), PageSerde(4, 2, 64, BF, "cachegen", levels=[31, 31, 15, 15])
+    want = [serde.encode(p) for p in pages]
+    torch.cuda.synchronize()
+    inside, done, out, real = threading.Event(), threading.Event(), {}, ops.rans_encode_into
+
+    def slow(*args, **kw):
+        r = real(*args, **kw)
+        if threading.current_thread().name == "slow":
+            inside.set()
+            out["other finished"] = done.wait(20)
+        return r
+
+    def work():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            out["slow"] = serde.encode(pages[0])
+
+    monkeypatch.setattr(ops, "rans_encode_into", slow)
+    t = threading.Thread(target=work, name="slow")
+    t.start()
+    assert inside.wait(20)
+
+    def other():
+        blobs = [serde.encode(p) for p in pages[1:]]
+        out["other"] = blobs, [torch.equal(serde.decode(b, DEV), serde.decode(w, DEV)) for b, w in zip(blobs, want[1:])]
+        done.set()
+
+    u = threading.Thread(target=other)
+    u.start()
+    t.join(40)
+    u.join(40)
+    assert out["other finished"] and out["slow"] == want[0] and out["other"] == (want[1:], [True] * 3)
+
+
 def _sampling_reference(row_bf16, temperature, top_p, top_k):
     """Float64 definition of the kept set: (threshold value, kept mass / largest probability, kept count)."""
     import numpy as np

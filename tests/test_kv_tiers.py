@@ -116,6 +116,15 @@ def test_rans_reference_roundtrip_and_gain():
     assert sizes[spc:2 * spc].astype(int).sum() == 0                     # a constant context costs nothing
 
 
+def test_page_serialiser_can_be_copied_and_pickled():
+    import pickle
+
+    page = torch.randn(3 * 2 * 2 * 64 * 64).to(torch.bfloat16)
+    cg = PageSerde(3, 2, 64, torch.bfloat16, "cachegen", levels=[127, 31, 15])
+    for twin in (copy.deepcopy(cg), pickle.loads(pickle.dumps(cg))):
+        assert twin.encode(page) == cg.encode(page)
+
+
 def test_cachegen_rans_payload_restores_like_the_range_coder():
     """Serde kind 2 (quantiser + rANS) read back on a CPU-only host equals kind 1 of the same page."""
     n_layers, n_kv, hd = 3, 1, 128

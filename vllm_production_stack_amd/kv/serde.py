@@ -22,7 +22,7 @@ from __future__ import annotations
 import ctypes
 import os
 import struct
-import threading
+from collections import deque
 
 import numpy as np
 import torch
@@ -35,6 +35,7 @@ SERDE_NAIVE, SERDE_CACHEGEN = 0, 1
 # host range coder, remains for CPU hosts and for blobs already stored
 SERDE_CACHEGEN_RANS = 2
 _RANS_HDR = struct.Struct("<IIQ")  # streams per context, streams, coded bytes
+_KEPT = 2  # pinned buffers a serialiser keeps for each direction
 _HDR = struct.Struct("<4sHHIIIIQ")
 
 _kvio = None
@@ -90,10 +91,31 @@ class PageSerde:
         self._levels_dev: dict = {}
         # Pinned buffers that pages pass through on their way between host and device, each with the event of the copy that
         # last read it: a pageable copy of a page's 3.5 MB takes 0.65 ms to the host and 0.13 ms to the device, a pinned one
-        # 0.07.  One for encoding; two for decoding, so that a page is copied in while the one before is on its way.
-        self._out_lock, self._in_lock = threading.Lock(), threading.Lock()
-        self._out_buf: torch.Tensor | None = None
-        self._in_bufs: list = [[None, None], [None, None]]
+        # 0.07.  A call takes one out and gives it back, so calls of several threads do not wait for each other; at most
+        # two of each kind are kept, which lets one thread copy a page in while the one before is on its way.
+        self._out_bufs: deque = deque()
+        self._in_bufs: deque = deque([(None, None)] * _KEPT)
+
+    def __getstate__(self):  # (pinned buffers, events and device tensors stay with the object they were made for)
+        return {**self.__dict__, "_levels_dev": {}, "_out_bufs": deque(), "_in_bufs": deque([(None, None)] * _KEPT)}
+
+    @staticmethod
+    def _take(bufs: deque, size: int) -> torch.Tensor:
+        """A pinned buffer of at least ``size`` bytes that no copy reads any more."""
+        try:
+            buf, read = bufs.popleft()
+        except IndexError:
+            buf = read = None
+        if read is not None:
+            read.synchronize()
+        if buf is None or buf.numel() < size:
+            buf = torch.empty(size + size // 8, dtype=torch.uint8, pin_memory=True)
+        return buf
+
+    @staticmethod
+    def _give(bufs: deque, buf: torch.Tensor, read=None) -> None:
+        if len(bufs) < _KEPT:
+            bufs.append((buf, read))
 
     def _header(self, payload_len: int) -> bytes:
         return _HDR.pack(MAGIC, 1, self.kind, self.n_layers, self.n_kv, self.head_dim, ops.PAGE,
@@ -108,9 +130,7 @@ class PageSerde:
             return _HDR.pack(MAGIC, 1, SERDE_NAIVE, self.n_layers, self.n_kv, self.head_dim, ops.PAGE,
                              len(raw)) + raw
         if self._rans_ok(flat.device):
-            with self._out_lock:
-                payload = self._rans_page(flat)
-                return b"".join((self._rans_header(payload.size), memoryview(payload)))
+            return self._rans_page(flat, lambda payload: b"".join((self._rans_header(payload.size), memoryview(payload))))
         sym_np, sc_np = self.quantize(flat)
         return self.pack(sym_np, sc_np)
 
@@ -124,8 +144,7 @@ class PageSerde:
         Otherwise the int8 symbols and fp32 scales come back for the host range coder
         -> (symbols, scales)."""
         if self._rans_ok(flat.device):
-            with self._out_lock:
-                return self._rans_page(flat).copy(), None
+            return self._rans_page(flat, np.copy), None
         sym, scales = ops.cachegen_encode(flat.contiguous(), self._levels(flat.device), self.unit_elems, self.n_layers)
         return sym.cpu().numpy(), scales.float().cpu().numpy()
 
@@ -135,9 +154,9 @@ class PageSerde:
             lv = self._levels_dev[device] = torch.tensor(self.levels, dtype=torch.int32, device=device)
         return lv
 
-    def _rans_page(self, flat: torch.Tensor) -> np.ndarray:
-        """The kind-2 payload of a page, in the pinned buffer (valid until the lock is given up).  Every stage writes its part
-        of the payload where it belongs; one copy brings the finished payload over."""
+    def _rans_page(self, flat: torch.Tensor, finish):
+        """``finish`` of a page's kind-2 payload, which lies in a pinned buffer until it returns.  Every stage writes its part of
+        the payload where it belongs; one copy brings the finished payload over."""
         n, dev, n_streams = flat.numel(), flat.device, self.n_layers * ops.RANS_SPC
         a = _RANS_HDR.size
         o = np.cumsum([0, 4 * (n // 64), 512 * self.n_layers, 4 * n_streams, 2 * n_streams]).tolist()
@@ -149,13 +168,14 @@ class PageSerde:
         if bad:
             raise RuntimeError("rans_encode: frequency table could not be normalised")
         size = a + o[4] + total
-        if self._out_buf is None or self._out_buf.numel() < size:
-            self._out_buf = torch.empty(size + size // 8, dtype=torch.uint8, pin_memory=True)
-        self._out_buf[a:size].copy_(body[:o[4] + total], non_blocking=True)
+        buf = self._take(self._out_bufs, size)
+        buf[a:size].copy_(body[:o[4] + total], non_blocking=True)
         torch.cuda.current_stream(dev).synchronize()
-        payload = self._out_buf.numpy()[:size]
+        payload = buf.numpy()[:size]
         payload[:a] = np.frombuffer(_RANS_HDR.pack(ops.RANS_SPC, n_streams, total), dtype=np.uint8)
-        return payload
+        done = finish(payload)
+        self._give(self._out_bufs, buf)
+        return done
 
     def rans_payload(self, sym: torch.Tensor, scales: torch.Tensor) -> np.ndarray:
         """Entropy-code quantised symbols where they are and return the kind-2 payload bytes."""
@@ -242,18 +262,13 @@ class PageSerde:
         """Host bytes on ``device``, through the next pinned buffer on a GPU (without waiting for the copy)."""
         if torch.device(device).type != "cuda":
             return torch.from_numpy(data.copy()).to(device)
-        with self._in_lock:
-            buf, read = slot = self._in_bufs[0]
-            self._in_bufs.reverse()
-            if read is not None:
-                read.synchronize()  # the copy that last read it has left
-            if buf is None or buf.numel() < data.size:
-                buf = slot[0] = torch.empty(data.size + data.size // 8, dtype=torch.uint8, pin_memory=True)
-            np.copyto(buf.numpy()[:data.size], data)
-            body = torch.empty(data.size, dtype=torch.uint8, device=device)
-            body.copy_(buf[:data.size], non_blocking=True)
-            slot[1] = torch.cuda.Event()
-            slot[1].record(torch.cuda.current_stream(body.device))
+        buf = self._take(self._in_bufs, data.size)
+        np.copyto(buf.numpy()[:data.size], data)
+        body = torch.empty(data.size, dtype=torch.uint8, device=device)
+        body.copy_(buf[:data.size], non_blocking=True)
+        read = torch.cuda.Event()
+        read.record(torch.cuda.current_stream(body.device))
+        self._give(self._in_bufs, buf, read)
         return body
 
     def restore(self, got: tuple, device) -> torch.Tensor:
