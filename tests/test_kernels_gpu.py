@@ -764,6 +764,20 @@ def test_cachegen_page_on_gpu_uses_the_rans_stage_and_matches_the_host_coder(mon
     assert (on_cpu - back.float()).abs().max().item() <= 0.02 * back.float().abs().max().item()
 
 
+def test_rans_takes_sizes_of_other_types_and_refuses_uneven_symbols():
+    from vllm_production_stack_amd.kv.serde import PageSerde
+
+    n_ctx, spc, n = 2, 256, 2 * 256 * 40
+    sym = torch.randint(-9, 10, (n,), device=DEV, dtype=torch.int8)
+    freq, states, sizes, coded = ops.rans_encode(sym, n_ctx, spc)
+    wide = torch.stack([freq, freq], 1)[:, 0]                      # every second value of a buffer
+    assert torch.equal(ops.rans_decode(wide, states, sizes.int(), coded, n, n_ctx, spc), sym)
+    with pytest.raises(ValueError):
+        ops.rans_encode(sym[:-8], n_ctx, spc)
+    with pytest.raises(ValueError):                                # no page of four layers
+        PageSerde(4, 2, 64, BF, "cachegen").encode(torch.zeros(9 * 8192 + 64, device=DEV, dtype=BF))
+
+
 def _codec_pages(n, geometry=(4, 2, 64)):
     """Pages that code to sizes between a few and nearly all of their symbols, small and large in turn."""
     layers, kv, hd = geometry

@@ -1151,8 +1151,6 @@ def rans_encode(sym, n_ctx, spc=RANS_SPC):
         sym = sym.clone()
     n, dev = sym.numel(), sym.device
     n_streams = n_ctx * spc
-    if n % n_ctx or (n // n_ctx) % spc:
-        raise ValueError("rans_encode: symbols do not divide into contexts / streams")
     freq = torch.empty(n_ctx * 256, dtype=torch.int16, device=dev)
     states = torch.empty(n_streams, dtype=torch.int32, device=dev)
     sizes = torch.empty(n_streams, dtype=torch.int16, device=dev)
@@ -1168,6 +1166,8 @@ def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC):
     synchronisation -> int64 [2] on the device: coded bytes, and contexts whose table could not be normalised (nothing of
     the result is valid unless 0)."""
     n, dev, lib = sym.numel(), sym.device, _kernels()
+    if n % n_ctx or (n // n_ctx) % spc:
+        raise ValueError("rans_encode: symbols do not divide into contexts / streams")
     n_streams = n_ctx * spc
     assert sym.is_cuda and sym.is_contiguous() and sym.element_size() == 1 and sym.data_ptr() % 4 == 0
     assert all(t.is_contiguous() and t.numel() * t.element_size() >= b for t, b in (
@@ -1189,7 +1189,9 @@ def rans_decode(freq, states, sizes, coded, n, n_ctx, spc=RANS_SPC):
         return torch.from_numpy(out.view(np.int8).copy())
     dev = coded.device
     lib = _kernels()
+    freq, states, sizes = freq.contiguous(), states.contiguous(), sizes.to(torch.int16).contiguous()
     assert coded.is_contiguous() and freq.numel() >= n_ctx * 256 and min(states.numel(), sizes.numel()) >= n_ctx * spc
+    assert freq.element_size() == 2 and states.element_size() == 4 and all(t.device == dev for t in (freq, states, sizes))
     ws = torch.empty(max(1, int(lib.vpsa_rans_decode_workspace(c_long(n), c_int(n_ctx), c_int(spc)))), dtype=torch.uint8, device=dev)
     sym = torch.empty(n, dtype=torch.int8, device=dev)
     _check(lib.vpsa_rans_decode(_p(coded), c_long(coded.numel()), _p(states), _p(freq), _p(sizes), _p(ws), _p(sym), c_long(n),
