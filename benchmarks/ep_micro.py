@@ -56,7 +56,8 @@ def main():
     for t in [int(v) for v in a.tokens.split(",")]:
         x = torch.randn(t, H, device=DEV).to(torch.bfloat16)
         w, ids = ops.moe_topk_softmax(torch.randn(t, E, device=DEV).to(torch.bfloat16), K)
-        fn = ops.moe_experts_grouped if t <= ops.MOE_MFMA_MAX_TOKENS else ops.moe_experts_prefill
+        sliced_fn, whole_fn = (ops.moe_experts_grouped if ops.moe_streams_experts(t, K, e) else ops.moe_experts_prefill
+                               for e in (E, per))
         state = {"i": 0}
 
         def nxt(ws):
@@ -65,7 +66,7 @@ def main():
 
         def run_sliced():
             w13, w2 = nxt(sliced)
-            fn(x, w13, w2, ids, w)
+            sliced_fn(x, w13, w2, ids, w)
 
         row = {"tokens": t, "ranks": n, "sliced_ms": round(timed(run_sliced, a.iters), 3)}
         per_rank = []
@@ -74,7 +75,7 @@ def main():
 
             def run_whole():
                 w13, w2 = nxt(whole)
-                fn(x, w13, w2, lids, lw, foreign=True)
+                whole_fn(x, w13, w2, lids, lw, foreign=True)
 
             per_rank.append({"pairs": int((lids < per).sum()), "ms": round(timed(run_whole, a.iters), 3)})
         row["whole_per_rank"] = per_rank

@@ -1187,7 +1187,7 @@ def test_moe_prefill_grouped_gemm_experts(t, hidden, inter, skew):
 
 
 @pytest.mark.parametrize("t,hidden,inter,ranks,skew", [
-    (3, 512, 1024, 2, False), (40, 512, 1024, 4, False), (40, 512, 1024, 2, True),
+    (3, 512, 1024, 2, False), (40, 512, 1024, 4, False), (40, 512, 1024, 2, True), (96, 512, 1024, 2, True),
     (300, 512, 1024, 2, False), (1024, 512, 1024, 4, True), (2048, 4096, 14336, 2, False)])
 def test_moe_expert_parallel_ranks_sum_to_the_whole_layer(t, hidden, inter, ranks, skew):
     """Expert parallelism: every rank holds a range of whole experts and runs only the pairs routed
@@ -1214,7 +1214,8 @@ def test_moe_expert_parallel_ranks_sum_to_the_whole_layer(t, hidden, inter, rank
         # poison what the allocator hands out next: rows of foreign pairs are never written and must not be read
         junk = torch.full((t * k, max(hidden, inter)), float("nan"), device=DEV, dtype=BF)
         del junk
-        fn = ops.moe_experts_grouped if t <= ops.MOE_MFMA_MAX_TOKENS else ops.moe_experts_prefill
+        fn = ops.moe_experts_grouped if ops.moe_streams_experts(t, k, per) else ops.moe_experts_prefill
+        assert (fn is ops.moe_experts_grouped) == (t < 300)   # (96 rows of one expert: two passes over its weights)
         out = fn(x, mine[0], mine[1], lids, lw, foreign=True).float()
         assert torch.isfinite(out).all()
         total += out

@@ -17,7 +17,9 @@ def any_shape(monkeypatch):
 
 
 @pytest.mark.parametrize("m", [1, 16, 17, 33, 48, 63, 80, 97, 112, 127, 128, 129, 200, 256])
-@pytest.mark.parametrize("n,k,kind", [(128, 64, ""), (256, 192, "bias"), (128, 1088, ""), (256, 2624, "bias"), (384, 1088, "pair"), (256, 128, "pair")])
+@pytest.mark.parametrize("n,k,kind", [(128, 64, ""), (256, 192, "bias"), (128, 1088, ""), (256, 2624, "bias"), (384, 1088, "pair"), (256, 128, "pair"),
+                                      # eight, nine and seventeen ranges of the reduction: its sums are read eight at a time
+                                      (256, 4096, ""), (256, 4672, "bias"), (128, 8704, ""), (256, 4672, "pair"), (128, 8704, "pair")])
 def test_matches_float64(any_shape, m, n, k, kind):
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     x = torch.randn(m, k + 8, generator=g, device=DEV).to(BF)[:, :k]   # rows of a wider tensor
@@ -25,6 +27,8 @@ def test_matches_float64(any_shape, m, n, k, kind):
     b = torch.randn(n, generator=g, device=DEV).to(BF) if kind == "bias" else None
     got = ops._mid_gemm(x, w, b, kind == "pair")
     assert got is not None
+    if k >= 4096:
+        assert ops._mid_splits(m, n, k, kind == "pair") == {4096: 8, 4672: 9, 8704: 17}[k]
     want = x.double() @ w.double().t()
     if kind == "pair":
         want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
@@ -65,6 +69,7 @@ def test_operands_on_another_device_are_refused(m):
     assert ops.linear_add_norm(x, w, res, b.cpu(), 1e-5) is None
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 @pytest.mark.parametrize("m", [24, 90])
 def test_calls_that_something_follows_stay_with_the_library(m):
     """Gradients of the bias alone, forward-mode tangents, vmap and traces, at rows where the kernel takes plain calls."""
@@ -159,7 +164,8 @@ def test_experts_off_the_16_byte_boundary():
     assert torch.equal(ops.moe_experts_grouped(x, w13, w2, ids, wt), ops.moe_experts_grouped(x.clone(), w13.clone(), w2.clone(), ids, wt))
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 256, 1024), (3, 1280, 1088), (16, 4096, 1024), (17, 5120, 1088), (40, 8192, 2624), (130, 128, 1088)])
+@pytest.mark.parametrize("m,n,k", [(1, 256, 1024), (3, 1280, 1088), (16, 4096, 1024), (17, 5120, 1088), (40, 8192, 2624), (130, 128, 1088),
+                                   (5, 256, 4096), (3, 256, 4672), (17, 384, 8704)])
 def test_sum_with_residual_and_norm(any_shape, m, n, k):
     """One reduction against the separate passes: the same roundings, so the residual stream is equal and the norm differs by its
     sum of squares' order (one unit in the last place of 16 bits)."""
@@ -176,11 +182,12 @@ def test_sum_with_residual_and_norm(any_shape, m, n, k):
     assert ops.linear_add_norm(x[:, 1:], w[:, 1:].contiguous(), res, ln, 1e-5) is None and torch.equal(res, kept)
 
 
-@pytest.mark.parametrize("m,n_q,n_kv,bias", [(1, 32, 8, False), (3, 5, 1, True), (17, 8, 8, True), (40, 32, 8, False)])
-def test_sum_with_rotation_and_cache_write(any_shape, m, n_q, n_kv, bias):
+@pytest.mark.parametrize("m,n_q,n_kv,bias,k", [(1, 32, 8, False, 1088), (3, 5, 1, True, 1088), (17, 8, 8, True, 1088), (40, 32, 8, False, 1088),
+                                               (5, 2, 1, False, 4096), (3, 2, 1, True, 4672), (17, 4, 1, False, 8704)])
+def test_sum_with_rotation_and_cache_write(any_shape, m, n_q, n_kv, bias, k):
     """Query rows and the pages that a decode step's projection leaves against the separate passes, one row without a slot."""
     g = torch.Generator(device=DEV).manual_seed(m)
-    k, n = 1088, (n_q + 2 * n_kv) * 128
+    n = (n_q + 2 * n_kv) * 128
     x = torch.randn(m, k, generator=g, device=DEV).to(BF)
     w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF)
     b = torch.randn(n, generator=g, device=DEV).to(BF) if bias else None
@@ -195,3 +202,92 @@ def test_sum_with_rotation_and_cache_write(any_shape, m, n_q, n_kv, bias):
     ops.rope_and_cache(qkv, positions, slots, cos_sin, want_pool, 1, n_q, n_kv, 128)
     q = ops.decode_qkv(x, w, b, pool, 1, positions, slots, cos_sin, n_q, n_kv)
     assert torch.equal(q, qkv[:, :n_q * 128]) and torch.equal(pool, want_pool)
+
+
+def _decoder(layers, g):
+    import dataclasses
+
+    from vllm_production_stack_amd.engine.config import PRESETS
+    from vllm_production_stack_amd.models.transformer import LayerWeights, TransformerModel
+
+    cfg = dataclasses.replace(PRESETS["llama-3-8b"], num_layers=layers, hidden_size=1024, intermediate_size=2048, num_heads=8,
+                              num_kv_heads=2, vocab_size=1024)
+    h, i, d = cfg.hidden_size, cfg.intermediate_size, cfg.head_dim
+    model = TransformerModel(cfg, BF, DEV, 1024)
+
+    def rnd(*shape, std=None):
+        return torch.empty(shape, device=DEV, dtype=BF).normal_(0, std or shape[-1] ** -0.5, generator=g)
+
+    for _ in range(layers):
+        lw = LayerWeights()
+        lw.ln1, lw.ln2 = rnd(h, std=0.3) + 1, rnd(h, std=0.3) + 1
+        lw.wqkv, lw.wo = rnd((cfg.num_heads + 2 * cfg.num_kv_heads) * d, h), rnd(h, cfg.num_heads * d)
+        lw.w_gate_up, lw.w_down = rnd(2 * i, h), rnd(h, i)
+        model.layers.append(lw)
+    model.embed, model.norm, model.lm_head = rnd(cfg.vocab_size, h, std=1), rnd(h, std=0.3) + 1, rnd(cfg.vocab_size, h)
+    return cfg, model
+
+
+@pytest.mark.parametrize("grouped", [False, True])
+@torch.inference_mode()
+def test_decoder_steps_with_the_fused_reductions(monkeypatch, grouped):
+    """A decode step (one row without a slot, as in a padded graph) and a short prefill of three layers, with the reductions that also
+    update the residual stream, make the norm, rotate and write the cache, against the separate passes."""
+    from vllm_production_stack_amd.models.batch import BatchMeta
+
+    g = torch.Generator(device=DEV).manual_seed(11)
+    layers = 4 if grouped else 3
+    cfg, model = _decoder(layers, g)
+    nq, nkv, d = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
+    ctx = [1, 64, 65, 200, 300, 1]
+    table = torch.arange(6 * 5, dtype=torch.int32, device=DEV).view(6, 5)
+    start = torch.randn(31, layers, 2, nkv, 64 * d, generator=g, device=DEV).to(BF)
+
+    def pool():
+        return ops.LayerGroupedPool([start[:, :2].clone(), start[:, 2:].clone()]) if grouped else start.clone()
+
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    slots = table.gather(1, (pos // 64).long()[:, None])[:, 0].long() * 64 + pos % 64
+    slots[5] = -1
+    decode = BatchMeta(positions=pos, slots=slots, num_decode=6)
+    decode.dec_block_tables, decode.dec_ctx_lens = table, pos + 1
+    decode.dec_num_splits = 3
+    lens, total = [13, 40], 53
+    pre = BatchMeta(positions=torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV),
+                    slots=torch.cat([torch.arange(s * 320, s * 320 + n) for s, n in enumerate(lens)]).to(DEV))
+    pre.num_prefill_seqs, pre.pre_block_tables = 2, table[:2].contiguous()
+    pre.pre_ctx_lens = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    pre.pre_cu_q = torch.tensor([0, 13, 53], dtype=torch.int32, device=DEV)
+    pre.pre_tile_rows = ops.prefill_tile_rows(lens, nq, nkv)
+    ts, tq = ops.build_prefill_tiles(lens, nq, nkv, pre.pre_tile_rows, lens)
+    pre.pre_tile_seq, pre.pre_tile_q0 = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in (ts, tq))
+
+    def run(meta, rows):
+        p = pool()
+        ids = torch.arange(rows, device=DEV) * 17 % cfg.vocab_size
+        y = model.compute_logits(model.forward(ids, p, meta))
+        return y.float(), (torch.cat(p.groups, 1) if grouped else p).float()
+
+    was = ops.set_skinny_gemm(False)
+    want = [run(decode, 6), run(pre, total)]
+    ops.set_skinny_gemm(was)
+    monkeypatch.setattr(ops, "MID_MIN_FILL", 0.0)
+    taken = {"linear_add_norm": 0, "decode_attention_block": 0}
+    for name in taken:
+        def spy(*args, _name=name, _real=getattr(ops, name), **kw):
+            r = _real(*args, **kw)
+            taken[_name] += r is not None
+            return r
+        monkeypatch.setattr(ops, name, spy)
+    got = [run(decode, 6)]
+    assert taken == {"linear_add_norm": 2 * layers - 1, "decode_attention_block": layers}   # (the last down projection has no norm behind it)
+    got.append(run(pre, total))
+    assert taken == {"linear_add_norm": 2 * (2 * layers - 1), "decode_attention_block": layers}
+    for (y, p), (yw, pw) in zip(got, want):
+        # sums in another order flip last places of 16 bits, 2^-8 of a value at most (a cached entry), and three or four layers
+        # pass them on: 0.7 to 0.9 % of the logits' norm
+        assert float((y - yw).norm() / yw.norm()) < 2e-2
+        assert float((p - pw).norm() / pw.norm()) < 2 ** -8
+    untouched = torch.ones(31, dtype=torch.bool, device=DEV)
+    untouched[(slots[:5] // 64)] = False
+    assert torch.equal(got[0][1][untouched], start.float()[untouched])                      # nothing went to the row without a slot

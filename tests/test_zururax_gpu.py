@@ -148,12 +148,13 @@ def test_gemm_epilogues():
     assert close(ops.up_relu_sq(x.cuda(), w[0].cuda()), torch.relu(x.double() @ w[0].double().T) ** 2, 2e-2)
 
 
-@pytest.mark.parametrize("tokens", [1, 5, 40, 100])
+@pytest.mark.parametrize("tokens", [1, 5, 40, 100, 144, 145, 300])
 def test_mixture_units_small_and_large_batches(tokens):
-    """The routed units over sorted pairs: the weight-streaming kernels of decode-sized batches and the
-    grouped prefill GEMM give what the float64 definition gives."""
+    """The routed units over sorted pairs: the weight-streaming kernels of decode-sized batches (up to 48 rows a unit on
+    average) and the grouped prefill GEMM give what the float64 definition gives."""
     g = torch.Generator().manual_seed(tokens)
     e, hidden, inter, top = 6, 128, 512, 2
+    assert ops.moe_streams_experts(tokens, top, e) == (tokens <= 144)
     x = torch.randn(tokens, hidden, generator=g).to(torch.bfloat16)
     w13 = (torch.randn(e, 2 * inter, hidden, generator=g) * hidden ** -0.5).to(torch.bfloat16)
     w2 = (torch.randn(e, hidden, inter, generator=g) * inter ** -0.5).to(torch.bfloat16)
