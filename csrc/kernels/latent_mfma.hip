@@ -604,7 +604,8 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
            const void* cache, long page_stride, const int* block_tables, int bt_stride, const int* tiles,
            const int* positions, int n_tiles, int heads, const float* sink, void* out, long o_row, long o_head,
            float scale, int window, int splits, float* ws_o, float* ws_ml, int bucket, hipStream_t st) {
-  // entries of 512 + 64 values: pages straight into LDS (narrower ones keep three waves per SIMD in the kernel above)
+  // entries of 512 + 64 values: pages straight into LDS.  (A quarter of the channels has to be a block of eight 16-channel tiles, which
+  // leaves 512; of the others, those of up to 256 values have three waves per SIMD in the kernel above to hide their staging.)
   static bool attr_set[2] = {false, false};
   auto ready = [](const void* kernel, int lds, bool* done) {
     if (!*done) *done = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;

@@ -50,7 +50,8 @@ __global__ __launch_bounds__(256) void rans_hist_kernel(const uint8_t* __restric
   part[((long)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x] = h[threadIdx.x];
 }
 
-// What the encoder needs of a symbol of frequency f and start c.  With s = ceil(log2 f) and m = ceil(2^(31 + s) / f) the
+// What the encoder needs of a symbol of frequency f and start c: the published reciprocal form of the byte-wise rANS encoder
+// (F. Giesen's ryg_rans, after R. Alverson, "Integer Division Using Reciprocals").  With s = ceil(log2 f) and m = ceil(2^(31 + s) / f) the
 // quotient x / f of x < 2^31 is floor(x m / 2^(31 + s)): the product is off by less than x f / (f 2^(31 + s)) < 1 / f.  The new
 // state (x / f) 4096 + x % f + c is x + (x / f) (4096 - f) + c.  f = 1 would need m = 2^31 and a shift to the left; m = 2^32 - 1
 // gives x - 1 instead (x >= 1), and c + 4095 makes up for it.

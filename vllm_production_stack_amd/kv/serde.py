@@ -178,7 +178,8 @@ class PageSerde:
         return done
 
     def rans_payload(self, sym: torch.Tensor, scales: torch.Tensor) -> np.ndarray:
-        """Entropy-code quantised symbols where they are and return the kind-2 payload bytes."""
+        """The kind-2 payload of symbols that are quantised already, coded where they lie: on a CPU-only host the definition
+        that ``encode``'s pages on a GPU are equal to."""
         freq, states, sizes, coded = ops.rans_encode(sym.view(-1), self.n_layers)
         body = torch.cat([scales.float().contiguous().view(-1).view(torch.uint8),
                           freq.view(torch.uint8), states.view(torch.uint8), sizes.view(torch.uint8), coded])

@@ -96,6 +96,7 @@ def add_dyt_norm(residual, deltas, weight, bias, alpha, out_dtype, want_out: boo
 
 
 SCAN_FOLD_MIN_DECAY = 0.1    # decay^-16 stays below 1e16
+# Both measured for the walk token by token; the block form (``_retention_blocks``) joins neighbouring pieces into runs of its own.
 SCAN_PIECE_MIN_ROWS = 128   # sequences of a step shorter than this are walked in one go
 SCAN_PIECES_TARGET = 96     # pieces per launch that fill the chip (times heads and column blocks)
 
