@@ -271,23 +271,28 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //     row / 8 % 2 (applied to the source address: a wave's load fills 1 KiB of LDS in lane order).  The 16 rows of a K fragment
 //     then cover all banks, and so do the 8 rows x 32 bytes that half a wave reads transposed.
 //   * ds_read_b64_tr_b16 gives lane (c, g) the keys 4 g .. 4 g + 3 of channel c: the order in which the S accumulators hold them.
-//   * Two pages are on their way except while one is multiplied: the page after next is asked for as soon as its buffer is free,
-//     before the next one is waited for (a counted wait).  Waiting for each page before asking for another left 4.5 TB/s.
+//   * Two pages are on their way except while one is read: the page after next is asked for as soon as its buffer is free, before
+//     the next one is waited for (a counted wait).  Waiting for each page before asking for another left 4.5 TB/s.
 //   * Decode rows of at most 32 heads (QUARTERS): eight waves, four of which share 16 slots.  Each scores 16 keys of a page, the
 //     four exchange scores through 8 KB of LDS, keep the same softmax state and sum a quarter of the channels over all 64 keys.
 //     (With keys and states of its own a wave held all channels, and joining the four moved 130 KB through LDS at the end: 4 to 5 us
-//     that ranges of one or two pages could not hide.)  With 64 slots a tile keeps four waves busy by itself.
+//     that ranges of one or two pages could not hide.)  A quarter of a page's values fits into registers beside the rest, so the
+//     page is read whole before the scores go round: that barrier frees its buffer, and softmax and second product run with two
+//     pages on their way (one sequence of 26k entries 52 -> 49 us, 200 of 2k 115 -> 104).
+//     The weights enter as two parts of 16 bits, a matrix instruction more for every value fragment that is read: with one part and
+//     one maximum for all 64 keys the error against 64 bits was 2.03e-3 on average over batches and contexts, with a maximum for
+//     each quarter 1.97e-3, with two parts it is 1.66e-3, the rounding of the result.
+//     With 64 slots a tile keeps four waves busy by itself.
 //   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
 // Decode rows with their merge, in a graph, pages from memory; staged through registers / this: 32 heads, 32 sequences of 4k entries in 8
-// ranges 65 / 40 us, 8 of 8k in 32 42 / 31, one of 26k in 32 86 / 48, one of 2k, a page a range, 17.4 / 17.7; 16 heads, one of 2k 16.0 / 15.1.
-// Prefill tiles, 1500 rows of 16 heads behind 4500 entries: 855 / 728.
+// ranges 65 / 40 us, 8 of 8k in 32 42 / 32, one of 26k in 32 86 / 49, one of 3k 22.9 / 21.0, one of 2k, a page a range, 17.4 / 18.0; 16 heads,
+// one of 2k 16.1 / 15.4.  Prefill tiles, 1500 rows of 16 heads behind 4500 entries: 855 / 728.
 
 // o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
 // their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
 // channels a tile, keys 16 apart, eight tiles a block.
 template <int ROW, int J>
-__device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8& pf, const uint32_t (&at)[4]) {
-  u32x2 r[16];
+__device__ __forceinline__ void read_transposed(u32x2 (&r)[16], const uint32_t (&at)[4]) {
   asm volatile(
       "ds_read_b64_tr_b16 %0, %16 offset:%20\n\tds_read_b64_tr_b16 %1, %16 offset:%21\n\t"
       "ds_read_b64_tr_b16 %2, %17 offset:%20\n\tds_read_b64_tr_b16 %3, %17 offset:%21\n\t"
@@ -303,22 +308,36 @@ __device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8& pf, 
       : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(J * 256), "n"(J * 256 + 16 * ROW), "n"(J * 256 + 128),
         "n"(J * 256 + 128 + 16 * ROW)
       : "memory");
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const u32x4 a = {r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]};
-    o[8 * J + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), pf, o[8 * J + i], 0, 0, 0);
-  }
 }
 
-template <int ROW, int... J>
-__device__ __forceinline__ void all_products(f32x4* o, const bf16x8& pf, const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
+// PARTS 2: the weights in two parts of 16 bits, high and low.
+template <int PARTS>
+__device__ __forceinline__ void multiply_tiles(f32x4* o, const u32x2 (&r)[16], const bf16x8 (&pf)[PARTS]) {
+#pragma unroll
+  for (int part = 0; part < PARTS; ++part)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const u32x4 a = {r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]};
+      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), pf[part], o[i], 0, 0, 0);
+    }
+}
+
+template <int ROW, int J, int PARTS>
+__device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8 (&pf)[PARTS], const uint32_t (&at)[4]) {
+  u32x2 r[16];
+  read_transposed<ROW, J>(r, at);
+  multiply_tiles(o + 8 * J, r, pf);
+}
+template <int ROW, int PARTS, int... J>
+__device__ __forceinline__ void all_products(f32x4* o, const bf16x8 (&pf)[PARTS], const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
   (transposed_products<ROW, J>(o, pf, at), ...);
 }
+
 // How many of `splits` key ranges a decode row of `pages` pages is cut into.  A workgroup fills a CU (two pages in LDS) and what it
 // does once - queries, the first page's way, a partial result of 64 KB - takes about as long as four pages (two or three give the
 // same times), so more workgroups than a round of 256 only pay if their ranges are long: 100 sequences of 1000 entries in 8 ranges
-// of two pages were four rounds.  In a graph with the merge, all ranges / those used: 100 x 1000 entries 72 / 42 us, 40 x 3000 (7 / 6) 55 / 40,
-// 33 x 12000 (8 / 7) 139 / 94; 128 x 100, where a row has two pages, 22.5 / 24.
+// of two pages were four rounds.  In a graph with the merge, all ranges / those used: 100 x 1000 entries 74 / 43 us, 40 x 3000 (7 / 6) 56 / 42,
+// 33 x 12000 (8 / 7) 139 / 97; 128 x 100, where a row has two pages, 23 / 24.5.
 // `rows` are those of the step's batch bucket, not of the launch: a row's ranges, and with them the order of its sums, are the same
 // in a captured step that is padded to the bucket and in an eager one that is not.
 constexpr int WIDE_ONCE = 4;
@@ -430,32 +449,20 @@ __global__ __launch_bounds__(QUARTERS ? 512 : 256, QUARTERS ? 2 : 1) void latent
   for (int i = 0; i < 4; ++i)
     voff[i] = vr * ROW + (((2 * i + ((lane & 3) >> 1)) ^ fv) << 4) + (lane & 1) * 8 + part * DW * 32;
 
-  f32x4* scores = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;  // of four key quarters
-  auto multiply = [&](int p, int buf) {
+  f32x4 s[4];  // scores, then weights, of a page's keys
+  auto score = [&](int buf) {
     const char* img = lds + buf * PAGE_BYTES;
-    f32x4 s[4];
-    if (wave_active) {
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) s[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; ++nt) s[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const bf16x8 a = *reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128 + nt * 16 * ROW);
-          s[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], s[nt], 0, 0, 0);
-        }
-      if constexpr (QUARTERS) scores[part * 64] = s[0];
-    }
-    if constexpr (QUARTERS) {  // (not __syncthreads, which would wait for the page behind this one)
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-    }
-    if (!wave_active) return;
-    if constexpr (QUARTERS) {
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) s[nt] = scores[nt * 64];
-    }
+      for (int nt = 0; nt < NT; ++nt) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128 + nt * 16 * ROW);
+        s[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], s[nt], 0, 0, 0);
+      }
+  };
+  auto weigh = [&](int p) {
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) s[nt] *= scale2;
     if (p * PAGE + PAGE - 1 > t.pos0 || p * PAGE <= t.pos0 + t.n_tok - 1 - window) {
@@ -495,32 +502,75 @@ __global__ __launch_bounds__(QUARTERS ? 512 : 256, QUARTERS ? 2 : 1) void latent
 #pragma unroll
       for (int dt = 0; dt < DW; ++dt) o[dt] *= corr;
     }
-    const uint32_t page = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + buf * PAGE_BYTES;
+  };
+  auto weights = [&](int kk, bf16x8 (&pf)[QUARTERS ? 2 : 1]) {  // of keys 32 kk ..
+    u32x4 w, low;
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const uint32_t half = page + kk * 32 * ROW;
-      const uint32_t at[4] = {half + voff[0], half + voff[1], half + voff[2], half + voff[3]};
-      const u32x4 w = {pack_bf16x2(s[2 * kk][0], s[2 * kk][1]), pack_bf16x2(s[2 * kk][2], s[2 * kk][3]),
-                       pack_bf16x2(s[2 * kk + 1][0], s[2 * kk + 1][1]), pack_bf16x2(s[2 * kk + 1][2], s[2 * kk + 1][3])};
-      all_products<ROW>(o, __builtin_bit_cast(bf16x8, w), at, std::make_integer_sequence<int, DW / 8>());
+    for (int i = 0; i < 4; ++i) {
+      const float p0 = s[2 * kk + (i >> 1)][2 * (i & 1)], p1 = s[2 * kk + (i >> 1)][2 * (i & 1) + 1];
+      w[i] = pack_bf16x2(p0, p1);
+      if constexpr (QUARTERS) low[i] = pack_bf16x2(p0 - bf16lo(w[i]), p1 - bf16hi(w[i]));
     }
+    pf[0] = __builtin_bit_cast(bf16x8, w);
+    if constexpr (QUARTERS) pf[1] = __builtin_bit_cast(bf16x8, low);
+  };
+  auto everyone = [&]() {  // (not __syncthreads, which would wait for the pages on their way)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   };
 
   if (p_begin < p_end) load_page(p_begin, 0);
   if (p_begin + 1 < p_end) load_page(p_begin + 1, 1);
   for (int p = p_begin; p < p_end; ++p) {
     const int buf = (p - p_begin) & 1;
+    const uint32_t page = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + buf * PAGE_BYTES;
     // this page has landed (mine: all but the NI loads of the page behind it; everyone's: the barrier)
     if (p + 1 < p_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    multiply(p, buf);
-    if (p + 2 < p_end) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // my reads of this buffer are done; everyone's: the barrier
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      load_page(p + 2, buf);
+    if constexpr (QUARTERS) {
+      // a page is read whole before its scores go round: the barrier of that exchange frees its buffer as well
+      f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;  // of four key quarters
+      u32x2 v0[16], v1[16];
+      if (wave_active) {
+        score(buf);
+        round[part * 64] = s[0];
+        const uint32_t at0[4] = {page + voff[0], page + voff[1], page + voff[2], page + voff[3]};
+        read_transposed<ROW, 0>(v0, at0);
+        const uint32_t at1[4] = {at0[0] + 32 * ROW, at0[1] + 32 * ROW, at0[2] + 32 * ROW, at0[3] + 32 * ROW};
+        read_transposed<ROW, 0>(v1, at1);
+      }
+      everyone();
+      if (p + 2 < p_end) load_page(p + 2, buf);
+      if (wave_active) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
+        weigh(p);
+        bf16x8 pf[2];
+        weights(0, pf);
+        multiply_tiles(o, v0, pf);
+        weights(1, pf);
+        multiply_tiles(o, v1, pf);
+      }
+    } else {
+      if (wave_active) {
+        score(buf);
+        weigh(p);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const uint32_t half = page + kk * 32 * ROW;
+          const uint32_t at[4] = {half + voff[0], half + voff[1], half + voff[2], half + voff[3]};
+          bf16x8 pf[1];
+          weights(kk, pf);
+          all_products<ROW>(o, pf, at, std::make_integer_sequence<int, DW / 8>());
+        }
+      }
+      if (p + 2 < p_end) {
+        everyone();  // reads of this buffer are done
+        load_page(p + 2, buf);
+      }
     }
   }
 

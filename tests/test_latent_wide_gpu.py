@@ -51,6 +51,18 @@ def test_decode_rows(heads, splits, window):
     assert float((out.double() - want).norm() / want.norm()) < 6e-3
 
 
+@pytest.mark.parametrize("heads,splits", [(16, 1), (32, 1), (32, 4)])
+def test_weights_are_not_rounded_to_16_bits(heads, splits):
+    ctx = [100, 64, 200, 640, 33]
+    pool, table, q, sink = setup(ctx, [1] * len(ctx), heads, 50 + heads)
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    out = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, None, pos, sink, 0.05, splits=splits)
+    want = expected(pool, table, q, sink, ctx, [1] * len(ctx), 0.05, 1 << 30)
+    # only the result is: an error evenly spread over half a unit in the last place is 2^-9 / sqrt(3) of a power of two, 1.7e-3 of
+    # values spread over a binade; weights in 16 bits add as much again
+    assert float((out.double() - want).norm() / want.norm()) < 1.8e-3
+
+
 @pytest.mark.parametrize("heads,rows,splits,window", [(16, 43, 6, 1 << 30), (32, 100, 8, 1 << 30), (64, 33, 8, 1 << 30), (16, 90, 3, 200), (70, 300, 2, 64)])
 def test_decode_batches_beyond_a_round(heads, rows, splits, window):
     """More workgroups than CUs: fewer ranges are used than the caller's workspace holds, and some rows see one page or one key."""
