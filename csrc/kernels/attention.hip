@@ -522,8 +522,27 @@ __device__ __forceinline__ void mfma_s_next(f32x16& d, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "a"(b));
 }
 // Values produced by an asm MFMA are not known to the compiler's hazard recogniser: before vector
-// code reads them (rescale, epilogue) let the matrix pipe drain.
-__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+// code reads them (rescale, epilogue) let the matrix pipe drain.  The values are operands of the wait:
+// one that names nothing orders nothing but memory, and the compiler copied accumulators out in front
+// of it, right behind the MFMAs that were still writing them (`v_mfma a[0:15]`, `v_accvgpr_read a15`).
+// Tiles whose row maxima grew near the diagonal then lost parts of products: 15 to 20 % of the output's
+// norm where scores reach the tens, one register's 64 values in a launch now and then where they are
+// ordinary.  Times are the same (8192 rows, 32 heads over 4 layers: 12.07 -> 12.03 ms a pass).
+__device__ __forceinline__ void mfma_drain(f32x16 (&o)[2][4]) {
+  asm volatile("s_nop 15\n\ts_nop 15"
+               : "+a"(o[0][0]), "+a"(o[0][1]), "+a"(o[0][2]), "+a"(o[0][3]), "+a"(o[1][0]), "+a"(o[1][1]),
+                 "+a"(o[1][2]), "+a"(o[1][3])::"memory");
+}
+__device__ __forceinline__ void mfma_drain(f32x16 (&s)[2]) {
+  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1])::"memory");
+}
+// The other direction: scaled accumulators are written before the two wait states that an MFMA needs
+// behind a vector write of its operands.
+__device__ __forceinline__ void mfma_settle(f32x16 (&o)[2][4]) {
+  asm volatile("s_nop 1"
+               : "+a"(o[0][0]), "+a"(o[0][1]), "+a"(o[0][2]), "+a"(o[0][3]), "+a"(o[1][0]), "+a"(o[1][1]),
+                 "+a"(o[1][2]), "+a"(o[1][3])::"memory");
+}
 // Keeps a value (and the instruction that made it) where the source put it.
 #define VPSA_PIN(x) asm volatile("" : "+v"(x))
 
@@ -684,7 +703,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v3(
   auto rescale = [&](const float (&mt)[2]) {
     const bool grow = (mt[0] > m_run[0] + LAZY_THR) || (mt[1] > m_run[1] + LAZY_THR);
     if (__any(grow)) {
-      mfma_drain();
+      mfma_drain(o_acc);
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
         const float m_new = fmaxf(m_run[rb], mt[rb]);
@@ -696,6 +715,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v3(
 #pragma unroll
           for (int i = 0; i < 16; ++i) o_acc[rb][dt][i] *= alpha;
       }
+      mfma_settle(o_acc);
     }
   };
   auto exp_half = [&](const f32x16 (&s)[2], bf16x8 (&pf)[2][2]) {
@@ -975,7 +995,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v3(
     pv_half(lds + b_cur, 1, pf);
   }
 
-  mfma_drain();
+  mfma_drain(o_acc);
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const float l_tot = l_run[rb] + __shfl_xor(l_run[rb], 32, 64);
@@ -1273,7 +1293,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
   auto rescale = [&](const float (&mt)[2]) {
     const bool grow = (mt[0] > m_run[0] + LAZY_THR) || (mt[1] > m_run[1] + LAZY_THR);
     if (__any(grow)) {
-      mfma_drain();
+      mfma_drain(o_acc);
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
         const float m_new = fmaxf(m_run[rb], mt[rb]);
@@ -1289,7 +1309,9 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
         for (int j = 0; j < 4; ++j)
           pw1[rb][j] = pack_bf16x2(bf16lo(pw1[rb][j]) * alpha, bf16hi(pw1[rb][j]) * alpha);
       }
-      asm volatile("s_nop 1" ::: "memory");
+      VPSA_PIN(pw1[0]);
+      VPSA_PIN(pw1[1]);
+      mfma_settle(o_acc);
     }
   };
   // probabilities of 16-key slice `sh` of the scores `s`, packed; adds their sums to l_run
@@ -1483,7 +1505,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
     l_run[1] += ps[1][0] + ps[1][1];
     if (MASKED) {
       // tiles on the diagonal (at most two per block): mask and maxima after the matrix pipe drained
-      mfma_drain();
+      mfma_drain(sn);
       if (next_tile >= n_full) mask_half(next_tile, ktt, sn);
       max_half(sn, mn);
     } else {
@@ -1556,7 +1578,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
     // (the tail of the loop re-requests the last tile into free buffers: nothing may still be
     // on its way into LDS when this workgroup ends)
     if (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    mfma_drain();
+    mfma_drain(sA);
     if (last > 0) pv_slice(lds + b_wr, 1, 1, pw1);
     u32x4 pk[2];
     rescale(mA);
@@ -1576,7 +1598,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
     pv_slice(lds + b_cur, 1, 1, pk);
   }
 
-  mfma_drain();
+  mfma_drain(o_acc);
   if (!head_ok) return;  // (no barrier below)
   if (part >= 0) {
     // record = [2 row blocks][4 channel tiles][16 values][64 lanes] fp32, then [2][64] maxima and

@@ -174,6 +174,27 @@ def test_paged_prefill_matches_reference(n_q, n_kv, variant):
     assert err < REL_TOL, err
 
 
+@pytest.mark.parametrize("spread", [2, 20])
+@pytest.mark.parametrize("variant", [-1, 4, 5, 6, 7, 8, 9, 10, 11])
+def test_paged_prefill_with_growing_maxima(variant, spread):
+    """Scores of a few units and of tens: row maxima that grow from tile to tile, so that accumulators are read and scaled between
+    matrix instructions, on the diagonal too.  The reference's result, and equal bits in every launch.  (Accumulators read before
+    their matrix instruction had written them: heads off by half and more, and other bits in one launch of a few dozen.)"""
+    torch.manual_seed(8)
+    q_lens = [1000, 999]
+    pool = _v_offset_pool(40, 1, 8, seed=9)
+    bt = _block_tables(2, 16, 40, 10)
+    q = (torch.randn(sum(q_lens), 32 * 128, device=DEV) * spread).to(BF)
+    first, cu, ctx_t, _ = _run_prefill(q, pool, 0, bt, q_lens, q_lens, 32, 8, variant)
+    want = torch.zeros_like(q)
+    ref.paged_prefill(q, want, pool, 0, bt, cu, ctx_t, 32, 8, 128, 1.0 / math.sqrt(128))
+    err = _rel_row_err(first, want, 32)
+    assert err < REL_TOL, err
+    for i in range(100):
+        again = _run_prefill(q, pool, 0, bt, q_lens, q_lens, 32, 8, variant)[0]
+        assert torch.equal(first, again), (i, int((first != again).sum()))
+
+
 @pytest.mark.parametrize("variant", [-1, 8, 9, 10, 11])
 @pytest.mark.parametrize("rope", [False, True])
 @pytest.mark.parametrize("n_q,n_kv", [(32, 8), (28, 4), (12, 4), (10, 2)])
