@@ -1,8 +1,7 @@
 """Sleep and wake a full-size replica (random-init Llama-3-8B, the pool sized from HBM); prints one
 JSON line with the pool layout, the memory given back, the timings and whether the greedy tokens of
 two 3000-token prompts are the same after waking, next to whether a plain repeat without a nap gives
-the same tokens (on random-init weights the logits are nearly tied and full-size runs are not
-bitwise repeatable on either pool layout, so only that pair of answers says anything about the nap).
+the same tokens.
 
     python benchmarks/tools/sleep_wake_full_size.py [--kv-layer-groups G]"""
 import argparse
