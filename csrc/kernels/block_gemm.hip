@@ -1,0 +1,273 @@
+// Products of a few hundred to some ten thousand token rows for gfx950 whose 256 x 256 tiles would not fill the chip's 256 CUs in whole
+// rounds, or whose reductions are short: y[M, N] = epilogue(x[M, K] . W[N, K]^T + bias), tiles of several shapes on one scheme.
+//   * 256 threads, waves as 2 (rows) x 2 (columns); a wave multiplies 16 TM token rows with 16 TN weight rows on
+//     v_mfma_f32_16x16x32_bf16, a workgroup BM = 32 TM rows with BN = 32 TN columns.
+//   * Both operands go from memory straight into LDS in chunks of 64 along K (rows of 128 bytes, 16-byte piece j of row r at
+//     j ^ (r / 2) % 8: the 16 rows of a fragment cover every bank), S chunks in a ring.
+//   * One barrier a chunk, in its middle: the fragments of the chunk's second half and of the next chunk's first half are read while
+//     the matrix cores work on the half before, so that a lone wave on a SIMD keeps them busy; the chunk's place in the ring is
+//     requested again right behind that barrier, S - 1/2 chunks ahead of its use.
+//   * The weight rows are the MFMA's A operand and are ordered so that a lane ends with eight consecutive columns of a token row.
+// What bounds it: LDS, which carries (reads and the loads' writes) 128 bytes for every 64 x 96 x 96 of products in the largest shape, as many
+// cycles as the matrix cores need; with short reductions the time until a tile's first chunk is there and its epilogue (gelu 75
+// cycles of vector work a wave and value).  12000 rows, library with the activation's pass / this: 3072 x 768 with gelu 107 / 70 us,
+// 768 x 3072 57 / 48 (+ residual), three of 768 x 768 62 / 48, 768 x 2304 with gelu 50 / 42; 1500 rows, 2048 x 512 with gelu 26 / 11.
+#include <type_traits>
+
+#include "common.h"
+
+namespace {
+
+constexpr int BK = 64, ROWB = BK * 2;
+
+enum { ACT_NONE = 0, ACT_GELU = 1 };
+
+// Row r of an operand lies at (r / batch_rows) * bs + (r % batch_rows) * ld elements.
+struct Rows {
+  long ld, bs;
+};
+
+struct BlockArgs {
+  const uint16_t* a;
+  const uint16_t* w[3];     // the products of several weights of one shape stand side by side in c
+  const uint16_t* bias[3];  // or null
+  const uint16_t* res;      // added behind the activation, or null
+  uint16_t* c;
+  Rows ar, cr, rr;
+  int batch_rows, M, N, K, n_tiles;  // N: rows of one weight; n_tiles: column tiles of one weight
+  int parts;
+  uint32_t a_bytes, w_bytes;  // ends of the operands, for loads past the reduction's end
+};
+
+// x Phi(x).  Phi(-|x|) = exp(-x^2 / 2) t P(t), t = 1 / (1 + 0.31 |x|), P of degree 5 fitted here to the smallest relative error over
+// 0 <= |x| <= 14: 5e-6, also far out on the negative side.
+__device__ __forceinline__ float gelu(float x) {
+  const float ax = fabsf(x), t = __builtin_amdgcn_rcpf(fmaf(0.31f, ax, 1.f));
+  float p = -0.0739278644f;
+  p = fmaf(p, t, 0.1804467738f);
+  p = fmaf(p, t, 0.0157485195f);
+  p = fmaf(p, t, 0.1334278733f);
+  p = fmaf(p, t, 0.1204417273f);
+  p = fmaf(p, t, 0.1238606647f);
+  const float h = p * t * __builtin_amdgcn_exp2f(x * x * -0.72134752044448170f);
+  return x * (x >= 0.f ? 1.f - h : h);
+}
+
+template <int TM, int TN, int S, int ACT>
+__global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void block_gemm_kernel(const BlockArgs args) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, STAGE = (BM + BN) * ROWB, NL = TM + TN;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, g = lane >> 4, wr = wave >> 1, wc = wave & 1;
+  const int M = args.M, N = args.N, K = args.K;
+
+  // Tiles in blocks of an eighth of the row tiles (up to eight), column by column inside a block, cut in eight runs, one per XCD
+  // (workgroups go round them): those that share an L2 at any time are about a square of tiles.
+  int m0, n0, part;
+  {
+    const int m_tiles = (M + BM - 1) / BM, cols = args.n_tiles * args.parts, total = m_tiles * cols, blk = min(8, (m_tiles + 7) / 8);
+    const int bid = blockIdx.x, xcd = bid & 7, q = total >> 3, r = total & 7;
+    const int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
+    const int block = t / (blk * cols), rem = t - block * blk * cols, rows = min(blk, m_tiles - blk * block);
+    const int col = rem / rows;
+    m0 = (blk * block + rem - col * rows) * BM;
+    part = col / args.n_tiles;
+    n0 = (col - part * args.n_tiles) * BN;
+  }
+
+  // what this lane loads of a chunk: 8 rows of 8 pieces a KiB; rows past the last repeat it
+  uint32_t aoff[TM], woff[TN];
+  const int lrow = lane >> 3;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int r = 8 * (4 * i + wave) + lrow, row = min(m0 + r, M - 1);
+    const int b = row / args.batch_rows;
+    aoff[i] = (uint32_t)((b * args.ar.bs + (row - b * args.batch_rows) * args.ar.ld) * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int r = 8 * (4 * i + wave) + lrow, rr = r % (16 * TN), j = rr & 15, perm = 8 * (j >> 2) + 4 * ((rr >> 4) & 1) + (j & 3);
+    const int col = n0 + r / (16 * TN) * (16 * TN) + 32 * (rr >> 5) + perm;
+    woff[i] = (uint32_t)min(col, N - 1) * (uint32_t)(K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+  }
+  const int n = K / BK;
+  auto load = [&](int c, char* st, int i) {  // the i-th KiB of this wave; nothing past the last chunk (a buffer of no bytes)
+    const bool x = i < TM;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(x ? args.a : args.w[part]), 0, c < n ? (int)(x ? args.a_bytes : args.w_bytes) : 0, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)(st + (4 * i + wave) * 1024), 16,
+                                             (int)(x ? aoff[i % TM] : woff[(i - TM + TN) % TN]), c < n ? c * ROWB : 0, 0, 0);
+  };
+
+  // fragments: row c16 of a 16-row tile, piece 4 ks + g
+  const int fr = c16 * ROWB + ((g ^ (c16 >> 1)) << 4);
+  const int a_rd = wr * 16 * TM * ROWB, w_rd = (BM + wc * 16 * TN) * ROWB;
+  bf16x8 wf[2][TN], xf[2][TM];
+  auto read = [&](const char* st, int ks, int i) {
+    const int f = fr ^ (ks << 6);
+    if (i < TM) xf[ks][i % TM] = *reinterpret_cast<const bf16x8*>(st + a_rd + i * 2048 + f);
+    else wf[ks][(i - TM + TN) % TN] = *reinterpret_cast<const bf16x8*>(st + w_rd + (i - TM) * 2048 + f);
+  };
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  // Half a chunk: its matrix instructions, between the first two thirds of them the reads of the half that follows (from `from`) and
+  // between all of them the requests [lo, hi) of a later chunk c (into `to`).  The order is written out: left alone, the compiler puts
+  // all loads in front.
+  auto half = [&](int ks, const char* from, int lo, int hi, int c, char* to) {
+    constexpr int MMA = TM * TN, R = TM + TN, PER = MMA * 2 / (3 * R) > 0 ? MMA * 2 / (3 * R) : 1;
+#pragma unroll
+    for (int m = 0; m < MMA; ++m) {
+      acc[m / TM][m % TM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][m / TM], xf[ks][m % TM], acc[m / TM][m % TM], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (m % PER == 0 && m / PER < R) read(from, ks ^ 1, m / PER);
+#pragma unroll
+      for (int q = m * (hi - lo) / MMA; q < (m + 1) * (hi - lo) / MMA; ++q) load(c, to, lo + q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = (MMA - 1) / PER + 1; i < R; ++i) read(from, ks ^ 1, i);
+  };
+  // A chunk's place is free from the middle of the chunk on.  Three places and more: the requests into it are spread over a whole
+  // chunk's time; with two they all go out in the half that follows.
+  constexpr int L0 = S > 2 ? NL / 2 : NL;
+
+#pragma unroll
+  for (int c = 0; c < S; ++c) {
+#pragma unroll
+    for (int i = 0; i < (c < S - 1 ? NL : L0); ++i) load(c, lds + c * STAGE, i);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * NL + L0) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  char *st = lds, *prev = lds + (S - 1) * STAGE;
+#pragma unroll
+  for (int i = 0; i < NL; ++i) read(st, 0, i);
+  for (int c = 0; c < n; ++c) {
+    half(0, st, L0, NL, c + S - 1, prev);
+    // chunk c + 1 has landed (mine: all but the loads of the chunks behind it) and my reads of chunk c are done; everyone's: the barrier
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * NL) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    prev = st;
+    st = st + STAGE == lds + S * STAGE ? lds : st + STAGE;
+    half(1, st, 0, L0, c + S, prev);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still write to LDS when the wave ends
+
+  // accumulator [i][j]: token row 16 j + c16 of the wave's; registers of tiles 2 b, 2 b + 1: columns 8 g .. 8 g + 7 of the 32 of pair b
+  constexpr int NB = TN / 2;
+  const int col0 = n0 + wc * 16 * TN + 8 * g;
+  u32x4 bias[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    bias[b] = (u32x4){0, 0, 0, 0};
+    if (args.bias[part] != nullptr && col0 + 32 * b < N)
+      bias[b] = *reinterpret_cast<const u32x4*>(args.bias[part] + col0 + 32 * b);
+  }
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int row = m0 + wr * 16 * TM + 16 * j + c16;
+    if (row >= M) continue;
+    const int bt = row / args.batch_rows, tr = row - bt * args.batch_rows;
+    uint16_t* const cp = args.c + bt * args.cr.bs + tr * args.cr.ld + (long)part * N;
+    const uint16_t* const rp = args.res + bt * args.rr.bs + tr * args.rr.ld;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int col = col0 + 32 * b;
+      if (col >= N) continue;
+      float v[8];
+#pragma unroll
+      for (int p = 0; p < 8; ++p) {
+        v[p] = acc[2 * b + (p >> 2)][j][p & 3] + (p & 1 ? bf16hi(bias[b][p >> 1]) : bf16lo(bias[b][p >> 1]));
+        if (ACT == ACT_GELU) v[p] = gelu(v[p]);
+      }
+      if (args.res != nullptr) {
+        const u32x4 r = *reinterpret_cast<const u32x4*>(rp + col);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) v[p] += p & 1 ? bf16hi(r[p >> 1]) : bf16lo(r[p >> 1]);
+      }
+      const u32x4 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+      *reinterpret_cast<u32x4*>(cp + col) = o;
+    }
+  }
+}
+
+template <int TM, int TN, int S, int ACT>
+int launch(BlockArgs& args, hipStream_t stream) {
+  constexpr int LDS = (TM + TN) * S * 4096;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)block_gemm_kernel<TM, TN, S, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+      return -2;
+    attr_set = true;
+  }
+  args.n_tiles = (args.N + 32 * TN - 1) / (32 * TN);
+  const long blocks = (long)args.n_tiles * args.parts * ((args.M + 32 * TM - 1) / (32 * TM));
+  if (blocks >= (1L << 31)) return -1;
+  block_gemm_kernel<TM, TN, S, ACT><<<dim3((unsigned)blocks), 256, LDS, stream>>>(args);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+// The tile shapes, and what they cost: microseconds a chunk and beside the chunks (start, epilogue, and more of it with gelu) of a
+// round of one workgroup a CU, or, where two share a CU, of a round of two (a round that leaves half the places empty runs faster: its
+// own pair of numbers).  Fitted to the speech encoder's products (N, K of 512 to 3072, 1500 to 48000 rows); the choice by them is 2.6 %
+// off the best shape on average.
+struct Shape {
+  int bm, bn, per_cu;
+  float chunk, fixed, chunk1, fixed1, gelu;
+};
+constexpr Shape SHAPES[] = {{192, 192, 1, 0.76f, 8.38f, 0.f, 0.f, 3.f}, {128, 128, 1, 0.44f, 4.04f, 0.f, 0.f, 1.58f}, {128, 128, 2, 0.95f, 4.54f, 0.61f, 2.54f, 1.53f},
+                            {64, 128, 2, 0.60f, 2.09f, 0.27f, 2.87f, 0.78f},  {192, 128, 2, 1.36f, 5.82f, 0.75f, 3.69f, 2.17f}, {96, 192, 2, 1.09f, 4.70f, 0.66f, 2.74f, 1.38f}};
+
+int choose(int M, int N, int K, int parts, int act) {
+  int best = 0;
+  double best_t = 0;
+  for (int i = 0; i < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); ++i) {
+    const Shape& s = SHAPES[i];
+    const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * parts, round = 256 * s.per_cu;
+    const double gelu = act == ACT_GELU ? s.gelu : 0, full = K / BK * s.chunk + s.fixed + gelu;
+    const double half = s.per_cu > 1 ? K / BK * s.chunk1 + s.fixed1 + gelu / 2 : full;
+    const double left = (double)(tiles % round) / round;
+    const double t = tiles / round * full + (left == 0 ? 0 : left <= 0.5 ? half : half + (full - half) * (2 * left - 1));
+    if (i == 0 || t < best_t) best = i, best_t = t;
+  }
+  return best;
+}
+
+}  // namespace
+
+// c[r] = act(x[r] W_p^T + bias_p) + res[r], the columns of weights p = 0 .. parts - 1 (N rows of K each) side by side.  Rows r = 0 .. M - 1
+// in batches of batch_rows (one batch: M): strides of a row and of a batch in elements for x, c and res (c may be res).  act: 0 none,
+// 1 gelu (erf form).  Pieces of 16 bytes: N and strides multiples of 8, bases on 16 bytes; K a multiple of 64.  Returns 0, or a negative
+// number for what the kernel does not take.
+VPSA_EXPORT int vpsa_block_gemm(const void* x, long ld, long bs, const void* w0, const void* w1, const void* w2, const void* b0,
+                                const void* b1, const void* b2, int parts, void* c, long ldc, long cbs, const void* res, long ldr,
+                                long rbs, int batch_rows, int M, int N, int K, int act, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (N <= 0 || N % 8 != 0 || K <= 0 || K % BK != 0 || batch_rows <= 0 || parts < 1 || parts > 3 || act < 0 || act > 1) return -1;
+  if (((ld | bs | ldc | cbs | ldr | rbs) & 7) != 0 || ld < 0 || bs < 0 ||
+      (((uintptr_t)x | (uintptr_t)w0 | (uintptr_t)w1 | (uintptr_t)w2 | (uintptr_t)b0 | (uintptr_t)b1 | (uintptr_t)b2 | (uintptr_t)c |
+        (uintptr_t)res) & 15) != 0)
+    return -1;
+  const int last = batch_rows < M ? batch_rows - 1 : M - 1;
+  const double a_bytes = 2. * ((double)((M - 1) / batch_rows) * bs + (double)last * ld + K), w_bytes = 2. * N * K;
+  if (a_bytes >= 4294967296. || w_bytes >= 4294967296.) return -1;  // offsets of 32 bits
+  BlockArgs args = {(const uint16_t*)x,
+                    {(const uint16_t*)w0, (const uint16_t*)w1, (const uint16_t*)w2},
+                    {(const uint16_t*)b0, (const uint16_t*)b1, (const uint16_t*)b2},
+                    (const uint16_t*)res, (uint16_t*)c, {ld, bs}, {ldc, cbs}, {ldr, rbs}, batch_rows, M, N, K, 0, parts,
+                    (uint32_t)a_bytes, (uint32_t)w_bytes};
+#define SHAPE(TM, TN, S) return act == ACT_GELU ? launch<TM, TN, S, ACT_GELU>(args, stream) : launch<TM, TN, S, ACT_NONE>(args, stream)
+  switch (choose(M, N, K, parts, act)) {
+    case 0: SHAPE(6, 6, 3);
+    case 1: SHAPE(4, 4, 4);
+    case 2: SHAPE(4, 4, 2);
+    case 3: SHAPE(2, 4, 3);
+    case 4: SHAPE(6, 4, 2);
+    default: SHAPE(3, 6, 2);
+  }
+#undef SHAPE
+}

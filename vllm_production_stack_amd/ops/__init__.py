@@ -42,7 +42,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_block_gemm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -804,6 +804,32 @@ def decode_attention_block(x, w, bias, pool, layer, meta, n_q, n_kv, head_dim, s
     paged_decode(q, out, pool, layer, meta.dec_block_tables, meta.dec_ctx_lens, n_q, n_kv, head_dim, scale,
                  getattr(meta, "dec_num_splits", 1) or 1, getattr(meta, "dec_ws_o", None), getattr(meta, "dec_ws_ml", None))
     return out
+
+
+def block_linear(x, ws, biases, gelu=False, residual=None, out=None):
+    """act(x @ w.T + bias) (+ residual) for one to three weights of one shape, side by side in the last dimension
+    (``csrc/kernels/block_gemm.hip``).  x [B, T, K] with unit stride along K (rows may overlap, as a convolution's unfolded input
+    does); ``biases``: one or None for each weight; ``gelu``: its erf form; ``residual`` [B, T, N] or [T, N], added behind the
+    activation; ``out`` [B, T, N * len(ws)], may be ``residual``.  None (and nothing done) for operands the kernel does not take."""
+    b, t, k = x.shape
+    n = ws[0].shape[0]
+    res = residual if residual is None or residual.dim() == 3 else residual.unsqueeze(0).expand(b, -1, -1)
+    for v in (x, res, out, *ws, *biases):
+        if v is not None and (v.device != x.device or v.dtype != torch.bfloat16 or v.stride(-1) != 1):
+            return None
+    if (not x.is_cuda or any(w.shape != (n, k) or w.stride(0) != k for w in ws)
+            or any(v is not None and v.shape != (n,) for v in biases)
+            or (res is not None and (res.shape != (b, t, n) or len(ws) > 1))):
+        return None
+    if out is None:
+        out = torch.empty((b, t, n * len(ws)), dtype=x.dtype, device=x.device)
+    assert out.shape == (b, t, n * len(ws))
+    w, v = [_p(u) for u in ws] + [None, None], [_p(u) for u in biases] + [None, None]
+    rc = _kernels().vpsa_block_gemm(
+        _p(x), c_long(x.stride(1)), c_long(x.stride(0)), w[0], w[1], w[2], v[0], v[1], v[2], c_int(len(ws)), _p(out),
+        c_long(out.stride(1)), c_long(out.stride(0)), _p(res), c_long(0 if res is None else res.stride(1)),
+        c_long(0 if res is None else res.stride(0)), c_int(t), c_int(b * t), c_int(n), c_int(k), c_int(1 if gelu else 0), _stream())
+    return out if rc == 0 else None
 
 
 def pack_weight(w: torch.Tensor) -> torch.Tensor:
