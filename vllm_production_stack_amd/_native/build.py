@@ -34,7 +34,7 @@ TARGETS = {
          "kernels/lora.hip", "kernels/gemm.hip", "kernels/rans.hip", "kernels/sampling.hip",
          "kernels/grouped_gemm.hip", "kernels/packed_gemm.hip", "kernels/dense_attention.hip",
          "kernels/tile_gemm.hip", "kernels/latent.hip", "kernels/latent_mfma.hip", "kernels/seqmix.hip",
-         "kernels/retention.hip", "kernels/mid_gemm.hip", "kernels/block_gemm.hip"],
+         "kernels/chunk_scan.hip", "kernels/mid_gemm.hip", "kernels/block_gemm.hip"],
         [],
     ),
     "vpsa_kvio": ("hip", ["kvio/kvio.cpp"], []),
@@ -50,6 +50,7 @@ TARGETS = {
 # copied out one register at a time before the softmax can read it.
 SOURCE_FLAGS = {
     "kernels/attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "kernels/chunk_scan.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # the state lies in accumulators and is cut up by vector instructions
     "kernels/block_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # 256 registers and more: no copies between the files in the loop
 }
 # standalone executables: name -> (kind, sources, flags)
