@@ -32,6 +32,8 @@
 // Epilogues: bf16 store; SwiGLU (W = [gate rows | up rows], the first quadrant column of a wave is
 // gate and the second the matching up columns: silu(gate) * up, [rows, N / 2]); bf16 store of
 // accumulator + residual (the residual stream update of the o / down projections).
+#include <type_traits>
+
 #include "common.h"
 
 #define TG_BM 256
@@ -60,7 +62,11 @@ __device__ __forceinline__ void tg_glds16(const char* gptr, char* lds_dst) {
 // DBG: timing experiments with WRONG results (bit 0: no loads inside the K loop, bit 1: no fragment
 // reads inside the K loop, bit 2: every load inside the K loop re-requests K tile 0, i.e. hits in
 // cache); 0 in every production launch.
-template <int EPI, int DBG>
+// RAGGED: tiles of fewer than 193 rows go through with one, two or three of a quadrant's four 16-row tiles.  A group's rows are dealt
+// out evenly in units of 64, so that its last tile is not mostly padding: eight experts of 350 to 410 rows, 28672 x 4096 764 -> 714 us
+// and 4096 x 14336 360 -> 348; of 50 to 100 rows 436 -> 376 and 267 -> 243.  The instance without keeps its registers and its
+// instruction cache for the one form (1500 dense rows 0.9 % faster).
+template <int EPI, int DBG, bool RAGGED>
 __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     const uint16_t* __restrict__ a, long lda, const int* __restrict__ arow_idx,
     const uint16_t* __restrict__ w, long w_group_stride, const int* __restrict__ offsets, int n_groups, int max_rows,
@@ -89,7 +95,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     const int xcd = bid & 7, q = total >> 3, r = total & 7;
     t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
   }
-  int g = 0, row0 = 0, row_end = 0, n_idx = 0;
+  int g = 0, row0 = 0, row_end = 0, n_idx = 0, units = 4;  // units: 64 rows each that the tile holds
   for (int first = 0; g < n_groups; ++g) {
     const int lo = offsets ? offsets[g] : 0, hi = offsets ? offsets[g + 1] : max_rows;
     const int m_tiles = (hi - lo + TG_BM - 1) / TG_BM;
@@ -101,7 +107,9 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
       const int width = (band + 1) * TG_BAND <= n_tiles ? TG_BAND : n_tiles - band * TG_BAND;
       const int m_idx = rem / width;
       n_idx = band * TG_BAND + (rem - m_idx * width);
-      row0 = lo + m_idx * TG_BM;
+      const int all = (hi - lo + 63) / 64, each = all / m_tiles, more = all - each * m_tiles;
+      units = RAGGED ? each + (m_idx < more) : 4;
+      row0 = RAGGED ? lo + 64 * (m_idx * each + (m_idx < more ? m_idx : more)) : lo + m_idx * TG_BM;
       row_end = hi;
       break;
     }
@@ -113,11 +121,14 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
 
   const int wr = wave >> 2, wc = wave & 3;
 
+  // A tile of 64 MI rows: the same steps with MI of the four 16-row tiles in every quadrant.
+  auto body = [&](auto tag) {
+  constexpr int MI = decltype(tag)::value;
   // ---- per-lane source offsets (bytes) of the direct-to-LDS loads.  One wave instruction fills 8
   // LDS rows: lane -> (row = lane / 8, slot = lane % 8); instruction j (0, 1) of a half tile: wave
   // `wave` fills rows 64 j + 8 wave + lane / 8.  Slot s of LDS row r receives the 16-byte chunk
   // s ^ ((r >> 1) & 7) of the source row.
-  //   X half tile h, LDS row r:  tile row 128 (r / 64) + 64 h + r % 64
+  //   X half tile h, LDS row r:  tile row 32 MI (r / 64) + 16 MI h + r % 64
   //   W half tile h, LDS row r:  wave column block r / 32, MFMA tile (r % 32) / 16, MFMA row i = r % 16
   //                              -> column 64 (r / 32) + 32 h + 8 (i / 4) + 4 tile + i % 4
   uint32_t src_off[4][2];
@@ -129,7 +140,8 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
       const int chunk = lslot ^ ((r >> 1) & 7);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        int arow = row0 + 128 * (r >> 6) + 64 * h + (r & 63);
+        const int in_half = (r & 63) < 16 * MI ? r & 63 : 16 * MI - 1;  // (places past the tile's rows repeat one: never read)
+        int arow = row0 + 32 * MI * (r >> 6) + 16 * MI * h + in_half;
         if (arow >= row_end) arow = row_end - 1;  // rows past the group's end repeat its last row (never stored)
         const long src_row = arow_idx ? (long)arow_idx[arow] : (long)arow;
         src_off[h][j] = (uint32_t)((src_row * lda + chunk * 8) * 2);
@@ -167,16 +179,16 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
   const int x_rd = (wr * 64 + fr) * 128;
   const int w_rd = 2 * TG_HT + (wc * 32 + fr) * 128;
 
-  f32x4 acc[2][2][4][2];  // [quadrant row][quadrant column][row tile][column tile]
+  f32x4 acc[2][2][MI][2];  // [quadrant row][quadrant column][row tile][column tile]
 #pragma unroll
   for (int i0 = 0; i0 < 2; ++i0)
 #pragma unroll
     for (int i1 = 0; i1 < 2; ++i1)
 #pragma unroll
-      for (int i2 = 0; i2 < 4; ++i2)
+      for (int i2 = 0; i2 < MI; ++i2)
 #pragma unroll
         for (int i3 = 0; i3 < 2; ++i3) acc[i0][i1][i2][i3] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 xa[4][2];      // activation fragments of the current quadrant row: [row tile][k step]
+  bf16x8 xa[MI][2];      // activation fragments of the current quadrant row: [row tile][k step]
   bf16x8 wb[2][2][2];   // weight fragments of both quadrant columns: [quadrant column][column tile][k step]
 
   auto read_w = [&](int buf, int nh) {
@@ -190,7 +202,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
   auto read_x = [&](int buf, int mh) {
     if ((DBG & 2) && in_loop) return;
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) {
+    for (int mi = 0; mi < MI; ++mi) {
       xa[mi][0] = *reinterpret_cast<const bf16x8*>(lds + buf * TG_BUF + mh * TG_HT + mi * 2048 + x_rd + sl0);
       xa[mi][1] = *reinterpret_cast<const bf16x8*>(lds + buf * TG_BUF + mh * TG_HT + mi * 2048 + x_rd + sl1);
     }
@@ -200,7 +212,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
+      for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni)
           acc[mh][nh][mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[nh][ni][s], xa[mi][s], acc[mh][nh][mi][ni], 0, 0, 0);
@@ -237,7 +249,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
   // One K tile (LDS buffer B, tile index KT).  Phase = {fragment reads, one half-tile request,
   // barrier, 16 MFMAs, barrier}.  Requests: X-h1 of tile KT+1 (its slot was last read two phases
   // ago), then W-h0, X-h0, W-h1 of tile KT+2 into THIS buffer: W-h0 is read in phase 1 only and
-  // those reads are retired (lgkmcnt(8): the four W reads are issued first) before phase 1's first
+  // those reads are retired (a counted wait: the four W reads are issued first) before phase 1's first
   // barrier, so it may be overwritten from phase 2 on; X-h0 (read in phase 1) from phase 3; W-h1
   // (phase 2) from phase 4; X-h1 (phase 3) from the next tile's phase 1.  The counted wait of phase
   // 4 leaves the three youngest half tiles in flight: everything of tile KT+1 has landed before the
@@ -248,7 +260,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     TG_SB();                                                    \
     read_x(B, 0);                                               \
     TG_SB();                                                    \
-    asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");          \
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * MI) : "memory");          \
     TG_BAR();                                                   \
     TG_LGKM0();                                                 \
     mma(0, 0);                                                  \
@@ -291,23 +303,23 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
   if (wr == 0) TG_BAR();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be writing LDS when the wave ends
 
-  // ---- epilogue.  Accumulator [mh][nh][mi][ni]: lane -> output row 128 wr + 64 mh + 16 mi + lane % 16,
+  // ---- epilogue.  Accumulator [mh][nh][mi][ni]: lane -> output row 32 MI wr + 16 MI mh + 16 mi + lane % 16,
   // register e -> column 64 wc + 32 nh + 8 (lane / 16) + 4 ni + e.
-  float rs[2][4];  // the rows' factors, all loads in flight
+  float rs[2][MI];  // the rows' factors, all loads in flight
   if (EPI == TG_EPI_GLU_CLAMP) {
 #pragma unroll
     for (int mh = 0; mh < 2; ++mh)
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
-        const int row = row0 + 128 * wr + 64 * mh + 16 * mi + fr;
+      for (int mi = 0; mi < MI; ++mi) {
+        const int row = row0 + 32 * MI * wr + 16 * MI * mh + 16 * mi + fr;
         rs[mh][mi] = row_scale ? row_scale[row < row_end ? row : row_end - 1] : 1.f;
       }
   }
 #pragma unroll
   for (int mh = 0; mh < 2; ++mh) {
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) {
-      const int row = row0 + 128 * wr + 64 * mh + 16 * mi + fr;
+    for (int mi = 0; mi < MI; ++mi) {
+      const int row = row0 + 32 * MI * wr + 16 * MI * mh + 16 * mi + fr;
       if (TG_PAIRED(EPI)) {
         const int col = n_idx * 128 + wc * 32 + 8 * fq;
         float v[8];
@@ -371,6 +383,14 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
       }
     }
   }
+  };
+  if constexpr (!RAGGED) return body(std::integral_constant<int, 4>());
+  switch (units) {
+    case 1: return body(std::integral_constant<int, 1>());
+    case 2: return body(std::integral_constant<int, 2>());
+    case 3: return body(std::integral_constant<int, 3>());
+    default: return body(std::integral_constant<int, 4>());
+  }
 }
 
 static int g_tg_debug = 0;
@@ -404,16 +424,18 @@ VPSA_EXPORT int vpsa_tile_gemm(const void* a, long lda, const void* arow_idx, co
   const long blocks = (long)n_tiles * m_tiles_max;
   if (blocks > 0x7fffffffL) return -1;
   const long wstride = (long)n * k;
+  // (an even deal gives every tile four units exactly when the rows' units are four times the tiles)
+  const bool ragged = offsets || (max_rows + 63) / 64 != 4 * m_tiles_max;
 #define TG_LAUNCH(E, D)                                                                                               \
   do {                                                                                                               \
-    static bool attr_set = false;                                                                                    \
-    if (!attr_set) {                                                                                                 \
-      if (hipFuncSetAttribute((const void*)tile_gemm_kernel<E, D>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS) != \
-          hipSuccess)                                                                                                \
+    static bool attr_set[2] = {false, false};                                                                        \
+    const auto kernel = D == 0 && ragged ? tile_gemm_kernel<E, D, D == 0> : tile_gemm_kernel<E, D, false>;             \
+    if (!attr_set[ragged]) {                                                                                         \
+      if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS) != hipSuccess)   \
         return -2;                                                                                                   \
-      attr_set = true;                                                                                               \
+      attr_set[ragged] = true;                                                                                       \
     }                                                                                                                \
-    tile_gemm_kernel<E, D><<<dim3((unsigned)blocks), dim3(512), TG_LDS, stream>>>(                                       \
+    kernel<<<dim3((unsigned)blocks), dim3(512), TG_LDS, stream>>>(                                       \
         (const uint16_t*)a, lda, (const int*)arow_idx, (const uint16_t*)w, wstride, (const int*)offsets, n_groups,   \
         max_rows, (uint16_t*)c, ldc, (const uint16_t*)resid, ldr, n, k, n_tiles, act_limit, act_alpha, act_bias,    \
         (const float*)row_scale);                                                                                    \
