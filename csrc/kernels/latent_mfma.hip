@@ -282,11 +282,16 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //     The weights enter as two parts of 16 bits, a matrix instruction more for every value fragment that is read: with one part and
 //     one maximum for all 64 keys the error against 64 bits was 2.03e-3 on average over batches and contexts, with a maximum for
 //     each quarter 1.97e-3, with two parts it is 1.66e-3, the rounding of the result.
-//     With 64 slots a tile keeps four waves busy by itself.
+//   * Tiles of 64 slots: eight waves, two of which share 16 slots: each scores 32 keys and sums 256 channels, scores go round through 16 KB
+//     of LDS.  The page is read as often as by four waves with 16 slots each, but a SIMD has a second wave while one waits for LDS, and
+//     nothing else hides that: a page takes 3.1 us instead of 4.5 (32 heads, 2000 rows behind 6000 entries 1978 -> 1402 us).  What bounds it
+//     is that reading, 550 KB a page (2.2 us at 128 bytes a cycle); waves of 32 slots would halve it but their queries alone are 144 registers.
+//   * Lists of few tiles are cut along the keys (ops/latent.py): 200 rows of 16 heads behind 3800 entries 289 -> 68 us, 25 of 32 behind 6000
+//     429 -> 43, 1000 of 16 behind 3000 294 -> 211.
 //   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
 // Decode rows with their merge, in a graph, pages from memory; staged through registers / this: 32 heads, 32 sequences of 4k entries in 8
 // ranges 65 / 40 us, 8 of 8k in 32 42 / 32, one of 26k in 32 86 / 49, one of 3k 22.9 / 21.0, one of 2k, a page a range, 17.4 / 18.0; 16 heads,
-// one of 2k 16.1 / 15.4.  Prefill tiles, 1500 rows of 16 heads behind 4500 entries: 855 / 728.
+// one of 2k 16.1 / 15.4.
 
 // o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
 // their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
@@ -341,6 +346,7 @@ __device__ __forceinline__ void all_products(f32x4* o, const bf16x8 (&pf)[PARTS]
 // `rows` are those of the step's batch bucket, not of the launch: a row's ranges, and with them the order of its sums, are the same
 // in a captured step that is padded to the bucket and in an eager one that is not.
 constexpr int WIDE_ONCE = 4;
+constexpr int TILE_RANGE_PAGES = 4;  // a prefill tile's ranges are no shorter (the launch's count is chosen from the widest table)
 __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   int best = 1 << 30, used = splits;
   for (int r = 1; rows * splits > 256; ++r) {
@@ -351,23 +357,25 @@ __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   return used;
 }
 
-template <int RANK, int ROT, bool QUARTERS>
-__global__ __launch_bounds__(QUARTERS ? 512 : 256, QUARTERS ? 2 : 1) void latent_wide_kernel(
+// SHARE: waves that share 16 slots, each of which scores its part of a page's keys and sums its part of the channels (1: none).
+template <int RANK, int ROT, int SHARE>
+__global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void latent_wide_kernel(
     const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
     long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
     int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
     const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
     int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
   constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, DT = RANK / 16, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW;
-  constexpr int WAVES = QUARTERS ? 8 : 4;
+  constexpr bool QUARTERS = SHARE == 4;
+  constexpr int WAVES = SHARE > 1 ? 8 : 4;
   constexpr int NI = PAGE_BYTES / (1024 * WAVES);  // KiB of a page that a wave loads
-  constexpr int NT = QUARTERS ? 1 : 4;             // 16-key tiles of a page that a wave scores
-  constexpr int DW = QUARTERS ? DT / 4 : DT;       // 16-channel tiles that it sums
+  constexpr int NT = 4 / SHARE;                    // 16-key tiles of a page that a wave scores
+  constexpr int DW = DT / SHARE;                   // 16-channel tiles that it sums
   static_assert(ENTRY % 64 == 0 && DW % 8 == 0, "chunks are exchanged within groups of eight");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c16 = lane & 15, g = lane >> 4;
-  const int sg = QUARTERS ? wave >> 2 : wave, part = QUARTERS ? wave & 3 : 0;  // slots; keys and channels
+  const int sg = wave / SHARE, part = wave % SHARE;  // slots; keys and channels
   LatTile t;
   if (tiles) {
     const int* e = tiles + 6 * blockIdx.x;
@@ -402,7 +410,7 @@ __global__ __launch_bounds__(QUARTERS ? 512 : 256, QUARTERS ? 2 : 1) void latent
   const int my_pos = valid ? t.pos0 + tok : -1;
   const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
   const int p_first = max(0, t.pos0 - window + 1) / PAGE;
-  const int used = tiles ? splits : wide_splits(n_pages - p_first, bucket, splits);
+  const int used = tiles ? min(splits, max(1, (n_pages - p_first) / TILE_RANGE_PAGES)) : wide_splits(n_pages - p_first, bucket, splits);
   const int per = (n_pages - p_first + used - 1) / used;
   const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
   if (splits > 1 && p_begin >= p_end) {  // nothing to see: the merge passes over the record
@@ -555,8 +563,22 @@ __global__ __launch_bounds__(QUARTERS ? 512 : 256, QUARTERS ? 2 : 1) void latent
         multiply_tiles(o, v1, pf);
       }
     } else {
-      if (wave_active) {
+      if constexpr (SHARE > 1) {
+        f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;
+        if (wave_active) {
+          score(buf);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) round[(NT * part + nt) * 64] = s[nt];
+        }
+        everyone();
+        if (wave_active) {
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
+        }
+      } else if (wave_active) {
         score(buf);
+      }
+      if (wave_active) {
         weigh(p);
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
@@ -663,10 +685,10 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
   };
   if constexpr (!ROT_ONLY && RANK == 512 && ROT == 64) {
     const int quarters = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
-    const int lds = 2 * 64 * (RANK + ROT) * 2 + (quarters ? 8 * 1024 : 0);
-    const auto kernel = quarters ? latent_wide_kernel<RANK, ROT, true> : latent_wide_kernel<RANK, ROT, false>;
+    const int lds = 2 * 64 * (RANK + ROT) * 2 + (quarters ? 8 * 1024 : 16 * 1024);
+    const auto kernel = quarters ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 2>;
     if (!ready((const void*)kernel, lds, &attr_set[quarters])) return -2;
-    kernel<<<dim3(n_tiles, splits), dim3(quarters ? 512 : 256), lds, st>>>(
+    kernel<<<dim3(n_tiles, splits), dim3(512), lds, st>>>(
         (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
         page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
         window, splits, ws_o, ws_ml, bucket);

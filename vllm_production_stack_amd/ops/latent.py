@@ -264,6 +264,27 @@ def build_latent_tiles(q_lens, ctx_lens, heads: int):
     return tiles[order].astype(np.int32)
 
 
+# A work list of fewer tiles than the chip has CUs (one workgroup each) leaves the rest idle while every tile walks its pages alone,
+# and 300 tiles run as one full round and a nearly empty second.  A range costs its pages and, once, about as much as eight (queries,
+# the first page's way, its partial result and the merge's part of it).
+LATENT_RANGE_ONCE = 8
+LATENT_RANGE_MIN_PAGES = 4
+
+
+def latent_tile_splits(n_tiles: int, pages: int, rank: int, rot: int, latent: bool) -> int:
+    """Key ranges that the tiles of a work list are cut into; ``pages``: the width of the block tables."""
+    if not (latent and (rank, rot) == (512, 64)) or n_tiles == 0:
+        return 1
+    best, cost = 1, -(-n_tiles // 256) * (pages + LATENT_RANGE_ONCE // 4)
+    for e in range(2, min(64, pages // LATENT_RANGE_MIN_PAGES) + 1):
+        if n_tiles * e > 1024:
+            break
+        c = -(-n_tiles * e // 256) * (-(-pages // e) + LATENT_RANGE_ONCE)
+        if c < cost:
+            best, cost = e, c
+    return best
+
+
 def latent_expanded_supported(rank: int, rot: int) -> bool:
     """Does the tile kernel take value | key entries of this shape (``latent_attention`` without ``q_lat``)?"""
     return bool(_ops()._kernels().vpsa_latent_mfma_expanded(c_int(rank), c_int(rot)))
@@ -320,7 +341,8 @@ def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, pos
     if (tiles is not None or row_seq is None) and _mfma_ok(q_lat, q_rot, pool, out):
         if tiles is not None:
             assert tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.shape[1] == 6
-            n_tiles, splits = tiles.shape[0], 1
+            n_tiles = tiles.shape[0]
+            splits = latent_tile_splits(n_tiles, block_tables.shape[1], rank, rot, q_lat is not None)
         else:
             n_tiles = t * ((heads + LATENT_TILE_SLOTS - 1) // LATENT_TILE_SLOTS)
             bucket *= n_tiles // t
