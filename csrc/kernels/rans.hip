@@ -24,6 +24,10 @@
 // Coder: 32-bit state, byte-wise renormalisation, lower bound 2^23.  The encoder runs over its
 // symbols backwards and writes its bytes backwards into a private scratch slot, so the decoder
 // reads forwards; the slots are then gathered into one dense byte string at the prefix sum of the sizes.
+#include <string.h>
+
+#include <thread>
+
 #include "common.h"
 
 #define RANS_BITS 12
@@ -444,4 +448,80 @@ VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* 
   hipLaunchKernelGGL(rans_decode_kernel, dim3(spc / 64, n_ctx), dim3(64), 0, stream, (const uint8_t*)coded, coded_len, ctx_bytes,
                      (const uint16_t*)sizes, (const uint32_t*)states, table, (uint8_t*)sym, ctx_len, spc);
   return 0;
+}
+
+// ---------------------------------------------------------------------------------
+// What a KV page's stored form needs of the host in one call each way.  A call spends its host time beside the copy of 3.5 MB (45 us from
+// cache, 60 to 90 from memory) on launches, buffers and views: coming back a page took 178 us of host time for 117 of kernels and copies.
+extern "C" int vpsa_cachegen_decode(const void* symbols, const float* scales, void* staging, long n_elems, long unit_elems,
+                                    hipStream_t stream);
+
+struct PageParts {
+  char *scales, *freq, *states, *sizes, *coded;
+};
+static PageParts page_parts(void* body, long n, int n_ctx, int spc) {
+  char* p = (char*)body;
+  const long groups = n / 64 * 4, freq = 512L * n_ctx, streams = (long)n_ctx * spc;
+  return {p, p + groups, p + groups + freq, p + groups + freq + 4 * streams, p + groups + freq + 6 * streams};
+}
+static long page_symbols(long n) { return (n + 255) & ~255L; }
+
+// A page's parts, scales fp32 [n / 64] | freq | states | sizes | coded bytes, lie side by side in `body` on the device.
+// Bytes of the workspace of vpsa_page_decode (symbols | the coder's), 0: the shape is not taken.
+VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
+  const long coder = vpsa_rans_decode_workspace(n, n_ctx, spc);
+  return coder > 0 && n % 64 == 0 ? page_symbols(n) + coder : 0;
+}
+
+// A host copy of a few MB in pieces, each on a thread of its own where one can be had: a page comes out of memory, not of a cache.  Pages of
+// 3.5 MB coded, with one thread / four: four to the host and into a store 1502 / 1255 us, twelve back 1814 / 1700.  The threads end with the
+// object.
+class HostCopies {
+ public:
+  ~HostCopies() {
+    for (auto& t : threads_)
+      if (t.joinable()) t.join();
+  }
+  void start(int i, void* to, const void* from, long n) {
+    try {
+      threads_[i] = std::thread([=] { memcpy(to, from, n); });
+    } catch (...) {  // no thread to be had
+      memcpy(to, from, n);
+    }
+  }
+  static constexpr int MOST = 3;
+
+ private:
+  std::thread threads_[MOST];
+};
+
+static void copy_in_parts(char* to, const char* from, long size) {
+  HostCopies copies;
+  const long each = (size / (HostCopies::MOST + 1) + 4095) & ~4095L;  // whole pages
+  long at = 0;
+  for (int i = 0; i < HostCopies::MOST && at + each < size; ++i, at += each) copies.start(i, to + at, from + at, each);
+  memcpy(to + at, from + at, size - at);
+}
+
+// `size` bytes from the device to `to` by way of a pinned buffer.  Over on return.  (Four parts, each leaving the buffer while the next is on
+// its way, were no faster, 158 us a page against 162, and on the way back they cost the device 50 us a page: a copy's start is 10 to 15.)
+VPSA_EXPORT int vpsa_fetch(const void* from, void* pinned, void* to, long size, hipStream_t stream) {
+  const bool sent = hipMemcpyAsync(pinned, from, size, hipMemcpyDeviceToHost, stream) == hipSuccess;
+  if (hipStreamSynchronize(stream) != hipSuccess || !sent) return -3;
+  copy_in_parts((char*)to, (const char*)pinned, size);
+  return 0;
+}
+
+// `size` host bytes at `from` (a page's parts) through the pinned buffer into `body`, then symbols and values.  Not waited for:
+// the buffer is read until the copy is over.
+VPSA_EXPORT int vpsa_page_decode(const void* from, void* pinned, void* body, long size, long n, int n_ctx, int spc, long unit_elems, void* ws,
+                                 void* out, hipStream_t stream) {
+  if (vpsa_page_workspace(n, n_ctx, spc) <= 0) return -1;
+  const PageParts at = page_parts(body, n, n_ctx, spc);
+  const long coded = size - (at.coded - (char*)body);
+  if (coded < 0) return -1;
+  copy_in_parts((char*)pinned, (const char*)from, size);
+  if (hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, stream) != hipSuccess) return -3;
+  const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, (char*)ws + page_symbols(n), ws, n, n_ctx, spc, stream);
+  return rc ? rc : vpsa_cachegen_decode(ws, (const float*)at.scales, out, n, unit_elems, stream);
 }

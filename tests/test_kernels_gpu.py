@@ -1306,3 +1306,11 @@ def test_layer_norm_takes_and_refuses_what_the_library_does():
     for bad_w, bad_b in ((w[:248], b), (w, b[:128]), (w.view(2, 128), b), (w.cpu(), b), (w, b.cpu())):
         with pytest.raises(RuntimeError):
             ops.layer_norm(rows, bad_w, bad_b, 1e-5)
+
+
+@pytest.mark.parametrize("size", [1, 16, 4095, 16384, 16385, 3 * 16384 + 5, 3455418])
+def test_bytes_come_through_a_pinned_buffer_in_parts(size):
+    src = torch.randint(0, 256, (size + 7,), dtype=torch.uint8, device=DEV)
+    pinned, dst = torch.empty(size, dtype=torch.uint8, pin_memory=True), torch.full((size + 64,), 9, dtype=torch.uint8)
+    ops.fetch_bytes(src, pinned, dst.data_ptr() + 32, size)
+    assert torch.equal(dst[32:32 + size], src[:size].cpu()) and bool((dst[:32] == 9).all()) and bool((dst[32 + size:] == 9).all())

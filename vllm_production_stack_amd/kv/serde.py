@@ -38,6 +38,10 @@ _RANS_HDR = struct.Struct("<IIQ")  # streams per context, streams, coded bytes
 _KEPT = 2  # pinned buffers a serialiser keeps for each direction
 _HDR = struct.Struct("<4sHHIIIIQ")
 
+# a bytes object made at its size and filled before anyone else sees it (the C API's way to build one without a second copy)
+_new_bytes = ctypes.PYFUNCTYPE(ctypes.py_object, ctypes.c_void_p, ctypes.c_ssize_t)(("PyBytes_FromStringAndSize", ctypes.pythonapi))
+_bytes_at = ctypes.PYFUNCTYPE(ctypes.c_void_p, ctypes.py_object)(("PyBytes_AsString", ctypes.pythonapi))
+
 _kvio = None
 
 
@@ -130,7 +134,7 @@ class PageSerde:
             return _HDR.pack(MAGIC, 1, SERDE_NAIVE, self.n_layers, self.n_kv, self.head_dim, ops.PAGE,
                              len(raw)) + raw
         if self._rans_ok(flat.device):
-            return self._rans_page(flat, lambda payload: b"".join((self._rans_header(payload.size), memoryview(payload))))
+            return self._rans_page(flat, self._new_blob)
         sym_np, sc_np = self.quantize(flat)
         return self.pack(sym_np, sc_np)
 
@@ -144,7 +148,7 @@ class PageSerde:
         Otherwise the int8 symbols and fp32 scales come back for the host range coder
         -> (symbols, scales)."""
         if self._rans_ok(flat.device):
-            return self._rans_page(flat, np.copy), None
+            return self._rans_page(flat, self._new_payload), None
         sym, scales = ops.cachegen_encode(flat.contiguous(), self._levels(flat.device), self.unit_elems, self.n_layers)
         return sym.cpu().numpy(), scales.float().cpu().numpy()
 
@@ -154,26 +158,42 @@ class PageSerde:
             lv = self._levels_dev[device] = torch.tensor(self.levels, dtype=torch.int32, device=device)
         return lv
 
-    def _rans_page(self, flat: torch.Tensor, finish):
-        """``finish`` of a page's kind-2 payload, which lies in a pinned buffer until it returns.  Every stage writes its part of
-        the payload where it belongs; one copy brings the finished payload over."""
+    def _new_blob(self, payload: int):
+        """(a stored page with room for ``payload`` bytes behind its header, the payload's address)"""
+        blob = _new_bytes(None, _HDR.size + payload)
+        at = _bytes_at(blob)
+        ctypes.memmove(at, self._rans_header(payload), _HDR.size)
+        return blob, at + _HDR.size
+
+    @staticmethod
+    def _new_payload(payload: int):
+        out = np.empty(payload, dtype=np.uint8)
+        return out, out.ctypes.data
+
+    def _rans_page(self, flat: torch.Tensor, new):
+        """A page's kind-2 payload in what ``new`` makes for its size.  Every stage writes its part of the payload where it belongs,
+        the last one the size into pinned memory; then the payload is copied to the host in parts, and out of the pinned buffer
+        behind them."""
         n, dev, n_streams = flat.numel(), flat.device, self.n_layers * ops.RANS_SPC
-        a = _RANS_HDR.size
-        o = np.cumsum([0, 4 * (n // 64), 512 * self.n_layers, 4 * n_streams, 2 * n_streams]).tolist()
-        body = torch.empty(o[4] + 2 * n, dtype=torch.uint8, device=dev)
+        o1 = 4 * (n // 64)
+        o2 = o1 + 512 * self.n_layers
+        o3 = o2 + 4 * n_streams
+        o4 = o3 + 2 * n_streams
+        body = torch.empty(o4 + 2 * n, dtype=torch.uint8, device=dev)
         sym, _ = ops.cachegen_encode(flat.contiguous(), self._levels(dev), self.unit_elems, self.n_layers,
-                                     scales=body[:o[1]].view(torch.float32))
-        total, bad = ops.rans_encode_into(sym.view(-1), self.n_layers, body[o[1]:o[2]], body[o[2]:o[3]], body[o[3]:o[4]],
-                                          body[o[4]:]).tolist()
+                                     scales=body[:o1].view(torch.float32))
+        buf = self._take(self._out_bufs, o4 + n)  # (a value rarely codes to more than a byte)
+        meta = buf[:16].view(torch.int64)
+        ops.rans_encode_into(sym.view(-1), self.n_layers, body[o1:o2], body[o2:o3], body[o3:o4], body[o4:], meta=meta)
+        torch.cuda.current_stream(dev).synchronize()
+        total, bad = meta.tolist()
         if bad:
             raise RuntimeError("rans_encode: frequency table could not be normalised")
-        size = a + o[4] + total
-        buf = self._take(self._out_bufs, size)
-        buf[a:size].copy_(body[:o[4] + total], non_blocking=True)
-        torch.cuda.current_stream(dev).synchronize()
-        payload = buf.numpy()[:size]
-        payload[:a] = np.frombuffer(_RANS_HDR.pack(ops.RANS_SPC, n_streams, total), dtype=np.uint8)
-        done = finish(payload)
+        if buf.numel() < o4 + total:
+            buf = self._take(self._out_bufs, o4 + total)
+        done, at = new(_RANS_HDR.size + o4 + total)
+        ctypes.memmove(at, _RANS_HDR.pack(ops.RANS_SPC, n_streams, total), _RANS_HDR.size)
+        ops.fetch_bytes(body, buf, at + _RANS_HDR.size, o4 + total)
         self._give(self._out_bufs, buf)
         return done
 
@@ -244,33 +264,27 @@ class PageSerde:
         """rANS payload (host bytes) -> KV page on ``device``: one host-to-device copy, entropy
         decode and dequantisation on the GPU (NumPy definitions on a CPU-only host)."""
         spc, n_streams, coded_len = _RANS_HDR.unpack_from(payload, 0)
-        n_groups = self.page_elems // 64
-        a = _RANS_HDR.size
-        cuts = np.cumsum([a, 4 * n_groups, 2 * 256 * self.n_layers, 4 * n_streams, 2 * n_streams, coded_len])
-        if n_streams != self.n_layers * spc or cuts[-1] > payload.size:
+        n, a = self.page_elems, _RANS_HDR.size
+        o1 = 4 * (n // 64)
+        o2 = o1 + 2 * 256 * self.n_layers
+        o3 = o2 + 4 * n_streams
+        o4 = o3 + 2 * n_streams
+        size = o4 + coded_len
+        if n_streams != self.n_layers * spc or a + size > payload.size:
             raise ValueError("damaged cachegen payload")
-        body = self._to_device(payload[a:cuts[-1]], device)
-        o = cuts - a
-        scales = body[o[0]:o[1]].view(torch.float32)
-        freq = body[o[1]:o[2]].view(torch.int16)
-        states = body[o[2]:o[3]].view(torch.int32)
-        sizes = body[o[3]:o[4]].view(torch.int16)
-        coded = body[o[4]:o[5]]
-        sym = ops.rans_decode(freq, states, sizes, coded, self.page_elems, self.n_layers, spc)
-        return ops.cachegen_decode(sym, scales, self.unit_elems)
-
-    def _to_device(self, data: np.ndarray, device) -> torch.Tensor:
-        """Host bytes on ``device``, through the next pinned buffer on a GPU (without waiting for the copy)."""
-        if torch.device(device).type != "cuda":
-            return torch.from_numpy(data.copy()).to(device)
-        buf = self._take(self._in_bufs, data.size)
-        np.copyto(buf.numpy()[:data.size], data)
-        body = torch.empty(data.size, dtype=torch.uint8, device=device)
-        body.copy_(buf[:data.size], non_blocking=True)
-        read = torch.cuda.Event()
-        read.record(torch.cuda.current_stream(body.device))
-        self._give(self._in_bufs, buf, read)
-        return body
+        body = payload[a:a + size]
+        if torch.device(device).type == "cuda":
+            body = np.ascontiguousarray(body)
+            buf = self._take(self._in_bufs, size)
+            out = ops.page_decode(body.ctypes.data, buf, size, n, self.n_layers, self.unit_elems, device, spc)
+            read = torch.cuda.Event()
+            read.record(torch.cuda.current_stream(out.device))
+            self._give(self._in_bufs, buf, read)
+            return out
+        body = torch.from_numpy(body.copy()).to(device)
+        sym = ops.rans_decode(body[o1:o2].view(torch.int16), body[o2:o3].view(torch.int32), body[o3:o4].view(torch.int16), body[o4:],
+                              n, self.n_layers, spc)
+        return ops.cachegen_decode(sym, body[:o1].view(torch.float32), self.unit_elems)
 
     def restore(self, got: tuple, device) -> torch.Tensor:
         """Finish what ``unpack`` started (its "codec" and "rans" results)."""

@@ -35,7 +35,7 @@ def _kernels():
             "vpsa_moe_gemv", "vpsa_moe_mfma", "vpsa_lora_shrink", "vpsa_lora_expand",
             "vpsa_skinny_gemm", "vpsa_hbm_read_probe", "vpsa_set_gemm_variant", "vpsa_stream_gemm",
             "vpsa_stream_gemm_splits", "vpsa_set_stream_targets", "vpsa_rans_encode",
-            "vpsa_rans_decode", "vpsa_sample", "vpsa_grouped_gemm", "vpsa_packed_gemm",
+            "vpsa_rans_decode", "vpsa_fetch", "vpsa_page_decode", "vpsa_sample", "vpsa_grouped_gemm", "vpsa_packed_gemm",
             "vpsa_packed_gemm_splits", "vpsa_set_packed_target", "vpsa_dense_decode_attention", "vpsa_dense_attention",
             "vpsa_tile_gemm", "vpsa_tile_gemm_debug", "vpsa_paged_prefill_split",
             "vpsa_embed_scale", "vpsa_add_rmsnorm", "vpsa_rmsnorm_rows", "vpsa_latent_kv_write", "vpsa_rope_pairs",
@@ -49,7 +49,8 @@ def _kernels():
             "vpsa_embed_rmsnorm", "vpsa_depth_mix_rmsnorm", "vpsa_poly_norm", "vpsa_soft_cap", "vpsa_mingru",
         ):
             getattr(lib, name).restype = c_int
-        for name in ("vpsa_prefill_split_record_bytes", "vpsa_rans_workspace", "vpsa_rans_decode_workspace"):
+        for name in ("vpsa_prefill_split_record_bytes", "vpsa_rans_workspace", "vpsa_rans_decode_workspace",
+                     "vpsa_page_workspace"):
             getattr(lib, name).restype = c_long
         if os.environ.get("VPSA_PREFILL_VARIANT"):  # pin one prefill kernel for A/B runs
             lib.vpsa_set_prefill_variant(c_int(int(os.environ["VPSA_PREFILL_VARIANT"])))
@@ -1187,10 +1188,10 @@ def rans_encode(sym, n_ctx, spc=RANS_SPC):
     return freq, states, sizes, coded[:total].clone()
 
 
-def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC):
+def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC, meta=None):
     """``rans_encode`` on the device into the caller's tensors (``coded`` with room for two bytes a symbol), without a
-    synchronisation -> int64 [2] on the device: coded bytes, and contexts whose table could not be normalised (nothing of
-    the result is valid unless 0)."""
+    synchronisation -> int64 [2] on the device, or ``meta`` (on the device or in pinned host memory): coded bytes, and contexts
+    whose table could not be normalised (nothing of the result is valid unless 0)."""
     n, dev, lib = sym.numel(), sym.device, _kernels()
     if n % n_ctx or (n // n_ctx) % spc:
         raise ValueError("rans_encode: symbols do not divide into contexts / streams")
@@ -1199,7 +1200,9 @@ def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC):
     assert all(t.is_contiguous() and t.numel() * t.element_size() >= b for t, b in (
         (freq, 512 * n_ctx), (states, 4 * n_streams), (sizes, 2 * n_streams), (coded, 2 * n)))
     ws = torch.empty(max(1, int(lib.vpsa_rans_workspace(c_long(n), c_int(n_ctx), c_int(spc)))), dtype=torch.uint8, device=dev)
-    meta = torch.empty(2, dtype=torch.int64, device=dev)
+    if meta is None:
+        meta = torch.empty(2, dtype=torch.int64, device=dev)
+    assert meta.dtype == torch.int64 and meta.is_contiguous() and meta.numel() == 2 and (meta.device == dev or meta.is_pinned())
     _check(lib.vpsa_rans_encode(_p(sym), c_long(n), c_int(n_ctx), c_int(spc), _p(ws), _p(freq), _p(states), _p(sizes), _p(coded),
                                 _p(meta), _stream()), "rans_encode")
     return meta
@@ -1223,6 +1226,30 @@ def rans_decode(freq, states, sizes, coded, n, n_ctx, spc=RANS_SPC):
     _check(lib.vpsa_rans_decode(_p(coded), c_long(coded.numel()), _p(states), _p(freq), _p(sizes), _p(ws), _p(sym), c_long(n),
                                 c_int(n_ctx), c_int(spc), _stream()), "rans_decode")
     return sym
+
+
+def fetch_bytes(src, pinned, dst: int, size: int) -> None:
+    """The first ``size`` bytes of ``src`` (uint8, on the device) to host memory at ``dst``, through ``pinned`` (as large, pinned): the
+    buffer is emptied behind the copy that fills it.  Over on return; other threads run meanwhile."""
+    assert src.is_cuda and src.is_contiguous() and min(src.numel(), pinned.numel()) >= size and not pinned.is_cuda
+    _check(_kernels().vpsa_fetch(_p(src), _p(pinned), c_void_p(dst), c_long(size), _stream()), "fetch_bytes")
+
+
+def page_decode(src: int, pinned, size: int, n: int, n_ctx: int, unit_elems: int, device, spc=RANS_SPC):
+    """A page's quantised and coded parts (``size`` host bytes at ``src``: scales fp32 [n / 64] | freq u16 [n_ctx * 256] | states u32 and
+    sizes u16 [n_ctx * spc] | coded bytes) -> bf16 [n] on ``device``, by way of ``pinned``, which the device reads until what has been
+    queued so far is over."""
+    lib = _kernels()
+    ws = int(lib.vpsa_page_workspace(c_long(n), c_int(n_ctx), c_int(spc)))
+    if ws <= 0 or unit_elems % 8192:
+        raise ValueError("page_decode: symbols do not divide into contexts / streams")
+    assert pinned.numel() >= size and not pinned.is_cuda
+    out = torch.empty(n, dtype=torch.bfloat16, device=device)
+    at = (size + 255) // 256 * 256
+    work = torch.empty(at + ws, dtype=torch.uint8, device=device)   # the page's parts | workspace
+    _check(lib.vpsa_page_decode(c_void_p(src), _p(pinned), _p(work), c_long(size), c_long(n), c_int(n_ctx), c_int(spc),
+                                c_long(unit_elems), c_void_p(work.data_ptr() + at), _p(out), _stream()), "page_decode")
+    return out
 
 
 # --------------------------------------------------------------------------- MoE routing
