@@ -211,7 +211,7 @@ class TransformerModel:
         cfg = self.cfg
         t = x.shape[0]
         e, k = self.local_experts, cfg.num_experts_per_tok
-        logits = F.linear(x, lw.router)
+        logits = ops.moe_router(x, lw.router)
         w, ids = ops.moe_topk_softmax(logits, k)
         mfma = x.is_cuda and ops.moe_streams_experts(t, k, e) and ops.moe_mfma_supported(x.shape[1], lw.w2.shape[2])
         tiled = (x.is_cuda and not (decode_only or t <= 16)

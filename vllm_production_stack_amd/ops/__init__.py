@@ -31,7 +31,7 @@ def _kernels():
             "vpsa_rmsnorm", "vpsa_rope_cache", "vpsa_kv_cache_write", "vpsa_paged_prefill_rope", "vpsa_prefill_fuses_rope", "vpsa_silu_mul", "vpsa_argmax_bf16",
             "vpsa_paged_prefill", "vpsa_set_prefill_variant", "vpsa_prefill_tile_rows", "vpsa_set_decode_variant", "vpsa_paged_decode", "vpsa_kv_gather_pages",
             "vpsa_kv_scatter_pages", "vpsa_cachegen_encode", "vpsa_cachegen_decode",
-            "vpsa_moe_topk_softmax", "vpsa_moe_align", "vpsa_moe_permute", "vpsa_moe_combine",
+            "vpsa_moe_topk_softmax", "vpsa_moe_router", "vpsa_moe_align", "vpsa_moe_permute", "vpsa_moe_combine",
             "vpsa_moe_gemv", "vpsa_moe_mfma", "vpsa_lora_shrink", "vpsa_lora_expand",
             "vpsa_skinny_gemm", "vpsa_hbm_read_probe", "vpsa_set_gemm_variant", "vpsa_stream_gemm",
             "vpsa_stream_gemm_splits", "vpsa_set_stream_targets", "vpsa_rans_encode",
@@ -1253,6 +1253,18 @@ def page_decode(src: int, pinned, size: int, n: int, n_ctx: int, unit_elems: int
 
 
 # --------------------------------------------------------------------------- MoE routing
+def moe_router(x, w):
+    """A mixture's router product ``x @ w.T`` (``csrc/kernels/moe.hip`` for up to 64 experts, else the library)."""
+    if (x.is_cuda and x.dim() == 2 and w.device == x.device and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous()
+            and 0 < w.shape[0] <= 64 and x.shape[1] == w.shape[1] and x.shape[1] % 128 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0 and not _followed(x, w)):
+        out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+        _check(_kernels().vpsa_moe_router(_p(x), c_long(x.stride(0)), _p(w), _p(out), c_int(x.shape[0]), c_int(w.shape[0]),
+                                          c_int(x.shape[1]), _stream()), "moe_router")
+        return out
+    return torch.nn.functional.linear(x, w)
+
+
 def moe_topk_softmax(logits, topk, renorm=True):
     if not logits.is_cuda:
         return reference.moe_topk_softmax(logits, topk, renorm)
