@@ -1602,11 +1602,13 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
   if (!head_ok) return;  // (no barrier below)
   if (part >= 0) {
     // record = [2 row blocks][4 channel tiles][16 values][64 lanes] fp32, then [2][64] maxima and
-    // [2][64] sums: lane-major, so that the combine kernel (same lane roles) reads it back whole
+    // [2][64] sums: lane-major, so that the combine kernel (same lane roles) reads it back whole.  Rows past the sequence's (a
+    // quarter of a tile on average, 35 MB of 97 rows' records with them) are neither written nor read.
     float* rec = split_ws + ((long)(part * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       const float l_tot = l_run[rb] + __shfl_xor(l_run[rb], 32, 64);
+      if (!row_ok[rb] || !head_ok) continue;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -1635,11 +1637,13 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
   }
 }
 
-// Merge the partial records of split work-list entries.  grid = (groups, head groups, 8): group g =
+// Merge the partial records of split work-list entries.  grid = (groups, head groups, 16): group g =
 // (sequence, first row of the tile, first record, number of records); blockIdx.z picks one (row
-// block, channel tile) slice of the record, a wave is a head and its lanes hold what they hold in
-// the attention kernel's epilogue: 16 values each, so the merge of a tile is spread over 8 x the
-// head groups workgroups and every record is read with whole-wave contiguous loads.
+// block, channel tile, half of its values) slice of the record, a wave is a head and its lanes hold what they hold in
+// the attention kernel's epilogue: 8 values each, so the merge of a tile is spread over 16 x the
+// head groups workgroups and every record is read with whole-wave contiguous loads.  (Slices of 16 values left half the CUs without a
+// workgroup: 97 rows of 32 heads in 16 ranges 11.4 -> 9.6 us, with the rows
+// that are left out above.)
 __global__ __launch_bounds__(256) void prefill_combine_kernel(
     const float* __restrict__ split_ws, const int* __restrict__ groups, uint16_t* __restrict__ out,
     long out_stride, const int* __restrict__ cu_q, int n_q, int n_kv) {
@@ -1648,39 +1652,40 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(
   const int seq = groups[4 * blockIdx.x], q0 = groups[4 * blockIdx.x + 1], part0 = groups[4 * blockIdx.x + 2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5;
-  const int by = blockIdx.y, rb = blockIdx.z >> 2, dt = blockIdx.z & 3;
+  const int by = blockIdx.y, rb = blockIdx.z >> 3, dt = (blockIdx.z >> 1) & 3, half = blockIdx.z & 1;
   const int G = n_q / n_kv, groups_per_kv = (G + 3) >> 2;
   const int head_slot = (by % groups_per_kv) * 4 + wave;
   if (head_slot >= G) return;  // a spare wave of the last head group
   const int head = (by / groups_per_kv) * G + head_slot;
   const int row0 = cu_q[seq], q_len = cu_q[seq + 1] - row0;
   const int row = q0 + 32 * rb + r;
-  const float* rec0 = split_ws + ((long)(part0 * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS;
+  if (row >= q_len) return;
+  const float* rec0 = split_ws + ((long)(part0 * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS + lane;
   const long rec_step = (long)gridDim.y * 4 * SPLIT_REC_FLOATS;
+  const int at = ((rb * 4 + dt) * 16 + 8 * half) * 64;
   float m = NEG_BIG;
-  for (int p = 0; p < nparts; ++p) m = fmaxf(m, rec0[p * rec_step + 8192 + rb * 64 + lane]);
+#pragma unroll 8
+  for (int p = 0; p < nparts; ++p) m = fmaxf(m, rec0[p * rec_step + 8192 + rb * 64]);
   float l = 0.f;
-  float o[16];
+  float o[8];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) o[i] = 0.f;
+  for (int i = 0; i < 8; ++i) o[i] = 0.f;
 #pragma unroll 4
   for (int p = 0; p < nparts; ++p) {
     const float* rec = rec0 + p * rec_step;
-    const float f = __builtin_amdgcn_exp2f(rec[8192 + rb * 64 + lane] - m);
-    l += f * rec[8192 + 128 + rb * 64 + lane];
+    const float f = __builtin_amdgcn_exp2f(rec[8192 + rb * 64] - m);
+    l += f * rec[8192 + 128 + rb * 64];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[i] += f * rec[((rb * 4 + dt) * 16 + i) * 64 + lane];
+    for (int i = 0; i < 8; ++i) o[i] += f * rec[at + i * 64];
   }
-  if (row < q_len) {
-    const float inv = 1.f / l;
-    uint16_t* op = out + (long)(row0 + row) * out_stride + head * HEAD_DIM;
+  const float inv = 1.f / l;
+  uint16_t* op = out + (long)(row0 + row) * out_stride + head * HEAD_DIM + 32 * dt + 16 * half + 4 * h;
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      u32x2 w;
-      w[0] = pack_bf16x2(o[4 * g4] * inv, o[4 * g4 + 1] * inv);
-      w[1] = pack_bf16x2(o[4 * g4 + 2] * inv, o[4 * g4 + 3] * inv);
-      *reinterpret_cast<u32x2*>(op + 32 * dt + 8 * g4 + 4 * h) = w;
-    }
+  for (int g4 = 0; g4 < 2; ++g4) {
+    u32x2 w;
+    w[0] = pack_bf16x2(o[4 * g4] * inv, o[4 * g4 + 1] * inv);
+    w[1] = pack_bf16x2(o[4 * g4 + 2] * inv, o[4 * g4 + 3] * inv);
+    *reinterpret_cast<u32x2*>(op + 8 * g4) = w;
   }
 }
 
@@ -1834,7 +1839,7 @@ VPSA_EXPORT int vpsa_paged_prefill_split(const void* q, long q_stride, void* out
                          VPSA_PREFILL_ARGS);
     }
     if (tile_split != nullptr && num_groups > 0)
-      hipLaunchKernelGGL(prefill_combine_kernel, dim3(num_groups, n_kv * ((G + 3) / 4), 8), block, 0, stream,
+      hipLaunchKernelGGL(prefill_combine_kernel, dim3(num_groups, n_kv * ((G + 3) / 4), 16), block, 0, stream,
                          (const float*)split_ws, groups, (uint16_t*)out, out_stride, cu_q, n_q, n_kv);
     return 0;
   }
