@@ -11,8 +11,8 @@
 // 32-bit matrix instructions 1.7e-7 to 3.0e-7; gated, whose 1 - a comes from the exponential: 0.9e-7, token by token 1.2e-7.
 //   * What bounds it: vector work (a block costs a wave 1000 instructions, half of them to cut the state up, and a SIMD's two waves
 //     2 x 166 matrix instructions) and the barriers between staging, scores and products; HBM has a third of its traffic.
-//   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1564 / 309 us,
-//     fixed 128 x 256 701 / 396; 1000 rows: gated (16 heads, three sequences) 229 / 55, fixed (one) 154 / 85; 200 rows of two 199 / 37.
+//   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1564 / 297 us,
+//     fixed 128 x 256 701 / 385; 1000 rows: gated (16 heads, three sequences) 229 / 55, fixed (one) 154 / 84; 200 rows of two 199 / 37.
 //   * 1 / R must stay in range: a block in which some |R| leaves 2^-60 .. 2^60 is taken again with half its tokens (a block of one token
 //     divides by nothing); fixed decays know their longest block beforehand.
 //   * A workgroup holds a head's whole 128 x VD state in accumulators, 32 columns a wave, so q, k and the scores are made once for all
@@ -35,6 +35,7 @@ constexpr int TN = 2;      // tiles of 16 value columns a wave holds
 constexpr int IMG = RT * RD * 2;  // one part of q^ or k^
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
   int* const flags = reinterpret_cast<int*>(kpow + 36);
   float* const one = reinterpret_cast<float*>(ps);           // a single token's q, k and v in 32 bits
 
-  const int head = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int head = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g = lane >> 4;
   int seq, r0, r1;
   if (PHASE == 0) {
     seq = blockIdx.y, r0 = args.seq_cu[seq], r1 = args.seq_cu[seq + 1];
@@ -180,8 +181,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
     seq = run.seq;
     run_rows(args.pieces, args.seq_pieces, seq, blockIdx.y - run.first, args.group, &r0, &r1);
   }
+  // (the same for all lanes, and said so: bounds, branches and the positions' addresses stay in scalar registers)
+  r0 = __builtin_amdgcn_readfirstlane(r0), r1 = __builtin_amdgcn_readfirstlane(r1);
   if (r1 <= r0) return;
-  const int slot = args.seq_state[seq], heads = args.heads;
+  const int slot = __builtin_amdgcn_readfirstlane(args.seq_state[seq]), heads = args.heads;
   float* const out = args.out;
   if (slot < 0) {  // rows of no sequence: their output is zero
     if (PHASE != 1)
@@ -220,6 +223,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
     float p = 1.f;
     longest = 1;
     while (longest < RT && (p *= a) >= R_MIN && p <= R_MAX) ++longest;
+    longest = __builtin_amdgcn_readfirstlane(longest);
   }
   float pgate[GATED ? 4 : 1];  // gated, phase 1: the run's total decay of this thread's channels
   if (GATED)
@@ -234,10 +238,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
   // QU neighbouring rows.  A group of four channels is half a 16-byte chunk of a row.
   u32x2 rq[QU], rk[QU];
   u32x4 rv[VU];
-  int rpos[QU / 2];
   f32x4 co[QU / 2], si[QU / 2];
 #pragma unroll
   for (int u = 0; u < QU / 2; ++u) co[u] = si[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  constexpr bool EARLY = NW == 8;  // table rows are asked for a block ahead (four waves have no registers for them)
   const int half = args.rot_dims >> 1, layout = args.layout;
   int ch0, ch1;  // gated: ch0 alone
   if (GATED) {
@@ -271,7 +275,6 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
       if (row < nr) {
         rk[u] = *reinterpret_cast<const u32x2*>(base + args.k_col + at);
         if (PHASE != 1) rq[u] = *reinterpret_cast<const u32x2*>(base + args.q_col + at);
-        if (!GATED && args.rot_dims && !(u & 1)) rpos[u >> 1] = args.positions[r + row];
       }
     }
 #pragma unroll
@@ -281,16 +284,27 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
       if (row < nr) rv[u] = *reinterpret_cast<const u32x4*>(vbase + (uint32_t)row * (uint32_t)args.p_stride + vch);
     }
   };
-  constexpr bool EARLY = NW == 8;  // (four waves have no registers for them between blocks)
-  auto fetch_turns = [&](int r) {  // the table rows of what `fetch` has asked for
-    if (!turn) return;
+  // The table rows of what `fetch` has asked for.  A wave's positions come as scalars, four rows in a row: as vector loads they would
+  // have to be waited for, and with them all that was asked for before.
+  typedef __attribute__((address_space(4))) const int* scalar_ptr;
+  const scalar_ptr positions = (scalar_ptr)(uintptr_t)args.positions;
+  i32x4 spos[QU / 2];
+  auto fetch_positions = [&](int r) {
+    if (GATED || args.rot_dims == 0) return;
 #pragma unroll
     for (int u = 0; u < QU / 2; ++u)
-      if (row_of(2 * u) < r1 - r) {
-        const float* cs = args.cos_sin + (long)rpos[u] * args.rot_dims + 4 * (tid & 15);
-        co[u] = *reinterpret_cast<const f32x4*>(cs);
-        si[u] = *reinterpret_cast<const f32x4*>(cs + half);
-      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) spos[u][i] = positions[min(r + 4 * wave + u * (NT / 16) + i, r1 - 1)];
+  };
+  auto fetch_turns = [&]() {
+    if (!turn) return;
+#pragma unroll
+    for (int u = 0; u < QU / 2; ++u) {
+      const int pos = g & 2 ? (g & 1 ? spos[u][3] : spos[u][2]) : (g & 1 ? spos[u][1] : spos[u][0]);
+      const float* cs = args.cos_sin + (long)pos * args.rot_dims + 4 * (tid & 15);
+      co[u] = *reinterpret_cast<const f32x4*>(cs);
+      si[u] = *reinterpret_cast<const f32x4*>(cs + half);
+    }
   };
   auto put_k = [&](int row, int ch, const float* x) {  // four channels in their parts
     uint32_t a[3], b[3];
@@ -460,12 +474,13 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
   const int tr_chunk = (((c >> 1) & 1) ^ swz(tr_row)) * 16 + (c & 1) * 8;  // four channels 4 (c % 4) of sixteen
 
   __syncthreads();
-  odd = __syncthreads_or(odd);
+  odd = __builtin_amdgcn_readfirstlane(__syncthreads_or(odd));
   int r = r0, cap = longest, good = 0;
   fetch(r);
-  if (EARLY) fetch_turns(r);
+  fetch_positions(r);
+  if (EARLY) fetch_turns();
   while (r < r1) {
-    if (!EARLY) fetch_turns(r);
+    if (!EARLY) fetch_turns();
     int nb = min(odd ? 1 : cap, r1 - r);
     for (;;) {
       __syncthreads();  // the block before is done with LDS
@@ -474,6 +489,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
       int any = 0;
 #pragma unroll
       for (int w = 0; w < NW; ++w) any |= flags[w];
+      any = __builtin_amdgcn_readfirstlane(any);
       if (any & 1) {
         odd = 1;
         if (nb == 1) break;
@@ -487,7 +503,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
     }
     if (nb == cap && ++good == 4 && cap < longest) cap = min(2 * cap, longest), good = 0;
     const int nx = r + nb;
-    if (nx < r1) fetch(nx);
+    if (nx < r1) {
+      fetch(nx);
+      fetch_positions(nx);
+    }
 
     // S' = A S0
 #pragma unroll
@@ -522,7 +541,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
           if (g == 0) out[((long)r * heads + head) * VD + col0 + 16 * n + c] = o[n];
         }
       }
-      if (EARLY && nx < r1) fetch_turns(nx);
+      if (EARLY && nx < r1) fetch_turns();
       r = nx;
       continue;
     }
@@ -620,7 +639,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
       }
       __syncthreads();  // the scores are there
     }
-    if (EARLY && nx < r1) fetch_turns(nx);
+    if (EARLY && nx < r1) fetch_turns();
     bf16x8 vf[VT][TN];
     const int at_v = fresh(tr_row * VROW + (tr_chunk ^ (wave * TN << 5))), at_t = fresh(tr_row * 256 + tr_chunk);
 #pragma unroll
@@ -655,20 +674,28 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
         }
       }
     }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      bf16x8 kf[3];
+    // a tile's operands are read while the tile before is multiplied (left alone the compiler waits for every read by itself: with the
+    // positions as scalars, 309 -> 297 us gated, 396 -> 385 fixed)
+    bf16x8 kf[2][3];
+    auto read_k = [&](int t) {
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
         const char* k = ks + p * IMG + (at_t ^ (t << 5));
-        kf[p] = read_tr(k, k + 16 * 256);
+        kf[t & 1][p] = read_tr(k, k + 16 * 256);
       }
+    };
+    read_k(0);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      if (t + 1 < 8) read_k(t + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int p = 2; p >= 0; --p)
 #pragma unroll
         for (int vp = min(VT - 1, 2 - p); vp >= 0; --vp)
 #pragma unroll
-          for (int n = 0; n < TN; ++n) S[t][n] = mma(kf[p], vf[vp][n], S[t][n]);
+          for (int n = 0; n < TN; ++n) S[t][n] = mma(kf[t & 1][p], vf[vp][n], S[t][n]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     r = nx;
   }
