@@ -9,8 +9,10 @@
 //     its accumulators hold four consecutive outputs of a token, as in the streaming kernel of gemm.hip, whose reduction
 //     (partial sums in 32 bits, fixed order) closes a split product.
 //   * Workgroups start at different chunks of their range (see `first`).
-// 28672 x 4096 with the gated unit: 8 rows 45.2 -> 39.4 us (5.96 TB/s of weights), 64 rows 57.2 -> 42.1; 128256 x 4096, 8 rows: 191 -> 161
-// (6.5 TB/s); 4096 x 14336, 88 rows: 50.1 -> 31.6.  The whole range stands at the dispatch in ops/__init__.py.
+//   * What bounds it: HBM up to 64 rows.  Beyond, LDS: with eight token tiles a chunk is 32 KiB in and 80 KiB out beside 512 cycles of
+//     products, in 1700 to 1900 cycles (activations that a CU's first-level cache holds are no faster).
+// 28672 x 4096 with the gated unit: 8 rows 45.2 -> 37.5 us (6.26 TB/s of weights), 64 rows 57.2 -> 40.1, 97 rows 60.6 -> 48.2; 128256 x
+// 4096, 8 rows: 191 -> 161 (6.5 TB/s); 4096 x 14336, 88 rows: 50.1 -> 31.  The whole range stands at the dispatch in ops/__init__.py.
 #include "common.h"
 
 namespace {
@@ -18,6 +20,10 @@ namespace {
 constexpr int BN = 128, BK = 64, STAGES = 4, ROWB = BK * 2;
 
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
+
+// The chunk a workgroup begins with: the XCDs' an eighth of 64 chunks apart, and within an XCD, whose workgroups' numbers are eight
+// apart, three (with 3 * block an XCD's workgroups met on eight chunks of 64: 28672 x 4096, 1 to 40 rows, 39.5 -> 37.5 us).
+__device__ __forceinline__ int first_chunk(int block, int n) { return ((block >> 3) * 3 + (block & 7) * 8) % n; }
 
 // acc[i][t] += W tile i of the wave x token tile t over chunks [0, n) of both operands: NA * 64 weight rows and MT * 16 token rows a
 // chunk, all of it in LDS stages.  The weight rows lie w_row bytes apart from wp on, those from the 64th on w_half further; xrow(r): bytes
@@ -76,19 +82,36 @@ __device__ __forceinline__ void stream_product(const char* __restrict__ wp, uint
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (c + STAGES - 1 < n) load(c + STAGES - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // The products follow the reads at a distance of two token tiles.  Left to itself the compiler reads two tiles and waits for both
+    // (28672 x 4096 with 97 rows, eight tiles 55 us, seven 58); all of the chunk's reads before its products: 54 with seven, 57 with eight;
+    // at two or four tiles' distance 48 and 51.
     const char* st = lds + (c & (STAGES - 1)) * STAGE;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 a[NA];
+    bf16x8 a[2][NA], b[2 * MT];
+    auto read_a = [&](int ks) {
 #pragma unroll
       for (int i = 0; i < NA; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(st + arow[i] * ROWB + fr + (f[ks] ^ ((2 * (arow[i] >> 4) & 7) << 4)));
+        a[ks][i] = *reinterpret_cast<const bf16x8*>(st + arow[i] * ROWB + fr + (f[ks] ^ ((2 * (arow[i] >> 4) & 7) << 4)));
+    };
+    auto read_b = [&](int j) {  // token tile j % MT of the chunk's half j / MT
+      b[j] = *reinterpret_cast<const bf16x8*>(st + (BN + 16 * (j % MT)) * ROWB + fr + (f[j / MT] ^ ((2 * (j % MT) & 7) << 4)));
+    };
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(st + (BN + 16 * t) * ROWB + fr + (f[ks] ^ ((2 * t & 7) << 4)));
+    for (int j = 0; j < 2; ++j) {
+      if (j % MT == 0) read_a(j / MT);
+      read_b(j);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < NA; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][t], 0, 0, 0);
+    for (int j = 0; j < 2 * MT; ++j) {
+      if (j + 2 < 2 * MT) {
+        if (j + 2 == MT) read_a(1);
+        read_b(j + 2);
+        __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        acc[i][j % MT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j / MT][i], b[j], acc[i][j % MT], 0, 0, 0);
     }
   }
   __syncthreads();
@@ -111,13 +134,13 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
   const int mrows = min(M - m0, 16 * MT);
   const int arow[2] = {PAIR ? 16 * wave : 32 * wave, PAIR ? 64 + 16 * wave : 32 * wave + 16};
   f32x4 acc[2][MT];
-  // Workgroups walk their chunks from different ones on: rows whose length is a power of two put a chunk of all 128 rows on the
-  // same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
+  // Workgroups walk their chunks from different ones on (first_chunk): rows whose length is a power of two put a chunk of all 128 rows on
+  // the same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
   stream_product<MT, 2, POLICY>(
       reinterpret_cast<const char*>(w + (long)n0 * K) + (long)c0 * ROWB, (uint32_t)(K * 2), (PAIR ? n_out : 64) * (long)(K * 2),
       reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB,
       [&](int r) { return (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)); },  // rows past the last repeat it
-      n, n > 0 ? (int)(blockIdx.x * 3 % n) : 0, lds, arow, acc);
+      n, n > 0 ? first_chunk(blockIdx.x, n) : 0, lds, arow, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int j = 16 * t + c16;
@@ -181,7 +204,7 @@ __global__ __launch_bounds__(256, 1) void mid_experts_kernel(const uint16_t* __r
         reinterpret_cast<const char*>(w + ((long)e * N + n0) * K), (uint32_t)(K * 2), n_out * (long)(K * 2),
         reinterpret_cast<const char*>(UNIT ? x : x + (long)(r0 + m0) * K),
         [&](int r) { return (uint32_t)(UNIT ? sorted_tok[r0 + m0 + min(r, last)] : min(r, last)) * (uint32_t)(K * 2); },
-        n, (int)((blockIdx.x * 3 + e) % n), lds, arow, acc);
+        n, (first_chunk(blockIdx.x, n) + e) % n, lds, arow, acc);
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const int j = 16 * t + c16;
@@ -463,16 +486,14 @@ static int mid_product(const void* x, long xs, const void* w, const void* bias, 
 #define MID(MT)                                                                                             \
   return pair ? launch_mid<MT, true>(x, xs, w, bias, y, ys, (float*)ws, M, N, K, S, stream)                 \
               : launch_mid<MT, false>(x, xs, w, bias, y, ys, (float*)ws, M, N, K, S, stream)
-  // Above 96 rows the whole block of eight tiles: what bounds it there is the schedule and not the rows (7 tiles are no faster than
-  // 8 on the gated unit and slower elsewhere: steps of 97 and 110 rows behind cached tokens 3.45 and 3.12 ms with 7, 3.33 and 3.01
-  // with 8; below, 90 rows take 2.68 with 6 and 2.85 with 8, 72 rows 2.57 with 5 and 2.75).
-  switch (M > 96 ? 8 : (M + 15) / 16) {
+  switch ((M + 15) / 16) {
     case 1: MID(1);
     case 2: MID(2);
     case 3: MID(3);
     case 4: MID(4);
     case 5: MID(5);
     case 6: MID(6);
+    case 7: MID(7);
     default: MID(8);
   }
 #undef MID

@@ -53,6 +53,21 @@ def test_dispatch():
         assert ops._mid_gemm(x[:40].clone().requires_grad_(), w, None, False) is None
 
 
+@pytest.mark.parametrize("m", [96, 97, 112, 128])
+def test_two_rounds_of_a_block_of_rows(m):
+    """Two rounds of workgroups with 97 to 128 rows where the second is three quarters full (448 workgroups), not where it is half (400).
+    Eight chunks: workgroups start at each of them."""
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x = torch.randn(129, 512, generator=g, device=DEV).to(BF)
+    w = (torch.randn(57344, 512, generator=g, device=DEV) * 512 ** -0.5).to(BF)
+    got = ops._mid_gemm(x[:m], w, None, True)
+    gu = x[:m].double() @ w.double().t()
+    want = torch.nn.functional.silu(gu[:, :28672]) * gu[:, 28672:]
+    assert float(((got.double() - want).abs() - want.abs() * 2 ** -8 - 1e-5).max()) < 0   # as above: one rounding to 16 bits
+    assert (ops._mid_gemm(x[:m], w[:51200], None, True) is not None) == (m <= 96)
+    assert ops._mid_gemm(x, w, None, True) is None
+
+
 @pytest.mark.parametrize("m", [1, 24, 90])
 def test_operands_on_another_device_are_refused(m):
     """A weight, bias or norm that still lies on the host raises, as in the library, and no kernel reads it."""

@@ -691,19 +691,20 @@ def _stream_gemm(x2, w, bias, pair):
 
 # ``mid_gemm`` (128 weight rows a workgroup, both operands straight into LDS) against what ran before, microseconds in a graph over
 # weights that no cache holds (library with its activation pass, or the kernels above up to 16 rows / mid_gemm):
-#   28672 x 4096 pair    1 row 43.6/39.4    24 rows 50.4/40.2    64 rows 57.2/42.1    104 rows 60.6/55.5    128 rows 61.9/53.3
-#   4096 x 14336         1     25.1/21.4    24      29.0/23.1    64      39.2/28.1    128      75.2/38.8    200      56.9/53.3
-#   6144 x 4096          1     12.9/12.0    24      14.4/13.6    64      17.5/16.6    104      23.2/21.6    200      26.2/32.3
-#   4096 x 4096          1      9.8/10.0    24      13.1/11.4    64      14.9/13.9    104      16.1/17.6
-#   128256 x 4096        1      190/162     24       198/167     64       214/191     104       236/243
-#   57344 x 8192 pair    1      172/146     64       194/161     104      203/219
-#   8192 x 28672         1       90/76      64       147/105     200      311/204
+#   28672 x 4096 pair    1 row 43.6/37.5    24 rows 50.4/37.6    64 rows 57.2/40.1    112 rows 59.2/49     128 rows 59.3/51
+#   4096 x 14336         1     25.1/21.4    24      29.0/23.1    64      39.2/28.1    128      75.7/37.9    200      56.7/50.1
+#   6144 x 4096          1     12.9/12.0    24      14.4/13.6    64      17.5/16.6    112      24.1/22.0    200      25.9/30.5
+#   4096 x 4096          1      9.8/10.0    24      13.1/11.4    64      14.9/13.9     97      16.4/17.0
+#   128256 x 4096        1      190/162     24       198/167     64       214/191     112       236/218     128       239/228
+#   57344 x 8192 pair    1      172/146     64       194/161     112      203/190     128       199/197     160       210/383
+#   8192 x 28672         1       90/76      64       147/105     128      203/116     200       312/165
 #   3584 x 18944         1       46/25      24       108/26      200      121/66
 #   37888 x 3584 pair    1     48.4/53.6    64      64.9/65.7  (296 workgroups: a second round nearly empty)
 #   2048 x 2048          1      5.7/7.2     64       8.7/9.9   (64 workgroups)
 MID_MIN_FILL = 0.75      # of the rounds of one workgroup per CU
 MID_ROWS = 96            # every shape that fills the chip
-MID_ROWS_ONE_ROUND = 128  # one round, and partial sums (32 bits, written and read) below three quarters of the weights' bytes
+MID_ROWS_BLOCK = 128     # one round or full ones (448 workgroups win by 2 to 6 %), and partial sums (32 bits, written and read) below
+MID_BLOCK_FILL = 0.875   # three quarters of the weights' bytes
 MID_ROWS_LONG = 256      # reductions beyond 8192, where the library's pick is poor at every batch
 
 
@@ -719,7 +720,8 @@ def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
         return 0
     if m <= MID_ROWS or (not pair and k > STREAM_MAX_K):
         return splits
-    if m <= MID_ROWS_ONE_ROUND and wgs <= TILE_CUS and (splits == 1 if pair else 16 * m * splits <= 3 * k):
+    if (m <= MID_ROWS_BLOCK and (wgs <= TILE_CUS or wgs >= MID_BLOCK_FILL * TILE_CUS * (-(-wgs // TILE_CUS)))
+            and (splits == 1 if pair else 16 * m * splits <= 3 * k)):
         return splits
     return 0
 
