@@ -197,6 +197,25 @@ def test_sum_with_residual_and_norm(any_shape, m, n, k):
     assert ops.linear_add_norm(x[:, 1:], w[:, 1:].contiguous(), res, ln, 1e-5) is None and torch.equal(res, kept)
 
 
+@pytest.mark.parametrize("m", [96, 97, 112, 128])
+def test_sum_with_norm_of_a_block_of_rows(m):
+    """Partial sums of up to the weights' bytes (128 rows in eight ranges) where the reduction makes the norm, three quarters elsewhere."""
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x = torch.randn(129, 4096, generator=g, device=DEV).to(BF)
+    w = (torch.randn(4096, 4096, generator=g, device=DEV) / 64).to(BF)
+    res, ln = torch.randn(129, 4096, generator=g, device=DEV).to(BF), torch.randn(4096, generator=g, device=DEV).to(BF)
+    got_res, kept = res[:m].clone(), res.clone()
+    got = ops.linear_add_norm(x[:m], w, got_res, ln, 1e-5)
+    assert got is not None and (ops._mid_gemm(x[:m], w, None, False) is not None) == (m <= 96)
+    assert ops.linear_add_norm(x, w, res, ln, 1e-5) is None and torch.equal(res, kept)
+    add = x[:m].double() @ w.double().t()
+    want = add + res[:m].double()
+    # two roundings to 16 bits, of the sum and of the new row: half a unit in the last place, 2^-9, of each and the first's share again
+    assert float(((got_res.double() - want).abs() - 2 ** -8 * (add.abs() + want.abs()) - 1e-5).max()) < 0
+    norm = got_res.double() * (got_res.double().square().mean(1, keepdim=True) + 1e-5).rsqrt() * ln.double()
+    assert float(((got.double() - norm).abs() - 2 ** -8 * norm.abs() - 1e-5).max()) < 0
+
+
 @pytest.mark.parametrize("m,n_q,n_kv,bias,k", [(1, 32, 8, False, 1088), (3, 5, 1, True, 1088), (17, 8, 8, True, 1088), (40, 32, 8, False, 1088),
                                                (5, 2, 1, False, 4096), (3, 2, 1, True, 4672), (17, 4, 1, False, 8704)])
 def test_sum_with_rotation_and_cache_write(any_shape, m, n_q, n_kv, bias, k):

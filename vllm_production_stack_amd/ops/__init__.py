@@ -704,12 +704,16 @@ def _stream_gemm(x2, w, bias, pair):
 MID_MIN_FILL = 0.75      # of the rounds of one workgroup per CU
 MID_ROWS = 96            # every shape that fills the chip
 MID_ROWS_BLOCK = 128     # one round or full ones (448 workgroups win by 2 to 6 %), and partial sums (32 bits, written and read) below
-MID_BLOCK_FILL = 0.875   # three quarters of the weights' bytes
+MID_BLOCK_FILL = 0.875   # MID_SUMS quarters of the weights' bytes
+MID_SUMS = 3
+MID_SUMS_NORM = 4        # where the reduction also makes the residual stream and the norm, whose own pass takes 4.9 us beside the library
+                         # (with it / mid_gemm, 4096 x 4096: 97 rows 20.2/18.1, 113 21.2/19.7, 128 28.8/20.3; 3584 x 3584: 97 rows 22.4/17.1)
 MID_ROWS_LONG = 256      # reductions beyond 8192, where the library's pick is poor at every batch
 
 
-def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
-    """Workgroups along the reduction when ``mid_gemm`` should take the shape, else 0."""
+def _mid_splits(m: int, n: int, k: int, pair: bool, sums: int = MID_SUMS) -> int:
+    """Workgroups along the reduction when ``mid_gemm`` should take the shape, else 0.  ``sums``: quarters of the weights' bytes that
+    the partial sums of a block of rows may have."""
     if not 0 < m <= MID_ROWS_LONG:
         return 0
     splits = int(_kernels().vpsa_mid_gemm_splits(c_int(m), c_int(n), c_int(k), c_int(1 if pair else 0)))
@@ -721,7 +725,7 @@ def _mid_splits(m: int, n: int, k: int, pair: bool) -> int:
     if m <= MID_ROWS or (not pair and k > STREAM_MAX_K):
         return splits
     if (m <= MID_ROWS_BLOCK and (wgs <= TILE_CUS or wgs >= MID_BLOCK_FILL * TILE_CUS * (-(-wgs // TILE_CUS)))
-            and (splits == 1 if pair else 16 * m * splits <= 3 * k)):
+            and (splits == 1 if pair else 16 * m * splits <= sums * k)):
         return splits
     return 0
 
@@ -734,14 +738,14 @@ def _followed(*ts) -> bool:
             or torch._C._len_torch_dispatch_stack() > 0)
 
 
-def _mid_takes(x2, w, bias, pair) -> int:
+def _mid_takes(x2, w, bias, pair, sums=MID_SUMS) -> int:
     """``_mid_splits`` for operands that ``mid_gemm`` reads, else 0."""
     if not (_skinny_enabled and x2.is_cuda and w.device == x2.device and x2.dim() == 2 and x2.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
             and (bias is None or (bias.device == x2.device and bias.dtype == torch.bfloat16 and bias.is_contiguous()
                                   and bias.shape == w.shape[:1]))):
         return 0
-    splits = _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair)
+    splits = _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair, sums)
     return 0 if splits and _followed(x2, w, bias) else splits
 
 
@@ -761,7 +765,7 @@ def _mid_gemm(x2, w, bias, pair):
 def linear_add_norm(x, w, residual, weight, eps):
     """``residual += x @ w.T`` and the norm of the new rows, ``rmsnorm(residual) * weight``, when ``mid_gemm`` splits the product: its
     reduction then makes both.  None (and nothing done) otherwise."""
-    splits = _mid_takes(x, w, None, False)
+    splits = _mid_takes(x, w, None, False, MID_SUMS_NORM)
     m, n = x.shape[0], w.shape[0]
     if (splits < 2 or n > 8192 or residual.shape != (m, n) or residual.dtype != torch.bfloat16 or not residual.is_contiguous()
             or residual.device != x.device or weight.device != x.device or weight.dtype != torch.bfloat16 or weight.shape != (n,)
