@@ -14,6 +14,8 @@
 //
 // The number of valid positions is read from device memory (position counter + 1), so a captured
 // HIP graph replays the same launch for every decode step.
+#include <type_traits>
+
 #include "common.h"
 
 #define DA_KEYS 4  // keys in flight per 8-lane group
@@ -155,13 +157,16 @@ VPSA_EXPORT int vpsa_dense_decode_attention(const void* q, long q_bs, const void
 //                                                   they are; V stays row-major in LDS and is read
 //                                                   through the transposing ds_read_b64_tr_b16, whose
 //                                                   4-key blocks are exactly the accumulator's key order
-// A wave and tile cost 512 cycles of matrix instructions, 512 of exponentials and about 500 of other vector work, so what bounds
-// this is how well waves overlap: rows of 128 B without padding (K's 16-byte chunks are swapped by key bits 1..3, V's halves by
-// key bit 1: both kinds of read stay free of bank conflicts) and 144 registers let three workgroups share a CU; padded rows and
-// 177 registers held two.  The scale goes into the exponent's fused multiply, the mask only touches the last tile, and a
-// window's query blocks run on one XCD.  Measured: 8 windows x 12 heads x 1500 positions 153 -> 93 us (0.6 PFLOP/s), 2 windows
-// 55.5 -> 37.5, 32 windows x 8 heads 324 -> 198.  Four workgroups a CU (128 registers, 16 spilled): 104 us.  A maximum that
-// follows only in steps of 2^8 is no faster and rounds the largest probability: error 1.9e-3 -> 2.3e-3.
+// A wave and tile cost 512 cycles of matrix instructions, 512 of exponentials and 640 of other vector work, in 1900 (vector
+// units 55 % busy, matrix units 27 %), so what bounds this is how well they overlap, and 1152 workgroups are one and a half
+// rounds of 768.  Rows of 128 B without padding (K's 16-byte chunks are swapped by key bits 1..3, V's halves by key bit 1: both
+// kinds of read stay free of bank conflicts) and 144 registers let three workgroups share a CU; padded rows and 177 registers
+// held two.  The scale goes into the exponent's fused multiply, the mask only touches the last tile, and a window's query
+// blocks run on one XCD.  Measured: 8 windows x 12 heads x 1500 positions 153 -> 97 us, 2 windows 55.5 -> 41, 32 windows x 8
+// heads 324 -> 225.  Then, with the queries waited for before the loop, K read two products ahead, the mask in a tile of its
+// own and a slice's products under the next slice's exponentials: 97.3 -> 94.1 (0.59 PFLOP/s), one window 31.0 -> 28.9, four
+// query rows 32 -> 26, 32 windows x 8 heads 225 -> 219.  Four workgroups a CU (128 registers, 16 spilled): 104 us.  A maximum
+// that follows only in steps of 2^8 is no faster and rounds the largest probability: error 1.9e-3 -> 2.3e-3.
 // The [B, heads, Tq, Tk] score matrix never exists in memory.
 #define DF_KT 64
 
@@ -217,6 +222,10 @@ __global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
   stage_load(0);
   stage_write(0);
   __syncthreads();
+  // The queries have arrived before the loop: waited for at their first use inside it, every tile would wait there, and with them
+  // for the tile that is being loaded.
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(qf[ks]));
 
   f32x16 o_acc[2];
 #pragma unroll
@@ -229,24 +238,38 @@ __global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
   const int tr_off = (4 * hf + tr_row) * 64 + ((16 * ((lane >> 4) & 1) + 4 * (lane & 3)) ^ ((tr_row & 2) << 4));
   const int k_off = r * 64, k_swz = (r >> 1) & 7;
 
-  for (int t = 0; t < n_tiles; ++t) {
+  auto tile = [&](int t, auto masked) {
     const int buf = t & 1;
-    if (t + 1 < n_tiles) stage_load(t + 1);
+    if (!masked.value) stage_load(t + 1);
+    // the products follow the reads at a distance of two
     f32x16 s_acc[2];
+    bf16x8 kf[8], vf[4][2];
+    auto read_k = [&](int j) {
+      kf[j] = *(const bf16x8*)(&lds_k[buf][32 * (j >> 2) * 64 + k_off + 8 * ((2 * (j & 3) + hf) ^ k_swz)]);
+    };
+    auto read_v = [&](int s4) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+      for (int cb = 0; cb < 2; ++cb) {
+        const uint16_t* blk = &lds_v[buf][16 * s4 * 64] + (tr_off ^ (32 * cb));
+        vf[s4][cb] = lds_tr_pair(blk, blk + 8 * 64);
+      }
+    };
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s_acc[kb][i] = 0.f;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 a = *(const bf16x8*)(&lds_k[buf][32 * kb * 64 + k_off + 8 * ((2 * ks + hf) ^ k_swz)]);
-        s_acc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s_acc[kb], 0, 0, 0);
-      }
+    for (int j = 0; j < 2; ++j) read_k(j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j + 2 < 8) read_k(j + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      s_acc[j >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[j], qf[j & 3], s_acc[j >> 2], 0, 0, 0);
     }
     // accumulator register i of block kb, half hf = key 64 t + 32 kb + 8 (i >> 2) + 4 hf + (i & 3)
-    const int kbase = t * DF_KT;
-    const bool need_mask = kbase + DF_KT > Tk;
-    if (need_mask) {
+    if (masked.value) {
+      const int kbase = t * DF_KT;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -263,36 +286,33 @@ __global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
     float psum = 0.f;
-    bf16x8 pf[4];
+    read_v(0);
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        u32x4 pk;
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[kb][8 * s + 2 * jj], scale_log2e, -m_new));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[kb][8 * s + 2 * jj + 1], scale_log2e, -m_new));
-          psum += p0 + p1;
-          pk[jj] = pack_bf16x2(p0, p1);
-        }
-        pf[kb * 2 + s] = __builtin_bit_cast(bf16x8, pk);
-      }
-    l_run = l_run * alpha + psum;
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
+    for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o_acc[cb][i] *= alpha;
+    // a slice's products run under the next one's exponentials
 #pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const uint16_t* blk = &lds_v[buf][16 * s4 * 64] + (tr_off ^ (32 * cb));
-        const bf16x8 a = lds_tr_pair(blk, blk + 8 * 64);
-        o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pf[s4], o_acc[cb], 0, 0, 0);
+    for (int s4 = 0; s4 < 4; ++s4) {
+      if (s4 + 1 < 4) read_v(s4 + 1);
+      u32x4 pk;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[s4 >> 1][8 * (s4 & 1) + 2 * jj], scale_log2e, -m_new));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[s4 >> 1][8 * (s4 & 1) + 2 * jj + 1], scale_log2e, -m_new));
+        psum += p0 + p1;
+        pk[jj] = pack_bf16x2(p0, p1);
       }
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+        o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[s4][cb], __builtin_bit_cast(bf16x8, pk), o_acc[cb], 0, 0, 0);
     }
-    if (t + 1 < n_tiles) stage_write(buf ^ 1);
+    l_run = l_run * alpha + psum;
+    if (!masked.value) stage_write(buf ^ 1);
     __syncthreads();
-  }
+  };
+  for (int t = 0; t + 1 < n_tiles; ++t) tile(t, std::false_type{});
+  tile(n_tiles - 1, std::true_type{});
   // O^T accumulator register i of block cb, half hf = channel 32 cb + 8 (i >> 2) + 4 hf + (i & 3)
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   if (qrow < Tq) {

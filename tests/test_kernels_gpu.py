@@ -623,6 +623,19 @@ def test_dense_attention_matches_fp32(b, heads, tq, tk):
     assert not ops.dense_attention_supported(q.float(), k.float(), v.float(), heads)
 
 
+@pytest.mark.parametrize("tq,tk", [(33, 63), (31, 64), (128, 65), (4, 127), (97, 128), (1, 129), (129, 192)])
+def test_dense_attention_at_tile_edges(tq, tk):
+    """The last key tile has a pass of its own: full, one key short, one key, behind none, one or two others."""
+    torch.manual_seed(tq + tk)
+    q, k, v = [torch.randn(3, t, 128, device=DEV).to(BF) for t in (tq, tk, tk)]
+    got = ops.dense_attention(q, k, v, 2).double()
+    qh, kh, vh = [t.double().view(3, -1, 2, 64).transpose(1, 2) for t in (q, k, v)]
+    p = torch.softmax(qh @ kh.transpose(-1, -2) * 0.125, dim=-1)
+    want, size = [(p @ t).transpose(1, 2).reshape(3, tq, 128) for t in (vh, vh.abs())]
+    # probabilities and the result are rounded to 16 bits once (half a unit: 2^-9 of a value), scores and sums kept in 32
+    assert float(((got - want).abs() - 2 ** -9 * (size + want.abs()) - 2 ** -14 * size).max()) < 0
+
+
 def test_qkv_projection_split_for_prefill_sized_batches():
     """From 4096 rows on the fused q/k/v projection is two library GEMMs writing into one buffer
     (the library is slow at the fused width): same result as the single call, one contiguous
