@@ -3,12 +3,15 @@ server sharing between two engines, controller reporting, P->D page push, serde.
 
 import asyncio
 import copy
+import gc
 import threading
+import weakref
 
 import numpy as np
 import pytest
 import torch
 
+from vllm_production_stack_amd import ops
 from vllm_production_stack_amd.cache_server import CacheServer
 from vllm_production_stack_amd.engine.config import EngineConfig, KVOffloadConfig, KVTransferConfig
 from vllm_production_stack_amd.engine.llm_engine import LLMEngine
@@ -209,6 +212,91 @@ def _serve_in_thread(coro_factory):
     t.start()
     box["ready"].wait(10)
     return loop, box["obj"]
+
+
+class _Device:
+    """A device whose copies are over only when somebody waits: stands in for the calls of ``PageSerde.decode`` on a GPU, and notes
+    pinned buffers that go back to their allocator while a copy still reads them."""
+
+    def __init__(self, monkeypatch, fail=False):
+        self.queued, self.over, self.early, self.buffers, self.fail = 0, 0, 0, 0, fail
+        self.lock, self.all_in, self.reads = threading.RLock(), None, {}
+        empty, dev = torch.empty, self
+
+        class Event:
+            def record(self, stream=None):
+                self.at = dev.queued
+
+            def synchronize(self):
+                dev.over = max(dev.over, self.at)
+
+        class Stream:
+            def synchronize(self):
+                dev.over = dev.queued
+
+        def pinned_empty(*size, pin_memory=False, **kw):
+            t = empty(*size, **kw)
+            if pin_memory:
+                with dev.lock:
+                    dev.buffers += 1
+                    key = dev.buffers
+                t.key = key
+                weakref.finalize(t, dev.freed, key)
+            return t
+
+        def page_decode(src, pinned, size, n, n_ctx, unit_elems, device, spc=ops.RANS_SPC):
+            with dev.lock:
+                dev.queued += 1
+                dev.reads[pinned.key] = dev.queued
+            if dev.all_in is not None:
+                dev.all_in.wait(20)
+            if dev.fail:
+                raise RuntimeError("cachegen_decode: unsupported arguments")
+            return empty(n, dtype=torch.bfloat16)
+
+        monkeypatch.setattr(torch, "empty", pinned_empty)
+        monkeypatch.setattr(torch.cuda, "Event", Event)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream())
+        monkeypatch.setattr(ops, "page_decode", page_decode)
+
+    def freed(self, key):
+        self.early += self.reads.get(key, 0) > self.over
+
+
+def _rans_blob(monkeypatch):
+    sd = PageSerde(3, 2, 64, torch.bfloat16, "cachegen", levels=[31, 31, 15])
+    sym, scales = ops.cachegen_encode(torch.randn(sd.page_elems).bfloat16(), torch.tensor(sd.levels, dtype=torch.int32), sd.unit_elems, 3)
+    return sd, sd.pack(sd.rans_payload(sym, scales), None)
+
+
+@pytest.mark.parametrize("callers", [1, 2, 3, 5])
+def test_pinned_buffers_outlive_the_copies_that_read_them(callers, monkeypatch):
+    """More callers at once than a serialiser keeps buffers, and a serialiser that ends with copies still queued."""
+    sd, blob = _rans_blob(monkeypatch)
+    dev = _Device(monkeypatch)
+    dev.all_in = threading.Barrier(callers)
+    threads = [threading.Thread(target=sd.decode, args=(blob, torch.device("cuda"))) for _ in range(callers)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(30)
+    gc.collect()
+    assert dev.queued == callers and dev.buffers == callers and dev.early == 0
+    dev.all_in = None
+    sd.decode(blob, torch.device("cuda"))
+    del sd, threads, t
+    gc.collect()
+    assert dev.early == 0 and dev.over == dev.queued
+
+
+def test_pinned_buffers_outlive_a_call_that_fails(monkeypatch):
+    sd, blob = _rans_blob(monkeypatch)
+    dev = _Device(monkeypatch, fail=True)
+    for _ in range(4):
+        with pytest.raises(RuntimeError):
+            sd.decode(blob, torch.device("cuda"))
+    gc.collect()
+    assert dev.queued == 4 and dev.early == 0
 
 
 @pytest.mark.parametrize("serde", ["naive", "cachegen"])

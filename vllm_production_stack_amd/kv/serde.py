@@ -84,6 +84,26 @@ def default_levels(n_layers: int) -> list[int]:
     return [127 if i < a else (31 if i < b else 15) for i in range(n_layers)]
 
 
+class _Pinned:
+    """A pinned buffer on its way through a call, and what the device still has to pass before the buffer's memory may be used again.
+    Its copies are queued by the kernel library, so torch's allocator knows nothing of them: whoever lets go of the buffer waits."""
+
+    __slots__ = ("bytes", "busy")
+
+    def __init__(self, size: int):
+        self.bytes = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+        self.busy = None  # a stream or an event: over with its ``synchronize``
+
+    def wait(self) -> None:
+        if self.busy is not None:
+            self.busy.synchronize()
+            self.busy = None
+
+    def __del__(self):
+        if getattr(self, "busy", None) is not None:
+            self.wait()
+
+
 class PageSerde:
     def __init__(self, n_layers: int, n_kv: int, head_dim: int, dtype: torch.dtype, kind: str = "naive",
                  levels: list[int] | None = None):
@@ -93,33 +113,33 @@ class PageSerde:
         self.unit_elems = n_kv * ops.PAGE * head_dim
         self.levels = levels or default_levels(n_layers)
         self._levels_dev: dict = {}
-        # Pinned buffers that pages pass through on their way between host and device, each with the event of the copy that
-        # last read it: a pageable copy of a page's 3.5 MB takes 0.65 ms to the host and 0.13 ms to the device, a pinned one
-        # 0.07.  A call takes one out and gives it back, so calls of several threads do not wait for each other; at most
-        # two of each kind are kept, which lets one thread copy a page in while the one before is on its way.
+        # Pinned buffers that pages pass through on their way between host and device: a pageable copy of a page's 3.5 MB takes
+        # 0.65 ms to the host and 0.13 ms to the device, a pinned one 0.07.  A call takes one out and gives it back, so calls of
+        # several threads do not wait for each other; at most two of each kind are kept, which lets one thread copy a page in
+        # while the one before is on its way.
         self._out_bufs: deque = deque()
-        self._in_bufs: deque = deque([(None, None)] * _KEPT)
+        self._in_bufs: deque = deque([None] * _KEPT)
 
-    def __getstate__(self):  # (pinned buffers, events and device tensors stay with the object they were made for)
-        return {**self.__dict__, "_levels_dev": {}, "_out_bufs": deque(), "_in_bufs": deque([(None, None)] * _KEPT)}
+    def __getstate__(self):  # (pinned buffers and device tensors stay with the object they were made for)
+        return {**self.__dict__, "_levels_dev": {}, "_out_bufs": deque(), "_in_bufs": deque([None] * _KEPT)}
 
     @staticmethod
-    def _take(bufs: deque, size: int) -> torch.Tensor:
+    def _take(bufs: deque, size: int) -> _Pinned:
         """A pinned buffer of at least ``size`` bytes that no copy reads any more."""
         try:
-            buf, read = bufs.popleft()
+            buf = bufs.popleft()
         except IndexError:
-            buf = read = None
-        if read is not None:
-            read.synchronize()
-        if buf is None or buf.numel() < size:
-            buf = torch.empty(size + size // 8, dtype=torch.uint8, pin_memory=True)
+            buf = None
+        if buf is not None:
+            buf.wait()
+        if buf is None or buf.bytes.numel() < size:
+            buf = _Pinned(size + size // 8)
         return buf
 
     @staticmethod
-    def _give(bufs: deque, buf: torch.Tensor, read=None) -> None:
+    def _give(bufs: deque, buf: _Pinned) -> None:
         if len(bufs) < _KEPT:
-            bufs.append((buf, read))
+            bufs.append(buf)
 
     def _header(self, payload_len: int) -> bytes:
         return _HDR.pack(MAGIC, 1, self.kind, self.n_layers, self.n_kv, self.head_dim, ops.PAGE,
@@ -182,18 +202,23 @@ class PageSerde:
         body = torch.empty(o4 + 2 * n, dtype=torch.uint8, device=dev)
         sym, _ = ops.cachegen_encode(flat.contiguous(), self._levels(dev), self.unit_elems, self.n_layers,
                                      scales=body[:o1].view(torch.float32))
+        ops.ensure_device()
+        stream = torch.cuda.current_stream()  # the one that the kernel library queues on
         buf = self._take(self._out_bufs, o4 + n)  # (a value rarely codes to more than a byte)
-        meta = buf[:16].view(torch.int64)
+        buf.busy = stream
+        meta = buf.bytes[:16].view(torch.int64)
         ops.rans_encode_into(sym.view(-1), self.n_layers, body[o1:o2], body[o2:o3], body[o3:o4], body[o4:], meta=meta)
-        torch.cuda.current_stream(dev).synchronize()
+        stream.synchronize()
         total, bad = meta.tolist()
         if bad:
             raise RuntimeError("rans_encode: frequency table could not be normalised")
-        if buf.numel() < o4 + total:
+        if buf.bytes.numel() < o4 + total:
             buf = self._take(self._out_bufs, o4 + total)
+            buf.busy = stream
         done, at = new(_RANS_HDR.size + o4 + total)
         ctypes.memmove(at, _RANS_HDR.pack(ops.RANS_SPC, n_streams, total), _RANS_HDR.size)
-        ops.fetch_bytes(body, buf, at + _RANS_HDR.size, o4 + total)
+        ops.fetch_bytes(body, buf.bytes, at + _RANS_HDR.size, o4 + total)
+        buf.busy = None  # (fetched: nothing is queued behind it)
         self._give(self._out_bufs, buf)
         return done
 
@@ -275,11 +300,14 @@ class PageSerde:
         body = payload[a:a + size]
         if torch.device(device).type == "cuda":
             body = np.ascontiguousarray(body)
+            ops.ensure_device()
+            stream = torch.cuda.current_stream()  # the one that the kernel library queues on
             buf = self._take(self._in_bufs, size)
-            out = ops.page_decode(body.ctypes.data, buf, size, n, self.n_layers, self.unit_elems, device, spc)
-            read = torch.cuda.Event()
-            read.record(torch.cuda.current_stream(out.device))
-            self._give(self._in_bufs, buf, read)
+            buf.busy = stream  # until there is an event, also if the call ends early
+            out = ops.page_decode(body.ctypes.data, buf.bytes, size, n, self.n_layers, self.unit_elems, device, spc)
+            buf.busy = torch.cuda.Event()
+            buf.busy.record(stream)
+            self._give(self._in_bufs, buf)
             return out
         body = torch.from_numpy(body.copy()).to(device)
         sym = ops.rans_decode(body[o1:o2].view(torch.int16), body[o2:o3].view(torch.int32), body[o3:o4].view(torch.int16), body[o4:],
