@@ -23,6 +23,12 @@
 //   * 128 columns: two workgroups share a CU, and while one cuts and stages, the other multiplies.  256: one of eight waves (four waves of
 //     64 columns spill 250 registers).
 // A block with a value that is not finite, and all after it in the run, go token by token on vector arithmetic, for zero times infinity.
+// Gates that forget too fast for blocks of more than eight tokens (a quarter and less a token, or now and then all at once) take the
+// rest of their run token by token as well, 16 tokens in 32 bits in LDS at a time: 1.8 us a token of both phases with two workgroups a
+// CU, where blocks of eight cost 16, and of one the same.  8192 rows, 32 heads, 128 x 128, in blocks down to one token / so, by the mean
+// logit behind a lower bound of 0: 0 546 / 518, -2 1064 / 927, -6 2095 / 963, -14 4146 / 979, -40 8252 / 976; token by token out of memory 1559.
+// 200 rows 64 / 67, 111 / 117, 199 / 121, 371 / 121, 712 / 121; 206.  The loop stands behind the blocks' and not inside: shared by turns, its
+// registers and theirs spilled (302 -> 338 where no gate forgets).
 // Pieces: the step's list is walked in runs of `group` pieces of one sequence.  Phase 1 makes the runs' end states from zero,
 // chain_kernel turns them into start states, phase 2 computes the outputs; phase 0 walks whole sequences from slot to slot.
 #include "common.h"
@@ -33,6 +39,7 @@ constexpr int RT = 32;     // tokens of a block
 constexpr int RD = 128;    // state rows (key channels)
 constexpr int TN = 2;      // tiles of 16 value columns a wave holds
 constexpr int IMG = RT * RD * 2;  // one part of q^ or k^
+constexpr int WALK = 8;    // blocks of so few tokens cost more than the tokens one by one
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -322,6 +329,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2*>(p + i * IMG) = (u32x2){a[i], b[i]};
   };
+  // gated: s = sigmoid(x) and 1 - s of a fetched logit, from one exponential: 1 - a would lose what a near 1 rounds away
+  auto gate = [&](int u, int i, f32x4 bias, float* s, float* rest) {
+    sigmoids((i & 1 ? bf16hi(rk[u][i >> 1]) : bf16lo(rk[u][i >> 1])) + bias[i], s, rest);
+  };
   // registers -> LDS for the first nb rows; bit 0: a value is not finite, bit 1: out of range.  Rows past them: k^ is zero, q^ and v
   // are never used with anything else.
   auto stage = [&](int nb) {
@@ -338,10 +349,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
         const bool in = row_of(u) < nb;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          // s = sigmoid(x) and 1 - s from one exponential: 1 - a would lose what a near 1 rounds away
-          const float x = (i & 1 ? bf16hi(rk[u][i >> 1]) : bf16lo(rk[u][i >> 1])) + bias[i];
           float s, rest;
-          sigmoids(x, &s, &rest);
+          gate(u, i, bias, &s, &rest);
           a[u][i] = in ? low[i] + (1.f - low[i]) * s : 1.f;
           k[u][i] = in ? (1.f - low[i]) * rest : 0.f;
           sum = fmaf(a[u][i], 0.f, sum);
@@ -380,12 +389,6 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
         const int ch = fresh(ch0);
         put_k(row_of(u), ch, k[u]);
         if (PHASE != 1) put_q(row_of(u), ch, q);
-        if (nb == 1 && row_of(u) == 0)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            one[RD + ch0 + i] = k[u][i];
-            if (PHASE != 1) one[ch0 + i] = q[i];
-          }
       }
     } else {
 #pragma unroll
@@ -454,7 +457,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
       } else {
         *reinterpret_cast<u32x4*>(to) = w;
       }
-      if (nb == 1 && row == 0)
+      if (!GATED && nb == 1 && row == 0)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           one[2 * RD + vch + 2 * i] = VT == 3 ? silu(bf16lo(w[i])) : bf16lo(w[i]);
@@ -467,6 +470,36 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
     if (lane == 0) flags[wave] = any;
   };
 
+  // gated: 16 tokens (from the 16 * h-th fetched row on) for the walk token by token: k | a | q in 32 bits, and with the first all of v
+  float* const walk_k = reinterpret_cast<float*>(ks);
+  float* const walk_a = walk_k + 16 * RD;
+  float* const walk_q = reinterpret_cast<float*>(qs);
+  static_assert(2 * 16 * RD * 4 <= 3 * IMG && 16 * RD * 4 <= 3 * IMG, "place of the walk's operands");
+  auto stage_walk = [&](int h) {
+    const f32x4 bias = *reinterpret_cast<const f32x4*>(args.gate_bias + head * RD + ch0);
+    const f32x4 low = *reinterpret_cast<const f32x4*>(args.gate_lower + head * RD + ch0);
+#pragma unroll
+    for (int u = 0; u < QU; ++u) {
+      if (row_of(u) >> 4 != h) continue;
+      f32x4 a, k, q;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float s, rest;
+        gate(u, i, bias, &s, &rest);
+        a[i] = low[i] + (1.f - low[i]) * s;
+        k[i] = (1.f - low[i]) * rest;
+        q[i] = silu(i & 1 ? bf16hi(rq[u][i >> 1]) : bf16lo(rq[u][i >> 1]));
+      }
+      const int at = fresh((row_of(u) & 15) * RD + ch0);
+      *reinterpret_cast<f32x4*>(walk_k + at) = k;
+      *reinterpret_cast<f32x4*>(walk_a + at) = a;
+      if (PHASE != 1) *reinterpret_cast<f32x4*>(walk_q + at) = q;
+    }
+#pragma unroll
+    for (int u = 0; u < VU; ++u)
+      if (h == 0) *reinterpret_cast<u32x4*>(vs + (vrow + 16 * u) * VROW + (((vch >> 3) ^ swz(vrow + 16 * u)) << 4)) = rv[u];
+  };
+
   // fragment addresses within an image; a tile further is an XOR away
   const int row16 = c * 256 + ((g >> 1) ^ swz(c)) * 16 + (g & 1) * 8;  // k^ for the scores: channels 4 g .. of tile 0
   const int row_q = c * 256 + (g ^ swz_q(c)) * 16;
@@ -476,13 +509,19 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
   __syncthreads();
   odd = __builtin_amdgcn_readfirstlane(__syncthreads_or(odd));
   int r = r0, cap = longest, good = 0;
+  int wait = 1;   // good blocks of 16 tokens and more before a longer one is tried: doubled where that failed
+  // gated: blocks of WALK tokens and fewer, and tries that end with one, before the rest of the run goes token by token (one token that
+  // forgets all takes eight of them; in a run of few tokens they would be most of its time)
+  int left = max(1, min(12, (r1 - r0) / 32));
+  bool walk = false;
   fetch(r);
   fetch_positions(r);
   if (EARLY) fetch_turns();
   while (r < r1) {
     if (!EARLY) fetch_turns();
-    int nb = min(odd ? 1 : cap, r1 - r);
-    for (;;) {
+    int nb = min(odd && !GATED ? 1 : cap, r1 - r);
+    walk = GATED && (odd || left <= 0);
+    while (!walk) {
       __syncthreads();  // the block before is done with LDS
       stage(nb);
       __syncthreads();
@@ -497,11 +536,17 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
       } else if ((any & 2) && nb > 1) {
         nb = cap = nb >> 1;
         good = 0;
+        if (nb > WALK) wait = min(2 * wait, 16);
+        else --left;
       } else {
         break;
       }
+      walk = GATED && (odd || left <= 0);
     }
-    if (nb == cap && ++good == 4 && cap < longest) cap = min(2 * cap, longest), good = 0;
+    if (walk) break;
+    if (nb <= WALK) --left;
+    if (nb == longest) wait = 1;
+    if (nb == cap && cap < longest && ++good >= (cap > WALK ? wait : 1)) cap = min(2 * cap, longest), good = 0;
     const int nx = r + nb;
     if (nx < r1) {
       fetch(nx);
@@ -522,7 +567,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
     if (GATED && PHASE == 1 && tid < 32)
 #pragma unroll
       for (int i = 0; i < 4; ++i) pgate[i] *= pn[ch0 + i];
-    if (odd) {  // one token on vector arithmetic
+    if (!GATED && odd) {  // one token on vector arithmetic
       float o[TN];
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
@@ -696,6 +741,63 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
 #pragma unroll
           for (int n = 0; n < TN; ++n) S[t][n] = mma(kf[t & 1][p], vf[vp][n], S[t][n]);
       __builtin_amdgcn_sched_barrier(0);
+    }
+    r = nx;
+  }
+  // token by token, the same channels and columns a lane
+  while (GATED && r < r1) {
+    const int rows = min(RT, r1 - r), nx = r + rows;
+    for (int h = 0; 16 * h < rows; ++h) {
+      const int m = min(rows - 16 * h, 16);
+      __syncthreads();  // what was there before has been read
+      stage_walk(h);
+      if (16 * h + m == rows && nx < r1) fetch(nx);
+      __syncthreads();
+      if (PHASE == 1 && tid < 32) {
+#pragma unroll 4
+        for (int i = 0; i < m; ++i) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(walk_a + i * RD + ch0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) pgate[j] *= a[j];
+        }
+      }
+      for (int i = 0; i < m; ++i) {
+        float v[TN], o[TN];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          const int col = fresh(col0 + 16 * n + c), row = 16 * h + i;
+          v[n] = bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(vs + row * VROW + (((col >> 3) ^ swz(row)) << 4) + (col & 7) * 2));
+          o[n] = 0.f;
+        }
+        f32x4 a[2], k[2], q[2];  // a tile's are read while the tile before is computed
+        const int at = fresh(i * RD + 4 * g);
+        auto read = [&](int t) {
+          a[t & 1] = *reinterpret_cast<const f32x4*>(walk_a + at + 16 * t);
+          k[t & 1] = *reinterpret_cast<const f32x4*>(walk_k + at + 16 * t);
+          if (PHASE != 1) q[t & 1] = *reinterpret_cast<const f32x4*>(walk_q + at + 16 * t);
+        };
+        read(0);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          if (t + 1 < 8) read(t + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              S[t][n][j] = fmaf(k[t & 1][j], v[n], S[t][n][j] * a[t & 1][j]);
+              if (PHASE != 1) o[n] = fmaf(S[t][n][j], q[t & 1][j], o[n]);
+            }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (PHASE != 1)
+#pragma unroll
+          for (int n = 0; n < TN; ++n) {
+            o[n] += __shfl_xor(o[n], 16, 64);
+            o[n] += __shfl_xor(o[n], 32, 64);
+            if (g == 0) out[((long)(r + 16 * h + i) * heads + head) * VD + col0 + 16 * n + c] = o[n];
+          }
+      }
     }
     r = nx;
   }

@@ -15,13 +15,17 @@ def i32(x):
     return torch.tensor(x, dtype=torch.int32, device=DEV)
 
 
-def gated(heads, vdim, lens, starts, lower, bias, seed=0, slots=None, pieces=True):
-    """(outputs, expected, states, expected states) of one call; ``lower`` / ``bias``: (least, most) per channel."""
+def gated(heads, vdim, lens, starts, lower, bias, seed=0, slots=None, pieces=True, resets=()):
+    """(outputs, expected, states, expected states) of one call; ``lower`` / ``bias``: (least, most) per channel; ``resets``: rows
+    whose gates are nothing in every fifth channel."""
     g = torch.Generator().manual_seed(seed)
     t, hd = sum(lens), heads * 128
     proj = torch.randn(t, 2 * hd + heads * vdim, generator=g).bfloat16()
     lo = torch.rand(hd, generator=g) * (lower[1] - lower[0]) + lower[0]
     b = torch.rand(hd, generator=g) * (bias[1] - bias[0]) + bias[0]
+    if resets:
+        lo[::5] = 0
+        proj[list(resets), hd:2 * hd] = -60
     slots = list(range(len(lens))) if slots is None else slots
     state = torch.randn(len(lens), hd * vdim + 4, generator=g)
     pj = proj.double()
@@ -69,25 +73,64 @@ def test_gates_that_forget_at_once(bias):
         assert off(out, want) < 5e-7 and off(st, ends) < 1e-6
 
 
+# gates that are nothing now and then among others that last: blocks that shrink and grow again, runs that end token by token, runs that
+# begin or end with such a token, sequences too short for a second try
+@pytest.mark.parametrize("vdim", [128, 256])
+@pytest.mark.parametrize("lens,pieces,every,first", [([700], True, 7, 3), ([700], True, 45, 0), ([900, 300], True, 250, 31), ([300], False, 100, 50),
+                                                     ([20, 9, 40], False, 20, 5), ([33], False, 33, 32), ([130], False, 16, 15)])
+def test_gates_that_forget_now_and_then(vdim, lens, pieces, every, first):
+    resets = range(first, sum(lens), every)
+    out, want, st, ends = gated(2, vdim, lens, [4] * len(lens), (0.2, 0.9), (1.0, 3.0), seed=7, pieces=pieces, resets=resets)
+    assert off(out, want) < 5e-7 and off(st, ends) < 1e-6
+
+
+def test_gates_that_forget_cost_a_few_times_the_others():
+    """Token by token a run takes about three times as long as in blocks of 32 tokens; in blocks that shrink to one token it took 27."""
+    heads, t = 32, 4096
+    hd = heads * 128
+    g = torch.Generator(device=DEV).manual_seed(2)
+    proj = torch.randn(t, 3 * hd, generator=g, device=DEV).bfloat16()
+    state, lower = torch.zeros(1, hd * 128, device=DEV), torch.zeros(hd, device=DEV)
+    pieces = tuple(torch.from_numpy(c).to(DEV) for c in ops.build_scan_pieces([t]))
+    pos, cu, slot = torch.arange(t, dtype=torch.int32, device=DEV), i32([0, t]), i32([0])
+
+    def time(logit):
+        bias, best = torch.full((hd,), logit, device=DEV), float("inf")
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ops.recurrent_scan(proj, 0, hd, 2 * hd, heads, 128, 128, state, 0, cu, slot, pos, gate_bias=bias, gate_lower=lower, pieces=pieces)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    usual = time(2.0)
+    assert max(time(logit) for logit in (-6.0, -14.0, -40.0)) < 6 * usual
+
+
 def test_rows_of_no_sequence():
     out, want, st, ends = gated(2, 128, [40, 60], [0, 8], (0.2, 0.9), (1.0, 3.0), slots=[-1, 1], pieces=False)
     assert (out[:40] == 0).all() and off(out, want) < 5e-7 and off(st, ends) < 1e-6
 
 
-def test_a_value_that_is_not_finite_stays_in_its_column():
+@pytest.mark.parametrize("t,pieces", [(70, False), (300, True)])
+def test_a_value_that_is_not_finite_stays_in_its_column(t, pieces):
     g = torch.Generator().manual_seed(5)
-    hd, t = 128, 70
+    hd = 128
+    cut = ops.build_scan_pieces([t], target=6) if pieces else None
+    cut = None if cut is None else tuple(torch.from_numpy(c).to(DEV) for c in cut)
     proj = torch.randn(t, 3 * hd, generator=g).bfloat16().to(DEV)
     proj[40, 2 * hd + 7] = float("inf")
     args = (i32([0, t]), i32([0]), torch.arange(t, dtype=torch.int32, device=DEV))
     out = ops.recurrent_scan(proj, 0, hd, 2 * hd, 1, 128, 128, torch.zeros(1, 128 * 128, device=DEV), 0, *args,
-                             gate_bias=torch.ones(128, device=DEV), gate_lower=torch.full((128,), 0.5, device=DEV))
+                             gate_bias=torch.ones(128, device=DEV), gate_lower=torch.full((128,), 0.5, device=DEV), pieces=cut)
     bad = ~torch.isfinite(out[:, 0])
     assert bad[40:, 7].all() and int(bad.sum()) == t - 40
     # and it stays as it was beside a step in which the value is finite
     proj[40, 2 * hd + 7] = 1.0
     ref = ops.recurrent_scan(proj, 0, hd, 2 * hd, 1, 128, 128, torch.zeros(1, 128 * 128, device=DEV), 0, *args,
-                             gate_bias=torch.ones(128, device=DEV), gate_lower=torch.full((128,), 0.5, device=DEV))
+                             gate_bias=torch.ones(128, device=DEV), gate_lower=torch.full((128,), 0.5, device=DEV), pieces=cut)
     keep = [i for i in range(128) if i != 7]
     assert off(out[:, 0, keep], ref[:, 0, keep].double().cpu()) < 5e-7
 
