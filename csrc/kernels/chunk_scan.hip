@@ -14,7 +14,7 @@
 //   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1564 / 297 us,
 //     fixed 128 x 256 701 / 385; 1000 rows: gated (16 heads, three sequences) 229 / 55, fixed (one) 154 / 84; 200 rows of two 199 / 37.
 //   * 1 / R must stay in range: a block in which some |R| leaves 2^-60 .. 2^60 is taken again with half its tokens (a block of one token
-//     divides by nothing); fixed decays know their longest block beforehand.
+//     divides by nothing); fixed decays know their longest block beforehand, and those that need shorter ones go to retention.hip.
 //   * A workgroup holds a head's whole 128 x VD state in accumulators, 32 columns a wave, so q, k and the scores are made once for all
 //     columns.  S' is cut into parts as it lies in the accumulators: register r of lane (c, g) is row 4 g + r of
 //     a 16-row tile, and two tiles are one operand of 32 channels.  The outputs come out transposed: four columns of a token a lane.

@@ -147,7 +147,7 @@ def test_fixed_decay_without_pieces_matches_the_walk(vdim, act):
     pos = torch.cat([torch.arange(3, 3 + n) for n in lens]).int().to(DEV)
     cols = (0, hd, 2 * hd, heads, 128, vdim)
     whole = start.clone()
-    out = ops.recurrent_scan(proj, *cols, whole, 0, i32([0, 40, 49, 82]), i32([0, 1, 2]), pos, decay=decay, act=act)
+    out = ops.recurrent_scan(proj, *cols, whole, 0, i32([0, 40, 49, 82]), i32([0, 1, 2]), pos, decay=decay, act=act, min_decay=0.4)
     step, rows, at = start.clone(), [], 0
     for s, n in enumerate(lens):
         for k in range(0, n, seqmix.SCAN_BLOCK_MIN_ROWS - 1):

@@ -57,13 +57,16 @@ def off(got, want):
     return float((got.double().cpu() - want).norm() / want.norm())
 
 
-@pytest.mark.parametrize("heads,vdim,lens,starts,rot,layout,act", [
+SHAPES = [
     (2, 256, [128], [0], 128, 0, False),            # whole blocks, one sequence
     (1, 128, [129, 1, 16, 17], [0, 5, 0, 9], 128, 1, False),   # one token past a block, one-token and half-block sequences
     (3, 256, [150, 333], [40, 0], 64, 0, False),    # partial rotation, a continued sequence first
     (2, 128, [287], [0], 0, 0, True),               # silu inputs
     (2, 256, [160], [7], 8, 1, False),
-])
+]
+
+
+@pytest.mark.parametrize("heads,vdim,lens,starts,rot,layout,act", SHAPES)
 def test_blocks_match_the_recurrence(heads, vdim, lens, starts, rot, layout, act):
     decay = [0.999, 0.5, 0.05][:heads]  # the last one's 32nd power is far below what 32 bits can divide by
     call, kw, want, ends = inputs(heads, vdim, lens, starts, decay, rot, layout, act)
@@ -75,12 +78,48 @@ def test_blocks_match_the_recurrence(heads, vdim, lens, starts, rot, layout, act
     assert off(out, want) < tol and off(call[7][:, 4:], ends) < tol
 
 
-def test_rows_of_no_sequence_and_values_that_are_not_finite():
+# the smallest decay as the host knows it: a whole block's products in range (just so in the last), which is what the other form needs
+@pytest.mark.parametrize("heads,vdim,lens,starts,rot,layout,act", SHAPES)
+def test_blocks_of_known_decays(heads, vdim, lens, starts, rot, layout, act):
+    for decay in ([0.999, 0.5, 0.9][:heads], [seqmix.SCAN_BLOCK_MIN_DECAY * 1.0001] * heads):
+        call, kw, want, ends = inputs(heads, vdim, lens, starts, decay, rot, layout, act)
+        out = ops.recurrent_scan(*call, **kw, min_decay=min(decay))
+        tol = 2e-5 if rot else 2e-6  # as above
+        assert off(out, want) < tol and off(call[7][:, 4:], ends) < tol
+
+
+def test_decays_that_forget_cost_no_more():
+    """Decays that a block's 32 tokens cannot divide by, known or not: as long as others, at most twice the blocks that divide (in
+    blocks as short as they would need, 4 to 25 times)."""
+    heads, t, vdim = 32, 4096, 128
+    g = torch.Generator(device=DEV).manual_seed(2)
+    proj = torch.randn(t, heads * (256 + vdim), generator=g, device=DEV).bfloat16()
+    state, pos = torch.zeros(1, heads * 128 * vdim, device=DEV), torch.arange(t, dtype=torch.int32, device=DEV)
+    pieces = tuple(torch.from_numpy(c).to(DEV) for c in ops.build_scan_pieces([t]))
+    args = (proj, 0, heads * 128, heads * 256, heads, 128, vdim, state, 0, i32([0, t]), i32([0]), pos)
+
+    def time(decay, known):
+        d, best = torch.full((heads,), decay, device=DEV), float("inf")
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ops.recurrent_scan(*args, decay=d, pieces=pieces, min_decay=known)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    usual = time(0.97, 0.97)
+    assert max(time(d, known) for d in (1e-3, 1e-6, 1e-19) for known in (0.0, d)) < 2.5 * usual
+
+
+@pytest.mark.parametrize("known", [0.0, 0.9])
+def test_rows_of_no_sequence_and_values_that_are_not_finite(known):
     call, kw, want, _ = inputs(2, 128, [140, 40], [0, 0], [0.9, 0.99], 0, 0, False, seed=3)
     call[10] = i32([-1, 1])
     call[0][150, call[3]:call[3] + 4] = float("inf")   # token 10 of the second sequence
     before = call[7].clone()
-    out = ops.recurrent_scan(*call, **kw)
+    out = ops.recurrent_scan(*call, **kw, min_decay=known)
     assert (out[:140] == 0).all() and torch.equal(call[7][0], before[0])
     assert off(out[140:150], want[140:150]) < 2e-6     # tokens before it see nothing of it
     assert torch.isfinite(out[140:, 1]).all() and off(out[140:, 1], want[140:, 1]) < 2e-6

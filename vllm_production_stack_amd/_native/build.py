@@ -34,7 +34,7 @@ TARGETS = {
          "kernels/lora.hip", "kernels/gemm.hip", "kernels/rans.hip", "kernels/sampling.hip",
          "kernels/grouped_gemm.hip", "kernels/packed_gemm.hip", "kernels/dense_attention.hip",
          "kernels/tile_gemm.hip", "kernels/latent.hip", "kernels/latent_mfma.hip", "kernels/seqmix.hip",
-         "kernels/chunk_scan.hip", "kernels/mid_gemm.hip", "kernels/block_gemm.hip"],
+         "kernels/chunk_scan.hip", "kernels/retention.hip", "kernels/mid_gemm.hip", "kernels/block_gemm.hip"],
         [],
     ),
     "vpsa_kvio": ("hip", ["kvio/kvio.cpp"], []),

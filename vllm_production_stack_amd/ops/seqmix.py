@@ -98,7 +98,10 @@ def add_dyt_norm(residual, deltas, weight, bias, alpha, out_dtype, want_out: boo
 SCAN_FOLD_MIN_DECAY = 0.1    # decay^-16 stays below 1e16
 SCAN_BLOCK_MIN_ROWS = 8      # rows per sequence of a step without pieces from which blocks (5 us for up to 32 tokens) beat the walk token
                              # by token (about 1.3 us a token)
-# Both measured for the walk token by token; the block form (``_retention_blocks``) joins neighbouring pieces into runs of its own.
+# Fixed decays from which a block's 32 tokens divide by no product below 2^-60; others need shorter blocks, which cost as much each
+# (``csrc/kernels/retention.hip`` has both sides measured).
+SCAN_BLOCK_MIN_DECAY = 2.0 ** (-60 / 31)
+# Both measured for the walk token by token; the block forms join neighbouring pieces into runs of their own.
 SCAN_PIECE_MIN_ROWS = 128   # sequences of a step shorter than this are walked in one go
 SCAN_PIECES_TARGET = 96     # pieces per launch that fill the chip (times heads and column blocks)
 
@@ -123,8 +126,9 @@ def build_scan_pieces(q_lens, target: int = SCAN_PIECES_TARGET):
 
 
 def _retention_blocks(proj, q_col, k_col, v_col, dim, vdim, cos_sin=None, rot_dims=0, layout=0, gates=()) -> bool:
-    """Rows that the block form on the matrix cores (``csrc/kernels/chunk_scan.hip``) takes: bf16, 128 key channels, 128 or 256
-    value channels (its waves hold 32 columns each), 16-byte loads, a rotation whose partners lie in groups of four."""
+    """Rows that the block forms on the matrix cores (``csrc/kernels/chunk_scan.hip``, ``retention.hip``) take: bf16, 128 key
+    channels, 128 or 256 value channels (their waves hold 32 columns each), 16-byte loads, a rotation whose partners lie in groups of
+    four."""
     return (proj.dtype == torch.bfloat16 and dim == 128 and vdim in (128, 256) and rot_dims % 8 == 0 and layout in (0, 1)
             and proj.stride(0) % 8 == 0 and proj.data_ptr() % 16 == 0 and (q_col | k_col | v_col) % 8 == 0
             and (rot_dims == 0 or (cos_sin.data_ptr() % 16 == 0 and cos_sin.is_contiguous()))
@@ -143,9 +147,9 @@ def recurrent_scan(proj, q_col: int, k_col: int, v_col: int, heads: int, dim: in
     ``cos_sin`` over their first ``rot_dims`` channels (``layout`` 0: pairs (i, i + rot_dims / 2), 1: pairs
     (2 i, 2 i + 1)) and k is multiplied by ``k_scale`` afterwards.
 
-    ``min_decay``: the smallest of the decays as the host knows it; from ``SCAN_FOLD_MIN_DECAY`` up the kernel
-    folds the decay into the staged keys and queries of a 16-token block (two operations per state element and
-    token instead of three).
+    ``min_decay``: the smallest of the decays as the host knows it; from ``SCAN_BLOCK_MIN_DECAY`` up the decay is folded into the
+    keys and queries of 32-token blocks on the matrix cores, or, where those do not take the rows, from ``SCAN_FOLD_MIN_DECAY``
+    up into those of 16 tokens on vector arithmetic (two operations per state element and token instead of three).
 
     ``act`` (with ``decay``, no rotation): q, k and v pass through silu first.
 
@@ -171,9 +175,21 @@ def recurrent_scan(proj, q_col: int, k_col: int, v_col: int, heads: int, dim: in
     assert rot_dims <= dim and rot_dims % 2 == 0 and not (act and (gated or rot_dims))
     out = torch.empty((proj.shape[0], heads, vdim), dtype=torch.float32, device=proj.device)
     n_seqs = seq_state.numel()
-    if ((pieces is not None or proj.shape[0] >= SCAN_BLOCK_MIN_ROWS * n_seqs)
-            and _retention_blocks(proj, q_col, k_col, v_col, dim, vdim, cos_sin, 0 if gated else rot_dims, layout,
-                                  (gate_bias, gate_lower) if gated else ())):
+    rot_dims = 0 if gated else rot_dims
+    blocks = _retention_blocks(proj, q_col, k_col, v_col, dim, vdim, cos_sin, rot_dims, layout, (gate_bias, gate_lower) if gated else ())
+    whole_blocks = gated or min_decay >= SCAN_BLOCK_MIN_DECAY
+    if blocks and not whole_blocks and pieces is not None:
+        pc, sp = pieces
+        _i32(pc, sp)
+        assert pc.shape[1] == 3 and sp.numel() == seq_cu.numel()
+        ws_state = torch.empty((pc.shape[0], heads, dim, vdim), dtype=torch.float32, device=proj.device)
+        o._check(o._kernels().vpsa_retention_scan(
+            o._p(proj), c_long(proj.stride(0)), c_int(q_col), c_int(k_col), c_int(v_col), c_int(heads), c_int(vdim),
+            _at(state, state_off), c_long(state.stride(0)), o._p(seq_cu), o._p(seq_state), c_int(n_seqs), o._p(positions),
+            o._p(decay), o._p(cos_sin), c_int(rot_dims), c_int(layout), c_float(k_scale), c_int(1 if act else 0), o._p(out),
+            o._p(pc), o._p(sp), c_int(pc.shape[0]), o._p(ws_state), o._stream()), "retention_scan")
+        return out
+    if blocks and whole_blocks and (pieces is not None or proj.shape[0] >= SCAN_BLOCK_MIN_ROWS * n_seqs):
         pc = sp = ws_state = ws_decay = None
         if pieces is not None:
             pc, sp = pieces
@@ -184,7 +200,7 @@ def recurrent_scan(proj, q_col: int, k_col: int, v_col: int, heads: int, dim: in
         o._check(o._kernels().vpsa_chunk_scan(
             o._p(proj), c_long(proj.stride(0)), c_int(q_col), c_int(k_col), c_int(v_col), c_int(heads), c_int(vdim),
             _at(state, state_off), c_long(state.stride(0)), o._p(seq_cu), o._p(seq_state), c_int(n_seqs), o._p(positions),
-            o._p(decay), o._p(cos_sin), c_int(0 if gated else rot_dims), c_int(layout), c_float(k_scale), c_int(1 if act else 0),
+            o._p(decay), o._p(cos_sin), c_int(rot_dims), c_int(layout), c_float(k_scale), c_int(1 if act else 0),
             o._p(gate_bias), o._p(gate_lower), o._p(out), o._p(pc), o._p(sp), c_int(0 if pc is None else pc.shape[0]),
             o._p(ws_state), o._p(ws_decay), o._stream()), "chunk_scan")
         return out
