@@ -346,7 +346,13 @@ __device__ __forceinline__ void all_products(f32x4* o, const bf16x8 (&pf)[PARTS]
 // `rows` are those of the step's batch bucket, not of the launch: a row's ranges, and with them the order of its sums, are the same
 // in a captured step that is padded to the bucket and in an eager one that is not.
 constexpr int WIDE_ONCE = 4;
-constexpr int TILE_RANGE_PAGES = 4;  // a prefill tile's ranges are no shorter (the launch's count is chosen from the widest table)
+// A prefill tile's ranges are no shorter than this (the launch's count is chosen from the widest table).  A tile of one range finishes its
+// rows itself, and the merge passes over it (300 rows of 32 heads behind a table of 512 pages, two ranges a tile: 44 -> 32 us; 28 uncut).
+constexpr int TILE_RANGE_PAGES = 4;
+__device__ __forceinline__ int tile_ranges(int pos0, int n_tok, int window, int splits) {
+  const int pages = (pos0 + n_tok + PAGE - 1) / PAGE - max(0, pos0 - window + 1) / PAGE;
+  return min(splits, max(1, pages / TILE_RANGE_PAGES));
+}
 __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   int best = 1 << 30, used = splits;
   for (int r = 1; rows * splits > 256; ++r) {
@@ -410,11 +416,12 @@ __global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void late
   const int my_pos = valid ? t.pos0 + tok : -1;
   const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
   const int p_first = max(0, t.pos0 - window + 1) / PAGE;
-  const int used = tiles ? min(splits, max(1, (n_pages - p_first) / TILE_RANGE_PAGES)) : wide_splits(n_pages - p_first, bucket, splits);
+  const int used = tiles ? tile_ranges(t.pos0, t.n_tok, window, splits) : wide_splits(n_pages - p_first, bucket, splits);
+  const bool whole = splits == 1 || (tiles && used == 1);
   const int per = (n_pages - p_first + used - 1) / used;
   const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
   if (splits > 1 && p_begin >= p_end) {  // nothing to see: the merge passes over the record
-    if (tid < t.n_tok * t.hcount) {
+    if (!whole && tid < t.n_tok * t.hcount) {
       const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + tid;
       ws_ml[2 * rec] = -INFINITY;
       ws_ml[2 * rec + 1] = 0.f;
@@ -439,7 +446,7 @@ __global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void late
                                        (__attribute__((address_space(3))) void*)(lds + buf * PAGE_BYTES + (WAVES * i + wave) * 1024),
                                        16, 0, QUARTERS ? 2 : 0);  // 2: non-temporal
   };
-  const bool seeded = splits == 1 && sink != nullptr && valid;
+  const bool seeded = whole && sink != nullptr && valid;
   float m = seeded ? sink[head] * LOG2E : -INFINITY;
   float l = seeded ? 1.f : 0.f;
   f32x4 o[DW];
@@ -597,7 +604,7 @@ __global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void late
   }
 
   if (!valid) return;
-  if (splits == 1) {
+  if (whole) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     uint16_t* dst = out + row * o_row + head * o_head + part * DW * 16 + 4 * g;
 #pragma unroll
@@ -623,12 +630,12 @@ __global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void late
 __global__ __launch_bounds__(128) void latent_merge_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                                                            const int* __restrict__ tiles, int heads,
                                                            const float* __restrict__ sink, uint16_t* __restrict__ out,
-                                                           long o_row, long o_head, int splits, int rank) {
+                                                           long o_row, long o_head, int splits, int rank, int window) {
   const int tile = blockIdx.x, slot = blockIdx.y;
   int row0, n_tok, head0, hcount;
   if (tiles) {
     const int* e = tiles + 6 * tile;
-    if (e[0] < 0) return;
+    if (e[0] < 0 || (window && tile_ranges(e[3], e[2], window, splits) == 1)) return;
     row0 = e[1], n_tok = e[2], head0 = e[4], hcount = e[5];
   } else {
     const int runs = (heads + 63) >> 6;
@@ -703,7 +710,7 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
   }
   if (splits > 1)
     latent_merge_kernel<<<dim3(n_tiles, tiles ? 64 : min(heads, 64)), dim3(128), 0, st>>>(
-        ws_o, ws_ml, tiles, heads, sink, (uint16_t*)out, o_row, o_head, splits, RANK);
+        ws_o, ws_ml, tiles, heads, sink, (uint16_t*)out, o_row, o_head, splits, RANK, !ROT_ONLY && RANK == 512 && ROT == 64 ? window : 0);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -15,6 +15,7 @@ import guzovik_oracle as go
 from vllm_production_stack_amd.engine.config import EngineConfig, guzovik_config, guzovik_layers, resolve_model
 from vllm_production_stack_amd.engine.llm_engine import LLMEngine
 from vllm_production_stack_amd.models.latent_mixer import LatentAttention
+from vllm_production_stack_amd.ops import latent
 
 DEV, DT, TOL = "cpu", "float32", 2e-5
 CPU = torch.device("cpu")
@@ -53,6 +54,20 @@ def test_rotation_of_neighbours_by_hand():
     assert go.visible(4, 2).int().tolist() == [[1, 0, 0, 0], [1, 1, 0, 0], [0, 1, 1, 0], [0, 0, 1, 1]]
     p = go.weights_with_unit_sink(torch.zeros(1, 3, dtype=torch.float64), torch.tensor([[True, True, False]]))
     assert torch.allclose(p, torch.tensor([[1 / 3, 1 / 3, 0.0]], dtype=torch.float64))
+
+
+def test_latent_ranges_follow_the_window():
+    """A tile's keys are cut for the pages that it sees: behind a long context as in a table of the window's pages, and not at all
+    where the list fills the chip."""
+    def cut(tiles, pages, *window):
+        return latent.latent_tile_splits(tiles, pages, 512, 64, True, *window)
+
+    for tiles in (1, 13, 100, 300, 750):
+        for window in (100, 512, 2048):
+            assert cut(tiles, 512, window) == cut(tiles, 4096, window) <= cut(tiles, 512)
+            assert cut(tiles, 5, window) == cut(tiles, min(5, window // 64 + 1 + (window % 64 > 0)))
+    assert cut(200, 512, 2048) == cut(500, 512, 2048) == cut(150, 512, 512) == cut(13, 512, 100) == 1
+    assert cut(300, 512) > 1 and cut(13, 512, 2048) > 1
 
 
 def test_expanded_entries_cover_the_windows():

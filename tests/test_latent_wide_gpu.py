@@ -105,8 +105,8 @@ def test_prefill_tiles(heads):
 
 @pytest.mark.parametrize("heads,rows_of,ctx,window", [
     (16, [20], [3000], 1 << 30), (32, [3, 40], [200, 1500], 1 << 30), (64, [70], [1100], 1 << 30), (16, [9, 1, 130], [9, 513, 700], 1 << 30),
-    (32, [50], [2000], 300), (7, [33], [640], 1 << 30)])
-def test_prefill_tiles_cut_along_the_keys(heads, rows_of, ctx, window):
+    (32, [50], [2000], 300), (7, [33], [640], 1 << 30), (32, [50], [2000], 900), (16, [30, 7], [3000, 60], 1500)])
+def test_prefill_tiles_cut_along_the_keys(heads, rows_of, ctx, window, monkeypatch):
     """Lists of few tiles: ranges of the keys and a merge, tiles that see fewer pages than the list has ranges, an unused entry."""
     pool, table, q, sink = setup(ctx, rows_of, heads, 7 + heads)
     table = torch.nn.functional.pad(table, (0, 60))   # wider than the longest context
@@ -115,6 +115,9 @@ def test_prefill_tiles_cut_along_the_keys(heads, rows_of, ctx, window):
     assert latent.latent_tile_splits(tiles.shape[0], table.shape[1], RANK, ROT, True) > 1
     seq = torch.tensor([i for i, n in enumerate(rows_of) for _ in range(n)], dtype=torch.int32, device=DEV)
     pos = torch.tensor([c - n + k for n, c in zip(rows_of, ctx) for k in range(n)], dtype=torch.int32, device=DEV)
+    asked, cut = [], latent.latent_tile_splits
+    monkeypatch.setattr(latent, "latent_tile_splits", lambda *a: asked.append(a) or cut(*a))
     out = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, seq, pos, sink, 0.05, tiles=tiles, window=window)
     want = expected(pool, table, q, sink, ctx, rows_of, 0.05, window)
     assert float((out.double() - want).norm() / want.norm()) < 6e-3   # as above
+    assert asked == [(tiles.shape[0], table.shape[1], RANK, ROT, True, window)]

@@ -265,21 +265,28 @@ def build_latent_tiles(q_lens, ctx_lens, heads: int):
 
 
 # A work list of fewer tiles than the chip has CUs (one workgroup each) leaves the rest idle while every tile walks its pages alone,
-# and 300 tiles run as one full round and a nearly empty second.  A range costs its pages and, once, about as much as eight (queries,
-# the first page's way, its partial result and the merge's part of it).
-LATENT_RANGE_ONCE = 8
+# and 300 tiles run as one full round and a nearly empty second.  A range costs its pages and, once, as much as about five and a half
+# (queries, the first page's way, its partial result and the merge's part of it); six where the workgroups are more than one round, and
+# eight there if the tiles see different numbers of pages, for the uncut list ends with the short ones.  13 tiles of 9 pages in one /
+# two ranges 40 / 33 us, 100 of 33 114 / 79, 150 of 9 41 / 64, 300 of 33 in one / three 230 / 206; 325 of 11 to 32 in one / two 129 / 164.
+LATENT_RANGE_ALONE, LATENT_RANGE_EVEN, LATENT_RANGE_UNEVEN = 5.5, 6, 8
 LATENT_RANGE_MIN_PAGES = 4
 
 
-def latent_tile_splits(n_tiles: int, pages: int, rank: int, rot: int, latent: bool) -> int:
-    """Key ranges that the tiles of a work list are cut into; ``pages``: the width of the block tables."""
+def latent_tile_splits(n_tiles: int, pages: int, rank: int, rot: int, latent: bool, window: int = NO_WINDOW) -> int:
+    """Key ranges that the tiles of a work list are cut into; ``pages``: the width of the block tables, of which a tile sees those
+    of its last ``window`` entries."""
     if not (latent and (rank, rot) == (512, 64)) or n_tiles == 0:
         return 1
-    best, cost = 1, -(-n_tiles // 256) * (pages + LATENT_RANGE_ONCE // 4)
+    seen = -(-window // PAGE) + 1
+    rounds_once = LATENT_RANGE_EVEN if seen < pages else LATENT_RANGE_UNEVEN
+    pages = min(pages, seen)
+    best, cost = 1, -(-n_tiles // 256) * (pages + 2)
     for e in range(2, min(64, pages // LATENT_RANGE_MIN_PAGES) + 1):
         if n_tiles * e > 1024:
             break
-        c = -(-n_tiles * e // 256) * (-(-pages // e) + LATENT_RANGE_ONCE)
+        rounds = -(-n_tiles * e // 256)
+        c = rounds * (-(-pages // e) + (rounds_once if rounds > 1 else LATENT_RANGE_ALONE))
         if c < cost:
             best, cost = e, c
     return best
@@ -342,7 +349,7 @@ def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, pos
         if tiles is not None:
             assert tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.shape[1] == 6
             n_tiles = tiles.shape[0]
-            splits = latent_tile_splits(n_tiles, block_tables.shape[1], rank, rot, q_lat is not None)
+            splits = latent_tile_splits(n_tiles, block_tables.shape[1], rank, rot, q_lat is not None, window)
         else:
             n_tiles = t * ((heads + LATENT_TILE_SLOTS - 1) // LATENT_TILE_SLOTS)
             bucket *= n_tiles // t
