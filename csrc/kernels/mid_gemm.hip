@@ -21,9 +21,19 @@ constexpr int BN = 128, BK = 64, STAGES = 4, ROWB = BK * 2;
 
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// The chunk a workgroup begins with: the XCDs' an eighth of 64 chunks apart, and within an XCD, whose workgroups' numbers are eight
-// apart, three (with 3 * block an XCD's workgroups met on eight chunks of 64: 28672 x 4096, 1 to 40 rows, 39.5 -> 37.5 us).
-__device__ __forceinline__ int first_chunk(int block, int n) { return ((block >> 3) * 3 + (block & 7) * 8) % n; }
+// The chunk of its n that a workgroup begins with: those of the XCDs an eighth of the row apart, and within an XCD, whose workgroups'
+// numbers are eight apart, three.  With 3 * block an XCD's workgroups meet on the eighths of a row of 64 chunks (28672 x 4096, 1 to
+// 40 rows, 39.3 -> 38.5 us), all of them on one chunk of a range of eight (4096 x 4096 in eight ranges, 1 / 64 rows 10.3 -> 10.0 / 14.4 -> 13.8),
+// and beyond 48 rows ranges are far slower (8192 x 28672, 128 rows 135 -> 109; 3584 x 18944 49.3 -> 40.3).  But it stays where it is the
+// better one.  `whole`: unsplit products with rows of 128 chunks and more, where it spreads an XCD over all of the row (28672 x 8192,
+// 8 / 64 rows 74 / 77 against 83 / 84), or of more than a round of workgroups, which get out of step by themselves (57344 x 8192 145 / 149
+// against 166 / 176; 128256 x 4096, 96 rows 195 against 200).  And ranges of fewer than 16 chunks that have no whole eighths (2560 x 9728 in
+// twelve, 128 rows 22.8 against 23.4).
+__host__ __device__ __forceinline__ int first_chunk(int block, int n, bool whole) {
+  const int eighth = n / 8;
+  if (whole || (n < 16 && (n & 7))) return block * 3 % n;
+  return ((block >> 3) * 3 + (block & 7) * (eighth - (eighth % 3 == 0))) % n;  // (threes and a multiple of three would meet)
+}
 
 // acc[i][t] += W tile i of the wave x token tile t over chunks [0, n) of both operands: NA * 64 weight rows and MT * 16 token rows a
 // chunk, all of it in LDS stages.  The weight rows lie w_row bytes apart from wp on, those from the 64th on w_half further; xrow(r): bytes
@@ -140,7 +150,7 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
       reinterpret_cast<const char*>(w + (long)n0 * K) + (long)c0 * ROWB, (uint32_t)(K * 2), (PAIR ? n_out : 64) * (long)(K * 2),
       reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB,
       [&](int r) { return (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)); },  // rows past the last repeat it
-      n, n > 0 ? first_chunk(blockIdx.x, n) : 0, lds, arow, acc);
+      n, n > 0 ? first_chunk(blockIdx.x, n, S == 1 && (n >= 128 || gridDim.x > 256)) : 0, lds, arow, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int j = 16 * t + c16;
@@ -204,7 +214,7 @@ __global__ __launch_bounds__(256, 1) void mid_experts_kernel(const uint16_t* __r
         reinterpret_cast<const char*>(w + ((long)e * N + n0) * K), (uint32_t)(K * 2), n_out * (long)(K * 2),
         reinterpret_cast<const char*>(UNIT ? x : x + (long)(r0 + m0) * K),
         [&](int r) { return (uint32_t)(UNIT ? sorted_tok[r0 + m0 + min(r, last)] : min(r, last)) * (uint32_t)(K * 2); },
-        n, (first_chunk(blockIdx.x, n) + e) % n, lds, arow, acc);
+        n, (first_chunk(blockIdx.x, n, false) + e) % n, lds, arow, acc);
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const int j = 16 * t + c16;
@@ -546,3 +556,6 @@ VPSA_EXPORT int vpsa_mid_gemm_qkv(const void* x, long xs, const void* w, const v
       n_q, n_kv, S);
   return 0;
 }
+
+// Where a workgroup of a product begins (tests).
+VPSA_EXPORT int vpsa_mid_first_chunk(int block, int n, int whole) { return n > 0 ? first_chunk(block, n, whole != 0) : -1; }

@@ -1,0 +1,26 @@
+"""Rules of the native kernels that the host can be asked for: no GPU takes part."""
+
+from ctypes import c_int
+
+import pytest
+
+from vllm_production_stack_amd import ops
+
+
+# chunks of a product's reduction or of one of its ranges: rows of 4096, 3584, 2048, 3072, 6144 and ranges of eight and more chunks
+@pytest.mark.parametrize("n", [8, 16, 24, 28, 32, 40, 48, 56, 64, 72, 96, 112, 120])
+def test_workgroups_of_a_projection_begin_apart(n):
+    def first(block):
+        return ops._kernels().vpsa_mid_first_chunk(c_int(block), c_int(n), c_int(0))
+
+    assert all(0 <= first(b) < n for b in range(512))
+    assert len({first(b) for b in range(8)}) == 8                        # the XCDs (workgroups go round them)
+    for xcd in range(8):                                                 # an XCD's, as many as there are CUs
+        assert len({first(b) for b in range(xcd, 256, 8)}) >= min(32, n // (3 if n % 3 == 0 else 1))
+    assert len({first(b) for b in range(256)}) >= 0.8 * n                # no part of the row that nobody begins with
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 12, 13, 64, 128, 152, 224])
+def test_workgroups_of_whole_products_begin_apart(n):
+    starts = [ops._kernels().vpsa_mid_first_chunk(c_int(b), c_int(n), c_int(1)) for b in range(512)]
+    assert all(0 <= s < n for s in starts) and len(set(starts)) >= n // (3 if n % 3 == 0 else 1)

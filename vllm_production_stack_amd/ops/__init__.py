@@ -42,7 +42,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_chunk_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_block_gemm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_chunk_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_first_chunk", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_block_gemm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -691,16 +691,17 @@ def _stream_gemm(x2, w, bias, pair):
 
 # ``mid_gemm`` (128 weight rows a workgroup, both operands straight into LDS) against what ran before, microseconds in a graph over
 # weights that no cache holds (library with its activation pass, or the kernels above up to 16 rows / mid_gemm):
-#   28672 x 4096 pair    1 row 43.6/37.5    24 rows 50.4/37.6    64 rows 57.2/40.1    112 rows 59.2/49     128 rows 59.3/51
-#   4096 x 14336         1     25.1/21.4    24      29.0/23.1    64      39.2/28.1    128      75.7/37.9    200      56.7/50.1
-#   6144 x 4096          1     12.9/12.0    24      14.4/13.6    64      17.5/16.6    112      24.1/22.0    200      25.9/30.5
-#   4096 x 4096          1      9.8/10.0    24      13.1/11.4    64      14.9/13.9     97      16.4/17.0
-#   128256 x 4096        1      190/162     24       198/167     64       214/191     112       236/218     128       239/228
-#   57344 x 8192 pair    1      172/146     64       194/161     112      203/190     128       199/197     160       210/383
-#   8192 x 28672         1       90/76      64       147/105     128      203/116     200       312/165
-#   3584 x 18944         1       46/25      24       108/26      200      121/66
-#   37888 x 3584 pair    1     48.4/53.6    64      64.9/65.7  (296 workgroups: a second round nearly empty)
-#   2048 x 2048          1      5.7/7.2     64       8.7/9.9   (64 workgroups)
+#   28672 x 4096 pair    1 row 43.6/36.6    24 rows 51.1/36.6    64 rows 51.7/38.5    112 rows 56.8/48.2    128 rows 56.3/50.7
+#   4096 x 14336         1     25.1/22.4    24      27.5/23.7    64      38.6/27.9    128      71.2/35.7    200      54.1/48.2
+#   6144 x 4096          1     12.9/12.5    24      15.1/14.2    64      18.3/17.0    112      23.9/20.6    200      26.1/30.6
+#   4096 x 4096          1      9.8/9.7     24      13.4/11.5    64      15.2/13.4     97      16.3/16.4
+#   128256 x 4096        1      190/160     24       196/164     64       208/183     112       232/213     128       233/224
+#   57344 x 8192 pair    1      172/146     64       194/150     112      200/178     128       203/186     160       208/364
+#   28672 x 8192 pair    1      113/72      64       101/72      112      111/89      128       112/93      160       121/185
+#   8192 x 28672         1       86/71      64       140/89      128      201/112     200      307/172
+#   3584 x 18944         1       46/26      24       107/27      64        90/32      128       99/40       200      122/61
+#   37888 x 3584 pair    1     48.4/54.1    64      64.8/64.8  (296 workgroups: a second round nearly empty)
+#   2048 x 2048          1      5.7/7.4     64       8.7/10.6  (64 workgroups)
 MID_MIN_FILL = 0.75      # of the rounds of one workgroup per CU
 MID_ROWS = 96            # every shape that fills the chip
 MID_ROWS_BLOCK = 128     # one round or full ones (448 workgroups win by 2 to 6 %), and partial sums (32 bits, written and read) below
