@@ -1,6 +1,6 @@
 """Rules of the native kernels that the host can be asked for: no GPU takes part."""
 
-from ctypes import c_int
+from ctypes import c_int, c_long
 
 import pytest
 
@@ -24,3 +24,12 @@ def test_workgroups_of_a_projection_begin_apart(n):
 def test_workgroups_of_whole_products_begin_apart(n):
     starts = [ops._kernels().vpsa_mid_first_chunk(c_int(b), c_int(n), c_int(1)) for b in range(512)]
     assert all(0 <= s < n for s in starts) and len(set(starts)) >= n // (3 if n % 3 == 0 else 1)
+
+
+def test_threads_that_share_a_copy():
+    """A copy has a thread for every whole MB, up to four: starting one costs more than copying less."""
+    def parts(size):
+        return ops._kernels().vpsa_copy_parts(c_long(size))
+
+    assert [parts(n) for n in (0, 1, 51 << 10, 1 << 20, (2 << 20) - 1)] == [1] * 5
+    assert [parts(n) for n in (2 << 20, 3 << 20, 4 << 20, 7 << 20, 1 << 40)] == [2, 3, 4, 4, 4]
