@@ -18,7 +18,8 @@
 // The router's product, logits[t, e] = x[t] . w[e] rounded to bf16, for up to 64 experts: a workgroup takes 16 tokens, its waves quarters of
 // the reduction (a token's row is read once, 64 bytes of 16 rows an instruction, 16 on their way), and their sums meet in LDS.  What
 // bounds it is the way of the rows to too few CUs; the library's tile of 16 x 16 walks the whole reduction with one wave: 1531 tokens of
-// 4096 channels, 8 experts 16.6 -> 10.7 us (the loads one at a time, as the compiler puts them by itself: 15).
+// 4096 channels, 8 experts 16.6 -> 10.7 us in a step (the loads one at a time, as the compiler puts them by itself: 15).  ops.moe_router_takes
+// has the sizes where it is the better choice.
 template <int ET>
 __global__ __launch_bounds__(256) void moe_router_kernel(const uint16_t* __restrict__ x, long x_stride, const uint16_t* __restrict__ w,
                                                          uint16_t* __restrict__ logits, int tokens, int n_experts, int hidden) {

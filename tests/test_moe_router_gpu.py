@@ -12,7 +12,9 @@ BF = torch.bfloat16
 
 @pytest.mark.parametrize("tokens", [1, 15, 16, 17, 1531])
 @pytest.mark.parametrize("experts,hidden", [(1, 128), (8, 4096), (16, 256), (17, 1152), (33, 640), (64, 2048)])
-def test_router(tokens, experts, hidden):
+def test_router(tokens, experts, hidden, monkeypatch):
+    monkeypatch.setattr(ops, "MOE_ROUTER_WEIGHTS", 1 << 30)  # (where the library is the better choice as well)
+    monkeypatch.setattr(ops, "MOE_ROUTER_TOKENS", 1 << 30)
     torch.manual_seed(tokens + experts)
     x = torch.randn(tokens, hidden + 8, device="cuda").to(BF)[:, :hidden]
     w = (torch.randn(experts, hidden, device="cuda") * hidden ** -0.5).to(BF)

@@ -1260,11 +1260,31 @@ def page_decode(src: int, pinned, size: int, n: int, n_ctx: int, unit_elems: int
 
 
 # --------------------------------------------------------------------------- MoE routing
+# A router's product of ``csrc/kernels/moe.hip`` beside the library's, microseconds in a graph (library / kernel), which reads 16 rows of
+# weights and activations an instruction and has a workgroup for 16 tokens: short rows and few experts are its side, and one round.
+#   8 experts of 4096    8 tokens 7.9/6.2    300 tokens 8.1/7.7    4096 tokens 12.0/8.6    6000 tokens 11.6/14.6
+#   8 of 6144            8        6.9/8.4    300        7.1/10.6
+#   16 of 2048           8        5.3/4.7    300        5.7/5.6    4096         5.9/6.1
+#   16 of 4096           8        7.8/7.5    300        8.1/9.0
+#   32 of 1024           8        4.7/4.4    300        5.5/5.0    6000         5.7/7.8
+#   32 of 4096           8        7.4/11.0   300        7.5/12.6
+#   64 of 512            8        4.0/4.0    300        4.5/3.9
+#   64 of 2048           8        5.6/10.4   300        5.6/11.3
+MOE_ROUTER_WEIGHTS = 32768  # elements, experts rounded up to 8, 16, 32 or 64
+MOE_ROUTER_TOKENS = 4096
+
+
+def moe_router_takes(tokens: int, experts: int, hidden: int) -> bool:
+    """Does a router's product run in the framework's kernel?"""
+    return (0 < experts <= 64 and hidden % 128 == 0 and tokens <= MOE_ROUTER_TOKENS
+            and hidden * (1 << (max(experts, 8) - 1).bit_length()) <= MOE_ROUTER_WEIGHTS)
+
+
 def moe_router(x, w):
-    """A mixture's router product ``x @ w.T`` (``csrc/kernels/moe.hip`` for up to 64 experts, else the library)."""
+    """A mixture's router product ``x @ w.T`` (``csrc/kernels/moe.hip`` where ``moe_router_takes`` it, else the library)."""
     if (x.is_cuda and x.dim() == 2 and w.device == x.device and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous()
-            and 0 < w.shape[0] <= 64 and x.shape[1] == w.shape[1] and x.shape[1] % 128 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0 and not _followed(x, w)):
+            and w.dim() == 2 and x.shape[1] == w.shape[1] and moe_router_takes(x.shape[0], w.shape[0], w.shape[1]) and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and not _followed(x, w)):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
         _check(_kernels().vpsa_moe_router(_p(x), c_long(x.stride(0)), _p(w), _p(out), c_int(x.shape[0]), c_int(w.shape[0]),
                                           c_int(x.shape[1]), _stream()), "moe_router")
