@@ -101,3 +101,17 @@ def test_fused_encoder_against_the_general_one(model, windows, frames, monkeypat
     general = m.encode(mel)
     err, base = ((v.double() - want.double()).norm() / want.double().norm() for v in (got, general))
     assert got.shape == want.shape and err <= 1.2 * base + 1e-3, (err, base)  # fewer roundings to 16 bits than the general form
+
+
+@pytest.mark.parametrize("b,t", [(1, 151), (2, 1), (3, 389), (1, 750)])
+def test_heads_of_other_widths_on_the_general_path(b, t):
+    """16 channels a head (no kernel has them): one window, one position, odd lengths."""
+    from vllm_production_stack_amd.models import whisper
+
+    q, k, v = (_rand(b, t, 64) for _ in range(3))
+    got = whisper._attend(q, k, v, 4).double()
+    qh, kh, vh = (x.double().cpu().view(b, t, 4, 16).transpose(1, 2) for x in (q, k, v))
+    p = torch.softmax(qh @ kh.transpose(-1, -2) * 0.25, dim=-1)
+    want, size = ((p @ x).transpose(1, 2).reshape(b, t, 64).cuda() for x in (vh, vh.abs()))
+    # scores (up to about 6), probabilities and the result are rounded to 16 bits once each
+    assert bool(((got - want).abs() <= (2 ** -9 + 6 * 2 ** -8) * size + want.abs() * 2 ** -8).all())

@@ -76,6 +76,19 @@ def test_greedy_matches_dense(model):
         ids.append(tok)
 
 
+@pytest.mark.parametrize("t", [1, 7, 16])
+def test_small_mixture_batches_multiply_no_transposed_view(t, monkeypatch):
+    """All experts on all rows: batched products in 16 bits take right operands whose rows are contiguous (others can fault a GPU)."""
+    model = make_engine("tiny-mixtral").runner.model
+    lw, x = model.layers[0], torch.randn(t, model.cfg.hidden_size, generator=torch.Generator().manual_seed(t))
+    seen, product = [], torch.matmul
+    monkeypatch.setattr(torch, "matmul", lambda a, b: seen.append(b) or product(a, b))
+    got = model._moe(x, lw, True)
+    assert len(seen) == 2 and all(b.is_contiguous() and b.stride(-1) == 1 for b in seen) and got.is_contiguous()
+    w, ids = ref.moe_topk_softmax(torch.nn.functional.linear(x, lw.router), model.cfg.num_experts_per_tok, True)
+    assert torch.allclose(got, ref.moe_experts(x, lw.w13, lw.w2, ids, w), atol=1e-5)
+
+
 def test_chunked_prefill_equals_whole_prompt():
     g = torch.Generator().manual_seed(1)
     prompt = torch.randint(16, 500, (300,), generator=g).tolist()

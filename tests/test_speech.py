@@ -158,6 +158,21 @@ def test_width3_convolutions_as_gemms_match_conv1d():
         assert (got - want).abs().max().item() < 1e-4
 
 
+@pytest.mark.parametrize("b,tq,tk", [(1, 151, 151), (2, 1, 1), (3, 5, 388), (1, 4, 1500)])
+def test_general_attention_multiplies_no_transposed_view(b, tq, tk, monkeypatch):
+    """Batched products in 16 bits take right operands whose rows are contiguous (others can fault a GPU), one window or one position
+    among them, where the heads of a view fold into the batch without a copy."""
+    g = torch.Generator().manual_seed(b * tq)
+    q, k, v = (torch.randn(b, n, 64, generator=g) for n in (tq, tk, tk))
+    seen, product = [], torch.matmul
+    monkeypatch.setattr(torch, "matmul", lambda x, y: seen.append(y) or product(x, y))
+    got = W._attend(q, k, v, 4)
+    assert len(seen) == 2 and all(y.stride(-1) == 1 for y in seen) and seen[0].is_contiguous()
+    heads = [t.view(b, -1, 4, 16).transpose(1, 2) for t in (q, k, v)]
+    want = torch.nn.functional.scaled_dot_product_attention(*heads).transpose(1, 2).reshape(b, tq, 64)
+    assert torch.allclose(got, want, atol=1e-5)
+
+
 def test_graph_decode_step_reproduces_the_eager_loop(hf_checkpoint):
     """The static-buffer decode step the GPU captures as a graph (token, position and finished
     flags on the device, history read back at the end), replayed here without a capture: same

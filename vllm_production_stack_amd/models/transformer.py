@@ -239,10 +239,12 @@ class TransformerModel:
             # sync) and mix with the routing matrix.
             dense = torch.zeros((t, e), dtype=torch.float32, device=x.device)
             dense.scatter_add_(1, ids.long(), w)
-            gu = torch.matmul(x.unsqueeze(0), lw.w13.transpose(1, 2))  # [E, T, 2I]
-            act = ops.silu_and_mul(gu.view(e * t, -1)).view(e, t, -1)
-            y = torch.matmul(act, lw.w2.transpose(1, 2))  # [E, T, H]
-            return (y.float() * dense.t().unsqueeze(-1)).sum(0).to(x.dtype)
+            # (weights on the left, right operands copied: a batched bf16 product whose right operand is a transposed view can
+            # fault the GPU; contiguous() leaves a single row's view as it is)
+            gu = torch.matmul(lw.w13, x.t().clone(memory_format=torch.contiguous_format)).transpose(1, 2)  # [E, T, 2I]
+            act = ops.silu_and_mul(gu.reshape(e * t, -1)).view(e, t, -1)
+            y = torch.matmul(lw.w2, act.transpose(1, 2).clone(memory_format=torch.contiguous_format))  # [E, H, T]
+            return (y.float() * dense.t().unsqueeze(1)).sum(0).t().to(x.dtype).contiguous()
         if tiled:
             # Prefill chunks of any size: two grouped matrix-core GEMMs over the device-sorted
             # (token, expert) pairs (gate_up gathers its rows and fuses SwiGLU).  The host never reads

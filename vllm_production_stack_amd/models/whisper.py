@@ -224,9 +224,11 @@ def _attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int,
     if mask is None and hd == 64 and ops.dense_attention_supported(q, k, v, heads):
         return ops.dense_attention(q, k, v, heads)  # bf16 on the GPU: MFMA flash kernel
     qh = (q * (hd ** -0.5)).view(b, tq, heads, hd).transpose(1, 2)
-    kh = k.view(b, tk, heads, hd).transpose(1, 2)
+    # (a copy: a batched bf16 product whose right operand is a transposed view can fault the GPU; contiguous() leaves a single
+    # position's view as it is)
+    kt = k.view(b, tk, heads, hd).permute(0, 2, 3, 1).clone(memory_format=torch.contiguous_format)
     vh = v.view(b, tk, heads, hd).transpose(1, 2)
-    s = torch.matmul(qh, kh.transpose(-1, -2))
+    s = torch.matmul(qh, kt)
     if mask is not None:
         s = s + mask.to(s.dtype)
     p = torch.softmax(s, dim=-1)
