@@ -12,6 +12,7 @@ import aiohttp
 import numpy as np
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from vllm_production_stack_amd.engine import audio
 from vllm_production_stack_amd.engine.config import EngineConfig
@@ -156,6 +157,31 @@ def test_width3_convolutions_as_gemms_match_conv1d():
         got = m._conv3(x.transpose(1, 2), "c", stride)
         assert got.shape == want.shape
         assert (got - want).abs().max().item() < 1e-4
+
+
+class _BatchedProducts(TorchDispatchMode):
+    """Right operands of the batched products that reach the library."""
+
+    def __init__(self):
+        super().__init__()
+        self.right = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if func in (torch.ops.aten.bmm.default, torch.ops.aten.baddbmm.default):
+            self.right.append(args[-1])
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("b,frames", [(1, 301), (2, 60), (3, 2)])
+def test_encoder_multiplies_no_transposed_view(b, frames):
+    """The encoder of heads that no kernel covers: its convolutions and projections as plain products, attention with right operands
+    whose rows are contiguous (a batched 16-bit product of a transposed view can fault a GPU)."""
+    m = W.WhisperModel(W.WHISPER_PRESETS["tiny-whisper"], torch.bfloat16, torch.device("cpu"))
+    m.init_random(1)
+    with torch.no_grad(), _BatchedProducts() as products:
+        out = W.WhisperModel.encode.__wrapped__(m, torch.randn(b, m.cfg.num_mel_bins, frames))
+    assert out.shape == (b, (frames + 1) // 2, 64) and len(products.right) == 2 * m.cfg.encoder_layers
+    assert all(r.stride(-1) == 1 for r in products.right)
 
 
 @pytest.mark.parametrize("b,tq,tk", [(1, 151, 151), (2, 1, 1), (3, 5, 388), (1, 4, 1500)])

@@ -361,7 +361,9 @@ class WhisperModel:
         t_out = (t - 1) // stride + 1
         xp = F.pad(x, (0, 0, 1, 1))
         cols = xp.as_strided((b, t_out, 3 * ci), ((t + 2) * ci, stride * ci, 1))
-        return F.linear(cols, w2[1], self.w[prefix + ".bias"])
+        # (as rows of one product: over batches of overlapping rows F.linear is a batched one with the weight as a transposed view,
+        # which can fault the GPU in 16 bits)
+        return F.linear(cols.contiguous().view(b * t_out, 3 * ci), w2[1], self.w[prefix + ".bias"]).view(b, t_out, -1)
 
     def _conv_rows(self, prefix: str) -> torch.Tensor:
         """A convolution's kernel as the weight of ``_conv3``'s product, its rows filled up with zeros to a multiple of 64."""
