@@ -1608,7 +1608,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       const float l_tot = l_run[rb] + __shfl_xor(l_run[rb], 32, 64);
-      if (!row_ok[rb] || !head_ok) continue;
+      if (!row_ok[rb]) continue;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll

@@ -363,17 +363,18 @@ __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   return used;
 }
 
-// SHARE: waves that share 16 slots, each of which scores its part of a page's keys and sums its part of the channels (1: none).
+// SHARE: waves that share 16 slots, each of which scores its part of a page's keys and sums its part of the channels.
 template <int RANK, int ROT, int SHARE>
-__global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void latent_wide_kernel(
+__global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
     long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
     int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
     const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
     int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
   constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, DT = RANK / 16, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW;
+  static_assert(SHARE == 2 || SHARE == 4, "eight waves for four or two groups of 16 slots");
   constexpr bool QUARTERS = SHARE == 4;
-  constexpr int WAVES = SHARE > 1 ? 8 : 4;
+  constexpr int WAVES = 8;
   constexpr int NI = PAGE_BYTES / (1024 * WAVES);  // KiB of a page that a wave loads
   constexpr int NT = 4 / SHARE;                    // 16-key tiles of a page that a wave scores
   constexpr int DW = DT / SHARE;                   // 16-channel tiles that it sums
@@ -570,22 +571,16 @@ __global__ __launch_bounds__(SHARE > 1 ? 512 : 256, SHARE > 1 ? 2 : 1) void late
         multiply_tiles(o, v1, pf);
       }
     } else {
-      if constexpr (SHARE > 1) {
-        f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;
-        if (wave_active) {
-          score(buf);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) round[(NT * part + nt) * 64] = s[nt];
-        }
-        everyone();
-        if (wave_active) {
-#pragma unroll
-          for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
-        }
-      } else if (wave_active) {
-        score(buf);
-      }
+      f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;
       if (wave_active) {
+        score(buf);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) round[(NT * part + nt) * 64] = s[nt];
+      }
+      everyone();
+      if (wave_active) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
         weigh(p);
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
