@@ -474,10 +474,10 @@ VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
 }
 
 // A host copy of some MB in pieces, each on a thread of its own where one can be had: a page comes out of memory, not of a cache.  The
-// threads end with the object.  A piece is no smaller than a MB: a thread takes 15 to 20 us to start and end.  A page to a bytes object / back
-// on the device, one thread / four / pieces of a MB: 51 KB coded 115 / 183 / 124 us and 68 / 152 / 77, 1.2 MB 229 / 251 / 232 and 184 / 219 / 187, 2.8 MB
-// 332 / 375 / 294 and 305 / 298 / 294, 7 MB 606 / 528 / 490 and 546 / 450 / 448.
-constexpr long COPY_PART = 1 << 20;
+// threads end with the object.  A piece is no smaller than 768 KB: a thread takes 15 to 20 us to start and end.  A page to a bytes object / back
+// on the device, one thread / four: 51 KB coded 115 / 183 us and 68 / 152, 1.2 MB 229 / 251 and 184 / 219, 7 MB 606 / 528 and 546 / 450; four pages of
+// 3.4 MB out in one, three, four pieces 1600 / 1505 / 1355, twelve back 1800 / 1675 / 1720.
+constexpr long COPY_PART = 768 << 10;
 class HostCopies {
  public:
   ~HostCopies() {
