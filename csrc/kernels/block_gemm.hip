@@ -10,8 +10,9 @@
 //   * The weight rows are the MFMA's A operand and are ordered so that a lane ends with eight consecutive columns of a token row.
 // What bounds it: LDS, which carries (reads and the loads' writes) 128 bytes for every 64 x 96 x 96 of products in the largest shape, as many
 // cycles as the matrix cores need; with short reductions the time until a tile's first chunk is there and its epilogue (gelu 75
-// cycles of vector work a wave and value).  12000 rows, library with the activation's pass / this: 3072 x 768 with gelu 107 / 70 us,
-// 768 x 3072 57 / 48 (+ residual), three of 768 x 768 62 / 48, 768 x 2304 with gelu 50 / 42; 1500 rows, 2048 x 512 with gelu 26 / 11.
+// cycles of vector work a wave and value).  12000 rows in a loop over the same operands, library with the activation's pass / this: 3072 x
+// 768 with gelu 107 / 70 us, 768 x 3072 57 / 48 (+ residual), three of 768 x 768 62 / 48, 768 x 2304 with gelu 50 / 42; 1500 rows, 2048 x 512 with
+// gelu 26 / 11.  In an encoder of 12 layers, where a product's operands come from memory, the first three take 82 to 86, 56 to 58 and 55 to 58.
 #include <type_traits>
 
 #include "common.h"

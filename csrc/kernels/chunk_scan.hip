@@ -11,8 +11,8 @@
 // 32-bit matrix instructions 1.7e-7 to 3.0e-7; gated, whose 1 - a comes from the exponential: 0.9e-7, token by token 1.2e-7.
 //   * What bounds it: vector work (a block costs a wave 1000 instructions, half of them to cut the state up, and a SIMD's two waves
 //     2 x 166 matrix instructions) and the barriers between staging, scores and products; HBM has a third of its traffic.
-//   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1564 / 297 us,
-//     fixed 128 x 256 701 / 385; 1000 rows: gated (16 heads, three sequences) 229 / 55, fixed (one) 154 / 84; 200 rows of two 199 / 37.
+//   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1559 / 291 us,
+//     fixed 128 x 256, rotated, 702 / 347; 1000 rows: gated (16 heads, three sequences) 229 / 55, fixed (one) 154 / 84; 200 rows of two 199 / 37.
 //   * 1 / R must stay in range: a block in which some |R| leaves 2^-60 .. 2^60 is taken again with half its tokens (a block of one token
 //     divides by nothing); fixed decays know their longest block beforehand, and those that need shorter ones go to retention.hip.
 //   * A workgroup holds a head's whole 128 x VD state in accumulators, 32 columns a wave, so q, k and the scores are made once for all
@@ -719,8 +719,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
         }
       }
     }
-    // a tile's operands are read while the tile before is multiplied (left alone the compiler waits for every read by itself: with the
-    // positions as scalars, 309 -> 297 us gated, 396 -> 385 fixed)
+    // a tile's operands are read while the tile before is multiplied (left alone the compiler waits for every read by itself; with the
+    // positions as scalars, 4 % gated, 3 % fixed)
     bf16x8 kf[2][3];
     auto read_k = [&](int t) {
 #pragma unroll
