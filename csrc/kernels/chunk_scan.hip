@@ -8,10 +8,11 @@
 // it comes (three behind silu), and products of parts down to 2^-24 of the largest go through v_mfma_f32_16x16x32_bf16 (three instructions
 // for k^ v and the scores' product with v, six for S'^T q^ and the scores; sums in 32 bits, those of the small products apart).  A 32-bit
 // instruction does a sixteenth of that work per cycle.  Error against 64 bits, fixed decay: 1.1e-7 (64 rows) to 1.7e-7 (8192 rows), on
-// 32-bit matrix instructions 1.7e-7 to 3.0e-7; gated, whose 1 - a comes from the exponential: 0.9e-7, token by token 1.2e-7.
+// 32-bit matrix instructions 1.7e-7 to 3.0e-7; gated, whose 1 - a comes from the exponential: 0.9e-7, token by token in seqmix.hip 1.2e-7; gates
+// around a half 0.7e-7 against 0.5e-7, gates that forget (token by token here as well) 0.5e-7 both.
 //   * What bounds it: vector work (a block costs a wave 1000 instructions, half of them to cut the state up, and a SIMD's two waves
 //     2 x 166 matrix instructions) and the barriers between staging, scores and products; HBM has a third of its traffic.
-//   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1559 / 291 us,
+//   * Measured, token by token or on 32-bit matrix instructions / here: 8192 rows of two sequences, 32 heads: gated 128 x 128 1559 / 296 us,
 //     fixed 128 x 256, rotated, 702 / 347; 1000 rows: gated (16 heads, three sequences) 229 / 55, fixed (one) 154 / 84; 200 rows of two 199 / 37.
 //   * 1 / R must stay in range: a block in which some |R| leaves 2^-60 .. 2^60 is taken again with half its tokens (a block of one token
 //     divides by nothing); fixed decays know their longest block beforehand, and those that need shorter ones go to retention.hip.
@@ -26,8 +27,8 @@
 // Gates that forget too fast for blocks of more than eight tokens (a quarter and less a token, or now and then all at once) take the
 // rest of their run token by token as well, 16 tokens in 32 bits in LDS at a time: 1.8 us a token of both phases with two workgroups a
 // CU, where blocks of eight cost 16, and of one the same.  8192 rows, 32 heads, 128 x 128, in blocks down to one token / so, by the mean
-// logit behind a lower bound of 0: 0 546 / 518, -2 1064 / 927, -6 2095 / 963, -14 4146 / 979, -40 8252 / 976; token by token out of memory 1559.
-// 200 rows 64 / 67, 111 / 117, 199 / 121, 371 / 121, 712 / 121; 206.  The loop stands behind the blocks' and not inside: shared by turns, its
+// logit behind a lower bound of 0: 0 546 / 527, -2 1064 / 942, -6 2095 / 979, -14 4146 / 994, -40 8252 / 994; token by token out of memory 1559.
+// 200 rows 64 / 69, 111 / 119, 199 / 123, 371 / 123, 712 / 123; 206.  The loop stands behind the blocks' and not inside: shared by turns, its
 // registers and theirs spilled (302 -> 338 where no gate forgets).
 // Pieces: the step's list is walked in runs of `group` pieces of one sequence.  Phase 1 makes the runs' end states from zero,
 // chain_kernel turns them into start states, phase 2 computes the outputs; phase 0 walks whole sequences from slot to slot.
@@ -51,18 +52,22 @@ __device__ __forceinline__ float reciprocal(float x) {
   const float r = __builtin_amdgcn_rcpf(x);
   return fmaf(fmaf(-x, r, 1.f), r, r);
 }
-// sigmoid(x) and sigmoid(-x) from t = exp(-|x|): 1 / (1 + t) and t / (1 + t).  exp(y) = 2^h (1 + e ln 2) with h + e = y / ln 2, h rounded.
-__device__ __forceinline__ void sigmoids(float x, float* s, float* rest) {
+// exp(-|x|) = 2^h (1 + e ln 2) with h + e = -|x| / ln 2, h rounded.
+__device__ __forceinline__ float exp_minus(float x) {
   const float y = -fabsf(x), h = y * 1.44269504f, e = fmaf(y, 1.44269504f, -h) + y * 1.92596299e-8f;
-  const float t2 = __builtin_amdgcn_exp2f(h), t = h < -200.f ? 0.f : fmaf(t2, e * 0.693147181f, t2);
-  const float r = reciprocal(1.f + t);
+  const float t2 = __builtin_amdgcn_exp2f(h);
+  return h < -200.f ? 0.f : fmaf(t2, e * 0.693147181f, t2);
+}
+// sigmoid(x) and sigmoid(-x) from t = exp(-|x|): 1 / (1 + t) and t / (1 + t).  The Newton step takes 1 - r (1 + t) without rounding 1 + t
+// (1 - r is exact), so that a quotient has its own rounding and little else.
+__device__ __forceinline__ void sigmoids(float x, float* s, float* rest) {
+  const float t = exp_minus(x), r0 = __builtin_amdgcn_rcpf(1.f + t), r = fmaf(fmaf(-t, r0, 1.f - r0), r0, r0);
   *s = x >= 0.f ? r : t * r;
   *rest = x >= 0.f ? t * r : r;
 }
 __device__ __forceinline__ float silu(float x) {
-  float s, rest;
-  sigmoids(x, &s, &rest);
-  return x * s;
+  const float t = exp_minus(x), r = __builtin_amdgcn_rcpf(1.f + t), n = x >= 0.f ? x : x * t, q = n * r;
+  return fabsf(q) < __builtin_inff() ? fmaf(fmaf(-t, q, n - q), r, q) : q;  // (n - q is exact: n / 2 <= q <= n)
 }
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
 
@@ -380,9 +385,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
           most = fmaxf(most, fabsf(Rr));
           k[u][i] *= Rr;
           if (PHASE != 1) {
-            float x = i & 1 ? bf16hi(rq[u][i >> 1]) : bf16lo(rq[u][i >> 1]), s, rest;
-            sigmoids(x, &s, &rest);
-            q[i] = x * s * reciprocal(Rr);
+            q[i] = silu(i & 1 ? bf16hi(rq[u][i >> 1]) : bf16lo(rq[u][i >> 1])) * reciprocal(Rr);
             most = fmaxf(most, fabsf(q[i]) * 1e-16f);
           }
         }
@@ -762,12 +765,12 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
         }
       }
       for (int i = 0; i < m; ++i) {
-        float v[TN], o[TN];
+        float v[TN], o[TN][2];  // two sums a column: a row's channels in one chain of 32 round more than the sums of before
 #pragma unroll
         for (int n = 0; n < TN; ++n) {
           const int col = fresh(col0 + 16 * n + c), row = 16 * h + i;
           v[n] = bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(vs + row * VROW + (((col >> 3) ^ swz(row)) << 4) + (col & 7) * 2));
-          o[n] = 0.f;
+          o[n][0] = o[n][1] = 0.f;
         }
         f32x4 a[2], k[2], q[2];  // a tile's are read while the tile before is computed
         const int at = fresh(i * RD + 4 * g);
@@ -786,16 +789,17 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(const ScanArgs a
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               S[t][n][j] = fmaf(k[t & 1][j], v[n], S[t][n][j] * a[t & 1][j]);
-              if (PHASE != 1) o[n] = fmaf(S[t][n][j], q[t & 1][j], o[n]);
+              if (PHASE != 1) o[n][t & 1] = fmaf(S[t][n][j], q[t & 1][j], o[n][t & 1]);
             }
           __builtin_amdgcn_sched_barrier(0);
         }
         if (PHASE != 1)
 #pragma unroll
           for (int n = 0; n < TN; ++n) {
-            o[n] += __shfl_xor(o[n], 16, 64);
-            o[n] += __shfl_xor(o[n], 32, 64);
-            if (g == 0) out[((long)(r + 16 * h + i) * heads + head) * VD + col0 + 16 * n + c] = o[n];
+            float sum = o[n][0] + o[n][1];
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            if (g == 0) out[((long)(r + 16 * h + i) * heads + head) * VD + col0 + 16 * n + c] = sum;
           }
       }
     }

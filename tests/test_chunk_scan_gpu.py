@@ -84,6 +84,14 @@ def test_gates_that_forget_now_and_then(vdim, lens, pieces, every, first):
     assert off(out, want) < 5e-7 and off(st, ends) < 1e-6
 
 
+@pytest.mark.parametrize("bias", [(-4.0, -2.0), (-12.0, 2.0), (-130.0, 3.0)])
+def test_token_by_token_rounds_no_more_than_one_value(bias):
+    """Runs that go token by token: gates, keys and queries in 32 bits with about one rounding each, a channel's part of an output in
+    chains of 16: together below the largest rounding of one value, 2^-24 (5.2e-8; one chain of 32 and quotients of rounded sums 6.3e-8)."""
+    out, want, st, ends = gated(2, 128, [300, 33], [4, 4], (0.0, 0.0), bias, seed=3)
+    assert off(out, want) < 2 ** -24 and off(st, ends) < 2 ** -24
+
+
 def test_gates_that_forget_cost_a_few_times_the_others():
     """Token by token a run takes about three times as long as in blocks of 32 tokens; in blocks that shrink to one token it took 27."""
     heads, t = 32, 4096
