@@ -474,10 +474,11 @@ VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
 }
 
 // A host copy of some MB in pieces, each on a thread of its own where one can be had: a page comes out of memory, not of a cache.  The
-// threads end with the object.  A piece is no smaller than 768 KB: a thread takes 15 to 20 us to start and end.  A page to a bytes object / back
+// threads end with the object.  A piece is no smaller than 640 KB: a thread takes 15 to 20 us to start and end.  A page to a bytes object / back
 // on the device, one thread / four: 51 KB coded 115 / 183 us and 68 / 152, 1.2 MB 229 / 251 and 184 / 219, 7 MB 606 / 528 and 546 / 450; four pages of
-// 3.4 MB out in one, three, four pieces 1600 / 1505 / 1355, twelve back 1800 / 1675 / 1720.
-constexpr long COPY_PART = 768 << 10;
+// 3.4 MB out in one, three, four pieces 1600 / 1505 / 1355, twelve back 1800 / 1675 / 1720; one of 1.5 MB into memory of the caller's in one,
+// two, three 224 / 209 / 209, back 80 / 81 / 82 (in four 214 and 86).
+constexpr long COPY_PART = 640 << 10;
 class HostCopies {
  public:
   ~HostCopies() {

@@ -27,13 +27,13 @@ def test_workgroups_of_whole_products_begin_apart(n):
 
 
 def test_threads_that_share_a_copy():
-    """A copy has a thread for every 768 KB, up to four: starting one costs more than copying less."""
+    """A copy has a thread for every 640 KB, up to four: starting one costs more than copying less."""
     def parts(size):
         return ops._kernels().vpsa_copy_parts(c_long(size))
 
     kb = 1 << 10
-    assert [parts(n) for n in (0, 1, 51 * kb, 768 * kb, 1536 * kb - 1)] == [1] * 5
-    assert [parts(n) for n in (1536 * kb, 2304 * kb, 3072 * kb, 7 << 20, 1 << 40)] == [2, 3, 4, 4, 4]
+    assert [parts(n) for n in (0, 1, 51 * kb, 640 * kb, 1280 * kb - 1)] == [1] * 5
+    assert [parts(n) for n in (1280 * kb, 1920 * kb, 2560 * kb, 7 << 20, 1 << 40)] == [2, 3, 4, 4, 4]
 
 
 def test_routers_that_the_kernel_takes():

@@ -1322,7 +1322,7 @@ def test_layer_norm_takes_and_refuses_what_the_library_does():
 
 
 @pytest.mark.parametrize("size", [1, 16, 4095, 16384, 16385, 3 * 16384 + 5, 3455418,
-                                  (1536 << 10) - 1, 1536 << 10, (2304 << 10) + 4097, (3 << 20) - 5, (5 << 20) + 1])
+                                  (1280 << 10) - 1, 1280 << 10, (1920 << 10) + 4097, (2560 << 10) - 5, (5 << 20) + 1])
 def test_bytes_come_through_a_pinned_buffer_in_parts(size):
     src = torch.randint(0, 256, (size + 7,), dtype=torch.uint8, device=DEV)
     pinned, dst = torch.empty(size, dtype=torch.uint8, pin_memory=True), torch.full((size + 64,), 9, dtype=torch.uint8)
