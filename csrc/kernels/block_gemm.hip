@@ -16,12 +16,13 @@
 #include <type_traits>
 
 #include "common.h"
+#include "mid_reduce.h"
 
 namespace {
 
 constexpr int BK = 64, ROWB = BK * 2;
 
-enum { ACT_NONE = 0, ACT_GELU = 1 };
+enum { ACT_NONE = 0, ACT_GELU = 1, ACT_SILU = 2 };  // SILU: w is [gate rows | up rows], silu(gate) * up
 
 // Row r of an operand lies at (r / batch_rows) * bs + (r % batch_rows) * ld elements.
 struct Rows {
@@ -37,6 +38,8 @@ struct BlockArgs {
   Rows ar, cr, rr;
   int batch_rows, M, N, K, n_tiles;  // N: rows of one weight; n_tiles: column tiles of one weight
   int parts;
+  float* ws;  // splits > 1: partial sums [splits, M, N]
+  int splits;
   uint32_t a_bytes, w_bytes;  // ends of the operands, for loads past the reduction's end
 };
 
@@ -54,8 +57,10 @@ __device__ __forceinline__ float gelu(float x) {
   return x * (x >= 0.f ? 1.f - h : h);
 }
 
-template <int TM, int TN, int S, int ACT>
+// STREAM: few row tiles, weights read about once, by non-temporal loads and from another chunk on for every column tile.
+template <int TM, int TN, int S, int ACT, bool STREAM>
 __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void block_gemm_kernel(const BlockArgs args) {
+  constexpr bool PAIR = ACT == ACT_SILU;
   constexpr int BM = 32 * TM, BN = 32 * TN, STAGE = (BM + BN) * ROWB, NL = TM + TN;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -64,16 +69,24 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
 
   // Tiles in blocks of an eighth of the row tiles (up to eight), column by column inside a block, cut in eight runs, one per XCD
   // (workgroups go round them): those that share an L2 at any time are about a square of tiles.
-  int m0, n0, part;
+  int m0, n0, part, split = 0, c0 = 0, n = K / BK, first = 0;  // chunks c0 .. c0 + n - 1 of the reduction, from c0 + first round
   {
-    const int m_tiles = (M + BM - 1) / BM, cols = args.n_tiles * args.parts, total = m_tiles * cols, blk = min(8, (m_tiles + 7) / 8);
+    const int m_tiles = (M + BM - 1) / BM, cols = args.n_tiles * args.parts, tiles = m_tiles * cols, total = STREAM ? tiles * args.splits : tiles, blk = min(8, (m_tiles + 7) / 8);
     const int bid = blockIdx.x, xcd = bid & 7, q = total >> 3, r = total & 7;
-    const int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
+    int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
+    if (STREAM) {
+      split = t / tiles;
+      t -= split * tiles;
+      const int per = n / args.splits, extra = n - per * args.splits;
+      c0 = split * per + min(split, extra);
+      n = per + (split < extra);
+    }
     const int block = t / (blk * cols), rem = t - block * blk * cols, rows = min(blk, m_tiles - blk * block);
     const int col = rem / rows;
     m0 = (blk * block + rem - col * rows) * BM;
     part = col / args.n_tiles;
     n0 = (col - part * args.n_tiles) * BN;
+    if (STREAM) first = col * 3 % n;
   }
 
   // what this lane loads of a chunk: 8 rows of 8 pieces a KiB; rows past the last repeat it
@@ -88,16 +101,20 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     const int r = 8 * (4 * i + wave) + lrow, rr = r % (16 * TN), j = rr & 15, perm = 8 * (j >> 2) + 4 * ((rr >> 4) & 1) + (j & 3);
-    const int col = n0 + r / (16 * TN) * (16 * TN) + 32 * (rr >> 5) + perm;
-    woff[i] = (uint32_t)min(col, N - 1) * (uint32_t)(K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    // PAIR: tiles 2 b, 2 b + 1 of a wave are 16 gate rows and the up rows beside them
+    const int col = PAIR ? n0 / 2 + r / (16 * TN) * (8 * TN) + 16 * (rr >> 5) + j : n0 + r / (16 * TN) * (16 * TN) + 32 * (rr >> 5) + perm;
+    const int row = PAIR ? min(col, N / 2 - 1) + ((rr >> 4) & 1 ? N / 2 : 0) : min(col, N - 1);
+    woff[i] = (uint32_t)row * (uint32_t)(K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
   }
-  const int n = K / BK;
   auto load = [&](int c, char* st, int i) {  // the i-th KiB of this wave; nothing past the last chunk (a buffer of no bytes)
     const bool x = i < TM;
     const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(x ? args.a : args.w[part]), 0, c < n ? (int)(x ? args.a_bytes : args.w_bytes) : 0, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)(st + (4 * i + wave) * 1024), 16,
-                                             (int)(x ? aoff[i % TM] : woff[(i - TM + TN) % TN]), c < n ? c * ROWB : 0, 0, 0);
+    const auto to = (__attribute__((address_space(3))) void*)(st + (4 * i + wave) * 1024);
+    const int off = (int)(x ? aoff[i % TM] : woff[(i - TM + TN) % TN]);
+    const int at = c >= n ? 0 : STREAM ? (c0 + (c + first < n ? c + first : c + first - n)) * ROWB : c * ROWB;
+    if (STREAM && !x) __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to, 16, off, at, 0, 2);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to, 16, off, at, 0, 0);
   };
 
   // fragments: row c16 of a 16-row tile, piece 4 ks + g
@@ -160,6 +177,37 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
 
   // accumulator [i][j]: token row 16 j + c16 of the wave's; registers of tiles 2 b, 2 b + 1: columns 8 g .. 8 g + 7 of the 32 of pair b
   constexpr int NB = TN / 2;
+  if (STREAM && args.splits > 1) {
+    float* const ws = args.ws + (long)split * M * N;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int row = m0 + wr * 16 * TM + 16 * j + c16;
+      if (row >= M) continue;
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const int col = PAIR ? n0 / 2 + wc * 8 * TN + 16 * (i >> 1) + 4 * g : n0 + wc * 16 * TN + 32 * (i >> 1) + 8 * g + 4 * (i & 1);
+        if (col < (PAIR ? N / 2 : N)) *reinterpret_cast<f32x4*>(ws + (long)row * N + col + (PAIR && (i & 1) ? N / 2 : 0)) = acc[i][j];
+      }
+    }
+    return;
+  }
+  if constexpr (PAIR) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int row = m0 + wr * 16 * TM + 16 * j + c16;
+      if (row >= M) continue;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int col = n0 / 2 + wc * 8 * TN + 16 * b + 4 * g;
+        if (col >= N / 2) continue;
+        f32x4 s = acc[2 * b][j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = s[e] / (1.f + __expf(-s[e])) * acc[2 * b + 1][j][e];
+        *reinterpret_cast<u32x2*>(args.c + row * args.cr.ld + col) = (u32x2){pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+      }
+    }
+    return;
+  }
   const int col0 = n0 + wc * 16 * TN + 8 * g;
   u32x4 bias[NB];
 #pragma unroll
@@ -196,19 +244,19 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
   }
 }
 
-template <int TM, int TN, int S, int ACT>
+template <int TM, int TN, int S, int ACT, bool STREAM = false>
 int launch(BlockArgs& args, hipStream_t stream) {
   constexpr int LDS = (TM + TN) * S * 4096;
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)block_gemm_kernel<TM, TN, S, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)block_gemm_kernel<TM, TN, S, ACT, STREAM>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
       return -2;
     attr_set = true;
   }
   args.n_tiles = (args.N + 32 * TN - 1) / (32 * TN);
-  const long blocks = (long)args.n_tiles * args.parts * ((args.M + 32 * TM - 1) / (32 * TM));
+  const long blocks = (long)args.n_tiles * args.parts * args.splits * ((args.M + 32 * TM - 1) / (32 * TM));
   if (blocks >= (1L << 31)) return -1;
-  block_gemm_kernel<TM, TN, S, ACT><<<dim3((unsigned)blocks), 256, LDS, stream>>>(args);
+  block_gemm_kernel<TM, TN, S, ACT, STREAM><<<dim3((unsigned)blocks), 256, LDS, stream>>>(args);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -259,7 +307,7 @@ VPSA_EXPORT int vpsa_block_gemm(const void* x, long ld, long bs, const void* w0,
   BlockArgs args = {(const uint16_t*)x,
                     {(const uint16_t*)w0, (const uint16_t*)w1, (const uint16_t*)w2},
                     {(const uint16_t*)b0, (const uint16_t*)b1, (const uint16_t*)b2},
-                    (const uint16_t*)res, (uint16_t*)c, {ld, bs}, {ldc, cbs}, {ldr, rbs}, batch_rows, M, N, K, 0, parts,
+                    (const uint16_t*)res, (uint16_t*)c, {ld, bs}, {ldc, cbs}, {ldr, rbs}, batch_rows, M, N, K, 0, parts, nullptr, 1,
                     (uint32_t)a_bytes, (uint32_t)w_bytes};
 #define SHAPE(TM, TN, S) return act == ACT_GELU ? launch<TM, TN, S, ACT_GELU>(args, stream) : launch<TM, TN, S, ACT_NONE>(args, stream)
   switch (choose(M, N, K, parts, act)) {
@@ -271,4 +319,69 @@ VPSA_EXPORT int vpsa_block_gemm(const void* x, long ld, long bs, const void* w0,
     default: SHAPE(3, 6, 2);
   }
 #undef SHAPE
+}
+
+// Projections of 97 to 512 rows: up to 256 in one row tile of the smallest height that holds them, beyond in two; 128 weight rows a
+// workgroup, the reduction split until about every CU has one (ranges of six chunks at least), as in mid_gemm.hip, whose reductions close it.
+// Against mid_gemm's two blocks of 128 rows the weights pass through LDS once, and a wave multiplies 64 weight rows with half of the
+// token rows instead of 32 with all (a third less to read from LDS).  What bounds it: with all operands in the caches 28672 x 4096 takes 35 us
+// with 128 rows and 54 with 256 (1.1 PFLOP/s), with weights from memory 48 and 58: the two do not quite overlap.  More
+// chunks on their way (five stages), 64 weight rows a workgroup and two workgroups a CU changed nothing or were slower; non-temporal
+// loads of the weights take 5 % off, other start chunks for every column tile 1 to 2 %.
+// Library with its activation or norm pass / this: 28672 x 4096 with the gated unit, 129 rows 61.6 / 49.3 us, 256 rows 72.0 / 58.3; 4096 x 14336 with
+// the norm, 129 rows 58.4 / 38.1, 512 rows 93.1 / 68.2.  A step of 8 layers: 150 rows behind 3000 tokens 1938 -> 1610, 256 sequences 2578 -> 2243.
+static int block_splits(int M, int N, int K) {
+  const int blocks = (N + 127) / 128 * ((M + 255) / 256), most = K / BK / 6, s = 256 / (blocks > 0 ? blocks : 1);
+  return s > most ? (most > 0 ? most : 1) : s < 1 ? 1 : s;
+}
+
+// Workgroups along the reduction, 0 where the kernel does not tile the shape.
+VPSA_EXPORT int vpsa_block_proj_splits(int M, int N, int K, int pair) {
+  if (M <= 0 || M > 512 || N <= 0 || N % (pair ? 16 : 8) != 0 || K <= 0 || K % BK != 0 || (long)N * K * 2 >= (1L << 32)) return 0;
+  return block_splits(M, N, K);
+}
+
+static int block_product(const void* x, long xs, const void* w, const void* bias, void* y, long ys, void* ws, int M, int N, int K, int pair,
+                         int S, hipStream_t stream) {
+  if (M <= 0 || S <= 0 || S != vpsa_block_proj_splits(M, N, K, pair) || (S > 1 && !ws)) return -1;
+  if (xs < K || (xs & 7) || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws) & 15) || (double)M * xs * 2 >= 4294967296.) return -1;
+  if (S == 1 && ((ys & 7) || ((uintptr_t)y & 15) || ((uintptr_t)bias & 15))) return -1;
+  BlockArgs args = {(const uint16_t*)x, {(const uint16_t*)w, nullptr, nullptr}, {S == 1 ? (const uint16_t*)bias : nullptr, nullptr, nullptr},
+                    nullptr, (uint16_t*)y, {xs, 0}, {ys, 0}, {0, 0}, M, M, N, K, 0, 1, (float*)ws, S,
+                    (uint32_t)(2 * ((M - 1) * xs + K)), (uint32_t)(2L * N * K)};
+#define SHAPE(TM, S) return pair ? launch<TM, 4, S, ACT_SILU, true>(args, stream) : launch<TM, 4, S, ACT_NONE, true>(args, stream)
+  switch ((M + 32 * ((M + 255) / 256) - 1) / (32 * ((M + 255) / 256))) {
+    case 5: SHAPE(5, 4);
+    case 6: SHAPE(6, 3);
+    case 7: SHAPE(7, 3);
+    case 8: SHAPE(8, 3);
+    default: SHAPE(4, 4);
+  }
+#undef SHAPE
+}
+
+// y [M, N] = x W^T (+ bias), or silu(gate) * up [M, N / 2] with pair (w = [gate rows | up rows]).  x rows of stride xs, y rows of stride ys;
+// ws: fp32 workspace of S * M * N elements (unused when S == 1).
+VPSA_EXPORT int vpsa_block_proj(const void* x, long xs, const void* w, const void* bias, void* y, long ys, void* ws, int M, int N, int K,
+                                int pair, int S, hipStream_t stream) {
+  if ((ys & 3) || ((uintptr_t)y & 7) || (pair && bias)) return -1;
+  const int rc = block_product(x, xs, w, bias, y, ys, ws, M, N, K, pair, S, stream);
+  return rc || S == 1 ? rc : mid_reduce(ws, bias, y, ys, M, N, S, pair, stream);
+}
+
+// residual [M, N] += x W^T, y [M, N] = rms norm of the new rows * weight; S > 1.
+VPSA_EXPORT int vpsa_block_proj_norm(const void* x, long xs, const void* w, void* residual, const void* weight, void* y, void* ws, int M,
+                                     int N, int K, int S, float eps, hipStream_t stream) {
+  if (S < 2 || !mid_reduce_norm_takes(residual, weight, y, N)) return -1;
+  const int rc = block_product(x, xs, w, nullptr, nullptr, 0, ws, M, N, K, 0, S, stream);
+  return rc ? rc : mid_reduce_norm(ws, residual, weight, y, M, N, S, eps, stream);
+}
+
+// One token per sequence: q rotated to q_out, k rotated and v to the cache, as vpsa_mid_gemm_qkv; S > 1.
+VPSA_EXPORT int vpsa_block_proj_qkv(const void* x, long xs, const void* w, const void* bias, void* q_out, void* ws, int M, int K, int S,
+                                    const int* positions, const long* slots, const float* cos_sin, void* cache, long page_stride,
+                                    long v_offset, int n_q, int n_kv, hipStream_t stream) {
+  if (S < 2 || !mid_reduce_qkv_takes(q_out, bias, cos_sin)) return -1;
+  const int rc = block_product(x, xs, w, nullptr, nullptr, 0, ws, M, (n_q + 2 * n_kv) * HEAD_DIM, K, 0, S, stream);
+  return rc ? rc : mid_reduce_qkv(ws, bias, q_out, positions, slots, cos_sin, cache, page_stride, v_offset, M, n_q, n_kv, S, stream);
 }

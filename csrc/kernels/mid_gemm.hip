@@ -14,6 +14,7 @@
 // 28672 x 4096 with the gated unit: 8 rows 45.2 -> 37.5 us (6.26 TB/s of weights), 64 rows 57.2 -> 40.1, 97 rows 60.6 -> 48.2; 128256 x
 // 4096, 8 rows: 191 -> 161 (6.5 TB/s); 4096 x 14336, 88 rows: 50.1 -> 31.  The whole range stands at the dispatch in ops/__init__.py.
 #include "common.h"
+#include "mid_reduce.h"
 
 namespace {
 
@@ -509,14 +510,7 @@ static int mid_product(const void* x, long xs, const void* w, const void* bias, 
 #undef MID
 }
 
-// x [M, K] (row stride xs elements, 16-byte aligned rows), w [N, K] contiguous, bias [N] or null, y [M, N] (or [M, N / 2] when
-// pair != 0; row stride ys).  ws: fp32 workspace of S * M * N elements (unused when S == 1).
-VPSA_EXPORT int vpsa_mid_gemm(const void* x, long xs, const void* w, const void* bias, void* y, long ys, void* ws, int M, int N,
-                              int K, int pair, int S, hipStream_t stream) {
-  if (M <= 0) return 0;
-  if ((ys & 3) || ((uintptr_t)y & 7) || (pair && bias)) return -1;
-  const int rc = mid_product(x, xs, w, bias, y, ys, ws, M, N, K, pair, S, stream);
-  if (rc || S == 1) return rc;
+int mid_reduce(const void* ws, const void* bias, void* y, long ys, int M, int N, int S, int pair, hipStream_t stream) {
   const int n_out = pair ? N / 2 : N;
   const dim3 grid((n_out / 4 + 255) / 256, M);
   if (pair) mid_reduce_kernel<true><<<grid, 256, 0, stream>>>((const float*)ws, (const uint16_t*)bias, (uint16_t*)y, ys, M, N, S);
@@ -524,13 +518,11 @@ VPSA_EXPORT int vpsa_mid_gemm(const void* x, long xs, const void* w, const void*
   return 0;
 }
 
-// residual [M, N] += x W^T, y [M, N] = rms norm of the new rows * weight; a split product (S > 1), N a multiple of 4 up to 8192.
-VPSA_EXPORT int vpsa_mid_gemm_norm(const void* x, long xs, const void* w, void* residual, const void* weight, void* y, void* ws, int M,
-                                   int N, int K, int S, float eps, hipStream_t stream) {
-  if (M <= 0) return 0;
-  if (S < 2 || N % 4 != 0 || N > 8192 || (((uintptr_t)residual | (uintptr_t)weight | (uintptr_t)y) & 7)) return -1;
-  const int rc = mid_product(x, xs, w, nullptr, nullptr, 0, ws, M, N, K, 0, S, stream);
-  if (rc) return rc;
+bool mid_reduce_norm_takes(const void* residual, const void* weight, const void* y, int N) {
+  return N % 4 == 0 && N <= 8192 && (((uintptr_t)residual | (uintptr_t)weight | (uintptr_t)y) & 7) == 0;
+}
+
+int mid_reduce_norm(const void* ws, void* residual, const void* weight, void* y, int M, int N, int S, float eps, hipStream_t stream) {
   const int threads = N >= 4096 ? 1024 : (N / 4 + 63) / 64 * 64;
   if (N <= 4096)
     mid_reduce_norm_kernel<1><<<M, threads, 0, stream>>>((const float*)ws, (uint16_t*)residual, (const uint16_t*)weight, (uint16_t*)y, M,
@@ -541,20 +533,46 @@ VPSA_EXPORT int vpsa_mid_gemm_norm(const void* x, long xs, const void* w, void* 
   return 0;
 }
 
+bool mid_reduce_qkv_takes(const void* q_out, const void* bias, const void* cos_sin) {
+  return !((uintptr_t)q_out & 3) && !((uintptr_t)bias & 3) && !((uintptr_t)cos_sin & 7);
+}
+
+int mid_reduce_qkv(const void* ws, const void* bias, void* q_out, const int* positions, const long* slots, const float* cos_sin,
+                   void* cache, long page_stride, long v_offset, int M, int n_q, int n_kv, int S, hipStream_t stream) {
+  mid_reduce_qkv_kernel<<<dim3(M, (n_q + 2 * n_kv + 7) / 8), 256, 0, stream>>>(
+      (const float*)ws, (const uint16_t*)bias, (uint16_t*)q_out, positions, slots, cos_sin, (uint16_t*)cache, page_stride, v_offset, M,
+      n_q, n_kv, S);
+  return 0;
+}
+
+// x [M, K] (row stride xs elements, 16-byte aligned rows), w [N, K] contiguous, bias [N] or null, y [M, N] (or [M, N / 2] when
+// pair != 0; row stride ys).  ws: fp32 workspace of S * M * N elements (unused when S == 1).
+VPSA_EXPORT int vpsa_mid_gemm(const void* x, long xs, const void* w, const void* bias, void* y, long ys, void* ws, int M, int N,
+                              int K, int pair, int S, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if ((ys & 3) || ((uintptr_t)y & 7) || (pair && bias)) return -1;
+  const int rc = mid_product(x, xs, w, bias, y, ys, ws, M, N, K, pair, S, stream);
+  return rc || S == 1 ? rc : mid_reduce(ws, bias, y, ys, M, N, S, pair, stream);
+}
+
+// residual [M, N] += x W^T, y [M, N] = rms norm of the new rows * weight; a split product (S > 1), N a multiple of 4 up to 8192.
+VPSA_EXPORT int vpsa_mid_gemm_norm(const void* x, long xs, const void* w, void* residual, const void* weight, void* y, void* ws, int M,
+                                   int N, int K, int S, float eps, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (S < 2 || !mid_reduce_norm_takes(residual, weight, y, N)) return -1;
+  const int rc = mid_product(x, xs, w, nullptr, nullptr, 0, ws, M, N, K, 0, S, stream);
+  return rc ? rc : mid_reduce_norm(ws, residual, weight, y, M, N, S, eps, stream);
+}
+
 // q | k | v = x W^T (+ bias) of one token per sequence: q rotated to q_out [M, n_q * 128], k rotated and v to the cache (layer base
 // `cache`; slots < 0: nowhere); a split product (S > 1), N = (n_q + 2 n_kv) * 128.
 VPSA_EXPORT int vpsa_mid_gemm_qkv(const void* x, long xs, const void* w, const void* bias, void* q_out, void* ws, int M, int K, int S,
                                   const int* positions, const long* slots, const float* cos_sin, void* cache, long page_stride,
                                   long v_offset, int n_q, int n_kv, hipStream_t stream) {
   if (M <= 0) return 0;
-  const int N = (n_q + 2 * n_kv) * HEAD_DIM;
-  if (S < 2 || ((uintptr_t)q_out & 3) || ((uintptr_t)bias & 3) || ((uintptr_t)cos_sin & 7)) return -1;
-  const int rc = mid_product(x, xs, w, nullptr, nullptr, 0, ws, M, N, K, 0, S, stream);
-  if (rc) return rc;
-  mid_reduce_qkv_kernel<<<dim3(M, (n_q + 2 * n_kv + 7) / 8), 256, 0, stream>>>(
-      (const float*)ws, (const uint16_t*)bias, (uint16_t*)q_out, positions, slots, cos_sin, (uint16_t*)cache, page_stride, v_offset, M,
-      n_q, n_kv, S);
-  return 0;
+  if (S < 2 || !mid_reduce_qkv_takes(q_out, bias, cos_sin)) return -1;
+  const int rc = mid_product(x, xs, w, nullptr, nullptr, 0, ws, M, (n_q + 2 * n_kv) * HEAD_DIM, K, 0, S, stream);
+  return rc ? rc : mid_reduce_qkv(ws, bias, q_out, positions, slots, cos_sin, cache, page_stride, v_offset, M, n_q, n_kv, S, stream);
 }
 
 // Where a workgroup of a product begins (tests).

@@ -280,7 +280,9 @@ class TransformerModel:
         """An output projection, its all-reduce, the residual stream's update and the norm that reads it next."""
         eps = self.cfg.norm_eps
         if self.tp_size == 1 and packed is None and (self.lora is None or meta.lora_slots is None):
-            y = ops.linear_add_norm(x, w, residual, norm, eps)
+            y = ops.block_add_norm(x, w, residual, norm, eps)
+            if y is None:
+                y = ops.linear_add_norm(x, w, residual, norm, eps)
             if y is not None:
                 return y
         h = self._out_proj(name, layer, x, w, packed, residual, meta)

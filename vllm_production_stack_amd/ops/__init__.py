@@ -712,9 +712,9 @@ MID_SUMS_NORM = 4        # where the reduction also makes the residual stream an
 MID_ROWS_LONG = 256      # reductions beyond 8192, where the library's pick is poor at every batch
 
 
-def _mid_splits(m: int, n: int, k: int, pair: bool, sums: int = MID_SUMS) -> int:
+def _mid_splits(m: int, n: int, k: int, pair: bool, sums: int = MID_SUMS, rows: int = MID_ROWS_BLOCK) -> int:
     """Workgroups along the reduction when ``mid_gemm`` should take the shape, else 0.  ``sums``: quarters of the weights' bytes that
-    the partial sums of a block of rows may have."""
+    the partial sums of up to ``rows`` rows may have."""
     if not 0 < m <= MID_ROWS_LONG:
         return 0
     splits = int(_kernels().vpsa_mid_gemm_splits(c_int(m), c_int(n), c_int(k), c_int(1 if pair else 0)))
@@ -725,7 +725,7 @@ def _mid_splits(m: int, n: int, k: int, pair: bool, sums: int = MID_SUMS) -> int
         return 0
     if m <= MID_ROWS or (not pair and k > STREAM_MAX_K):
         return splits
-    if (m <= MID_ROWS_BLOCK and (wgs <= TILE_CUS or wgs >= MID_BLOCK_FILL * TILE_CUS * (-(-wgs // TILE_CUS)))
+    if (m <= rows and (wgs <= TILE_CUS or wgs >= MID_BLOCK_FILL * TILE_CUS * (-(-wgs // TILE_CUS)))
             and (splits == 1 if pair else 16 * m * splits <= sums * k)):
         return splits
     return 0
@@ -739,14 +739,65 @@ def _followed(*ts) -> bool:
             or torch._C._len_torch_dispatch_stack() > 0)
 
 
-def _mid_takes(x2, w, bias, pair, sums=MID_SUMS) -> int:
-    """``_mid_splits`` for operands that ``mid_gemm`` reads, else 0."""
-    if not (_skinny_enabled and x2.is_cuda and w.device == x2.device and x2.dim() == 2 and x2.dtype == torch.bfloat16
+# ``block_gemm``'s projections (one row tile of up to 256 rows or two, split sums closed by mid_gemm's reductions), library with its
+# activation or norm pass / mid_gemm / block, the same way:
+#   28672 x 4096 pair    97 rows 59.2/47.5/44.8    128 rows 60.2/49.1/48.3    129 rows 61.6/-/49.3    200 rows 71.2/-/55.0    256 rows 72.0/-/58.3
+#   57344 x 8192 pair    97      196/198/171       128      196/188/182       129      204/-/187      200      220/-/207      256      221/-/232
+#   128256 x 4096        97      233/218/209       128      235/227/219       129      288/-/225      200      297/-/243      256      299/-/264
+#   152064 x 3584        97      237/235/241       128      243/250/251       129      257/-/253      200      324/-/273      256      319/-/286
+#   4096 x 14336, norm   97      53.8/35.0/35.3    128      80.0/38.3/38.8    129      58.4/46.6/38.1 256      65.8/51.1/45.7 512      93.1/-/68.2
+#   8192 x 28672, norm   97      201/107/97        128      211/115/103       129      305/175/104    256      323/172/124    512      314/-/227
+#   3584 x 18944, norm   97      97.5/39.2/38.1    128      100/43.2/41.2     129      104/60.3/41.5  256      126/62.6/48.5  512      201/-/82
+#   8192 x 8192, norm    97      43.7/36.6/37.4    128      53.9/40.0/39.9    129      52.9/54.5/40.3 256      81.4/57.0/47.8 512      80.9/-/76.7
+#   4096 x 4096, norm   129      25.9/21.7/21.9    200      26.2/22.4/23.9    256      26.9/24.2/27.6 300      29.5/-/29.7    512      33.9/-/35.0
+#   3584 x 3584, norm   129      23.7/20.3/22.1    200      23.9/21.2/26.0    256      24.5/22.6/27.9 300      27.8/-/28.6    512      30.5/-/32.2
+#   6144 x 4096         129      38.4/29.7/24.9    150      39.4/30.4/26.3    176      25.7/30.1/27.3 230      26.3/30.8/29.9 256      39.9/31.6/30.9
+#   10240 x 8192        129      58.3/81.1/45.3    200      67.6/82.3/49.4    256      89.1/84.1/54.3 300      75.0/-/88.5    (two row tiles, 160 workgroups)
+BLOCK_MIN_ROWS = 97
+BLOCK_MAX_ROWS = 256             # one row tile
+BLOCK_MAX_ROWS_LONG = 512        # two: split products (unsplit 28672 x 4096, 300 rows: 80 with the library, 104)
+BLOCK_MID_ELEMS = 1 << 26        # up to 128 rows mid_gemm keeps split products of smaller weights
+BLOCK_SUMS_QKV = 8               # where the reduction also rotates and writes the cache, a launch of 12 us of its own with 256 rows
+
+
+def _block_splits(m: int, n: int, k: int, pair: bool, sums: int = MID_SUMS) -> int:
+    """Workgroups along the reduction when ``block_gemm``'s projections should take the shape, else 0.  ``sums``: quarters of the
+    weights' bytes that the partial sums may have (twice their rows: written and read)."""
+    if not BLOCK_MIN_ROWS <= m <= BLOCK_MAX_ROWS_LONG:
+        return 0
+    splits = int(_kernels().vpsa_block_proj_splits(c_int(m), c_int(n), c_int(k), c_int(1 if pair else 0)))
+    wgs = -(-n // 128) * splits * (-(-m // BLOCK_MAX_ROWS))
+    rounds = -(-wgs // TILE_CUS)
+    if splits <= 0 or wgs < (MID_MIN_FILL if rounds == 1 else MID_BLOCK_FILL) * TILE_CUS * rounds:
+        return 0
+    if splits == 1:  # (full tiles in a second round that is not: 57344 x 8192; up to 128 rows short reductions: 152064 x 3584)
+        if m > BLOCK_MAX_ROWS or (rounds > 1 and (k < STREAM_MAX_K // 2 if m <= MID_ROWS_BLOCK else m > 224 and wgs < 0.9 * TILE_CUS * rounds)):
+            return 0
+        return splits
+    if pair or (m <= MID_ROWS_BLOCK and n * k <= BLOCK_MID_ELEMS) or 16 * m * splits > sums * k:
+        return 0
+    return splits
+
+
+def _reads(x2, w, bias) -> bool:
+    """Operands that the projection kernels of small batches read."""
+    return (_skinny_enabled and x2.is_cuda and w.device == x2.device and x2.dim() == 2 and x2.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and x2.stride(1) == 1 and x2.shape[1] == w.shape[1]
             and (bias is None or (bias.device == x2.device and bias.dtype == torch.bfloat16 and bias.is_contiguous()
-                                  and bias.shape == w.shape[:1]))):
+                                  and bias.shape == w.shape[:1])))
+
+
+def _mid_takes(x2, w, bias, pair, sums=MID_SUMS, rows=MID_ROWS_BLOCK) -> int:
+    """``_mid_splits`` for operands that ``mid_gemm`` reads, else 0."""
+    splits = _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair, sums, rows) if _reads(x2, w, bias) else 0
+    return 0 if splits and _followed(x2, w, bias) else splits
+
+
+def _block_takes(x2, w, bias, pair, sums=MID_SUMS) -> int:
+    """``_block_splits`` for operands that ``block_gemm`` reads, else 0."""
+    if x2.dim() != 2 or not BLOCK_MIN_ROWS <= x2.shape[0] <= BLOCK_MAX_ROWS_LONG or not _reads(x2, w, bias):
         return 0
-    splits = _mid_splits(x2.shape[0], w.shape[0], w.shape[1], pair, sums)
+    splits = _block_splits(x2.shape[0], w.shape[0], w.shape[1], pair, sums)
     return 0 if splits and _followed(x2, w, bias) else splits
 
 
@@ -755,18 +806,44 @@ def _mid_gemm(x2, w, bias, pair):
     splits = _mid_takes(x2, w, bias, pair)
     if not splits:
         return None
+    return _split_product(_kernels().vpsa_mid_gemm, x2, w, bias, pair, splits)
+
+
+def _block_proj(x2, w, bias, pair):
+    """Projection of about a hundred to a few hundred rows (``csrc/kernels/block_gemm.hip``), or None where another kernel is the better
+    choice."""
+    splits = _block_takes(x2, w, bias, pair)
+    if not splits:
+        return None
+    return _split_product(_kernels().vpsa_block_proj, x2, w, bias, pair, splits)
+
+
+def _split_product(entry, x2, w, bias, pair, splits):
     m, n, k = x2.shape[0], w.shape[0], w.shape[1]
     out = torch.empty((m, n // 2 if pair else n), dtype=x2.dtype, device=x2.device)
     ws = torch.empty((splits * m * n,), dtype=torch.float32, device=x2.device) if splits > 1 else None
-    rc = _kernels().vpsa_mid_gemm(_p(x2), c_long(x2.stride(0)), _p(w), _p(bias), _p(out), c_long(out.stride(0)), _p(ws), c_int(m),
-                                  c_int(n), c_int(k), c_int(1 if pair else 0), c_int(splits), _stream())
+    rc = entry(_p(x2), c_long(x2.stride(0)), _p(w), _p(bias), _p(out), c_long(out.stride(0)), _p(ws), c_int(m),
+               c_int(n), c_int(k), c_int(1 if pair else 0), c_int(splits), _stream())
     return out if rc == 0 else None
 
 
 def linear_add_norm(x, w, residual, weight, eps):
     """``residual += x @ w.T`` and the norm of the new rows, ``rmsnorm(residual) * weight``, when ``mid_gemm`` splits the product: its
     reduction then makes both.  None (and nothing done) otherwise."""
-    splits = _mid_takes(x, w, None, False, MID_SUMS_NORM)
+    return _add_norm("vpsa_mid_gemm_norm", _mid_takes(x, w, None, False, MID_SUMS_NORM), x, w, residual, weight, eps)
+
+
+def block_add_norm(x, w, residual, weight, eps):
+    """As ``linear_add_norm``, for the batches from 97 rows on that ``block_gemm`` takes, or ``mid_gemm`` in two blocks of 128 rows."""
+    if x.dim() != 2 or not BLOCK_MIN_ROWS <= x.shape[0] <= BLOCK_MAX_ROWS_LONG:
+        return None
+    y = _add_norm("vpsa_block_proj_norm", _block_takes(x, w, None, False, MID_SUMS_NORM), x, w, residual, weight, eps)
+    if y is None and x.shape[0] > MID_ROWS_BLOCK:
+        y = _add_norm("vpsa_mid_gemm_norm", _mid_takes(x, w, None, False, MID_SUMS_NORM, MID_ROWS_LONG), x, w, residual, weight, eps)
+    return y
+
+
+def _add_norm(entry, splits, x, w, residual, weight, eps):
     m, n = x.shape[0], w.shape[0]
     if (splits < 2 or n > 8192 or residual.shape != (m, n) or residual.dtype != torch.bfloat16 or not residual.is_contiguous()
             or residual.device != x.device or weight.device != x.device or weight.dtype != torch.bfloat16 or weight.shape != (n,)
@@ -774,15 +851,18 @@ def linear_add_norm(x, w, residual, weight, eps):
         return None
     y = torch.empty_like(residual)
     ws = torch.empty((splits * m * n,), dtype=torch.float32, device=x.device)
-    rc = _kernels().vpsa_mid_gemm_norm(_p(x), c_long(x.stride(0)), _p(w), _p(residual), _p(weight), _p(y), _p(ws), c_int(m), c_int(n),
-                                       c_int(w.shape[1]), c_int(splits), c_float(eps), _stream())
+    rc = getattr(_kernels(), entry)(_p(x), c_long(x.stride(0)), _p(w), _p(residual), _p(weight), _p(y), _p(ws), c_int(m),
+                                    c_int(n), c_int(w.shape[1]), c_int(splits), c_float(eps), _stream())
     return y if rc == 0 else None
 
 
 def decode_qkv(x, w, bias, pool, layer, positions, slots, cos_sin, n_q, n_kv):
-    """q / k / v projection, rotary embedding and cache write of one token per sequence, when ``mid_gemm`` splits the projection: its
-    reduction then rotates and writes the cache.  The query rows [T, n_q * 128], or None (and nothing done) otherwise."""
-    splits = _mid_takes(x, w, bias, False)
+    """q / k / v projection, rotary embedding and cache write of one token per sequence, when ``mid_gemm`` or ``block_gemm``
+    splits the projection: its reduction then rotates and writes the cache.  The query rows [T, n_q * 128], or None (and nothing done)
+    otherwise."""
+    splits, entry = _mid_takes(x, w, bias, False), "vpsa_mid_gemm_qkv"
+    if splits < 2:
+        splits, entry = _block_takes(x, w, bias, False, BLOCK_SUMS_QKV), "vpsa_block_proj_qkv"
     m = x.shape[0]
     if splits < 2 or pool.dtype != torch.bfloat16 or w.shape[0] != (n_q + 2 * n_kv) * HEAD_DIM_HIP:
         return None
@@ -791,9 +871,9 @@ def decode_qkv(x, w, bias, pool, layer, positions, slots, cos_sin, n_q, n_kv):
     q = torch.empty((m, n_q * HEAD_DIM_HIP), dtype=x.dtype, device=x.device)
     ws = torch.empty((splits * m * w.shape[0],), dtype=torch.float32, device=x.device)
     base = pool.data_ptr() + layer * pool.stride(1) * 2
-    rc = _kernels().vpsa_mid_gemm_qkv(_p(x), c_long(x.stride(0)), _p(w), _p(bias), _p(q), _p(ws), c_int(m), c_int(w.shape[1]),
-                                      c_int(splits), _p(positions), _p(slots), _p(cos_sin), c_void_p(base), c_long(pool.stride(0)),
-                                      c_long(pool.stride(2)), c_int(n_q), c_int(n_kv), _stream())
+    rc = getattr(_kernels(), entry)(_p(x), c_long(x.stride(0)), _p(w), _p(bias), _p(q), _p(ws), c_int(m), c_int(w.shape[1]),
+                                    c_int(splits), _p(positions), _p(slots), _p(cos_sin), c_void_p(base), c_long(pool.stride(0)),
+                                    c_long(pool.stride(2)), c_int(n_q), c_int(n_kv), _stream())
     return q if rc == 0 else None
 
 
@@ -949,7 +1029,7 @@ def tile_rows(x, w, pair: bool = False) -> int:
 def linear(x, w, bias=None, packed=None):
     """y = x @ w.T (+ bias).  Prefill-sized batches run the hand-written 256 x 256 MFMA kernel
     (``csrc/kernels/tile_gemm.hip``) when its tiles fill the chip; batches of up to a hundred rows or so ``mid_gemm.hip``
-    where its workgroups do (``_mid_splits``), of up to 16 rows otherwise
+    and of up to a few hundred ``block_gemm.hip`` where their workgroups do (``_mid_splits``, ``_block_splits``), of up to 16 rows otherwise
     the weight-streaming MFMA kernels of ``csrc/kernels/gemm.hip`` (which one depends on the
     weight's shape); everything else goes to the library GEMM (hipBLASLt).  ``packed``:
     ``pack_weight(w)`` when the caller keeps one (decode-only steps): up to 64 rows then stream
@@ -958,7 +1038,9 @@ def linear(x, w, bias=None, packed=None):
         y = packed_linear(x, packed, w.shape[0], w.shape[1], bias, False)
         if y is not None:
             return y
-    y = _mid_gemm(x, w, bias, False)
+    y = _block_proj(x, w, bias, False)
+    if y is None:
+        y = _mid_gemm(x, w, bias, False)
     if y is not None:
         return y
     if x.dim() == 2 and x.shape[0] <= SMALL_BATCH_ROWS and _skinny_ok(x, w, bias):
@@ -1021,7 +1103,9 @@ def gate_up_silu(x, w_gate_up, packed=None):
         y = packed_linear(x, packed, w_gate_up.shape[0], w_gate_up.shape[1], None, True)
         if y is not None:
             return y
-    y = _mid_gemm(x, w_gate_up, None, True)
+    y = _block_proj(x, w_gate_up, None, True)
+    if y is None:
+        y = _mid_gemm(x, w_gate_up, None, True)
     if y is not None:
         return y
     if x.dim() == 2 and x.shape[0] <= PAIR_STREAM_MAX_ROWS and _skinny_ok(x, w_gate_up, None):
