@@ -1,0 +1,98 @@
+"""Products of 256 x 256 tiles whose last tiles are cut along the reduction (``csrc/kernels/tile_tail.h``): alone and behind whole rounds, even and
+uneven row tiles, the passes that close them, and which calls the dispatch hands over."""
+
+import pytest
+import torch
+
+from vllm_production_stack_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV, BF = torch.device("cuda"), torch.bfloat16
+
+
+def _inputs(m, n, k):
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    return torch.randn(m, k, generator=g, device=DEV).to(BF), (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF), g
+
+
+def _close(got, want, extra=0.):
+    # sums in 32 bits, one rounding to 16: half a unit in the last place, 2^-9, of every value
+    assert float(((got.double() - want).abs() - want.abs() * 2 ** -8 - extra - 1e-5).max()) < 0
+
+
+# (rows, columns, reduction, ranges): one tile, a row more than a unit of 64 and than a tile, whole row tiles, columns that end inside a tile,
+# a full round of tiles before 1, 17 and 128 of them, uneven ranges; 127 tiles are cut, 129 are not
+@pytest.mark.parametrize("m,n,k,splits", [(1, 256, 1600, 4), (65, 520, 1664, 4), (257, 264, 2048, 5), (512, 768, 2112, 5), (300, 1024, 4160, 10),
+                                          (4097, 4096, 3072, 8), (4352, 4112, 3136, 7), (6144, 4096, 4672, 2), (256, 127 * 256, 2112, 2),
+                                          (256, 129 * 256, 2112, 1)])
+def test_plain_gated_and_residual(m, n, k, splits):
+    x, w, g = _inputs(m, n, k)
+    assert ops.tile_tail(m, n, k) == splits
+    want = x.double() @ w.double().t()
+    _close(ops.tile_gemm(x, w), want)
+    r = torch.randn(m, n, generator=g, device=DEV).to(BF)
+    add = want + r.double()
+    _close(ops.tile_gemm(x, w, residual=r), add)
+    _close(ops.tile_gemm(x, w, residual=r, out=r), add)                          # in place
+    if n % 64 == 0:
+        gate, up = want[:, :n // 2], want[:, n // 2:]
+        _close(ops.tile_gemm(x, w, silu_mul=True), torch.nn.functional.silu(gate) * up)
+
+
+@pytest.mark.parametrize("m,n,k", [(600, 4096, 8192), (257, 520, 8192), (2100, 8192, 8192), (4100, 4096, 4096)])
+def test_residual_and_norm(m, n, k):
+    x, w, g = _inputs(m, n, k)
+    res, ln = torch.randn(m, n, generator=g, device=DEV).to(BF), torch.randn(n, generator=g, device=DEV).to(BF)
+    want = x.double() @ w.double().t() + res.double()
+    got = ops.tile_add_norm(x, w, res, ln, 1e-5)
+    assert got is not None
+    _close(res, want)
+    norm = res.double() * (res.double().square().mean(1, keepdim=True) + 1e-5).rsqrt() * ln.double()
+    assert float(((got.double() - norm).abs() - 2 ** -8 * norm.abs() - 1e-5).max()) < 0
+
+
+@pytest.mark.parametrize("tokens", [40, 130, 300, 700, 1100])
+@pytest.mark.parametrize("routing", ["spread", "one expert", "few"])
+def test_experts(tokens, routing):
+    """Experts without rows, with a few, with more than a tile; routings whose tiles have a tail and none."""
+    g = torch.Generator(device=DEV).manual_seed(tokens)
+    e, h, i, k = 8, 1032, 2048, 2
+    x = torch.randn(tokens, h, generator=g, device=DEV).to(BF)[:, :1024].contiguous()
+    w13 = (torch.randn(e, 2 * i, 1024, generator=g, device=DEV) / 32).to(BF)
+    w2 = (torch.randn(e, h, i, generator=g, device=DEV) * i ** -0.5).to(BF)
+    top = {"spread": e, "one expert": 1, "few": 3}[routing]
+    first = torch.randint(0, top, (tokens,), generator=g, device=DEV)
+    ids = torch.stack([first, (first + 1) % e], 1).int()
+    wt = torch.rand(tokens, k, generator=g, device=DEV)
+    wt[::7, 1] = 0                                                               # pairs that do not count
+    got = ops.moe_experts_prefill(x, w13, w2, ids, wt)
+    want = torch.zeros(tokens, h, dtype=torch.float64, device=DEV)
+    for c in range(e):
+        t, j = (ids == c).nonzero(as_tuple=True)
+        gate, up = (x[t].double() @ w13[c].double().t()).chunk(2, dim=1)
+        want.index_add_(0, t, wt[t, j, None].double() * ((torch.nn.functional.silu(gate) * up) @ w2[c].double().t()))
+    # activations and result rounded to 16 bits: 2^-9 of the norm each
+    assert float((got.double() - want).norm() / want.norm()) < 5e-3
+    y, pos = ops.moe_experts_prefill(x, w13, w2, ids, wt, combine=False)         # uncut, summed by the caller
+    assert float((ops.moe_combine(y, wt, pos, tokens).double() - want).norm() / want.norm()) < 6e-3
+
+
+def test_dispatch():
+    x, w, _ = _inputs(700, 4096, 8192)
+    assert ops._tile_takes(x, w) and not ops._tile_takes(x[:256], w)
+    assert not ops._tile_takes(x[:, :4096], w[:, :4096].contiguous())            # the library is ahead: short reductions, no whole round
+    assert not ops._tile_takes(x.float(), w) and not ops._tile_takes(x, w.cpu()) and not ops._tile_takes(x, w, False, x[0].cpu())
+    off = torch.empty(700 * 8192 + 1, device=DEV, dtype=BF)[1:].view(700, 8192)
+    assert not ops._tile_takes(off, w)                                           # rows off their 16 bytes
+    gu = torch.empty(28672, 512, device=DEV, dtype=BF)
+    assert ops._tile_takes(x[:300, :512], gu, True) and not ops._tile_takes(x[:256, :512], gu, True)
+    with torch.enable_grad():
+        assert not ops._tile_takes(x.clone().requires_grad_(), w)
+        leaf = x[:300].clone().requires_grad_()
+        ops.linear(leaf, w).sum().backward()
+        assert leaf.grad is not None
+    old = ops.set_tile_gemm(False)
+    try:
+        assert not ops._tile_takes(x, w)
+    finally:
+        ops.set_tile_gemm(old)

@@ -283,6 +283,8 @@ class TransformerModel:
             y = ops.block_add_norm(x, w, residual, norm, eps)
             if y is None:
                 y = ops.linear_add_norm(x, w, residual, norm, eps)
+            if y is None:
+                y = ops.tile_add_norm(x, w, residual, norm, eps)
             if y is not None:
                 return y
         h = self._out_proj(name, layer, x, w, packed, residual, meta)

@@ -843,6 +843,21 @@ def block_add_norm(x, w, residual, weight, eps):
     return y
 
 
+def tile_add_norm(x, w, residual, weight, eps):
+    """As ``linear_add_norm``, for products of the prefill GEMM with a split tail: the pass that closes it also makes the norm."""
+    m, n = x.shape[0], w.shape[0]
+    if (not _tile_takes(x, w, False, residual) or n > 8192 or not residual.is_contiguous() or residual.shape != (m, n)
+            or residual.dtype != torch.bfloat16 or residual.device != x.device or weight.device != x.device or weight.dtype != torch.bfloat16 or weight.shape != (n,)
+            or not weight.is_contiguous() or residual.data_ptr() % 8 or weight.data_ptr() % 8 or tile_tail(m, n, w.shape[1]) <= 1):
+        return None
+    ws = tail_parts(x.device)
+    tile_gemm(x, w, residual=residual, out=residual, parts=ws)
+    y = torch.empty_like(residual)
+    rc = _kernels().vpsa_tile_tail_norm(_p(ws), _p(residual), _p(weight), _p(y), c_int(m), c_int(n), c_int(w.shape[1]), c_float(eps), _stream())
+    _check(rc, "tile_tail_norm")
+    return y
+
+
 def _add_norm(entry, splits, x, w, residual, weight, eps):
     m, n = x.shape[0], w.shape[0]
     if (splits < 2 or n > 8192 or residual.shape != (m, n) or residual.dtype != torch.bfloat16 or not residual.is_contiguous()
@@ -979,9 +994,8 @@ STREAM_MAX_K = 8192
 
 # The prefill GEMM (``tile_gemm``: 256 x 256 tiles, one workgroup per CU) is used when its tiles fill
 # the chip's 256 CUs in whole rounds: measured on MI355X against the library at 8192 rows 0.95-0.98x
-# plain, 1.08x with the SwiGLU epilogue fused (profiles/r3_tile_gemm_micro_v1.jsonl); with the last
-# round of tiles half empty (e.g. 4096 x 4096 at 4616 rows: 304 tiles = 1.19 rounds) the library's
-# stream-K decomposition wins, and below ~1k rows every 256-row tile is mostly padding.
+# plain, 1.08x with the SwiGLU epilogue fused (profiles/r3_tile_gemm_micro_v1.jsonl).  Where they do not,
+# ``_tile_takes`` looks at what the cut tail saves.
 TILE_MIN_ROWS = int(os.environ.get("VPSA_TILE_MIN_ROWS", "1024"))
 TILE_MIN_FILL = float(os.environ.get("VPSA_TILE_MIN_FILL", "0.85"))
 TILE_CUS = 256
@@ -1026,6 +1040,45 @@ def tile_rows(x, w, pair: bool = False) -> int:
     return m
 
 
+# With the last round's tiles cut (``tile_tail``) and the activation in the epilogue the kernel is ahead of the library at other sizes as
+# well, microseconds, library with its activation or norm pass / here (weights that no cache holds):
+#   28672 x 4096 pair     257 rows 80/74     512 rows 109/99    700 rows 169/149   1200 rows 282/233    2100 rows 437/390    5300 rows 1044/921
+#   57344 x 8192 pair     300      318/304   512      422/369   1000     813/699   1500      1112/1017
+#   37888 x 3584 pair     300      121/105   512      150/131   1000     324/232   1500      384/335
+#   16384 x 2048 pair     300      36/38     512      42/47     700      54/48     1500      107/96     (300, 512: half a round, short reductions)
+#   4096 x 14336, norm    600      124/81    1000     144/107   1500     181/163   2100      249/251    4200      790/401     5300     785/482
+#   8192 x 28672, norm    700      331/315   1000     392/351   1500     561/573   2100      1440/751   4200      2066/1411
+#   3584 x 18944, norm    700      173/95    1500     281/181   2100     353/249   5300      1089/587
+#   2048 x 8192, norm     700      50/47     1500     70/68     3000     101/102
+#   10240 x 8192          512      96/88     700      110/106   1000     140/161   2100      304/291
+#   6144 x 4096           512      39/48     1000     56/63     3000     139/132   3500      145/148    6000      244/236
+#   4096 x 4096, norm     512      35/44     1000     49/55     4200     155/151   5300      173/181    6000      190/196
+TILE_TAIL_ROWS = TILE_MIN_ROWS if "VPSA_TILE_MIN_ROWS" in os.environ else 257
+TILE_PAIR_FILL = 0.7         # of the rounds, where the kernel also saves the activation's pass
+TILE_LONG_CHUNKS = 128       # reductions from which on a product with a cut tail is ahead ...
+TILE_TAIL_SPLITS = 4         # ... and elsewhere the ranges that a tail behind whole rounds has
+
+
+def _tile_takes(x, w, pair: bool = False, *others) -> bool:
+    """Whether the prefill GEMM should take all rows of ``x @ w.T``: ``tile_rows``, or the rule above for plain and gated products.  ``others``:
+    a bias or residual that the epilogue adds."""
+    if tile_rows(x, w, pair):
+        return True
+    if not (_tile_enabled and x.is_cuda and x.dim() == 2 and x.shape[0] >= TILE_TAIL_ROWS and w.dim() == 2
+            and x.shape[1] == w.shape[1] and tile_gemm_supported(w.shape[0], w.shape[1], pair) and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and all(t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0)
+                                          for t in (x, w, *others))
+            and x.shape[0] * x.stride(0) < 1 << 31):
+        return False
+    m, (n, k) = x.shape[0], w.shape
+    tiles, splits = -(-m // 256) * (-(-n // 256)), tile_tail(m, n, k, pair)
+    if pair:
+        takes = splits > 1 and tiles >= TILE_CUS or tiles >= TILE_PAIR_FILL * TILE_CUS * -(-tiles // TILE_CUS)
+    else:
+        takes = splits > 1 and (k >= 64 * TILE_LONG_CHUNKS or (tiles >= TILE_CUS and splits >= TILE_TAIL_SPLITS))
+    return takes and not _followed(x, w, *others)
+
+
 def linear(x, w, bias=None, packed=None):
     """y = x @ w.T (+ bias).  Prefill-sized batches run the hand-written 256 x 256 MFMA kernel
     (``csrc/kernels/tile_gemm.hip``) when its tiles fill the chip; batches of up to a hundred rows or so ``mid_gemm.hip``
@@ -1051,15 +1104,9 @@ def linear(x, w, bias=None, packed=None):
             y = _stream_gemm(x, w, bias, False)
         if y is not None:
             return y
-    rows = tile_rows(x, w) if (bias is None or bias.dtype == torch.bfloat16) else 0
-    if rows:
-        m = x.shape[0]
-        out = torch.empty((m, w.shape[0]), dtype=x.dtype, device=x.device)
+    if (bias is None or bias.dtype == torch.bfloat16) and _tile_takes(x, w, False, bias):
         # a bias is a "residual" with row stride 0
-        tile_gemm(x[:rows], w, residual=None if bias is None else bias.view(1, -1).expand(rows, -1), out=out[:rows])
-        if rows < m:
-            out[rows:] = linear(x[rows:], w, bias)
-        return out
+        return tile_gemm(x, w, residual=None if bias is None else bias.view(1, -1).expand(x.shape[0], -1))
     return torch.nn.functional.linear(x, w, bias)
 
 
@@ -1067,12 +1114,9 @@ def linear_add(x, w, residual, packed=None):
     """The residual-stream update of an output projection: ``residual += x @ w.T`` inside the GEMM's
     epilogue when the prefill kernel takes the shape (returns None: nothing is left to add), else
     returns ``x @ w.T`` for the caller's fused add + norm."""
-    rows = tile_rows(x, w) if residual.is_contiguous() else 0
-    if not rows:
+    if not residual.is_contiguous() or not _tile_takes(x, w, False, residual):
         return linear(x, w, None, packed)
-    tile_gemm(x[:rows], w, residual=residual[:rows], out=residual[:rows])
-    if rows < x.shape[0]:
-        residual[rows:] += linear(x[rows:], w)
+    tile_gemm(x, w, residual=residual, out=residual)
     return None
 
 
@@ -1087,7 +1131,7 @@ def qkv_linear(x, w, bias, q_cols: int):
     hand-written kernel does not take and that have no bias go to the library as two GEMMs,
     [q | k v], each writing its column range of ONE output buffer (same bits as the single call)."""
     if (bias is None and x.is_cuda and x.dim() == 2 and x.shape[0] >= SPLIT_QKV_MIN_ROWS
-            and x.dtype == torch.bfloat16 and 0 < q_cols < w.shape[0] and not tile_rows(x, w)):
+            and x.dtype == torch.bfloat16 and 0 < q_cols < w.shape[0] and not _tile_takes(x, w)):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
         torch.matmul(x, w[:q_cols].t(), out=out[:, :q_cols])
         torch.matmul(x, w[q_cols:].t(), out=out[:, q_cols:])
@@ -1114,14 +1158,8 @@ def gate_up_silu(x, w_gate_up, packed=None):
             y = _skinny(x, w_gate_up, None, True)
         if y is not None:
             return y
-    rows = tile_rows(x, w_gate_up, True)
-    if rows:
-        m = x.shape[0]
-        out = torch.empty((m, w_gate_up.shape[0] // 2), dtype=x.dtype, device=x.device)
-        tile_gemm(x[:rows], w_gate_up, silu_mul=True, out=out[:rows])
-        if rows < m:
-            silu_and_mul(torch.nn.functional.linear(x[rows:], w_gate_up), out=out[rows:])
-        return out
+    if _tile_takes(x, w_gate_up, True):
+        return tile_gemm(x, w_gate_up, silu_mul=True)
     return silu_and_mul(torch.nn.functional.linear(x, w_gate_up))
 
 
@@ -1557,7 +1595,7 @@ def tile_gemm_supported(n: int, k: int, silu_mul: bool = False) -> bool:
 
 
 def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, residual=None, out=None, glu_clamp=None,
-              relu_sq=False, xielu=None, gelu_mul=False, row_scale=None):
+              relu_sq=False, xielu=None, gelu_mul=False, row_scale=None, parts=None):
     """The prefill GEMM (``csrc/kernels/tile_gemm.hip``): out[r] = epilogue(a[arow_idx[r] or r] @ w[g]^T).
 
     a [*, K] bf16; w [N, K] (dense) or [G, N, K] (grouped, with offsets [G + 1] int32 ON THE DEVICE:
@@ -1568,7 +1606,8 @@ def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, resi
     relu_sq: out = relu(product)^2.  xielu = (a_pos, a_neg): out = a_pos z^2 + z / 2 for z > 0, else
     a_neg (exp(z) - 1 - z) + z / 2.  gelu_mul: paired like silu_mul, out = gelu(gate) * up with gelu in its tanh
     form.  row_scale (fp32 [rows], with glu_clamp): gate and up of an output row are multiplied by its factor before
-    the clamps.  Rows at or past offsets[G] are left unwritten."""
+    the clamps.  Rows at or past offsets[G] are left unwritten.  ``parts``: the workspace (``tail_parts``) of a caller that closes the
+    tail's split tiles itself; dense products are closed here."""
     paired = silu_mul or glu_clamp is not None or gelu_mul
     if w.dim() == 2:
         w = w.unsqueeze(0)
@@ -1598,12 +1637,34 @@ def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, resi
         epi, alpha, bias = 5, float(xielu[0]), float(xielu[1])
     if gelu_mul:
         epi = 6
+    ws = parts
+    if ws is None and offsets is None and epi <= 2 and tile_tail(rows, n, k, paired) > 1:
+        ws = tail_parts(a.device)
     rc = _kernels().vpsa_tile_gemm(_p(a), c_long(a.stride(0)), _p(arow_idx), _p(w), _p(offsets), c_int(g), _p(out),
                                    c_long(out.stride(0)), c_int(rows), c_int(n), c_int(k), c_int(epi), _p(residual),
                                    c_long(residual.stride(0) if residual is not None else 0), c_long(a.shape[0]),
-                                   c_float(lim), c_float(alpha), c_float(bias), _p(row_scale), _stream())
+                                   c_float(lim), c_float(alpha), c_float(bias), _p(row_scale), _p(ws), _stream())
     _check(rc, "tile_gemm")
+    if ws is not None and parts is None:
+        _tail_finish(ws, None, 1, out, rows, n, k, epi, residual)
     return out
+
+
+def tile_tail(rows: int, n: int, k: int, paired: bool = False) -> int:
+    """Ranges of the reduction that the last tiles of a dense product are cut in (1: none is), ``csrc/kernels/tile_tail.h``."""
+    n_tiles = (n // 2 + 127) // 128 if paired else (n + 255) // 256
+    return int(_kernels().vpsa_tile_tail(c_int((rows + 255) // 256 * n_tiles), c_int(k)))
+
+
+def tail_parts(device):
+    """Room for the partial sums of a round of tail workgroups, 256 tiles of 256 x 256."""
+    return torch.empty(256 << 16, dtype=torch.float32, device=device)
+
+
+def _tail_finish(ws, offsets, groups, out, rows, n, k, epi, residual=None):
+    rc = _kernels().vpsa_tile_tail_finish(_p(ws), _p(offsets), c_int(groups), _p(out), c_long(out.stride(0)), c_int(rows), c_int(n), c_int(k),
+                                          c_int(epi), _p(residual), c_long(0 if residual is None else residual.stride(0)), _stream())
+    _check(rc, "tile_tail_finish")
 
 
 def grouped_gemm_supported(n: int, k: int, silu_mul: bool = False) -> bool:
@@ -1614,7 +1675,7 @@ def moe_experts_prefill(x, w13, w2, ids, weights, gather=True, foreign=False, co
     """Expert MLP for prefill-sized batches: the (token, k) pairs are sorted by expert on the device
     and two grouped matrix-core GEMMs run over all experts at once: gate_up gathers its token
     rows by index and fuses silu(gate) * up, down writes the sorted rows that the weighted combine
-    gathers back.  Four launches, no host synchronisation."""
+    gathers back; split tiles of the last product's tail are summed there too.  Four launches, no host synchronisation."""
     t, k = ids.shape
     if not x.is_cuda:
         return reference.moe_experts(x, w13, w2, ids, weights)
@@ -1628,10 +1689,20 @@ def moe_experts_prefill(x, w13, w2, ids, weights, gather=True, foreign=False, co
         act = gg(x, w13, offsets, rows=t * k, arow_idx=sorted_tok, silu_mul=True)
     else:  # copy the rows into sorted order first (timing comparison)
         act = gg(moe_permute(x, sorted_tok), w13, offsets, rows=t * k, silu_mul=True)
-    y = gg(act, w2, offsets, rows=t * k)
-    if not combine:  # the caller sums the pairs itself
-        return y, pos
-    return moe_combine(y, weights, pos, t)
+    # (from eight rounds of tiles on there is no tail: tile_tail.h; the host knows the least that a routing can make)
+    if not combine or gg is not tile_gemm or -(-t * k // 256) * -(-w2.shape[1] // 256) >= 8 * TILE_CUS or w2.shape[1] % 8 or t == 0:
+        y = gg(act, w2, offsets, rows=t * k)
+        if not combine:  # the caller sums the pairs itself
+            return y, pos
+        return moe_combine(y, weights, pos, t)
+    ws = tail_parts(x.device)
+    y = tile_gemm(act, w2, offsets, rows=t * k, parts=ws)
+    assert weights.dtype == torch.float32 and pos.dtype == torch.int32
+    out = torch.empty((t, w2.shape[1]), dtype=x.dtype, device=x.device)
+    rc = _kernels().vpsa_moe_combine_parts(_p(ws), _p(offsets), c_int(n_experts), c_int(t * k), c_int(w2.shape[2]), _p(y),
+                                           _p(weights.contiguous()), _p(pos), _p(out), c_int(t), c_int(w2.shape[1]), c_int(k), _stream())
+    _check(rc, "moe_combine_parts")
+    return out
 
 
 def moe_experts_small_batch(x, w13, w2, ids, weights):
