@@ -1121,6 +1121,47 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
   const int last = kt1 - 1 - kt0;
   const int n_full = n_full_all - kt0;
 
+  const int* bt = block_tables + (long)seq * max_blocks + kt0;
+  const long kv_head_off = (long)kvh * PAGE * HEAD_DIM;
+  // DIRECT: the tile goes from global memory into its swizzled LDS image without passing through
+  // registers.  One load instruction of a wave fills one contiguous KiB of LDS, lane l the 16 bytes
+  // at l * 16: four keys' rows of the K image (16 slots each) or eight channels' rows of the V image
+  // (8 slots each).  The swizzle is therefore applied to the SOURCE: the lane reads the chunk whose
+  // place in the image its slot is.  Instruction i of wave w fills KiB 4 i + w of the 16.
+  int gk_off[4], gv_off[4];  // element offsets inside one head's K part / V part
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int kib = 4 * i + wave;
+    const int key = 4 * kib + (lane >> 4), c = (lane & 15) ^ (key & 15);
+    gk_off[i] = (c >> 2) * (PAGE * 32) + key * 32 + (c & 3) * 8;
+    const int d = 8 * kib + (lane >> 3), cv = (lane & 7) ^ ((d >> 1) & 7);
+    gv_off[i] = (cv >> 2) * (HEAD_DIM * 32) + d * 32 + (cv & 3) * 8;
+  }
+  auto direct_op = [&](const uint16_t* head_kp, char* buf, int i) {  // i = 0..7: K KiB, then V KiB
+    typedef __attribute__((address_space(3))) void* lds_ptr_t;
+    typedef const __attribute__((address_space(1))) void* glb_ptr_t;
+    if (i < 4)
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(head_kp + gk_off[i]), (lds_ptr_t)(buf + (4 * i + wave) * 1024),
+                                       16, 0, 0);
+    else
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(head_kp + v_offset + gv_off[i - 4]),
+                                       (lds_ptr_t)(buf + 16384 + (4 * (i - 4) + wave) * 1024), 16, 0, 0);
+  };
+  auto direct_tile = [&](int tile, char* buf) {
+    const uint16_t* head_kp = cache + (long)bt[tile] * page_stride + kv_head_off;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) direct_op(head_kp, buf, i);
+  };
+
+  // the first two tiles are on their way before the query rows are asked for and rotated
+  if (DIRECT) {
+    direct_tile(0, lds);
+    direct_tile(last < 1 ? last : 1, lds + 32768);
+    // the first step multiplies an empty pending slice (pw1 = 0) by V^T of "tile -1": give that buffer finite contents
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(lds + 65536 + 16384 + (i * 256 + tid) * 16) = (u32x4){0, 0, 0, 0};
+  }
+
   bf16x8 qf[2][8];
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
@@ -1161,8 +1202,6 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
     }
   }
 
-  const int* bt = block_tables + (long)seq * max_blocks + kt0;
-  const long kv_head_off = (long)kvh * PAGE * HEAD_DIM;
   my_pos[0] -= kt0 * PAGE;  // (the rotary table above took the absolute positions)
   my_pos[1] -= kt0 * PAGE;
 
@@ -1192,36 +1231,6 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
       *reinterpret_cast<u32x4*>(buf + wv_off[i]) = sv[i];
     }
   };
-  // DIRECT: the tile goes from global memory into its swizzled LDS image without passing through
-  // registers.  One load instruction of a wave fills one contiguous KiB of LDS, lane l the 16 bytes
-  // at l * 16: four keys' rows of the K image (16 slots each) or eight channels' rows of the V image
-  // (8 slots each).  The swizzle is therefore applied to the SOURCE: the lane reads the chunk whose
-  // place in the image its slot is.  Instruction i of wave w fills KiB 4 i + w of the 16.
-  int gk_off[4], gv_off[4];  // element offsets inside one head's K part / V part
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int kib = 4 * i + wave;
-    const int key = 4 * kib + (lane >> 4), c = (lane & 15) ^ (key & 15);
-    gk_off[i] = (c >> 2) * (PAGE * 32) + key * 32 + (c & 3) * 8;
-    const int d = 8 * kib + (lane >> 3), cv = (lane & 7) ^ ((d >> 1) & 7);
-    gv_off[i] = (cv >> 2) * (HEAD_DIM * 32) + d * 32 + (cv & 3) * 8;
-  }
-  auto direct_op = [&](const uint16_t* head_kp, char* buf, int i) {  // i = 0..7: K KiB, then V KiB
-    typedef __attribute__((address_space(3))) void* lds_ptr_t;
-    typedef const __attribute__((address_space(1))) void* glb_ptr_t;
-    if (i < 4)
-      __builtin_amdgcn_global_load_lds((glb_ptr_t)(head_kp + gk_off[i]), (lds_ptr_t)(buf + (4 * i + wave) * 1024),
-                                       16, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds((glb_ptr_t)(head_kp + v_offset + gv_off[i - 4]),
-                                       (lds_ptr_t)(buf + 16384 + (4 * (i - 4) + wave) * 1024), 16, 0, 0);
-  };
-  auto direct_tile = [&](int tile, char* buf) {
-    const uint16_t* head_kp = cache + (long)bt[tile] * page_stride + kv_head_off;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) direct_op(head_kp, buf, i);
-  };
-
   f32x16 o_acc[2][4];
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb)
@@ -1519,9 +1528,6 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
   int b_cur = 0, b_nxt = 32768, b_wr = 65536;
 
   if (DIRECT) {
-    direct_tile(0, lds);
-    direct_tile(0, lds + 65536);  // (finite contents for the empty pending slice, see below)
-    direct_tile(last < 1 ? last : 1, lds + 32768);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   } else {
     stage_load(0);
@@ -1601,8 +1607,8 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
   mfma_drain(o_acc);
   if (!head_ok) return;  // (no barrier below)
   if (part >= 0) {
-    // record = [2 row blocks][4 channel tiles][16 values][64 lanes] fp32, then [2][64] maxima and
-    // [2][64] sums: lane-major, so that the combine kernel (same lane roles) reads it back whole.  Rows past the sequence's (a
+    // record = [2 row blocks][4 channel tiles][4][64 lanes][4 values] fp32, then [2][64] maxima and
+    // [2][64] sums: a KiB a store, and the combine kernel (same lane roles) reads it back whole.  Rows past the sequence's (a
     // quarter of a tile on average, 35 MB of 97 rows' records with them) are neither written nor read.
     float* rec = split_ws + ((long)(part * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS;
 #pragma unroll
@@ -1612,7 +1618,9 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) rec[((rb * 4 + dt) * 16 + i) * 64 + lane] = o_acc[rb][dt][i];
+        for (int i = 0; i < 16; i += 4)
+          *reinterpret_cast<f32x4*>(rec + (((rb * 4 + dt) * 4 + (i >> 2)) * 64 + lane) * 4) =
+              (f32x4){o_acc[rb][dt][i], o_acc[rb][dt][i + 1], o_acc[rb][dt][i + 2], o_acc[rb][dt][i + 3]};
       rec[8192 + rb * 64 + lane] = m_run[rb];
       rec[8192 + 128 + rb * 64 + lane] = l_tot;
     }
@@ -1643,7 +1651,7 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
 // the attention kernel's epilogue: 8 values each, so the merge of a tile is spread over 16 x the
 // head groups workgroups and every record is read with whole-wave contiguous loads.  (Slices of 16 values left half the CUs without a
 // workgroup: 97 rows of 32 heads in 16 ranges 11.4 -> 9.6 us, with the rows
-// that are left out above.)
+// that are left out above; with 16 bytes a load instead of 4, 9.3 -> 8.2, 200 rows in 24 ranges 9.2 -> 7.4.)
 __global__ __launch_bounds__(256) void prefill_combine_kernel(
     const float* __restrict__ split_ws, const int* __restrict__ groups, uint16_t* __restrict__ out,
     long out_stride, const int* __restrict__ cu_q, int n_q, int n_kv) {
@@ -1660,12 +1668,12 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(
   const int row0 = cu_q[seq], q_len = cu_q[seq + 1] - row0;
   const int row = q0 + 32 * rb + r;
   if (row >= q_len) return;
-  const float* rec0 = split_ws + ((long)(part0 * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS + lane;
+  const float* rec0 = split_ws + ((long)(part0 * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS;
   const long rec_step = (long)gridDim.y * 4 * SPLIT_REC_FLOATS;
-  const int at = ((rb * 4 + dt) * 16 + 8 * half) * 64;
+  const int at = (((rb * 4 + dt) * 4 + 2 * half) * 64 + lane) * 4, am = 8192 + rb * 64 + lane;
   float m = NEG_BIG;
 #pragma unroll 8
-  for (int p = 0; p < nparts; ++p) m = fmaxf(m, rec0[p * rec_step + 8192 + rb * 64]);
+  for (int p = 0; p < nparts; ++p) m = fmaxf(m, rec0[p * rec_step + am]);
   float l = 0.f;
   float o[8];
 #pragma unroll
@@ -1673,10 +1681,14 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(
 #pragma unroll 4
   for (int p = 0; p < nparts; ++p) {
     const float* rec = rec0 + p * rec_step;
-    const float f = __builtin_amdgcn_exp2f(rec[8192 + rb * 64] - m);
-    l += f * rec[8192 + 128 + rb * 64];
+    const float f = __builtin_amdgcn_exp2f(rec[am] - m);
+    l += f * rec[am + 128];
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(rec + at), hi = *reinterpret_cast<const f32x4*>(rec + at + 256);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] += f * rec[at + i * 64];
+    for (int i = 0; i < 4; ++i) {
+      o[i] += f * lo[i];
+      o[i + 4] += f * hi[i];
+    }
   }
   const float inv = 1.f / l;
   uint16_t* op = out + (long)(row0 + row) * out_stride + head * HEAD_DIM + 32 * dt + 16 * half + 4 * h;

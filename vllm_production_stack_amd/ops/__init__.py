@@ -411,9 +411,9 @@ def build_prefill_tiles(q_lens, n_q, n_kv, rows=None, ctx_lens=None):
 SPLIT_MIN_KEY_TILES = 8     # a piece is at least this long (the kernel needs >= 3 in the last one)
 SPLIT_MAX_ROUNDS = 3        # longer lists lose at most a quarter of a round and are left alone
 SPLIT_CANDIDATES = 8        # round counts tried, starting at the list's own
-SPLIT_WG_OVERHEAD = 10.0    # a workgroup's prologue + epilogue, in key-tile times (measured: 7 rounds
-                            # of 55-tile pieces take 62 tile times each on a full chip)
-SPLIT_MERGE_COST = 25.0     # the merge launch, in key-tile times
+SPLIT_WG_OVERHEAD = 7.0     # a workgroup's prologue + epilogue, in key-tile times (1.9 us; a lone round of n tiles takes 14 + 1.9 n)
+SPLIT_MERGE_COST = 6.0      # the merge launch, in key-tile times (7 to 8 us and the gap before it; at 25, the times before the stroke: 16 rows
+                            # behind 2000 tokens 50/22 us, 97 behind 2000 56/28, 512 behind 2000 66/43, 2900 behind 12000 642/590)
 SPLIT_RECORD_COST = 0.15    # writing + reading one partial record, in key-tile times
 PREFILL_SPLITS = os.environ.get("VPSA_PREFILL_SPLITS", "1") != "0"
 
