@@ -353,16 +353,18 @@ def latent_attention(q_lat, q_rot, pool, offset: int, block_tables, row_seq, pos
         else:
             n_tiles = t * ((heads + LATENT_TILE_SLOTS - 1) // LATENT_TILE_SLOTS)
             bucket *= n_tiles // t
-        ws_o = ws_ml = None
-        if splits > 1:
-            ws_o = torch.empty((n_tiles * splits * LATENT_TILE_SLOTS * rank,), dtype=torch.float32, device=out.device)
-            ws_ml = torch.empty((n_tiles * splits * LATENT_TILE_SLOTS * 2,), dtype=torch.float32, device=out.device)
+        ws, ws_o, ws_ml = None, None, None
+        if splits > 1:  # partial outputs, then maxima and sums
+            slots = n_tiles * splits * LATENT_TILE_SLOTS
+            ws = torch.empty((slots * (rank + 2),), dtype=torch.float32, device=out.device)
+            ws_o = ws.data_ptr()
+            ws_ml = ws_o + 4 * slots * rank
+        assert pool.dim() == 2 and pool.stride(1) == 1 and offset + PAGE * (rank + rot) <= pool.shape[1]
+        qr, os_ = q_rot.stride(), out.stride()
         o._check(o._kernels().vpsa_latent_attention_mfma(
-            o._p(q_lat), c_long(ql_row), c_long(ql_head), o._p(q_rot), c_long(q_rot.stride(0)),
-            c_long(q_rot.stride(1)), _layer_base(pool, offset, rank + rot), c_long(pool.stride(0)), o._p(block_tables),
-            c_int(block_tables.stride(0)), o._p(tiles), o._p(positions), c_int(n_tiles), c_int(heads), o._p(sink),
-            o._p(out), c_long(out.stride(0)), c_long(out.stride(1)), c_int(rank), c_int(rot), c_float(scale),
-            c_int(window), c_int(splits), o._p(ws_o), o._p(ws_ml), c_int(bucket), o._stream()), "latent_attention_mfma")
+            o._at(q_lat), ql_row, ql_head, q_rot.data_ptr(), qr[0], qr[1], pool.data_ptr() + offset * pool.element_size(), pool.stride(0),
+            block_tables.data_ptr(), block_tables.stride(0), o._at(tiles), positions.data_ptr(), n_tiles, heads, o._at(sink), out.data_ptr(),
+            os_[0], os_[1], rank, rot, scale, window, splits, ws_o, ws_ml, bucket, o._raw_stream()), "latent_attention_mfma")
         return out
     if q_lat is None:
         raise ValueError("value | key entries: operands the tile kernel does not take")

@@ -198,11 +198,10 @@ def recurrent_scan(proj, q_col: int, k_col: int, v_col: int, heads: int, dim: in
             ws_state = torch.empty((pc.shape[0], heads, dim, vdim), dtype=torch.float32, device=proj.device)
             ws_decay = torch.empty((pc.shape[0], heads, dim), dtype=torch.float32, device=proj.device) if gated else None
         o._check(o._kernels().vpsa_chunk_scan(
-            o._p(proj), c_long(proj.stride(0)), c_int(q_col), c_int(k_col), c_int(v_col), c_int(heads), c_int(vdim),
-            _at(state, state_off), c_long(state.stride(0)), o._p(seq_cu), o._p(seq_state), c_int(n_seqs), o._p(positions),
-            o._p(decay), o._p(cos_sin), c_int(rot_dims), c_int(layout), c_float(k_scale), c_int(1 if act else 0),
-            o._p(gate_bias), o._p(gate_lower), o._p(out), o._p(pc), o._p(sp), c_int(0 if pc is None else pc.shape[0]),
-            o._p(ws_state), o._p(ws_decay), o._stream()), "chunk_scan")
+            proj.data_ptr(), proj.stride(0), q_col, k_col, v_col, heads, vdim, state.data_ptr() + 4 * state_off, state.stride(0),
+            seq_cu.data_ptr(), seq_state.data_ptr(), n_seqs, positions.data_ptr(), o._at(decay), o._at(cos_sin), rot_dims, layout, k_scale,
+            1 if act else 0, o._at(gate_bias), o._at(gate_lower), out.data_ptr(), o._at(pc), o._at(sp), 0 if pc is None else pc.shape[0],
+            o._at(ws_state), o._at(ws_decay), o._raw_stream()), "chunk_scan")
         return out
     # what enters the recurrence besides v, prepared in fp32 by a pass of its own: q' | k' (| gates)
     prep = torch.empty((proj.shape[0], heads, 3 if gated else 2, dim), dtype=torch.float32, device=proj.device)
