@@ -24,8 +24,14 @@
 // Coder: 32-bit state, byte-wise renormalisation, lower bound 2^23.  The encoder runs over its
 // symbols backwards and writes its bytes backwards into a private scratch slot, so the decoder
 // reads forwards; the slots are then gathered into one dense byte string at the prefix sum of the sizes.
+#include <pthread.h>
 #include <string.h>
 
+#include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <deque>
+#include <mutex>
 #include <thread>
 
 #include "common.h"
@@ -473,42 +479,96 @@ VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
   return coder > 0 && n % 64 == 0 ? page_symbols(n) + coder : 0;
 }
 
-// A host copy of some MB in pieces, each on a thread of its own where one can be had: a page comes out of memory, not of a cache.  The
-// threads end with the object.  A piece is no smaller than 640 KB: a thread takes 15 to 20 us to start and end.  A page to a bytes object / back
-// on the device, one thread / four: 51 KB coded 115 / 183 us and 68 / 152, 1.2 MB 229 / 251 and 184 / 219, 7 MB 606 / 528 and 546 / 450; four pages of
-// 3.4 MB out in one, three, four pieces 1600 / 1505 / 1355, twelve back 1800 / 1675 / 1720; one of 1.5 MB into memory of the caller's in one,
-// two, three 224 / 209 / 209, back 80 / 81 / 82 (in four 214 and 86).
+// A host copy of some MB in pieces: a page comes out of memory, not of a cache, and one thread draws 24 to 33 GB/s.  Up to three threads
+// help; they wait for copies of any caller, and end after two seconds without one (they are shared by a process: started for every copy
+// they cost 15 to 20 us each).  Host memory to host memory, one thread / started for the copy / waiting: 1.5 MB 34 / 30 / 15 us, 3.5 MB 107 / 50 / 33, 8 MB
+// 259 / 142 / 101.
 constexpr long COPY_PART = 640 << 10;
-class HostCopies {
+class CopyHelpers {
  public:
-  ~HostCopies() {
-    for (auto& t : threads_)
-      if (t.joinable()) t.join();
-  }
-  void start(int i, void* to, const void* from, long n) {
-    try {
-      threads_[i] = std::thread([=] { memcpy(to, from, n); });
-    } catch (...) {  // no thread to be had
-      memcpy(to, from, n);
-    }
-  }
   static constexpr int MOST = 3;
+  // `left` falls by one for every piece that is over.
+  struct Piece {
+    char* to;
+    const char* from;
+    long n;
+    std::atomic<int>* left;
+  };
+
+  // Never ends: a helper may outlive the process's other objects.  A fork has none of its parent's threads and begins with its own.
+  static CopyHelpers& shared() {
+    static std::atomic<CopyHelpers*> all{nullptr};
+    static const int forks = pthread_atfork(nullptr, nullptr, [] { all.store(nullptr); });
+    (void)forks;
+    CopyHelpers* mine = all.load(std::memory_order_acquire);
+    if (mine == nullptr) {
+      CopyHelpers* const made = new CopyHelpers;
+      if (all.compare_exchange_strong(mine, made)) return *made;
+      delete made;
+    }
+    return *mine;
+  }
+  // Queues the pieces; whatever no helper takes is taken by `finish`.
+  void start(const Piece* pieces, int n) {
+    {
+      std::lock_guard<std::mutex> hold(lock_);
+      queue_.insert(queue_.end(), pieces, pieces + n);
+      for (; helpers_ < MOST; ++helpers_) {
+        try {
+          std::thread([this] { help(); }).detach();
+        } catch (...) {  // no thread to be had
+          break;
+        }
+      }
+    }
+    ready_.notify_all();
+  }
+  void finish(const std::atomic<int>& left) {
+    while (left.load(std::memory_order_acquire) > 0)
+      if (!copy_one()) std::this_thread::yield();
+  }
 
  private:
-  std::thread threads_[MOST];
+  bool copy_one() {
+    std::unique_lock<std::mutex> hold(lock_);
+    if (queue_.empty()) return false;
+    const Piece p = queue_.front();
+    queue_.pop_front();
+    hold.unlock();
+    memcpy(p.to, p.from, p.n);
+    p.left->fetch_sub(1, std::memory_order_release);
+    return true;
+  }
+  void help() {
+    for (;;) {
+      if (copy_one()) continue;
+      std::unique_lock<std::mutex> hold(lock_);
+      if (!ready_.wait_for(hold, std::chrono::seconds(2), [this] { return !queue_.empty(); })) {
+        --helpers_;
+        return;
+      }
+    }
+  }
+  std::mutex lock_;
+  std::condition_variable ready_;
+  std::deque<Piece> queue_;
+  int helpers_ = 0;
 };
 
 VPSA_EXPORT int vpsa_copy_parts(long size) {
   const long parts = size / COPY_PART;
-  return parts < 1 ? 1 : parts > HostCopies::MOST ? HostCopies::MOST + 1 : (int)parts;
+  return parts < 1 ? 1 : parts > CopyHelpers::MOST ? CopyHelpers::MOST + 1 : (int)parts;
 }
 
 static void copy_in_parts(char* to, const char* from, long size) {
-  HostCopies copies;
   const int parts = vpsa_copy_parts(size);
   const long each = size / parts & ~4095L;  // whole pages
-  for (int i = 0; i < parts - 1; ++i, to += each, from += each, size -= each) copies.start(i, to, from, each);
+  std::atomic<int> left{parts - 1};
+  CopyHelpers::Piece pieces[CopyHelpers::MOST];
+  for (int i = 0; i < parts - 1; ++i, to += each, from += each, size -= each) pieces[i] = {to, from, each, &left};
+  if (parts > 1) CopyHelpers::shared().start(pieces, parts - 1);
   memcpy(to, from, size);
+  if (parts > 1) CopyHelpers::shared().finish(left);
 }
 
 // `size` bytes from the device to `to` by way of a pinned buffer.  Over on return.  (Four parts, each leaving the buffer while the next is on
@@ -520,16 +580,35 @@ VPSA_EXPORT int vpsa_fetch(const void* from, void* pinned, void* to, long size, 
   return 0;
 }
 
-// `size` host bytes at `from` (a page's parts) through the pinned buffer into `body`, then symbols and values.  Not waited for:
-// the buffer is read until the copy is over.
+// The copy of a page on a stream of its own, so that it runs beside the kernels of the page before it (3.5 MB: 70 us of copy, 53 of kernels);
+// `stream` waits for it.  fresh: `body` is new to the caller, and what `stream` still has to do may touch its memory.  Below 2 MB the
+// events cost the host, which is behind there anyway, what the copy takes (a page of 1.5 MB of many, one stream / two: 87 / 91 us; of 3.5 MB
+// 143 / 115, of 8 MB 238 / 196; with helpers that wait).
+constexpr long COPY_AHEAD = 2 << 20;
+static int page_copy(void* body, const void* pinned, long size, int fresh, hipStream_t copies, hipStream_t stream) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (size < COPY_AHEAD || copies == stream || hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
+    return hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, stream) == hipSuccess ? 0 : -3;
+  hipEvent_t event;
+  if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) return -3;
+  bool ok = !fresh || (hipEventRecord(event, stream) == hipSuccess && hipStreamWaitEvent(copies, event, 0) == hipSuccess);
+  const bool sent = ok && hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, copies) == hipSuccess;
+  ok = sent && hipEventRecord(event, copies) == hipSuccess && hipStreamWaitEvent(stream, event, 0) == hipSuccess;
+  if (sent && !ok) (void)hipStreamSynchronize(copies);  // nothing may read the buffer that the caller does not know of
+  (void)hipEventDestroy(event);  // (released when it has passed)
+  return ok ? 0 : -3;
+}
+
+// `size` host bytes at `from` (a page's parts) through the pinned buffer into `body` by way of `copies`, then symbols and values.  Not waited
+// for: pinned buffer and body are in use until `stream` has come past this call.
 VPSA_EXPORT int vpsa_page_decode(const void* from, void* pinned, void* body, long size, long n, int n_ctx, int spc, long unit_elems, void* ws,
-                                 void* out, hipStream_t stream) {
+                                 void* out, int fresh, hipStream_t copies, hipStream_t stream) {
   if (vpsa_page_workspace(n, n_ctx, spc) <= 0) return -1;
   const PageParts at = page_parts(body, n, n_ctx, spc);
   const long coded = size - (at.coded - (char*)body);
   if (coded < 0) return -1;
   copy_in_parts((char*)pinned, (const char*)from, size);
-  if (hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, stream) != hipSuccess) return -3;
+  if (const int rc = page_copy(body, pinned, size, fresh, copies, stream)) return rc;
   const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, (char*)ws + page_symbols(n), ws, n, n_ctx, spc, stream);
   return rc ? rc : vpsa_cachegen_decode(ws, (const float*)at.scales, out, n, unit_elems, stream);
 }
