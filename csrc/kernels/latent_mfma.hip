@@ -1,4 +1,4 @@
-// Latent attention on the matrix cores (gfx950, bf16): prefill tiles and decode rows in one kernel.
+// Latent attention on the matrix cores (gfx950, bf16): prefill tiles and decode rows.
 //
 // In latent space every head of a token attends over the SAME entries (latent | rotated key part,
 // RANK + ROT values per token), so a work item is a tile of up to 64 query slots = (token, head) pairs
@@ -30,7 +30,6 @@
 // (max = sink, sum = 1).  With key-range splits every split writes unnormalised partial outputs and
 // (max, sum) to a workspace and a merge kernel adds the sink and normalises.
 #include "common.h"
-#include <utility>
 
 namespace {
 
@@ -263,7 +262,7 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
   }
 }
 
-// The same walk for wide entries (RANK + ROT a multiple of 64, value accumulators of a wave in registers): pages go straight
+// The same walk for wide entries (512 + 64), decode rows here and tiles of 64 slots in the kernel behind it: pages go straight
 // into LDS, two of them, and the second product reads its transposed operand from the K image through the transposing LDS read.
 // What it replaces was bound by staging: a page passed through 128 registers into a K and a V^T image (137 KB of LDS writes with
 // 4 x 4 transposes) between two barriers, and a decode tile of 32 heads left two of the four waves idle meanwhile.
@@ -273,7 +272,7 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //   * ds_read_b64_tr_b16 gives lane (c, g) the keys 4 g .. 4 g + 3 of channel c: the order in which the S accumulators hold them.
 //   * Two pages are on their way except while one is read: the page after next is asked for as soon as its buffer is free, before
 //     the next one is waited for (a counted wait).  Waiting for each page before asking for another left 4.5 TB/s.
-//   * Decode rows of at most 32 heads (QUARTERS): eight waves, four of which share 16 slots.  Each scores 16 keys of a page, the
+//   * Decode rows of at most 32 heads: eight waves, four of which share 16 slots.  Each scores 16 keys of a page, the
 //     four exchange scores through 8 KB of LDS, keep the same softmax state and sum a quarter of the channels over all 64 keys.
 //     (With keys and states of its own a wave held all channels, and joining the four moved 130 KB through LDS at the end: 4 to 5 us
 //     that ranges of one or two pages could not hide.)  A quarter of a page's values fits into registers beside the rest, so the
@@ -282,12 +281,6 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //     The weights enter as two parts of 16 bits, a matrix instruction more for every value fragment that is read: with one part and
 //     one maximum for all 64 keys the error against 64 bits was 2.03e-3 on average over batches and contexts, with a maximum for
 //     each quarter 1.97e-3, with two parts it is 1.66e-3, the rounding of the result.
-//   * Tiles of 64 slots: eight waves, two of which share 16 slots: each scores 32 keys and sums 256 channels, scores go round through 16 KB
-//     of LDS.  The page is read as often as by four waves with 16 slots each, but a SIMD has a second wave while one waits for LDS, and
-//     nothing else hides that: a page takes 3.1 us instead of 4.5 (32 heads, 2000 rows behind 6000 entries 1978 -> 1402 us).  What bounds it
-//     is that reading, 550 KB a page (2.2 us at 128 bytes a cycle); waves of 32 slots would halve it but their queries alone are 144 registers.
-//   * Lists of few tiles are cut along the keys (ops/latent.py): 200 rows of 16 heads behind 3800 entries 289 -> 68 us, 25 of 32 behind 6000
-//     429 -> 43, 1000 of 16 behind 3000 294 -> 211.
 //   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
 // Decode rows with their merge, in a graph, pages from memory; staged through registers / this: 32 heads, 32 sequences of 4k entries in 8
 // ranges 65 / 40 us, 8 of 8k in 32 42 / 32, one of 26k in 32 86 / 49, one of 3k 22.9 / 21.0, one of 2k, a page a range, 17.4 / 18.0; 16 heads,
@@ -296,7 +289,7 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 // o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
 // their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
 // channels a tile, keys 16 apart, eight tiles a block.
-template <int ROW, int J>
+template <int ROW>
 __device__ __forceinline__ void read_transposed(u32x2 (&r)[16], const uint32_t (&at)[4]) {
   asm volatile(
       "ds_read_b64_tr_b16 %0, %16 offset:%20\n\tds_read_b64_tr_b16 %1, %16 offset:%21\n\t"
@@ -310,34 +303,19 @@ __device__ __forceinline__ void read_transposed(u32x2 (&r)[16], const uint32_t (
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7]), "=&v"(r[8]),
         "=&v"(r[9]), "=&v"(r[10]), "=&v"(r[11]), "=&v"(r[12]), "=&v"(r[13]), "=&v"(r[14]), "=&v"(r[15])
-      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(J * 256), "n"(J * 256 + 16 * ROW), "n"(J * 256 + 128),
-        "n"(J * 256 + 128 + 16 * ROW)
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(0), "n"(16 * ROW), "n"(128), "n"(128 + 16 * ROW)
       : "memory");
 }
 
-// PARTS 2: the weights in two parts of 16 bits, high and low.
-template <int PARTS>
-__device__ __forceinline__ void multiply_tiles(f32x4* o, const u32x2 (&r)[16], const bf16x8 (&pf)[PARTS]) {
+// The weights in two parts of 16 bits, high and low.
+__device__ __forceinline__ void multiply_tiles(f32x4* o, const u32x2 (&r)[16], const bf16x8 (&pf)[2]) {
 #pragma unroll
-  for (int part = 0; part < PARTS; ++part)
+  for (int part = 0; part < 2; ++part)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const u32x4 a = {r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]};
-      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), pf[part], o[i], 0, 0, 0);
-    }
+    for (int i = 0; i < 8; ++i)
+      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, (u32x4){r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]}),
+                                                     pf[part], o[i], 0, 0, 0);
 }
-
-template <int ROW, int J, int PARTS>
-__device__ __forceinline__ void transposed_products(f32x4* o, const bf16x8 (&pf)[PARTS], const uint32_t (&at)[4]) {
-  u32x2 r[16];
-  read_transposed<ROW, J>(r, at);
-  multiply_tiles(o + 8 * J, r, pf);
-}
-template <int ROW, int PARTS, int... J>
-__device__ __forceinline__ void all_products(f32x4* o, const bf16x8 (&pf)[PARTS], const uint32_t (&at)[4], std::integer_sequence<int, J...>) {
-  (transposed_products<ROW, J>(o, pf, at), ...);
-}
-
 // How many of `splits` key ranges a decode row of `pages` pages is cut into.  A workgroup fills a CU (two pages in LDS) and what it
 // does once - queries, the first page's way, a partial result of 64 KB - takes about as long as four pages (two or three give the
 // same times), so more workgroups than a round of 256 only pay if their ranges are long: 100 sequences of 1000 entries in 8 ranges
@@ -363,44 +341,29 @@ __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   return used;
 }
 
-// SHARE: waves that share 16 slots, each of which scores its part of a page's keys and sums its part of the channels.
-template <int RANK, int ROT, int SHARE>
+// Decode rows of at most 32 heads.
+template <int RANK, int ROT>
 __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
     long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
-    int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
-    const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
-    int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
+    int bt_stride, const int* __restrict__ positions, int heads, const float* __restrict__ sink, uint16_t* __restrict__ out,
+    long o_row, long o_head, float scale, int window, int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
   constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, DT = RANK / 16, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW;
-  static_assert(SHARE == 2 || SHARE == 4, "eight waves for four or two groups of 16 slots");
-  constexpr bool QUARTERS = SHARE == 4;
-  constexpr int WAVES = 8;
+  constexpr int WAVES = 8, SHARE = 4;              // waves that share 16 slots
   constexpr int NI = PAGE_BYTES / (1024 * WAVES);  // KiB of a page that a wave loads
-  constexpr int NT = 4 / SHARE;                    // 16-key tiles of a page that a wave scores
   constexpr int DW = DT / SHARE;                   // 16-channel tiles that it sums
-  static_assert(ENTRY % 64 == 0 && DW % 8 == 0, "chunks are exchanged within groups of eight");
+  static_assert(ENTRY % 64 == 0 && DW == 8, "chunks are exchanged within groups of eight; eight tiles a block of reads");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c16 = lane & 15, g = lane >> 4;
   const int sg = wave / SHARE, part = wave % SHARE;  // slots; keys and channels
-  LatTile t;
-  if (tiles) {
-    const int* e = tiles + 6 * blockIdx.x;
-    t = {e[0], e[1], e[2], e[3], e[4], e[5]};
-  } else {
-    const int runs = (heads + 63) >> 6;
-    const int row = blockIdx.x / runs, h0 = (blockIdx.x % runs) << 6;
-    t = {row, row, 1, positions[row], h0, min(64, heads - h0)};
-  }
-  if (t.seq < 0) return;
-  const int slot = sg * 16 + c16;
-  const bool valid = slot < t.n_tok * t.hcount;
-  const bool wave_active = sg * 16 < t.n_tok * t.hcount;  // wave-uniform
+  const int row = blockIdx.x, slot = sg * 16 + c16;
+  const int pos = positions[row];
+  const bool valid = slot < heads;
+  const bool wave_active = sg * 16 < heads;  // wave-uniform
   const float scale2 = scale * LOG2E;
-  const int tok = valid ? slot / t.hcount : 0;
-  const int head = t.head0 + (valid ? slot % t.hcount : 0);
-  const long row = t.row0 + tok;
-  // (a slot past the tile reads the tile's first query, and nothing of it is stored: no branch, no select.)  In a single round every
+  const int head = valid ? slot : 0;
+  // (a slot past the heads reads the first one's query, and nothing of it is stored: no branch, no select.)  In a single round every
   // range may be used, and the queries are on their way while the row's position and page are looked up (one sequence of 2k entries
   // 18.6 -> 17.7 us); with more, most of the workgroups have nothing to do (100 x 400 entries 37 -> 31 if they don't load them).
   bf16x8 qf[KS];
@@ -409,20 +372,17 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     for (int ks = 0; ks < KS; ++ks) {
       const int d = 32 * ks + 8 * g;
       qf[ks] = __builtin_bit_cast(
-          bf16x8, 32 * ks < RANK ? ld16(q_lat + row * ql_row + head * ql_head + d) : ld16(q_rot + row * qr_row + head * qr_head + (d - RANK)));
+          bf16x8, 32 * ks < RANK ? ld16(q_lat + (long)row * ql_row + head * ql_head + d) : ld16(q_rot + (long)row * qr_row + head * qr_head + (d - RANK)));
     }
   };
   const bool all_used = bucket * splits <= 256;
   if (all_used) load_q();
-  const int my_pos = valid ? t.pos0 + tok : -1;
-  const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
-  const int p_first = max(0, t.pos0 - window + 1) / PAGE;
-  const int used = tiles ? tile_ranges(t.pos0, t.n_tok, window, splits) : wide_splits(n_pages - p_first, bucket, splits);
-  const bool whole = splits == 1 || (tiles && used == 1);
+  const int n_pages = (pos + PAGE) / PAGE, p_first = max(0, pos - window + 1) / PAGE;
+  const int used = wide_splits(n_pages - p_first, bucket, splits);
   const int per = (n_pages - p_first + used - 1) / used;
   const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
   if (splits > 1 && p_begin >= p_end) {  // nothing to see: the merge passes over the record
-    if (!whole && tid < t.n_tok * t.hcount) {
+    if (tid < heads) {
       const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + tid;
       ws_ml[2 * rec] = -INFINITY;
       ws_ml[2 * rec + 1] = 0.f;
@@ -430,8 +390,7 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     return;
   }
   if (!all_used) load_q();
-  const int my_first = my_pos - window;
-  const int* bt = block_tables + (long)t.seq * bt_stride;
+  const int* bt = block_tables + (long)row * bt_stride;
 
   int src_off[NI];  // bytes into a page of what this lane loads into byte (WAVES i + wave) * 1024 + lane * 16 of the image
 #pragma unroll
@@ -445,21 +404,21 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     for (int i = 0; i < NI; ++i)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + src_off[i]),
                                        (__attribute__((address_space(3))) void*)(lds + buf * PAGE_BYTES + (WAVES * i + wave) * 1024),
-                                       16, 0, QUARTERS ? 2 : 0);  // 2: non-temporal
+                                       16, 0, 2);  // 2: non-temporal
   };
-  const bool seeded = whole && sink != nullptr && valid;
+  const bool seeded = splits == 1 && sink != nullptr && valid;
   float m = seeded ? sink[head] * LOG2E : -INFINITY;
   float l = seeded ? 1.f : 0.f;
   f32x4 o[DW];
 #pragma unroll
   for (int dt = 0; dt < DW; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  // K fragment of (key tile nt, step ks): row 16 nt + c16, chunk 4 ks + g; V^T fragment of (d tile dt, 16 keys from 16 n):
+  // K fragment of (this wave's key tile, step ks): row 16 part + c16, chunk 4 ks + g; V^T fragment of (d tile dt, 16 keys from 16 n):
   // the lane points at row 16 n + 4 g + lane / 4 % 4, channels 16 dt + 4 (lane % 4)
   const int fk = ((c16 >> 1) & 3) << 1 | (c16 >> 3);
   int koff[2], voff[4];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) koff[i] = (16 * NT * part + c16) * ROW + (((i * 4 + g) ^ fk) << 4);
+  for (int i = 0; i < 2; ++i) koff[i] = (16 * part + c16) * ROW + (((i * 4 + g) ^ fk) << 4);
   const int vr = 4 * g + ((lane >> 2) & 3), fv = ((vr >> 1) & 3) << 1 | (vr >> 3);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -468,26 +427,21 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
   f32x4 s[4];  // scores, then weights, of a page's keys
   auto score = [&](int buf) {
     const char* img = lds + buf * PAGE_BYTES;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) s[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    s[0] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128 + nt * 16 * ROW);
-        s[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks], s[nt], 0, 0, 0);
-      }
+      s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128), qf[ks], s[0], 0, 0, 0);
   };
   auto weigh = [&](int p) {
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) s[nt] *= scale2;
-    if (p * PAGE + PAGE - 1 > t.pos0 || p * PAGE <= t.pos0 + t.n_tok - 1 - window) {
+    if (p * PAGE + PAGE - 1 > pos || p * PAGE <= pos - window) {
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = p * PAGE + 16 * nt + 4 * g + e;
-          if (key > my_pos || key <= my_first) s[nt][e] = -INFINITY;
+          if (key > pos || key <= pos - window) s[nt][e] = -INFINITY;
         }
     }
     float mx = -INFINITY;
@@ -519,16 +473,16 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
       for (int dt = 0; dt < DW; ++dt) o[dt] *= corr;
     }
   };
-  auto weights = [&](int kk, bf16x8 (&pf)[QUARTERS ? 2 : 1]) {  // of keys 32 kk ..
+  auto weights = [&](int kk, bf16x8 (&pf)[2]) {  // of keys 32 kk ..
     u32x4 w, low;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float p0 = s[2 * kk + (i >> 1)][2 * (i & 1)], p1 = s[2 * kk + (i >> 1)][2 * (i & 1) + 1];
       w[i] = pack_bf16x2(p0, p1);
-      if constexpr (QUARTERS) low[i] = pack_bf16x2(p0 - bf16lo(w[i]), p1 - bf16hi(w[i]));
+      low[i] = pack_bf16x2(p0 - bf16lo(w[i]), p1 - bf16hi(w[i]));
     }
     pf[0] = __builtin_bit_cast(bf16x8, w);
-    if constexpr (QUARTERS) pf[1] = __builtin_bit_cast(bf16x8, low);
+    pf[1] = __builtin_bit_cast(bf16x8, low);
   };
   auto everyone = [&]() {  // (not __syncthreads, which would wait for the pages on their way)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -546,62 +500,35 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if constexpr (QUARTERS) {
-      // a page is read whole before its scores go round: the barrier of that exchange frees its buffer as well
-      f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;  // of four key quarters
-      u32x2 v0[16], v1[16];
-      if (wave_active) {
-        score(buf);
-        round[part * 64] = s[0];
-        const uint32_t at0[4] = {page + voff[0], page + voff[1], page + voff[2], page + voff[3]};
-        read_transposed<ROW, 0>(v0, at0);
-        const uint32_t at1[4] = {at0[0] + 32 * ROW, at0[1] + 32 * ROW, at0[2] + 32 * ROW, at0[3] + 32 * ROW};
-        read_transposed<ROW, 0>(v1, at1);
-      }
-      everyone();
-      if (p + 2 < p_end) load_page(p + 2, buf);
-      if (wave_active) {
+    // a page is read whole before its scores go round: the barrier of that exchange frees its buffer as well
+    f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;  // of four key quarters
+    u32x2 v0[16], v1[16];
+    if (wave_active) {
+      score(buf);
+      round[part * 64] = s[0];
+      const uint32_t at0[4] = {page + voff[0], page + voff[1], page + voff[2], page + voff[3]};
+      read_transposed<ROW>(v0, at0);
+      const uint32_t at1[4] = {at0[0] + 32 * ROW, at0[1] + 32 * ROW, at0[2] + 32 * ROW, at0[3] + 32 * ROW};
+      read_transposed<ROW>(v1, at1);
+    }
+    everyone();
+    if (p + 2 < p_end) load_page(p + 2, buf);
+    if (wave_active) {
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
-        weigh(p);
-        bf16x8 pf[2];
-        weights(0, pf);
-        multiply_tiles(o, v0, pf);
-        weights(1, pf);
-        multiply_tiles(o, v1, pf);
-      }
-    } else {
-      f32x4* round = reinterpret_cast<f32x4*>(lds + 2 * PAGE_BYTES) + sg * 256 + lane;
-      if (wave_active) {
-        score(buf);
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) round[(NT * part + nt) * 64] = s[nt];
-      }
-      everyone();
-      if (wave_active) {
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
-        weigh(p);
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const uint32_t half = page + kk * 32 * ROW;
-          const uint32_t at[4] = {half + voff[0], half + voff[1], half + voff[2], half + voff[3]};
-          bf16x8 pf[1];
-          weights(kk, pf);
-          all_products<ROW>(o, pf, at, std::make_integer_sequence<int, DW / 8>());
-        }
-      }
-      if (p + 2 < p_end) {
-        everyone();  // reads of this buffer are done
-        load_page(p + 2, buf);
-      }
+      for (int nt = 0; nt < 4; ++nt) s[nt] = round[nt * 64];
+      weigh(p);
+      bf16x8 pf[2];
+      weights(0, pf);
+      multiply_tiles(o, v0, pf);
+      weights(1, pf);
+      multiply_tiles(o, v1, pf);
     }
   }
 
   if (!valid) return;
-  if (whole) {
+  if (splits == 1) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    uint16_t* dst = out + row * o_row + head * o_head + part * DW * 16 + 4 * g;
+    uint16_t* dst = out + (long)row * o_row + head * o_head + part * DW * 16 + 4 * g;
 #pragma unroll
     for (int dt = 0; dt < DW; ++dt) {
       u32x2 w = {pack_bf16x2(o[dt][0] * inv, o[dt][1] * inv), pack_bf16x2(o[dt][2] * inv, o[dt][3] * inv)};
@@ -615,6 +542,298 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     if (g == 0 && part == 0) {
       ws_ml[2 * rec] = m * LN2;
       ws_ml[2 * rec + 1] = l;
+    }
+  }
+}
+
+// Tiles of 64 slots (prefill chunks, decode rows of more than 32 heads), images and pages as above.  What bounds a tile is reading a
+// page's fragments from LDS.  Eight waves, two of which shared 16 slots, read every fragment four times, 550 KB a page, and took 3.1 us
+// for it; waves of 32 slots read half of that, but two on a SIMD spill (143 to 285 registers of 256, 0.79x).  So four waves with all 64
+// slots, one on a SIMD, whose queries take the 256 accumulator registers:
+//   * A wave scores 16 of a page's keys for all slots and sums a quarter of the channels over all keys: each K and V^T fragment is read
+//     once and multiplied with four tiles of slots.  The waves exchange their keys' maxima by slot, then the weights in 16 bits (9 KB
+//     instead of 16 KB of scores).  A lane adds up its own keys' weights; the sums meet at the end.
+//   * Nothing but the order of instructions hides a wait: reads run three fragments in front of their products, the next page's loads
+//     go out one a step of the scores (all at once, they held those up), and rows past the list's last page load no bytes.
+//   * Queries come through LDS (below): 5 us a workgroup less than as fragments from memory.
+// 2.3 us a page.  32 heads: 2000 rows behind 6000 entries 1399 -> 1070 us, 2000 of one sequence 248 -> 200, 600 behind 7400 565 -> 447,
+// 200 behind 3800 122 -> 98, 20 behind 1980 32.7 -> 29.6; 16 heads, 60 behind 7940 47.0 -> 41.4; decode rows, 32 sequences of 4k
+// entries, 64 heads 49.7 -> 42.7, 128 heads 76.6 -> 63.0.  Errors against 64 bits are what they were, to five digits.
+// Lists of few tiles are cut along the keys (ops/latent.py).
+__device__ __forceinline__ bf16x8 read_transposed_pair(const char* lo, const char* hi) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)lo);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)hi);
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+__device__ __forceinline__ float max_of_groups(float x) {  // over the lanes c, c + 16, c + 32, c + 48
+  const uint32_t u = __float_as_uint(x);
+  const auto far = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t v = __float_as_uint(fmaxf(__uint_as_float(far[0]), __uint_as_float(far[1])));
+  const auto near = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return fmaxf(__uint_as_float(near[0]), __uint_as_float(near[1]));
+}
+
+template <int RANK, int ROT>
+__global__ __launch_bounds__(256, 1) void latent_tile_kernel(
+    const uint16_t* __restrict__ q_lat, long ql_row, long ql_head, const uint16_t* __restrict__ q_rot, long qr_row,
+    long qr_head, const uint16_t* __restrict__ cache, long page_stride, const int* __restrict__ block_tables,
+    int bt_stride, const int* __restrict__ tiles, const int* __restrict__ positions, int heads,
+    const float* __restrict__ sink, uint16_t* __restrict__ out, long o_row, long o_head, float scale, int window,
+    int splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, int bucket) {
+  constexpr int ENTRY = RANK + ROT, KS = ENTRY / 32, ROW = ENTRY * 2, PAGE_BYTES = 64 * ROW, NS = 4;
+  constexpr int NI = PAGE_BYTES / 4096;  // KiB of a page that a wave loads
+  constexpr int DW = RANK / 64;          // 16-channel tiles that a wave sums
+  static_assert(ENTRY % 64 == 0 && NI <= 20, "chunks are exchanged within groups of eight; three bits a load");
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, part = __builtin_amdgcn_readfirstlane(tid >> 6);  // keys and channels
+  const int c16 = lane & 15, g = lane >> 4;
+  LatTile t;
+  if (tiles) {
+    const int* e = tiles + 6 * blockIdx.x;
+    t = {e[0], e[1], e[2], e[3], e[4], e[5]};
+  } else {
+    const int runs = (heads + 63) >> 6;
+    const int row = blockIdx.x / runs, h0 = (blockIdx.x % runs) << 6;
+    t = {row, row, 1, positions[row], h0, min(64, heads - h0)};
+  }
+  if (t.seq < 0) return;
+  const int n_slots = t.n_tok * t.hcount;
+  const int n_pages = (t.pos0 + t.n_tok + PAGE - 1) / PAGE;
+  const int p_first = max(0, t.pos0 - window + 1) / PAGE;
+  const int used = tiles ? tile_ranges(t.pos0, t.n_tok, window, splits) : wide_splits(n_pages - p_first, bucket, splits);
+  const bool whole = splits == 1 || (tiles && used == 1);
+  const int per = (n_pages - p_first + used - 1) / used;
+  const int p_begin = p_first + blockIdx.y * per, p_end = min(n_pages, p_begin + per);
+  if (splits > 1 && p_begin >= p_end) {  // nothing to see: the merge passes over the record
+    if (!whole && tid < n_slots) {
+      const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + tid;
+      ws_ml[2 * rec] = -INFINITY;
+      ws_ml[2 * rec + 1] = 0.f;
+    }
+    return;
+  }
+  const int* bt = block_tables + (long)t.seq * bt_stride;
+  // chunk (4 i + part) * 64 + lane of the image comes from the chunk whose low three bits are those of lane ^ f(row): three bits a load
+  uint32_t swizzle[2] = {0, 0};
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = ((4 * i + part) * 64 + lane) / (ROW / 16);
+    swizzle[i / 10] |= (uint32_t)(((r >> 1) & 3) << 1 | ((r >> 3) & 1)) << (3 * (i % 10));
+  }
+  // the i-th KiB of this wave of page p (past the last: of no bytes)
+  auto load = [&](int p, int buf, int i) {
+    const __amdgpu_buffer_rsrc_t src =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(cache + (long)bt[min(p, p_end - 1)] * page_stride), 0, p < p_end ? PAGE_BYTES : 0, 0x00020000);
+    uint32_t f = swizzle[i / 10];
+    asm volatile("" : "+v"(f));  // (or the compiler keeps all the addresses)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)(lds + buf * PAGE_BYTES + (4 * i + part) * 1024), 16,
+                                             (int)((lane ^ ((f >> (3 * (i % 10))) & 7)) * 16), (4 * i + part) * 1024, 0, 0);
+  };
+  static_assert(NI == KS, "a load a step");
+  // The queries come through LDS, where the second page will lie: read as fragments from memory, by every wave, they were lines used by
+  // half, and took as long as two pages.  Latent parts of 1 KiB a slot, then rotated parts of 128 bytes, 16-byte chunks exchanged so that
+  // a fragment's rows lie on different banks.  (A slot past the tile reads the tile's first query, and nothing of it is stored.)
+  static_assert(RANK == 512 && ROT == 64, "a wave's load is a query's latent part or eight rotated ones");
+  char* const queries = lds + PAGE_BYTES;
+  const bool seeded = whole && sink != nullptr;
+  float seed[NS] = {0.f, 0.f, 0.f, 0.f};
+  if (seeded)  // (asked for before the rest, that nothing of it is waited for)
+#pragma unroll
+    for (int j = 0; j < NS; ++j) seed[j] = sink[t.head0 + (16 * j + c16) % t.hcount];
+  {
+    int tok = 16 * part / t.hcount, head = 16 * part - tok * t.hcount;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const bool valid = 16 * part + i < n_slots;
+      const uint16_t* const q = q_lat + (t.row0 + (valid ? tok : 0)) * ql_row + (t.head0 + (valid ? head : 0)) * ql_head;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)q, 0, RANK * 2, 0x00020000),
+                                               (__attribute__((address_space(3))) void*)(queries + (16 * part + i) * 1024), 16, (lane ^ i) * 16, 0, 0, 0);
+      if (++head == t.hcount) ++tok, head = 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int at = 16 * part + 8 * i + (lane >> 3), slot = at < n_slots ? at : 0, of = slot / t.hcount;
+      const uint16_t* const q = q_rot + (t.row0 + of) * qr_row + (t.head0 + slot - of * t.hcount) * qr_head + ((lane ^ (at >> 1)) & 7) * 8;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)q,
+                                       (__attribute__((address_space(3))) void*)(queries + 64 * 1024 + (2 * part + i) * 1024), 16, 0, 0);
+    }
+  }
+  if (p_begin < p_end)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) load(p_begin, 0, i);
+
+  const float scale2 = scale * LOG2E;
+  bf16x8 qf[NS][KS];
+  int* const last_seen = reinterpret_cast<int*>(lds + 2 * PAGE_BYTES + 9 * 1024) + c16;  // by slot
+  float m[NS], l[NS];  // l: of this lane's keys alone
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const int slot = 16 * j + c16;
+    const bool valid = slot < n_slots;
+    m[j] = seeded && valid ? seed[j] * LOG2E : -INFINITY;
+    l[j] = seeded && valid && part == 0 && g == 0 ? 1.f : 0.f;
+    if (part == 0 && g == 0) last_seen[16 * j] = valid ? t.pos0 + slot / t.hcount : -1;  // (read behind the first page's barrier)
+  }
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NI) : "memory");  // the queries have landed (a tile sees a page)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const int row = 16 * j + c16, lat = row * 1024 + ((g ^ (c16 & 3)) << 4 | (c16 & 12) << 4);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      qf[j][ks] = *reinterpret_cast<const bf16x8*>(queries + (32 * ks < RANK ? (lat ^ ((ks & 3) << 6)) + (ks >> 2) * 256
+                                                                             : 64 * 1024 + row * 128 + (((4 * ks + g) ^ (row >> 1)) & 7) * 16));
+    }
+#pragma unroll
+    for (int ks = 0; ks < RANK / 32; ++ks) asm volatile("" : "+a"(qf[j][ks]));  // in accumulator registers: the others are taken
+  }
+  f32x4 o[NS][DW];
+#pragma unroll
+  for (int j = 0; j < NS; ++j)
+#pragma unroll
+    for (int dt = 0; dt < DW; ++dt) o[j][dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  // K fragment of (this wave's key tile, step ks): row 16 part + c16, chunk 4 ks + g; V^T fragments: see latent_wide_kernel
+  const int fk = ((c16 >> 1) & 3) << 1 | (c16 >> 3);
+  const int koff = (16 * part + c16) * ROW + ((g ^ fk) << 4);
+  const int vr = 4 * g + ((lane >> 2) & 3), fv = ((vr >> 1) & 3) << 1 | (vr >> 3);
+  const int voff = vr * ROW + ((((lane & 3) >> 1) ^ fv) << 4) + (lane & 1) * 8 + part * DW * 32;
+  float* const maxima = reinterpret_cast<float*>(lds + 2 * PAGE_BYTES);                // [slot][key tile]
+  u32x2* const weights = reinterpret_cast<u32x2*>(lds + 2 * PAGE_BYTES + 1024) + lane;  // [key tile][slot tile][lane]
+  auto everyone = [&]() {  // (not __syncthreads, which would wait for the page on its way)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  for (int p = p_begin; p < p_end; ++p) {
+    const int buf = (p - p_begin) & 1;
+    const char* const img = lds + buf * PAGE_BYTES;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this page has landed; behind the barrier nobody reads the other any more
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    f32x4 s[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) s[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    {
+      constexpr int AHEAD = 3;  // the products follow the reads
+      bf16x8 kf[KS];
+      auto read_k = [&](int ks) { kf[ks] = *reinterpret_cast<const bf16x8*>(img + (koff ^ ((ks & 1) << 6)) + (ks >> 1) * 128); };
+#pragma unroll
+      for (int ks = 0; ks < AHEAD; ++ks) read_k(ks);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (ks + AHEAD < KS) read_k(ks + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NS; ++j) s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[j][ks], s[j], 0, 0, 0);
+        load(p + 1, buf ^ 1, ks);  // (all of them in front of the scores would hold those up)
+      }
+    }
+    const bool masked = p * PAGE + PAGE - 1 > t.pos0 || p * PAGE <= t.pos0 + t.n_tok - 1 - window;
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      s[j] *= scale2;
+      if (masked) {
+        const int my_pos = last_seen[16 * j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = p * PAGE + 16 * part + 4 * g + e;
+          if (key > my_pos || key <= my_pos - window) s[j][e] = -INFINITY;
+        }
+      }
+      const float mx = max_of_groups(fmaxf(fmaxf(s[j][0], s[j][1]), fmaxf(s[j][2], s[j][3])));
+      if (g == 0) maxima[(16 * j + c16) * 4 + part] = mx;
+    }
+    everyone();
+    f32x4 mx[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) mx[j] = *reinterpret_cast<const f32x4*>(maxima + (16 * j + c16) * 4);
+    float corr[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      const float mn = fmaxf(m[j], fmaxf(fmaxf(mx[j][0], mx[j][1]), fmaxf(mx[j][2], mx[j][3])));
+      const bool dead = mn == -INFINITY;
+      const float mref = dead ? 0.f : mn;
+      corr[j] = dead ? 1.f : __builtin_amdgcn_exp2f(m[j] - mref);
+      float w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_exp2f(s[j][e] - mref);
+      weights[(part * NS + j) * 64] = (u32x2){pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
+      l[j] = l[j] * corr[j] + ((w[0] + w[1]) + (w[2] + w[3]));
+      m[j] = mn;
+    }
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+      if (!__all(corr[j] == 1.f)) {
+#pragma unroll
+        for (int dt = 0; dt < DW; ++dt) o[j][dt] *= corr[j];
+      }
+    {
+      constexpr int AHEAD = 3;
+      bf16x8 vf[2 * DW], pf[2][NS];
+      auto read_v = [&](int x) {  // keys 32 (x / DW) .., channel tile x % DW
+        const char* const at = img + (voff ^ ((x & 3) << 5)) + (x % DW >> 2) * 128 + x / DW * 32 * ROW;
+        vf[x] = read_transposed_pair(at, at + 16 * ROW);
+      };
+      auto read_p = [&](int kk) {
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+          const u32x2 lo = weights[(2 * kk * NS + j) * 64], hi = weights[((2 * kk + 1) * NS + j) * 64];
+          pf[kk][j] = __builtin_bit_cast(bf16x8, (u32x4){lo[0], lo[1], hi[0], hi[1]});
+        }
+      };
+#pragma unroll
+      for (int x = 0; x < AHEAD; ++x) read_v(x);
+      everyone();
+      read_p(0);
+#pragma unroll
+      for (int x = 0; x < 2 * DW; ++x) {
+        if (x + AHEAD < 2 * DW) read_v(x + AHEAD);
+        if (x == DW - 2) read_p(1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NS; ++j) o[j][x % DW] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[x], pf[x / DW][j], o[j][x % DW], 0, 0, 0);
+      }
+    }
+  }
+
+  // the waves' and lanes' shares of the sums (nothing may still write to LDS)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    l[j] += __shfl_xor(l[j], 16, 64);
+    l[j] += __shfl_xor(l[j], 32, 64);
+    if (g == 0) maxima[(16 * j + c16) * 4 + part] = l[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const int slot = 16 * j + c16;
+    if (slot >= n_slots) continue;
+    const f32x4 all = *reinterpret_cast<const f32x4*>(maxima + (16 * j + c16) * 4);
+    const float sum = (all[0] + all[1]) + (all[2] + all[3]);
+    if (whole) {
+      const float inv = sum > 0.f ? 1.f / sum : 0.f;
+      uint16_t* dst = out + (long)(t.row0 + slot / t.hcount) * o_row + (t.head0 + slot % t.hcount) * o_head + part * DW * 16 + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < DW; ++dt)
+        *reinterpret_cast<u32x2*>(dst + 16 * dt) = (u32x2){pack_bf16x2(o[j][dt][0] * inv, o[j][dt][1] * inv),
+                                                          pack_bf16x2(o[j][dt][2] * inv, o[j][dt][3] * inv)};
+    } else {
+      const long rec = ((long)blockIdx.x * splits + blockIdx.y) * 64 + slot;
+      float* dst = ws_o + rec * RANK + part * DW * 16 + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < DW; ++dt) *reinterpret_cast<f32x4*>(dst + 16 * dt) = o[j][dt];
+      if (g == 0 && part == 0) {
+        ws_ml[2 * rec] = m[j] * LN2;
+        ws_ml[2 * rec + 1] = sum;
+      }
     }
   }
 }
@@ -686,14 +905,22 @@ int launch(const void* q_lat, long ql_row, long ql_head, const void* q_rot, long
     return *done;
   };
   if constexpr (!ROT_ONLY && RANK == 512 && ROT == 64) {
-    const int quarters = !tiles && heads <= 32;  // (a prefill tile fills its 64 slots)
-    const int lds = 2 * 64 * (RANK + ROT) * 2 + (quarters ? 8 * 1024 : 16 * 1024);
-    const auto kernel = quarters ? latent_wide_kernel<RANK, ROT, 4> : latent_wide_kernel<RANK, ROT, 2>;
-    if (!ready((const void*)kernel, lds, &attr_set[quarters])) return -2;
-    kernel<<<dim3(n_tiles, splits), dim3(512), lds, st>>>(
-        (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
-        page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
-        window, splits, ws_o, ws_ml, bucket);
+    constexpr int PAGES = 2 * 64 * (RANK + ROT) * 2;
+    if (!tiles && heads <= 32) {  // (a prefill tile fills its 64 slots)
+      const auto kernel = latent_wide_kernel<RANK, ROT>;
+      if (!ready((const void*)kernel, PAGES + 8 * 1024, &attr_set[1])) return -2;
+      kernel<<<dim3(n_tiles, splits), dim3(512), PAGES + 8 * 1024, st>>>(
+          (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
+          page_stride, block_tables, bt_stride, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale, window,
+          splits, ws_o, ws_ml, bucket);
+    } else {
+      const auto kernel = latent_tile_kernel<RANK, ROT>;
+      if (!ready((const void*)kernel, PAGES + 9 * 1024 + 256, &attr_set[0])) return -2;
+      kernel<<<dim3(n_tiles, splits), dim3(256), PAGES + 9 * 1024 + 256, st>>>(
+          (const uint16_t*)q_lat, ql_row, ql_head, (const uint16_t*)q_rot, qr_row, qr_head, (const uint16_t*)cache,
+          page_stride, block_tables, bt_stride, tiles, positions, heads, sink, (uint16_t*)out, o_row, o_head, scale,
+          window, splits, ws_o, ws_ml, bucket);
+    }
   } else {
     constexpr int LDS = 64 * ((ROT_ONLY ? ROT : RANK + ROT) * 2 + 16) + RANK * (64 * 2 + 16);
     const auto kernel = latent_mfma_kernel<RANK, ROT, ROT_ONLY>;

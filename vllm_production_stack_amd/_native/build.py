@@ -51,6 +51,7 @@ TARGETS = {
 SOURCE_FLAGS = {
     "kernels/attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels/chunk_scan.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # the state lies in accumulators and is cut up by vector instructions
+    "kernels/latent_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # the tile kernel: queries in accumulator registers, sums in the others
     "kernels/block_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # 256 registers and more: no copies between the files in the loop
 }
 # standalone executables: name -> (kind, sources, flags)

@@ -267,8 +267,9 @@ def build_latent_tiles(q_lens, ctx_lens, heads: int):
 # A work list of fewer tiles than the chip has CUs (one workgroup each) leaves the rest idle while every tile walks its pages alone,
 # and 300 tiles run as one full round and a nearly empty second.  A range costs its pages and, once, as much as about five and a half
 # (queries, the first page's way, its partial result and the merge's part of it); six where the workgroups are more than one round, and
-# eight there if the tiles see different numbers of pages, for the uncut list ends with the short ones.  13 tiles of 9 pages in one /
-# two ranges 40 / 33 us, 100 of 33 114 / 79, 150 of 9 41 / 64, 300 of 33 in one / three 230 / 206; 325 of 11 to 32 in one / two 129 / 164.
+# eight there if the tiles see different numbers of pages, for the uncut list ends with the short ones.  10 tiles of 16 pages in one /
+# four ranges 49 / 26 us, 30 of 125 in one / eight / nine 300 / 60 / 95, 150 of 47 in one / two / three 123 / 142 / 114, 300 of 125 in one /
+# three 571 / 447; 260 of 28 to 32 in one / two 138 / 146, 550 of 46 to 63 403 / 410.
 LATENT_RANGE_ALONE, LATENT_RANGE_EVEN, LATENT_RANGE_UNEVEN = 5.5, 6, 8
 LATENT_RANGE_MIN_PAGES = 4
 
