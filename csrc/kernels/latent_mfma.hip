@@ -282,9 +282,8 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //     one maximum for all 64 keys the error against 64 bits was 2.03e-3 on average over batches and contexts, with a maximum for
 //     each quarter 1.97e-3, with two parts it is 1.66e-3, the rounding of the result.
 //   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
-// Decode rows with their merge, in a graph, pages from memory; staged through registers / this: 32 heads, 32 sequences of 4k entries in 8
-// ranges 65 / 40 us, 8 of 8k in 32 42 / 32, one of 26k in 32 86 / 49, one of 3k 22.9 / 21.0, one of 2k, a page a range, 17.4 / 18.0; 16 heads,
-// one of 2k 16.1 / 15.4.
+// Decode rows with their merge, pages from memory, staged through registers / this: 32 heads, 32 sequences of 4k entries in 8 ranges
+// 65 / 35 us, 8 of 8k in 32 42 / 27, one of 26k in 32 86 / 45.
 
 // o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
 // their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
@@ -363,16 +362,28 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
   const bool wave_active = sg * 16 < heads;  // wave-uniform
   const float scale2 = scale * LOG2E;
   const int head = valid ? slot : 0;
-  // (a slot past the heads reads the first one's query, and nothing of it is stored: no branch, no select.)  In a single round every
-  // range may be used, and the queries are on their way while the row's position and page are looked up (one sequence of 2k entries
-  // 18.6 -> 17.7 us); with more, most of the workgroups have nothing to do (100 x 400 entries 37 -> 31 if they don't load them).
-  bf16x8 qf[KS];
+  // The queries come through LDS, where the second page will lie: latent parts of 1 KiB, then rotated parts of 128 bytes, 16-byte chunks
+  // exchanged so that a fragment's rows lie on different banks.  (Four waves read the same 16 rows, and a fragment read from memory takes
+  // half of every line; with the second page asked for only behind these reads, 32 sequences of 4k entries, 32 heads, still take 38.7 ->
+  // 35.3 us, 100 of 1000 40.1 -> 36.7, one of 26k 48.4 -> 44.9; 16 heads 31.4 -> 29.1, 30.0 -> 27.3, 37.0 -> 34.5.)  In a single round
+  // every range may be used, and the queries are on their way while the row's position and page are looked up (one sequence of 2k
+  // entries 18.6 -> 17.7 us); with more, most of the workgroups have nothing to do (100 x 400 entries 37 -> 31 if they don't load them).
+  static_assert(RANK == 512 && ROT == 64, "a wave's load is a query's latent part or eight rotated ones");
+  char* const queries = lds + PAGE_BYTES;
   auto load_q = [&]() {
+    const uint16_t* const ql = q_lat + (long)row * ql_row;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int d = 32 * ks + 8 * g;
-      qf[ks] = __builtin_bit_cast(
-          bf16x8, 32 * ks < RANK ? ld16(q_lat + (long)row * ql_row + head * ql_head + d) : ld16(q_rot + (long)row * qr_row + head * qr_head + (d - RANK)));
+    for (int i = 0; i < 4; ++i) {
+      const int of = 4 * wave + i;
+      if (of < heads)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)(ql + of * ql_head), 0, RANK * 2, 0x00020000),
+                                                 (__attribute__((address_space(3))) void*)(queries + of * 1024), 16, (lane ^ (of & 15)) * 16, 0, 0, 0);
+    }
+    if (wave < 4) {
+      const int at = 8 * wave + (lane >> 3);
+      const uint16_t* const q = q_rot + (long)row * qr_row + (at < heads ? at : 0) * qr_head + ((lane ^ (at >> 1)) & 7) * 8;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)q,
+                                       (__attribute__((address_space(3))) void*)(queries + 32 * 1024 + wave * 1024), 16, 0, 0);
     }
   };
   const bool all_used = bucket * splits <= 256;
@@ -387,6 +398,7 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
       ws_ml[2 * rec] = -INFINITY;
       ws_ml[2 * rec + 1] = 0.f;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (nothing may still be on its way to LDS)
     return;
   }
   if (!all_used) load_q();
@@ -424,6 +436,7 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
   for (int i = 0; i < 4; ++i)
     voff[i] = vr * ROW + (((2 * i + ((lane & 3) >> 1)) ^ fv) << 4) + (lane & 1) * 8 + part * DW * 32;
 
+  bf16x8 qf[KS];
   f32x4 s[4];  // scores, then weights, of a page's keys
   auto score = [&](int buf) {
     const char* img = lds + buf * PAGE_BYTES;
@@ -490,8 +503,19 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     asm volatile("" ::: "memory");
   };
 
-  if (p_begin < p_end) load_page(p_begin, 0);
-  if (p_begin + 1 < p_end) load_page(p_begin + 1, 1);
+  if (p_begin < p_end) {
+    load_page(p_begin, 0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");  // the queries have landed
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int of = valid ? slot : 0, lat = of * 1024 + ((g ^ (of & 3)) << 4 | (of & 12) << 4);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = *reinterpret_cast<const bf16x8*>(queries + (32 * ks < RANK ? (lat ^ ((ks & 3) << 6)) + (ks >> 2) * 256
+                                                                          : 32 * 1024 + of * 128 + (((4 * ks + g) ^ (of >> 1)) & 7) * 16));
+    everyone();
+    if (p_begin + 1 < p_end) load_page(p_begin + 1, 1);
+  }
   for (int p = p_begin; p < p_end; ++p) {
     const int buf = (p - p_begin) & 1;
     const uint32_t page = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + buf * PAGE_BYTES;
