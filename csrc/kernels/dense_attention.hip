@@ -147,7 +147,7 @@ VPSA_EXPORT int vpsa_dense_decode_attention(const void* q, long q_bs, const void
 // attending to each other; decoder prompt rows attending to the encoder output).
 //
 // One workgroup = 4 waves x 32 query rows against 64-key tiles staged through LDS (double
-// buffered: the next tile's global loads are in flight during the current tile's math, one
+// buffered: the next tile is on its way to LDS during the current tile's math, one
 // barrier per tile).  Per wave and tile:
 //   S^T[64 keys x 32 queries] = K_tile . Q^T        8 x v_mfma_f32_32x32x16_bf16, K rows from LDS
 //                                                   (ds_read_b128), Q^T fragments kept in registers
@@ -157,16 +157,18 @@ VPSA_EXPORT int vpsa_dense_decode_attention(const void* q, long q_bs, const void
 //                                                   they are; V stays row-major in LDS and is read
 //                                                   through the transposing ds_read_b64_tr_b16, whose
 //                                                   4-key blocks are exactly the accumulator's key order
-// A wave and tile cost 512 cycles of matrix instructions, 512 of exponentials and 640 of other vector work, in 1900 (vector
-// units 55 % busy, matrix units 27 %), so what bounds this is how well they overlap, and 1152 workgroups are one and a half
-// rounds of 768.  Rows of 128 B without padding (K's 16-byte chunks are swapped by key bits 1..3, V's halves by key bit 1: both
-// kinds of read stay free of bank conflicts) and 144 registers let three workgroups share a CU; padded rows and 177 registers
-// held two.  The scale goes into the exponent's fused multiply, the mask only touches the last tile, and a window's query
-// blocks run on one XCD.  Measured: 8 windows x 12 heads x 1500 positions 153 -> 97 us, 2 windows 55.5 -> 41, 32 windows x 8
-// heads 324 -> 225.  Then, with the queries waited for before the loop, K read two products ahead, the mask in a tile of its
+// A wave and tile cost 512 cycles of matrix instructions, 512 of exponentials and 640 of other vector work, in 1500 where the chip
+// is full (32 windows x 12 heads), so vector work bounds this.  Rows of 128 B without padding (K's 16-byte chunks are swapped by key
+// bits 1..3, V's halves by key bit 1: both kinds of read stay free of bank conflicts) and tiles that go to LDS without passing
+// through registers (122 instead of 138) let four workgroups share a CU.  Of 8 windows x 12 heads the last 128 of 1152 workgroups
+// then run alone, 26 us for what takes 16 beside others.  (The next tile's scores under this one's exponentials need 182
+// registers: two workgroups a CU, 23.4 us for one window instead of 26.5 but 91 for 8 and 305 for 32.)  The scale goes into the
+// exponent's fused multiply, the mask only touches the last tile, and a window's query blocks run on one XCD.  Measured: 8
+// windows x 12 heads x 1500 positions 153 -> 97 us, 2 windows 55.5 -> 41, 32 windows x 8 heads 324 -> 225.  Then, with the queries waited for before the loop, K read two products ahead, the mask in a tile of its
 // own and a slice's products under the next slice's exponentials: 97.3 -> 94.1 (0.59 PFLOP/s), one window 31.0 -> 28.9, four
-// query rows 32 -> 26, 32 windows x 8 heads 225 -> 219.  Four workgroups a CU (128 registers, 16 spilled): 104 us.  A maximum
-// that follows only in steps of 2^8 is no faster and rounds the largest probability: error 1.9e-3 -> 2.3e-3.
+// query rows 32 -> 26, 32 windows x 8 heads 225 -> 219.  Then, with tiles straight into LDS and four workgroups instead of three:
+// 93.1 -> 87.7, 32 windows x 12 heads 303 -> 284, two 38.7 -> 36.9, one 27.5 -> 26.5.  A
+// maximum that follows only in steps of 2^8 is no faster and rounds the largest probability: error 1.9e-3 -> 2.3e-3.
 // The [B, heads, Tq, Tk] score matrix never exists in memory.
 #define DF_KT 64
 
@@ -180,13 +182,23 @@ __device__ __forceinline__ bf16x8 lds_tr_pair(const uint16_t* lo, const uint16_t
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-__global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
+// 16 bytes a lane from global memory into LDS, in lane order from `to`.  In assembly because the compiler waits for all loads of the builtin
+// in front of any read from LDS; whoever reads what is loaded waits for it.  (A scalar register that a vector instruction wrote may be read
+// five states later.)
+__device__ __forceinline__ void load_to_lds(const void* src, uint32_t to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to) : "m0", "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const uint16_t* at) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint16_t*)at;
+}
+
+__global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
     const uint16_t* __restrict__ q, long q_bs, long q_ts, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, long kv_bs, long kv_ts, uint16_t* __restrict__ out, long o_bs,
     long o_ts, int Tq, int Tk, int heads, int pairs, int q_blocks, float scale_log2e) {
   __shared__ __attribute__((aligned(16))) uint16_t lds_k[2][DF_KT * 64];
   __shared__ __attribute__((aligned(16))) uint16_t lds_v[2][DF_KT * 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hf = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 31, hf = lane >> 5;
   // workgroups go round the eight XCDs: one pair's query blocks follow each other on one of them and share its L2
   const int at = blockIdx.x >> 3, pair = at / q_blocks * 8 + (blockIdx.x & 7);
   if (pair >= pairs) return;
@@ -200,27 +212,29 @@ __global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
 
   const uint16_t* kbase_p = k + b * kv_bs + h * 64;
   const uint16_t* vbase_p = v + b * kv_bs + h * 64;
-  const int srow = tid >> 3, sc = tid & 7;
-  u32x4 kreg[2], vreg[2];
-  auto stage_load = [&](int t) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      int key = t * DF_KT + srow + 32 * i;
-      key = key < Tk ? key : Tk - 1;
-      kreg[i] = *(const u32x4*)(kbase_p + (long)key * kv_ts + 8 * sc);
-      vreg[i] = *(const u32x4*)(vbase_p + (long)key * kv_ts + 8 * sc);
-    }
-  };
-  auto stage_write = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      *(u32x4*)(&lds_k[buf][(srow + 32 * i) * 64 + 8 * (sc ^ ((srow >> 1) & 7))]) = kreg[i];
-      *(u32x4*)(&lds_v[buf][(srow + 32 * i) * 64 + 8 * (sc ^ ((srow & 2) << 1))]) = vreg[i];
-    }
-  };
   const int n_tiles = (Tk + DF_KT - 1) / DF_KT;
-  stage_load(0);
-  stage_write(0);
+  // A wave's load is eight keys' rows: keys 8 wave .. and 32 further of a tile.  LDS is filled in lane order, so the chunks are swapped
+  // on the way there: the source of chunk c of key j is K's c ^ (j / 2 % 8), V's c ^ (j % 4 / 2 * 4).
+  const int row0 = 8 * wave + (lane >> 3);
+  const int kc = 8 * ((lane & 7) ^ ((row0 >> 1) & 7)), vc = 8 * ((lane & 7) ^ ((row0 & 2) << 1));
+  const long row_step = kv_ts * 32;
+  const uint16_t *ksrc = kbase_p + row0 * kv_ts + kc, *vsrc = vbase_p + row0 * kv_ts + vc;
+  auto stage = [&](int t) {
+    const int buf = t & 1;
+    const uint16_t *k1 = ksrc + row_step, *v1 = vsrc + row_step;
+    if (t == n_tiles - 1) {  // keys past the last read the last one
+      const long back0 = max(0, t * DF_KT + row0 - (Tk - 1)) * kv_ts, back1 = max(0, t * DF_KT + row0 + 32 - (Tk - 1)) * kv_ts;
+      ksrc -= back0, vsrc -= back0, k1 -= back1, v1 -= back1;
+    }
+    const uint32_t kd = lds_address(&lds_k[buf][512 * wave]), vd = lds_address(&lds_v[buf][512 * wave]);
+    load_to_lds(ksrc, kd);
+    load_to_lds(vsrc, vd);
+    load_to_lds(k1, kd + 4096);
+    load_to_lds(v1, vd + 4096);
+    ksrc = k1 + row_step, vsrc = v1 + row_step;
+  };
+  stage(0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   // The queries have arrived before the loop: waited for at their first use inside it, every tile would wait there, and with them
   // for the tile that is being loaded.
@@ -240,7 +254,7 @@ __global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
 
   auto tile = [&](int t, auto masked) {
     const int buf = t & 1;
-    if (!masked.value) stage_load(t + 1);
+    if (!masked.value) stage(t + 1);
     // the products follow the reads at a distance of two
     f32x16 s_acc[2];
     bf16x8 kf[8], vf[4][2];
@@ -308,7 +322,7 @@ __global__ __launch_bounds__(256, 3) void dense_attn_fwd_kernel(
         o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[s4][cb], __builtin_bit_cast(bf16x8, pk), o_acc[cb], 0, 0, 0);
     }
     l_run = l_run * alpha + psum;
-    if (!masked.value) stage_write(buf ^ 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tile has landed
     __syncthreads();
   };
   for (int t = 0; t + 1 < n_tiles; ++t) tile(t, std::false_type{});
