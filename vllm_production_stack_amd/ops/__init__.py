@@ -177,9 +177,9 @@ def layer_norm(x, weight, bias, eps, residual=None):
     if (x.is_cuda and 0 < hidden <= 2048 and hidden % 8 == 0 and rows_at % 8 == 0 and weight is not None and bias is not None
             and weight.shape == bias.shape == (hidden,) and weight.is_contiguous() and bias.is_contiguous()
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1))
+            and not _followed(x, weight, bias, residual)  # (before the addresses, which a function transform's tensors have not)
             and (residual is None or (residual.is_contiguous() and residual.shape == x.shape and _lies_with(x, residual)))
-            and _lies_with(x, x) and _lies_with(x, weight) and _lies_with(x, bias)
-            and not _followed(x, weight, bias, residual)):
+            and _lies_with(x, x) and _lies_with(x, weight) and _lies_with(x, bias)):
         y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         rc = _kernels().vpsa_layernorm(x.data_ptr(), _at(residual), weight.data_ptr(), bias.data_ptr(), y.data_ptr(), x.numel() // hidden,
                                        hidden, rows_at, eps, _raw_stream())
