@@ -96,3 +96,28 @@ def test_dispatch():
         assert not ops._tile_takes(x, w)
     finally:
         ops.set_tile_gemm(old)
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_calls_that_something_follows_stay_with_the_library():
+    """Gradients, forward-mode tangents, vmap and traces at rows that only the rule for cut tails takes; bias, residual and gated products."""
+    from torch.autograd import forward_ad
+
+    x, w, g = _inputs(600, 4096, 8192)
+    b, t = torch.randn(4096, generator=g, device=DEV).to(BF), torch.randn(600, 8192, generator=g, device=DEV).to(BF)
+    assert ops._tile_takes(x, w, False, b) and not ops.tile_rows(x, w)
+    lib = torch.nn.functional.linear
+    with torch.enable_grad():
+        leaf = b.clone().requires_grad_()
+        ops.linear(x, w, leaf).sum().backward()
+        assert torch.equal(leaf.grad, torch.full_like(b, 600))
+    with torch.no_grad(), forward_ad.dual_level():
+        assert torch.equal(forward_ad.unpack_dual(ops.linear(forward_ad.make_dual(x, t), w, b)).tangent, lib(t, w))
+    with torch.no_grad():
+        xs = torch.stack([x, t])
+        assert torch.func.vmap(lambda q: ops.linear(q, w, b))(xs).shape == (2, 600, 4096)
+        taken = []
+        torch.func.vmap(lambda q: taken.append(ops._tile_takes(q, w, True)) or q)(xs)
+        assert taken == [False]
+        traced = torch.jit.trace(lambda q: ops.linear(q, w, b), (x,), check_trace=False)
+        assert torch.equal(traced(t), lib(t, w, b))

@@ -1099,7 +1099,7 @@ def _tile_takes(x, w, pair: bool = False, *others) -> bool:
         return True
     if not (_tile_enabled and x.is_cuda and x.dim() == 2 and x.shape[0] >= TILE_TAIL_ROWS and w.dim() == 2
             and x.shape[1] == w.shape[1] and tile_gemm_supported(w.shape[0], w.shape[1], pair) and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.is_contiguous() and all(t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0)
+            and w.is_contiguous() and not _followed(x, w, *others) and all(t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0)
                                           for t in (x, w, *others))
             and x.shape[0] * x.stride(0) < 1 << 31):
         return False
@@ -1109,7 +1109,7 @@ def _tile_takes(x, w, pair: bool = False, *others) -> bool:
         takes = splits > 1 and tiles >= TILE_CUS or tiles >= TILE_PAIR_FILL * TILE_CUS * -(-tiles // TILE_CUS)
     else:
         takes = splits > 1 and (k >= 64 * TILE_LONG_CHUNKS or (tiles >= TILE_CUS and splits >= TILE_TAIL_SPLITS))
-    return takes and not _followed(x, w, *others)
+    return takes
 
 
 def linear(x, w, bias=None, packed=None):
