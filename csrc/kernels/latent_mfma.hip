@@ -29,6 +29,8 @@
 // Softmax state (running max, sum) is fp32 per slot, scores in powers of two; an optional per-head sink logit starts the state
 // (max = sink, sum = 1).  With key-range splits every split writes unnormalised partial outputs and
 // (max, sum) to a workspace and a merge kernel adds the sink and normalises.
+#include <float.h>
+
 #include "common.h"
 
 namespace {
@@ -580,9 +582,14 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
 //   * Nothing but the order of instructions hides a wait: reads run three fragments in front of their products, the next page's loads
 //     go out one a step of the scores (all at once, they held those up), and rows past the list's last page load no bytes.
 //   * Queries come through LDS (below): 5 us a workgroup less than as fragments from memory.
-// 2.3 us a page.  32 heads: 2000 rows behind 6000 entries 1399 -> 1070 us, 2000 of one sequence 248 -> 200, 600 behind 7400 565 -> 447,
-// 200 behind 3800 122 -> 98, 20 behind 1980 32.7 -> 29.6; 16 heads, 60 behind 7940 47.0 -> 41.4; decode rows, 32 sequences of 4k
-// entries, 64 heads 49.7 -> 42.7, 128 heads 76.6 -> 63.0.  Errors against 64 bits are what they were, to five digits.
+//   * Nothing runs beside a lone wave's vector instructions, so those between the two products count in full, 1 % of the time for
+//     every 20: the four slot tiles' maxima over lane groups take three swaps together, scores are scaled where they are weighed, one
+//     branch holds masks and negative scales, the state starts at a finite number, a wave's weights lie as the second product reads them
+//     (2000 rows behind 6000 entries 1070 -> 919 us, 60 behind 7940 59.6 -> 54.7).  Reads of the next page's keys or of the values further
+//     ahead, and the page's loads in the first half of the scores, are slower by 0 to 2 %.
+// 2.1 us a page.  32 heads: 2000 rows behind 6000 entries 1399 -> 919 us, 2000 of one sequence 248 -> 178, 600 behind 7400 565 -> 390,
+// 200 behind 3800 122 -> 88, 20 behind 1980 32.7 -> 27.6; 16 heads, 60 behind 7940 47.0 -> 38.4; decode rows, 32 sequences of 4k
+// entries, 64 heads 49.7 -> 41, 128 heads 76.6 -> 61.  Errors against 64 bits are what they were, to four digits.
 // Lists of few tiles are cut along the keys (ops/latent.py).
 __device__ __forceinline__ bf16x8 read_transposed_pair(const char* lo, const char* hi) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -592,12 +599,27 @@ __device__ __forceinline__ bf16x8 read_transposed_pair(const char* lo, const cha
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-__device__ __forceinline__ float max_of_groups(float x) {  // over the lanes c, c + 16, c + 32, c + 48
-  const uint32_t u = __float_as_uint(x);
-  const auto far = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const uint32_t v = __float_as_uint(fmaxf(__uint_as_float(far[0]), __uint_as_float(far[1])));
-  const auto near = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  return fmaxf(__uint_as_float(near[0]), __uint_as_float(near[1]));
+// (In assembly where a value comes from another lane or from LDS: the compiler would quieten it first, two instructions more for one.)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float max_of_swapped(uint32_t a, uint32_t b) {  // (two states before a swap reads what a vector instruction wrote)
+  float r;
+  asm("v_max_f32 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// Lane group g: the maximum of x[g] over the four groups' lanes of one number.  Swapping halves of two values leaves two of their four
+// parts in each half, and then swapping groups of 16 lanes the four values in the four groups.
+__device__ __forceinline__ float max_of_groups(const float (&x)[4]) {
+  const auto half = [](float a, float b) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return max_of_swapped(both[0], both[1]);
+  };
+  const float even = half(x[0], x[2]), odd = half(x[1], x[3]);
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(even), __float_as_uint(odd), false, false);
+  return max_of_swapped(both[0], both[1]);
 }
 
 template <int RANK, int ROT>
@@ -689,7 +711,7 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
 #pragma unroll
     for (int i = 0; i < NI; ++i) load(p_begin, 0, i);
 
-  const float scale2 = scale * LOG2E;
+  const float scale2 = fmaxf(fabsf(scale) * LOG2E, FLT_MIN);  // (maxima and masks come before it: positive, and the scores' sign where it is not)
   bf16x8 qf[NS][KS];
   int* const last_seen = reinterpret_cast<int*>(lds + 2 * PAGE_BYTES + 9 * 1024) + c16;  // by slot
   float m[NS], l[NS];  // l: of this lane's keys alone
@@ -697,7 +719,7 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
   for (int j = 0; j < NS; ++j) {
     const int slot = 16 * j + c16;
     const bool valid = slot < n_slots;
-    m[j] = seeded && valid ? seed[j] * LOG2E : -INFINITY;
+    m[j] = seeded && valid ? fmaxf(seed[j] * LOG2E, -FLT_MAX) : -FLT_MAX;  // (finite: a page of which a slot sees nothing needs no care)
     l[j] = seeded && valid && part == 0 && g == 0 ? 1.f : 0.f;
     if (part == 0 && g == 0) last_seen[16 * j] = valid ? t.pos0 + slot / t.hcount : -1;  // (read behind the first page's barrier)
   }
@@ -727,7 +749,7 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
   const int vr = 4 * g + ((lane >> 2) & 3), fv = ((vr >> 1) & 3) << 1 | (vr >> 3);
   const int voff = vr * ROW + ((((lane & 3) >> 1) ^ fv) << 4) + (lane & 1) * 8 + part * DW * 32;
   float* const maxima = reinterpret_cast<float*>(lds + 2 * PAGE_BYTES);                // [slot][key tile]
-  u32x2* const weights = reinterpret_cast<u32x2*>(lds + 2 * PAGE_BYTES + 1024) + lane;  // [key tile][slot tile][lane]
+  u32x4* const weights = reinterpret_cast<u32x4*>(lds + 2 * PAGE_BYTES + 1024) + lane;  // [keys 32 ..][slot tile][lane][16 of the keys]
   auto everyone = [&]() {  // (not __syncthreads, which would wait for the page on its way)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -759,10 +781,10 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
       }
     }
     const bool masked = p * PAGE + PAGE - 1 > t.pos0 || p * PAGE <= t.pos0 + t.n_tok - 1 - window;
+    if (masked || scale < 0.f) {
 #pragma unroll
-    for (int j = 0; j < NS; ++j) {
-      s[j] *= scale2;
-      if (masked) {
+      for (int j = 0; j < NS; ++j) {
+        if (scale < 0.f) s[j] = -s[j];
         const int my_pos = last_seen[16 * j];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -770,9 +792,11 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
           if (key > my_pos || key <= my_pos - window) s[j][e] = -INFINITY;
         }
       }
-      const float mx = max_of_groups(fmaxf(fmaxf(s[j][0], s[j][1]), fmaxf(s[j][2], s[j][3])));
-      if (g == 0) maxima[(16 * j + c16) * 4 + part] = mx;
     }
+    float top[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) top[j] = fmaxf(fmaxf(s[j][0], s[j][1]), fmaxf(s[j][2], s[j][3]));
+    maxima[lane * 4 + part] = max_of_groups(top) * scale2;
     everyone();
     f32x4 mx[NS];
 #pragma unroll
@@ -780,14 +804,12 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
     float corr[NS];
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-      const float mn = fmaxf(m[j], fmaxf(fmaxf(mx[j][0], mx[j][1]), fmaxf(mx[j][2], mx[j][3])));
-      const bool dead = mn == -INFINITY;
-      const float mref = dead ? 0.f : mn;
-      corr[j] = dead ? 1.f : __builtin_amdgcn_exp2f(m[j] - mref);
+      const float mn = max3(max3(m[j], mx[j][0], mx[j][1]), mx[j][2], mx[j][3]);
+      corr[j] = __builtin_amdgcn_exp2f(m[j] - mn);
       float w[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_exp2f(s[j][e] - mref);
-      weights[(part * NS + j) * 64] = (u32x2){pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
+      for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_exp2f(fmaf(s[j][e], scale2, -mn));
+      reinterpret_cast<u32x2*>(weights + ((part >> 1) * NS + j) * 64)[part & 1] = (u32x2){pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
       l[j] = l[j] * corr[j] + ((w[0] + w[1]) + (w[2] + w[3]));
       m[j] = mn;
     }
@@ -806,10 +828,7 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
       };
       auto read_p = [&](int kk) {
 #pragma unroll
-        for (int j = 0; j < NS; ++j) {
-          const u32x2 lo = weights[(2 * kk * NS + j) * 64], hi = weights[((2 * kk + 1) * NS + j) * 64];
-          pf[kk][j] = __builtin_bit_cast(bf16x8, (u32x4){lo[0], lo[1], hi[0], hi[1]});
-        }
+        for (int j = 0; j < NS; ++j) pf[kk][j] = __builtin_bit_cast(bf16x8, weights[(kk * NS + j) * 64]);
       };
 #pragma unroll
       for (int x = 0; x < AHEAD; ++x) read_v(x);

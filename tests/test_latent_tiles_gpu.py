@@ -78,3 +78,16 @@ def test_no_sink_a_sink_of_no_weight_and_a_nan():
     assert bool(got2[3, 2].isnan().all())
     got2[3, 2] = got[0][3, 2]
     assert torch.equal(got2, got[0])
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 1e-42])
+def test_scales_of_any_sign(scale):
+    """Scores turn their order with a negative scale and mean nothing with one of zero; a window that some pages' slots see nothing of."""
+    rows_of, ctx, heads = [40, 5], [300, 5], 16
+    pool, table, q, sink = setup(ctx, rows_of, heads, 11)
+    seq = torch.tensor([0] * 40 + [1] * 5, dtype=torch.int32, device=DEV)
+    pos = torch.cat([torch.arange(c - n, c, dtype=torch.int32) for c, n in zip(ctx, rows_of)]).to(DEV)
+    tiles = torch.from_numpy(ops.build_latent_tiles(rows_of, ctx, heads)).to(DEV)
+    for window in (1 << 30, 66):
+        got = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, seq, pos, sink, scale, tiles=tiles, window=window)
+        close(got, pool, table, q, sink, ctx, rows_of, scale, window)
