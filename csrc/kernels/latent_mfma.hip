@@ -284,8 +284,11 @@ __global__ __launch_bounds__(256, RANK + ROT <= 256 && RANK <= 128 ? 3 : 1) void
 //     one maximum for all 64 keys the error against 64 bits was 2.03e-3 on average over batches and contexts, with a maximum for
 //     each quarter 1.97e-3, with two parts it is 1.66e-3, the rounding of the result.
 //   * Decode rows read a page once: non-temporal loads (5.6 against 4.5 TB/s without the arithmetic).
+//     The exchange, softmax and second product of a page stand between its last read and the next one's first: maxima over lane groups
+//     by lane swaps instead of through LDS, sums kept by lane until the end, scores scaled where they are weighed (32 heads, one sequence of
+//     26k entries 44.7 -> 40.8 us, 200 of 2k 98.6 -> 93.5, 32 of 4k 35.4 -> 34.3; 16 heads, one of 26k 34.5 -> 30.4).
 // Decode rows with their merge, pages from memory, staged through registers / this: 32 heads, 32 sequences of 4k entries in 8 ranges
-// 65 / 35 us, 8 of 8k in 32 42 / 27, one of 26k in 32 86 / 45.
+// 65 / 34 us, 8 of 8k in 32 42 / 26, one of 26k in 32 86 / 41.
 
 // o[dt] += V^T fragment of d tile dt x P^T.  In assembly because the compiler makes the builtin wait for the pages that are on
 // their way into LDS; the reads are waited for in the block that issues them.  32 keys: two transposed reads of 4 keys x 16
@@ -342,6 +345,36 @@ __device__ __forceinline__ int wide_splits(int pages, int rows, int splits) {
   return used;
 }
 
+// (In assembly where a value comes from another lane or from LDS: the compiler would quieten it first, two instructions more for one.)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float max_of_swapped(uint32_t a, uint32_t b) {  // (two states before a swap reads what a vector instruction wrote)
+  float r;
+  asm("v_max_f32 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// The maximum over the lanes c, c + 16, c + 32, c + 48.
+__device__ __forceinline__ float max_of_groups(float x) {
+  const auto far = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const uint32_t half = __float_as_uint(max_of_swapped(far[0], far[1]));
+  const auto near = __builtin_amdgcn_permlane16_swap(half, half, false, false);
+  return max_of_swapped(near[0], near[1]);
+}
+// Lane group g: the maximum of x[g] over the four groups' lanes of one number.  Swapping halves of two values leaves two of their four
+// parts in each half, and then swapping groups of 16 lanes the four values in the four groups.
+__device__ __forceinline__ float max_of_groups(const float (&x)[4]) {
+  const auto half = [](float a, float b) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return max_of_swapped(both[0], both[1]);
+  };
+  const float even = half(x[0], x[2]), odd = half(x[1], x[3]);
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(even), __float_as_uint(odd), false, false);
+  return max_of_swapped(both[0], both[1]);
+}
+
 // Decode rows of at most 32 heads.
 template <int RANK, int ROT>
 __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
@@ -362,7 +395,7 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
   const int pos = positions[row];
   const bool valid = slot < heads;
   const bool wave_active = sg * 16 < heads;  // wave-uniform
-  const float scale2 = scale * LOG2E;
+  const float scale2 = fmaxf(fabsf(scale) * LOG2E, FLT_MIN);  // (as in the kernel behind this one)
   const int head = valid ? slot : 0;
   // The queries come through LDS, where the second page will lie: latent parts of 1 KiB, then rotated parts of 128 bytes, 16-byte chunks
   // exchanged so that a fragment's rows lie on different banks.  (Four waves read the same 16 rows, and a fragment read from memory takes
@@ -421,8 +454,8 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
                                        16, 0, 2);  // 2: non-temporal
   };
   const bool seeded = splits == 1 && sink != nullptr && valid;
-  float m = seeded ? sink[head] * LOG2E : -INFINITY;
-  float l = seeded ? 1.f : 0.f;
+  float m = seeded ? fmaxf(sink[head] * LOG2E, -FLT_MAX) : -FLT_MAX;
+  float l = seeded && g == 0 ? 1.f : 0.f;  // of this lane's keys alone
   f32x4 o[DW];
 #pragma unroll
   for (int dt = 0; dt < DW; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -448,40 +481,33 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
       s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(img + koff[ks & 1] + (ks >> 1) * 128), qf[ks], s[0], 0, 0, 0);
   };
   auto weigh = [&](int p) {
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) s[nt] *= scale2;
-    if (p * PAGE + PAGE - 1 > pos || p * PAGE <= pos - window) {
+    if (scale < 0.f || p * PAGE + PAGE - 1 > pos || p * PAGE <= pos - window) {
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+          if (scale < 0.f) s[nt][e] = -s[nt][e];
           const int key = p * PAGE + 16 * nt + 4 * g + e;
           if (key > pos || key <= pos - window) s[nt][e] = -INFINITY;
         }
     }
-    float mx = -INFINITY;
+    float mx = max3(s[0][0], s[0][1], s[0][2]);
+    mx = max3(mx, s[0][3], s[1][0]);
+    mx = max3(mx, s[1][1], s[1][2]);
+    mx = max3(mx, s[1][3], s[2][0]);
+    mx = max3(mx, s[2][1], s[2][2]);
+    mx = max3(mx, s[2][3], s[3][0]);
+    mx = max3(mx, s[3][1], s[3][2]);
+    const float mn = fmaxf(m, max_of_groups(max3(mx, s[3][3], s[3][3])) * scale2);
+    const float corr = __builtin_amdgcn_exp2f(m - mn);
+    float ps[4];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < 4; ++nt) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[nt][e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);
-    const bool dead = mn == -INFINITY;
-    const float mref = dead ? 0.f : mn;
-    const float corr = dead ? 1.f : __builtin_amdgcn_exp2f(m - mref);
-    float ps = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float pv = __builtin_amdgcn_exp2f(s[nt][e] - mref);
-        s[nt][e] = pv;
-        ps += pv;
-      }
-    ps += __shfl_xor(ps, 16, 64);
-    ps += __shfl_xor(ps, 32, 64);
-    l = l * corr + ps;
+      for (int e = 0; e < 4; ++e) s[nt][e] = __builtin_amdgcn_exp2f(fmaf(s[nt][e], scale2, -mn));
+      ps[nt] = (s[nt][0] + s[nt][1]) + (s[nt][2] + s[nt][3]);
+    }
+    l = l * corr + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
     m = mn;
     if (!__all(corr == 1.f)) {
 #pragma unroll
@@ -551,6 +577,8 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
     }
   }
 
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
   if (!valid) return;
   if (splits == 1) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -597,29 +625,6 @@ __device__ __forceinline__ bf16x8 read_transposed_pair(const char* lo, const cha
   const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)lo);
   const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)hi);
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-// (In assembly where a value comes from another lane or from LDS: the compiler would quieten it first, two instructions more for one.)
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-__device__ __forceinline__ float max_of_swapped(uint32_t a, uint32_t b) {  // (two states before a swap reads what a vector instruction wrote)
-  float r;
-  asm("v_max_f32 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-// Lane group g: the maximum of x[g] over the four groups' lanes of one number.  Swapping halves of two values leaves two of their four
-// parts in each half, and then swapping groups of 16 lanes the four values in the four groups.
-__device__ __forceinline__ float max_of_groups(const float (&x)[4]) {
-  const auto half = [](float a, float b) {
-    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return max_of_swapped(both[0], both[1]);
-  };
-  const float even = half(x[0], x[2]), odd = half(x[1], x[3]);
-  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(even), __float_as_uint(odd), false, false);
-  return max_of_swapped(both[0], both[1]);
 }
 
 template <int RANK, int ROT>

@@ -91,3 +91,14 @@ def test_scales_of_any_sign(scale):
     for window in (1 << 30, 66):
         got = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, seq, pos, sink, scale, tiles=tiles, window=window)
         close(got, pool, table, q, sink, ctx, rows_of, scale, window)
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 1e-42])
+@pytest.mark.parametrize("heads,splits", [(16, 1), (32, 3)])
+def test_decode_rows_with_scales_of_any_sign(scale, heads, splits):
+    ctx = [1, 64, 65, 500]
+    pool, table, q, sink = setup(ctx, [1] * len(ctx), heads, heads)
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    for window in (1 << 30, 70):
+        got = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, None, pos, sink, scale, splits=splits, window=window)
+        close(got, pool, table, q, sink, ctx, [1] * len(ctx), scale, window)
