@@ -375,6 +375,17 @@ __device__ __forceinline__ float max_of_groups(const float (&x)[4]) {
   return max_of_swapped(both[0], both[1]);
 }
 
+// Scores are scaled behind their masks and maxima: by a positive number, their sign turned before where the scale is negative.  (Comparisons
+// and not fmaxf, which would drop a NaN that has to reach the result; the same for a sink, at which the running maximum starts.)
+__device__ __forceinline__ float positive_scale(float scale) {
+  const float x = fabsf(scale) * LOG2E;
+  return x < FLT_MIN ? FLT_MIN : x;
+}
+__device__ __forceinline__ float finite_seed(float sink) {
+  const float x = sink * LOG2E;
+  return x < -FLT_MAX ? -FLT_MAX : x;
+}
+
 // Decode rows of at most 32 heads.
 template <int RANK, int ROT>
 __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
@@ -395,7 +406,7 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
   const int pos = positions[row];
   const bool valid = slot < heads;
   const bool wave_active = sg * 16 < heads;  // wave-uniform
-  const float scale2 = fmaxf(fabsf(scale) * LOG2E, FLT_MIN);  // (as in the kernel behind this one)
+  const float scale2 = positive_scale(scale);
   const int head = valid ? slot : 0;
   // The queries come through LDS, where the second page will lie: latent parts of 1 KiB, then rotated parts of 128 bytes, 16-byte chunks
   // exchanged so that a fragment's rows lie on different banks.  (Four waves read the same 16 rows, and a fragment read from memory takes
@@ -454,7 +465,7 @@ __global__ __launch_bounds__(512, 2) void latent_wide_kernel(
                                        16, 0, 2);  // 2: non-temporal
   };
   const bool seeded = splits == 1 && sink != nullptr && valid;
-  float m = seeded ? fmaxf(sink[head] * LOG2E, -FLT_MAX) : -FLT_MAX;
+  float m = seeded ? finite_seed(sink[head]) : -FLT_MAX;
   float l = seeded && g == 0 ? 1.f : 0.f;  // of this lane's keys alone
   f32x4 o[DW];
 #pragma unroll
@@ -716,7 +727,7 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
 #pragma unroll
     for (int i = 0; i < NI; ++i) load(p_begin, 0, i);
 
-  const float scale2 = fmaxf(fabsf(scale) * LOG2E, FLT_MIN);  // (maxima and masks come before it: positive, and the scores' sign where it is not)
+  const float scale2 = positive_scale(scale);
   bf16x8 qf[NS][KS];
   int* const last_seen = reinterpret_cast<int*>(lds + 2 * PAGE_BYTES + 9 * 1024) + c16;  // by slot
   float m[NS], l[NS];  // l: of this lane's keys alone
@@ -724,7 +735,7 @@ __global__ __launch_bounds__(256, 1) void latent_tile_kernel(
   for (int j = 0; j < NS; ++j) {
     const int slot = 16 * j + c16;
     const bool valid = slot < n_slots;
-    m[j] = seeded && valid ? fmaxf(seed[j] * LOG2E, -FLT_MAX) : -FLT_MAX;  // (finite: a page of which a slot sees nothing needs no care)
+    m[j] = seeded && valid ? finite_seed(seed[j]) : -FLT_MAX;  // (finite: a page of which a slot sees nothing needs no care)
     l[j] = seeded && valid && part == 0 && g == 0 ? 1.f : 0.f;
     if (part == 0 && g == 0) last_seen[16 * j] = valid ? t.pos0 + slot / t.hcount : -1;  // (read behind the first page's barrier)
   }

@@ -102,3 +102,21 @@ def test_decode_rows_with_scales_of_any_sign(scale, heads, splits):
     for window in (1 << 30, 70):
         got = ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, None, pos, sink, scale, splits=splits, window=window)
         close(got, pool, table, q, sink, ctx, [1] * len(ctx), scale, window)
+
+
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("heads", [16, 40])
+def test_a_sink_or_scale_that_is_no_number_reaches_the_result(tiled, heads):
+    ctx, rows_of = ([90], [20]) if tiled else ([90, 7], [1, 1])
+    pool, table, q, sink = setup(ctx, rows_of, heads, 3)
+    seq = torch.zeros(20, dtype=torch.int32, device=DEV) if tiled else None
+    pos = torch.cat([torch.arange(c - n, c, dtype=torch.int32) for c, n in zip(ctx, rows_of)]).to(DEV)
+    kw = {"tiles": torch.from_numpy(ops.build_latent_tiles(rows_of, ctx, heads)).to(DEV)} if tiled else {"splits": 1}
+    run = lambda s, scale: ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, seq, pos, s, scale, **kw)
+    want, nan = run(sink, 0.3), sink.clone()
+    nan[3] = float("nan")  # one head: nothing else changes
+    got = run(nan, 0.3)
+    assert bool(got[:, 3].isnan().all())
+    got[:, 3] = want[:, 3]
+    assert torch.equal(got, want)
+    assert bool(run(sink, float("nan")).isnan().all())
