@@ -121,3 +121,52 @@ def test_calls_that_something_follows_stay_with_the_library():
         assert taken == [False]
         traced = torch.jit.trace(lambda q: ops.linear(q, w, b), (x,), check_trace=False)
         assert torch.equal(traced(t), lib(t, w, b))
+
+
+# a cut tail, and rows that fill whole rounds of tiles
+SIZES = [(600, 4096, 8192), (4096, 4096, 4096)]
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_followed_calls_by_either_rule(m, n, k):
+    """Gradients, tangents, vmap and traces of plain, residual and split q | k | v products."""
+    from torch.autograd import forward_ad
+
+    x, w, g = _inputs(m, n, k)
+    b, t = torch.randn(n, generator=g, device=DEV).to(BF), torch.randn(m, k, generator=g, device=DEV).to(BF)
+    lib = torch.nn.functional.linear
+    assert ops._tile_takes(x, w, False, b) and bool(ops.tile_rows(x, w)) == (m == 4096)
+    with torch.enable_grad():
+        leaf = b.clone().requires_grad_()
+        ops.linear(x, w, leaf).sum().backward()
+        assert torch.equal(leaf.grad, torch.full_like(b, m))
+        for call in (lambda a: ops.linear(a, w), lambda a: ops.qkv_linear(a, w, None, 2048),
+                     lambda a: ops.linear_add(a, w, torch.zeros(m, n, device=DEV, dtype=BF))):
+            leaf = x.clone().requires_grad_()
+            assert ops.tile_rows(leaf, w) == 0
+            call(leaf).sum().backward()
+            assert leaf.grad is not None and float(leaf.grad.float().norm()) > 0
+    with torch.no_grad(), forward_ad.dual_level():
+        assert torch.equal(forward_ad.unpack_dual(ops.linear(forward_ad.make_dual(x, t), w, b)).tangent, lib(t, w))
+    with torch.no_grad():
+        xs = torch.stack([x, t])
+        assert torch.func.vmap(lambda q: ops.linear(q, w, b))(xs).shape == (2, m, n)
+        traced = torch.jit.trace(lambda q: ops.linear(q, w, b), (x,), check_trace=False)
+        assert torch.equal(traced(t), lib(t, w, b))
+
+
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_operands_off_their_16_bytes(m, n, k):
+    """Left to the library, by either rule."""
+    x, w, g = _inputs(m, n, k)
+    r, b = torch.randn(m, n, generator=g, device=DEV).to(BF), torch.randn(n, generator=g, device=DEV).to(BF)
+
+    def moved(t):
+        off = torch.empty(t.numel() + 1, device=DEV, dtype=BF)[1:].view(t.shape)
+        off.copy_(t)
+        return off
+
+    xo, wo, ro, bo = moved(x), moved(w), moved(r), moved(b)
+    assert not (ops._tile_takes(xo, w) or ops._tile_takes(x, wo) or ops._tile_takes(x, w, False, ro) or ops._tile_takes(x, w, False, bo))
+    assert ops.tile_rows(xo, w) == ops.tile_rows(x, wo) == 0

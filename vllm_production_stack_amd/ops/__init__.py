@@ -875,9 +875,8 @@ def block_add_norm(x, w, residual, weight, eps):
 def tile_add_norm(x, w, residual, weight, eps):
     """As ``linear_add_norm``, for products of the prefill GEMM with a split tail: the pass that closes it also makes the norm."""
     m, n = x.shape[0], w.shape[0]
-    if (not _tile_takes(x, w, False, residual) or n > 8192 or not residual.is_contiguous() or residual.shape != (m, n)
-            or residual.dtype != torch.bfloat16 or residual.device != x.device or weight.device != x.device or weight.dtype != torch.bfloat16 or weight.shape != (n,)
-            or not weight.is_contiguous() or residual.data_ptr() % 8 or weight.data_ptr() % 8 or tile_tail(m, n, w.shape[1]) <= 1):
+    if (not _tile_takes(x, w, False, residual) or n > 8192 or not residual.is_contiguous() or residual.shape != (m, n) or weight.shape != (n,) or weight.device != x.device or weight.dtype != torch.bfloat16
+            or not weight.is_contiguous() or weight.data_ptr() % 8 or tile_tail(m, n, w.shape[1]) <= 1 or _followed(weight)):
         return None
     ws = tail_parts(x.device)
     tile_gemm(x, w, residual=residual, out=residual, parts=ws)
@@ -1052,25 +1051,32 @@ if _shape_log is not None:
     atexit.register(lambda: print("VPSA_SHAPE_LOG", sorted(_shape_log.items(), key=lambda kv: -kv[1])[:60], file=sys.stderr, flush=True))
 
 
+def _tile_reads(x, w, *others) -> bool:
+    """Whether the prefill GEMM may read these operands, whatever its sizes: a call that something follows from outside is left to the library
+    before any address is read (a function transform's tensors have none), and so is what does not lie on the 16 bytes of its
+    loads or beyond their 32-bit offsets.  ``others``: a bias or residual that the epilogue adds, or None."""
+    return (x.shape[1] == w.shape[1] and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and x.shape[0] * x.stride(0) < 1 << 31 and not _followed(x, w, *others)
+            and all(t is None or _lies_with(x, t) for t in (x, w, *others)))
+
+
+def _tile_fills(m: int, n: int, k: int, pair: bool) -> bool:
+    """Whether whole tiles of these sizes fill their rounds."""
+    if _shape_log is not None:
+        _shape_log[(m, n, k)] = _shape_log.get((m, n, k), 0) + 1
+    if m < TILE_MIN_ROWS or not tile_gemm_supported(n, k, pair):
+        return False
+    tiles = -(-m // 256) * (-(-(n // 2) // 128) if pair else -(-n // 256))
+    return tiles / (-(-tiles // TILE_CUS) * TILE_CUS) >= TILE_MIN_FILL
+
+
 def tile_rows(x, w, pair: bool = False) -> int:
     """How many leading rows of ``x`` the prefill GEMM should take for ``x @ w.T``: all of them
     (a ragged last row tile is handled inside the kernel; a separate small GEMM for the remainder
     costs more than the padding), or 0 when the library is the better choice for this shape."""
-    if not (_tile_enabled and x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and w.dim() == 2 and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0):
+    if not (_tile_enabled and x.is_cuda and x.dim() == w.dim() == 2) or not _tile_fills(x.shape[0], *w.shape, pair):
         return 0
-    m, (n, k) = x.shape[0], w.shape
-    if _shape_log is not None:
-        _shape_log[(m, n, k)] = _shape_log.get((m, n, k), 0) + 1
-    if m < TILE_MIN_ROWS or not tile_gemm_supported(n, k, pair):
-        return 0
-    m_tiles = (m + 255) // 256
-    n_tiles = (n // 2 + 127) // 128 if pair else (n + 255) // 256
-    tiles = m_tiles * n_tiles
-    rounds = (tiles + TILE_CUS - 1) // TILE_CUS
-    if tiles / (rounds * TILE_CUS) < TILE_MIN_FILL:
-        return 0
-    return m
+    return x.shape[0] if _tile_reads(x, w) else 0
 
 
 # With the last round's tiles cut (``tile_tail``) and the activation in the epilogue the kernel is ahead of the library at other sizes as
@@ -1093,23 +1099,22 @@ TILE_TAIL_SPLITS = 4         # ... and elsewhere the ranges that a tail behind w
 
 
 def _tile_takes(x, w, pair: bool = False, *others) -> bool:
-    """Whether the prefill GEMM should take all rows of ``x @ w.T``: ``tile_rows``, or the rule above for plain and gated products.  ``others``:
-    a bias or residual that the epilogue adds."""
-    if tile_rows(x, w, pair):
-        return True
-    if not (_tile_enabled and x.is_cuda and x.dim() == 2 and x.shape[0] >= TILE_TAIL_ROWS and w.dim() == 2
-            and x.shape[1] == w.shape[1] and tile_gemm_supported(w.shape[0], w.shape[1], pair) and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.is_contiguous() and not _followed(x, w, *others) and all(t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0)
-                                          for t in (x, w, *others))
-            and x.shape[0] * x.stride(0) < 1 << 31):
+    """Whether the prefill GEMM should take all rows of ``x @ w.T``: by size as ``tile_rows`` does, or by the rule above for plain and gated
+    products, and in both cases operands that it reads.  ``others``: a bias or residual that the epilogue adds."""
+    if not (_tile_enabled and x.is_cuda and x.dim() == w.dim() == 2):
         return False
     m, (n, k) = x.shape[0], w.shape
+    return (_tile_fills(m, n, k, pair) or _tile_tail_pays(m, n, k, pair)) and _tile_reads(x, w, *others)
+
+
+def _tile_tail_pays(m: int, n: int, k: int, pair: bool) -> bool:
+    """The rule above, for sizes."""
+    if m < TILE_TAIL_ROWS or not tile_gemm_supported(n, k, pair):
+        return False
     tiles, splits = -(-m // 256) * (-(-n // 256)), tile_tail(m, n, k, pair)
     if pair:
-        takes = splits > 1 and tiles >= TILE_CUS or tiles >= TILE_PAIR_FILL * TILE_CUS * -(-tiles // TILE_CUS)
-    else:
-        takes = splits > 1 and (k >= 64 * TILE_LONG_CHUNKS or (tiles >= TILE_CUS and splits >= TILE_TAIL_SPLITS))
-    return takes
+        return splits > 1 and tiles >= TILE_CUS or tiles >= TILE_PAIR_FILL * TILE_CUS * -(-tiles // TILE_CUS)
+    return splits > 1 and (k >= 64 * TILE_LONG_CHUNKS or (tiles >= TILE_CUS and splits >= TILE_TAIL_SPLITS))
 
 
 def linear(x, w, bias=None, packed=None):
@@ -1137,7 +1142,7 @@ def linear(x, w, bias=None, packed=None):
             y = _stream_gemm(x, w, bias, False)
         if y is not None:
             return y
-    if (bias is None or bias.dtype == torch.bfloat16) and _tile_takes(x, w, False, bias):
+    if _tile_takes(x, w, False, bias):
         # a bias is a "residual" with row stride 0
         return tile_gemm(x, w, residual=None if bias is None else bias.view(1, -1).expand(x.shape[0], -1))
     return torch.nn.functional.linear(x, w, bias)
@@ -1164,7 +1169,7 @@ def qkv_linear(x, w, bias, q_cols: int):
     hand-written kernel does not take and that have no bias go to the library as two GEMMs,
     [q | k v], each writing its column range of ONE output buffer (same bits as the single call)."""
     if (bias is None and x.is_cuda and x.dim() == 2 and x.shape[0] >= SPLIT_QKV_MIN_ROWS
-            and x.dtype == torch.bfloat16 and 0 < q_cols < w.shape[0] and not _tile_takes(x, w)):
+            and x.dtype == torch.bfloat16 and 0 < q_cols < w.shape[0] and not _tile_takes(x, w) and not _followed(x, w)):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
         torch.matmul(x, w[:q_cols].t(), out=out[:, :q_cols])
         torch.matmul(x, w[q_cols:].t(), out=out[:, q_cols:])
