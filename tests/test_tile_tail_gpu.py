@@ -157,6 +157,15 @@ def test_followed_calls_by_either_rule(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", SIZES)
+def test_biases_that_are_not_a_row_of_the_product(m, n, k):
+    x, w, g = _inputs(m, n, k)
+    b = torch.randn(2 * n, generator=g, device=DEV).to(BF)
+    want = x.double() @ w.double().t()
+    _close(ops.linear(x, w, b[::2]), want + b[::2].double(), 2 ** -6)   # (the library may round the product, below 8, before it adds)
+    _close(ops.linear(x, w, b[:1]), want + b[:1].double(), 2 ** -6)     # one value for all columns
+
+
+@pytest.mark.parametrize("m,n,k", SIZES)
 def test_operands_off_their_16_bytes(m, n, k):
     """Left to the library, by either rule."""
     x, w, g = _inputs(m, n, k)

@@ -875,7 +875,7 @@ def block_add_norm(x, w, residual, weight, eps):
 def tile_add_norm(x, w, residual, weight, eps):
     """As ``linear_add_norm``, for products of the prefill GEMM with a split tail: the pass that closes it also makes the norm."""
     m, n = x.shape[0], w.shape[0]
-    if (not _tile_takes(x, w, False, residual) or n > 8192 or not residual.is_contiguous() or residual.shape != (m, n) or weight.shape != (n,) or weight.device != x.device or weight.dtype != torch.bfloat16
+    if (not _tile_takes(x, w, False, residual) or n > 8192 or weight.shape != (n,) or weight.device != x.device or weight.dtype != torch.bfloat16
             or not weight.is_contiguous() or weight.data_ptr() % 8 or tile_tail(m, n, w.shape[1]) <= 1 or _followed(weight)):
         return None
     ws = tail_parts(x.device)
@@ -1054,9 +1054,11 @@ if _shape_log is not None:
 def _tile_reads(x, w, *others) -> bool:
     """Whether the prefill GEMM may read these operands, whatever its sizes: a call that something follows from outside is left to the library
     before any address is read (a function transform's tensors have none), and so is what does not lie on the 16 bytes of its
-    loads or beyond their 32-bit offsets.  ``others``: a bias or residual that the epilogue adds, or None."""
+    loads or beyond their 32-bit offsets.  ``others``: a bias [N] or residual [M, N] that the epilogue adds, or None."""
+    m, n = x.shape[0], w.shape[0]
     return (x.shape[1] == w.shape[1] and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.is_contiguous() and x.shape[0] * x.stride(0) < 1 << 31 and not _followed(x, w, *others)
+            and w.is_contiguous() and m * x.stride(0) < 1 << 31 and not _followed(x, w, *others)
+            and all(t is None or (t.shape == ((n,) if t.dim() == 1 else (m, n)) and t.is_contiguous()) for t in others)
             and all(t is None or _lies_with(x, t) for t in (x, w, *others)))
 
 
@@ -1152,7 +1154,7 @@ def linear_add(x, w, residual, packed=None):
     """The residual-stream update of an output projection: ``residual += x @ w.T`` inside the GEMM's
     epilogue when the prefill kernel takes the shape (returns None: nothing is left to add), else
     returns ``x @ w.T`` for the caller's fused add + norm."""
-    if not residual.is_contiguous() or not _tile_takes(x, w, False, residual):
+    if not _tile_takes(x, w, False, residual):
         return linear(x, w, None, packed)
     tile_gemm(x, w, residual=residual, out=residual)
     return None
