@@ -130,7 +130,7 @@ SIZES = [(600, 4096, 8192), (4096, 4096, 4096)]
 @pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 @pytest.mark.parametrize("m,n,k", SIZES)
 def test_followed_calls_by_either_rule(m, n, k):
-    """Gradients, tangents, vmap and traces of plain, residual and split q | k | v products."""
+    """Gradients, tangents, vmap and traces of plain, gated, residual and split q | k | v products."""
     from torch.autograd import forward_ad
 
     x, w, g = _inputs(m, n, k)
@@ -141,7 +141,7 @@ def test_followed_calls_by_either_rule(m, n, k):
         leaf = b.clone().requires_grad_()
         ops.linear(x, w, leaf).sum().backward()
         assert torch.equal(leaf.grad, torch.full_like(b, m))
-        for call in (lambda a: ops.linear(a, w), lambda a: ops.qkv_linear(a, w, None, 2048),
+        for call in (lambda a: ops.linear(a, w), lambda a: ops.gate_up_silu(a, w), lambda a: ops.qkv_linear(a, w, None, 2048),
                      lambda a: ops.linear_add(a, w, torch.zeros(m, n, device=DEV, dtype=BF))):
             leaf = x.clone().requires_grad_()
             assert ops.tile_rows(leaf, w) == 0
@@ -152,6 +152,7 @@ def test_followed_calls_by_either_rule(m, n, k):
     with torch.no_grad():
         xs = torch.stack([x, t])
         assert torch.func.vmap(lambda q: ops.linear(q, w, b))(xs).shape == (2, m, n)
+        assert torch.func.vmap(lambda q: ops.gate_up_silu(q, w))(xs).shape == (2, m, n // 2)
         traced = torch.jit.trace(lambda q: ops.linear(q, w, b), (x,), check_trace=False)
         assert torch.equal(traced(t), lib(t, w, b))
 

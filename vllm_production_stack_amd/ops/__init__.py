@@ -1213,7 +1213,7 @@ def hbm_read_probe(buf, blocks=2048):
 
 # --------------------------------------------------------------------------- MLP / sampling
 def silu_and_mul(x, out=None):
-    if not x.is_cuda:
+    if not x.is_cuda or (out is None and _followed(x)):
         y = reference.silu_and_mul(x)
         if out is not None:
             out.copy_(y)
