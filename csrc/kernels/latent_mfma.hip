@@ -926,9 +926,11 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(const float* __restri
     float big = wave_reduce_max(ms);
     if (sink) big = fmaxf(big, sink[head]);
     const float f = ms == -INFINITY ? 0.f : __expf(ms - big);
-    float den = wave_reduce_sum(f == 0.f ? 0.f : ls * f);
-    if (sink) den += __expf(sink[head] - big);
-    fac[s] = den > 0.f ? f / den : 0.f;
+    // (a sum that is no number counts whatever its factor: the maximum of a row of NaN is the lowest finite number, below any sink.  A NaN
+    // denominator passes the comparison and every factor becomes one.)
+    float den = wave_reduce_sum(f == 0.f && ls == ls ? 0.f : ls * f);
+    if (sink) den += sink[head] == big ? 1.f : __expf(sink[head] - big);  // (1 also for an infinite sink, which leaves the entries nothing)
+    fac[s] = den == 0.f ? 0.f : f / den;
   }
   __syncthreads();
   for (int d = threadIdx.x * 4; d < rank; d += 512) {

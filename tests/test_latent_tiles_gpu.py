@@ -120,3 +120,32 @@ def test_a_sink_or_scale_that_is_no_number_reaches_the_result(tiled, heads):
     got[:, 3] = want[:, 3]
     assert torch.equal(got, want)
     assert bool(run(sink, float("nan")).isnan().all())
+
+
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("heads", [16, 40])
+def test_what_is_no_number_reaches_the_result_over_key_ranges(tiled, heads):
+    """The same where several ranges hold a row and a merge joins them, and an infinite sink, which leaves the entries no weight."""
+    ctx, rows_of = ([1500], [20]) if tiled else ([1500, 7, 300], [1, 1, 1])
+    pool, table, q, sink = setup(ctx, rows_of, heads, 3)
+    seq = torch.zeros(20, dtype=torch.int32, device=DEV) if tiled else None
+    pos = torch.cat([torch.arange(c - n, c, dtype=torch.int32) for c, n in zip(ctx, rows_of)]).to(DEV)
+    kw = {"splits": 3}
+    if tiled:
+        kw = {"tiles": torch.from_numpy(ops.build_latent_tiles(rows_of, ctx, heads)).to(DEV)}
+        assert ops.latent.latent_tile_splits(kw["tiles"].shape[0], table.shape[1], RANK, 64, True) > 1
+    run = lambda s, scale=0.3, q=q: ops.latent_attention(q[..., :RANK], q[..., RANK:], pool, 8, table, seq, pos, s, scale, **kw)
+    nan, inf, q2 = sink.clone(), sink.clone(), q.clone()
+    nan[3], inf[3], q2[1, 2, 5] = float("nan"), float("inf"), float("nan")
+    for s in (sink, None):
+        want = run(s)
+        assert bool(want.isfinite().all())
+        got = run(s, q=q2)  # one (token, head) pair: nothing else changes
+        assert bool(got[1, 2].isnan().all())
+        got[1, 2] = want[1, 2]
+        assert torch.equal(got, want)
+        assert bool(run(s, float("nan")).isnan().all())
+    want, got, none = run(sink), run(nan), run(inf)
+    assert bool(got[:, 3].isnan().all()) and bool((none[:, 3] == 0).all())
+    got[:, 3] = none[:, 3] = want[:, 3]
+    assert torch.equal(got, want) and torch.equal(none, want)
