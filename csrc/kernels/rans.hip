@@ -580,35 +580,51 @@ VPSA_EXPORT int vpsa_fetch(const void* from, void* pinned, void* to, long size, 
   return 0;
 }
 
-// The copy of a page on a stream of its own, so that it runs beside the kernels of the page before it (3.5 MB: 70 us of copy, 53 of kernels);
-// `stream` waits for it.  fresh: `body` is new to the caller, and what `stream` still has to do may touch its memory.  Below 2 MB the
+// The stream of the current device that pages' bytes come in on, this library's own: a stream out of torch's pool may be handed to someone
+// else, who queues on it or captures it.  Made on the first call, one a device, and kept; null where none can be had.
+VPSA_EXPORT hipStream_t vpsa_page_copy_stream() {
+  static std::atomic<hipStream_t> streams[64];
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return nullptr;
+  hipStream_t mine = streams[device].load(std::memory_order_acquire);
+  if (mine != nullptr) return mine;
+  hipStream_t made = nullptr;
+  if (hipStreamCreateWithFlags(&made, hipStreamNonBlocking) != hipSuccess) return nullptr;
+  if (streams[device].compare_exchange_strong(mine, made)) return made;
+  (void)hipStreamDestroy(made);
+  return mine;
+}
+
+// The copy of a page on that stream, so that it runs beside the kernels of the page before it (3.5 MB: 70 us of copy, 53 of kernels);
+// `stream` waits for it, and it for nothing but the copies before it: all callers share it.  fresh: `body` is new to the caller, and what
+// `stream` still has to do may touch its memory; the copy then stands in `stream`, where nobody else waits for it.  Below 2 MB the
 // events cost the host, which is behind there anyway, what the copy takes (a page of 1.5 MB of many, one stream / two: 87 / 91 us; of 3.5 MB
 // 143 / 115, of 8 MB 238 / 196; with helpers that wait).
 constexpr long COPY_AHEAD = 2 << 20;
-static int page_copy(void* body, const void* pinned, long size, int fresh, hipStream_t copies, hipStream_t stream) {
+static int page_copy(void* body, const void* pinned, long size, int fresh, hipStream_t stream) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (size < COPY_AHEAD || copies == stream || hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
-    return hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, stream) == hipSuccess ? 0 : -3;
+  const bool ahead = !fresh && size >= COPY_AHEAD && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+  const hipStream_t copies = ahead ? vpsa_page_copy_stream() : nullptr;
+  if (copies == nullptr) return hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, stream) == hipSuccess ? 0 : -3;
   hipEvent_t event;
   if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) return -3;
-  bool ok = !fresh || (hipEventRecord(event, stream) == hipSuccess && hipStreamWaitEvent(copies, event, 0) == hipSuccess);
-  const bool sent = ok && hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, copies) == hipSuccess;
-  ok = sent && hipEventRecord(event, copies) == hipSuccess && hipStreamWaitEvent(stream, event, 0) == hipSuccess;
+  const bool sent = hipMemcpyAsync(body, pinned, size, hipMemcpyHostToDevice, copies) == hipSuccess;
+  const bool ok = sent && hipEventRecord(event, copies) == hipSuccess && hipStreamWaitEvent(stream, event, 0) == hipSuccess;
   if (sent && !ok) (void)hipStreamSynchronize(copies);  // nothing may read the buffer that the caller does not know of
   (void)hipEventDestroy(event);  // (released when it has passed)
   return ok ? 0 : -3;
 }
 
-// `size` host bytes at `from` (a page's parts) through the pinned buffer into `body` by way of `copies`, then symbols and values.  Not waited
+// `size` host bytes at `from` (a page's parts) through the pinned buffer into `body`, then symbols and values.  Not waited
 // for: pinned buffer and body are in use until `stream` has come past this call.
 VPSA_EXPORT int vpsa_page_decode(const void* from, void* pinned, void* body, long size, long n, int n_ctx, int spc, long unit_elems, void* ws,
-                                 void* out, int fresh, hipStream_t copies, hipStream_t stream) {
+                                 void* out, int fresh, hipStream_t stream) {
   if (vpsa_page_workspace(n, n_ctx, spc) <= 0) return -1;
   const PageParts at = page_parts(body, n, n_ctx, spc);
   const long coded = size - (at.coded - (char*)body);
   if (coded < 0) return -1;
   copy_in_parts((char*)pinned, (const char*)from, size);
-  if (const int rc = page_copy(body, pinned, size, fresh, copies, stream)) return rc;
+  if (const int rc = page_copy(body, pinned, size, fresh, stream)) return rc;
   const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, (char*)ws + page_symbols(n), ws, n, n_ctx, spc, stream);
   return rc ? rc : vpsa_cachegen_decode(ws, (const float*)at.scales, out, n, unit_elems, stream);
 }

@@ -31,7 +31,7 @@ _ARGUMENTS = {
     "vpsa_dense_attention": "pllppllplliiiifp",
     "vpsa_chunk_scan": "pliiiiiplppippp" "iifippppp" "ippp",
     "vpsa_latent_attention_mfma": "pllpllplpippiippl" "liifiippip",
-    "vpsa_page_decode": "ppplliilppipp",
+    "vpsa_page_decode": "ppplliilppip",
 }
 
 
@@ -1404,14 +1404,11 @@ def fetch_bytes(src, pinned, dst: int, size: int) -> None:
     _check(_kernels().vpsa_fetch(_p(src), _p(pinned), c_void_p(dst), c_long(size), _stream()), "fetch_bytes")
 
 
-_copy_streams: dict = {}  # device index -> the stream that pages' bytes come in on
-
-
 def page_decode(src: int, pinned, size: int, n: int, n_ctx: int, unit_elems: int, device, spc=RANS_SPC):
     """A page's quantised and coded parts (``size`` host bytes at ``src``: scales fp32 [n / 64] | freq u16 [n_ctx * 256] | states u32 and
     sizes u16 [n_ctx * spc] | coded bytes) -> bf16 [n] on ``device``, by way of ``pinned``, which the device reads until what has been
-    queued so far is over.  A stream of its own takes the bytes into a buffer that stays with ``pinned`` (its ``body``), so that they come
-    in beside the kernels of the page before: no call may use ``pinned`` again, nor let go of it, before this one is over."""
+    queued so far is over.  The bytes come into a device buffer that stays with ``pinned`` (its ``body``), from the second page on, on a stream of
+    the kernel library's, beside the kernels of the page before: no call may use ``pinned`` again, nor let go of it, before this one is over."""
     lib = _kernels()
     ws = int(lib.vpsa_page_workspace(c_long(n), c_int(n_ctx), c_int(spc)))
     if ws <= 0 or unit_elems % 8192:
@@ -1422,12 +1419,10 @@ def page_decode(src: int, pinned, size: int, n: int, n_ctx: int, unit_elems: int
     body = getattr(pinned, "body", None)
     fresh = body is None or body.numel() < size or body.device != out.device
     if fresh:
-        body = pinned.body = torch.empty(max(size, pinned.numel()), dtype=torch.uint8, device=device)
-    copies = _copy_streams.get(out.device.index)
-    if copies is None:
-        copies = _copy_streams.setdefault(out.device.index, torch.cuda.Stream(out.device))
+        body = torch.empty(max(size, pinned.numel()), dtype=torch.uint8, device=device)
     _check(lib.vpsa_page_decode(src, pinned.data_ptr(), body.data_ptr(), size, n, n_ctx, spc, unit_elems, work.data_ptr(), out.data_ptr(),
-                                int(fresh), copies.cuda_stream, _raw_stream()), "page_decode")
+                                int(fresh), _raw_stream()), "page_decode")
+    pinned.body = body
     return out
 
 
