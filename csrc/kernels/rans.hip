@@ -24,17 +24,12 @@
 // Coder: 32-bit state, byte-wise renormalisation, lower bound 2^23.  The encoder runs over its
 // symbols backwards and writes its bytes backwards into a private scratch slot, so the decoder
 // reads forwards; the slots are then gathered into one dense byte string at the prefix sum of the sizes.
-#include <pthread.h>
 #include <string.h>
 
 #include <atomic>
-#include <chrono>
-#include <condition_variable>
-#include <deque>
-#include <mutex>
-#include <thread>
 
 #include "common.h"
+#include "host_copies.h"
 
 #define RANS_BITS 12
 #define RANS_M (1u << RANS_BITS)
@@ -479,97 +474,7 @@ VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
   return coder > 0 && n % 64 == 0 ? page_symbols(n) + coder : 0;
 }
 
-// A host copy of some MB in pieces: a page comes out of memory, not of a cache, and one thread draws 24 to 33 GB/s.  Up to three threads
-// help; they wait for copies of any caller, and end after two seconds without one (they are shared by a process: started for every copy
-// they cost 15 to 20 us each).  Host memory to host memory, one thread / started for the copy / waiting: 1.5 MB 34 / 30 / 15 us, 3.5 MB 107 / 50 / 33, 8 MB
-// 259 / 142 / 101.
-constexpr long COPY_PART = 640 << 10;
-class CopyHelpers {
- public:
-  static constexpr int MOST = 3;
-  // `left` falls by one for every piece that is over.
-  struct Piece {
-    char* to;
-    const char* from;
-    long n;
-    std::atomic<int>* left;
-  };
-
-  // Never ends: a helper may outlive the process's other objects.  A fork has none of its parent's threads and begins with its own.
-  static CopyHelpers& shared() {
-    static std::atomic<CopyHelpers*> all{nullptr};
-    static const int forks = pthread_atfork(nullptr, nullptr, [] { all.store(nullptr); });
-    (void)forks;
-    CopyHelpers* mine = all.load(std::memory_order_acquire);
-    if (mine == nullptr) {
-      CopyHelpers* const made = new CopyHelpers;
-      if (all.compare_exchange_strong(mine, made)) return *made;
-      delete made;
-    }
-    return *mine;
-  }
-  // Queues the pieces; whatever no helper takes is taken by `finish`.
-  void start(const Piece* pieces, int n) {
-    {
-      std::lock_guard<std::mutex> hold(lock_);
-      queue_.insert(queue_.end(), pieces, pieces + n);
-      for (; helpers_ < MOST; ++helpers_) {
-        try {
-          std::thread([this] { help(); }).detach();
-        } catch (...) {  // no thread to be had
-          break;
-        }
-      }
-    }
-    ready_.notify_all();
-  }
-  void finish(const std::atomic<int>& left) {
-    while (left.load(std::memory_order_acquire) > 0)
-      if (!copy_one()) std::this_thread::yield();
-  }
-
- private:
-  bool copy_one() {
-    std::unique_lock<std::mutex> hold(lock_);
-    if (queue_.empty()) return false;
-    const Piece p = queue_.front();
-    queue_.pop_front();
-    hold.unlock();
-    memcpy(p.to, p.from, p.n);
-    p.left->fetch_sub(1, std::memory_order_release);
-    return true;
-  }
-  void help() {
-    for (;;) {
-      if (copy_one()) continue;
-      std::unique_lock<std::mutex> hold(lock_);
-      if (!ready_.wait_for(hold, std::chrono::seconds(2), [this] { return !queue_.empty(); })) {
-        --helpers_;
-        return;
-      }
-    }
-  }
-  std::mutex lock_;
-  std::condition_variable ready_;
-  std::deque<Piece> queue_;
-  int helpers_ = 0;
-};
-
-VPSA_EXPORT int vpsa_copy_parts(long size) {
-  const long parts = size / COPY_PART;
-  return parts < 1 ? 1 : parts > CopyHelpers::MOST ? CopyHelpers::MOST + 1 : (int)parts;
-}
-
-static void copy_in_parts(char* to, const char* from, long size) {
-  const int parts = vpsa_copy_parts(size);
-  const long each = size / parts & ~4095L;  // whole pages
-  std::atomic<int> left{parts - 1};
-  CopyHelpers::Piece pieces[CopyHelpers::MOST];
-  for (int i = 0; i < parts - 1; ++i, to += each, from += each, size -= each) pieces[i] = {to, from, each, &left};
-  if (parts > 1) CopyHelpers::shared().start(pieces, parts - 1);
-  memcpy(to, from, size);
-  if (parts > 1) CopyHelpers::shared().finish(left);
-}
+VPSA_EXPORT int vpsa_copy_parts(long size) { return copy_parts(size); }
 
 // `size` bytes from the device to `to` by way of a pinned buffer.  Over on return.  (Four parts, each leaving the buffer while the next is on
 // its way, were no faster, 158 us a page against 162, and on the way back they cost the device 50 us a page: a copy's start is 10 to 15.)
