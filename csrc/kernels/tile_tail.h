@@ -15,7 +15,9 @@ struct TileTail {
 // A round is 256 workgroups, one a CU.  Its last round costs a product a whole tile's time however few tiles it has: up to half a round of
 // them are cut so that they fill it.  A range costs what a whole tile does beside its chunks (about six chunks' time for its first loads and
 // its 256 KiB of sums) and the tail a pass of 5 to 13 us, 4 to 9 chunks' time: fewer than six chunks a range are not worth it, nor a tail
-// alone that saves fewer than 16 chunks (4096 x 4096, 1000 rows 83 us whole, 55 cut; 16384 x 2048 gated, 300 rows, 16 saved 38 and 44).  Behind whole
+// alone that saves fewer than 16 chunks.  Whole / cut, microseconds, the chunks saved in brackets: 512 x 6144, 24 chunks 39.9 / 35.0 (18), 250 x
+// 1536, 23 chunks 31.6 / 27.2 (16); the last product and the sum of eight experts, hidden 2816, 400 tokens, 32 chunks 111 / 107 (16).  (Dense
+// products whose ranges fill the round need 22, a pass of their own: ops/__init__.py.)  Behind whole
 // rounds workgroups are out of step and part of the last one's time is hidden: 36 chunks (28672 x 4096 gated, 336 tiles, 43 saved 157 and 145;
 // 896 tiles, 32 saved 341 and 341; 4096 x 4096, 384 tiles, 32 saved 196 and 206), and none behind eight and more (37888 x 3584, 3108 tiles 1063
 // and 1089).

@@ -180,3 +180,20 @@ def test_operands_off_their_16_bytes(m, n, k):
     xo, wo, ro, bo = moved(x), moved(w), moved(r), moved(b)
     assert not (ops._tile_takes(xo, w) or ops._tile_takes(x, wo) or ops._tile_takes(x, w, False, ro) or ops._tile_takes(x, w, False, bo))
     assert ops.tile_rows(xo, w) == ops.tile_rows(x, wo) == 0
+
+
+@pytest.mark.parametrize("m,n,k,form,cut", [(300, 16384, 2048, "gated", False), (256, 127 * 256, 2112, "plain", False), (256, 127 * 256, 3136, "plain", True),
+                                            (500, 85 * 128, 2048, "residual", True), (1024, 4096, 1792, "plain", False), (200, 512, 1536, "plain", True)])
+def test_dense_tails_are_cut_where_their_own_pass_pays(monkeypatch, m, n, k, form, cut):
+    x, w, g = _inputs(m, n, k)
+    asked, parts = [], ops.tail_parts
+    monkeypatch.setattr(ops, "tail_parts", lambda *a: asked.append(a) or parts(*a))
+    want = x.double() @ w.double().t()
+    if form == "gated":
+        _close(ops.tile_gemm(x, w, silu_mul=True), torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:])
+    elif form == "residual":
+        r = torch.randn(m, n, generator=g, device=DEV).to(BF)
+        _close(ops.tile_gemm(x, w, residual=r), want + r.double())
+    else:
+        _close(ops.tile_gemm(x, w), want)
+    assert bool(asked) == cut

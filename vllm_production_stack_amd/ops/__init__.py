@@ -1683,7 +1683,7 @@ def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, resi
     if gelu_mul:
         epi = 6
     ws = parts
-    if ws is None and offsets is None and epi <= 2 and tile_tail(rows, n, k, paired) > 1:
+    if ws is None and offsets is None and epi <= 2 and _tail_pass_pays(rows, n, k, paired):
         ws = tail_parts(a.device)
     rc = _kernels().vpsa_tile_gemm(_p(a), c_long(a.stride(0)), _p(arow_idx), _p(w), _p(offsets), c_int(g), _p(out),
                                    c_long(out.stride(0)), c_int(rows), c_int(n), c_int(k), c_int(epi), _p(residual),
@@ -1699,6 +1699,15 @@ def tile_tail(rows: int, n: int, k: int, paired: bool = False) -> int:
     """Ranges of the reduction that the last tiles of a dense product are cut in (1: none is), ``csrc/kernels/tile_tail.h``."""
     n_tiles = (n // 2 + 127) // 128 if paired else (n + 255) // 256
     return int(_kernels().vpsa_tile_tail(c_int((rows + 255) // 256 * n_tiles), c_int(k)))
+
+
+def _tail_pass_pays(rows: int, n: int, k: int, paired: bool) -> bool:
+    """Whether a dense product's tail is cut, given the pass of its own that closes it: 5 to 10 us for the launch and little else while the
+    ranges are few, twice that where they fill a round and their sums take 64 MB.  A tail alone then has to save 22 chunks: whole / cut,
+    microseconds, 16384 x 2048 gated, 300 rows, 16 saved 38.5 / 44; x 2304, 18 saved 42.8 / 47; x 2560, 20 saved 53.2 / 51.9; 4096 x 2560
+    residual, 2048 rows, 20 saved 59.0 / 59.8; 4096 x 1792, 1024 rows, 21 saved 38.2 / 40.0; 10880 x 2048, 500 rows, 22 saved 48.0 / 45.2."""
+    splits, tiles, chunks = tile_tail(rows, n, k, paired), -(-rows // 256) * (-(-(n // 2) // 128) if paired else -(-n // 256)), k // 64
+    return splits > 1 and (tiles >= TILE_CUS or tiles * splits <= 224 or chunks - chunks // splits >= 22)
 
 
 def tail_parts(device):
