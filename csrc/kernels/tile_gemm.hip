@@ -88,7 +88,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
   // contiguous runs, one per XCD (workgroups go to XCDs round robin), so the workgroups that share
   // an XCD's L2 at any time are (row tiles of one group) x (one band).
   const TileRows rows_of = {offsets, n_groups, max_rows, n_tiles, RAGGED};
-  const int total = rows_of.tiles();
+  const int total = TAIL ? rows_of.tiles_by_wave() : rows_of.tiles();  // (with a tail the grid has 256 workgroups more that may have nothing to do)
   const TileTail tail = TAIL ? tile_tail(total, k_total / TG_BK) : TileTail{total, 1};
   const int bid = blockIdx.x, units_all = tail.cut + (total - tail.cut) * tail.splits;
   if (bid >= units_all) return;
@@ -586,7 +586,7 @@ __global__ __launch_bounds__(1024) void tail_norm_kernel(const float* __restrict
 __global__ __launch_bounds__(256) void moe_combine_parts_kernel(const float* __restrict__ ws, const TileRows rows_of, int k_total,
                                                                 const uint16_t* __restrict__ y, const float* __restrict__ weights,
                                                                 const int* __restrict__ pos, uint16_t* __restrict__ out, int hidden, int topk) {
-  const int tok = blockIdx.x, total = rows_of.tiles();
+  const int tok = blockIdx.x, total = rows_of.tiles_by_wave();
   const TileTail tail = tile_tail(total, k_total / TG_BK);
   if (tail.splits == 1) {  // (a routing without a tail: wider reads, no search)
     for (int i = threadIdx.x * 8; i < hidden; i += 256 * 8) {

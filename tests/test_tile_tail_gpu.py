@@ -197,3 +197,23 @@ def test_dense_tails_are_cut_where_their_own_pass_pays(monkeypatch, m, n, k, for
     else:
         _close(ops.tile_gemm(x, w), want)
     assert bool(asked) == cut
+
+
+@pytest.mark.parametrize("experts,tokens,inner", [(70, 50, 1536), (130, 300, 1536), (64, 40, 2048), (8, 130, 1408), (9, 130, 1472)])
+def test_experts_by_the_wave_and_short_reductions(monkeypatch, experts, tokens, inner):
+    """More experts than a wave has lanes, of which some have no rows; reductions of 22 chunks, which no routing cuts, and of 23."""
+    g = torch.Generator(device=DEV).manual_seed(experts)
+    asked, parts = [], ops.tail_parts
+    monkeypatch.setattr(ops, "tail_parts", lambda *a: asked.append(a) or parts(*a))
+    h, k = 512, 4
+    x = torch.randn(tokens, h, generator=g, device=DEV).to(BF)
+    w13 = (torch.randn(experts, 2 * inner, h, generator=g, device=DEV) * h ** -0.5).to(BF)
+    w2 = (torch.randn(experts, h, inner, generator=g, device=DEV) * inner ** -0.5).to(BF)
+    ids = torch.stack([torch.randperm(experts - 3, generator=g, device=DEV)[:k] for _ in range(tokens)]).int()
+    wt = torch.rand(tokens, k, generator=g, device=DEV)
+    got = ops.moe_experts_prefill(x, w13, w2, ids, wt)
+    assert bool(asked) == (inner >= 23 * 64)
+    y, pos = ops.moe_experts_prefill(x, w13, w2, ids, wt, combine=False)
+    want = (y.double()[pos.long()].view(tokens, k, h) * wt[:, :, None].double()).sum(1)
+    # a pair's value rounded to 16 bits once less, or not at all where its tile is whole, and the sum: 2^-9 of the norm each
+    assert float((got.double() - want).norm() / want.norm()) < 6e-3

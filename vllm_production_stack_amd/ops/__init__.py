@@ -1701,6 +1701,9 @@ def tile_tail(rows: int, n: int, k: int, paired: bool = False) -> int:
     return int(_kernels().vpsa_tile_tail(c_int((rows + 255) // 256 * n_tiles), c_int(k)))
 
 
+TAIL_MIN_CHUNKS = 23  # the shortest reduction that saves 16 chunks in ranges of six or more
+
+
 def _tail_pass_pays(rows: int, n: int, k: int, paired: bool) -> bool:
     """Whether a dense product's tail is cut, given the pass of its own that closes it: 5 to 10 us for the launch and little else while the
     ranges are few, twice that where they fill a round and their sums take 64 MB.  A tail alone then has to save 22 chunks: whole / cut,
@@ -1743,8 +1746,10 @@ def moe_experts_prefill(x, w13, w2, ids, weights, gather=True, foreign=False, co
         act = gg(x, w13, offsets, rows=t * k, arow_idx=sorted_tok, silu_mul=True)
     else:  # copy the rows into sorted order first (timing comparison)
         act = gg(moe_permute(x, sorted_tok), w13, offsets, rows=t * k, silu_mul=True)
-    # (from eight rounds of tiles on there is no tail: tile_tail.h; the host knows the least that a routing can make)
-    if not combine or gg is not tile_gemm or -(-t * k // 256) * -(-w2.shape[1] // 256) >= 8 * TILE_CUS or w2.shape[1] % 8 or t == 0:
+    # (from eight rounds of tiles on there is no tail, and none of short reductions whatever the routing (tile_tail.h); the host knows the
+    # least number of tiles that a routing can make)
+    if (not combine or gg is not tile_gemm or -(-t * k // 256) * -(-w2.shape[1] // 256) >= 8 * TILE_CUS or w2.shape[2] < 64 * TAIL_MIN_CHUNKS
+            or w2.shape[1] % 8 or t == 0):
         y = gg(act, w2, offsets, rows=t * k)
         if not combine:  # the caller sums the pairs itself
             return y, pos
