@@ -217,3 +217,16 @@ def test_experts_by_the_wave_and_short_reductions(monkeypatch, experts, tokens, 
     want = (y.double()[pos.long()].view(tokens, k, h) * wt[:, :, None].double()).sum(1)
     # a pair's value rounded to 16 bits once less, or not at all where its tile is whole, and the sum: 2^-9 of the norm each
     assert float((got.double() - want).norm() / want.norm()) < 6e-3
+
+
+@pytest.mark.parametrize("topk", [256, 257])
+def test_experts_with_many_pairs_a_token(topk):
+    g = torch.Generator(device=DEV).manual_seed(topk)
+    x = torch.randn(3, 128, generator=g, device=DEV).to(BF)
+    w13 = (torch.randn(260, 2 * 1536, 128, generator=g, device=DEV) * 128 ** -0.5).to(BF)
+    w2 = (torch.randn(260, 128, 1536, generator=g, device=DEV) * 1536 ** -0.5).to(BF)
+    ids = torch.stack([torch.randperm(260, generator=g, device=DEV)[:topk] for _ in range(3)]).int()
+    wt = torch.rand(3, topk, generator=g, device=DEV)
+    y, pos = ops.moe_experts_prefill(x, w13, w2, ids, wt, combine=False)
+    want = (y.double()[pos.long()].view(3, topk, 128) * wt[:, :, None].double()).sum(1)
+    assert float((ops.moe_experts_prefill(x, w13, w2, ids, wt).double() - want).norm() / want.norm()) < 6e-3

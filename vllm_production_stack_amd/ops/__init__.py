@@ -1747,9 +1747,9 @@ def moe_experts_prefill(x, w13, w2, ids, weights, gather=True, foreign=False, co
     else:  # copy the rows into sorted order first (timing comparison)
         act = gg(moe_permute(x, sorted_tok), w13, offsets, rows=t * k, silu_mul=True)
     # (from eight rounds of tiles on there is no tail, and none of short reductions whatever the routing (tile_tail.h); the host knows the
-    # least number of tiles that a routing can make)
+    # least number of tiles that a routing can make.  A thread finds each pair's place: 256 a token.)
     if (not combine or gg is not tile_gemm or -(-t * k // 256) * -(-w2.shape[1] // 256) >= 8 * TILE_CUS or w2.shape[2] < 64 * TAIL_MIN_CHUNKS
-            or w2.shape[1] % 8 or t == 0):
+            or w2.shape[1] % 8 or k > 256 or t == 0):
         y = gg(act, w2, offsets, rows=t * k)
         if not combine:  # the caller sums the pairs itself
             return y, pos
