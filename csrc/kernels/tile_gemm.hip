@@ -501,7 +501,7 @@ __device__ __forceinline__ f32x4 tail_sum(const float* __restrict__ p, int split
   return s;
 }
 
-// The tail's tiles: sums, epilogue, 16-bit outputs.  Grid (tail tiles, 32): eight rows a workgroup, 64 threads a row of 256 columns (32 of
+// A dense product's tail: sums, epilogue, 16-bit outputs.  Grid (tail tiles, 32): eight rows a workgroup, 64 threads a row of 256 columns (32 of
 // 128 pairs).  Bound by the launch and the sums' way from the memory-side cache.
 template <int EPI>
 __global__ __launch_bounds__(256) void tail_finish_kernel(const float* __restrict__ ws, const TileRows rows_of, int k_total, int n_total,
@@ -654,10 +654,10 @@ TileRows tile_rows_of(const void* offsets, int n_groups, int max_rows, int n, bo
 // Ranges that the tail's tiles of a product are cut in, 1 where there is no tail: `tiles` tiles, reductions of k.
 VPSA_EXPORT int vpsa_tile_tail(int tiles, int k) { return tile_tail(tiles, k / TG_BK).splits; }
 
-// The passes behind vpsa_tile_gemm with a workspace: the tail's outputs (epi 0, 1, 2 and its arguments as there) ...
-VPSA_EXPORT int vpsa_tile_tail_finish(const void* ws, const void* offsets, int n_groups, void* c, long ldc, int max_rows, int n, int k, int epi,
-                                      const void* resid, long ldr, hipStream_t stream) {
-  const TileRows rows_of = tile_rows_of(offsets, n_groups, max_rows, n, epi == TG_EPI_SWIGLU);
+// The passes behind vpsa_tile_gemm with a workspace: the tail's outputs of a dense product (epi 0, 1, 2 and its arguments as there) ...
+VPSA_EXPORT int vpsa_tile_tail_finish(const void* ws, void* c, long ldc, int rows, int n, int k, int epi, const void* resid, long ldr,
+                                      hipStream_t stream) {
+  const TileRows rows_of = tile_rows_of(nullptr, 1, rows, n, epi == TG_EPI_SWIGLU);
   const dim3 grid(TG_CUS / 2, TG_BM / 8);  // (a tail has up to half a round of tiles)
 #define FINISH(E)                                                                                                                  \
   tail_finish_kernel<E><<<grid, 256, 0, stream>>>((const float*)ws, rows_of, k, n, (uint16_t*)c, ldc, (const uint16_t*)resid, ldr)

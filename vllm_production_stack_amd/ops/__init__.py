@@ -1691,7 +1691,7 @@ def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, resi
                                    c_float(lim), c_float(alpha), c_float(bias), _p(row_scale), _p(ws), _stream())
     _check(rc, "tile_gemm")
     if ws is not None and parts is None:
-        _tail_finish(ws, None, 1, out, rows, n, k, epi, residual)
+        _tail_finish(ws, out, rows, n, k, epi, residual)
     return out
 
 
@@ -1718,9 +1718,9 @@ def tail_parts(device):
     return torch.empty(256 << 16, dtype=torch.float32, device=device)
 
 
-def _tail_finish(ws, offsets, groups, out, rows, n, k, epi, residual=None):
-    rc = _kernels().vpsa_tile_tail_finish(_p(ws), _p(offsets), c_int(groups), _p(out), c_long(out.stride(0)), c_int(rows), c_int(n), c_int(k),
-                                          c_int(epi), _p(residual), c_long(0 if residual is None else residual.stride(0)), _stream())
+def _tail_finish(ws, out, rows, n, k, epi, residual):
+    rc = _kernels().vpsa_tile_tail_finish(_p(ws), _p(out), c_long(out.stride(0)), c_int(rows), c_int(n), c_int(k), c_int(epi), _p(residual),
+                                          c_long(0 if residual is None else residual.stride(0)), _stream())
     _check(rc, "tile_tail_finish")
 
 
