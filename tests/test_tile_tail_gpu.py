@@ -230,3 +230,32 @@ def test_experts_with_many_pairs_a_token(topk):
     y, pos = ops.moe_experts_prefill(x, w13, w2, ids, wt, combine=False)
     want = (y.double()[pos.long()].view(3, topk, 128) * wt[:, :, None].double()).sum(1)
     assert float((ops.moe_experts_prefill(x, w13, w2, ids, wt).double() - want).norm() / want.norm()) < 6e-3
+
+
+@pytest.mark.parametrize("m,n,k,slots", [(1, 256, 1600, 4), (512, 768, 2112, 30), (300, 1024, 4160, 80), (4097, 4096, 3072, 128), (6144, 4096, 4672, 256)])
+def test_workspaces_hold_what_the_tail_has(monkeypatch, m, n, k, slots):
+    x, w, g = _inputs(m, n, k)
+    buf = torch.full((256 << 16,), 7.0, device=DEV)
+    monkeypatch.setattr(ops, "tail_parts", lambda device, s: buf[:s << 16] if s == slots else None)
+    _close(ops.tile_gemm(x, w), x.double() @ w.double().t())
+    assert bool((buf[slots << 16:] == 7).all()) and not bool((buf[:slots << 16] == 7).all())
+
+
+@pytest.mark.parametrize("tokens,inner", [(3, 1536), (40, 2048), (300, 2048)])
+def test_workspaces_of_experts_hold_the_tail_of_any_routing(monkeypatch, tokens, inner):
+    g = torch.Generator(device=DEV).manual_seed(tokens)
+    e, h = 5, 520
+    x = torch.randn(tokens, 512, generator=g, device=DEV).to(BF)
+    w13 = (torch.randn(e, 2 * inner, 512, generator=g, device=DEV) / 23).to(BF)
+    w2 = (torch.randn(e, h, inner, generator=g, device=DEV) * inner ** -0.5).to(BF)
+    buf, asked = torch.empty(256 << 16, device=DEV), []
+    monkeypatch.setattr(ops, "tail_parts", lambda device, s: asked.append(s) or buf[:s << 16])
+    wt = torch.rand(tokens, 2, generator=g, device=DEV)
+    for first in (0, 4):                                                          # one or two experts with all pairs, or all with some
+        ids = torch.stack([torch.arange(tokens, device=DEV) % (first + 1), torch.full((tokens,), 1, device=DEV)], 1).int()
+        buf.fill_(7.0)
+        got = ops.moe_experts_prefill(x, w13, w2, ids, wt)
+        assert bool((buf[asked[-1] << 16:] == 7).all())
+        y, pos = ops.moe_experts_prefill(x, w13, w2, ids, wt, combine=False)
+        want = (y.double()[pos.long()].view(tokens, 2, h) * wt[:, :, None].double()).sum(1)
+        assert float((got.double() - want).norm() / want.norm()) < 6e-3

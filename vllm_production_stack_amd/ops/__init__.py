@@ -878,7 +878,7 @@ def tile_add_norm(x, w, residual, weight, eps):
     if (not _tile_takes(x, w, False, residual) or n > 8192 or weight.shape != (n,) or weight.device != x.device or weight.dtype != torch.bfloat16
             or not weight.is_contiguous() or weight.data_ptr() % 8 or tile_tail(m, n, w.shape[1]) <= 1 or _followed(weight)):
         return None
-    ws = tail_parts(x.device)
+    ws = tail_parts(x.device, _tail_slots(m, n, w.shape[1], False))
     tile_gemm(x, w, residual=residual, out=residual, parts=ws)
     y = torch.empty_like(residual)
     rc = _kernels().vpsa_tile_tail_norm(_p(ws), _p(residual), _p(weight), _p(y), c_int(m), c_int(n), c_int(w.shape[1]), c_float(eps), _stream())
@@ -1068,7 +1068,7 @@ def _tile_fills(m: int, n: int, k: int, pair: bool) -> bool:
         _shape_log[(m, n, k)] = _shape_log.get((m, n, k), 0) + 1
     if m < TILE_MIN_ROWS or not tile_gemm_supported(n, k, pair):
         return False
-    tiles = -(-m // 256) * (-(-(n // 2) // 128) if pair else -(-n // 256))
+    tiles = _tiles(m, n, pair)
     return tiles / (-(-tiles // TILE_CUS) * TILE_CUS) >= TILE_MIN_FILL
 
 
@@ -1684,7 +1684,7 @@ def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, resi
         epi = 6
     ws = parts
     if ws is None and offsets is None and epi <= 2 and _tail_pass_pays(rows, n, k, paired):
-        ws = tail_parts(a.device)
+        ws = tail_parts(a.device, _tail_slots(rows, n, k, paired))
     rc = _kernels().vpsa_tile_gemm(_p(a), c_long(a.stride(0)), _p(arow_idx), _p(w), _p(offsets), c_int(g), _p(out),
                                    c_long(out.stride(0)), c_int(rows), c_int(n), c_int(k), c_int(epi), _p(residual),
                                    c_long(residual.stride(0) if residual is not None else 0), c_long(a.shape[0]),
@@ -1695,10 +1695,13 @@ def tile_gemm(a, w, offsets=None, rows=None, arow_idx=None, silu_mul=False, resi
     return out
 
 
+def _tiles(rows: int, n: int, paired: bool) -> int:
+    return -(-rows // 256) * (-(-(n // 2) // 128) if paired else -(-n // 256))
+
+
 def tile_tail(rows: int, n: int, k: int, paired: bool = False) -> int:
     """Ranges of the reduction that the last tiles of a dense product are cut in (1: none is), ``csrc/kernels/tile_tail.h``."""
-    n_tiles = (n // 2 + 127) // 128 if paired else (n + 255) // 256
-    return int(_kernels().vpsa_tile_tail(c_int((rows + 255) // 256 * n_tiles), c_int(k)))
+    return int(_kernels().vpsa_tile_tail(c_int(_tiles(rows, n, paired)), c_int(k)))
 
 
 TAIL_MIN_CHUNKS = 23  # the shortest reduction that saves 16 chunks in ranges of six or more
@@ -1709,13 +1712,18 @@ def _tail_pass_pays(rows: int, n: int, k: int, paired: bool) -> bool:
     ranges are few, twice that where they fill a round and their sums take 64 MB.  A tail alone then has to save 22 chunks: whole / cut,
     microseconds, 16384 x 2048 gated, 300 rows, 16 saved 38.5 / 44; x 2304, 18 saved 42.8 / 47; x 2560, 20 saved 53.2 / 51.9; 4096 x 2560
     residual, 2048 rows, 20 saved 59.0 / 59.8; 4096 x 1792, 1024 rows, 21 saved 38.2 / 40.0; 10880 x 2048, 500 rows, 22 saved 48.0 / 45.2."""
-    splits, tiles, chunks = tile_tail(rows, n, k, paired), -(-rows // 256) * (-(-(n // 2) // 128) if paired else -(-n // 256)), k // 64
+    splits, tiles, chunks = tile_tail(rows, n, k, paired), _tiles(rows, n, paired), k // 64
     return splits > 1 and (tiles >= TILE_CUS or tiles * splits <= 224 or chunks - chunks // splits >= 22)
 
 
-def tail_parts(device):
-    """Room for the partial sums of a round of tail workgroups, 256 tiles of 256 x 256."""
-    return torch.empty(256 << 16, dtype=torch.float32, device=device)
+def _tail_slots(rows: int, n: int, k: int, paired: bool) -> int:
+    """Ranges of tail tiles that a dense product has in all."""
+    return _tiles(rows, n, paired) % TILE_CUS * tile_tail(rows, n, k, paired)
+
+
+def tail_parts(device, slots: int = TILE_CUS):
+    """Room for the partial sums of that many tail workgroups, a tile of 256 x 256 each; a round of them is the most there is."""
+    return torch.empty(slots << 16, dtype=torch.float32, device=device)
 
 
 def _tail_finish(ws, out, rows, n, k, epi, residual):
@@ -1754,7 +1762,8 @@ def moe_experts_prefill(x, w13, w2, ids, weights, gather=True, foreign=False, co
         if not combine:  # the caller sums the pairs itself
             return y, pos
         return moe_combine(y, weights, pos, t)
-    ws = tail_parts(x.device)
+    tiles = (t * k // 256 + n_experts) * -(-w2.shape[1] // 256)  # the most that a routing makes
+    ws = tail_parts(x.device, min(TILE_CUS, tiles * (w2.shape[2] // 64 // 6)))
     y = tile_gemm(act, w2, offsets, rows=t * k, parts=ws)
     assert weights.dtype == torch.float32 and pos.dtype == torch.int32
     out = torch.empty((t, w2.shape[1]), dtype=x.dtype, device=x.device)
