@@ -1652,8 +1652,9 @@ __global__ __launch_bounds__(256, 1) void paged_prefill_kernel_v4(
 // head groups workgroups and every record is read with whole-wave contiguous loads.  (Slices of 16 values left half the CUs without a
 // workgroup: 97 rows of 32 heads in 16 ranges 11.4 -> 9.6 us, with the rows
 // that are left out above; with 16 bytes a load instead of 4, 9.3 -> 8.2, 200 rows in 24 ranges 9.2 -> 7.4.)
-// Eight records' loads are on their way at a time, and no remainder is read one by one: with four, 58 rows in 32 ranges took 12.9 us, now
-// 12.0 (a whole step of 8 layers 1395 -> 1385; with branches around each record's loads, which the compiler waits at, 18.9).
+// Eight records' loads are on their way at a time, the first eight beside the other records' maxima, and no remainder is read one by one: 58 rows in
+// 32 ranges 12.9 us with four at a time, 12.0 with eight (18.9 with branches around each record's loads, which the compiler waits at),
+// 10.4 with the maxima beside the first (with 4 bytes a load 11.1); 97 rows in 16 8.3 -> 7.4; a step of 8 layers, 58 rows 1382 -> 1369.
 __global__ __launch_bounds__(256) void prefill_combine_kernel(
     const float* __restrict__ split_ws, const int* __restrict__ groups, uint16_t* __restrict__ out,
     long out_stride, const int* __restrict__ cu_q, int n_q, int n_kv) {
@@ -1673,30 +1674,26 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(
   const float* rec0 = split_ws + ((long)(part0 * gridDim.y + by) * 4 + wave) * SPLIT_REC_FLOATS;
   const long rec_step = (long)gridDim.y * 4 * SPLIT_REC_FLOATS;
   const int at = (((rb * 4 + dt) * 4 + 2 * half) * 64 + lane) * 4, am = 8192 + rb * 64 + lane;
-  float m = NEG_BIG;
-  for (int p0 = 0; p0 < nparts; p0 += 8) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) m = fmaxf(m, rec0[(p0 + j < nparts ? p0 + j : nparts - 1) * rec_step + am]);
-  }
-  float l = 0.f;
+  float m = NEG_BIG, l = 0.f;
   float o[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[i] = 0.f;
   // N records whose loads are all on their way before the first is used
-  auto add = [&](int p, auto count) {
-    constexpr int N = decltype(count)::value;
-    float top[N], sum[N];
-    f32x4 lo[N], hi[N];
+  float top[8], sum[8];
+  f32x4 lo[8], hi[8];
+  auto load = [&](int p, auto count) {
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
+    for (int j = 0; j < decltype(count)::value; ++j) {
       const float* rec = rec0 + (p + j) * rec_step;
       top[j] = rec[am];
       sum[j] = rec[am + 128];
       lo[j] = *reinterpret_cast<const f32x4*>(rec + at);
       hi[j] = *reinterpret_cast<const f32x4*>(rec + at + 256);
     }
+  };
+  auto add = [&](auto count) {
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
+    for (int j = 0; j < decltype(count)::value; ++j) {
       const float f = __builtin_amdgcn_exp2f(top[j] - m);
       l += f * sum[j];
 #pragma unroll
@@ -1706,11 +1703,32 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(
       }
     }
   };
+  constexpr std::integral_constant<int, 8> eight;
+  const auto rest = [&](int p, auto count) {
+    if (nparts & decltype(count)::value) load(p, count), add(count), p += decltype(count)::value;
+    return p;
+  };
   int p = 0;
-  for (; p + 8 <= nparts; p += 8) add(p, std::integral_constant<int, 8>());
-  if (nparts & 4) add(p, std::integral_constant<int, 4>()), p += 4;
-  if (nparts & 2) add(p, std::integral_constant<int, 2>()), p += 2;
-  if (nparts & 1) add(p, std::integral_constant<int, 1>());
+  if (nparts >= 8) {
+    load(0, eight);  // (on their way beside the other maxima)
+    for (int p0 = 8; p0 < nparts; p0 += 24) {
+      float x[24];
+#pragma unroll
+      for (int j = 0; j < 24; ++j) x[j] = rec0[(p0 + j < nparts ? p0 + j : nparts - 1) * rec_step + am];
+#pragma unroll
+      for (int j = 0; j < 24; ++j) m = fmaxf(m, x[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, top[j]);
+    add(eight);
+    for (p = 8; p + 8 <= nparts; p += 8) load(p, eight), add(eight);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, rec0[(j < nparts ? j : nparts - 1) * rec_step + am]);
+  }
+  p = rest(p, std::integral_constant<int, 4>());
+  p = rest(p, std::integral_constant<int, 2>());
+  rest(p, std::integral_constant<int, 1>());
   const float inv = 1.f / l;
   uint16_t* op = out + (long)(row0 + row) * out_stride + head * HEAD_DIM + 32 * dt + 16 * half + 4 * h;
 #pragma unroll

@@ -32,3 +32,9 @@ def test_any_number_of_ranges(ranges):
     want = torch.zeros_like(q)
     ref.paged_prefill(q, want, pool, 0, bt, cu, ctx_t, n_q, n_kv, hd, scale)
     assert _rel_row_err(out, want, n_q) < REL_TOL
+
+
+@pytest.mark.parametrize("ranges", [10, 31, 32, 33, 57])
+def test_maxima_behind_the_first_eight_records(ranges):
+    """Read beside the first run's values, 24 at a time: one such run, a whole one and one more, a third."""
+    test_any_number_of_ranges(ranges)
