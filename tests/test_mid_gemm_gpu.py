@@ -325,3 +325,29 @@ def test_decoder_steps_with_the_fused_reductions(monkeypatch, grouped):
     untouched = torch.ones(31, dtype=torch.bool, device=DEV)
     untouched[(slots[:5] // 64)] = False
     assert torch.equal(got[0][1][untouched], start.float()[untouched])                      # nothing went to the row without a slot
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+@pytest.mark.parametrize("m,n,k", [(1, 520, 512), (8, 2048, 2048), (16, 256, 4096), (40, 1024, 8192)])
+def test_followed_calls_of_few_rows(m, n, k):
+    """Gradients, tangents, vmap and traces where the streaming kernels are the ones that take the size, plain, gated and of a packed copy."""
+    from torch.autograd import forward_ad
+
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, t = (torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    w = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(torch.bfloat16)
+    lib = torch.nn.functional.linear
+    packed = ops.pack_weight(w) if ops.packed_supported(n, k) else None
+    with torch.enable_grad():
+        for call in (lambda a: ops.linear(a, w), lambda a: ops.gate_up_silu(a, w), lambda a: ops.linear(a, w, None, packed)):
+            leaf = x.clone().requires_grad_()
+            call(leaf).sum().backward()
+            assert leaf.grad is not None and float(leaf.grad.float().norm()) > 0
+    with torch.no_grad(), forward_ad.dual_level():
+        assert torch.equal(forward_ad.unpack_dual(ops.linear(forward_ad.make_dual(x, t), w)).tangent, lib(t, w))
+    with torch.no_grad():
+        xs = torch.stack([x, t])
+        assert torch.func.vmap(lambda q: ops.linear(q, w))(xs).shape == (2, m, n)
+        assert torch.func.vmap(lambda q: ops.gate_up_silu(q, w))(xs).shape == (2, m, n // 2)
+        traced = torch.jit.trace(lambda q: ops.linear(q, w), (x,), check_trace=False)
+        assert torch.equal(traced(t), lib(t, w))

@@ -1003,7 +1003,8 @@ def packed_linear(x2, wp, n: int, k: int, bias=None, pair: bool = False):
 def _skinny_ok(x, w, bias):
     return (_skinny_enabled and x.is_cuda and w.device == x.device and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.is_contiguous() and x.dim() == 2 and 0 < x.shape[0] <= SKINNY_MAX_ROWS and x.stride(1) == 1
-            and (bias is None or (bias.device == x.device and bias.dtype == torch.bfloat16 and bias.is_contiguous())))
+            and (bias is None or (bias.device == x.device and bias.dtype == torch.bfloat16 and bias.is_contiguous()))
+            and not _followed(x, w, bias))
 
 
 # Dispatch thresholds of shapes that mid_gemm below does not take, measured on MI355X (profiles/gemm_micro_graph.jsonl, HIP-graph replay,
