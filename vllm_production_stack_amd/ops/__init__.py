@@ -799,7 +799,12 @@ def _block_splits(m: int, n: int, k: int, pair: bool, sums: int = MID_SUMS) -> i
     rounds = -(-wgs // TILE_CUS)
     if splits <= 0 or wgs < (MID_MIN_FILL if rounds == 1 else MID_BLOCK_FILL) * TILE_CUS * rounds:
         return 0
-    if splits == 1:  # (full tiles in a second round that is not: 57344 x 8192; up to 128 rows short reductions: 152064 x 3584)
+    if splits == 1:
+        # In one round always.  In several, each begins and ends once more: up to 128 rows reductions of 64 chunks and more carry that
+        # (128256 x 4096, 97 rows 209 us against 218 and 233), of 56 no more (152064 x 3584 241 against 235 and 237; nothing measured between);
+        # beyond, the products do, up to 224 rows in any rounds that got here (57344 x 8192, 448 workgroups of 512, 200 rows 207
+        # against 220), with rows that fill the tile where the last round is nearly full (256 rows: 152064 x 3584, 1188 of 1280, 286 against 319;
+        # 448 of 512, 232 against 221: the line between 0.875 and 0.93).
         if m > BLOCK_MAX_ROWS or (rounds > 1 and (k < STREAM_MAX_K // 2 if m <= MID_ROWS_BLOCK else m > 224 and wgs < 0.9 * TILE_CUS * rounds)):
             return 0
         return splits
