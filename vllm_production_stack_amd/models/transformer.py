@@ -322,9 +322,9 @@ class TransformerModel:
             else:
                 x = ops.rms_norm(h, lw.ln1, cfg.norm_eps, residual)
             attn = None
-            if decode_only and not adapters:
-                attn = ops.decode_attention_block(x, lw.wqkv, lw.bqkv, pool, li, meta, self.n_q, self.n_kv, self.head_dim,
-                                                  self.scale, self.cos_sin)
+            if not adapters:
+                block = ops.decode_attention_block if decode_only else ops.prompt_attention_block
+                attn = block(x, lw.wqkv, lw.bqkv, pool, li, meta, self.n_q, self.n_kv, self.head_dim, self.scale, self.cos_sin)
             if attn is None:
                 qkv = self._lora("qkv", gl, x, ops.qkv_linear(x, lw.wqkv, lw.bqkv, self.n_q * self.head_dim), meta)
                 attn = self._attention(qkv, pool, li, meta)

@@ -942,6 +942,33 @@ def decode_attention_block(x, w, bias, pool, layer, meta, n_q, n_kv, head_dim, s
     return out
 
 
+# The projection's reduction also rotates and writes the cache: a launch less a layer.  A step of 8 layers, apart / together: 32 rows behind
+# 1500 tokens 1121 / 1084 us, 64 behind 3000 1270 / 1221, 97 behind 20900 1650 / 1601, 150 behind 3000 1577 / 1534, 256 behind 2000 1818 / 1701; with two
+# row tiles 300 behind 1500 2152 / 2122, but 400 2221 / 2274, 512 2488 / 2512: the cache's own kernel writes whole lines of V, the reduction single values.
+PROMPT_QKV_ROWS = BLOCK_MAX_ROWS
+
+
+def prompt_attention_block(x, w, bias, pool, layer, meta, n_q, n_kv, head_dim, scale, cos_sin):
+    """As ``decode_attention_block`` for a short step with prompt rows, behind decode rows or by themselves."""
+    if isinstance(pool, LayerGroupedPool):
+        pool, layer = pool.for_layer(layer)
+    nd = meta.num_decode
+    if (meta.num_prefill_seqs <= 0 or x.dim() != 2 or x.shape[0] > PROMPT_QKV_ROWS or meta.slots is None or head_dim != HEAD_DIM_HIP
+            or _generic_attention(x, head_dim)):
+        return None
+    q = decode_qkv(x, w, bias, pool, layer, meta.positions, meta.slots, cos_sin, n_q, n_kv)
+    if q is None:
+        return None
+    out = (torch.zeros_like if getattr(meta, "pre_padded", False) else torch.empty_like)(q)
+    if nd > 0:
+        paged_decode(q[:nd], out[:nd], pool, layer, meta.dec_block_tables, meta.dec_ctx_lens, n_q, n_kv, head_dim, scale,
+                     getattr(meta, "dec_num_splits", 1) or 1, getattr(meta, "dec_ws_o", None), getattr(meta, "dec_ws_ml", None))
+    paged_prefill(q[nd:], out[nd:], pool, layer, meta.pre_block_tables, meta.pre_cu_q, meta.pre_ctx_lens, meta.pre_tile_seq,
+                  meta.pre_tile_q0, n_q, n_kv, head_dim, scale, meta.pre_tile_rows, split=getattr(meta, "pre_split", None),
+                  split_ws=getattr(meta, "pre_split_ws", None), groups=getattr(meta, "pre_split_groups", None))
+    return out
+
+
 def block_linear(x, ws, biases, gelu=False, residual=None, out=None):
     """act(x @ w.T + bias) (+ residual) for one to three weights of one shape, side by side in the last dimension
     (``csrc/kernels/block_gemm.hip``).  x [B, T, K] with unit stride along K (rows may overlap, as a convolution's unfolded input
