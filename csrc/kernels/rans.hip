@@ -11,14 +11,14 @@
 // share statistics), ctx_len symbols each.  A context is cut into spc streams; stream j owns
 // symbols j, j + spc, j + 2 spc, ... so that at every step the 64 lanes of a wave touch 64
 // consecutive bytes (coalesced loads in the encoder, coalesced stores in the decoder).
-// One thread codes one stream; a workgroup is one wave (64 streams), so that a page's 16384 streams reach every CU: what bounds
+// One thread codes one stream; a workgroup has 64 streams, so that a page's 16384 streams reach every CU: what bounds
 // both directions is a stream's chain of dependent steps, not arithmetic or bytes.  The chain is kept short:
 //   encoder  symbols and their table entries are read a batch of eight ahead, the division by a symbol's frequency is a
 //            multiplication, coded bytes leave four at a time;
-//   decoder  one table entry per step (symbol, frequency and offset within it), the wave's coded bytes staged in LDS and
-//            consumed from a register window, at most two bytes a step without a loop.
+//   decoder  one table entry per step (symbol, frequency and offset within it), the streams' coded bytes staged in LDS and read
+//            two at a time, at most two bytes a step without a loop.
 // Page of a 32-layer cache with 8 KV heads (4.2 M symbols): coding loop 107 -> 25 us, with tables and gathering 150 -> 47; decoding
-// 118 -> 33 us (before: 64 workgroups, symbols and coded bytes read and written one at a time from memory, divisions).
+// 118 -> 24 us (before: 64 workgroups, symbols and coded bytes read and written one at a time from memory, divisions).
 // Per context: a 256-entry frequency table normalised to 2^12,
 // built from a histogram of that very page (it travels with the blob: 512 B per context).
 // Coder: 32-bit state, byte-wise renormalisation, lower bound 2^23.  The encoder runs over its
@@ -277,119 +277,145 @@ __global__ __launch_bounds__(256) void rans_pack_kernel(const uint8_t* __restric
   }
 }
 
-// grid n_ctx, block 1024: a context's 4096 decoder entries, symbol | (freq - 1) << 8 | (slot - cum) << 20, and the bytes of its
-// streams.  (A damaged table gives entries of some symbol; every field is masked to its width.)
-__global__ __launch_bounds__(1024) void rans_decode_tables_kernel(const uint16_t* __restrict__ freq, uint32_t* __restrict__ table,
-                                                                  const uint16_t* __restrict__ sizes, int spc,
-                                                                  long* __restrict__ ctx_bytes) {
-  __shared__ uint32_t cum[256], fr[256];
-  __shared__ long part[16];
-  const int t = threadIdx.x;
-  uint32_t f = 0;
-  if (t < 256) {
-    f = freq[blockIdx.x * 256 + t];
-    fr[t] = f;
-  }
-  long sum = 0;
-  for (int i = t; i < spc; i += 1024) sum += sizes[(long)blockIdx.x * spc + i];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  if ((t & 63) == 0) part[t >> 6] = sum;
-  const int before = wave_before((int)f);  // (of the wave's 64 symbols)
-  if (t < 256) cum[t] = before;
-  __syncthreads();
-  if (t == 0) {
-    long s = 0;
-    for (int w = 0; w < 16; ++w) s += part[w];
-    ctx_bytes[blockIdx.x] = s;
-  }
-  if (t < 256) {
-    uint32_t c = cum[t];
-    for (int w = 0; w < (t >> 6); ++w) c += cum[w * 64 + 63] + fr[w * 64 + 63];
-    f = c;
-  }
-  __syncthreads();
-  if (t < 256) cum[t] = f;
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t slot = t + 1024 * i;
-    int s = 0;  // the last symbol that starts at or before the slot (those before it with the same start do not occur)
-#pragma unroll
-    for (int step = 128; step > 0; step >>= 1)
-      if (cum[s + step] <= slot) s += step;
-    table[blockIdx.x * (long)RANS_M + slot] = (uint32_t)s | ((fr[s] - 1) & 0xfff) << 8 | ((slot - cum[s]) & 0xfff) << 20;
-  }
-}
-
-// A stream's symbols; `word` reads words i and i + 1 of the wave's coded bytes, from LDS or (streams too long for it) from memory.
-// Two copies of the loop: one that may load from memory waits for its own stores at every step.  The words around the next
-// byte are read in the same wait as the state's table entry.
-template <typename F>
-__device__ __forceinline__ void rans_decode_stream(F word, uint32_t rp, uint32_t x, const uint32_t* tab,
-                                                   uint8_t* __restrict__ out, int len, int spc) {
-  for (int k = 0; k < len; ++k) {
-    const uint32_t e = tab[x & (RANS_M - 1)];
-    const uint64_t w = word(rp >> 2);
-    const uint32_t lo = (uint32_t)w, hi = (uint32_t)(w >> 32);
-    *out = (uint8_t)e;
-    out += spc;
-    const uint32_t q = x >> RANS_BITS;  // 20 bits (19 of a state the encoder leaves)
-    x = __umul24((e >> 8) & 0xfff, q) + (q + (e >> 20));
-    const uint32_t b = __builtin_amdgcn_alignbyte(hi, lo, rp & 3);  // the next byte lowest
-    const uint32_t x1 = (x << 8) | (b & 0xff), x2 = (x1 << 8) | ((b >> 8) & 0xff);
+// A stream's symbols; `pair` gives the two bytes at a place of the wave's coded bytes, the first one higher, from LDS or (streams too
+// long for it) from memory.  Two copies of the loop: one that may load from memory waits for its own stores at every step.  DIR: which way the
+// places run.  What bounds it is the chain from a state to the next, and every instruction of a wave that has its SIMD to itself stands in
+// it: an entry of two words, f | symbol << 24 and the offset, makes the new state one instruction (a 24-bit product takes the first as it is),
+// the bytes come in by one funnel shift, a row's place is a scalar, places are bounded once in 16 steps.  15 instructions a step instead
+// of 27; left alone, the compiler moves the second read behind a branch where no byte is due, and the shift behind another: 35 us a page
+// instead of 24.
+template <int DIR, typename F>
+__device__ __forceinline__ void rans_decode_stream(F pair, int at, uint32_t x, const u32x2* tab, uint8_t* __restrict__ out, int lane, int len,
+                                                   int spc) {
+  auto step = [&](__amdgpu_buffer_rsrc_t to, uint32_t row) {  // (a row's place is a scalar beside the lane's)
+    const uint32_t q = x >> RANS_BITS;
+    u32x2 e = tab[x & (RANS_M - 1)];
+    uint32_t p = pair(at);
+    asm volatile("" : "+v"(p), "+v"(e));  // both reads are under way before anything of either is used (not behind a branch where no byte is due)
+    x = __umul24(e[0], q) + e[1];  // (a state the encoder leaves has 19 bits in q)
     const bool one = x < RANS_LOW, two = x < (RANS_LOW >> 8);
-    x = two ? x2 : one ? x1 : x;
-    rp += one + two;
+    uint32_t in = __builtin_amdgcn_alignbit(x, p << 16, two ? 16 : 24);
+    asm volatile("" : "+v"(in));
+    x = one ? in : x;
+    at += one ? DIR : 0;
+    at += two ? DIR : 0;
+    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(e[0] >> 24), to, lane, row, 0);
+  };
+  constexpr int RUN = 16;
+  for (; len >= RUN; len -= RUN, out += (long)RUN * spc) {
+    if (DIR < 0) at = max(at, 2 * RUN);  // (an undamaged stream's places are past DECODE_SLACK)
+    const auto to = __builtin_amdgcn_make_buffer_rsrc(out, 0, -1, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < RUN; ++k) step(to, (uint32_t)k * (uint32_t)spc);
   }
+  if (DIR < 0) at = max(at, 2 * RUN);
+  for (; len > 0; --len, out += spc) step(__builtin_amdgcn_make_buffer_rsrc(out, 0, -1, 0x00020000), 0);
 }
 
-// grid (spc / 64, n_ctx), block 64.  The wave's coded bytes lie side by side, behind those of the contexts and of the context's
-// streams before it; they are staged when they fit (a stream's share of LDS_WORDS is 320 bytes, a symbol rarely takes one).
-// coded_len bounds every read (a damaged blob decodes to garbage, never out of bounds), and a step takes at most two bytes
-// whatever the state is.
-__global__ __launch_bounds__(64) void rans_decode_kernel(const uint8_t* __restrict__ coded, long coded_len,
-                                                         const long* __restrict__ ctx_bytes, const uint16_t* __restrict__ sizes,
-                                                         const uint32_t* __restrict__ states, const uint32_t* __restrict__ table,
-                                                         uint8_t* __restrict__ sym, long ctx_len, int spc) {
-  constexpr int LDS_WORDS = 64 * 80;
-  __shared__ __attribute__((aligned(16))) uint32_t tab[RANS_M];
-  __shared__ uint32_t bytes[LDS_WORDS];
-  const int ctx = blockIdx.y, t = threadIdx.x;
-  const u32x4* tp = reinterpret_cast<const u32x4*>(table + (long)ctx * RANS_M);
+#define DECODE_THREADS 256
+#define DECODE_SLACK 64  // bytes below any that a stream reads: places are bounded once in so many steps that they move by less
+// grid (spc / 64, n_ctx).  The workgroup makes the context's 4096 table entries and brings in the coded bytes of its 64 streams, which lie side
+// by side behind those of all streams before them; then every wave decodes 16 streams, a lane each.  The bytes are staged when they fit (a stream's
+// share is 320, a symbol rarely takes one), last byte first, so that a pair is one read.  coded_len bounds every read (a damaged blob
+// decodes to garbage, never out of bounds: a damaged table gives entries of some symbol, every field masked to its width), and a step takes
+// at most two bytes whatever the state is.  A page of 16384 streams of 256 symbols: tables in a launch of their own 4 us and one wave for all 64
+// streams 33; in one launch 32 with one wave (which waited for memory ten times in a row before its first step), 28 with four (fewer lanes meet
+// in a bank of LDS; eight waves 32), 24 with the loop above.
+__global__ __launch_bounds__(DECODE_THREADS) void rans_decode_kernel(const uint8_t* __restrict__ coded, long coded_len, const uint16_t* __restrict__ freq,
+                                                          const uint16_t* __restrict__ sizes, const uint32_t* __restrict__ states,
+                                                          uint8_t* __restrict__ sym, long ctx_len, int spc) {
+  typedef uint16_t any_u16 __attribute__((aligned(1)));
+  constexpr int LDS_WORDS = 64 * 80 + DECODE_SLACK / 4, LDS_BYTES = LDS_WORDS * 4;
+  __shared__ __attribute__((aligned(16))) u32x2 tab[RANS_M];
+  __shared__ __attribute__((aligned(16))) uint32_t bytes[LDS_WORDS];
+  constexpr int NT = DECODE_THREADS, WAVES = NT / 64, EACH = 64 / WAVES;  // streams of a wave
+  __shared__ uint32_t cum[256], fr[256], in_wave[4];
+  __shared__ long part[WAVES];
+  const int ctx = blockIdx.y, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const uint32_t f = t < 256 ? freq[ctx * 256 + t] : 0;
+  const long stream0 = (long)ctx * spc + blockIdx.x * 64;
+  const int n = sizes[stream0 + lane];  // (every wave: the bytes of the workgroup's streams)
+  const uint32_t x0 = states[stream0 + lane];
+  // bytes before the workgroup's first stream
+  long first = 0;
+  if (((uintptr_t)sizes & 15) == 0) {
+    const u32x4* const sz = reinterpret_cast<const u32x4*>(sizes);
+    const long pieces = stream0 / 8;  // (whole: stream0 is a multiple of 64)
+    for (long i0 = 0; i0 < pieces; i0 += NT * 8) {
+      u32x4 v[8];
 #pragma unroll
-  for (int i = 0; i < RANS_M / 256; ++i) reinterpret_cast<u32x4*>(tab)[t + 64 * i] = tp[t + 64 * i];
-  const uint16_t* sz = sizes + (long)ctx * spc;
-  long first = 0;  // byte of the wave's first stream
-  for (int i = t; i < ctx; i += 64) first += ctx_bytes[i];
-  for (int i = t; i < (int)blockIdx.x * 64; i += 64) first += sz[i];
+      for (int j = 0; j < 8; ++j) {
+        const long i = i0 + t + NT * j;
+        v[j] = sz[i < pieces ? i : 0];
+        if (i >= pieces) v[j] = (u32x4){0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) first += (v[j][w] & 0xffff) + (v[j][w] >> 16);
+    }
+  } else {
+    for (long i = t; i < stream0; i += NT) first += sizes[i];
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
-  const int n = sz[blockIdx.x * 64 + t], before = wave_before(n), all = __shfl(before + n, 63, 64);
-  const uint32_t x = states[(long)ctx * spc + blockIdx.x * 64 + t];
+  const int cum0 = wave_before((int)f), before = wave_before(n), all = __shfl(before + n, 63, 64);
+  if (t < 256) fr[t] = f;
+  if (lane == 63) {
+    if (wave < 4) in_wave[wave] = (uint32_t)cum0 + f;
+    part[wave] = first;
+  }
+  __syncthreads();
+  if (t < 256) {
+    uint32_t c = (uint32_t)cum0;
+    for (int w = 0; w < wave; ++w) c += in_wave[w];
+    cum[t] = c;
+  }
+  first = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) first += part[w];
   // words of the coded bytes, counted from the aligned word that holds byte 0
   const int lead = (int)((uintptr_t)coded & 3);
   const uint32_t* cw = reinterpret_cast<const uint32_t*>(coded - lead);
   const long n_words = (coded_len + lead + 3) >> 2;
   const long w0 = (first + lead) >> 2, w1 = min((first + all + lead + 3) >> 2, n_words);
-  const bool staged = w1 - w0 < LDS_WORDS;
+  const bool staged = w1 - w0 < LDS_WORDS - DECODE_SLACK / 4;
   const int held = staged ? max((int)(w1 - w0), 0) : 0;
-#pragma unroll 8
-  for (int i = t; i < held; i += 64) bytes[i] = cw[w0 + i];
+  constexpr int AHEAD = 3584 / NT;  // words that a thread asks for before it waits: a page's usual share at once
+  uint32_t v[AHEAD];
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) v[j] = t + NT * j < held ? cw[w0 + t + NT * j] : 0u;
   __syncthreads();
-  uint8_t* out = sym + (long)ctx * ctx_len + blockIdx.x * 64 + t;
+  // the last symbol that starts at or before the slot (those before it with the same start do not occur)
+#pragma unroll 4
+  for (int i = 0; i < (int)RANS_M / NT; ++i) {
+    const uint32_t slot = t + NT * i;
+    int s = 0;
+#pragma unroll
+    for (int step = 128; step > 0; step >>= 1)
+      if (cum[s + step] <= slot) s += step;
+    tab[slot] = (u32x2){((fr[s] - 1) & 0xfff) + 1 | (uint32_t)s << 24, (slot - cum[s]) & 0xfff};
+  }
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j)
+    if (t + NT * j < held) bytes[LDS_WORDS - 1 - (t + NT * j)] = __builtin_bswap32(v[j]);
+  for (int i = t + NT * AHEAD; i < held; i += NT) bytes[LDS_WORDS - 1 - i] = __builtin_bswap32(cw[w0 + i]);
+  __syncthreads();
+  uint8_t* out = sym + (long)ctx * ctx_len + blockIdx.x * 64 + EACH * wave;
   const int len = (int)(ctx_len / spc);
-  const uint32_t rp = (uint32_t)((first + lead) & 3) + (uint32_t)before;
+  const uint32_t rp = __shfl((uint32_t)((first + lead) & 3) + (uint32_t)before, (EACH * wave + lane) & 63, 64);
+  const uint32_t x = __shfl(x0, (EACH * wave + lane) & 63, 64);
+  if (lane >= EACH) return;
   if (staged)
-    rans_decode_stream([&](uint32_t i) {
-      const uint32_t at = min(i, (uint32_t)LDS_WORDS - 2);
-      return (uint64_t)bytes[at + 1] << 32 | bytes[at];
-    }, rp, x, tab, out, len, spc);
+    rans_decode_stream<-1>([&](int i) {
+      return (uint32_t)*reinterpret_cast<const any_u16*>(reinterpret_cast<const char*>(bytes) + i);
+    }, LDS_BYTES - 2 - (int)rp, x, tab, out, lane, len, spc);
   else
-    rans_decode_stream([&](uint32_t i) {
-      const uint32_t lo = w0 + i < n_words ? cw[w0 + i] : 0u, hi = w0 + i + 1 < n_words ? cw[w0 + i + 1] : 0u;
-      return (uint64_t)hi << 32 | lo;
-    }, rp, x, tab, out, len, spc);
+    rans_decode_stream<1>([&](uint32_t i) {
+      const uint32_t lo = w0 + (i >> 2) < n_words ? cw[w0 + (i >> 2)] : 0u, hi = w0 + (i >> 2) + 1 < n_words ? cw[w0 + (i >> 2) + 1] : 0u;
+      const uint32_t b = __builtin_amdgcn_alignbyte(hi, lo, i & 3);  // the next byte lowest
+      return (b & 0xff) << 8 | ((b >> 8) & 0xff);
+    }, (int)rp, x, tab, out, lane, len, spc);
 }
 
 static bool rans_shape_ok(long n, int n_ctx, int spc) {
@@ -431,23 +457,12 @@ VPSA_EXPORT int vpsa_rans_encode(const void* sym, long n, int n_ctx, int spc, vo
   return 0;
 }
 
-// Bytes of the decoder's workspace: tables | bytes per context.
-VPSA_EXPORT long vpsa_rans_decode_workspace(long n, int n_ctx, int spc) {
-  if (!rans_shape_ok(n, n_ctx, spc)) return 0;
-  return (long)n_ctx * (RANS_M * 4 + 8);
-}
-
-// Only freq, states and sizes travel beside the coded bytes; ws 16-byte aligned.
-VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* states, const void* freq, const void* sizes,
-                                 void* ws, void* sym, long n, int n_ctx, int spc, hipStream_t stream) {
+// Only freq, states and sizes travel beside the coded bytes.
+VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* states, const void* freq, const void* sizes, void* sym,
+                                 long n, int n_ctx, int spc, hipStream_t stream) {
   if (!rans_shape_ok(n, n_ctx, spc)) return -1;
-  const long ctx_len = n / n_ctx;
-  uint32_t* table = (uint32_t*)ws;
-  long* ctx_bytes = (long*)(table + (long)n_ctx * RANS_M);
-  hipLaunchKernelGGL(rans_decode_tables_kernel, dim3(n_ctx), dim3(1024), 0, stream, (const uint16_t*)freq, table,
-                     (const uint16_t*)sizes, spc, ctx_bytes);
-  hipLaunchKernelGGL(rans_decode_kernel, dim3(spc / 64, n_ctx), dim3(64), 0, stream, (const uint8_t*)coded, coded_len, ctx_bytes,
-                     (const uint16_t*)sizes, (const uint32_t*)states, table, (uint8_t*)sym, ctx_len, spc);
+  hipLaunchKernelGGL(rans_decode_kernel, dim3(spc / 64, n_ctx), dim3(DECODE_THREADS), 0, stream, (const uint8_t*)coded, coded_len, (const uint16_t*)freq,
+                     (const uint16_t*)sizes, (const uint32_t*)states, (uint8_t*)sym, n / n_ctx, spc);
   return 0;
 }
 
@@ -468,11 +483,8 @@ static PageParts page_parts(void* body, long n, int n_ctx, int spc) {
 static long page_symbols(long n) { return (n + 255) & ~255L; }
 
 // A page's parts, scales fp32 [n / 64] | freq | states | sizes | coded bytes, lie side by side in `body` on the device.
-// Bytes of the workspace of vpsa_page_decode (symbols | the coder's), 0: the shape is not taken.
-VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
-  const long coder = vpsa_rans_decode_workspace(n, n_ctx, spc);
-  return coder > 0 && n % 64 == 0 ? page_symbols(n) + coder : 0;
-}
+// Bytes of the workspace of vpsa_page_decode (symbols), 0: the shape is not taken.
+VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) { return rans_shape_ok(n, n_ctx, spc) && n % 64 == 0 ? page_symbols(n) : 0; }
 
 VPSA_EXPORT int vpsa_copy_parts(long size) { return copy_parts(size); }
 
@@ -530,6 +542,6 @@ VPSA_EXPORT int vpsa_page_decode(const void* from, void* pinned, void* body, lon
   if (coded < 0) return -1;
   copy_in_parts((char*)pinned, (const char*)from, size);
   if (const int rc = page_copy(body, pinned, size, fresh, stream)) return rc;
-  const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, (char*)ws + page_symbols(n), ws, n, n_ctx, spc, stream);
+  const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, ws, n, n_ctx, spc, stream);
   return rc ? rc : vpsa_cachegen_decode(ws, (const float*)at.scales, out, n, unit_elems, stream);
 }
