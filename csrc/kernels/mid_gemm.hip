@@ -128,11 +128,13 @@ __device__ __forceinline__ void stream_product(const char* __restrict__ wp, uint
   __syncthreads();
 }
 
-template <int MT, bool PAIR>
+// FACTORS (unsplit, one token tile): squares are sums of 16 squares of the rows behind x [M, K / 16], K up to 8192; a row's factor 1 /
+// sqrt(their sum / K + eps) is applied to its outputs.
+template <int MT, bool PAIR, bool FACTORS = false>
 __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __restrict__ x, long x_stride,
                                                           const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
                                                           uint16_t* __restrict__ y, long y_stride, float* __restrict__ ws, int M,
-                                                          int N, int K, int S) {
+                                                          int N, int K, int S, const float* __restrict__ squares, float eps) {
   // weights are read once: non-temporal loads, except where the partial sums of many rows want the memory-side cache as well
   constexpr int POLICY = PAIR || MT <= 3 ? 2 : 0;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -145,6 +147,15 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
   const int mrows = min(M - m0, 16 * MT);
   const int arow[2] = {PAIR ? 16 * wave : 32 * wave, PAIR ? 64 + 16 * wave : 32 * wave + 16};
   f32x4 acc[2][MT];
+  // a wave sums four rows' squares; asked for before the stream, used behind it
+  f32x4 sq[4][2];
+  if constexpr (FACTORS)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // 256 sums of a row at a time, nothing past them
+      const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(squares) + (long)min(4 * wave + i, M - 1) * (K / 16), 0, K / 16 * 4, 0x00020000);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) sq[i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, 16 * lane + 1024 * j, 0, 0));
+    }
   // Workgroups walk their chunks from different ones on (first_chunk): rows whose length is a power of two put a chunk of all 128 rows on
   // the same few memory channels, and workgroups in step would meet there (28672 x 4096: 44.7 -> 39.5 us, 128256 x 4096: 205 -> 160).
   stream_product<MT, 2, POLICY>(
@@ -152,6 +163,16 @@ __global__ __launch_bounds__(256, 1) void mid_gemm_kernel(const uint16_t* __rest
       reinterpret_cast<const char*>(x + (long)m0 * x_stride) + (long)c0 * ROWB,
       [&](int r) { return (uint32_t)(min(r, mrows - 1) * (int)(x_stride * 2)); },  // rows past the last repeat it
       n, n > 0 ? first_chunk(blockIdx.x, n, S == 1 && (n >= 128 || gridDim.x > 256)) : 0, lds, arow, acc);
+  if constexpr (FACTORS) {
+    float* const factor = reinterpret_cast<float*>(lds);  // (nothing reads or loads there any more)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float tot = wave_reduce_sum(sq[i][0][0] + sq[i][0][1] + sq[i][0][2] + sq[i][0][3] + sq[i][1][0] + sq[i][1][1] + sq[i][1][2] + sq[i][1][3]);
+      if (lane == 0) factor[4 * wave + i] = rsqrtf(tot / (float)K + eps);
+    }
+    __syncthreads();
+    acc[0][0] *= factor[c16], acc[1][0] *= factor[c16];
+  }
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int j = 16 * t + c16;
@@ -410,19 +431,19 @@ __global__ __launch_bounds__(256) void mid_reduce_qkv_kernel(const float* __rest
   }
 }
 
-template <int MT, bool PAIR>
+template <int MT, bool PAIR, bool FACTORS = false>
 int launch_mid(const void* x, long xs, const void* w, const void* bias, void* y, long ys, float* ws, int M, int N, int K, int S,
-               hipStream_t stream) {
+               hipStream_t stream, const float* squares = nullptr, float eps = 0.f) {
   constexpr int LDS = STAGES * (BN + 16 * MT) * ROWB;
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)mid_gemm_kernel<MT, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)mid_gemm_kernel<MT, PAIR, FACTORS>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
       return -2;
     attr_set = true;
   }
   const int n_out = PAIR ? N / 2 : N;
-  mid_gemm_kernel<MT, PAIR><<<dim3(n_out / (PAIR ? BN / 2 : BN), S, (M + 127) / 128), 256, LDS, stream>>>(
-      (const uint16_t*)x, xs, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ys, ws, M, N, K, S);
+  mid_gemm_kernel<MT, PAIR, FACTORS><<<dim3(n_out / (PAIR ? BN / 2 : BN), S, (M + 127) / 128), 256, LDS, stream>>>(
+      (const uint16_t*)x, xs, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ys, ws, M, N, K, S, squares, eps);
   return 0;
 }
 
@@ -553,6 +574,16 @@ VPSA_EXPORT int vpsa_mid_gemm(const void* x, long xs, const void* w, const void*
   if ((ys & 3) || ((uintptr_t)y & 7) || (pair && bias)) return -1;
   const int rc = mid_product(x, xs, w, bias, y, ys, ws, M, N, K, pair, S, stream);
   return rc || S == 1 ? rc : mid_reduce(ws, bias, y, ys, M, N, S, pair, stream);
+}
+
+// y [M, N / 2] = silu(gate) * up, gate | up = x W^T times the rows' factors 1 / sqrt(sum of squares / K + eps), squares [M, K / 16]: M up to 16,
+// K up to 8192, an unsplit shape.
+VPSA_EXPORT int vpsa_mid_unit_factors(const void* x, long xs, const float* squares, float eps, const void* w, void* y, long ys, int M, int N,
+                                      int K, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (M > 16 || K > 8192 || vpsa_mid_gemm_splits(M, N, K, 1) != 1 || (ys & 3) || ((uintptr_t)y & 7)) return -1;
+  if ((xs & 7) || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)squares) & 15) || xs * 256 >= (1L << 31)) return -1;
+  return launch_mid<1, true, true>(x, xs, w, nullptr, y, ys, nullptr, M, N, K, 1, stream, squares, eps);
 }
 
 // residual [M, N] += x W^T, y [M, N] = rms norm of the new rows * weight; a split product (S > 1), N a multiple of 4 up to 8192.

@@ -34,7 +34,7 @@ TARGETS = {
          "kernels/lora.hip", "kernels/gemm.hip", "kernels/rans.hip", "kernels/sampling.hip",
          "kernels/grouped_gemm.hip", "kernels/packed_gemm.hip", "kernels/dense_attention.hip",
          "kernels/tile_gemm.hip", "kernels/latent.hip", "kernels/latent_mfma.hip", "kernels/seqmix.hip",
-         "kernels/chunk_scan.hip", "kernels/retention.hip", "kernels/mid_gemm.hip", "kernels/block_gemm.hip"],
+         "kernels/chunk_scan.hip", "kernels/retention.hip", "kernels/mid_gemm.hip", "kernels/block_gemm.hip", "kernels/row_gemm.hip"],
         [],
     ),
     "vpsa_kvio": ("hip", ["kvio/kvio.cpp"], []),
@@ -52,6 +52,7 @@ SOURCE_FLAGS = {
     "kernels/attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels/chunk_scan.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # the state lies in accumulators and is cut up by vector instructions
     "kernels/latent_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # the tile kernel: queries in accumulator registers, sums in the others
+    "kernels/row_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # token rows and sums in the registers that the loads fill
     "kernels/block_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # 256 registers and more: no copies between the files in the loop
 }
 # standalone executables: name -> (kind, sources, flags)

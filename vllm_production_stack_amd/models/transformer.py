@@ -310,9 +310,17 @@ class TransformerModel:
         decode_only = meta.num_prefill_seqs == 0
         adapters = self.lora is not None and meta.lora_slots is not None
         x = None  # the norm the next layer starts with, where the projection before it made it
+        rows = None  # or what it makes itself the norm from (decode steps of a few rows)
+        few = decode_only and not adapters and self.tp_size == 1 and cfg.num_experts == 0
+
+        def fits(i):
+            return few and i < len(self.layers) and ops.row_layer_takes(residual, self.layers[i], pool, meta, self.n_q, self.n_kv,
+                                                                        self.head_dim, self.cos_sin)
+
+        here = None  # whether this layer takes them, where the one before has asked
         for li, lw in enumerate(self.layers):
             gl = self.first_layer + li  # global layer index (adapters are keyed by it)
-            if x is not None:
+            if x is not None or rows is not None:
                 pass
             elif residual is None:
                 residual = h
@@ -322,12 +330,23 @@ class TransformerModel:
             else:
                 x = ops.rms_norm(h, lw.ln1, cfg.norm_eps, residual)
             attn = None
-            if not adapters:
+            if rows is not None:
+                attn = ops.row_attention_block(rows, cfg.norm_eps, lw.wqkv, lw.bqkv, pool, li, meta, self.n_q, self.n_kv, self.head_dim,
+                                               self.scale, self.cos_sin)
+            elif not adapters:
                 block = ops.decode_attention_block if decode_only else ops.prompt_attention_block
                 attn = block(x, lw.wqkv, lw.bqkv, pool, li, meta, self.n_q, self.n_kv, self.head_dim, self.scale, self.cos_sin)
             if attn is None:
                 qkv = self._lora("qkv", gl, x, ops.qkv_linear(x, lw.wqkv, lw.bqkv, self.n_q * self.head_dim), meta)
                 attn = self._attention(qkv, pool, li, meta)
+            if fits(li) if here is None else here:
+                rows = ops.row_add(attn, lw.wo, residual, lw.ln2)
+                act = ops.row_gate_up(rows, cfg.norm_eps, lw.w_gate_up)
+                here = fits(li + 1)
+                rows = ops.row_add(act, lw.w_down, residual, self.layers[li + 1].ln1 if here else None)
+                h, x, rows = None, None, rows if here else None
+                continue
+            rows = None
             x = self._out_norm("o", gl, attn, lw.wo, None, residual, lw.ln2, meta)
             if cfg.num_experts > 0:
                 h, x = tp_all_reduce(self._moe(x, lw, decode_only)), None

@@ -54,7 +54,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_chunk_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_first_chunk", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_block_gemm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_chunk_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_first_chunk", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_row_gemm_takes", "vpsa_row_add", "vpsa_row_qkv", "vpsa_mid_unit_factors", "vpsa_block_gemm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
@@ -733,6 +733,7 @@ def _stream_gemm(x2, w, bias, pair):
 #   37888 x 3584 pair    1     48.4/54.1    64      64.8/64.8  (296 workgroups: a second round nearly empty)
 #   2048 x 2048          1      5.7/7.4     64       8.7/10.6  (64 workgroups)
 MID_MIN_FILL = 0.75      # of the rounds of one workgroup per CU
+MID_MIN_FILL_ROWS = 192  # the same as workgroups
 MID_ROWS = 96            # every shape that fills the chip
 MID_ROWS_BLOCK = 128     # one round or full ones (448 workgroups win by 2 to 6 %), and partial sums (32 bits, written and read) below
 MID_BLOCK_FILL = 0.875   # MID_SUMS quarters of the weights' bytes
@@ -937,6 +938,85 @@ def decode_attention_block(x, w, bias, pool, layer, meta, n_q, n_kv, head_dim, s
     q = decode_qkv(x, w, bias, pool, layer, meta.positions, meta.slots, cos_sin, n_q, n_kv)
     if q is None:
         return None
+    out = torch.empty_like(q)
+    paged_decode(q, out, pool, layer, meta.dec_block_tables, meta.dec_ctx_lens, n_q, n_kv, head_dim, scale,
+                 getattr(meta, "dec_num_splits", 1) or 1, getattr(meta, "dec_ws_o", None), getattr(meta, "dec_ws_ml", None))
+    return out
+
+
+# ``row_gemm``'s products of a few rows (whole in one launch; what closes the one before and opens the next is made beside them) against
+# ``mid_gemm``'s, whose reductions are launches of their own, microseconds in a graph over weights that no cache holds (mid / row; q | k | v with
+# rotation and cache, output projections with the stream's update and the norm, gated unit):
+#   hidden 4096, 14336 wide    1 row 13.9/12.4  11.6/9.2   38.9/39.7  23.9/20.8    8 rows 14.5/12.8  11.9/9.3  38.8/39.3  24.6/21.2    16 rows 15.2/15.4  12.6/10.5  38.9/39.5  25.2/24.4
+#   3584, 18944                1     11.0/10.8  10.6/8.3   51.0/57.0  28.1/24.7    8      11.6/11.5  11.1/8.7  52.8/57.4  28.8/26.8    (296 workgroups: a second round)
+#   8192, 28672                1     33.2/31.6  29.2/25.8  149/150    79.2/74.3    16     33.8/37.6  29.9/28.5  148/150    79.5/92.7
+# A step of 8 layers (hidden 4096): 1 sequence 899 / 880, 2 936 / 877, 4 1098 / 1034, 8 1053 / 1006, 12 1118 / 1095, 14 1069 / 1047, 16 1072 / 1072.
+ROW_ROWS = 14
+
+
+def row_layer_takes(residual, lw, pool, meta, n_q, n_kv, head_dim, cos_sin) -> bool:
+    """Whether a decoder layer of a decode step takes ``row_gemm``'s products: few rows, projections that fill three quarters of the chip's
+    workgroups, a gated unit in one round of them, operands that the kernels read."""
+    m, h = residual.shape
+    if isinstance(pool, LayerGroupedPool):
+        pool = pool.groups[0]
+    if (m > ROW_ROWS or not residual.is_cuda or head_dim != HEAD_DIM_HIP or meta.slots is None or meta.num_decode != m or meta.num_prefill_seqs > 0
+            or lw.w_gate_up is None or lw.w_gate_up_p is not None or lw.w_down_p is not None or pool.dtype != torch.bfloat16
+            or _generic_attention(residual, head_dim) or h > 8192):
+        return False
+    q, i = n_q * head_dim, lw.w_down.shape[1]
+    if (lw.wqkv.shape != (q + 2 * n_kv * head_dim, h) or lw.wo.shape != (h, q) or lw.w_gate_up.shape != (2 * i, h) or lw.w_down.shape != (h, i)
+            or h // 16 < MID_MIN_FILL_ROWS or not MID_MIN_FILL_ROWS <= i // 64 <= TILE_CUS
+            or int(_kernels().vpsa_mid_gemm_splits(c_int(m), c_int(2 * i), c_int(h), c_int(1))) != 1):
+        return False
+    lib = _kernels()
+    if not all(lib.vpsa_row_gemm_takes(c_int(m), c_int(w.shape[0]), c_int(w.shape[1])) for w in (lw.wqkv, lw.wo, lw.w_down)):
+        return False
+    norms = [t for t in (lw.ln1, lw.ln2) if t.shape == (h,) and t.is_contiguous()]
+    if not _reads(residual, lw.wqkv, lw.bqkv) or not _reads(residual, lw.w_gate_up, None) or len(norms) < 2 or not residual.is_contiguous():
+        return False
+    ws = (lw.wo, lw.w_down)
+    return (all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.device == residual.device for w in ws)
+            and all(_lies_with(residual, t) for t in (residual, *norms, lw.wqkv, lw.wo, lw.w_gate_up, lw.w_down))
+            and (lw.bqkv is None or lw.bqkv.data_ptr() % 8 == 0) and cos_sin.data_ptr() % 16 == 0
+            and not _followed(residual, lw.wqkv, lw.bqkv, lw.wo, lw.w_gate_up, lw.w_down, *norms))
+
+
+def row_add(x, w, residual, norm):
+    """``residual += x @ w.T``; with ``norm`` also what the next product starts from: (the new rows times it, sums of 16 of their squares each)."""
+    m, n = residual.shape
+    assert x.shape == (m, w.shape[1]) and x.stride(1) == 1 and w.shape[0] == n
+    normed, squares = None, None
+    if norm is not None:
+        normed, squares = torch.empty_like(residual), torch.empty((m, n // 16), dtype=torch.float32, device=x.device)
+    _check(_kernels().vpsa_row_add(_p(x), c_long(x.stride(0)), _p(w), _p(residual), _p(norm), _p(normed), _p(squares), c_int(m), c_int(n),
+                                   c_int(w.shape[1]), _stream()), "row_add")
+    return normed, squares
+
+
+def row_gate_up(rows, eps, w):
+    """The gated unit of ``row_add``'s rows, normed."""
+    normed, squares = rows
+    m, k = normed.shape
+    y = torch.empty((m, w.shape[0] // 2), dtype=normed.dtype, device=normed.device)
+    _check(_kernels().vpsa_mid_unit_factors(_p(normed), c_long(k), _p(squares), c_float(eps), _p(w), _p(y), c_long(y.stride(0)), c_int(m),
+                                            c_int(w.shape[0]), c_int(k), _stream()), "row_gate_up")
+    return y
+
+
+def row_attention_block(rows, eps, w, bias, pool, layer, meta, n_q, n_kv, head_dim, scale, cos_sin):
+    """``decode_attention_block`` of ``row_add``'s rows, normed."""
+    if isinstance(pool, LayerGroupedPool):
+        pool, layer = pool.for_layer(layer)
+    normed, squares = rows
+    m, k = normed.shape
+    assert meta.positions.dtype == torch.int32 and meta.slots.dtype == torch.int64 and min(meta.positions.shape[0], meta.slots.shape[0]) >= m
+    assert cos_sin.dtype == torch.float32 and cos_sin.shape[1] == HEAD_DIM_HIP
+    q = torch.empty((m, n_q * HEAD_DIM_HIP), dtype=normed.dtype, device=normed.device)
+    base = pool.data_ptr() + layer * pool.stride(1) * 2
+    _check(_kernels().vpsa_row_qkv(_p(normed), c_long(k), _p(squares), c_float(eps), _p(w), _p(bias), _p(q), c_int(m), c_int(k), _p(meta.positions),
+                                   _p(meta.slots), _p(cos_sin), c_void_p(base), c_long(pool.stride(0)), c_long(pool.stride(2)), c_int(n_q),
+                                   c_int(n_kv), _stream()), "row_qkv")
     out = torch.empty_like(q)
     paged_decode(q, out, pool, layer, meta.dec_block_tables, meta.dec_ctx_lens, n_q, n_kv, head_dim, scale,
                  getattr(meta, "dec_num_splits", 1) or 1, getattr(meta, "dec_ws_o", None), getattr(meta, "dec_ws_ml", None))
