@@ -146,7 +146,7 @@ VPSA_EXPORT int vpsa_dense_decode_attention(const void* q, long q_bs, const void
 // Bidirectional attention over dense Q/K/V for 64-channel heads (speech encoder: 1500 positions
 // attending to each other; decoder prompt rows attending to the encoder output).
 //
-// One workgroup = 4 waves x 32 query rows against 64-key tiles staged through LDS (double
+// One workgroup = 4 waves x 32 query rows (or 2 pairs of waves, below) against 64-key tiles staged through LDS (double
 // buffered: the next tile is on its way to LDS during the current tile's math, one
 // barrier per tile).  Per wave and tile:
 //   S^T[64 keys x 32 queries] = K_tile . Q^T        8 x v_mfma_f32_32x32x16_bf16, K rows from LDS
@@ -160,8 +160,13 @@ VPSA_EXPORT int vpsa_dense_decode_attention(const void* q, long q_bs, const void
 // A wave and tile cost 512 cycles of matrix instructions, 512 of exponentials and 640 of other vector work, in 1500 where the chip
 // is full (32 windows x 12 heads), so vector work bounds this.  Rows of 128 B without padding (K's 16-byte chunks are swapped by key
 // bits 1..3, V's halves by key bit 1: both kinds of read stay free of bank conflicts) and tiles that go to LDS without passing
-// through registers (122 instead of 138) let four workgroups share a CU.  Of 8 windows x 12 heads the last 128 of 1152 workgroups
-// then run alone, 26 us for what takes 16 beside others.  (The next tile's scores under this one's exponentials need 182
+// through registers (122 instead of 138) let four workgroups share a CU.  Of 8 windows x 12 heads 128 of 1152 workgroups are left behind
+// the first 1024 (74.0 us by themselves); started behind them they come to lie on few CUs.  So they are cut in two (dense_attn_rows<true>: half the
+// rows, a pair of waves shares them and takes every other tile, K's and V's two tiles loaded in turn) and 256 of the first 1024, one
+// on each CU, go on with them: 84.2 -> 80.8 us, 88 pairs 79.9 -> 74.8, 22 windows x 8 heads 140.3 -> 135.4; with 256 or 512 left the halves share
+// CUs and gain nothing (89.4 / 89.6, 106 / 111), so they stay whole.  Up to 256 workgroups in all are cut as well: eight pairs 23.6 -> 15.8, 12 and
+// 16 pairs 23.9 -> 22.3 (half of the halves share a CU; 24 pairs 34.2 / 34.2), four query rows of 64 pairs 21.9 -> 14.2.  (The
+// two waves with 32 keys of every tile: 18.7 where this takes 17.7.)  (The next tile's scores under this one's exponentials need 182
 // registers: two workgroups a CU, 23.4 us for one window instead of 26.5 but 91 for 8 and 305 for 32.)  The scale goes into the
 // exponent's fused multiply, the mask only touches the last tile, and a window's query blocks run on one XCD.  Measured: 8
 // windows x 12 heads x 1500 positions 153 -> 97 us, 2 windows 55.5 -> 41, 32 windows x 8 heads 324 -> 225.  Then, with the queries waited for before the loop, K read two products ahead, the mask in a tile of its
@@ -193,18 +198,16 @@ __device__ __forceinline__ uint32_t lds_address(const uint16_t* at) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint16_t*)at;
 }
 
-__global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
+// The rows from row_of_block on of head h in window b.  PAIRS false: 128 rows, a wave takes 32 of them with all keys.  true: 64 rows, two
+// waves share 32 of them, one takes the tiles of even number, the other those of odd number, and they meet in LDS at the end.
+template <bool PAIRS>
+__device__ __forceinline__ void dense_attn_rows(
     const uint16_t* __restrict__ q, long q_bs, long q_ts, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, long kv_bs, long kv_ts, uint16_t* __restrict__ out, long o_bs,
-    long o_ts, int Tq, int Tk, int heads, int pairs, int q_blocks, float scale_log2e) {
-  __shared__ __attribute__((aligned(16))) uint16_t lds_k[2][DF_KT * 64];
-  __shared__ __attribute__((aligned(16))) uint16_t lds_v[2][DF_KT * 64];
+    long o_ts, int Tq, int Tk, int h, int b, int row_of_block, float scale_log2e, uint16_t (*lds_k)[DF_KT * 64], uint16_t (*lds_v)[DF_KT * 64]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 31, hf = lane >> 5;
-  // workgroups go round the eight XCDs: one pair's query blocks follow each other on one of them and share its L2
-  const int at = blockIdx.x >> 3, pair = at / q_blocks * 8 + (blockIdx.x & 7);
-  if (pair >= pairs) return;
-  const int h = pair % heads, b = pair / heads;
-  const int qrow = at % q_blocks * 128 + wave * 32 + r;
+  const int part = wave & 1;  // PAIRS
+  const int qrow = row_of_block + (PAIRS ? wave >> 1 : wave) * 32 + r;
   const int qc = qrow < Tq ? qrow : Tq - 1;
   const uint16_t* qp = q + b * q_bs + (long)qc * q_ts + h * 64;
   bf16x8 qf[4];
@@ -234,7 +237,22 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
     load_to_lds(v1, vd + 4096);
     ksrc = k1 + row_step, vsrc = v1 + row_step;
   };
-  stage(0);
+  // PAIRS: tiles 2 i and 2 i + 1 of one operand
+  auto stage_two = [&](int i, const uint16_t*& src, const uint16_t* base, int c, uint16_t (*to)[DF_KT * 64]) {
+    const uint32_t at = lds_address(&to[0][512 * wave]);
+    if (2 * i + 2 < n_tiles) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        load_to_lds(src, at + 4096 * x);
+        src += row_step;
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) load_to_lds(base + min(128 * i + 32 * x + row0, Tk - 1) * kv_ts + c, at + 4096 * x);
+    }
+  };
+  if constexpr (PAIRS) stage_two(0, ksrc, kbase_p, kc, lds_k);
+  else stage(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   // The queries have arrived before the loop: waited for at their first use inside it, every tile would wait there, and with them
@@ -253,22 +271,11 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
   const int tr_off = (4 * hf + tr_row) * 64 + ((16 * ((lane >> 4) & 1) + 4 * (lane & 3)) ^ ((tr_row & 2) << 4));
   const int k_off = r * 64, k_swz = (r >> 1) & 7;
 
-  auto tile = [&](int t, auto masked) {
-    const int buf = t & 1;
-    if (!masked.value) stage(t + 1);
-    // the products follow the reads at a distance of two
-    f32x16 s_acc[2];
-    bf16x8 kf[8], vf[4][2];
-    auto read_k = [&](int j) {
-      kf[j] = *(const bf16x8*)(&lds_k[buf][32 * (j >> 2) * 64 + k_off + 8 * ((2 * (j & 3) + hf) ^ k_swz)]);
-    };
-    auto read_v = [&](int s4) {
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const uint16_t* blk = &lds_v[buf][16 * s4 * 64] + (tr_off ^ (32 * cb));
-        vf[s4][cb] = lds_tr_pair(blk, blk + 8 * 64);
-      }
-    };
+  f32x16 s_acc[2];
+  // scores of a tile at kt, its first key t * 64 where some are masked; returns what the sums so far have to be multiplied with
+  auto scores = [&](const uint16_t* kt, int t, auto masked) {
+    bf16x8 kf[8];  // the products follow the reads at a distance of two
+    auto read_k = [&](int j) { kf[j] = *(const bf16x8*)(kt + 32 * (j >> 2) * 64 + k_off + 8 * ((2 * (j & 3) + hf) ^ k_swz)); };
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -289,7 +296,7 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          if (kbase + 32 * kb + 8 * (i >> 2) + 4 * hf + (i & 3) >= Tk) s_acc[kb][i] = -1e30f;
+          if (kbase + 32 * kb + 8 * (i >> 2) + 4 * hf + (i & 3) >= Tk) s_acc[kb][i] = -INFINITY;
     }
     float mx = -1e30f;
 #pragma unroll
@@ -301,6 +308,17 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
     const float m_new = fmaxf(m_run, mx);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
+    return alpha;
+  };
+  auto values = [&](const uint16_t* vt, float alpha) {
+    bf16x8 vf[4][2];
+    auto read_v = [&](int s4) {
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        const uint16_t* blk = vt + 16 * s4 * 64 + (tr_off ^ (32 * cb));
+        vf[s4][cb] = lds_tr_pair(blk, blk + 8 * 64);
+      }
+    };
     float psum = 0.f;
     read_v(0);
 #pragma unroll
@@ -314,8 +332,8 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
       u32x4 pk;
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[s4 >> 1][8 * (s4 & 1) + 2 * jj], scale_log2e, -m_new));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[s4 >> 1][8 * (s4 & 1) + 2 * jj + 1], scale_log2e, -m_new));
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[s4 >> 1][8 * (s4 & 1) + 2 * jj], scale_log2e, -m_run));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[s4 >> 1][8 * (s4 & 1) + 2 * jj + 1], scale_log2e, -m_run));
         psum += p0 + p1;
         pk[jj] = pack_bf16x2(p0, p1);
       }
@@ -324,13 +342,56 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
         o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[s4][cb], __builtin_bit_cast(bf16x8, pk), o_acc[cb], 0, 0, 0);
     }
     l_run = l_run * alpha + psum;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tile has landed
-    __syncthreads();
   };
-  for (int t = 0; t + 1 < n_tiles; ++t) tile(t, std::false_type{});
-  tile(n_tiles - 1, std::true_type{});
+  if constexpr (PAIRS) {
+    // V's two tiles are on their way during the scores, K's next two during the exponentials: each barrier ends the reads of the one
+    // and shows that the other has landed.
+    auto two = [&](int i, auto masked) {
+      stage_two(i, vsrc, vbase_p, vc, lds_v);
+      const float alpha = scores(lds_k[part], 2 * i + part, masked);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (!masked.value) stage_two(i + 1, ksrc, kbase_p, kc, lds_k);
+      values(lds_v[part], alpha);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    };
+    const int n = (n_tiles + 1) >> 1;
+    for (int i = 0; i + 1 < n; ++i) two(i, std::false_type{});
+    two(n - 1, std::true_type{});
+  } else {
+    auto tile = [&](int t, auto masked) {
+      const int buf = t & 1;
+      if (!masked.value) stage(t + 1);
+      const float alpha = scores(lds_k[buf], t, masked);
+      values(lds_v[buf], alpha);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tile has landed
+      __syncthreads();
+    };
+    for (int t = 0; t + 1 < n_tiles; ++t) tile(t, std::false_type{});
+    tile(n_tiles - 1, std::true_type{});
+  }
   // O^T accumulator register i of block cb, half hf = channel 32 cb + 8 (i >> 2) + 4 hf + (i & 3)
-  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  if constexpr (PAIRS) {  // (the tiles' places are free behind the last barrier: 34 values of 64 lanes, twice)
+    float* const ex = reinterpret_cast<float*>(&lds_k[0][0]) + (wave >> 1) * (34 * 64) + lane;
+    if (part) {
+      ex[0] = m_run;
+      ex[64] = l_tot;
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ex[(2 + 16 * cb + i) * 64] = o_acc[cb][i];
+    }
+    __syncthreads();
+    if (part) return;
+    const float m = fmaxf(m_run, ex[0]), a0 = __builtin_amdgcn_exp2f(m_run - m), a1 = __builtin_amdgcn_exp2f(ex[0] - m);
+    l_tot = l_tot * a0 + ex[64] * a1;
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o_acc[cb][i] = o_acc[cb][i] * a0 + ex[(2 + 16 * cb + i) * 64] * a1;
+  }
   if (qrow < Tq) {
     const float inv = 1.f / l_tot;
     uint16_t* op = out + b * o_bs + (long)qrow * o_ts + h * 64;
@@ -346,6 +407,27 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
   }
 }
 
+// Blocks of 128 rows, by `whole` workgroups (a multiple of 8); `left` blocks more in two of 64 each, by those workgroups from `first` on
+// when they are done with theirs (whole 0: by workgroups of their own).
+__global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
+    const uint16_t* __restrict__ q, long q_bs, long q_ts, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, long kv_bs, long kv_ts, uint16_t* __restrict__ out, long o_bs,
+    long o_ts, int Tq, int Tk, int heads, int pairs, int q_blocks, int whole, int first, int left, float scale_log2e) {
+  __shared__ __attribute__((aligned(16))) uint16_t lds[4][DF_KT * 64];
+  // workgroups go round the eight XCDs: one pair's query blocks follow each other on one of them and share its L2
+  const int xcd = blockIdx.x & 7;
+  auto rows = [&](auto pairs_of_waves, int at, int row) {
+    const int pair = at / q_blocks * 8 + xcd;
+    row += at % q_blocks * 128;
+    if (pair < pairs && row < Tq)
+      dense_attn_rows<decltype(pairs_of_waves)::value>(q, q_bs, q_ts, k, v, kv_bs, kv_ts, out, o_bs, o_ts, Tq, Tk, pair % heads, pair / heads,
+                                                       row, scale_log2e, lds, lds + 2);
+  };
+  if ((int)blockIdx.x < whole) rows(std::false_type{}, blockIdx.x >> 3, 0);
+  const int past = (int)blockIdx.x - first;
+  if (past >= 0 && past < 2 * left) rows(std::true_type{}, (whole >> 3) + (past >> 4), (past >> 3 & 1) * 64);
+}
+
 // q [B][Tq][heads * 64], k / v [B][Tk][heads * 64], out [B][Tq][heads * 64]; strides in elements
 // (batch, position), unit stride over channels, every row start 16-byte aligned (out: 8-byte).
 // Every query attends to every key.  Returns -1 for arguments the kernel does not cover.
@@ -359,8 +441,11 @@ VPSA_EXPORT int vpsa_dense_attention(const void* q, long q_bs, long q_ts, const 
   const int q_blocks = (Tq + 127) / 128;
   const long pairs = (long)B * heads, groups = (pairs + 7) / 8 * 8 * q_blocks;
   if (groups >= (1L << 31)) return -1;
-  hipLaunchKernelGGL(dense_attn_fwd_kernel, dim3((unsigned)groups), dim3(256), 0, stream,
+  int left = (int)(groups % 1024);  // (behind whole rounds of four a CU; the lines: see above)
+  if (left > (groups < 1024 ? 256 : 128) || Tk <= DF_KT) left = 0;  // (two tiles at least)
+  const int whole = (int)groups - left;
+  hipLaunchKernelGGL(dense_attn_fwd_kernel, dim3(whole ? whole : 2 * left), dim3(256), 0, stream,
                      (const uint16_t*)q, q_bs, q_ts, (const uint16_t*)k, (const uint16_t*)v, kv_bs, kv_ts,
-                     (uint16_t*)out, o_bs, o_ts, Tq, Tk, heads, (int)pairs, q_blocks, scale * 1.4426950408889634f);
+                     (uint16_t*)out, o_bs, o_ts, Tq, Tk, heads, (int)pairs, q_blocks, whole, whole ? whole - 1024 : 0, left, scale * 1.4426950408889634f);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
