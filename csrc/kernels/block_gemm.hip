@@ -8,11 +8,15 @@
 //     the matrix cores work on the half before, so that a lone wave on a SIMD keeps them busy; the chunk's place in the ring is
 //     requested again right behind that barrier, S - 1/2 chunks ahead of its use.
 //   * The weight rows are the MFMA's A operand and are ordered so that a lane ends with eight consecutive columns of a token row.
+//   * Where there are more tiles than the chip holds at once, as many workgroups as it holds make several each: the ring goes on with the next
+//     tile's chunks while the last ones of a tile are multiplied and its epilogue runs.
 // What bounds it: LDS, which carries (reads and the loads' writes) 128 bytes for every 64 x 96 x 96 of products in the largest shape, as many
 // cycles as the matrix cores need; with short reductions the time until a tile's first chunk is there and its epilogue (gelu 75
 // cycles of vector work a wave and value).  12000 rows in a loop over the same operands, library with the activation's pass / this: 3072 x
 // 768 with gelu 107 / 70 us, 768 x 3072 57 / 48 (+ residual), three of 768 x 768 62 / 48, 768 x 2304 with gelu 50 / 42; 1500 rows, 2048 x 512 with
-// gelu 26 / 11.  In an encoder of 12 layers, where a product's operands come from memory, the first three take 82 to 86, 56 to 58 and 55 to 58.
+// gelu 26 / 11.  Over operands that no cache holds, a workgroup for every tile / several tiles a workgroup with the costs below: the first
+// 78.9 / 72.7, the second 62.4 / 62.4, the third 53.5 / 45.7, one 768 x 768 with a residual 25.6 / 22.6, 117 products of 1500 to 48000 rows 6 % (one, 7500
+// rows of 768 x 3072, 44 / 54); an encoder of 12 layers, 8 windows 3733 / 3565, 2 1746 / 1640, 32 13.66 / 12.97 ms, none of 1 to 32 windows slower.
 #include <type_traits>
 
 #include "common.h"
@@ -57,8 +61,9 @@ __device__ __forceinline__ float gelu(float x) {
   return x * (x >= 0.f ? 1.f - h : h);
 }
 
-// STREAM: few row tiles, weights read about once, by non-temporal loads and from another chunk on for every column tile.
-template <int TM, int TN, int S, int ACT, bool STREAM>
+// STREAM: few row tiles, weights read about once, by non-temporal loads and from another chunk on for every column tile.  MANY: a workgroup
+// makes several tiles.
+template <int TM, int TN, int S, int ACT, bool STREAM, bool MANY>
 __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void block_gemm_kernel(const BlockArgs args) {
   constexpr bool PAIR = ACT == ACT_SILU;
   constexpr int BM = 32 * TM, BN = 32 * TN, STAGE = (BM + BN) * ROWB, NL = TM + TN;
@@ -69,52 +74,61 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
 
   // Tiles in blocks of an eighth of the row tiles (up to eight), column by column inside a block, cut in eight runs, one per XCD
   // (workgroups go round them): those that share an L2 at any time are about a square of tiles.
-  int m0, n0, part, split = 0, c0 = 0, n = K / BK, first = 0;  // chunks c0 .. c0 + n - 1 of the reduction, from c0 + first round
-  {
-    const int m_tiles = (M + BM - 1) / BM, cols = args.n_tiles * args.parts, tiles = m_tiles * cols, total = STREAM ? tiles * args.splits : tiles, blk = min(8, (m_tiles + 7) / 8);
-    const int bid = blockIdx.x, xcd = bid & 7, q = total >> 3, r = total & 7;
-    int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
+  const int m_tiles = (M + BM - 1) / BM, cols = args.n_tiles * args.parts, tiles = m_tiles * cols, total = STREAM ? tiles * args.splits : tiles;
+  const int xcd = blockIdx.x & 7, run = (total >> 3) + (xcd < (total & 7)), run0 = xcd * (total >> 3) + min(xcd, total & 7);
+  int at = blockIdx.x >> 3;  // in the run; then every (gridDim.x + 7) / 8-th
+  int split = 0, c0 = 0, n = K / BK, first = 0;  // chunks c0 .. c0 + n - 1 of the reduction, from c0 + first round
+  int m0, n0, part;                              // the tile whose chunks are loaded
+  auto place = [&]() {
+    int t = run0 + at;
     if (STREAM) {
       split = t / tiles;
       t -= split * tiles;
-      const int per = n / args.splits, extra = n - per * args.splits;
-      c0 = split * per + min(split, extra);
-      n = per + (split < extra);
     }
-    const int block = t / (blk * cols), rem = t - block * blk * cols, rows = min(blk, m_tiles - blk * block);
+    const int blk = min(8, (m_tiles + 7) / 8), block = t / (blk * cols), rem = t - block * blk * cols, rows = min(blk, m_tiles - blk * block);
     const int col = rem / rows;
     m0 = (blk * block + rem - col * rows) * BM;
     part = col / args.n_tiles;
     n0 = (col - part * args.n_tiles) * BN;
-    if (STREAM) first = col * 3 % n;
-  }
+    if (STREAM) {
+      const int per = n / args.splits, extra = n - per * args.splits;
+      c0 = split * per + min(split, extra);
+      n = per + (split < extra);
+      first = col * 3 % n;
+    }
+  };
+  place();
 
   // what this lane loads of a chunk: 8 rows of 8 pieces a KiB; rows past the last repeat it
   uint32_t aoff[TM], woff[TN];
   const int lrow = lane >> 3;
+  auto rows_of_tile = [&]() {
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int r = 8 * (4 * i + wave) + lrow, row = min(m0 + r, M - 1);
-    const int b = row / args.batch_rows;
-    aoff[i] = (uint32_t)((b * args.ar.bs + (row - b * args.batch_rows) * args.ar.ld) * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
-  }
+    for (int i = 0; i < TM; ++i) {
+      const int r = 8 * (4 * i + wave) + lrow, row = min(m0 + r, M - 1);
+      const int b = row / args.batch_rows;
+      aoff[i] = (uint32_t)((b * args.ar.bs + (row - b * args.batch_rows) * args.ar.ld) * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
 #pragma unroll
-  for (int i = 0; i < TN; ++i) {
-    const int r = 8 * (4 * i + wave) + lrow, rr = r % (16 * TN), j = rr & 15, perm = 8 * (j >> 2) + 4 * ((rr >> 4) & 1) + (j & 3);
-    // PAIR: tiles 2 b, 2 b + 1 of a wave are 16 gate rows and the up rows beside them
-    const int col = PAIR ? n0 / 2 + r / (16 * TN) * (8 * TN) + 16 * (rr >> 5) + j : n0 + r / (16 * TN) * (16 * TN) + 32 * (rr >> 5) + perm;
-    const int row = PAIR ? min(col, N / 2 - 1) + ((rr >> 4) & 1 ? N / 2 : 0) : min(col, N - 1);
-    woff[i] = (uint32_t)row * (uint32_t)(K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
-  }
-  auto load = [&](int c, char* st, int i) {  // the i-th KiB of this wave; nothing past the last chunk (a buffer of no bytes)
+    for (int i = 0; i < TN; ++i) {
+      const int r = 8 * (4 * i + wave) + lrow, rr = r % (16 * TN), j = rr & 15, perm = 8 * (j >> 2) + 4 * ((rr >> 4) & 1) + (j & 3);
+      // PAIR: tiles 2 b, 2 b + 1 of a wave are 16 gate rows and the up rows beside them
+      const int col = PAIR ? n0 / 2 + r / (16 * TN) * (8 * TN) + 16 * (rr >> 5) + j : n0 + r / (16 * TN) * (16 * TN) + 32 * (rr >> 5) + perm;
+      const int row = PAIR ? min(col, N / 2 - 1) + ((rr >> 4) & 1 ? N / 2 : 0) : min(col, N - 1);
+      woff[i] = (uint32_t)row * (uint32_t)(K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
+  };
+  rows_of_tile();
+  bool more = false;  // behind the last chunk come those of the next tile
+  auto load = [&](int c, char* st, int i) {  // the i-th KiB of this wave; nothing past the last tile's last chunk (a buffer of no bytes)
     const bool x = i < TM;
     const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(x ? args.a : args.w[part]), 0, c < n ? (int)(x ? args.a_bytes : args.w_bytes) : 0, 0x00020000);
+        (void*)(x ? args.a : args.w[part]), 0, c < n || (MANY && more) ? (int)(x ? args.a_bytes : args.w_bytes) : 0, 0x00020000);
     const auto to = (__attribute__((address_space(3))) void*)(st + (4 * i + wave) * 1024);
     const int off = (int)(x ? aoff[i % TM] : woff[(i - TM + TN) % TN]);
-    const int at = c >= n ? 0 : STREAM ? (c0 + (c + first < n ? c + first : c + first - n)) * ROWB : c * ROWB;
-    if (STREAM && !x) __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to, 16, off, at, 0, 2);
-    else __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to, 16, off, at, 0, 0);
+    const int from = c >= n ? (MANY && more ? (c - n) * ROWB : 0) : STREAM ? (c0 + (c + first < n ? c + first : c + first - n)) * ROWB : c * ROWB;
+    if (STREAM && !x) __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to, 16, off, from, 0, 2);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to, 16, off, from, 0, 0);
   };
 
   // fragments: row c16 of a 16-row tile, piece 4 ks + g
@@ -127,10 +141,6 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
     else wf[ks][(i - TM + TN) % TN] = *reinterpret_cast<const bf16x8*>(st + w_rd + (i - TM) * 2048 + f);
   };
   f32x4 acc[TN][TM];
-#pragma unroll
-  for (int i = 0; i < TN; ++i)
-#pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   // Half a chunk: its matrix instructions, between the first two thirds of them the reads of the half that follows (from `from`) and
   // between all of them the requests [lo, hi) of a later chunk c (into `to`).  The order is written out: left alone, the compiler puts
   // all loads in front.
@@ -163,124 +173,158 @@ __global__ __launch_bounds__(256, (TM + TN) * S * 4096 <= 81920 ? 2 : 1) void bl
   char *st = lds, *prev = lds + (S - 1) * STAGE;
 #pragma unroll
   for (int i = 0; i < NL; ++i) read(st, 0, i);
-  for (int c = 0; c < n; ++c) {
-    half(0, st, L0, NL, c + S - 1, prev);
-    // chunk c + 1 has landed (mine: all but the loads of the chunks behind it) and my reads of chunk c are done; everyone's: the barrier
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * NL) : "memory");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    prev = st;
-    st = st + STAGE == lds + S * STAGE ? lds : st + STAGE;
-    half(1, st, 0, L0, c + S, prev);
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still write to LDS when the wave ends
+  for (;;) {  // a tile
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int tm0 = m0, tn0 = n0, tpart = part;  // the tile that is multiplied
+    for (int c = 0; c < n; ++c) {
+      half(0, st, L0, NL, c + S - 1, prev);
+      // chunk c + 1 has landed (mine: all but the loads of the chunks behind it) and my reads of chunk c are done; everyone's: the barrier
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * NL) : "memory");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      prev = st;
+      st = st + STAGE == lds + S * STAGE ? lds : st + STAGE;
+      if (MANY && c + S == n) {
+        at += (gridDim.x + 7) >> 3;
+        more = at < run;
+        if (more) {
+          asm volatile("" ::: "memory");  // a branch: without it the compiler works the places out in every chunk and selects
+          place();
+          rows_of_tile();
+          asm volatile("" ::: "memory");
+        }
+      }
+      half(1, st, 0, L0, c + S, prev);
+    }
+    if (!MANY || !more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still write to LDS when the wave ends
 
-  // accumulator [i][j]: token row 16 j + c16 of the wave's; registers of tiles 2 b, 2 b + 1: columns 8 g .. 8 g + 7 of the 32 of pair b
-  constexpr int NB = TN / 2;
-  if (STREAM && args.splits > 1) {
-    float* const ws = args.ws + (long)split * M * N;
+    // accumulator [i][j]: token row 16 j + c16 of the wave's; registers of tiles 2 b, 2 b + 1: columns 8 g .. 8 g + 7 of the 32 of pair b
+    constexpr int NB = TN / 2;
+    if (STREAM && args.splits > 1) {
+      float* const ws = args.ws + (long)split * M * N;
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int row = m0 + wr * 16 * TM + 16 * j + c16;
-      if (row >= M) continue;
+      for (int j = 0; j < TM; ++j) {
+        const int row = tm0 + wr * 16 * TM + 16 * j + c16;
+        if (row >= M) continue;
 #pragma unroll
-      for (int i = 0; i < TN; ++i) {
-        const int col = PAIR ? n0 / 2 + wc * 8 * TN + 16 * (i >> 1) + 4 * g : n0 + wc * 16 * TN + 32 * (i >> 1) + 8 * g + 4 * (i & 1);
-        if (col < (PAIR ? N / 2 : N)) *reinterpret_cast<f32x4*>(ws + (long)row * N + col + (PAIR && (i & 1) ? N / 2 : 0)) = acc[i][j];
+        for (int i = 0; i < TN; ++i) {
+          const int col = PAIR ? tn0 / 2 + wc * 8 * TN + 16 * (i >> 1) + 4 * g : tn0 + wc * 16 * TN + 32 * (i >> 1) + 8 * g + 4 * (i & 1);
+          if (col < (PAIR ? N / 2 : N)) *reinterpret_cast<f32x4*>(ws + (long)row * N + col + (PAIR && (i & 1) ? N / 2 : 0)) = acc[i][j];
+        }
       }
+      return;
     }
-    return;
-  }
-  if constexpr (PAIR) {
+    if constexpr (PAIR) {
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int row = m0 + wr * 16 * TM + 16 * j + c16;
-      if (row >= M) continue;
+      for (int j = 0; j < TM; ++j) {
+        const int row = tm0 + wr * 16 * TM + 16 * j + c16;
+        if (row >= M) continue;
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const int col = n0 / 2 + wc * 8 * TN + 16 * b + 4 * g;
-        if (col >= N / 2) continue;
-        f32x4 s = acc[2 * b][j];
+        for (int b = 0; b < NB; ++b) {
+          const int col = tn0 / 2 + wc * 8 * TN + 16 * b + 4 * g;
+          if (col >= N / 2) continue;
+          f32x4 s = acc[2 * b][j];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] = s[e] / (1.f + __expf(-s[e])) * acc[2 * b + 1][j][e];
-        *reinterpret_cast<u32x2*>(args.c + row * args.cr.ld + col) = (u32x2){pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+          for (int e = 0; e < 4; ++e) s[e] = s[e] / (1.f + __expf(-s[e])) * acc[2 * b + 1][j][e];
+          *reinterpret_cast<u32x2*>(args.c + row * args.cr.ld + col) = (u32x2){pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+        }
       }
+      return;
     }
-    return;
-  }
-  const int col0 = n0 + wc * 16 * TN + 8 * g;
-  u32x4 bias[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    bias[b] = (u32x4){0, 0, 0, 0};
-    if (args.bias[part] != nullptr && col0 + 32 * b < N)
-      bias[b] = *reinterpret_cast<const u32x4*>(args.bias[part] + col0 + 32 * b);
-  }
-#pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int row = m0 + wr * 16 * TM + 16 * j + c16;
-    if (row >= M) continue;
-    const int bt = row / args.batch_rows, tr = row - bt * args.batch_rows;
-    uint16_t* const cp = args.c + bt * args.cr.bs + tr * args.cr.ld + (long)part * N;
-    const uint16_t* const rp = args.res + bt * args.rr.bs + tr * args.rr.ld;
+    const int col0 = tn0 + wc * 16 * TN + 8 * g;
+    u32x4 bias[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int col = col0 + 32 * b;
-      if (col >= N) continue;
-      float v[8];
-#pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        v[p] = acc[2 * b + (p >> 2)][j][p & 3] + (p & 1 ? bf16hi(bias[b][p >> 1]) : bf16lo(bias[b][p >> 1]));
-        if (ACT == ACT_GELU) v[p] = gelu(v[p]);
-      }
-      if (args.res != nullptr) {
-        const u32x4 r = *reinterpret_cast<const u32x4*>(rp + col);
-#pragma unroll
-        for (int p = 0; p < 8; ++p) v[p] += p & 1 ? bf16hi(r[p >> 1]) : bf16lo(r[p >> 1]);
-      }
-      const u32x4 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
-      *reinterpret_cast<u32x4*>(cp + col) = o;
+      bias[b] = (u32x4){0, 0, 0, 0};
+      if (args.bias[tpart] != nullptr && col0 + 32 * b < N)
+        bias[b] = *reinterpret_cast<const u32x4*>(args.bias[tpart] + col0 + 32 * b);
     }
+    // waited for here: on its way into the next tile, past rows that are not there, it would be waited for among the first reads of every chunk
+    if (MANY) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) asm volatile("" : "+v"(bias[b]));
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int row = tm0 + wr * 16 * TM + 16 * j + c16;
+      if (row >= M) continue;
+      const int bt = row / args.batch_rows, tr = row - bt * args.batch_rows;
+      uint16_t* const cp = args.c + bt * args.cr.bs + tr * args.cr.ld + (long)tpart * N;
+      const uint16_t* const rp = args.res + bt * args.rr.bs + tr * args.rr.ld;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int col = col0 + 32 * b;
+        if (col >= N) continue;
+        float v[8];
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+          v[p] = acc[2 * b + (p >> 2)][j][p & 3] + (p & 1 ? bf16hi(bias[b][p >> 1]) : bf16lo(bias[b][p >> 1]));
+          if (ACT == ACT_GELU) v[p] = gelu(v[p]);
+        }
+        if (args.res != nullptr) {
+          const u32x4 r = *reinterpret_cast<const u32x4*>(rp + col);
+#pragma unroll
+          for (int p = 0; p < 8; ++p) v[p] += p & 1 ? bf16hi(r[p >> 1]) : bf16lo(r[p >> 1]);
+        }
+        const u32x4 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+        *reinterpret_cast<u32x4*>(cp + col) = o;
+      }
+    }
+    if (!MANY || !more) return;
+    more = false;
   }
+}
+
+template <int TM, int TN, int S, int ACT, bool STREAM, bool MANY>
+int start(const BlockArgs& args, long blocks, hipStream_t stream) {
+  constexpr int LDS = (TM + TN) * S * 4096;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)block_gemm_kernel<TM, TN, S, ACT, STREAM, MANY>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) !=
+        hipSuccess)
+      return -2;
+    attr_set = true;
+  }
+  block_gemm_kernel<TM, TN, S, ACT, STREAM, MANY><<<dim3((unsigned)blocks), 256, LDS, stream>>>(args);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 template <int TM, int TN, int S, int ACT, bool STREAM = false>
 int launch(BlockArgs& args, hipStream_t stream) {
-  constexpr int LDS = (TM + TN) * S * 4096;
-  static bool attr_set = false;
-  if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)block_gemm_kernel<TM, TN, S, ACT, STREAM>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
-      return -2;
-    attr_set = true;
-  }
   args.n_tiles = (args.N + 32 * TN - 1) / (32 * TN);
   const long blocks = (long)args.n_tiles * args.parts * args.splits * ((args.M + 32 * TM - 1) / (32 * TM));
   if (blocks >= (1L << 31)) return -1;
-  block_gemm_kernel<TM, TN, S, ACT, STREAM><<<dim3((unsigned)blocks), 256, LDS, stream>>>(args);
-  return hipGetLastError() == hipSuccess ? 0 : -3;
+  constexpr int ROUND = (TM + TN) * S * 4096 <= 81920 ? 512 : 256;  // what the chip holds
+  if constexpr (!STREAM)
+    if (blocks > ROUND && args.K / BK >= S) return start<TM, TN, S, ACT, false, true>(args, ROUND, stream);
+  return start<TM, TN, S, ACT, STREAM, false>(args, blocks, stream);
 }
 
-// The tile shapes, and what they cost: microseconds a chunk and beside the chunks (start, epilogue, and more of it with gelu) of a
-// round of one workgroup a CU, or, where two share a CU, of a round of two (a round that leaves half the places empty runs faster: its
-// own pair of numbers).  Fitted to the speech encoder's products (N, K of 512 to 3072, 1500 to 48000 rows); the choice by them is 2.6 %
-// off the best shape on average.
+// The tile shapes, and what they cost in microseconds: a chunk and what stands beside a tile's chunks (epilogue) in a round of one
+// workgroup a CU, or, where two share a CU, of two (a round that leaves at least half the places empty has a CU to each workgroup and a pair of
+// numbers of its own; beyond that some CU has two); more of the epilogue with gelu and with a residual; a launch's start.  Fitted to the speech
+// encoder's products (N, K of 512 to 3072, 1500 to 48000 rows, 117 in all); the choice by them is 0.8 % off the best shape on average, at the most
+// 13 (counting half-empty rounds in proportion: 3.0 and 28).
 struct Shape {
   int bm, bn, per_cu;
-  float chunk, fixed, chunk1, fixed1, gelu;
+  float chunk, fixed, chunk1, fixed1, gelu, res, start;
 };
-constexpr Shape SHAPES[] = {{192, 192, 1, 0.76f, 8.38f, 0.f, 0.f, 3.f}, {128, 128, 1, 0.44f, 4.04f, 0.f, 0.f, 1.58f}, {128, 128, 2, 0.95f, 4.54f, 0.61f, 2.54f, 1.53f},
-                            {64, 128, 2, 0.60f, 2.09f, 0.27f, 2.87f, 0.78f},  {192, 128, 2, 1.36f, 5.82f, 0.75f, 3.69f, 2.17f}, {96, 192, 2, 1.09f, 4.70f, 0.66f, 2.74f, 1.38f}};
+constexpr Shape SHAPES[] = {{192, 192, 1, 0.79f, 4.70f, 0.f, 0.f, 5.27f, 7.16f, 1.71f},   {128, 128, 1, 0.47f, 2.48f, 0.f, 0.f, 2.13f, 2.81f, 1.02f},
+                            {128, 128, 2, 0.95f, 2.45f, 0.64f, 2.22f, 2.38f, 4.28f, 2.12f}, {64, 128, 2, 0.63f, 1.25f, 0.32f, 0.96f, 0.98f, 1.97f, 1.86f},
+                            {192, 128, 2, 1.29f, 3.15f, 0.73f, 2.98f, 3.89f, 5.85f, 3.30f}, {96, 192, 2, 1.20f, 1.04f, 0.69f, 2.77f, 3.02f, 4.82f, 2.48f}};
 
-int choose(int M, int N, int K, int parts, int act) {
+int choose(int M, int N, int K, int parts, int act, bool res) {
   int best = 0;
   double best_t = 0;
   for (int i = 0; i < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); ++i) {
     const Shape& s = SHAPES[i];
-    const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * parts, round = 256 * s.per_cu;
-    const double gelu = act == ACT_GELU ? s.gelu : 0, full = K / BK * s.chunk + s.fixed + gelu;
-    const double half = s.per_cu > 1 ? K / BK * s.chunk1 + s.fixed1 + gelu / 2 : full;
-    const double left = (double)(tiles % round) / round;
-    const double t = tiles / round * full + (left == 0 ? 0 : left <= 0.5 ? half : half + (full - half) * (2 * left - 1));
+    const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * parts, round = 256 * s.per_cu, left = tiles % round;
+    const double more = (act == ACT_GELU ? s.gelu : 0) + (res ? s.res : 0), full = K / BK * s.chunk + s.fixed + more;
+    const double half = K / BK * s.chunk1 + s.fixed1 + more / 2;
+    const double t = s.start + tiles / round * full + (left == 0 ? 0 : s.per_cu > 1 && 2 * left <= round ? half : full);
     if (i == 0 || t < best_t) best = i, best_t = t;
   }
   return best;
@@ -310,7 +354,7 @@ VPSA_EXPORT int vpsa_block_gemm(const void* x, long ld, long bs, const void* w0,
                     (const uint16_t*)res, (uint16_t*)c, {ld, bs}, {ldc, cbs}, {ldr, rbs}, batch_rows, M, N, K, 0, parts, nullptr, 1,
                     (uint32_t)a_bytes, (uint32_t)w_bytes};
 #define SHAPE(TM, TN, S) return act == ACT_GELU ? launch<TM, TN, S, ACT_GELU>(args, stream) : launch<TM, TN, S, ACT_NONE>(args, stream)
-  switch (choose(M, N, K, parts, act)) {
+  switch (choose(M, N, K, parts, act, res != nullptr)) {
     case 0: SHAPE(6, 6, 3);
     case 1: SHAPE(4, 4, 4);
     case 2: SHAPE(4, 4, 2);
