@@ -359,7 +359,7 @@ __global__ __launch_bounds__(1024) void mid_reduce_norm_kernel(const float* __re
   }
 }
 
-// The reduction of a decode step's q | k | v projection, heads of 128 channels: q rotated to `q_out` [M, n_q * 128], k rotated and v to the
+// The reduction of a decode step's or short prompts' q | k | v projection, heads of 128 channels: q rotated to `q_out` [M, n_q * 128], k rotated and v to the
 // token's slot of the paged cache.  Grid (M, head groups of 8), 32 lanes a head: lane j holds channels 2 j, 2 j + 1 and their
 // rotation partners 64 further on.  Rounded to 16 bits before and after the rotation, as the separate passes do: what it saves
 // is their two launches (the same steps: one sequence 1724 -> 1677 us, 12 sequences 2088 -> 2028, 40 sequences of 21.5k tokens, 8 layers, 5134 -> 5103).

@@ -618,7 +618,7 @@ VPSA_EXPORT hipStream_t vpsa_page_copy_stream() {
   return mine;
 }
 
-// The copy of a page on that stream, so that it runs beside the kernels of the page before it (3.5 MB: 70 us of copy, 53 of kernels);
+// The copy of a page on that stream, so that it runs beside the kernels of the page before it (3.5 MB: 67 us of copy, 30 of kernels);
 // `stream` waits for it, and it for nothing but the copies before it: all callers share it.  fresh: `body` is new to the caller, and what
 // `stream` still has to do may touch its memory; the copy then stands in `stream`, where nobody else waits for it.  Below 2 MB the
 // events cost the host, which is behind there anyway, what the copy takes (a page of 1.5 MB of many, one stream / two: 87 / 91 us; of 3.5 MB
