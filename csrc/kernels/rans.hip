@@ -277,71 +277,6 @@ __global__ __launch_bounds__(256) void rans_pack_kernel(const uint8_t* __restric
   }
 }
 
-// A page's parts straight into pinned host memory `to` (16-byte aligned): the first workgroups write the coded bytes of 64 streams each behind the
-// `head_bytes` (a multiple of 16) that the others copy from `head`, in pieces of 16 bytes on their boundaries, gathered in LDS; the
-// pieces that two groups share go byte by byte.  Nothing past `cap`.  meta as rans_pack_kernel's.  What bounds it is the link: 3.45 MB take 61 us; by
-// way of device memory, with the host in between to learn the size, 15 + 64 and two waits (a whole page, host included, 208 -> 197 us; of 1.7 MB 155 -> 144).
-#define PUBLISH_HEAD_GROUPS 16
-__global__ __launch_bounds__(256) void rans_publish_kernel(const uint8_t* __restrict__ scratch, const uint16_t* __restrict__ sizes,
-                                                           const uint32_t* __restrict__ group_bytes, int groups, int slot,
-                                                           const u32x4* __restrict__ head, long head_bytes, uint8_t* __restrict__ to, long cap,
-                                                           const int* __restrict__ err, int n_ctx, long* __restrict__ meta) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  __shared__ long part[4];
-  __shared__ int at[64], len[64];
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, group = blockIdx.x;
-  if (group >= groups) {
-    const long n = head_bytes / 16;
-    u32x4* const out = reinterpret_cast<u32x4*>(to);
-    for (long i = (long)(group - groups) * 256 + t; i < n && i * 16 + 16 <= cap; i += 256 * PUBLISH_HEAD_GROUPS) out[i] = head[i];
-    return;
-  }
-  long sum = 0;
-  for (int i = t; i < group; i += 256) sum += group_bytes[i];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  if (lane == 0) part[wave] = sum;
-  if (wave == 0) {
-    const int n = sizes[(long)group * 64 + lane];
-    at[lane] = wave_before(n);
-    len[lane] = n;
-  }
-  __syncthreads();
-  const long base = part[0] + part[1] + part[2] + part[3], first = head_bytes + base;
-  const int lead = (int)(first & 15), all = at[63] + len[63];
-#pragma unroll 8
-  for (int i = 0; i < 16; ++i) {
-    const int s = wave * 16 + i, n = len[s];
-    const uint8_t* src = scratch + ((long)group * 64 + s) * slot + (slot - n);
-    uint8_t* dst = lds + lead + at[s];
-    uint8_t v[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = lane + 64 * q < n ? src[lane + 64 * q] : 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (lane + 64 * q < n) dst[lane + 64 * q] = v[q];
-    for (int q = lane + 256; q < n; q += 64) dst[q] = src[q];
-  }
-  __syncthreads();
-  // byte j of LDS is byte first - lead + j of the page; whole pieces [p0, p1) are this group's alone
-  uint8_t* const out = to + (first - lead);
-  const int room = (int)(cap - (first - lead) < lead + all ? (cap > first - lead ? cap - (first - lead) : 0) : lead + all);
-  const int p0 = lead ? 1 : 0, p1 = room / 16;
-  for (int p = p0 + t; p < p1; p += 256) reinterpret_cast<u32x4*>(out)[p] = reinterpret_cast<const u32x4*>(lds)[p];
-  if (t < 16 && lead && t >= lead && t < room) out[t] = lds[t];
-  const int j = p1 * 16 + (t - 64);
-  if (t >= 64 && t < 80 && p1 >= p0 && j < room) out[j] = lds[j];
-  if (group == groups - 1) {
-    int bad = 0;
-    for (int i = t; i < n_ctx; i += 256) bad += err[i];
-    bad = __syncthreads_count(bad != 0);
-    if (t == 0) {
-      meta[0] = base + all;
-      meta[1] = bad;
-    }
-  }
-}
-
 // A stream's symbols; `pair` gives the two bytes at a place of the wave's coded bytes, the first one higher, from LDS or (streams too
 // long for it) from memory.  Two copies of the loop: one that may load from memory waits for its own stores at every step.  DIR: which way the
 // places run.  What bounds it is the chain from a state to the next, and every instruction of a wave that has its SIMD to itself stands in
@@ -499,65 +434,27 @@ VPSA_EXPORT long vpsa_rans_workspace(long n, int n_ctx, int spc) {
   return (long)n_ctx * (RANS_HIST_BLOCKS * 1024 + 4096 + 16) + (long)n_ctx * spc * (4 + rans_slot(n, n_ctx, spc));
 }
 
-struct RansWork {
-  uint32_t* part;
-  u32x4* table;
-  int* err;
-  uint32_t* group_bytes;
-  uint8_t* scratch;
-};
-static RansWork rans_work(void* ws, int n_ctx, int spc) {
-  RansWork w;
-  w.part = (uint32_t*)ws;
-  w.table = (u32x4*)((char*)ws + (long)n_ctx * RANS_HIST_BLOCKS * 1024);
-  w.err = (int*)(w.table + (long)n_ctx * 256);
-  w.group_bytes = (uint32_t*)((char*)w.err + (long)n_ctx * 16);
-  w.scratch = (uint8_t*)(w.group_bytes + (long)n_ctx * spc);
-  return w;
-}
-
-// Histogram -> table -> per-stream coding, every stream's bytes in its slot.
-static void rans_code(const void* sym, long n, int n_ctx, int spc, const RansWork& w, void* freq, void* states, void* sizes, hipStream_t stream) {
-  const long ctx_len = n / n_ctx, per_block = (ctx_len / 4 + 255) / 256;
-  const int hb = (int)(per_block > RANS_HIST_BLOCKS ? RANS_HIST_BLOCKS : per_block);
-  hipLaunchKernelGGL(rans_hist_kernel, dim3(hb, n_ctx), dim3(256), 0, stream, (const uint8_t*)sym, w.part, ctx_len);
-  hipLaunchKernelGGL(rans_normalize_kernel, dim3(n_ctx), dim3(256), 0, stream, w.part, hb, (uint16_t*)freq, w.table, ctx_len, w.err);
-  hipLaunchKernelGGL(rans_encode_kernel, dim3(spc / 64, n_ctx), dim3(64), 0, stream, (const uint8_t*)sym, w.table, w.scratch,
-                     (uint32_t*)states, (uint16_t*)sizes, w.group_bytes, ctx_len, spc, rans_slot(n, n_ctx, spc));
-}
-
 // Histogram -> table -> per-stream coding -> dense bytes.  freq u16 [n_ctx * 256], states u32 and sizes u16 [n_ctx * spc], coded
 // with room for 2 n bytes, meta i64 [2] = coded bytes, contexts that could not be normalised; ws 16-byte aligned.
 VPSA_EXPORT int vpsa_rans_encode(const void* sym, long n, int n_ctx, int spc, void* ws, void* freq, void* states, void* sizes,
                                  void* coded, long* meta, hipStream_t stream) {
   if (!rans_shape_ok(n, n_ctx, spc)) return -1;
-  const RansWork w = rans_work(ws, n_ctx, spc);
-  rans_code(sym, n, n_ctx, spc, w, freq, states, sizes, stream);
-  hipLaunchKernelGGL(rans_pack_kernel, dim3((unsigned)((long)n_ctx * spc / 64)), dim3(256), 0, stream, w.scratch, (const uint16_t*)sizes,
-                     w.group_bytes, (uint8_t*)coded, rans_slot(n, n_ctx, spc), w.err, n_ctx, meta);
+  const long ctx_len = n / n_ctx, groups = (long)n_ctx * spc / 64;
+  const int slot = rans_slot(n, n_ctx, spc);
+  const long per_block = (ctx_len / 4 + 255) / 256;
+  const int hb = (int)(per_block > RANS_HIST_BLOCKS ? RANS_HIST_BLOCKS : per_block);
+  uint32_t* part = (uint32_t*)ws;
+  u32x4* table = (u32x4*)((char*)ws + (long)n_ctx * RANS_HIST_BLOCKS * 1024);
+  int* err = (int*)(table + (long)n_ctx * 256);
+  uint32_t* group_bytes = (uint32_t*)((char*)err + (long)n_ctx * 16);
+  uint8_t* scratch = (uint8_t*)(group_bytes + (long)n_ctx * spc);
+  hipLaunchKernelGGL(rans_hist_kernel, dim3(hb, n_ctx), dim3(256), 0, stream, (const uint8_t*)sym, part, ctx_len);
+  hipLaunchKernelGGL(rans_normalize_kernel, dim3(n_ctx), dim3(256), 0, stream, part, hb, (uint16_t*)freq, table, ctx_len, err);
+  hipLaunchKernelGGL(rans_encode_kernel, dim3(spc / 64, n_ctx), dim3(64), 0, stream, (const uint8_t*)sym, table, scratch,
+                     (uint32_t*)states, (uint16_t*)sizes, group_bytes, ctx_len, spc, slot);
+  hipLaunchKernelGGL(rans_pack_kernel, dim3((unsigned)groups), dim3(256), 0, stream, scratch, (const uint16_t*)sizes, group_bytes,
+                     (uint8_t*)coded, slot, err, n_ctx, meta);
   return 0;
-}
-
-// Bytes of LDS that 64 streams of this length may need on their way to the host, 0: too many (then vpsa_rans_encode and a copy).
-static int publish_bytes(long n, int n_ctx, int spc) {
-  if (!rans_shape_ok(n, n_ctx, spc)) return 0;
-  const int most = 64 * rans_slot(n, n_ctx, spc) + 32;
-  return most <= 65536 - 1024 ? most : 0;
-}
-VPSA_EXPORT int vpsa_rans_publishes(long n, int n_ctx, int spc) { return publish_bytes(n, n_ctx, spc) > 0; }
-
-// As vpsa_rans_encode, but the `head_bytes` at `head` on the device (freq, states and sizes may be among them) and the coded bytes go side by
-// side into pinned host memory `to` (16-byte aligned), as far as `cap` bytes reach: there when `stream` is past this call, like meta.
-VPSA_EXPORT int vpsa_rans_publish(const void* sym, long n, int n_ctx, int spc, void* ws, void* freq, void* states, void* sizes, const void* head,
-                                  long head_bytes, void* to, long cap, long* meta, hipStream_t stream) {
-  const int lds = publish_bytes(n, n_ctx, spc);
-  if (lds <= 0 || (head_bytes & 15) || (((uintptr_t)head | (uintptr_t)to) & 15)) return -1;
-  const RansWork w = rans_work(ws, n_ctx, spc);
-  rans_code(sym, n, n_ctx, spc, w, freq, states, sizes, stream);
-  const int groups = (int)((long)n_ctx * spc / 64);
-  hipLaunchKernelGGL(rans_publish_kernel, dim3(groups + PUBLISH_HEAD_GROUPS), dim3(256), lds, stream, w.scratch, (const uint16_t*)sizes,
-                     w.group_bytes, groups, rans_slot(n, n_ctx, spc), (const u32x4*)head, head_bytes, (uint8_t*)to, cap, w.err, n_ctx, meta);
-  return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 // Only freq, states and sizes travel beside the coded bytes.
@@ -589,13 +486,13 @@ static long page_symbols(long n) { return (n + 255) & ~255L; }
 // Bytes of the workspace of vpsa_page_decode (symbols), 0: the shape is not taken.
 VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) { return rans_shape_ok(n, n_ctx, spc) && n % 64 == 0 ? page_symbols(n) : 0; }
 
-// `size` host bytes to other host memory.  Over on return.
-VPSA_EXPORT void vpsa_host_copy(void* to, const void* from, long size) { copy_in_parts((char*)to, (const char*)from, size); }
-
 VPSA_EXPORT int vpsa_copy_parts(long size) { return copy_parts(size); }
 
 // `size` bytes from the device to `to` by way of a pinned buffer.  Over on return.  (Four parts, each leaving the buffer while the next is on
-// its way, were no faster, 158 us a page against 162, and on the way back they cost the device 50 us a page: a copy's start is 10 to 15.)
+// its way, were no faster, 158 us a page against 162, and on the way back they cost the device 50 us a page: a copy's start is 10 to 15.
+// A kernel that stores the coded bytes into pinned memory right behind the coder spares the host one of its two waits, 201 us a page against 213 to 220,
+// but its workgroups lie on the CUs as long as the link takes: a decode step of 12 sequences on another stream took 2830 us beside
+// one thread that encodes pages and 4170 to 4520 beside two, instead of 2160 and 2350; 1920 to 1990 by itself.)
 VPSA_EXPORT int vpsa_fetch(const void* from, void* pinned, void* to, long size, hipStream_t stream) {
   const bool sent = hipMemcpyAsync(pinned, from, size, hipMemcpyDeviceToHost, stream) == hipSuccess;
   if (hipStreamSynchronize(stream) != hipSuccess || !sent) return -3;

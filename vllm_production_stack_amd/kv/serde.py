@@ -35,7 +35,6 @@ SERDE_NAIVE, SERDE_CACHEGEN = 0, 1
 # host range coder, remains for CPU hosts and for blobs already stored
 SERDE_CACHEGEN_RANS = 2
 _RANS_HDR = struct.Struct("<IIQ")  # streams per context, streams, coded bytes
-_META = 64  # bytes before a page in its pinned buffer: what the coder says of it
 _KEPT = 2  # pinned buffers a serialiser keeps for each direction
 _HDR = struct.Struct("<4sHHIIIIQ")
 
@@ -192,42 +191,34 @@ class PageSerde:
         return out, out.ctypes.data
 
     def _rans_page(self, flat: torch.Tensor, new):
-        """A page's kind-2 payload in what ``new`` makes for its size.  Every stage writes its part of the payload where it belongs; the
-        last one brings them to pinned memory together with the coded bytes and their number, without the host in between."""
+        """A page's kind-2 payload in what ``new`` makes for its size.  Every stage writes its part of the payload where it belongs,
+        the last one the size into pinned memory; then the payload is copied to the host in parts, and out of the pinned buffer
+        behind them."""
         n, dev, n_streams = flat.numel(), flat.device, self.n_layers * ops.RANS_SPC
         o1 = 4 * (n // 64)
         o2 = o1 + 512 * self.n_layers
         o3 = o2 + 4 * n_streams
         o4 = o3 + 2 * n_streams
-        direct = n % self.n_layers == 0 and ops.rans_publishes(n, self.n_layers)
-        body = torch.empty(o4 + (0 if direct else 2 * n), dtype=torch.uint8, device=dev)
+        body = torch.empty(o4 + 2 * n, dtype=torch.uint8, device=dev)
         sym, _ = ops.cachegen_encode(flat.contiguous(), self._levels(dev), self.unit_elems, self.n_layers,
                                      scales=body[:o1].view(torch.float32))
         ops.ensure_device()
         stream = torch.cuda.current_stream()  # the one that the kernel library queues on
-        buf = self._take(self._out_bufs, _META + o4 + n)  # (a value rarely codes to more than a byte)
+        buf = self._take(self._out_bufs, o4 + n)  # (a value rarely codes to more than a byte)
         buf.busy = stream
         meta = buf.bytes[:16].view(torch.int64)
-        coded, page = (None, (body, buf.bytes[_META:])) if direct else (body[o4:], None)
-        ops.rans_encode_into(sym.view(-1), self.n_layers, body[o1:o2], body[o2:o3], body[o3:o4], coded, meta=meta, page=page)
+        ops.rans_encode_into(sym.view(-1), self.n_layers, body[o1:o2], body[o2:o3], body[o3:o4], body[o4:], meta=meta)
         stream.synchronize()
         total, bad = meta.tolist()
         if bad:
             raise RuntimeError("rans_encode: frequency table could not be normalised")
-        if buf.bytes.numel() < _META + o4 + total:
-            buf = self._take(self._out_bufs, _META + o4 + total)
+        if buf.bytes.numel() < o4 + total:
+            buf = self._take(self._out_bufs, o4 + total)
             buf.busy = stream
-            if direct:  # (once more, into a buffer that holds it)
-                ops.rans_encode_into(sym.view(-1), self.n_layers, body[o1:o2], body[o2:o3], body[o3:o4], None, meta=buf.bytes[:16].view(torch.int64),
-                                     page=(body, buf.bytes[_META:]))
-                stream.synchronize()
         done, at = new(_RANS_HDR.size + o4 + total)
         ctypes.memmove(at, _RANS_HDR.pack(ops.RANS_SPC, n_streams, total), _RANS_HDR.size)
-        if direct:
-            ops.host_copy(at + _RANS_HDR.size, buf.bytes.data_ptr() + _META, o4 + total)
-        else:
-            ops.fetch_bytes(body, buf.bytes, at + _RANS_HDR.size, o4 + total)
-        buf.busy = None  # (its bytes are out: nothing is queued behind them)
+        ops.fetch_bytes(body, buf.bytes, at + _RANS_HDR.size, o4 + total)
+        buf.busy = None  # (fetched: nothing is queued behind it)
         self._give(self._out_bufs, buf)
         return done
 

@@ -47,7 +47,7 @@ def _kernels():
             "vpsa_moe_gemv", "vpsa_moe_mfma", "vpsa_lora_shrink", "vpsa_lora_expand",
             "vpsa_skinny_gemm", "vpsa_hbm_read_probe", "vpsa_set_gemm_variant", "vpsa_stream_gemm",
             "vpsa_stream_gemm_splits", "vpsa_set_stream_targets", "vpsa_rans_encode",
-            "vpsa_rans_decode", "vpsa_fetch", "vpsa_rans_publish", "vpsa_rans_publishes", "vpsa_copy_parts", "vpsa_page_decode", "vpsa_sample", "vpsa_grouped_gemm", "vpsa_packed_gemm",
+            "vpsa_rans_decode", "vpsa_fetch", "vpsa_copy_parts", "vpsa_page_decode", "vpsa_sample", "vpsa_grouped_gemm", "vpsa_packed_gemm",
             "vpsa_packed_gemm_splits", "vpsa_set_packed_target", "vpsa_dense_decode_attention", "vpsa_dense_attention",
             "vpsa_tile_gemm", "vpsa_tile_gemm_debug", "vpsa_paged_prefill_split",
             "vpsa_embed_scale", "vpsa_add_rmsnorm", "vpsa_rmsnorm_rows", "vpsa_latent_kv_write", "vpsa_rope_pairs",
@@ -61,7 +61,6 @@ def _kernels():
             "vpsa_embed_rmsnorm", "vpsa_depth_mix_rmsnorm", "vpsa_poly_norm", "vpsa_soft_cap", "vpsa_mingru",
         ):
             getattr(lib, name).restype = c_int
-        lib.vpsa_host_copy.restype = None
         for name in ("vpsa_prefill_split_record_bytes", "vpsa_rans_workspace",
                      "vpsa_page_workspace"):
             getattr(lib, name).restype = c_long
@@ -1471,33 +1470,21 @@ def rans_encode(sym, n_ctx, spc=RANS_SPC):
     return freq, states, sizes, coded[:total].clone()
 
 
-def rans_publishes(n: int, n_ctx: int, spc=RANS_SPC) -> bool:
-    """Whether ``rans_encode_into`` takes ``page`` for symbols of this size."""
-    return bool(_kernels().vpsa_rans_publishes(c_long(n), c_int(n_ctx), c_int(spc)))
-
-
-def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC, meta=None, page=None):
+def rans_encode_into(sym, n_ctx, freq, states, sizes, coded, spc=RANS_SPC, meta=None):
     """``rans_encode`` on the device into the caller's tensors (``coded`` with room for two bytes a symbol), without a
     synchronisation -> int64 [2] on the device, or ``meta`` (on the device or in pinned host memory): coded bytes, and contexts
-    whose table could not be normalised (nothing of the result is valid unless 0).  ``page`` = (head, to): the coded bytes go to pinned host
-    memory ``to`` instead, behind a copy of the device bytes ``head``, as far as it reaches (``coded`` None)."""
+    whose table could not be normalised (nothing of the result is valid unless 0)."""
     n, dev, lib = sym.numel(), sym.device, _kernels()
     if n % n_ctx or (n // n_ctx) % spc:
         raise ValueError("rans_encode: symbols do not divide into contexts / streams")
     n_streams = n_ctx * spc
     assert sym.is_cuda and sym.is_contiguous() and sym.element_size() == 1 and sym.data_ptr() % 4 == 0
     assert all(t.is_contiguous() and t.numel() * t.element_size() >= b for t, b in (
-        (freq, 512 * n_ctx), (states, 4 * n_streams), (sizes, 2 * n_streams), *(() if page else ((coded, 2 * n),))))
+        (freq, 512 * n_ctx), (states, 4 * n_streams), (sizes, 2 * n_streams), (coded, 2 * n)))
     ws = torch.empty(max(1, int(lib.vpsa_rans_workspace(c_long(n), c_int(n_ctx), c_int(spc)))), dtype=torch.uint8, device=dev)
     if meta is None:
         meta = torch.empty(2, dtype=torch.int64, device=dev)
     assert meta.dtype == torch.int64 and meta.is_contiguous() and meta.numel() == 2 and (meta.device == dev or meta.is_pinned())
-    if page:
-        head, to = page
-        assert all(t.is_contiguous() and t.element_size() == 1 for t in page) and head.device == dev and to.is_pinned()
-        _check(lib.vpsa_rans_publish(_p(sym), c_long(n), c_int(n_ctx), c_int(spc), _p(ws), _p(freq), _p(states), _p(sizes), _p(head),
-                                     c_long(head.numel()), _p(to), c_long(to.numel()), _p(meta), _stream()), "rans_publish")
-        return meta
     _check(lib.vpsa_rans_encode(_p(sym), c_long(n), c_int(n_ctx), c_int(spc), _p(ws), _p(freq), _p(states), _p(sizes), _p(coded),
                                 _p(meta), _stream()), "rans_encode")
     return meta
@@ -1527,11 +1514,6 @@ def fetch_bytes(src, pinned, dst: int, size: int) -> None:
     buffer is emptied behind the copy that fills it.  Over on return; other threads run meanwhile."""
     assert src.is_cuda and src.is_contiguous() and min(src.numel(), pinned.numel()) >= size and not pinned.is_cuda
     _check(_kernels().vpsa_fetch(_p(src), _p(pinned), c_void_p(dst), c_long(size), _stream()), "fetch_bytes")
-
-
-def host_copy(dst: int, src: int, size: int) -> None:
-    """``size`` bytes between two places of host memory, by the caller and threads that help; other threads run meanwhile."""
-    _kernels().vpsa_host_copy(c_void_p(dst), c_void_p(src), c_long(size))
 
 
 def page_decode(src: int, pinned, size: int, n: int, n_ctx: int, unit_elems: int, device, spc=RANS_SPC):
