@@ -15,8 +15,8 @@
 // cycles of vector work a wave and value).  12000 rows in a loop over the same operands, library with the activation's pass / this: 3072 x
 // 768 with gelu 107 / 70 us, 768 x 3072 57 / 48 (+ residual), three of 768 x 768 62 / 48, 768 x 2304 with gelu 50 / 42; 1500 rows, 2048 x 512 with
 // gelu 26 / 11.  Over operands that no cache holds, a workgroup for every tile / several tiles a workgroup with the costs below: the first
-// 78.9 / 72.7, the second 62.4 / 62.4, the third 53.5 / 45.7, one 768 x 768 with a residual 25.6 / 22.6, 117 products of 1500 to 48000 rows 6 % (one, 7500
-// rows of 768 x 3072, 44 / 54); an encoder of 12 layers, 8 windows 3733 / 3565, 2 1746 / 1640, 32 13.66 / 12.97 ms, none of 1 to 32 windows slower.
+// 78.9 / 72.7, the second 62.4 / 62.4, the third 53.5 / 45.7, one 768 x 768 with a residual 25.6 / 22.6, 395 products of 1500 to 48000 rows 5.7 %; an encoder
+// of 12 layers, 8 windows 3733 / 3565, 2 1746 / 1640, 32 13.66 / 12.97 ms, none of 1 to 32 windows slower.
 #include <type_traits>
 
 #include "common.h"
@@ -292,6 +292,9 @@ int start(const BlockArgs& args, long blocks, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
+// Whether workgroups make several of the tiles: more than the chip holds, and reductions that a ring of so many places does not outrun.
+bool several(long tiles, int K, int round, int ring) { return tiles > round && K / BK >= ring; }
+
 template <int TM, int TN, int S, int ACT, bool STREAM = false>
 int launch(BlockArgs& args, hipStream_t stream) {
   args.n_tiles = (args.N + 32 * TN - 1) / (32 * TN);
@@ -299,38 +302,54 @@ int launch(BlockArgs& args, hipStream_t stream) {
   if (blocks >= (1L << 31)) return -1;
   constexpr int ROUND = (TM + TN) * S * 4096 <= 81920 ? 512 : 256;  // what the chip holds
   if constexpr (!STREAM)
-    if (blocks > ROUND && args.K / BK >= S) return start<TM, TN, S, ACT, false, true>(args, ROUND, stream);
+    if (several(blocks, args.K, ROUND, S)) return start<TM, TN, S, ACT, false, true>(args, ROUND, stream);
   return start<TM, TN, S, ACT, STREAM, false>(args, blocks, stream);
 }
 
 // The tile shapes, and what they cost in microseconds: a chunk and what stands beside a tile's chunks (epilogue) in a round of one
-// workgroup a CU, or, where two share a CU, of two (a round that leaves at least half the places empty has a CU to each workgroup and a pair of
-// numbers of its own; beyond that some CU has two); more of the epilogue with gelu and with a residual; a launch's start.  Fitted to the speech
-// encoder's products (N, K of 512 to 3072, 1500 to 48000 rows, 117 in all); the choice by them is 0.8 % off the best shape on average, at the most
-// 13 (counting half-empty rounds in proportion: 3.0 and 28).
+// workgroup a CU, or, where two share a CU, of two (up to half of such a round has a CU to each workgroup and a pair of numbers of its
+// own); more of the epilogue with gelu and with a residual; a launch's start.  A round that is not full is shorter, for its workgroups share memory and
+// power with fewer: `least` is the share of its time that it keeps with next to none, `over` where it stands between a half and a full round when the first
+// CUs have two.  Counted as whole beyond a half, 7500 rows of 768 x 3072 went to 192 x 128 (240 of 512 places, 60.5 us over operands from memory, 45.6 from
+// the caches) instead of 128 x 128 (354 of 512: 55.6 / 43.6), three 1280 x 1280 with 1500 rows took 26.9 / 26.4 instead of 23.1 / 23.3.  Fitted to 395 products of a
+// speech encoder (N, K of 384 to 5120, 1500 to 48000 rows), each over operands from memory and from the caches, and drawn towards the best choice:
+// in the mean of the two 0.3 % off the best shape on average, at the most 7 (with whole rounds 1.5 and 16).  Where the two disagree, the mean decides: 3000 rows of 768
+// x 3072 take 128 x 128 by itself on a CU, 35.9 / 24.5, 64 x 128 would 32.0 / 31.0.
 struct Shape {
   int bm, bn, per_cu;
-  float chunk, fixed, chunk1, fixed1, gelu, res, start;
+  float chunk, fixed, chunk1, fixed1, gelu, res, start, least, over;
 };
-constexpr Shape SHAPES[] = {{192, 192, 1, 0.79f, 4.70f, 0.f, 0.f, 5.27f, 7.16f, 1.71f},   {128, 128, 1, 0.47f, 2.48f, 0.f, 0.f, 2.13f, 2.81f, 1.02f},
-                            {128, 128, 2, 0.95f, 2.45f, 0.64f, 2.22f, 2.38f, 4.28f, 2.12f}, {64, 128, 2, 0.63f, 1.25f, 0.32f, 0.96f, 0.98f, 1.97f, 1.86f},
-                            {192, 128, 2, 1.29f, 3.15f, 0.73f, 2.98f, 3.89f, 5.85f, 3.30f}, {96, 192, 2, 1.20f, 1.04f, 0.69f, 2.77f, 3.02f, 4.82f, 2.48f}};
+constexpr Shape SHAPES[] = {{192, 192, 1, 0.82f, 3.68f, 0.f, 0.f, 5.50f, 8.76f, 6.85f, 0.73f, 1.00f}, {128, 128, 1, 0.52f, 1.87f, 0.f, 0.f, 2.43f, 3.19f, 3.12f, 0.67f, 1.00f},
+                            {128, 128, 2, 0.98f, 2.80f, 0.71f, 0.00f, 2.30f, 5.42f, 4.14f, 0.91f, 0.33f}, {64, 128, 2, 0.70f, 1.31f, 0.41f, 0.15f, 0.63f, 2.24f, 2.54f, 0.48f, 0.72f},
+                            {192, 128, 2, 1.26f, 2.21f, 0.95f, 0.34f, 3.86f, 8.20f, 6.63f, 0.66f, 0.55f}, {96, 192, 2, 1.19f, 1.94f, 0.93f, 0.00f, 2.42f, 6.76f, 4.92f, 0.60f, 0.17f}};
 
 int choose(int M, int N, int K, int parts, int act, bool res) {
   int best = 0;
   double best_t = 0;
   for (int i = 0; i < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); ++i) {
     const Shape& s = SHAPES[i];
-    const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * parts, round = 256 * s.per_cu, left = tiles % round;
-    const double more = (act == ACT_GELU ? s.gelu : 0) + (res ? s.res : 0), full = K / BK * s.chunk + s.fixed + more;
+    const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * parts, round = 256 * s.per_cu;
+    const double more = (act == ACT_GELU ? s.gelu : 0) + (res ? s.res : 0), full = K / BK * s.chunk + s.fixed + more, fill = (double)(tiles % round) / round;
     const double half = K / BK * s.chunk1 + s.fixed1 + more / 2;
-    const double t = s.start + tiles / round * full + (left == 0 ? 0 : s.per_cu > 1 && 2 * left <= round ? half : full);
+    const double left = fill == 0         ? 0
+                        : s.per_cu == 1   ? full * (s.least + (1 - s.least) * fill)
+                        : fill <= 0.5     ? half * (s.least + (1 - s.least) * 2 * fill)
+                                          : half + (full - half) * (s.over + (1 - s.over) * (2 * fill - 1));
+    const double t = s.start + tiles / round * full + left;
     if (i == 0 || t < best_t) best = i, best_t = t;
   }
   return best;
 }
 
 }  // namespace
+
+// The tile shape of a product (its place in SHAPES), plus 16 where workgroups make several tiles each.
+VPSA_EXPORT int vpsa_block_gemm_shape(int M, int N, int K, int parts, int act, int res) {
+  constexpr int RING[] = {3, 4, 2, 3, 2, 2};
+  const int i = choose(M, N, K, parts, act, res != 0);
+  const Shape& s = SHAPES[i];
+  return i + (several((long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * parts, K, 256 * s.per_cu, RING[i]) ? 16 : 0);
+}
 
 // c[r] = act(x[r] W_p^T + bias_p) + res[r], the columns of weights p = 0 .. parts - 1 (N rows of K each) side by side.  Rows r = 0 .. M - 1
 // in batches of batch_rows (one batch: M): strides of a row and of a batch in elements for x, c and res (c may be res).  act: 0 none,

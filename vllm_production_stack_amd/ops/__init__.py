@@ -54,7 +54,7 @@ def _kernels():
             "vpsa_latent_attention", "vpsa_sigmoid_gate", "vpsa_relu_sq", "vpsa_glu_clamp", "vpsa_group_topk",
             "vpsa_gather_rows", "vpsa_moe_finish", "vpsa_latent_mfma_supported", "vpsa_latent_mfma_expanded", "vpsa_latent_attention_mfma",
             "vpsa_moe_mfma_act",
-            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_chunk_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_first_chunk", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_row_gemm_takes", "vpsa_row_add", "vpsa_row_qkv", "vpsa_mid_unit_factors", "vpsa_block_gemm", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
+            "vpsa_add_dyt", "vpsa_recurrent_scan", "vpsa_chunk_scan", "vpsa_retention_scan", "vpsa_layernorm", "vpsa_mid_gemm", "vpsa_mid_first_chunk", "vpsa_mid_gemm_splits", "vpsa_mid_gemm_norm", "vpsa_mid_gemm_qkv", "vpsa_row_gemm_takes", "vpsa_row_add", "vpsa_row_qkv", "vpsa_mid_unit_factors", "vpsa_block_gemm", "vpsa_block_gemm_shape", "vpsa_head_rms", "vpsa_short_conv_qkv", "vpsa_window_attention",
             "vpsa_mix_heads", "vpsa_xielu", "vpsa_window_mfma_supported", "vpsa_window_attention_mfma", "vpsa_window_tile_slots",
             "vpsa_gated_add_rmsnorm", "vpsa_pool_blocks", "vpsa_diff_heads",
             "vpsa_window_kv_write",
