@@ -358,7 +358,15 @@ __device__ __forceinline__ void dense_attn_rows(
     };
     const int n = (n_tiles + 1) >> 1;
     for (int i = 0; i + 1 < n; ++i) two(i, std::false_type{});
-    two(n - 1, std::true_type{});
+    // of an odd number of tiles the last one has no partner: its place holds repeats of the last key, whose values may be infinite
+    if (2 * (n - 1) + part < n_tiles) {
+      two(n - 1, std::true_type{});
+    } else {
+      stage_two(n - 1, vsrc, vbase_p, vc, lds_v);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      __syncthreads();
+    }
   } else {
     auto tile = [&](int t, auto masked) {
       const int buf = t & 1;

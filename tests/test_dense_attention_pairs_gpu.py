@@ -45,3 +45,16 @@ def test_one_wave_of_a_pair_has_all_the_weight(first):
     for score in (-1000.0, float("-inf")):
         k[:, low, 0] = score
         check(q, k, v, 1)
+
+
+@pytest.mark.parametrize("tk", [128, 192, 320, 448])  # whole tiles: no key past the last one is read in its place
+@pytest.mark.parametrize("at", [0, 100, -1])
+def test_values_without_bound(tk, at):
+    torch.manual_seed(tk)
+    q, k, v = (torch.randn(2, t, 64, device="cuda").bfloat16() for t in (70, tk, tk))
+    v[0, at, 3], v[0, at, 40], v[1, at, 7] = float("inf"), float("-inf"), float("nan")
+    want = torch.softmax(q.double() @ k.double().transpose(-1, -2).contiguous() * 0.125, -1) @ v.double()
+    got = ops.dense_attention(q, k, v, 1).double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[got.isinf()], want[want.isinf()]) and torch.equal(got.isinf(), want.isinf())
+    bound = want.isfinite()
+    assert float((got - want)[bound].norm() / want[bound].norm()) < 2 ** -7
