@@ -311,7 +311,7 @@ class TransformerModel:
         adapters = self.lora is not None and meta.lora_slots is not None
         x = None  # the norm the next layer starts with, where the projection before it made it
         rows = None  # or what it makes itself the norm from (decode steps of a few rows)
-        few = decode_only and not adapters and self.tp_size == 1 and cfg.num_experts == 0
+        few = decode_only and not adapters and self.tp_size == 1 and cfg.num_experts == 0 and input_ids.shape[0] <= ops.ROW_ROWS
 
         def fits(i):
             return few and i < len(self.layers) and ops.row_layer_takes(residual, self.layers[i], pool, meta, self.n_q, self.n_kv,
@@ -346,7 +346,7 @@ class TransformerModel:
                 rows = ops.row_add(act, lw.w_down, residual, self.layers[li + 1].ln1 if here else None)
                 h, x, rows = None, None, rows if here else None
                 continue
-            rows = None
+            rows, here = None, None
             x = self._out_norm("o", gl, attn, lw.wo, None, residual, lw.ln2, meta)
             if cfg.num_experts > 0:
                 h, x = tp_all_reduce(self._moe(x, lw, decode_only)), None

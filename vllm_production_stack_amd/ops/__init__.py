@@ -964,8 +964,8 @@ def row_layer_takes(residual, lw, pool, meta, n_q, n_kv, head_dim, cos_sin) -> b
             or _generic_attention(residual, head_dim) or h > 8192):
         return False
     q, i = n_q * head_dim, lw.w_down.shape[1]
-    if (lw.wqkv.shape != (q + 2 * n_kv * head_dim, h) or lw.wo.shape != (h, q) or lw.w_gate_up.shape != (2 * i, h) or lw.w_down.shape != (h, i)
-            or h // 16 < MID_MIN_FILL_ROWS or not MID_MIN_FILL_ROWS <= i // 64 <= TILE_CUS
+    if (h // 16 < MID_MIN_FILL_ROWS or not MID_MIN_FILL_ROWS <= i // 64 <= TILE_CUS or lw.wqkv.shape != (q + 2 * n_kv * head_dim, h)
+            or lw.wo.shape != (h, q) or lw.w_gate_up.shape != (2 * i, h) or lw.w_down.shape != (h, i)
             or int(_kernels().vpsa_mid_gemm_splits(c_int(m), c_int(2 * i), c_int(h), c_int(1))) != 1):
         return False
     lib = _kernels()
