@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 typedef __bf16 bf16_t;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -16,6 +18,13 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #define WAVE 64
 
 #define VPSA_EXPORT extern "C" __attribute__((visibility("default")))
+
+// Launches a kernel: 0, or -3 where the runtime refuses it (what hipGetLastError says may be left from an earlier call).
+template <typename... P>
+inline int launched(void (*kernel)(P...), dim3 grid, int block, int lds, hipStream_t stream, std::common_type_t<P>... args) {
+  void* at[] = {(void*)&args...};
+  return hipLaunchKernel((const void*)kernel, grid, dim3(block), at, lds, stream) == hipSuccess ? 0 : -3;
+}
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t u) {
   return __uint_as_float(((uint32_t)u) << 16);

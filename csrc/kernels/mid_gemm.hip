@@ -442,9 +442,8 @@ int launch_mid(const void* x, long xs, const void* w, const void* bias, void* y,
     attr_set = true;
   }
   const int n_out = PAIR ? N / 2 : N;
-  mid_gemm_kernel<MT, PAIR, FACTORS><<<dim3(n_out / (PAIR ? BN / 2 : BN), S, (M + 127) / 128), 256, LDS, stream>>>(
-      (const uint16_t*)x, xs, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ys, ws, M, N, K, S, squares, eps);
-  return 0;
+  return launched(mid_gemm_kernel<MT, PAIR, FACTORS>, dim3(n_out / (PAIR ? BN / 2 : BN), S, (M + 127) / 128), 256, LDS, stream, (const uint16_t*)x, xs,
+                  (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ys, ws, M, N, K, S, squares, eps);
 }
 
 template <int MT>

@@ -461,9 +461,8 @@ VPSA_EXPORT int vpsa_rans_encode(const void* sym, long n, int n_ctx, int spc, vo
 VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* states, const void* freq, const void* sizes, void* sym,
                                  long n, int n_ctx, int spc, hipStream_t stream) {
   if (!rans_shape_ok(n, n_ctx, spc)) return -1;
-  hipLaunchKernelGGL(rans_decode_kernel, dim3(spc / 64, n_ctx), dim3(DECODE_THREADS), 0, stream, (const uint8_t*)coded, coded_len, (const uint16_t*)freq,
-                     (const uint16_t*)sizes, (const uint32_t*)states, (uint8_t*)sym, n / n_ctx, spc);
-  return 0;
+  return launched(rans_decode_kernel, dim3(spc / 64, n_ctx), DECODE_THREADS, 0, stream, (const uint8_t*)coded, coded_len, (const uint16_t*)freq,
+                  (const uint16_t*)sizes, (const uint32_t*)states, (uint8_t*)sym, n / n_ctx, spc);
 }
 
 // ---------------------------------------------------------------------------------

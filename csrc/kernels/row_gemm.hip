@@ -266,8 +266,7 @@ int launch(const RowArgs& a, hipStream_t stream) {
     attr_set = true;
   }
   const int tiles = a.N / 16;
-  row_gemm_kernel<EPI, AI><<<tiles < CUS ? tiles : CUS, 512, LDS, stream>>>(a);
-  return 0;
+  return launched(row_gemm_kernel<EPI, AI>, dim3(tiles < CUS ? tiles : CUS), 512, LDS, stream, a);
 }
 
 // Shapes that the kernels take (offsets within the weights have 32 bits).
