@@ -3,6 +3,7 @@
 from ctypes import c_int, c_long
 
 import pytest
+import torch
 
 from vllm_production_stack_amd import ops
 
@@ -42,3 +43,28 @@ def test_routers_that_the_kernel_takes():
     assert all(takes(t, e, h) for t in (1, 8, 1531, 4096) for e, h in ((2, 4096), (8, 4096), (16, 2048), (32, 1024), (60, 512), (64, 512)))
     assert not any(takes(8, e, h) for e, h in ((8, 6144), (9, 4096), (16, 4096), (32, 2048), (60, 2048), (64, 1024), (65, 128), (128, 128)))
     assert not takes(4097, 8, 4096) and not takes(8, 8, 4000)
+
+
+@pytest.mark.parametrize("heads,kv_heads,hidden", [(64, 8, 8192), (32, 8, 4096), (32, 4, 8192), (28, 4, 3584)])
+@pytest.mark.parametrize("rows", [1, 64, 96, 97, 112, 128, 129, 176, 256])
+def test_projections_that_write_the_cache_take_the_kernel_that_they_take_by_themselves(monkeypatch, heads, kv_heads, hidden, rows):
+    """Rotation and cache in the reduction are a launch less, no reason for the slower product."""
+    lib, called = ops._kernels(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            if name.endswith("_splits"):
+                return getattr(lib, name)
+            return lambda *args: called.append(name) or 0
+
+    n = (heads + 2 * kv_heads) * 128
+    x, w = torch.empty((rows, hidden), dtype=torch.bfloat16), torch.empty((n, hidden), dtype=torch.bfloat16)
+    slots, positions = torch.empty(rows, dtype=torch.int64), torch.empty(rows, dtype=torch.int32)
+    pool, cos_sin = torch.empty((2, 1, 2, kv_heads, 64 * 128), dtype=torch.bfloat16), torch.empty((64, 128))
+    monkeypatch.setattr(ops, "_kernels", Recorder)
+    monkeypatch.setattr(ops, "_reads", lambda *_: True)
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    with torch.no_grad():
+        itself = ["vpsa_block_proj_qkv"] if ops._block_splits(rows, n, hidden, False) > 1 else ["vpsa_mid_gemm_qkv"] if ops._mid_splits(rows, n, hidden, False) > 1 else []
+        ops.decode_qkv(x, w, None, pool, 0, positions, slots, cos_sin, heads, kv_heads)
+    assert called == itself or (not itself and called == ["vpsa_block_proj_qkv"])  # (which may take more partial sums here)

@@ -909,9 +909,11 @@ def decode_qkv(x, w, bias, pool, layer, positions, slots, cos_sin, n_q, n_kv):
     """q / k / v projection, rotary embedding and cache write of one token per sequence, when ``mid_gemm`` or ``block_gemm``
     splits the projection: its reduction then rotates and writes the cache.  The query rows [T, n_q * 128], or None (and nothing done)
     otherwise."""
-    splits, entry = _mid_takes(x, w, bias, False), "vpsa_mid_gemm_qkv"
+    # block_gemm first, as in the projections by themselves: up to 128 rows it takes what is too large for mid_gemm (10240 x 8192 with the cache, 97
+    # rows 41.7 us, with mid_gemm 44.8, 128 rows 44.9 and 50.0; projection and cache's own kernel 44.1 and 46.9)
+    splits, entry = _block_takes(x, w, bias, False, BLOCK_SUMS_QKV), "vpsa_block_proj_qkv"
     if splits < 2:
-        splits, entry = _block_takes(x, w, bias, False, BLOCK_SUMS_QKV), "vpsa_block_proj_qkv"
+        splits, entry = _mid_takes(x, w, bias, False), "vpsa_mid_gemm_qkv"
     m = x.shape[0]
     if splits < 2 or pool.dtype != torch.bfloat16 or w.shape[0] != (n_q + 2 * n_kv) * HEAD_DIM_HIP:
         return None
@@ -1025,6 +1027,9 @@ def row_attention_block(rows, eps, w, bias, pool, layer, meta, n_q, n_kv, head_d
 # The projection's reduction also rotates and writes the cache: a launch less a layer.  A step of 8 layers, apart / together: 32 rows behind
 # 1500 tokens 1121 / 1084 us, 64 behind 3000 1270 / 1221, 97 behind 20900 1650 / 1601, 150 behind 3000 1577 / 1534, 256 behind 2000 1818 / 1701; with two
 # row tiles 300 behind 1500 2152 / 2122, but 400 2221 / 2274, 512 2488 / 2512: the cache's own kernel writes whole lines of V, the reduction single values.
+# Other widths, a step of 4 layers behind 1500 tokens: 28 + 4 heads of 3584 channels with a bias, 16 rows 729 / 714, 80 898 / 876, 129 1003 / 982, 176 1027 / 1020, 240
+# 1140 / 1136, 256 1183 / 1125; 64 + 8 of 8192, 16 rows 1556 / 1537, 64 1805 / 1786, 112 1879 / 1855, 128 1935 / 1922, 224 2195 / 2186, 256 2388 / 2407 (runs differ by
+# 2 %; projection and cache alone 59.4 / 58.2); 32 + 4 of 8192, 128 rows 1331 / 1294, 256 1543 / 1473; 16 + 2 of 8192, 256 rows 1334 / 1271; 16 + 4 of 4096, 176 rows 763 / 751.
 PROMPT_QKV_ROWS = BLOCK_MAX_ROWS
 
 
