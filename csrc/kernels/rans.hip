@@ -320,7 +320,7 @@ __device__ __forceinline__ void rans_decode_stream(F pair, int at, uint32_t x, c
 // decodes to garbage, never out of bounds: a damaged table gives entries of some symbol, every field masked to its width), and a step takes
 // at most two bytes whatever the state is.  A page of 16384 streams of 256 symbols: tables in a launch of their own 4 us and one wave for all 64
 // streams 33; in one launch 32 with one wave (which waited for memory ten times in a row before its first step), 28 with four (fewer lanes meet
-// in a bank of LDS; eight waves 32), 24 with the loop above.
+// in a bank of LDS; eight waves 32), 24 with the loop above.  (53 KB of LDS: three a CU; with two, 80 contexts took two rounds, 49.6 us for 39.3.)
 __global__ __launch_bounds__(DECODE_THREADS) void rans_decode_kernel(const uint8_t* __restrict__ coded, long coded_len, const uint16_t* __restrict__ freq,
                                                           const uint16_t* __restrict__ sizes, const uint32_t* __restrict__ states,
                                                           uint8_t* __restrict__ sym, long ctx_len, int spc) {
@@ -329,8 +329,9 @@ __global__ __launch_bounds__(DECODE_THREADS) void rans_decode_kernel(const uint8
   __shared__ __attribute__((aligned(16))) u32x2 tab[RANS_M];
   __shared__ __attribute__((aligned(16))) uint32_t bytes[LDS_WORDS];
   constexpr int NT = DECODE_THREADS, WAVES = NT / 64, EACH = 64 / WAVES;  // streams of a wave
-  __shared__ uint32_t cum[256], fr[256], in_wave[4];
+  __shared__ uint32_t in_wave[4];
   __shared__ long part[WAVES];
+  uint32_t *const cum = bytes, *const fr = bytes + 256;  // (until the bytes come)
   const int ctx = blockIdx.y, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
   const uint32_t f = t < 256 ? freq[ctx * 256 + t] : 0;
   const long stream0 = (long)ctx * spc + blockIdx.x * 64;
@@ -396,6 +397,7 @@ __global__ __launch_bounds__(DECODE_THREADS) void rans_decode_kernel(const uint8
       if (cum[s + step] <= slot) s += step;
     tab[slot] = (u32x2){((fr[s] - 1) & 0xfff) + 1 | (uint32_t)s << 24, (slot - cum[s]) & 0xfff};
   }
+  if (held > LDS_WORDS - 512) __syncthreads();  // (the same for all threads; else nobody writes where the table was made from)
 #pragma unroll
   for (int j = 0; j < AHEAD; ++j)
     if (t + NT * j < held) bytes[LDS_WORDS - 1 - (t + NT * j)] = __builtin_bswap32(v[j]);
@@ -416,6 +418,126 @@ __global__ __launch_bounds__(DECODE_THREADS) void rans_decode_kernel(const uint8
       const uint32_t b = __builtin_amdgcn_alignbyte(hi, lo, i & 3);  // the next byte lowest
       return (b & 0xff) << 8 | ((b >> 8) & 0xff);
     }, (int)rp, x, tab, out, lane, len, spc);
+}
+
+// More workgroups than the chip holds (three a CU, by their LDS) stand in each other's way: four waves for 64 streams are four times the instructions, every one
+// makes its context's table and sums the sizes before it.  Those calls take two launches, one for tables and sums, one of a wave for 64
+// streams, four of them a CU: 80 contexts of 512 streams of 256 symbols 39.3 us by the kernel above, 41.3 by these, 126 contexts 61.0 / 50.2; of 16 symbols 17.1 / 14.6, 512
+// contexts 70.5 / 43.3, 2048 contexts 634 / 168.
+constexpr long DECODE_TOGETHER = 3 * 256;
+// grid n_ctx, block 1024: a context's 4096 decoder entries, symbol | (freq - 1) << 8 | (slot - cum) << 20, and the bytes of its
+// streams.  (A damaged table gives entries of some symbol; every field is masked to its width.)
+__global__ __launch_bounds__(1024) void rans_decode_tables_kernel(const uint16_t* __restrict__ freq, uint32_t* __restrict__ table,
+                                                                  const uint16_t* __restrict__ sizes, int spc,
+                                                                  long* __restrict__ ctx_bytes) {
+  __shared__ uint32_t cum[256], fr[256];
+  __shared__ long part[16];
+  const int t = threadIdx.x;
+  uint32_t f = 0;
+  if (t < 256) {
+    f = freq[blockIdx.x * 256 + t];
+    fr[t] = f;
+  }
+  long sum = 0;
+  for (int i = t; i < spc; i += 1024) sum += sizes[(long)blockIdx.x * spc + i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if ((t & 63) == 0) part[t >> 6] = sum;
+  const int before = wave_before((int)f);  // (of the wave's 64 symbols)
+  if (t < 256) cum[t] = before;
+  __syncthreads();
+  if (t == 0) {
+    long s = 0;
+    for (int w = 0; w < 16; ++w) s += part[w];
+    ctx_bytes[blockIdx.x] = s;
+  }
+  if (t < 256) {
+    uint32_t c = cum[t];
+    for (int w = 0; w < (t >> 6); ++w) c += cum[w * 64 + 63] + fr[w * 64 + 63];
+    f = c;
+  }
+  __syncthreads();
+  if (t < 256) cum[t] = f;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t slot = t + 1024 * i;
+    int s = 0;  // the last symbol that starts at or before the slot (those before it with the same start do not occur)
+#pragma unroll
+    for (int step = 128; step > 0; step >>= 1)
+      if (cum[s + step] <= slot) s += step;
+    table[blockIdx.x * (long)RANS_M + slot] = (uint32_t)s | ((fr[s] - 1) & 0xfff) << 8 | ((slot - cum[s]) & 0xfff) << 20;
+  }
+}
+
+// A stream's symbols; `word` reads words i and i + 1 of the wave's coded bytes, from LDS or (streams too long for it) from memory.
+// Two copies of the loop: one that may load from memory waits for its own stores at every step.  The words around the next
+// byte are read in the same wait as the state's table entry.
+template <typename F>
+__device__ __forceinline__ void rans_decode_many_stream(F word, uint32_t rp, uint32_t x, const uint32_t* tab,
+                                                   uint8_t* __restrict__ out, int len, int spc) {
+  for (int k = 0; k < len; ++k) {
+    const uint32_t e = tab[x & (RANS_M - 1)];
+    const uint64_t w = word(rp >> 2);
+    const uint32_t lo = (uint32_t)w, hi = (uint32_t)(w >> 32);
+    *out = (uint8_t)e;
+    out += spc;
+    const uint32_t q = x >> RANS_BITS;  // 20 bits (19 of a state the encoder leaves)
+    x = __umul24((e >> 8) & 0xfff, q) + (q + (e >> 20));
+    const uint32_t b = __builtin_amdgcn_alignbyte(hi, lo, rp & 3);  // the next byte lowest
+    const uint32_t x1 = (x << 8) | (b & 0xff), x2 = (x1 << 8) | ((b >> 8) & 0xff);
+    const bool one = x < RANS_LOW, two = x < (RANS_LOW >> 8);
+    x = two ? x2 : one ? x1 : x;
+    rp += one + two;
+  }
+}
+
+// grid (spc / 64, n_ctx), block 64.  The wave's coded bytes lie side by side, behind those of the contexts and of the context's
+// streams before it; they are staged when they fit (a stream's share of LDS_WORDS is 320 bytes, a symbol rarely takes one).
+// coded_len bounds every read (a damaged blob decodes to garbage, never out of bounds), and a step takes at most two bytes
+// whatever the state is.
+__global__ __launch_bounds__(64) void rans_decode_many_kernel(const uint8_t* __restrict__ coded, long coded_len,
+                                                         const long* __restrict__ ctx_bytes, const uint16_t* __restrict__ sizes,
+                                                         const uint32_t* __restrict__ states, const uint32_t* __restrict__ table,
+                                                         uint8_t* __restrict__ sym, long ctx_len, int spc) {
+  constexpr int LDS_WORDS = 64 * 80;
+  __shared__ __attribute__((aligned(16))) uint32_t tab[RANS_M];
+  __shared__ uint32_t bytes[LDS_WORDS];
+  const int ctx = blockIdx.y, t = threadIdx.x;
+  const u32x4* tp = reinterpret_cast<const u32x4*>(table + (long)ctx * RANS_M);
+#pragma unroll
+  for (int i = 0; i < RANS_M / 256; ++i) reinterpret_cast<u32x4*>(tab)[t + 64 * i] = tp[t + 64 * i];
+  const uint16_t* sz = sizes + (long)ctx * spc;
+  long first = 0;  // byte of the wave's first stream
+  for (int i = t; i < ctx; i += 64) first += ctx_bytes[i];
+  for (int i = t; i < (int)blockIdx.x * 64; i += 64) first += sz[i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
+  const int n = sz[blockIdx.x * 64 + t], before = wave_before(n), all = __shfl(before + n, 63, 64);
+  const uint32_t x = states[(long)ctx * spc + blockIdx.x * 64 + t];
+  // words of the coded bytes, counted from the aligned word that holds byte 0
+  const int lead = (int)((uintptr_t)coded & 3);
+  const uint32_t* cw = reinterpret_cast<const uint32_t*>(coded - lead);
+  const long n_words = (coded_len + lead + 3) >> 2;
+  const long w0 = (first + lead) >> 2, w1 = min((first + all + lead + 3) >> 2, n_words);
+  const bool staged = w1 - w0 < LDS_WORDS;
+  const int held = staged ? max((int)(w1 - w0), 0) : 0;
+#pragma unroll 8
+  for (int i = t; i < held; i += 64) bytes[i] = cw[w0 + i];
+  __syncthreads();
+  uint8_t* out = sym + (long)ctx * ctx_len + blockIdx.x * 64 + t;
+  const int len = (int)(ctx_len / spc);
+  const uint32_t rp = (uint32_t)((first + lead) & 3) + (uint32_t)before;
+  if (staged)
+    rans_decode_many_stream([&](uint32_t i) {
+      const uint32_t at = min(i, (uint32_t)LDS_WORDS - 2);
+      return (uint64_t)bytes[at + 1] << 32 | bytes[at];
+    }, rp, x, tab, out, len, spc);
+  else
+    rans_decode_many_stream([&](uint32_t i) {
+      const uint32_t lo = w0 + i < n_words ? cw[w0 + i] : 0u, hi = w0 + i + 1 < n_words ? cw[w0 + i + 1] : 0u;
+      return (uint64_t)hi << 32 | lo;
+    }, rp, x, tab, out, len, spc);
 }
 
 static bool rans_shape_ok(long n, int n_ctx, int spc) {
@@ -457,12 +579,25 @@ VPSA_EXPORT int vpsa_rans_encode(const void* sym, long n, int n_ctx, int spc, vo
   return 0;
 }
 
-// Only freq, states and sizes travel beside the coded bytes.
-VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* states, const void* freq, const void* sizes, void* sym,
+// Bytes of the decoder's workspace (calls of many contexts: tables | bytes per context), 0: none.
+VPSA_EXPORT long vpsa_rans_decode_workspace(long n, int n_ctx, int spc) {
+  return rans_shape_ok(n, n_ctx, spc) && (long)n_ctx * spc / 64 > DECODE_TOGETHER ? (long)n_ctx * (RANS_M * 4 + 8) : 0;
+}
+
+// Only freq, states and sizes travel beside the coded bytes; ws 16-byte aligned, or null where none is needed.
+VPSA_EXPORT int vpsa_rans_decode(const void* coded, long coded_len, const void* states, const void* freq, const void* sizes, void* ws, void* sym,
                                  long n, int n_ctx, int spc, hipStream_t stream) {
   if (!rans_shape_ok(n, n_ctx, spc)) return -1;
-  return launched(rans_decode_kernel, dim3(spc / 64, n_ctx), DECODE_THREADS, 0, stream, (const uint8_t*)coded, coded_len, (const uint16_t*)freq,
-                  (const uint16_t*)sizes, (const uint32_t*)states, (uint8_t*)sym, n / n_ctx, spc);
+  const long ctx_len = n / n_ctx;
+  if (vpsa_rans_decode_workspace(n, n_ctx, spc) == 0)
+    return launched(rans_decode_kernel, dim3(spc / 64, n_ctx), DECODE_THREADS, 0, stream, (const uint8_t*)coded, coded_len, (const uint16_t*)freq,
+                    (const uint16_t*)sizes, (const uint32_t*)states, (uint8_t*)sym, ctx_len, spc);
+  if (ws == nullptr || ((uintptr_t)ws & 15)) return -1;
+  uint32_t* table = (uint32_t*)ws;
+  long* ctx_bytes = (long*)(table + (long)n_ctx * RANS_M);
+  const int rc = launched(rans_decode_tables_kernel, dim3(n_ctx), 1024, 0, stream, (const uint16_t*)freq, table, (const uint16_t*)sizes, spc, ctx_bytes);
+  return rc ? rc : launched(rans_decode_many_kernel, dim3(spc / 64, n_ctx), 64, 0, stream, (const uint8_t*)coded, coded_len, ctx_bytes,
+                            (const uint16_t*)sizes, (const uint32_t*)states, table, (uint8_t*)sym, ctx_len, spc);
 }
 
 // ---------------------------------------------------------------------------------
@@ -482,8 +617,10 @@ static PageParts page_parts(void* body, long n, int n_ctx, int spc) {
 static long page_symbols(long n) { return (n + 255) & ~255L; }
 
 // A page's parts, scales fp32 [n / 64] | freq | states | sizes | coded bytes, lie side by side in `body` on the device.
-// Bytes of the workspace of vpsa_page_decode (symbols), 0: the shape is not taken.
-VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) { return rans_shape_ok(n, n_ctx, spc) && n % 64 == 0 ? page_symbols(n) : 0; }
+// Bytes of the workspace of vpsa_page_decode (symbols | the coder's), 0: the shape is not taken.
+VPSA_EXPORT long vpsa_page_workspace(long n, int n_ctx, int spc) {
+  return rans_shape_ok(n, n_ctx, spc) && n % 64 == 0 ? page_symbols(n) + vpsa_rans_decode_workspace(n, n_ctx, spc) : 0;
+}
 
 VPSA_EXPORT int vpsa_copy_parts(long size) { return copy_parts(size); }
 
@@ -544,6 +681,6 @@ VPSA_EXPORT int vpsa_page_decode(const void* from, void* pinned, void* body, lon
   if (coded < 0) return -1;
   copy_in_parts((char*)pinned, (const char*)from, size);
   if (const int rc = page_copy(body, pinned, size, fresh, stream)) return rc;
-  const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, ws, n, n_ctx, spc, stream);
+  const int rc = vpsa_rans_decode(at.coded, coded, at.states, at.freq, at.sizes, (char*)ws + page_symbols(n), ws, n, n_ctx, spc, stream);
   return rc ? rc : vpsa_cachegen_decode(ws, (const float*)at.scales, out, n, unit_elems, stream);
 }

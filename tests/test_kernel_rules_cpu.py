@@ -68,3 +68,15 @@ def test_projections_that_write_the_cache_take_the_kernel_that_they_take_by_them
         itself = ["vpsa_block_proj_qkv"] if ops._block_splits(rows, n, hidden, False) > 1 else ["vpsa_mid_gemm_qkv"] if ops._mid_splits(rows, n, hidden, False) > 1 else []
         ops.decode_qkv(x, w, None, pool, 0, positions, slots, cos_sin, heads, kv_heads)
     assert called == itself or (not itself and called == ["vpsa_block_proj_qkv"])  # (which may take more partial sums here)
+
+
+def test_entropy_decoders_of_many_contexts_have_a_launch_for_their_tables():
+    """What one round of workgroups holds is decoded in one launch without a workspace; a page that codes to more has room for the tables."""
+    def sizes(n_ctx, per_stream):
+        n = n_ctx * 512 * per_stream
+        return [int(f(c_long(n), c_int(n_ctx), c_int(512))) for f in (ops._kernels().vpsa_rans_decode_workspace, ops._kernels().vpsa_page_workspace)]
+
+    assert sizes(1, 4) == [0, 2048] and sizes(80, 256) == [0, 80 * 512 * 256] and sizes(96, 16) == [0, 96 * 512 * 16]
+    for n_ctx in (97, 126, 2048):
+        tables = n_ctx * (4096 * 4 + 8)
+        assert sizes(n_ctx, 16) == [tables, n_ctx * 512 * 16 + tables]

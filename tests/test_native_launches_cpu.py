@@ -10,7 +10,7 @@ from vllm_production_stack_amd import ops
 pytestmark = pytest.mark.skipif(torch.cuda.is_available(), reason="launches are refused where there is no GPU")
 AT = c_void_p(4096)  # no launch, so nothing reads there
 CALLS = {
-    "vpsa_rans_decode": (AT, c_long(64), AT, AT, AT, AT, c_long(2 * 512 * 4), c_int(2), c_int(512)),
+    "vpsa_rans_decode": (AT, c_long(64), AT, AT, AT, None, AT, c_long(2 * 512 * 4), c_int(2), c_int(512)),
     "vpsa_row_add": (AT, c_long(64), AT, AT, AT, AT, AT, c_int(3), c_int(128), c_int(64)),
     "vpsa_row_qkv": (AT, c_long(64), AT, c_float(1e-5), AT, AT, AT, c_int(3), c_int(64), AT, AT, AT, AT, c_long(64), c_long(64), c_int(2), c_int(1)),
     "vpsa_mid_unit_factors": (AT, c_long(512), AT, c_float(1e-5), AT, AT, c_long(16384), c_int(3), c_int(32768), c_int(512)),

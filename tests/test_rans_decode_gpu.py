@@ -26,3 +26,19 @@ def test_rans_decode_edges(per_stream, shift):
     at.copy_(sizes.view(torch.int16))
     got = ops.rans_decode(freq.view(torch.int16).to(DEV), states.view(torch.int32).to(DEV), at, coded.to(DEV), n, n_ctx, spc)
     assert torch.equal(got.cpu(), sym)
+
+
+# as many workgroups as the chip holds at once, and one context more (two launches, a wave for 64 streams)
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_ctx", [96, 97])
+@pytest.mark.parametrize("per_stream", [1, 17, 372])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rans_decode_many_contexts(n_ctx, per_stream, shift):
+    spc = 512
+    g = torch.Generator(device=DEV).manual_seed(per_stream)
+    sym = torch.randint(-64, 64, (n_ctx * spc * per_stream,), generator=g, device=DEV).to(torch.int8)
+    sym[-spc * per_stream:] = 5
+    freq, states, sizes, coded = ops.rans_encode(sym, n_ctx, spc)
+    at = torch.zeros(sizes.numel() + 8, dtype=torch.int16, device=DEV)[shift:shift + sizes.numel()]
+    at.copy_(sizes.view(torch.int16))
+    assert torch.equal(ops.rans_decode(freq, states, at, coded, sym.numel(), n_ctx, spc), sym)

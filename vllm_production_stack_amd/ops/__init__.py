@@ -61,7 +61,7 @@ def _kernels():
             "vpsa_embed_rmsnorm", "vpsa_depth_mix_rmsnorm", "vpsa_poly_norm", "vpsa_soft_cap", "vpsa_mingru",
         ):
             getattr(lib, name).restype = c_int
-        for name in ("vpsa_prefill_split_record_bytes", "vpsa_rans_workspace",
+        for name in ("vpsa_prefill_split_record_bytes", "vpsa_rans_workspace", "vpsa_rans_decode_workspace",
                      "vpsa_page_workspace"):
             getattr(lib, name).restype = c_long
         kinds = {"p": c_void_p, "l": c_long, "i": c_int, "f": c_float}
@@ -1508,8 +1508,10 @@ def rans_decode(freq, states, sizes, coded, n, n_ctx, spc=RANS_SPC):
     freq, states, sizes = freq.contiguous(), states.contiguous(), sizes.to(torch.int16).contiguous()
     assert coded.is_contiguous() and freq.numel() >= n_ctx * 256 and min(states.numel(), sizes.numel()) >= n_ctx * spc
     assert freq.element_size() == 2 and states.element_size() == 4 and all(t.device == dev for t in (freq, states, sizes))
+    size = int(lib.vpsa_rans_decode_workspace(c_long(n), c_int(n_ctx), c_int(spc)))
+    ws = torch.empty(size, dtype=torch.uint8, device=dev) if size else None
     sym = torch.empty(n, dtype=torch.int8, device=dev)
-    _check(lib.vpsa_rans_decode(_p(coded), c_long(coded.numel()), _p(states), _p(freq), _p(sizes), _p(sym), c_long(n), c_int(n_ctx),
+    _check(lib.vpsa_rans_decode(_p(coded), c_long(coded.numel()), _p(states), _p(freq), _p(sizes), _p(ws), _p(sym), c_long(n), c_int(n_ctx),
                                 c_int(spc), _stream()), "rans_decode")
     return sym
 
