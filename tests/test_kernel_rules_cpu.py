@@ -80,3 +80,12 @@ def test_entropy_decoders_of_many_contexts_have_a_launch_for_their_tables():
     for n_ctx in (97, 126, 2048):
         tables = n_ctx * (4096 * 4 + 8)
         assert sizes(n_ctx, 16) == [tables, n_ctx * 512 * 16 + tables]
+
+
+# widths and rows, microseconds of a decode step of 6 layers with the split products / with those of a few rows on an MI355X
+@pytest.mark.parametrize("hidden,rows,split,whole", [
+    (5120, 4, 724.6, 731.0), (5120, 8, 747.0, 770.1), (5120, 14, 783.1, 851.8), (6144, 1, 923.2, 900.5), (6144, 8, 954.8, 953.3), (6144, 11, 980.0, 1000.2),
+    (6144, 14, 991.3, 1032.1), (7168, 8, 975.3, 954.6), (7168, 11, 999.5, 1011.0), (7168, 14, 1012.2, 1048.0), (8192, 14, 1295.6, 1280.6), (4096, 14, 657.9, 634.7),
+    (3584, 14, 605.7, 593.3), (3072, 14, 530.6, 511.0)])
+def test_products_of_a_few_rows_are_taken_where_they_are_faster(hidden, rows, split, whole):
+    assert (rows <= ops.row_limit(hidden)) == (whole < split)

@@ -952,16 +952,28 @@ def decode_attention_block(x, w, bias, pool, layer, meta, n_q, n_kv, head_dim, s
 #   3584, 18944                1     11.0/10.8  10.6/8.3   51.0/57.0  28.1/24.7    8      11.6/11.5  11.1/8.7  52.8/57.4  28.8/26.8    (296 workgroups: a second round)
 #   8192, 28672                1     33.2/31.6  29.2/25.8  149/150    79.2/74.3    16     33.8/37.6  29.9/28.5  148/150    79.5/92.7
 # A step of 8 layers (hidden 4096): 1 sequence 899 / 880, 2 936 / 877, 4 1098 / 1034, 8 1053 / 1006, 12 1118 / 1095, 14 1069 / 1047, 16 1072 / 1072.
+# Other widths have 16 of the hidden rows a workgroup in more than one round, and the last one is as long as the others: a step of 6 layers, before / with
+# them: 5120 wide (320 of 512 workgroups) 1 row 714 / 713 us, 8 rows 747 / 770, 14 rows 783 / 852; 6144 (384) 1 row 2.5 % ahead, 8 955 / 953, 9 968 / 974, 14 991 / 1032; 7168
+# (448) 8 rows 2.1 % ahead, 9 0.4 %, 11 999 / 1011, 14 1012 / 1048; 8192 (whole rounds) 1 row 3.6 % ahead, 14 1.2; 3072, 3584 and 4096 (one round) 14 rows 2.1 to 3.7 %.
 ROW_ROWS = 14
+ROW_ROWS_PART = 8   # where a last round is from ROW_PART on, but not nearly, full: up to 8 token rows go through LDS in one group
+ROW_PART = 0.75
+
+
+def row_limit(hidden: int) -> int:
+    """Rows up to which a decode step takes ``row_gemm``'s products at a width."""
+    tiles = hidden // 16
+    fill = tiles / (-(-tiles // TILE_CUS) * TILE_CUS)
+    return ROW_ROWS if tiles <= TILE_CUS or fill > 0.95 else ROW_ROWS_PART if fill >= ROW_PART else 0
 
 
 def row_layer_takes(residual, lw, pool, meta, n_q, n_kv, head_dim, cos_sin) -> bool:
     """Whether a decoder layer of a decode step takes ``row_gemm``'s products: few rows, projections that fill three quarters of the chip's
-    workgroups, a gated unit in one round of them, operands that the kernels read."""
+    workgroups (``row_limit``), a gated unit in one round of them, operands that the kernels read."""
     m, h = residual.shape
     if isinstance(pool, LayerGroupedPool):
         pool = pool.groups[0]
-    if (m > ROW_ROWS or not residual.is_cuda or head_dim != HEAD_DIM_HIP or meta.slots is None or meta.num_decode != m or meta.num_prefill_seqs > 0
+    if (m > min(ROW_ROWS, row_limit(h)) or not residual.is_cuda or head_dim != HEAD_DIM_HIP or meta.slots is None or meta.num_decode != m or meta.num_prefill_seqs > 0
             or lw.w_gate_up is None or lw.w_gate_up_p is not None or lw.w_down_p is not None or pool.dtype != torch.bfloat16
             or _generic_attention(residual, head_dim) or h > 8192):
         return False
