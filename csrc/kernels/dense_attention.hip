@@ -164,8 +164,8 @@ VPSA_EXPORT int vpsa_dense_decode_attention(const void* q, long q_bs, const void
 // the first 1024 (74.0 us by themselves); started behind them they come to lie on few CUs.  So they are cut in two (dense_attn_rows<true>: half the
 // rows, a pair of waves shares them and takes every other tile, K's and V's two tiles loaded in turn) and 256 of the first 1024, one
 // on each CU, go on with them: 84.2 -> 80.8 us, 88 pairs 79.9 -> 74.8, 22 windows x 8 heads 140.3 -> 135.4; with 256 or 512 left the halves share
-// CUs and gain nothing (89.4 / 89.6, 106 / 111), so they stay whole.  Up to 256 workgroups in all are cut as well: eight pairs 23.6 -> 15.8, 12 and
-// 16 pairs 23.9 -> 22.3 (half of the halves share a CU; 24 pairs 34.2 / 34.2), four query rows of 64 pairs 21.9 -> 14.2.  (The
+// CUs and gain nothing (89.4 / 89.6, 106 / 111), so they stay whole.  Calls of up to 256 workgroups are cut as well where that pays (dense_blocks_cut): eight pairs 23.6 ->
+// 15.8, 12 and 16 pairs 23.9 -> 22.3 (half of the halves share a CU; 24 pairs 34.2 / 34.2), four query rows of 64 pairs 21.9 -> 14.2.  (The
 // two waves with 32 keys of every tile: 18.7 where this takes 17.7.)  (The next tile's scores under this one's exponentials need 182
 // registers: two workgroups a CU, 23.4 us for one window instead of 26.5 but 91 for 8 and 305 for 32.)  The scale goes into the
 // exponent's fused multiply, the mask only touches the last tile, and a window's query blocks run on one XCD.  Measured: 8
@@ -352,21 +352,14 @@ __device__ __forceinline__ void dense_attn_rows(
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (!masked.value) stage_two(i + 1, ksrc, kbase_p, kc, lds_k);
-      values(lds_v[part], alpha);
+      // (of an odd number of tiles the last one has no partner: its place holds repeats of the last key, whose values may be infinite)
+      if (!masked.value || 2 * i + part < n_tiles) values(lds_v[part], alpha);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     };
     const int n = (n_tiles + 1) >> 1;
     for (int i = 0; i + 1 < n; ++i) two(i, std::false_type{});
-    // of an odd number of tiles the last one has no partner: its place holds repeats of the last key, whose values may be infinite
-    if (2 * (n - 1) + part < n_tiles) {
-      two(n - 1, std::true_type{});
-    } else {
-      stage_two(n - 1, vsrc, vbase_p, vc, lds_v);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      __syncthreads();
-    }
+    two(n - 1, std::true_type{});
   } else {
     auto tile = [&](int t, auto masked) {
       const int buf = t & 1;
@@ -416,7 +409,9 @@ __device__ __forceinline__ void dense_attn_rows(
 }
 
 // Blocks of 128 rows, by `whole` workgroups (a multiple of 8); `left` blocks more in two of 64 each, by those workgroups from `first` on
-// when they are done with theirs (whole 0: by workgroups of their own).
+// when they are done with theirs (whole 0: by workgroups of their own).  WHOLE, CUT: whether there are such.  (In one kernel with the other
+// path the loop over whole tiles is scheduled otherwise: 200 keys, 288 workgroups 9.55 -> 10.4.)
+template <bool WHOLE, bool CUT>
 __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
     const uint16_t* __restrict__ q, long q_bs, long q_ts, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, long kv_bs, long kv_ts, uint16_t* __restrict__ out, long o_bs,
@@ -431,10 +426,25 @@ __global__ __launch_bounds__(256, 4) void dense_attn_fwd_kernel(
       dense_attn_rows<decltype(pairs_of_waves)::value>(q, q_bs, q_ts, k, v, kv_bs, kv_ts, out, o_bs, o_ts, Tq, Tk, pair % heads, pair / heads,
                                                        row, scale_log2e, lds, lds + 2);
   };
-  if ((int)blockIdx.x < whole) rows(std::false_type{}, blockIdx.x >> 3, 0);
+  if constexpr (WHOLE) rows(std::false_type{}, blockIdx.x >> 3, 0);  // (as many workgroups as there are)
   const int past = (int)blockIdx.x - first;
-  if (past >= 0 && past < 2 * left) rows(std::true_type{}, (whole >> 3) + (past >> 4), (past >> 3 & 1) * 64);
+  if (CUT && past >= 0 && past < 2 * left) rows(std::true_type{}, (whole >> 3) + (past >> 4), (past >> 3 & 1) * 64);
 }
+
+// Blocks of 128 rows that are cut in two (microseconds whole / cut).  Behind whole rounds of four a CU: up to 128 of them, see above.  In calls
+// that the chip holds at once a pair of waves spares half of the tiles and costs a wave's exchange.  Where every half has a CU to itself that pays from
+// two tiles on with more than 64 rows (32 workgroups, 65 keys 5.43 / 5.00, 129 6.23 / 5.99, 1500 22.8 / 14.9), from four on with fewer, whose second half is
+// empty (64 rows, 65 keys 4.80 / 4.97, 129 5.58 / 5.89, 200 6.34 / 6.03, 1500 22.0 / 14.7).  Up to 256 workgroups, whose halves share CUs, it does from 15
+// tiles on (192 workgroups, 129 keys 6.6 / 7.6, 300 8.2 / 9.3, 700 13.0 / 13.6, 800 14.3 / 14.2 to 14.6, 1000 16.9 / 15.9, 1500 23.5 / 21.7; 256, 700 keys 13.4 / 14.2,
+// 1000 17.4 / 16.5).
+static int dense_blocks_cut(long pairs, int Tq, int Tk) {
+  const long columns = (pairs + 7) / 8 * 8, groups = columns * ((Tq + 127) / 128), halves = columns * ((Tq + 63) / 64), left = groups % 1024;
+  if (Tk <= DF_KT) return 0;
+  if (groups >= 1024) return left <= 128 ? (int)left : 0;
+  if (halves <= 256) return Tk > (Tq > 64 ? 1 : 3) * DF_KT ? (int)left : 0;
+  return groups <= 256 && Tk > 14 * DF_KT ? (int)left : 0;
+}
+VPSA_EXPORT int vpsa_dense_attention_cut(int B, int heads, int Tq, int Tk) { return dense_blocks_cut((long)B * heads, Tq, Tk); }
 
 // q [B][Tq][heads * 64], k / v [B][Tk][heads * 64], out [B][Tq][heads * 64]; strides in elements
 // (batch, position), unit stride over channels, every row start 16-byte aligned (out: 8-byte).
@@ -449,11 +459,11 @@ VPSA_EXPORT int vpsa_dense_attention(const void* q, long q_bs, long q_ts, const 
   const int q_blocks = (Tq + 127) / 128;
   const long pairs = (long)B * heads, groups = (pairs + 7) / 8 * 8 * q_blocks;
   if (groups >= (1L << 31)) return -1;
-  int left = (int)(groups % 1024);  // (behind whole rounds of four a CU; the lines: see above)
-  if (left > (groups < 1024 ? 256 : 128) || Tk <= DF_KT) left = 0;  // (two tiles at least)
+  const int left = dense_blocks_cut(pairs, Tq, Tk);
   const int whole = (int)groups - left;
-  hipLaunchKernelGGL(dense_attn_fwd_kernel, dim3(whole ? whole : 2 * left), dim3(256), 0, stream,
-                     (const uint16_t*)q, q_bs, q_ts, (const uint16_t*)k, (const uint16_t*)v, kv_bs, kv_ts,
-                     (uint16_t*)out, o_bs, o_ts, Tq, Tk, heads, (int)pairs, q_blocks, whole, whole ? whole - 1024 : 0, left, scale * 1.4426950408889634f);
+  auto* const kernel = left == 0 ? dense_attn_fwd_kernel<true, false> : whole == 0 ? dense_attn_fwd_kernel<false, true> : dense_attn_fwd_kernel<true, true>;
+  hipLaunchKernelGGL(kernel, dim3(whole ? whole : 2 * left), dim3(256), 0, stream, (const uint16_t*)q, q_bs, q_ts, (const uint16_t*)k,
+                     (const uint16_t*)v, kv_bs, kv_ts, (uint16_t*)out, o_bs, o_ts, Tq, Tk, heads, (int)pairs, q_blocks, whole, whole ? whole - 1024 : 0, left,
+                     scale * 1.4426950408889634f);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -89,3 +89,16 @@ def test_entropy_decoders_of_many_contexts_have_a_launch_for_their_tables():
     (3584, 14, 605.7, 593.3), (3072, 14, 530.6, 511.0)])
 def test_products_of_a_few_rows_are_taken_where_they_are_faster(hidden, rows, split, whole):
     assert (rows <= ops.row_limit(hidden)) == (whole < split)
+
+
+# windows, heads, query rows, keys, microseconds with whole blocks of 128 rows / with blocks cut in two on an MI355X
+@pytest.mark.parametrize("b,heads,tq,tk,whole,cut", [
+    (1, 8, 1, 1500, 21.6, 13.9), (8, 8, 4, 1500, 21.8, 14.1), (1, 8, 64, 65, 4.80, 4.97), (2, 12, 64, 129, 5.60, 5.95), (3, 20, 4, 129, 5.23, 5.42), (3, 20, 64, 200, 6.49, 6.16),
+    (1, 12, 130, 65, 5.41, 5.00), (1, 8, 500, 129, 6.21, 6.00), (8, 8, 130, 300, 7.94, 7.11), (4, 8, 500, 448, 9.60, 8.25), (1, 8, 1500, 1500, 23.0, 15.4),
+    (1, 12, 1500, 129, 6.62, 7.55), (2, 8, 1500, 300, 8.22, 9.31), (1, 12, 1500, 700, 13.03, 13.62), (1, 12, 1500, 1000, 16.9, 15.9), (2, 8, 1500, 1500, 23.27, 22.29),
+    (8, 8, 500, 129, 6.99, 7.77), (3, 20, 500, 448, 10.46, 11.32), (8, 8, 500, 1500, 24.31, 23.42), (8, 12, 1500, 1500, 84.2, 80.8), (22, 8, 1500, 1500, 140.3, 135.4)])
+def test_attention_blocks_are_cut_where_that_is_faster(b, heads, tq, tk, whole, cut):
+    left = ops._kernels().vpsa_dense_attention_cut(c_int(b), c_int(heads), c_int(tq), c_int(tk))
+    assert (left > 0) == (cut < whole)
+    assert ops._kernels().vpsa_dense_attention_cut(c_int(b), c_int(heads), c_int(tq), c_int(64)) == 0  # a single tile
+    assert left <= -(-b * heads // 8) * 8 * -(-tq // 128) and left % 8 == 0
