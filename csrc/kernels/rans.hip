@@ -18,7 +18,7 @@
 //   decoder  one table entry per step (symbol, frequency and offset within it), the streams' coded bytes staged in LDS and read
 //            two at a time, at most two bytes a step without a loop.
 // Page of a 32-layer cache with 8 KV heads (4.2 M symbols): coding loop 107 -> 25 us, with tables and gathering 150 -> 47; decoding
-// 118 -> 24 us (before: 64 workgroups, symbols and coded bytes read and written one at a time from memory, divisions).
+// 118 -> 24 us, 29 beside the copy of the next page (before: 64 workgroups, symbols and coded bytes read and written one at a time from memory, divisions).
 // Per context: a 256-entry frequency table normalised to 2^12,
 // built from a histogram of that very page (it travels with the blob: 512 B per context).
 // Coder: 32-bit state, byte-wise renormalisation, lower bound 2^23.  The encoder runs over its
@@ -627,8 +627,9 @@ VPSA_EXPORT int vpsa_copy_parts(long size) { return copy_parts(size); }
 // `size` bytes from the device to `to` by way of a pinned buffer.  Over on return.  (Four parts, each leaving the buffer while the next is on
 // its way, were no faster, 158 us a page against 162, and on the way back they cost the device 50 us a page: a copy's start is 10 to 15.
 // A kernel that stores the coded bytes into pinned memory right behind the coder spares the host one of its two waits, 201 us a page against 213 to 220,
-// but its workgroups lie on the CUs as long as the link takes: a decode step of 12 sequences on another stream took 2830 us beside
-// one thread that encodes pages and 4170 to 4520 beside two, instead of 2160 and 2350; 1920 to 1990 by itself.)
+// but it gathers them in LDS, and its workgroups lie on the CUs as long as the link takes: products whose workgroups want most of a CU's LDS find no
+// place beside them.  A decode step of 12 sequences on another stream took 2830 us beside one thread that encodes pages and 4170 to 4520 beside two,
+// with the runtime's copy, which holds no LDS, 2100 to 2160 and 2350; 1920 by itself.)
 VPSA_EXPORT int vpsa_fetch(const void* from, void* pinned, void* to, long size, hipStream_t stream) {
   const bool sent = hipMemcpyAsync(pinned, from, size, hipMemcpyDeviceToHost, stream) == hipSuccess;
   if (hipStreamSynchronize(stream) != hipSuccess || !sent) return -3;
@@ -651,8 +652,8 @@ VPSA_EXPORT hipStream_t vpsa_page_copy_stream() {
   return mine;
 }
 
-// The copy of a page on that stream, so that it runs beside the kernels of the page before it (3.5 MB: 67 us of copy, 30 of kernels);
-// `stream` waits for it, and it for nothing but the copies before it: all callers share it.  fresh: `body` is new to the caller, and what
+// The copy of a page on that stream, so that it runs beside the kernels of the page before it (3.5 MB: 67 us of copy, 30 of kernels by themselves and
+// 34 beside it); `stream` waits for it, and it for nothing but the copies before it: all callers share it.  fresh: `body` is new to the caller, and what
 // `stream` still has to do may touch its memory; the copy then stands in `stream`, where nobody else waits for it.  Below 2 MB the
 // events cost the host, which is behind there anyway, what the copy takes (a page of 1.5 MB of many, one stream / two: 87 / 91 us; of 3.5 MB
 // 143 / 115, of 8 MB 238 / 196; with helpers that wait).

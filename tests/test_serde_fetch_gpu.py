@@ -1,5 +1,5 @@
-"""What a page's encoder leaves to the copy engine: kernels that store a page into host memory keep their places on the chip as long as the link takes,
-and a step on another stream waits for them."""
+"""What a page's encoder leaves to the runtime's copy: a kernel that gathers a page in LDS and stores it into host memory keeps its places on the chip as
+long as the link takes, and a step on another stream waits for them."""
 
 import pytest
 import torch
